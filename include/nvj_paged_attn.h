@@ -380,6 +380,22 @@ NVJ_API int nvj_qk_norm_rope_store_launch(void* stream,
                             int32_t num_kv_heads, int32_t head_dim, int64_t num_slots);
 
 /*
+ * The same with the new rows wherever the caller wants them: q rows of q_row_stride
+ * elements, which may be the projection itself (q_out = qkv: rotated in place); and,
+ * when not NULL, the K and V rows besides the cache (rows of kv_row_stride elements,
+ * written for every token whatever its slot; k_out may be the K part of qkv).
+ */
+NVJ_API int nvj_qk_norm_rope_rows_launch(void* stream,
+                            const void* qkv, int64_t qkv_row_stride,
+                            const int32_t* positions, const float* cos_sin_cache,
+                            int32_t max_position, const float* q_norm_weight,
+                            const float* k_norm_weight, float eps,
+                            const int32_t* slot_mapping, void* k_cache, void* v_cache,
+                            void* q_out, int64_t q_row_stride, void* k_out, void* v_out,
+                            int64_t kv_row_stride, int32_t num_tokens, int32_t num_heads,
+                            int32_t num_kv_heads, int32_t head_dim, int64_t num_slots);
+
+/*
  * Advance the device-resident metadata of a decode batch by one step, in
  * place.  Replaces the per-step host rebuild and upload of
  * ModelRunner._prepare_decode (engine/model_runner.py:334-376): once a step has
@@ -501,6 +517,65 @@ NVJ_API int nvj_add_rms_norm_launch(void* stream, const void* x, const void* res
  */
 NVJ_API int nvj_silu_and_mul_launch(void* stream, const void* x, int64_t x_row_stride,
                             void* y, int32_t num_tokens, int32_t intermediate);
+
+/*
+ * One step of the whole decoder stack for up to 16 token rows: a decode batch or a
+ * short prefill, up to the logits.  Covers the model of
+ * models/qwen3.py:130-172, 285-318, 366-393 and 472-491 (embedding; per layer
+ * RMSNorm, fused QKV, QK-RMSNorm, RoPE, KV store, attention, output projection,
+ * RMSNorm, SiLU MLP; final norm and tied LM head) as six launches per layer.
+ *
+ * Weights are bf16 [outputs, inputs] row-major, norm weights float32.  Projections
+ * and the residual stream are rounded to bf16 where a separate launch would have
+ * stored them.  head_dim must be 128, hidden 256, 512, 1024 or 2048,
+ * num_heads * head_dim and intermediate multiples of 256 and at most 3072; every
+ * pointer 16-byte aligned.
+ * Enqueue-only; nothing is allocated.
+ */
+typedef struct nvj_decoder_model {
+  const void* embed;          /* [vocab, hidden] bf16, also the LM head */
+  const float* final_norm;    /* [hidden] */
+  const float* cos_sin;       /* [max_position, head_dim]: cos | sin */
+  int32_t num_layers, hidden, num_heads, num_kv_heads, head_dim, intermediate, vocab;
+  int32_t max_position, block_size, num_blocks;
+  float eps, scale;
+} nvj_decoder_model;
+
+typedef struct nvj_decoder_layer {
+  const void* qkv;            /* [(Hq + 2 Hkv) * head_dim, hidden] bf16 */
+  const void* o;              /* [hidden, Hq * head_dim] */
+  const void* gate_up;        /* [2 * intermediate, hidden] */
+  const void* down;           /* [hidden, intermediate] */
+  const float* ln1;           /* [hidden] */
+  const float* ln2;           /* [hidden] */
+  const float* q_norm;        /* [head_dim], or NULL with k_norm */
+  const float* k_norm;
+  void* k_cache;              /* [num_blocks, block_size, Hkv, head_dim] bf16 */
+  void* v_cache;
+} nvj_decoder_layer;
+
+typedef struct nvj_decoder_batch {
+  const int32_t* input_ids;      /* [num_tokens]; out of range is clamped */
+  const int32_t* positions;      /* [num_tokens] */
+  const int32_t* slot_mapping;   /* [num_tokens] */
+  const int32_t* context_lens;   /* decode: [num_sequences] */
+  const int32_t* block_tables;   /* [num_sequences, max_blocks]; prefill: NULL = packed rows */
+  const int32_t* cu_seqlens_q;   /* prefill: [num_sequences + 1] */
+  const int32_t* cu_seqlens_k;
+  const int32_t* last_token_indices;  /* prefill: [num_sequences], the rows that get logits */
+  void* partials;                /* decode: as nvj_paged_decode_launch_counters (chunk 0) or */
+  size_t partial_bytes;          /*   the workspace of nvj_paged_decode_launch_phases */
+  void* counters;
+  size_t counter_bytes;
+  void* logits;                  /* [num_sequences, vocab] bf16, or NULL */
+  int32_t num_tokens, num_sequences, max_blocks, chunk, is_prefill, clear_counters;
+} nvj_decoder_batch;
+
+NVJ_API size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
+                            int32_t num_tokens);
+NVJ_API int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* model,
+                            const nvj_decoder_layer* layers, const nvj_decoder_batch* batch,
+                            void* workspace, size_t workspace_bytes);
 
 #ifdef __cplusplus
 }  /* extern "C" */

@@ -18,8 +18,35 @@ NVJ_DTYPE_BF16 = 0
 NVJ_DTYPE_F32 = 1
 NVJ_DTYPE_F16 = 2
 
-# every symbol include/nvj_paged_attn.h declares: name -> (restype, argtypes)
 _c = ctypes
+
+
+class DecoderModel(ctypes.Structure):
+    """``nvj_decoder_model``."""
+    _fields_ = [(n, _c.c_void_p) for n in ("embed", "final_norm", "cos_sin")] + [
+        (n, _c.c_int32) for n in ("num_layers", "hidden", "num_heads", "num_kv_heads", "head_dim",
+                                  "intermediate", "vocab", "max_position", "block_size",
+                                  "num_blocks")] + [("eps", _c.c_float), ("scale", _c.c_float)]
+
+
+class DecoderLayer(ctypes.Structure):
+    """``nvj_decoder_layer``."""
+    _fields_ = [(n, _c.c_void_p) for n in ("qkv", "o", "gate_up", "down", "ln1", "ln2", "q_norm",
+                                           "k_norm", "k_cache", "v_cache")]
+
+
+class DecoderBatch(ctypes.Structure):
+    """``nvj_decoder_batch``."""
+    _fields_ = [(n, _c.c_void_p) for n in (
+        "input_ids", "positions", "slot_mapping", "context_lens", "block_tables", "cu_seqlens_q",
+        "cu_seqlens_k", "last_token_indices")] + [
+        ("partials", _c.c_void_p), ("partial_bytes", _c.c_size_t), ("counters", _c.c_void_p),
+        ("counter_bytes", _c.c_size_t), ("logits", _c.c_void_p)] + [
+        (n, _c.c_int32) for n in ("num_tokens", "num_sequences", "max_blocks", "chunk",
+                                  "is_prefill", "clear_counters")]
+
+
+# every symbol include/nvj_paged_attn.h declares: name -> (restype, argtypes)
 SYMBOLS = {
     "nvj_error_string": (_c.c_char_p, [_c.c_int]),
     "nvj_abi_version": (_c.c_int, []),
@@ -57,6 +84,11 @@ SYMBOLS = {
         _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p,
         _c.c_void_p, _c.c_float, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p,
         _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int64]),
+    "nvj_qk_norm_rope_rows_launch": (_c.c_int, [
+        _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p,
+        _c.c_void_p, _c.c_float, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int64,
+        _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int32,
+        _c.c_int64]),
     "nvj_advance_decode_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p,
         _c.c_void_p, _c.c_int32, _c.c_int32, _c.c_int32]),
@@ -70,6 +102,10 @@ SYMBOLS = {
         _c.c_int32, _c.c_int32]),
     "nvj_silu_and_mul_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int32, _c.c_int32]),
+    "nvj_decoder_step_workspace_bytes": (_c.c_size_t, [_c.POINTER(DecoderModel), _c.c_int32]),
+    "nvj_decoder_step_launch": (_c.c_int, [
+        _c.c_void_p, _c.POINTER(DecoderModel), _c.POINTER(DecoderLayer), _c.POINTER(DecoderBatch),
+        _c.c_void_p, _c.c_size_t]),
 }
 NVJ_CHUNK_WHOLE_SEQUENCE = -1
 NVJ_STATIC_SCRATCH_BYTES = 16 << 20

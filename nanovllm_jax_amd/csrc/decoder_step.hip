@@ -1,0 +1,518 @@
+// One step of the whole decoder stack for a small number of token rows (a decode
+// batch, or a short prefill) as a chain of six launches per layer for gfx950.
+//
+// Covers the layer body of models/qwen3.py:130-172 and :285-318 of the reference
+// (fused QKV, per-head QK-RMSNorm, RoPE, store, attention, output projection,
+// pre-norm with fused residual, SiLU MLP), the embedding and the tied LM head
+// (:366-393, :472-491):
+//   1. norm_gemm QKV       RMSNorm in the prologue
+//   2. qk_norm_rope_store
+//   3. attention           the paged decode or the prefill kernel
+//   4. residual_gemm O     adds into the residual stream
+//   5. norm_gemm GATE_UP   RMSNorm in the prologue, SiLU(gate) * up in the epilogue
+//   6. residual_gemm DOWN
+// The residual stream h holds the unrounded fp32 sums that the next norm is taken
+// over; the sum that follows adds to their bf16 rounding, so every value is
+// rounded where the separate kernels (layer_glue.hip) round it.
+//
+// What bounds it: with few rows every product streams its weights once and the rest
+// is latency, so a launch is worth its fixed 2-3 us only if the weights it
+// needs are all requested before anything else is waited for, by all CUs (one CU
+// alone draws some 50 GB/s).  Each wave therefore issues the loads of its whole
+// share of the weights at once, straight into the registers the matrix core reads
+// them from (a wave's share is used by that wave only, LDS would add nothing), and
+// does the norm prologue under them.  The token rows are the N side of
+// v_mfma_f32_16x16x32_bf16 (weights A, rows B), 16 per column tile.
+//
+// Order of the sums.  A network of random bf16 weights doubles any difference of one
+// ulp from stage to stage until all roundings differ (two GEMM kernels that sum in
+// different orders end 2-3 % apart in the logits after 28 layers), so these
+// products sum in the order of the GEMMs a step of more rows runs through, and give
+// the same bits: the reduction is cut into `chains` interleaved runs of `run`
+// steps of 32, each chain is accumulated in order and the chains are added in
+// order (struct Chains).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "launch.h"
+#include "nvj_paged_attn.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int kMaxRows = 16;   // token rows of one step: one column tile
+
+__device__ __forceinline__ float bf16_to_f32(uint16_t b) {
+  return __uint_as_float((uint32_t)b << 16);
+}
+__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
+}
+__device__ __forceinline__ f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const bf16x2 p = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, p);
+}
+
+enum Epilogue { kPlain, kSiluMul };
+
+struct NormGemmArgs {
+  const float4* h;            // [rows, hidden] residual stream
+  const int32_t* row_index;   // rows to take from h, or null: row m is row m
+  const float* norm_weight;   // [hidden]
+  const char* weight;         // [outputs, hidden] bf16
+  uint16_t* out;              // kPlain [rows, outputs], kSiluMul [rows, outputs / 2]
+  float eps;
+  int num_tokens, outputs;
+};
+
+// RMSNorm of up to 16 rows of h into LDS as bf16, `WAVES` waves, a row each at a time;
+// the arithmetic and its order are those of add_rms_norm_kernel (layer_glue.hip).
+// 16-byte pieces are XOR-permuted by the row so that the B-operand reads are free of
+// bank conflicts.  hidden = 256 * RV.  Two halves, so that the caller can issue other
+// loads in between.
+template <int RV, int ROWS>
+struct NormPrologue {
+  static constexpr int kHidden = 256 * RV;
+  static constexpr int kPieces = kHidden / 8;               // of a row
+  static constexpr int kPerLane = (kPieces + 63) / 64;
+  float4 x[ROWS][kPerLane][2], g[kPerLane][2];
+
+  __device__ __forceinline__ void load(const NormGemmArgs& a, int wave, int waves, int lane) {
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+      const int token = min(wave + waves * j, a.num_tokens - 1);
+      const int row = a.row_index ? a.row_index[token] : token;
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) {
+        const int p = min(lane + 64 * i, kPieces - 1);
+        const float4* src = a.h + (int64_t)row * (kHidden / 4) + 2 * p;
+        x[j][i][0] = src[0];
+        x[j][i][1] = src[1];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+      const int p = min(lane + 64 * i, kPieces - 1);
+      g[i][0] = reinterpret_cast<const float4*>(a.norm_weight)[2 * p];
+      g[i][1] = reinterpret_cast<const float4*>(a.norm_weight)[2 * p + 1];
+    }
+  }
+
+  __device__ __forceinline__ void store(uint4* lds, float eps, int wave, int waves, int lane) const {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+      const int m = wave + waves * j;   // (a row beyond the last token repeats it)
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) {
+        if (kPieces % 64 == 0 || lane + 64 * i < kPieces) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const float4 v = x[j][i][u];
+            sum = sum + v.x * v.x;
+            sum = sum + v.y * v.y;
+            sum = sum + v.z * v.z;
+            sum = sum + v.w * v.w;
+          }
+        }
+      }
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+      const float rs = 1.0f / __builtin_sqrtf(sum * (1.0f / (float)kHidden) + eps);
+#pragma unroll
+      for (int i = 0; i < kPerLane; ++i) {
+        const int p = lane + 64 * i;
+        const float4 u = x[j][i][0], v = x[j][i][1], gu = g[i][0], gv = g[i][1];
+        if (kPieces % 64 == 0 || p < kPieces)
+          lds[m * kPieces + (p ^ m)] =
+              make_uint4(pack2(u.x * rs * gu.x, u.y * rs * gu.y),
+                         pack2(u.z * rs * gu.z, u.w * rs * gu.w),
+                         pack2(v.x * rs * gv.x, v.y * rs * gv.y),
+                         pack2(v.z * rs * gv.z, v.w * rs * gv.w));
+      }
+    }
+  }
+};
+
+// out[m][n] = bf16(norm(h[m]) . weight[n]) for up to 16 rows, four chains of single
+// steps: one 16-output tile per workgroup, a chain per wave.  kSiluMul: the tile is 8
+// gate and the matching 8 up columns.
+template <int RV, int ROWS, Epilogue EPI>
+__global__ __launch_bounds__(256) void norm_gemm_kernel(NormGemmArgs a) {
+  constexpr int kWaves = 4;                  // = chains
+  constexpr int kPieces = 32 * RV;
+  constexpr int kSteps = 8 * RV / kWaves;    // reduction steps of one chain
+  constexpr int kStride = 20;                // floats per row of partial sums
+  __shared__ uint4 rows[16 * kPieces];
+  __shared__ float red[kWaves][16 * kStride];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int half = a.outputs / 2;
+  const int n = EPI == kSiluMul ? (int)blockIdx.x * 8 + (r & 7) + (r < 8 ? 0 : half)
+                                : (int)blockIdx.x * 16 + r;
+  const char* wrow = a.weight + (int64_t)n * (kPieces * 16) + 64 * wave + 16 * kg;
+  NormPrologue<RV, ROWS> norm;
+  norm.load(a, wave, kWaves, lane);
+  // loads return in order: the weights are asked for right behind the rows, so that
+  // the norm waits for the rows alone
+  uint4 w[kSteps];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i)
+    w[i] = *reinterpret_cast<const uint4*>(wrow + 64 * kWaves * i);
+  __builtin_amdgcn_sched_barrier(0);
+  norm.store(rows, a.eps, wave, kWaves, lane);
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};   // D[output][row]
+  // (with fewer than 16 rows in LDS the other columns read what is there: not stored)
+  const int m = ROWS * kWaves >= 16 ? r : r % (ROWS * kWaves);
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i)
+    acc = mfma(w[i], rows[m * kPieces + ((4 * (kWaves * i + wave) + kg) ^ m)], acc);
+  *reinterpret_cast<f32x4*>(&red[wave][r * kStride + 4 * kg]) = acc;
+  __syncthreads();
+  auto total = [&](int row, int col) {
+    float v = red[0][row * kStride + col];
+#pragma unroll
+    for (int p = 1; p < kWaves; ++p) v += red[p][row * kStride + col];
+    return f32_to_bf16_rne(v);
+  };
+  if constexpr (EPI == kSiluMul) {
+    const int row = threadIdx.x >> 3, col = threadIdx.x & 7;
+    if (row < a.num_tokens) {
+      const float g = bf16_to_f32(total(row, col)), u = bf16_to_f32(total(row, 8 + col));
+      a.out[(int64_t)row * half + blockIdx.x * 8 + col] =
+          f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
+    }
+  } else {
+    const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
+    if (row < a.num_tokens)
+      a.out[(int64_t)row * a.outputs + blockIdx.x * 16 + col] = total(row, col);
+  }
+}
+
+// The same with one chain, for many outputs (the LM head): every wave owns a whole
+// 16-output tile, its weights in flight together.
+template <int RV, int ROWS>
+__global__ __launch_bounds__(256) void norm_gemm_wide_kernel(NormGemmArgs a) {
+  constexpr int kWaves = 4;
+  constexpr int kPieces = 32 * RV;
+  constexpr int kSteps = 8 * RV;
+  constexpr int kDepth = kSteps < 32 ? kSteps : 32;
+  __shared__ uint4 rows[16 * kPieces];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int n0 = (blockIdx.x * kWaves + wave) * 16;
+  const char* wrow =
+      a.weight + (int64_t)min(n0 + r, a.outputs - 1) * (kPieces * 16) + 16 * kg;
+  NormPrologue<RV, ROWS> norm;
+  norm.load(a, wave, kWaves, lane);
+  uint4 w[kDepth];
+#pragma unroll
+  for (int i = 0; i < kDepth; ++i) w[i] = *reinterpret_cast<const uint4*>(wrow + 64 * i);
+  __builtin_amdgcn_sched_barrier(0);
+  norm.store(rows, a.eps, wave, kWaves, lane);
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int m = ROWS * kWaves >= 16 ? r : r % (ROWS * kWaves);
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {
+    acc = mfma(w[i % kDepth], rows[m * kPieces + ((4 * i + kg) ^ m)], acc);
+    if (i + kDepth < kSteps)
+      w[i % kDepth] = *reinterpret_cast<const uint4*>(wrow + 64 * (i + kDepth));
+  }
+  if (r < a.num_tokens) {
+    uint16_t* dst = a.out + (int64_t)r * a.outputs + n0 + 4 * kg;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n0 + 4 * kg + e < a.outputs) dst[e] = f32_to_bf16_rne(acc[e]);
+  }
+}
+
+// h[m][n] = bf16(x[m][:] . weight[n][:]) + bf16(h[m][n]) for up to 16 rows.  A
+// workgroup owns NR outputs (the A rows repeat NR of them: narrower tiles put more CUs
+// on a matrix of few outputs) and has a wave for each of CHAINS x PARTS shares of the
+// reduction: T steps, whose operands all waves fetch at once.  The parts of a chain
+// hand its sum on through LDS, in order; the chains are added at the end.
+template <int NR, int CHAINS, int RUN, int PARTS, int T>
+__global__ __launch_bounds__(CHAINS * PARTS * 64) void residual_gemm_kernel(
+    const char* __restrict__ x, const char* __restrict__ weight, float* __restrict__ h,
+    int num_tokens, int outputs) {
+  constexpr int64_t kRowBytes = (int64_t)CHAINS * PARTS * T * 64;
+  __shared__ f32x4 sums[CHAINS][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chain = wave % CHAINS, part = wave / CHAINS;
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * NR;
+  const char* wrow = weight + (int64_t)(n0 + r % NR) * kRowBytes + 16 * kg;
+  const char* xrow = x + min(r, num_tokens - 1) * kRowBytes + 16 * kg;
+  uint4 w[T], b[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int j = part * T + i;   // step of the chain
+    const int at = 64 * (j / RUN * (CHAINS * RUN) + chain * RUN + j % RUN);
+    w[i] = *reinterpret_cast<const uint4*>(wrow + at);
+    b[i] = *reinterpret_cast<const uint4*>(xrow + at);
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) {
+    if (part == p) {
+      if (p > 0) acc = sums[chain][lane];
+#pragma unroll
+      for (int i = 0; i < T; ++i) acc = mfma(w[i], b[i], acc);
+      sums[chain][lane] = acc;
+    }
+    __syncthreads();
+  }
+  if (wave == 0 && r < num_tokens && 4 * kg < NR) {
+    f32x4 v = sums[0][lane];
+#pragma unroll
+    for (int c = 1; c < CHAINS; ++c) v += sums[c][lane];
+    float4* at = reinterpret_cast<float4*>(h + (int64_t)r * outputs + n0 + 4 * kg);
+    const float4 old = *at;
+    auto round = [](float f) { return bf16_to_f32(f32_to_bf16_rne(f)); };
+    *at = make_float4(round(v[0]) + round(old.x), round(v[1]) + round(old.y),
+                      round(v[2]) + round(old.z), round(v[3]) + round(old.w));
+  }
+}
+
+// Waves per chain: the shares are at most 12 steps (96 registers of operands).
+template <int CHAINS, int RUN, int PARTS>
+hipError_t launch_residual_gemm(hipStream_t s, const void* x, const void* weight, float* h,
+                                int num_tokens, int outputs, int reduction) {
+  constexpr int NR = 8;
+  const dim3 grid((unsigned)(outputs / NR)), block(CHAINS * PARTS * 64);
+#define NVJ_CASE(TV)                                                                              \
+  case TV:                                                                                        \
+    return nvj::launch(residual_gemm_kernel<NR, CHAINS, RUN, PARTS, TV>, grid, block, s,          \
+                       static_cast<const char*>(x), static_cast<const char*>(weight), h,          \
+                       num_tokens, outputs)
+  switch (reduction / (CHAINS * PARTS * 32)) {
+    NVJ_CASE(1); NVJ_CASE(2); NVJ_CASE(3); NVJ_CASE(4); NVJ_CASE(5); NVJ_CASE(6);
+    NVJ_CASE(7); NVJ_CASE(8); NVJ_CASE(9); NVJ_CASE(10); NVJ_CASE(11); NVJ_CASE(12);
+    default: return hipErrorInvalidValue;
+  }
+#undef NVJ_CASE
+}
+bool residual_gemm_takes(int64_t reduction) {
+  return reduction % 256 == 0 && reduction <= 12 * 256;   // both of the forms below: 8 waves
+}
+
+// h[m] = float(embed[ids[m]]), one wave per row.
+__global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict__ embed,
+                                                         const int32_t* __restrict__ ids,
+                                                         float4* __restrict__ h, int num_tokens,
+                                                         int pieces, int vocab) {
+  const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= num_tokens) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t id = min(max(ids[m], 0), vocab - 1);
+  for (int p = lane; p < pieces; p += 64) {
+    const uint4 v = embed[id * pieces + p];
+    float4* dst = h + ((int64_t)m * pieces + p) * 2;
+    dst[0] = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u),
+                         __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u));
+    dst[1] = make_float4(__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xFFFF0000u),
+                         __uint_as_float(v.w << 16), __uint_as_float(v.w & 0xFFFF0000u));
+  }
+}
+
+// hidden 256, 512, 1024 or 2048; one row per wave for up to 4 rows, else four
+#define NVJ_BY_ROW(LAUNCH)                                     \
+  switch (hidden) {                                            \
+    case 256: return few ? LAUNCH(1, 1) : LAUNCH(1, 4);        \
+    case 512: return few ? LAUNCH(2, 1) : LAUNCH(2, 4);        \
+    case 1024: return few ? LAUNCH(4, 1) : LAUNCH(4, 4);       \
+    default: return few ? LAUNCH(8, 1) : LAUNCH(8, 4);         \
+  }
+template <Epilogue EPI>
+hipError_t launch_norm_gemm(hipStream_t s, const NormGemmArgs& a, int hidden) {
+  const bool few = a.num_tokens <= 4;
+  const dim3 grid((unsigned)(a.outputs / 16)), block(256);
+#define NVJ_LAUNCH(RV, ROWS) nvj::launch(norm_gemm_kernel<RV, ROWS, EPI>, grid, block, s, a)
+  NVJ_BY_ROW(NVJ_LAUNCH)
+#undef NVJ_LAUNCH
+}
+hipError_t launch_norm_gemm_wide(hipStream_t s, const NormGemmArgs& a, int hidden) {
+  const bool few = a.num_tokens <= 4;
+  const dim3 grid((unsigned)((a.outputs + 63) / 64)), block(256);
+#define NVJ_LAUNCH(RV, ROWS) nvj::launch(norm_gemm_wide_kernel<RV, ROWS>, grid, block, s, a)
+  NVJ_BY_ROW(NVJ_LAUNCH)
+#undef NVJ_LAUNCH
+}
+#undef NVJ_BY_ROW
+
+constexpr size_t round256(size_t n) { return (n + 255) / 256 * 256; }
+
+struct StepBuffers {
+  size_t h, qkv, q, o, k_rows, act, bytes;
+};
+StepBuffers step_buffers(const nvj_decoder_model& m, int64_t tokens) {
+  StepBuffers b;
+  size_t at = 0;
+  auto take = [&](size_t bytes_per_token) {
+    const size_t here = at;
+    at += round256((size_t)tokens * bytes_per_token);
+    return here;
+  };
+  b.h = take((size_t)m.hidden * 4);
+  const size_t q_row = (size_t)m.num_heads * m.head_dim * 2;
+  const size_t kv_row = (size_t)m.num_kv_heads * m.head_dim * 2;
+  b.qkv = take(q_row + 2 * kv_row);
+  b.q = take(q_row);
+  b.o = take(q_row);
+  b.k_rows = take(kv_row);   // packed K
+  take(kv_row);              // and V
+  b.act = take((size_t)m.intermediate * 2);
+  b.bytes = at;
+  return b;
+}
+
+int check_model(const nvj_decoder_model* m) {
+  if (!m) return NVJ_ERR_NULL_POINTER;
+  if (m->num_layers <= 0 || m->hidden <= 0 || m->num_heads <= 0 || m->num_kv_heads <= 0 ||
+      m->intermediate <= 0 || m->vocab <= 0 || m->max_position <= 0 || m->block_size <= 0 ||
+      m->num_blocks <= 0 || m->num_heads % m->num_kv_heads != 0)
+    return NVJ_ERR_BAD_SHAPE;
+  // hidden: the row lengths the norm prologue is built for
+  if (m->head_dim != 128 ||
+      (m->hidden != 256 && m->hidden != 512 && m->hidden != 1024 && m->hidden != 2048) ||
+      !residual_gemm_takes((int64_t)m->num_heads * m->head_dim) ||
+      !residual_gemm_takes(m->intermediate))
+    return NVJ_ERR_UNSUPPORTED;
+  return NVJ_OK;
+}
+
+}  // namespace
+
+extern "C" size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
+                                                   int32_t num_tokens) {
+  if (check_model(model) != NVJ_OK || num_tokens <= 0) return 0;
+  return step_buffers(*model, num_tokens).bytes;
+}
+
+extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* model,
+                                       const nvj_decoder_layer* layers,
+                                       const nvj_decoder_batch* batch, void* workspace,
+                                       size_t workspace_bytes) {
+  const int bad = check_model(model);
+  if (bad != NVJ_OK) return bad;
+  if (!batch) return NVJ_ERR_NULL_POINTER;
+  const nvj_decoder_model& m = *model;
+  const nvj_decoder_batch& b = *batch;
+  if (b.num_tokens < 0 || b.num_sequences < 0 || (!b.is_prefill && b.num_tokens != b.num_sequences))
+    return NVJ_ERR_BAD_SHAPE;
+  if (b.num_tokens > kMaxRows || b.num_sequences > kMaxRows) return NVJ_ERR_UNSUPPORTED;
+  if (b.num_tokens == 0) return NVJ_OK;
+  if (!layers || !m.embed || !m.final_norm || !m.cos_sin || !b.input_ids || !b.positions ||
+      !b.slot_mapping || !workspace)
+    return NVJ_ERR_NULL_POINTER;
+  if (b.is_prefill ? (!b.cu_seqlens_q || !b.cu_seqlens_k || (b.logits && !b.last_token_indices))
+                   : !b.context_lens)
+    return NVJ_ERR_NULL_POINTER;
+  const StepBuffers at = step_buffers(m, b.num_tokens);
+  if (workspace_bytes < at.bytes) return NVJ_ERR_WORKSPACE;
+  uintptr_t bits = reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(m.embed) |
+                   reinterpret_cast<uintptr_t>(m.final_norm);
+  for (int i = 0; i < m.num_layers; ++i) {
+    const nvj_decoder_layer& l = layers[i];
+    if (!l.qkv || !l.o || !l.gate_up || !l.down || !l.ln1 || !l.ln2 || !l.k_cache || !l.v_cache)
+      return NVJ_ERR_NULL_POINTER;
+    if ((l.q_norm == nullptr) != (l.k_norm == nullptr)) return NVJ_ERR_NULL_POINTER;
+    for (const void* p : {l.qkv, l.o, l.gate_up, l.down, (const void*)l.ln1, (const void*)l.ln2,
+                          (const void*)l.k_cache, (const void*)l.v_cache})
+      bits |= reinterpret_cast<uintptr_t>(p);
+  }
+  if (bits & 15u) return NVJ_ERR_ALIGNMENT;
+
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  float* h = reinterpret_cast<float*>(ws + at.h);
+  const int tokens = b.num_tokens;
+  const int q_width = m.num_heads * m.head_dim;
+
+  hipError_t rc = nvj::launch(embed_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
+                              static_cast<const uint4*>(m.embed), b.input_ids,
+                              reinterpret_cast<float4*>(h), tokens, m.hidden / 8, m.vocab);
+  if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
+
+  NormGemmArgs a = {};
+  a.h = reinterpret_cast<const float4*>(h);
+  a.eps = m.eps;
+  a.num_tokens = tokens;
+  const bool packed = b.is_prefill && !b.block_tables;
+  char* k_rows = packed ? ws + at.k_rows : nullptr;
+  char* v_rows =
+      packed ? k_rows + round256((size_t)tokens * m.num_kv_heads * m.head_dim * 2) : nullptr;
+
+  for (int i = 0; i < m.num_layers; ++i) {
+    const nvj_decoder_layer& l = layers[i];
+    a.weight = static_cast<const char*>(l.qkv);
+    a.norm_weight = l.ln1;
+    a.outputs = q_width + 2 * m.num_kv_heads * m.head_dim;
+    a.out = reinterpret_cast<uint16_t*>(ws + at.qkv);
+    if (launch_norm_gemm<kPlain>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
+
+    int code = nvj_qk_norm_rope_rows_launch(
+        stream, ws + at.qkv, a.outputs, b.positions, m.cos_sin, m.max_position, l.q_norm, l.k_norm,
+        m.eps, b.slot_mapping, l.k_cache, l.v_cache, ws + at.q, q_width, k_rows, v_rows,
+        m.num_kv_heads * m.head_dim, tokens, m.num_heads, m.num_kv_heads, m.head_dim,
+        (int64_t)m.num_blocks * m.block_size);
+    if (code != NVJ_OK) return code;
+    if (packed)
+      code = nvj_prefill_attention_launch(stream, ws + at.q, k_rows, v_rows,
+                                          b.cu_seqlens_q, b.cu_seqlens_k, ws + at.o, tokens,
+                                          b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
+                                          m.scale, NVJ_DTYPE_BF16);
+    else if (b.is_prefill)
+      code = nvj_paged_prefill_attention_launch(
+          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.cu_seqlens_q, b.cu_seqlens_k,
+          ws + at.o, tokens, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
+          m.block_size, b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16);
+    else if (b.chunk == 0)
+      code = nvj_paged_decode_launch_counters(
+          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, ws + at.o,
+          b.partials, b.partial_bytes, b.counters, b.counter_bytes, b.num_sequences, m.num_heads,
+          m.num_kv_heads, m.head_dim, m.block_size, b.max_blocks, m.num_blocks, m.scale,
+          NVJ_DTYPE_BF16,
+          NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE |
+              (b.clear_counters && i == 0 ? NVJ_PHASE_CLEAR_COUNTERS : 0));
+    else
+      code = nvj_paged_decode_launch_phases(
+          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, ws + at.o,
+          b.partials, b.partial_bytes, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
+          m.block_size, b.max_blocks, m.num_blocks, m.scale, b.chunk, NVJ_DTYPE_BF16,
+          NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE);
+    if (code != NVJ_OK) return code;
+
+    rc = launch_residual_gemm<4, 1, 2>(s, ws + at.o, l.o, h, tokens, m.hidden, q_width);
+    if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
+    a.weight = static_cast<const char*>(l.gate_up);
+    a.norm_weight = l.ln2;
+    a.outputs = 2 * m.intermediate;
+    a.out = reinterpret_cast<uint16_t*>(ws + at.act);
+    if (launch_norm_gemm<kSiluMul>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
+    rc = launch_residual_gemm<2, 4, 4>(s, ws + at.act, l.down, h, tokens, m.hidden, m.intermediate);
+    if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
+  }
+  if (!b.logits) return NVJ_OK;
+  a.weight = static_cast<const char*>(m.embed);
+  a.norm_weight = m.final_norm;
+  a.outputs = m.vocab;
+  a.out = static_cast<uint16_t*>(b.logits);
+  a.row_index = b.is_prefill ? b.last_token_indices : nullptr;
+  a.num_tokens = b.num_sequences;
+  if (a.num_tokens == 0) return NVJ_OK;
+  return launch_norm_gemm_wide(s, a, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+}

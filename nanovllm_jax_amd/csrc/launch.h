@@ -16,10 +16,17 @@ namespace nvj {
 // Arguments are converted to the kernel's parameter types (the parameter pack
 // is deduced from the kernel alone) and handed over by address.
 template <typename... Params>
+inline hipError_t launch_lds(void (*kernel)(Params...), dim3 grid, dim3 block, size_t lds_bytes,
+                             hipStream_t stream, typename std::common_type<Params>::type... args) {
+  void* ptrs[] = {static_cast<void*>(&args)..., nullptr};
+  return hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, lds_bytes,
+                         stream);
+}
+// without dynamic LDS
+template <typename... Params>
 inline hipError_t launch(void (*kernel)(Params...), dim3 grid, dim3 block, hipStream_t stream,
                          typename std::common_type<Params>::type... args) {
-  void* ptrs[] = {static_cast<void*>(&args)..., nullptr};
-  return hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, 0, stream);
+  return launch_lds<Params...>(kernel, grid, block, 0, stream, args...);
 }
 
 }  // namespace nvj

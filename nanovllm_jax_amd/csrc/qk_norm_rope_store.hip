@@ -9,11 +9,15 @@
 // It reads the packed QKV projection output once and writes q (bf16) plus the
 // K and V cache rows; nothing else touches HBM.
 //
-// One wave64 per (token, head).  Lane l holds elements l and l + 64 of the
-// 128-wide head, which is exactly one rotary pair, so the rotation needs no
-// cross-lane traffic; the mean of squares is a 6-step xor butterfly.  The
-// arithmetic is a fixed sequence of IEEE fp32 operations (no contraction, no
-// approximate rsqrt) so that a CPU restatement reproduces it bit for bit:
+// Bytes in and out are what bounds it with many rows, the chain of dependent loads
+// (slot, position, its table row) with few.  16 lanes per (token, head), four heads
+// per wave: lane i holds elements 4i .. 4i+3 and 64+4i .. 64+4i+3, whole rotary
+// pairs in 8-byte loads, so the rotation needs no cross-lane traffic.  (One wave per
+// head, 2-byte loads, took 42.6 us for 4400 rows of 32 heads.)  With l the element
+// of the lower half, the mean of squares is the same xor butterfly over l whatever
+// lanes hold it.  The arithmetic is a fixed sequence of IEEE fp32 operations (no
+// contraction, no approximate rsqrt) so that a CPU restatement reproduces it bit for
+// bit:
 //   s_l   = fma(x2, x2, x1 * x1)            (fp32 values of the bf16 inputs)
 //   s_l  += s_(l ^ m)  for m = 32, 16, 8, 4, 2, 1
 //   r     = 1 / sqrt(s / 128 + eps)
@@ -29,7 +33,6 @@
 namespace {
 
 constexpr int kHeadDim = 128;
-constexpr int kHalf = 64;
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
@@ -39,68 +42,189 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
   return (uint16_t)((u + (((u >> 16) & 1u) + 0x7FFFu)) >> 16);
 }
 
-// grid.x = ceil(num_tokens * heads_total / 4), block = 256 (4 waves).
-__global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
-    const uint16_t* __restrict__ qkv, int64_t qkv_row_stride,   // [T, >= (Hq+2Hkv)*128] bf16
-    const int32_t* __restrict__ positions,                       // [T]
-    const float* __restrict__ cos_sin, int max_position,         // [max_position, 128]: cos | sin
-    const float* __restrict__ q_weight, const float* __restrict__ k_weight,  // [128] or null
-    float eps, const int32_t* __restrict__ slot_mapping,         // [T]
-    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,          // [num_slots, Hkv, 128]
-    uint16_t* __restrict__ q_out,                                 // [T, Hq, 128]
-    int num_tokens, int num_heads, int num_kv_heads, int64_t num_slots) {
+struct QkArgs {
+  const uint16_t* qkv;        // [T, >= (Hq+2Hkv)*128] bf16
+  int64_t qkv_row_stride;
+  const int32_t* positions;   // [T]
+  const float* cos_sin;       // [max_position, 128]: cos | sin
+  const float* q_weight;      // [128] or null
+  const float* k_weight;
+  const int32_t* slot_mapping;   // [T]
+  uint16_t* k_cache;          // [num_slots, Hkv, 128]
+  uint16_t* v_cache;
+  uint16_t* q_out;            // [T, >= Hq*128]; may be qkv itself
+  int64_t q_row_stride;
+  uint16_t* k_out;            // [T, >= Hkv*128] the new rows besides the cache, or null; may lie in qkv
+  uint16_t* v_out;
+  int64_t kv_row_stride;
+  float eps;
+  int max_position, num_tokens, num_heads, num_kv_heads;
+  int64_t num_slots;
+};
+
+// sum of the four elements' squares over the 64 elements of the lower half, in the
+// order of a butterfly over l = 4 * lane + e: masks 32 .. 4 are lanes 8 .. 1 apart,
+// masks 2 and 1 elements of a lane
+__device__ __forceinline__ float butterfly(float (&s)[4]) {
+#pragma unroll
+  for (int m = 8; m >= 1; m >>= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], m, 64);
+  return (s[0] + s[2]) + (s[1] + s[3]);
+}
+
+__device__ __forceinline__ void unpack4(uint2 p, float (&f)[4]) {
+  f[0] = __uint_as_float(p.x << 16); f[1] = __uint_as_float(p.x & 0xFFFF0000u);
+  f[2] = __uint_as_float(p.y << 16); f[3] = __uint_as_float(p.y & 0xFFFF0000u);
+}
+__device__ __forceinline__ uint2 pack4(const float (&f)[4]) {
+  return make_uint2(f32_to_bf16_rne(f[0]) | ((uint32_t)f32_to_bf16_rne(f[1]) << 16),
+                    f32_to_bf16_rne(f[2]) | ((uint32_t)f32_to_bf16_rne(f[3]) << 16));
+}
+
+// WIDE: everything is aligned for 8- and 16-byte accesses; otherwise element by
+// element (rows at odd offsets inside a larger buffer).
+template <bool WIDE>
+__device__ __forceinline__ uint2 load4(const uint16_t* p) {
+  if (WIDE) return *reinterpret_cast<const uint2*>(p);
+  return make_uint2(p[0] | ((uint32_t)p[1] << 16), p[2] | ((uint32_t)p[3] << 16));
+}
+template <bool WIDE>
+__device__ __forceinline__ float4 load4(const float* p) {
+  if (WIDE) return *reinterpret_cast<const float4*>(p);
+  return make_float4(p[0], p[1], p[2], p[3]);
+}
+template <bool WIDE>
+__device__ __forceinline__ void store4(uint16_t* p, uint2 v) {
+  if (WIDE) {
+    *reinterpret_cast<uint2*>(p) = v;
+  } else {
+    p[0] = (uint16_t)v.x; p[1] = (uint16_t)(v.x >> 16);
+    p[2] = (uint16_t)v.y; p[3] = (uint16_t)(v.y >> 16);
+  }
+}
+
+// grid.x = ceil(num_tokens * heads_total / 16), block = 256: 16 groups of 16 lanes.
+// Every load that depends on nothing but the (token, head) is issued together.
+template <bool WIDE>
+__global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(QkArgs a) {
 #pragma clang fp contract(off)
-  const int heads_total = num_heads + 2 * num_kv_heads;
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (unit >= (int64_t)num_tokens * heads_total) return;
+  const int heads_total = a.num_heads + 2 * a.num_kv_heads;
+  const int64_t unit = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (unit >= (int64_t)a.num_tokens * heads_total) return;
   const int token = (int)(unit / heads_total);
   const int head = (int)(unit - (int64_t)token * heads_total);
-  const int lane = threadIdx.x & 63;
-  const uint16_t* src = qkv + (int64_t)token * qkv_row_stride + (int64_t)head * kHeadDim;
-
-  const bool is_q = head < num_heads;
-  const bool is_k = !is_q && head < num_heads + num_kv_heads;
-  int64_t slot = 0;
-  if (!is_q) {
-    slot = slot_mapping[token];
-    if (slot < 0 || slot >= num_slots) return;   // skipped / dropped token
+  const int i = threadIdx.x & 15;
+  const uint16_t* src = a.qkv + (int64_t)token * a.qkv_row_stride + (int64_t)head * kHeadDim + 4 * i;
+  uint2 lo = load4<WIDE>(src), hi = load4<WIDE>(src + 64);
+  const int pos = min(max(a.positions[token], 0), a.max_position - 1);
+  const int64_t slot = a.slot_mapping[token];
+  const bool is_q = head < a.num_heads;
+  const bool is_k = !is_q && head < a.num_heads + a.num_kv_heads;
+  if (is_q || is_k) {
+    const float* cs = a.cos_sin + (int64_t)pos * kHeadDim + 4 * i;
+    const float4 c4 = load4<WIDE>(cs), s4 = load4<WIDE>(cs + 64);
+    const float* w = is_q ? a.q_weight : a.k_weight;
+    float x1[4], x2[4];
+    unpack4(lo, x1);
+    unpack4(hi, x2);
+    if (w != nullptr) {
+      const float4 wl = load4<WIDE>(w + 4 * i), wh = load4<WIDE>(w + 64 + 4 * i);
+      const float w1[4] = {wl.x, wl.y, wl.z, wl.w}, w2[4] = {wh.x, wh.y, wh.z, wh.w};
+      float s[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(x2[e], x2[e], x1[e] * x1[e]);
+      const float r = 1.0f / __builtin_sqrtf(butterfly(s) * (1.0f / kHeadDim) + a.eps);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x1[e] = bf16_to_f32(f32_to_bf16_rne(x1[e] * r * w1[e]));
+        x2[e] = bf16_to_f32(f32_to_bf16_rne(x2[e] * r * w2[e]));
+      }
+    }
+    const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
+    float y1[4], y2[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y1[e] = x1[e] * c[e] - x2[e] * sn[e];
+      y2[e] = x2[e] * c[e] + x1[e] * sn[e];
+    }
+    lo = pack4(y1);
+    hi = pack4(y2);
   }
-  if (!is_q && !is_k) {   // V: plain row copy into the cache
-    const int kvh = head - num_heads - num_kv_heads;
-    const uint32_t* s32 = reinterpret_cast<const uint32_t*>(src);
-    uint32_t* d32 = reinterpret_cast<uint32_t*>(v_cache + (slot * num_kv_heads + kvh) * kHeadDim);
-    d32[lane] = s32[lane];
+  auto put = [&](uint16_t* row) {
+    store4<WIDE>(row + 4 * i, lo);
+    store4<WIDE>(row + 64 + 4 * i, hi);
+  };
+  if (is_q) {
+    put(a.q_out + (int64_t)token * a.q_row_stride + (int64_t)head * kHeadDim);
     return;
   }
-
-  float x1 = bf16_to_f32(src[lane]);
-  float x2 = bf16_to_f32(src[lane + kHalf]);
-  const float* w = is_q ? q_weight : k_weight;
-  if (w != nullptr) {
-    float s = __builtin_fmaf(x2, x2, x1 * x1);
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-    const float r = 1.0f / __builtin_sqrtf(s * (1.0f / kHeadDim) + eps);
-    x1 = bf16_to_f32(f32_to_bf16_rne(x1 * r * w[lane]));
-    x2 = bf16_to_f32(f32_to_bf16_rne(x2 * r * w[lane + kHalf]));
-  }
-  int pos = positions[token];
-  pos = min(max(pos, 0), max_position - 1);
-  const float c = cos_sin[(int64_t)pos * kHeadDim + lane];
-  const float sn = cos_sin[(int64_t)pos * kHeadDim + kHalf + lane];
-  const float y1 = x1 * c - x2 * sn;
-  const float y2 = x2 * c + x1 * sn;
-  uint16_t* dst;
-  if (is_q) {
-    dst = q_out + ((int64_t)token * num_heads + head) * kHeadDim;
-  } else {
-    dst = k_cache + (slot * num_kv_heads + (head - num_heads)) * kHeadDim;
-  }
-  dst[lane] = f32_to_bf16_rne(y1);
-  dst[lane + kHalf] = f32_to_bf16_rne(y2);
+  const int kvh = head - a.num_heads - (is_k ? 0 : a.num_kv_heads);
+  uint16_t* rows = is_k ? a.k_out : a.v_out;
+  if (rows != nullptr) put(rows + (int64_t)token * a.kv_row_stride + (int64_t)kvh * kHeadDim);
+  if (slot >= 0 && slot < a.num_slots)   // else: skipped / dropped token
+    put((is_k ? a.k_cache : a.v_cache) + (slot * a.num_kv_heads + kvh) * kHeadDim);
 }
 
 }  // namespace
+
+extern "C" int nvj_qk_norm_rope_rows_launch(
+    void* stream, const void* qkv, int64_t qkv_row_stride, const int32_t* positions,
+    const float* cos_sin_cache, int32_t max_position, const float* q_norm_weight,
+    const float* k_norm_weight, float eps, const int32_t* slot_mapping, void* k_cache,
+    void* v_cache, void* q_out, int64_t q_row_stride, void* k_out, void* v_out,
+    int64_t kv_row_stride, int32_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_dim, int64_t num_slots) {
+  if (num_tokens < 0 || num_heads <= 0 || num_kv_heads <= 0 || max_position <= 0 || num_slots < 0)
+    return NVJ_ERR_BAD_SHAPE;
+  if (head_dim != kHeadDim) return NVJ_ERR_UNSUPPORTED;
+  const int64_t heads_total = (int64_t)num_heads + 2 * (int64_t)num_kv_heads;
+  if (qkv_row_stride < heads_total * kHeadDim || (qkv_row_stride & 1) ||
+      q_row_stride < (int64_t)num_heads * kHeadDim ||
+      ((k_out || v_out) && kv_row_stride < (int64_t)num_kv_heads * kHeadDim))
+    return NVJ_ERR_BAD_SHAPE;
+  if (num_tokens == 0) return NVJ_OK;
+  if (!qkv || !positions || !cos_sin_cache || !slot_mapping || !k_cache || !v_cache || !q_out)
+    return NVJ_ERR_NULL_POINTER;
+  if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return NVJ_ERR_NULL_POINTER;
+  const uintptr_t rows = reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(k_cache) |
+                         reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(q_out) |
+                         reinterpret_cast<uintptr_t>(k_out) | reinterpret_cast<uintptr_t>(v_out);
+  const int64_t strides = qkv_row_stride | q_row_stride | ((k_out || v_out) ? kv_row_stride : 0);
+  if ((rows & 3u) || (strides & 1)) return NVJ_ERR_ALIGNMENT;
+  const uintptr_t tables = reinterpret_cast<uintptr_t>(cos_sin_cache) |
+                           reinterpret_cast<uintptr_t>(q_norm_weight) |
+                           reinterpret_cast<uintptr_t>(k_norm_weight);
+  const bool wide = (rows & 7u) == 0 && (strides & 3) == 0 && (tables & 15u) == 0;
+  const int64_t units = (int64_t)num_tokens * heads_total;
+  const int64_t blocks = (units + 15) / 16;
+  if (blocks > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
+  QkArgs a;
+  a.qkv = static_cast<const uint16_t*>(qkv);
+  a.qkv_row_stride = qkv_row_stride;
+  a.positions = positions;
+  a.cos_sin = cos_sin_cache;
+  a.q_weight = q_norm_weight;
+  a.k_weight = k_norm_weight;
+  a.slot_mapping = slot_mapping;
+  a.k_cache = static_cast<uint16_t*>(k_cache);
+  a.v_cache = static_cast<uint16_t*>(v_cache);
+  a.q_out = static_cast<uint16_t*>(q_out);
+  a.q_row_stride = q_row_stride;
+  a.k_out = static_cast<uint16_t*>(k_out);
+  a.v_out = static_cast<uint16_t*>(v_out);
+  a.kv_row_stride = kv_row_stride;
+  a.eps = eps;
+  a.max_position = max_position;
+  a.num_tokens = num_tokens;
+  a.num_heads = num_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.num_slots = num_slots;
+  const auto kernel = wide ? qk_norm_rope_store_kernel<true> : qk_norm_rope_store_kernel<false>;
+  const hipError_t rc = nvj::launch(kernel, dim3((unsigned)blocks), dim3(256),
+                                    static_cast<hipStream_t>(stream), a);
+  return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+}
 
 extern "C" int nvj_qk_norm_rope_store_launch(void* stream, const void* qkv, int64_t qkv_row_stride,
                                              const int32_t* positions, const float* cos_sin_cache,
@@ -110,26 +234,9 @@ extern "C" int nvj_qk_norm_rope_store_launch(void* stream, const void* qkv, int6
                                              void* v_cache, void* q_out, int32_t num_tokens,
                                              int32_t num_heads, int32_t num_kv_heads,
                                              int32_t head_dim, int64_t num_slots) {
-  if (num_tokens < 0 || num_heads <= 0 || num_kv_heads <= 0 || max_position <= 0 || num_slots < 0)
-    return NVJ_ERR_BAD_SHAPE;
-  if (head_dim != kHeadDim) return NVJ_ERR_UNSUPPORTED;
-  const int64_t heads_total = (int64_t)num_heads + 2 * (int64_t)num_kv_heads;
-  if (qkv_row_stride < heads_total * kHeadDim || (qkv_row_stride & 1)) return NVJ_ERR_BAD_SHAPE;
-  if (num_tokens == 0) return NVJ_OK;
-  if (!qkv || !positions || !cos_sin_cache || !slot_mapping || !k_cache || !v_cache || !q_out)
-    return NVJ_ERR_NULL_POINTER;
-  if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return NVJ_ERR_NULL_POINTER;
-  if ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(k_cache) |
-       reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(q_out)) & 3u)
-    return NVJ_ERR_ALIGNMENT;
-  const int64_t units = (int64_t)num_tokens * heads_total;
-  const int64_t blocks = (units + 3) / 4;
-  if (blocks > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const hipError_t rc = nvj::launch(
-      qk_norm_rope_store_kernel, dim3((unsigned)blocks), dim3(256),
-      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(qkv), qkv_row_stride, positions, cos_sin_cache, max_position,
-      q_norm_weight, k_norm_weight, eps, slot_mapping, static_cast<uint16_t*>(k_cache),
-      static_cast<uint16_t*>(v_cache), static_cast<uint16_t*>(q_out), num_tokens, num_heads,
-      num_kv_heads, num_slots);
-  return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+  return nvj_qk_norm_rope_rows_launch(stream, qkv, qkv_row_stride, positions, cos_sin_cache,
+                                      max_position, q_norm_weight, k_norm_weight, eps, slot_mapping,
+                                      k_cache, v_cache, q_out, (int64_t)num_heads * kHeadDim,
+                                      nullptr, nullptr, 0, num_tokens, num_heads, num_kv_heads,
+                                      head_dim, num_slots);
 }

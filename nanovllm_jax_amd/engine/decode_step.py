@@ -20,6 +20,7 @@ temperature -> 0 limit of the reference's Gumbel-max sampler
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import numpy as np
@@ -36,6 +37,11 @@ from ..layers.prefill_attention import (paged_prefill_attention,
                                         variable_length_attention_prefill)
 from ..layers.qk_rope_store import qk_norm_rope_store
 from ..utils.context import AttentionContext, create_decode_context, create_prefill_context
+
+# Up to this many token rows a step runs as the native chain of fused launches
+# (nvj_decoder_step_launch), beyond it as library GEMMs with the element-wise
+# launches between them.
+_NATIVE_STEP_ROWS = 16
 
 __all__ = ["DecodeModelConfig", "DecodeStepRunner", "prepare_block_tables", "prepare_decode",
            "prepare_prefill", "advance_decode"]
@@ -208,6 +214,7 @@ class DecodeStepRunner:
             a.set_kv_cache(self.kv_cache[0, layer], self.kv_cache[1, layer])
             self.attn.append(a)
         self._graph = None
+        self._native_model = None       # (pointers it was built from, model, layers)
         self._eager_ws = None
         self._eager_ws_shapes = set()
 
@@ -238,7 +245,114 @@ class DecodeStepRunner:
         x1, x2 = x.chunk(2, dim=-1)
         return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], dim=-1)
 
+    _LAYER_WEIGHTS = ("qkv", "o", "gate_up", "down", "ln1", "ln2", "q_norm", "k_norm")
+
+    def _native(self):
+        """The model as the native step wants it: ``(model, layers)``, or None when it
+        is not one that step is built for.  Rebuilt when a weight or cache tensor has
+        been replaced; the look at the addresses is all an unchanged model costs."""
+        tensors = [self.embed, self.final_norm, self.cos_sin]
+        for lw, a in zip(self.layers, self.attn):
+            tensors += [lw[n] for n in self._LAYER_WEIGHTS]
+            tensors += [a.k_cache, a.v_cache]
+        key = [t.data_ptr() for t in tensors]
+        key.append(self.attn[0].scale)
+        if self._native_model is not None and self._native_model[0] == key:
+            return self._native_model[1]
+        c, a0 = self.cfg, self.attn[0]
+        f32 = {id(t) for lw in self.layers for t in (lw["ln1"], lw["ln2"], lw["q_norm"],
+                                                     lw["k_norm"])}
+        f32 |= {id(self.final_norm), id(self.cos_sin)}
+        ok = all(t.is_cuda and t.is_contiguous() and
+                 t.dtype == (torch.float32 if id(t) in f32 else torch.bfloat16) for t in tensors)
+        ok = ok and all(a.scale == a0.scale and a.block_size == c.block_size and
+                        a.k_cache.shape == a0.k_cache.shape == a.v_cache.shape and
+                        a.k_cache.dim() == 4 for a in self.attn)
+        built = None
+        if ok:
+            model = _lib.DecoderModel(
+                self.embed.data_ptr(), self.final_norm.data_ptr(), self.cos_sin.data_ptr(),
+                c.num_layers, c.hidden_size, c.num_heads, c.num_kv_heads, c.head_dim,
+                c.intermediate_size, self.embed.shape[0], self.cos_sin.shape[0], c.block_size,
+                a0.k_cache.shape[0], c.rms_norm_eps, a0.scale)
+            per = len(self._LAYER_WEIGHTS) + 2
+            layers = (_lib.DecoderLayer * c.num_layers)(
+                *[_lib.DecoderLayer(*key[3 + per * i:3 + per * (i + 1)])
+                  for i in range(c.num_layers)])
+            if _lib.load().nvj_decoder_step_workspace_bytes(ctypes.byref(model), 1) > 0:
+                built = (model, layers)
+        self._native_model = (key, built)
+        return built
+
+    def _native_forward(self, input_ids, positions, context: AttentionContext):
+        """The whole step as one native call, or None when it has to go the long way."""
+        tokens = input_ids.shape[0]
+        sl, bt = context.slot_mapping, context.block_tables
+        prefill = bool(context.is_prefill)
+        ints = [input_ids, positions, sl]
+        ints += [context.cu_seqlens_q, context.cu_seqlens_k] if prefill else [context.context_lens]
+        ws0 = self.attn[0].workspace
+        if not (0 < tokens <= _NATIVE_STEP_ROWS and self.fused_qk_rope_store
+                and self.fused_layer_glue and (prefill or bt is not None)
+                and (ws0 is None or isinstance(ws0, DecodeWorkspace))
+                and all(a.workspace is ws0 for a in self.attn)):
+            return None
+        if bt is not None:
+            ints.append(bt)
+        for t in ints:
+            if t is None or t.dtype != torch.int32 or not t.is_cuda or not t.is_contiguous() \
+                    or t.device != self.embed.device:
+                return None
+        sequences = context.cu_seqlens_q.shape[0] - 1 if prefill else tokens
+        if positions.shape != (tokens,) or sl.shape != (tokens,) or input_ids.dim() != 1 or \
+                (bt is not None and (bt.dim() != 2 or bt.shape[0] != sequences
+                                     or bt.shape[1] == 0)):
+            return None
+        if prefill:
+            if context.cu_seqlens_k.shape[0] != sequences + 1 or \
+                    not 0 < sequences <= _NATIVE_STEP_ROWS:
+                return None
+        elif context.context_lens.shape != (tokens,):
+            return None
+        built = self._native()
+        if built is None:
+            return None
+        model, layers = built
+        b = _lib.DecoderBatch(num_tokens=tokens, num_sequences=sequences, is_prefill=int(prefill))
+        b.input_ids, b.positions, b.slot_mapping = (input_ids.data_ptr(), positions.data_ptr(),
+                                                    sl.data_ptr())
+        if bt is not None:
+            b.block_tables, b.max_blocks = bt.data_ptr(), bt.shape[1]
+        if prefill:
+            b.cu_seqlens_q, b.cu_seqlens_k = (context.cu_seqlens_q.data_ptr(),
+                                              context.cu_seqlens_k.data_ptr())
+            last = context.last_token_indices.to(torch.int32).contiguous()
+            b.last_token_indices = last.data_ptr()
+        else:
+            ws = ws0 or self._eager_workspace(context)
+            b.context_lens, b.chunk = context.context_lens.data_ptr(), int(context.decode_split)
+            b.partials, b.partial_bytes = ws.buffer.data_ptr(), ws.buffer.numel()
+            if b.chunk == 0:
+                counters = ws._counters_for(4 * (1 + sequences * self.cfg.num_heads))
+                b.counters, b.counter_bytes = counters.data_ptr(), counters.numel() * 4
+                b.clear_counters, ws._clear_next = int(ws._clear_next), False
+        dev = input_ids.device
+        logits = torch.empty((sequences, model.vocab), dtype=torch.bfloat16, device=dev)
+        b.logits = logits.data_ptr()
+        lib = _lib.load()
+        need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens)
+        scratch = torch.empty(need, dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            code = lib.nvj_decoder_step_launch(
+                torch.cuda.current_stream(dev).cuda_stream, ctypes.byref(model), layers,
+                ctypes.byref(b), scratch.data_ptr(), need)
+        _lib.check(code, "nvj_decoder_step_launch")
+        return logits
+
     def forward(self, input_ids, positions, context: AttentionContext):
+        logits = self._native_forward(input_ids, positions, context)
+        if logits is not None:
+            return logits
         c = self.cfg
         h = F.embedding(input_ids.long(), self.embed)
         residual = None
@@ -304,11 +418,28 @@ class DecodeStepRunner:
     def make_inputs(self, last_tokens, seq_lens, block_tables):
         ids, pos, ctx, slots, bt = prepare_decode(last_tokens, seq_lens, block_tables,
                                                   self.cfg.block_size)
-        d = self.device
-        t = lambda a: torch.from_numpy(a).to(d)
         # the lengths are host integers here, as in the reference's filler: pick the split
         split = choose_split(ctx, self.cfg.num_kv_heads, self.cfg.num_heads)
-        return t(ids), t(pos), create_decode_context(t(ctx), t(slots), t(bt), split)
+        d_ids, d_pos, d_ctx, d_slots, d_bt = self._upload(ids, pos, ctx, slots, bt)
+        return d_ids, d_pos, create_decode_context(d_ctx, d_slots, d_bt, split)
+
+    def _upload(self, *arrays):
+        """int32 host arrays as device tensors, in one copy that nobody waits for: they
+        are laid out behind each other in a pinned block (which torch's host allocator
+        hands out again only when the copy is done) and come back as views of one
+        device block.  A copy from pageable memory, one per array, would wait each time
+        for everything in front of it on the stream."""
+        at, total = [], 0
+        for a in arrays:
+            at.append(total)
+            total += -(-a.size // 64) * 64          # 256-byte pieces
+        host = torch.empty(max(total, 1), dtype=torch.int32, pin_memory=True)
+        flat = host.numpy()
+        for a, o in zip(arrays, at):
+            flat[o:o + a.size] = a.reshape(-1)
+        block = torch.empty(max(total, 1), dtype=torch.int32, device=self.device)
+        block.copy_(host, non_blocking=True)
+        return [block[o:o + a.size].view(a.shape) for a, o in zip(arrays, at)]
 
     def make_prefill_inputs(self, token_lists, block_tables, num_cached_tokens=None):
         """Prefill inputs; with ``num_cached_tokens`` the context carries the block
@@ -317,11 +448,11 @@ class DecodeStepRunner:
         from the paged cache."""
         ids, pos, cu_q, cu_k, slots, max_q, max_k = prepare_prefill(
             token_lists, block_tables, self.cfg.block_size, num_cached_tokens)
-        d = self.device
-        t = lambda a: torch.from_numpy(a).to(d)
-        bt = t(prepare_block_tables(block_tables)) if num_cached_tokens is not None else None
-        return t(ids), t(pos), create_prefill_context(t(cu_q), t(cu_k), max_q, max_k, t(slots),
-                                                      block_tables=bt)
+        tables = ([prepare_block_tables(block_tables)] if num_cached_tokens is not None else [])
+        d_ids, d_pos, d_cu_q, d_cu_k, d_slots, *bt = self._upload(ids, pos, cu_q, cu_k, slots,
+                                                                  *tables)
+        return d_ids, d_pos, create_prefill_context(d_cu_q, d_cu_k, max_q, max_k, d_slots,
+                                                    block_tables=bt[0] if bt else None)
 
     def step(self, input_ids, positions, context):
         """Eager decode step: logits -> greedy token ids [batch] int64."""

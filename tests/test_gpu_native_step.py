@@ -1,0 +1,99 @@
+"""The native step (six fused launches per layer) against the same step through library
+GEMMs and separate launches, at the edges of its row counts and row lengths; and the QK
+norm / RoPE launch with rows in place, strided and at odd offsets."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import bits_to_torch, torch_to_bits
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,hidden,inter,heads", [(1, 256, 256, 2), (4, 512, 768, 4),
+                                                     (5, 1024, 3072, 16), (16, 1024, 512, 8),
+                                                     (16, 2048, 2560, 24)])
+@pytest.mark.parametrize("kind", ["decode", "packed", "paged"])
+def test_native_step_equals_the_long_way(rows, hidden, inter, heads, kind, monkeypatch):
+    print(f"case native step rows={rows} hidden={hidden} {kind}", flush=True)
+    from nanovllm_jax_amd.engine import decode_step as ds
+    cfg = ds.DecodeModelConfig(num_layers=2, hidden_size=hidden, num_heads=heads, num_kv_heads=2,
+                               head_dim=128, intermediate_size=inter, vocab_size=1000,
+                               max_position=1024, block_size=64, num_kvcache_blocks=80)
+    runner = ds.DecodeStepRunner(cfg, "cuda:0", seed=rows)
+    rng = np.random.Generator(np.random.PCG64(rows))
+    pages = rng.permutation(cfg.num_kvcache_blocks).tolist()
+    if kind == "decode":
+        lens = rng.integers(1, 250, rows).tolist()
+    else:                                     # new rows: one long prompt and short ones
+        lens = [rows] if rows < 5 else [rows - 3, 2, 1]
+    cached = [37] * len(lens) if kind == "paged" else [0] * len(lens)
+    tables = []
+    for n, c in zip(lens, cached):
+        tables.append([pages.pop() for _ in range(-(-(n + c) // cfg.block_size))])
+    if kind == "decode":
+        inputs = runner.make_inputs(rng.integers(0, 1000, rows).tolist(), lens, tables)
+    else:
+        toks = [rng.integers(0, 1000, n + c).tolist() for n, c in zip(lens, cached)]
+        inputs = runner.make_prefill_inputs(toks, tables, cached if kind == "paged" else None)
+    before = runner.kv_cache.clone()
+    assert runner._native_forward(*inputs) is not None       # the path under test is taken
+    runner.kv_cache.copy_(before)
+    got = runner.forward(*inputs).float()
+    kv = runner.kv_cache.clone()
+    runner.kv_cache.copy_(before)
+    monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+    want = runner.forward(*inputs).float()
+    torch.cuda.synchronize()
+    assert (got - want).abs().max().item() <= 0.02 * want.abs().max().item() + 0.02
+    err = (kv.float() - runner.kv_cache.float()).abs()
+    assert (err <= 0.03 + 0.03 * runner.kv_cache.float().abs()).all()
+
+
+@pytest.mark.parametrize("offset,pad", [(0, 0), (2, 6), (4, 4)])
+def test_qk_rows_in_place_and_unaligned(offset, pad):
+    print(f"case qk rows offset={offset} pad={pad}", flush=True)
+    from nanovllm_jax_amd import _lib
+    from oracle.paged_attention_oracle import qk_norm_rope_store_ref
+    T, hq, hkv, d = 7, 3, 2, 128
+    rng = np.random.Generator(np.random.PCG64(offset + 1))
+    width = (hq + 2 * hkv) * d
+    dev = "cuda:0"
+    buf = torch.randn(T, offset + width + pad, device=dev).to(torch.bfloat16)
+    view = buf[:, offset:offset + width]
+    pos = rng.integers(0, 60, T).astype(np.int32)
+    slots = np.array([5, -1, 9, 0, 64, 3, 2], np.int32)
+    cs = rng.standard_normal((60, d), dtype=np.float32)
+    qw, kw = (rng.standard_normal(d, dtype=np.float32) for _ in range(2))
+    kc = torch.zeros(16, hkv, d, dtype=torch.bfloat16, device=dev)
+    vc = torch.zeros_like(kc)
+    all_slots = np.arange(T, dtype=np.int32)               # every row stored: the packed rows
+    qkv_bits = torch_to_bits(view.contiguous())
+    zero = np.zeros((16, hkv, d), np.uint16)
+    want_q, want_k, want_v = qk_norm_rope_store_ref(qkv_bits, pos, cs, qw, kw, 1e-6, zero, zero,
+                                                    all_slots, hq, hkv)
+    up = lambda a: torch.from_numpy(a).to(dev)
+    t = [up(a) for a in (pos, cs, qw, kw, slots)]
+    v_rows = torch.zeros(T, hkv * d, dtype=torch.bfloat16, device=dev)
+    lib = _lib.load()
+    k_part = view.data_ptr() + 2 * hq * d
+    # (kv_row_stride is shared by k_out and v_out: V comes out in a second, cache-less call)
+    for k_out, v_out, stride in ((None, v_rows.data_ptr(), hkv * d),
+                                 (k_part, None, buf.stride(0))):
+        _lib.check(lib.nvj_qk_norm_rope_rows_launch(
+            torch.cuda.current_stream().cuda_stream, view.data_ptr(), buf.stride(0), t[0].data_ptr(),
+            t[1].data_ptr(), 60, t[2].data_ptr(), t[3].data_ptr(), 1e-6, t[4].data_ptr(),
+            kc.data_ptr(), vc.data_ptr(),
+            view.data_ptr() if k_out else torch.empty(T * hq * d, dtype=torch.bfloat16,
+                                                      device=dev).data_ptr(),
+            buf.stride(0) if k_out else hq * d, k_out, v_out, stride, T, hq, hkv, d, 16), "rows")
+    torch.cuda.synchronize()
+    got = torch_to_bits(view.contiguous()).reshape(T, hq + 2 * hkv, d)
+    assert np.array_equal(got[:, :hq], want_q.reshape(T, hq, d))
+    assert np.array_equal(got[:, hq:hq + hkv], want_k[:T])
+    assert np.array_equal(got[:, hq + hkv:], qkv_bits.reshape(T, -1, d)[:, hq + hkv:])
+    assert np.array_equal(torch_to_bits(v_rows).reshape(T, hkv, d), want_v[:T])
+    for i, s in enumerate(slots):
+        if 0 <= s < 16:
+            assert np.array_equal(torch_to_bits(kc)[s], want_k[i])
+            assert np.array_equal(torch_to_bits(vc)[s], want_v[i])
