@@ -452,6 +452,17 @@ NVJ_API int nvj_prefill_attention_launch(void* stream, const void* q, const void
                             int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype);
 
 /*
+ * The same with rows at a distance of their own (in elements, multiples of 8): q rows
+ * of q_row_stride, K and V rows of kv_row_stride (at most 2^22), so that all three may
+ * be parts of one projection buffer.  out is packed.
+ */
+NVJ_API int nvj_prefill_attention_rows_launch(void* stream, const void* q, int64_t q_row_stride,
+                            const void* k, const void* v, int64_t kv_row_stride,
+                            const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, void* out,
+                            int32_t total_q_tokens, int32_t batch, int32_t num_heads,
+                            int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype);
+
+/*
  * The same attention with keys and values read from the block-paged cache:
  * prompt rows behind a cached prefix (prefix caching, chunked prefill).  The
  * reference prepares exactly this call - cu_seqlens_k > cu_seqlens_q and

@@ -9,9 +9,14 @@
 // sequence, :232-243).  GQA maps query head h to kv head h / G.  Nothing is
 // padded and nothing of size max_len^2 is materialised.
 //
-// MFMA-bound.  One workgroup = 4 waves = 128 query rows of one (sequence, query
-// head); a wave owns 32 rows as two groups of 16 MFMA columns.  Keys are walked
-// 32 at a time.  The K rows and the V rows of a tile go from global memory
+// MFMA-bound.  One workgroup = 4 waves = 8 column groups of one (sequence, kv head),
+// a column group being 16 consecutive tokens of one query head (16 MFMA columns);
+// the groups of a sequence are numbered head first, so a workgroup takes 128 / G
+// tokens with all G heads that share their K/V, and a wave two column groups.  (128
+// tokens of one query head did about as well for long prompts, 1051 against 1011 us
+// for 8 x 4096, but a prompt of 30 tokens then fills a quarter of the columns, and
+// a tile walks keys that its first tokens do not see: 128 prompts of 16..300
+// tokens 177 against 134 us.)  Keys are walked 32 at a time.  The K rows and the V rows of a tile go from global memory
 // straight into LDS (global_load_lds_dwordx4: no staging registers, no LDS
 // write instructions), row-major with the 16-byte pieces of a row permuted so
 // that the reads below are free of bank conflicts, in rings of 4 tiles each,
@@ -46,8 +51,7 @@ constexpr int kPieces = 16;          // 16-byte pieces per (position, head) row
 // workgroups (1 or 2 groups) were 5-20 % slower.
 constexpr int kGroups = 2;           // column groups of 16 query rows per wave
 constexpr int kWaves = 4;
-constexpr int kRowsPerWave = 16 * kGroups;
-constexpr int kBM = kRowsPerWave * kWaves;   // query rows per workgroup
+constexpr int kColumnGroups = kGroups * kWaves;   // per workgroup: 128 query rows
 constexpr int kKeys = 32;            // keys per step
 constexpr int kTileBytes = kKeys * kD * 2;   // one K or V tile in LDS: 32 rows of 256 bytes
 // Both rings hold 4 tiles, tile t in slot t % 4: iteration i reads K of tile i and
@@ -310,23 +314,23 @@ __device__ __forceinline__ void v_read_addresses(lds_ptr v_lds, int r, int kg, l
 // Probabilities of one tile from its scores (fp32 online softmax on the
 // accumulator layout), already in B-operand layout.
 //   m_run[g]  reference point of the exponentials, mneg[g] = -m_run * sl2.
-// MASK: entries beyond `row_limit + 16*g + r` (causal) or `key_limit` (end of
-// the sequence), both relative to the first key of the tile, weigh exactly 0.
+// MASK: entries beyond `row_limit + token[g]` (causal) or `key_limit` (end of the
+// sequence), both relative to the first key of the tile, weigh exactly 0.
 // Must run after the previous tile has been accumulated: moving the reference
 // point rescales acc and lacc.
 template <bool MASK, bool F16>
 __device__ __forceinline__ void probabilities_of_tile(f32x4 (&sc)[kGroups][2], bf16x8 (&pb)[kGroups],
                                                       f32x4 (&acc)[kGroups][8], f32x4 (&lacc)[kGroups],
                                                       float (&m_run)[kGroups], float (&mneg)[kGroups],
-                                                      float sl2, int r, int kg, int row_limit,
-                                                      int key_limit) {
+                                                      float sl2, int kg, const int (&token)[kGroups],
+                                                      int row_limit, int key_limit) {
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
     f32x4& s0 = sc[g][0];
     f32x4& s1 = sc[g][1];
     // lane = (query row r of the group, key group kg): keys 4*kg + e and
     // 16 + 4*kg + e of the tile; `limit` = last key of the tile the row may see
-    const int limit = MASK ? min(row_limit + 16 * g + r, key_limit) : 0;
+    const int limit = MASK ? min(row_limit + token[g], key_limit) : 0;
     if (MASK) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -377,12 +381,14 @@ __device__ __forceinline__ void probabilities_of_tile(f32x4 (&sc)[kGroups][2], b
 }
 
 struct PrefillArgs {
-  const uint4* q;       // [Tq, Hq, 16] pieces
-  const uint4* k;       // [Tk, Hkv, 16] pieces
+  const uint4* q;       // Tq rows of Hq * 16 pieces, q_stride pieces apart
+  const uint4* k;       // Tk rows of Hkv * 16 pieces, kv_row_bytes apart
   const uint4* v;
   uint4* out;           // [Tq, Hq, 16] pieces
   const int32_t* cu_q;  // [B + 1]
   const int32_t* cu_k;  // [B + 1]; paged: the keys of a sequence, cached and new together
+  int64_t q_stride;
+  uint32_t kv_row_bytes;   // < 2^24 (checked by the host)
   int batch, num_heads, num_kv_heads, group;
   float scale_log2e;
   // paged only: k and v are the caches [num_blocks, block_size, Hkv, 16] pieces
@@ -390,7 +396,19 @@ struct PrefillArgs {
   int block_size, max_blocks, num_blocks;
 };
 
-// grid.x = 8 * ceil(tile bound * Hq / 8) workgroups (see the work-item mapping below).
+// Inclusive prefix sum over the 64 lanes of a wave with DPP moves.  (With shuffles
+// through LDS the lookup below took 5 us of a short prompt's workgroup.)
+__device__ __forceinline__ int wave_inclusive_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 -> rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 -> rows 2, 3
+  return x;
+}
+
+// grid.x = 8 * ceil(tile bound * Hkv / 8) workgroups (see the work-item mapping below).
 // PAGED: keys and values come from the block-paged cache through block_tables,
 // sequence i has len_k = cu_k[i+1] - cu_k[i] keys, and its len_q query rows are the
 // LAST len_q positions of the sequence (row j sees keys <= len_k - len_q + j):
@@ -413,18 +431,15 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
   // different XCDs (8 of them, each with its own L2), so the work list is cut
   // into 8 contiguous parts and workgroup id L takes item (L % 8) * part + L / 8:
   // one XCD then walks neighbouring items.  Items are ordered (kv head, query
-  // tile, query head of the group): neighbours share the K/V rows of one
-  // (sequence, kv head), which stay in that XCD's L2 instead of being fetched
-  // by all eight.  Later tiles of a sequence have more keys to walk and come
-  // first.
-  const int total_items = num_tiles_bound * a.num_heads;
+  // tile): neighbours share the K/V rows of one (sequence, kv head), which stay
+  // in that XCD's L2 instead of being fetched by all eight.  Later tiles of a
+  // sequence have more keys to walk and come first.
+  const int total_items = num_tiles_bound * a.num_kv_heads;
   const int part = (total_items + 7) / 8;
   const int item = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
   if (item >= total_items) return;
-  const int per_kv_head = num_tiles_bound * a.group;
-  const int kvh = item / per_kv_head;
-  const int in_kv = item - kvh * per_kv_head;
-  const int head = kvh * a.group + in_kv % a.group;
+  const int kvh = item / num_tiles_bound;
+  const int in_kv = item - kvh * num_tiles_bound;
   // Query tiles are numbered sequence by sequence.  A wave looks at 64 sequences
   // at a time, one per lane, with the offsets of 256 sequences fetched together
   // (one round trip per 256 sequences; a loop over the sequences one by one cost
@@ -432,30 +447,38 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
   // tiles: the work list was sized for a bound, and the items beyond the real
   // tiles sit at its end, where they delay nothing.  The real tiles are walked
   // from the last one down (the later tiles of a sequence have more keys).
-  int nt4[4], qb4[4], ql4[4], kb4[4], kl4[4];
+  const int group = a.group;
+  int nt4[4], incl4[4], qb4[4], ql4[4], kb4[4], kl4[4];
   auto load_offsets = [&](int base) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int s = min(base + 64 * k + lane, a.batch - 1);
-      qb4[k] = a.cu_q[s];
-      ql4[k] = a.cu_q[s + 1] - qb4[k];
-      kb4[k] = a.cu_k[s];
-      kl4[k] = a.cu_k[s + 1] - kb4[k];
-      nt4[k] = base + 64 * k + lane < a.batch ? (max(ql4[k], 0) + kBM - 1) / kBM : 0;
+      nt4[k] = incl4[k] = 0;
+      if (base + 64 * k < a.batch) {
+        const int s = min(base + 64 * k + lane, a.batch - 1);
+        qb4[k] = a.cu_q[s];
+        ql4[k] = a.cu_q[s + 1] - qb4[k];
+        kb4[k] = a.cu_k[s];
+        kl4[k] = a.cu_k[s + 1] - kb4[k];
+      }
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (base + 64 * k < a.batch) {
+        nt4[k] = base + 64 * k + lane < a.batch
+                     ? ((max(ql4[k], 0) + 15) / 16 * group + kColumnGroups - 1) / kColumnGroups
+                     : 0;
+        incl4[k] = wave_inclusive_scan(nt4[k]);   // tiles up to and including this lane's sequence
+      }
   };
   int real_tiles = 0;
   for (int base = 0; base < a.batch; base += 256) {
     load_offsets(base);
-    int sum = nt4[0] + nt4[1] + nt4[2] + nt4[3];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
-    real_tiles += sum;
+    for (int k = 0; k < 4; ++k) real_tiles += __builtin_amdgcn_readlane(incl4[k], 63);
   }
-  real_tiles = __builtin_amdgcn_readfirstlane(real_tiles);
-  if (in_kv / a.group >= real_tiles) return;   // beyond the real number of tiles
-  const int tile_id = real_tiles - 1 - in_kv / a.group;
-  int seq = -1, q0 = 0;
+  if (in_kv >= real_tiles) return;   // beyond the real number of tiles
+  const int tile_id = real_tiles - 1 - in_kv;
+  int seq = -1, c0 = 0;   // the sequence, its first column group of this tile
   int q_base = 0, len_q = 0, k_first = 0, k_count = 0;   // of that sequence, from the same loads
   {
     int before = 0;   // tiles of the sequences in front of this group of 64
@@ -464,65 +487,57 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         if (base + 64 * k < a.batch && seq < 0) {
-          const int nt = nt4[k];
-          int incl = nt;   // tiles up to and including this lane's sequence
-#pragma unroll
-          for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += up;
-          }
+          const int first = before + incl4[k] - nt4[k];
           const unsigned long long hit =
-              __ballot(nt > 0 && tile_id >= before + incl - nt && tile_id < before + incl);
+              __ballot(nt4[k] > 0 && tile_id >= first && tile_id < first + nt4[k]);
           if (hit != 0ull) {
             const int src = __builtin_ctzll(hit);
             seq = base + 64 * k + src;
-            q0 = (tile_id - before - __shfl(incl - nt, src, 64)) * kBM;
-            q_base = __shfl(qb4[k], src, 64);
-            len_q = __shfl(ql4[k], src, 64);
-            k_first = __shfl(kb4[k], src, 64);
-            k_count = __shfl(kl4[k], src, 64);
+            c0 = (tile_id - __builtin_amdgcn_readlane(first, src)) * kColumnGroups;
+            q_base = __builtin_amdgcn_readlane(qb4[k], src);
+            len_q = __builtin_amdgcn_readlane(ql4[k], src);
+            k_first = __builtin_amdgcn_readlane(kb4[k], src);
+            k_count = __builtin_amdgcn_readlane(kl4[k], src);
           }
-          before += __shfl(incl, 63, 64);
+          before += __builtin_amdgcn_readlane(incl4[k], 63);
         }
       }
     }
-    seq = __builtin_amdgcn_readfirstlane(seq);
-    q0 = __builtin_amdgcn_readfirstlane(q0);
-    q_base = __builtin_amdgcn_readfirstlane(q_base);
-    len_q = __builtin_amdgcn_readfirstlane(len_q);
-    k_first = __builtin_amdgcn_readfirstlane(k_first);
-    k_count = __builtin_amdgcn_readfirstlane(k_count);
   }
   if (seq < 0) return;   // (cannot happen: tile_id is a real tile)
   const int k_base = PAGED ? 0 : k_first;
   const int len_k = PAGED ? min(max(k_count, 0), a.max_blocks * a.block_size) : max(k_count, 0);
-  // key position of query row 0: rows are the tail of the sequence when paged
+  // key position of the first token: the new tokens are the tail of the sequence when paged
   const int off = PAGED ? max(len_k - len_q, 0) : 0;
-  const int q_end = min(q0 + kBM, len_q);           // rows [q0, q_end) are real
-  const int k_end = min(len_k, off + q_end);        // keys [0, k_end) are visible to some row
+  const int token_end = min((c0 + kColumnGroups - 1) / group * 16 + 16, len_q);   // of the tile
+  const int k_end = min(len_k, off + token_end);   // keys [0, k_end) are visible to some row
   const int nsteps = (k_end + kKeys - 1) / kKeys;
 
-  // ---- Q^T of both column groups as B operands: column r of group g is row
-  // q0 + 32*wave + 16*g + r; rows beyond the sequence are zero ----
+  // ---- Q^T of both column groups as B operands: column r of group g is token
+  // block0[g] + r of head[g]; tokens beyond the sequence are zero ----
+  int block0[kGroups], token[kGroups], head[kGroups];
   bf16x8 qreg[kGroups][4];
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
-    const int row = q0 + kRowsPerWave * wave + 16 * g + r;
+    const int c = c0 + kGroups * wave + g;
+    block0[g] = c / group * 16;
+    head[g] = kvh * group + c % group;
+    token[g] = block0[g] + r;
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-    const uint4* qrow =
-        a.q + ((int64_t)(q_base + min(row, len_q - 1)) * a.num_heads + head) * kPieces;
+    const uint4* qrow = a.q + (int64_t)(q_base + min(token[g], len_q - 1)) * a.q_stride +
+                        (int64_t)head[g] * kPieces;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const uint4 t = qrow[4 * s + kg];
-      qreg[g][s] = as_bf16x8(row < len_q ? t : zero);
+      qreg[g][s] = as_bf16x8(token[g] < len_q ? t : zero);
     }
   }
 
-  const uint32_t row_bytes = (uint32_t)a.num_kv_heads * (kD * 2);
+  const uint32_t row_bytes = a.kv_row_bytes;
   const char* k_head =
-      reinterpret_cast<const char*>(a.k + ((int64_t)k_base * a.num_kv_heads + kvh) * kPieces);
+      reinterpret_cast<const char*>(a.k + kvh * kPieces) + (int64_t)k_base * row_bytes;
   const char* v_head =
-      reinterpret_cast<const char*>(a.v + ((int64_t)k_base * a.num_kv_heads + kvh) * kPieces);
+      reinterpret_cast<const char*>(a.v + kvh * kPieces) + (int64_t)k_base * row_bytes;
   const const_i32_ptr table =
       PAGED ? (const_i32_ptr)(uintptr_t)(a.block_tables + (int64_t)seq * a.max_blocks) : cu_q;
 
@@ -551,7 +566,6 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
   // and starts the copies of tile i+2 into the ring slots last read in iteration
   // i-1 (K of tile i-1, V of tile i-2).  Before the barrier that ends it, every
   // lane waits for its copies of tile i+1.
-  const int wave_row0 = q0 + kRowsPerWave * wave;   // first query row of this wave
   if (nsteps > 0) {
     // V "of tile -1" (probabilities are zero there, but 0 * NaN is not 0)
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -567,8 +581,10 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
   // masked ones (the diagonal tile, or one that reaches past the last key),
   // then tiles whose keys no row of the wave sees, where it only helps to copy.
   // Separate loops rather than a branch inside one keep the accumulators in place.
-  const int n_active = min(nsteps, (off + wave_row0 + kRowsPerWave - 1) / kKeys + 1);
-  const int n_plain = min(min(off + wave_row0, k_end) / kKeys, n_active);
+  // A wave without a real row only helps to copy.
+  const int n_active =
+      block0[0] >= len_q ? 0 : min(nsteps, (off + block0[kGroups - 1] + 15) / kKeys + 1);
+  const int n_plain = min(min(off + block0[0] + 1, k_end) / kKeys, n_active);
 
   // Tile t lives in ring slot t % 4 (K and V alike).  Iteration i: scores of tile
   // i, accumulation of tile i-1, probabilities of tile i, copies of tile i+2 into
@@ -600,7 +616,7 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
     scores_of_tile<F16>(kaddr, (S) * kTileBytes, qreg, sc);                                  \
     accumulate_tile<F16>(vaddr, (((S) + 3) & 3) * kTileBytes, pb, acc, lacc);                \
     __builtin_amdgcn_s_setprio(0);                                                           \
-    probabilities_of_tile<false, F16>(sc, pb, acc, lacc, m_run, mneg, sl2, r, kg, 0, 0);     \
+    probabilities_of_tile<false, F16>(sc, pb, acc, lacc, m_run, mneg, sl2, kg, token, 0, 0); \
     __builtin_amdgcn_s_setprio(1);                                                           \
     copier.template issue_full<((S) + 2) & 3>((i) + 2, koff, voff);                          \
     NVJ_END_OF_TILE();                                                                       \
@@ -611,8 +627,8 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
     scores_of_tile<F16>(kaddr, ((i) & 3) * kTileBytes, qreg, sc);                            \
     accumulate_tile<F16>(vaddr, (((i) + 3) & 3) * kTileBytes, pb, acc, lacc);                \
     __builtin_amdgcn_s_setprio(0);                                                           \
-    probabilities_of_tile<MASKED, F16>(sc, pb, acc, lacc, m_run, mneg, sl2, r, kg, row_limit, \
-                                       key_limit);                                           \
+    probabilities_of_tile<MASKED, F16>(sc, pb, acc, lacc, m_run, mneg, sl2, kg, token,        \
+                                       row_limit, key_limit);                                \
     __builtin_amdgcn_s_setprio(1);                                                           \
     copier.issue((i) + 2, ((i) + 2) & 3, ((i) + 2) & 3);                                     \
     NVJ_END_OF_TILE();                                                                       \
@@ -629,7 +645,7 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
   for (; i < n_plain; ++i) NVJ_TILE(false, i, 0, 0);
   for (; i < n_active; ++i) {
     const int ks = i * kKeys;
-    NVJ_TILE(true, i, off + wave_row0 - ks, k_end - 1 - ks);
+    NVJ_TILE(true, i, off - ks, k_end - 1 - ks);
   }
   // the last tile of the wave is still to be accumulated; its V stays in place
   // until the copies of two iterations from now
@@ -643,32 +659,48 @@ __global__ __launch_bounds__(kWaves * 64, kGroups <= 2 ? 2 : 1) void prefill_att
 #undef NVJ_PLAIN_TILE_AT
 #undef NVJ_END_OF_TILE
 
-  // ---- epilogue: acc[g][jd][e] is O[row][dim = 16*jd + 4*kg + e] ----
+  // ---- epilogue: acc[g][jd][e] is O[token][dim = 16*jd + 4*kg + e].  The rows are
+  // turned in LDS (16-byte pieces permuted by the row as for K) so that every
+  // store writes four whole 256-byte rows instead of 32 bytes of 16 of them ----
+  __syncthreads();   // every wave is done with the rings, every copy has landed
+  char* stage = reinterpret_cast<char*>(k_ring) + wave * (kGroups * 16 * 256);
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
     const float l = lacc[g][0];   // already summed over every key of the row
-    const int row = wave_row0 + 16 * g + r;
-    if (row < len_q) {
-      const float inv = l > 0.f ? 1.0f / l : 0.f;   // no visible key at all -> zeros
-      uint2* orow = reinterpret_cast<uint2*>(
-          a.out + ((int64_t)(q_base + row) * a.num_heads + head) * kPieces);
+    const float inv = l > 0.f ? 1.0f / l : 0.f;   // no visible key at all -> zeros
 #pragma unroll
-      for (int jd = 0; jd < 8; ++jd) {
-        uint2 o;
-        o.x = Elem<F16>::pack2(acc[g][jd][0] * inv, acc[g][jd][1] * inv);
-        o.y = Elem<F16>::pack2(acc[g][jd][2] * inv, acc[g][jd][3] * inv);
-        orow[4 * jd + kg] = o;
-      }
+    for (int jd = 0; jd < 8; ++jd) {
+      uint2 o;
+      o.x = Elem<F16>::pack2(acc[g][jd][0] * inv, acc[g][jd][1] * inv);
+      o.y = Elem<F16>::pack2(acc[g][jd][2] * inv, acc[g][jd][3] * inv);
+      *reinterpret_cast<uint2*>(stage + (16 * g + r) * 256 +
+                                16 * k_position(r, 2 * jd + (kg >> 1)) + 8 * (kg & 1)) = o;
     }
   }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // rows of this wave only
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + kg, t = block0[g] + row;
+      const uint4 o = *reinterpret_cast<const uint4*>(stage + (16 * g + row) * 256 +
+                                                      16 * k_position(row, r));
+      if (t < len_q)
+        a.out[((int64_t)(q_base + t) * a.num_heads + head[g]) * kPieces + r] = o;
+    }
 }
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype) {
-  // every sequence adds at most one partly filled tile
-  const int64_t tiles = (int64_t)total_q_tokens / kBM + a.batch;
+  // every sequence adds at most one partly filled token block and one partly filled tile
+  if (((int64_t)total_q_tokens + 15) * a.group > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
+  const int64_t blocks = ((int64_t)total_q_tokens + 15 * (int64_t)a.batch) / 16;
+  const int64_t tiles =
+      (blocks * a.group + (kColumnGroups - 1) * (int64_t)a.batch) / kColumnGroups;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const int64_t items = tiles * a.num_heads;
+  const int64_t items = tiles * a.num_kv_heads;
   if (items > INT32_MAX - 8) return NVJ_ERR_BAD_SHAPE;
   const dim3 grid((unsigned)((items + 7) / 8 * 8)), block(kWaves * 64);
   const int nt = (int)tiles;
@@ -683,23 +715,26 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
 
 }  // namespace
 
-extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const void* k,
-                                            const void* v, const int32_t* cu_seqlens_q,
-                                            const int32_t* cu_seqlens_k, void* out,
-                                            int32_t total_q_tokens, int32_t batch,
-                                            int32_t num_heads, int32_t num_kv_heads,
-                                            int32_t head_dim, float scale, int32_t dtype) {
+extern "C" int nvj_prefill_attention_rows_launch(
+    void* stream, const void* q, int64_t q_row_stride, const void* k, const void* v,
+    int64_t kv_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, void* out,
+    int32_t total_q_tokens, int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_dim, float scale, int32_t dtype) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   if (total_q_tokens < 0 || batch < 0 || num_heads <= 0 || num_kv_heads <= 0)
     return NVJ_ERR_BAD_SHAPE;
   if (num_heads % num_kv_heads != 0) return NVJ_ERR_BAD_SHAPE;
   if (head_dim != kD) return NVJ_ERR_UNSUPPORTED;
   if (num_kv_heads > 32768) return NVJ_ERR_UNSUPPORTED;   // a key row stays below 2^24 bytes
+  if (q_row_stride < (int64_t)num_heads * kD || kv_row_stride < (int64_t)num_kv_heads * kD)
+    return NVJ_ERR_BAD_SHAPE;
+  if (kv_row_stride > (1 << 22)) return NVJ_ERR_UNSUPPORTED;
   if (!(scale >= 0.f)) return NVJ_ERR_BAD_SHAPE;   // the running max assumes a non-negative scale
   if (total_q_tokens == 0 || batch == 0) return NVJ_OK;
   if (!q || !k || !v || !cu_seqlens_q || !cu_seqlens_k || !out) return NVJ_ERR_NULL_POINTER;
-  if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-       reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(out)) & 15u)
+  if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+        reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(out)) & 15u) ||
+      ((q_row_stride | kv_row_stride) & 7))
     return NVJ_ERR_ALIGNMENT;
   PrefillArgs a = {};
   a.q = static_cast<const uint4*>(q);
@@ -708,12 +743,26 @@ extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const v
   a.out = static_cast<uint4*>(out);
   a.cu_q = cu_seqlens_q;
   a.cu_k = cu_seqlens_k;
+  a.q_stride = q_row_stride / 8;
+  a.kv_row_bytes = (uint32_t)kv_row_stride * 2;
   a.batch = batch;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;
   a.group = num_heads / num_kv_heads;
   a.scale_log2e = scale * kLog2e;
   return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype);
+}
+
+extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const void* k,
+                                            const void* v, const int32_t* cu_seqlens_q,
+                                            const int32_t* cu_seqlens_k, void* out,
+                                            int32_t total_q_tokens, int32_t batch,
+                                            int32_t num_heads, int32_t num_kv_heads,
+                                            int32_t head_dim, float scale, int32_t dtype) {
+  return nvj_prefill_attention_rows_launch(stream, q, (int64_t)num_heads * kD, k, v,
+                                           (int64_t)num_kv_heads * kD, cu_seqlens_q, cu_seqlens_k,
+                                           out, total_q_tokens, batch, num_heads, num_kv_heads,
+                                           head_dim, scale, dtype);
 }
 
 extern "C" int nvj_paged_prefill_attention_launch(
@@ -745,6 +794,8 @@ extern "C" int nvj_paged_prefill_attention_launch(
   a.out = static_cast<uint4*>(out);
   a.cu_q = cu_seqlens_q;
   a.cu_k = cu_seqlens_k;
+  a.q_stride = (int64_t)num_heads * kPieces;
+  a.kv_row_bytes = (uint32_t)num_kv_heads * (kD * 2);
   a.batch = batch;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;

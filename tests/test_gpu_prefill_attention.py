@@ -67,6 +67,32 @@ def test_prefill_batches_of_many_short_prompts(batch):
             assert np.array_equal(got[cu_q[i]], np.repeat(v[cu_k[i]], 2, axis=0)), i
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(6, 2), (5, 1), (24, 2), (16, 1), (4, 4)])
+def test_prefill_column_groups_and_rows_of_one_buffer(Hq, Hkv):
+    """Group sizes that do not divide the 8 column groups of a tile, lengths around the
+    16 tokens of a column group, and q, k, v as parts of one projection buffer."""
+    print(f"case prefill column groups Hq={Hq} Hkv={Hkv}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib
+    from oracle.paged_attention_oracle import variable_length_attention_prefill_ref
+    lens = [15, 16, 17, 1, 0, 40, 113]
+    q, k, v, cu_q, cu_k = _problem(90 + Hq, lens, lens, Hq, Hkv)
+    scale = 128 ** -0.5
+    want = variable_length_attention_prefill_ref(q, k, v, cu_q, cu_k, scale)
+    T, dev = sum(lens), "cuda:0"
+    buf = torch.cat([bits_to_torch(x, dev).reshape(T, -1) for x in (q, k, v)], 1).contiguous()
+    out = torch.empty(T, Hq, 128, dtype=torch.bfloat16, device=dev)
+    cq = torch.from_numpy(cu_q).to(dev)
+    at = buf.data_ptr()
+    _lib.check(_lib.load().nvj_prefill_attention_rows_launch(
+        torch.cuda.current_stream().cuda_stream, at, buf.shape[1], at + 256 * Hq,
+        at + 256 * (Hq + Hkv), buf.shape[1], cq.data_ptr(), cq.data_ptr(), out.data_ptr(), T,
+        len(lens), Hq, Hkv, 128, scale, _lib.NVJ_DTYPE_BF16), "rows")
+    torch.cuda.synchronize()
+    assert_close_bf16(torch_to_bits(out), want, what=f"rows Hq={Hq} Hkv={Hkv}")
+    assert np.array_equal(torch_to_bits(out), run_hip(q, k, v, cu_q, cu_k, scale))
+
+
 def test_prefill_reference_smoke_lengths():
     """Sequence lengths of the reference's prefill smoke test
     (test_mosaic_kernels.py:90-159): 512, 768, 1024, 1536; Hq=32, Hkv=8, D=128."""
