@@ -33,8 +33,7 @@ from ..layers.attention import Attention
 from ..layers.layernorm import rms_norm
 from ..layers.paged_attention import (DecodeWorkspace, choose_split, paged_attention,
                                       paged_decode_workspace_bytes)
-from ..layers.prefill_attention import (paged_prefill_attention,
-                                        variable_length_attention_prefill)
+from ..layers.prefill_attention import paged_prefill_attention
 from ..layers.qk_rope_store import qk_norm_rope_store
 from ..utils.context import AttentionContext, create_decode_context, create_prefill_context
 
@@ -356,8 +355,8 @@ class DecodeStepRunner:
         c = self.cfg
         h = F.embedding(input_ids.long(), self.embed)
         residual = None
-        cs = self.cos_sin[positions.long()][:, None, :]
-        cos, sin = cs.chunk(2, dim=-1)
+        if not self.fused_qk_rope_store:
+            cos, sin = self.cos_sin[positions.long()][:, None, :].chunk(2, dim=-1)
         qs, ks = c.num_heads * c.head_dim, c.num_kv_heads * c.head_dim
         for lw, attn in zip(self.layers, self.attn):
             if residual is None:
@@ -366,33 +365,25 @@ class DecodeStepRunner:
                 h, residual = self._rms(h, lw["ln1"], residual)
             qkv = F.linear(h, lw["qkv"])
             if self.fused_qk_rope_store:
-                q = qk_norm_rope_store(qkv, positions, self.cos_sin, lw["q_norm"], lw["k_norm"],
-                                       c.rms_norm_eps, attn.k_cache, attn.v_cache,
-                                       context.slot_mapping, c.num_heads, c.num_kv_heads,
-                                       c.head_dim)
-                if context.is_prefill and context.block_tables is not None:
-                    # prompt rows behind a cached prefix: keys and values, the rows the
-                    # fused launch just stored included, come from the paged cache
-                    o = paged_prefill_attention(q, attn.k_cache, attn.v_cache,
-                                                context.block_tables, context.cu_seqlens_q,
-                                                context.cu_seqlens_k, attn.scale)
-                elif context.is_prefill:
-                    # K/V of the prompt rows were normalised, rotated and stored by
-                    # the fused launch; the prefill kernel wants them packed, so
-                    # they are gathered back from the cache rows just written
-                    flat = (-1, c.num_kv_heads, c.head_dim)
-                    sl = context.slot_mapping.long()
-                    if bool((sl < 0).any()):    # a skipped row was never stored
-                        raise ValueError("packed prefill through the fused store needs every "
-                                         "prompt row stored: slot_mapping has negative entries")
-                    o = variable_length_attention_prefill(
-                        q, attn.k_cache.view(flat)[sl], attn.v_cache.view(flat)[sl],
-                        context.cu_seqlens_q, context.cu_seqlens_k, scale=attn.scale)
+                if context.is_prefill and context.block_tables is None:
+                    o = self._rotate_store_prefill(qkv, positions, lw, attn, context)
                 else:
-                    o = paged_attention(q, attn.k_cache, attn.v_cache, context.block_tables,
-                                        context.context_lens, attn.scale, attn.block_size,
-                                        chunk=context.decode_split,
-                                        workspace=attn.workspace or self._eager_workspace(context))
+                    q = qk_norm_rope_store(qkv, positions, self.cos_sin, lw["q_norm"],
+                                           lw["k_norm"], c.rms_norm_eps, attn.k_cache,
+                                           attn.v_cache, context.slot_mapping, c.num_heads,
+                                           c.num_kv_heads, c.head_dim)
+                    if context.is_prefill:
+                        # prompt rows behind a cached prefix: keys and values, the rows the
+                        # fused launch just stored included, come from the paged cache
+                        o = paged_prefill_attention(q, attn.k_cache, attn.v_cache,
+                                                    context.block_tables, context.cu_seqlens_q,
+                                                    context.cu_seqlens_k, attn.scale)
+                    else:
+                        o = paged_attention(q, attn.k_cache, attn.v_cache, context.block_tables,
+                                            context.context_lens, attn.scale, attn.block_size,
+                                            chunk=context.decode_split,
+                                            workspace=attn.workspace or
+                                            self._eager_workspace(context))
                 h = F.linear(o.reshape(-1, qs), lw["o"])
                 h, residual = self._rms(h, lw["ln2"], residual)
                 h = F.linear(self._silu_mul(F.linear(h, lw["gate_up"])), lw["down"])
@@ -413,6 +404,39 @@ class DecodeStepRunner:
         if context.is_prefill:                           # only the last token of each prompt
             h = h[context.last_token_indices.long()]     # (models/qwen3.py:472-491)
         return F.linear(h, self.embed)                   # logits [T or batch, vocab]
+
+    def _rotate_store_prefill(self, qkv, positions, lw, attn, context):
+        """QK-norm, RoPE and cache store of packed prompt rows in place in the projection
+        buffer, then attention over its q, k and v parts where they are."""
+        c, lib = self.cfg, _lib.load()
+        tokens, width = qkv.shape
+        if not (qkv.is_contiguous() and positions.is_contiguous()
+                and context.slot_mapping.is_contiguous() and positions.dtype == torch.int32
+                and context.slot_mapping.dtype == torch.int32
+                and positions.shape == context.slot_mapping.shape == (tokens,)
+                and attn.k_cache.is_contiguous() and attn.v_cache.is_contiguous()
+                and all(t.dtype == torch.int32 and t.is_contiguous()
+                        for t in (context.cu_seqlens_q, context.cu_seqlens_k))):
+            raise ValueError("prefill metadata must be contiguous int32, one entry per token")
+        q = qkv.data_ptr()
+        k = q + 2 * c.num_heads * c.head_dim
+        v = k + 2 * c.num_kv_heads * c.head_dim
+        out = torch.empty((tokens, c.num_heads, c.head_dim), dtype=qkv.dtype, device=qkv.device)
+        with torch.cuda.device(qkv.device):
+            stream = torch.cuda.current_stream(qkv.device).cuda_stream
+            _lib.check(lib.nvj_qk_norm_rope_rows_launch(
+                stream, q, width, positions.data_ptr(), self.cos_sin.data_ptr(),
+                self.cos_sin.shape[0], lw["q_norm"].data_ptr(), lw["k_norm"].data_ptr(),
+                c.rms_norm_eps, context.slot_mapping.data_ptr(), attn.k_cache.data_ptr(),
+                attn.v_cache.data_ptr(), q, width, k, None, width, tokens, c.num_heads,
+                c.num_kv_heads, c.head_dim, attn.k_cache.numel() // (c.num_kv_heads * c.head_dim)),
+                "nvj_qk_norm_rope_rows_launch")
+            _lib.check(lib.nvj_prefill_attention_rows_launch(
+                stream, q, width, k, v, width, context.cu_seqlens_q.data_ptr(),
+                context.cu_seqlens_k.data_ptr(), out.data_ptr(), tokens,
+                context.cu_seqlens_q.shape[0] - 1, c.num_heads, c.num_kv_heads, c.head_dim,
+                attn.scale, _lib.NVJ_DTYPE_BF16), "nvj_prefill_attention_rows_launch")
+        return out
 
     # -- one decode step ------------------------------------------------------
     def make_inputs(self, last_tokens, seq_lens, block_tables):
