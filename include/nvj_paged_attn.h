@@ -87,6 +87,20 @@ NVJ_API int nvj_store_kvcache_launch(void* stream,
                              int32_t k_dtype, int32_t v_dtype, int32_t cache_dtype);
 
 /*
+ * The same with what would otherwise be launches of their own: packed copies of the
+ * new rows in the cache's type ([num_tokens, num_kv_heads, head_dim], written for every
+ * token whatever its slot; NULL = none), and `clear_bytes` (a multiple of 4) of zeroes
+ * at `clear` (NULL = none), as the counters of a decode launched behind it need them.
+ * With num_tokens 0 nothing is done.
+ */
+NVJ_API int nvj_store_kvcache_rows_launch(void* stream, const void* key, const void* value,
+                            void* k_cache, void* v_cache, const int32_t* slot_mapping,
+                            int32_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
+                            int64_t num_slots, int32_t k_dtype, int32_t v_dtype,
+                            int32_t cache_dtype, void* k_rows, void* v_rows, void* clear,
+                            size_t clear_bytes);
+
+/*
  * How the positions of a call are split over workgroups is chosen by `chunk`:
  *
  *   chunk == 0  balanced split (the default), ONE launch for any mix of

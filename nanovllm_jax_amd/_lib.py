@@ -7,6 +7,7 @@ this path.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -53,6 +54,10 @@ SYMBOLS = {
     "nvj_store_kvcache_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p,
         _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_int32]),
+    "nvj_store_kvcache_rows_launch": (_c.c_int, [
+        _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p,
+        _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int64, _c.c_int32, _c.c_int32, _c.c_int32,
+        _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_size_t]),
     "nvj_paged_decode_default_chunk": (_c.c_int32, [_c.c_int32] * 4),
     "nvj_paged_decode_whole_sequence_workgroups": (_c.c_int32, [_c.c_int32] * 3),
     "nvj_paged_decode_workspace_bytes": (_c.c_size_t, [_c.c_int32] * 7),
@@ -161,6 +166,27 @@ def load() -> ctypes.CDLL:
                 f"{_LIB_PATH} has ABI version {got}, expected {NVJ_ABI_VERSION}: rebuild")
         _lib = lib
         return lib
+
+
+_host = None
+
+
+def load_host():
+    """The native host side (``csrc/host/nvj_host.cpp``), loaded once; missing is an
+    error, as for the library itself."""
+    global _host
+    if _host is None:
+        load()
+        path = os.path.join(os.path.dirname(_LIB_PATH), "nvj_host.so")
+        if not os.path.exists(path):
+            raise NativeLibraryError(
+                f"{path} not found: build it with `python -c 'import __graft_entry__ as g; "
+                "g.build()'`")
+        spec = importlib.util.spec_from_file_location("nvj_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(code: int, what: str) -> None:

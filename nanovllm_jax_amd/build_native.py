@@ -57,6 +57,30 @@ def build(verbose: bool = True, extra_flags: tuple[str, ...] = ()) -> str:
     return LIB_PATH
 
 
+def build_host(verbose: bool = True) -> str:
+    """Compile the native host side of an attention call (csrc/host) against torch's
+    headers with the host compiler; it links the library just built."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    out = os.path.join(NATIVE_DIR, "nvj_host.so")
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared",
+           "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(REPO_DIR, "include"),
+           *[x for p in include_paths() for x in ("-isystem", p)],
+           "-isystem", sysconfig.get_paths()["include"],
+           os.path.join(CSRC_DIR, "host", "nvj_host.cpp"),
+           *[x for p in library_paths() for x in ("-L", p)],
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-L", NATIVE_DIR, "-lnvj_paged_attn",
+           "-Wl,-rpath,$ORIGIN", "-o", out + ".tmp"]
+    if verbose:
+        print("[build]", " ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    os.replace(out + ".tmp", out)
+    return out
+
+
 def xla_ffi_include_dir() -> str | None:
     """Directory of the XLA FFI headers (they ship inside jaxlib), or None."""
     try:

@@ -1,0 +1,233 @@
+// The host side of one attention call as native code: takes the torch tensors of
+// Attention.__call__ as they are, checks them, allocates the output and enqueues the
+// store and the attention launches (layers/attention.py:436-480 of the reference).
+//
+// A small call is bound by the host: validation, allocation and two foreign calls of
+// 13 and 20 arguments cost 19 us in Python for 14 us of GPU work (one sequence of 700
+// positions).  Here they cost about 5.
+//
+// Anything that is not exactly the ordinary call (another device than the current
+// one, a view that is not contiguous, a type that has to be converted, a wrong shape)
+// is declined by returning None; the caller then takes its general path, which
+// converts it or names the mistake.  An error code of the library comes back as an int.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+
+#include "nvj_paged_attn.h"
+
+namespace {
+
+using at::Tensor;
+
+bool get(PyObject* o, const Tensor** t) {
+  if (!THPVariable_Check(o)) return false;
+  *t = &THPVariable_Unpack(o);
+  return true;
+}
+
+int type_code(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return NVJ_DTYPE_BF16;
+    case at::kHalf: return NVJ_DTYPE_F16;
+    case at::kFloat: return NVJ_DTYPE_F32;
+    default: return -1;
+  }
+}
+
+struct Caches {
+  const Tensor *k, *v;
+  int dtype;
+  int64_t num_blocks, page, heads, dim;
+};
+
+// What both phases ask of q, the new rows and the caches.
+bool layer_tensors(PyObject* const* args, int64_t device, const Tensor** q, const Tensor** key,
+                   const Tensor** value, Caches* c, const Tensor** slots) {
+  if (!get(args[0], q) || !get(args[1], key) || !get(args[2], value) || !get(args[3], &c->k) ||
+      !get(args[4], &c->v) || !get(args[5], slots))
+    return false;
+  for (const Tensor* t : {*q, *key, *value, c->k, c->v, *slots})
+    if (!t->is_cuda() || t->device().index() != device || !t->is_contiguous()) return false;
+  c->dtype = type_code(c->k->scalar_type());
+  if (c->dtype != NVJ_DTYPE_BF16 && c->dtype != NVJ_DTYPE_F16) return false;
+  if (c->k->dim() != 4 || c->v->sizes() != c->k->sizes() ||
+      c->v->scalar_type() != c->k->scalar_type())
+    return false;
+  c->num_blocks = c->k->size(0);
+  c->page = c->k->size(1);
+  c->heads = c->k->size(2);
+  c->dim = c->k->size(3);
+  const Tensor& qt = **q;
+  if (qt.dim() != 3 || qt.scalar_type() != c->k->scalar_type() || qt.size(2) != c->dim ||
+      c->heads == 0 || qt.size(1) % c->heads != 0)
+    return false;
+  for (const Tensor* t : {*key, *value})
+    if (t->dim() != 3 || t->size(0) != qt.size(0) || t->size(1) != c->heads ||
+        t->size(2) != c->dim ||
+        (t->scalar_type() != c->k->scalar_type() && t->scalar_type() != at::kFloat))
+      return false;
+  return (*slots)->scalar_type() == at::kInt && (*slots)->dim() == 1 &&
+         (*slots)->size(0) == qt.size(0);
+}
+
+bool int_tensor(PyObject* o, int64_t device, int64_t dims, const Tensor** t) {
+  return get(o, t) && (*t)->is_cuda() && (*t)->device().index() == device &&
+         (*t)->scalar_type() == at::kInt && (*t)->dim() == dims && (*t)->is_contiguous();
+}
+
+int store(void* stream, const Tensor& key, const Tensor& value, const Caches& c,
+          const Tensor& slots, void* k_rows, void* v_rows, void* clear, size_t clear_bytes) {
+  return nvj_store_kvcache_rows_launch(
+      stream, key.data_ptr(), value.data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
+      static_cast<const int32_t*>(slots.data_ptr()), (int32_t)key.size(0), (int32_t)c.heads,
+      (int32_t)c.dim, c.num_blocks * c.page, type_code(key.scalar_type()),
+      type_code(value.scalar_type()), c.dtype, k_rows, v_rows, clear, clear_bytes);
+}
+
+// decode(q, k, v, k_cache, v_cache, slot_mapping, block_tables, context_lens, scale,
+//        block_size, chunk, partials | None, counters | None, device, stream)
+PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 15) Py_RETURN_NONE;
+  const int64_t device = PyLong_AsLong(args[13]);
+  void* stream = PyLong_AsVoidPtr(args[14]);
+  const double scale = PyFloat_AsDouble(args[8]);
+  const long block_size = PyLong_AsLong(args[9]), chunk = PyLong_AsLong(args[10]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const Tensor *q, *key, *value, *slots, *tables, *lens;
+  Caches c;
+  if (!layer_tensors(args, device, &q, &key, &value, &c, &slots) ||
+      !int_tensor(args[6], device, 2, &tables) || !int_tensor(args[7], device, 1, &lens))
+    Py_RETURN_NONE;
+  const int64_t batch = q->size(0), heads = q->size(1), max_blocks = tables->size(1);
+  if (block_size != c.page || tables->size(0) != batch || lens->size(0) != batch || batch == 0 ||
+      max_blocks == 0 || (chunk != 0 && chunk != NVJ_CHUNK_WHOLE_SEQUENCE))
+    Py_RETURN_NONE;
+  void *partials = nullptr, *counters = nullptr;
+  size_t partial_bytes = 0, counter_bytes = 0, clear_bytes = 0;
+  Tensor own;
+  const Tensor *given, *given_counters;
+  if (chunk == 0) {
+    const size_t need = nvj_paged_decode_workspace_bytes(batch, heads, c.dim, max_blocks, c.page,
+                                                         c.heads, 0);
+    const size_t head = nvj_paged_decode_counter_bytes(batch, heads, c.heads);
+    if (need == 0) Py_RETURN_NONE;
+    if (args[11] == Py_None) {
+      // a workspace for this call alone: the store clears its counters on the way
+      own = at::empty({(int64_t)need}, q->options().dtype(at::kByte));
+      counters = own.data_ptr();
+      counter_bytes = clear_bytes = head;
+      partials = static_cast<char*>(counters) + head;
+      partial_bytes = need - head;
+    } else {
+      if (!get(args[11], &given) || !get(args[12], &given_counters) ||
+          given->device() != q->device() || given_counters->device() != q->device() ||
+          !given->is_contiguous() || !given_counters->is_contiguous())
+        Py_RETURN_NONE;
+      partials = given->data_ptr();
+      partial_bytes = given->nbytes();
+      counters = given_counters->data_ptr();
+      counter_bytes = given_counters->nbytes();
+      if (partial_bytes + head < need || counter_bytes < head) Py_RETURN_NONE;
+    }
+  }
+  Tensor out = at::empty_like(*q);
+  int code = store(stream, *key, *value, c, *slots, nullptr, nullptr, clear_bytes ? counters : nullptr,
+                   clear_bytes);
+  if (code == NVJ_OK) {
+    const int32_t* table_ptr = static_cast<const int32_t*>(tables->data_ptr());
+    const int32_t* lens_ptr = static_cast<const int32_t*>(lens->data_ptr());
+    code = chunk == 0
+               ? nvj_paged_decode_launch_counters(
+                     stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(), table_ptr, lens_ptr,
+                     out.data_ptr(), partials, partial_bytes, counters, counter_bytes, batch, heads,
+                     c.heads, c.dim, c.page, max_blocks, c.num_blocks, (float)scale, c.dtype,
+                     NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE)
+               : nvj_paged_decode_launch_phases(
+                     stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(), table_ptr, lens_ptr,
+                     out.data_ptr(), nullptr, 0, batch, heads, c.heads, c.dim, c.page, max_blocks,
+                     c.num_blocks, (float)scale, chunk, c.dtype,
+                     NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE);
+  }
+  return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+}
+
+// prefill(q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k,
+//         block_tables | None, scale, block_size, device, stream, num_heads,
+//         num_kv_heads)
+PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 15) Py_RETURN_NONE;
+  const int64_t device = PyLong_AsLong(args[11]);
+  void* stream = PyLong_AsVoidPtr(args[12]);
+  const double scale = PyFloat_AsDouble(args[9]);
+  const long block_size = PyLong_AsLong(args[10]);
+  const long layer_heads = PyLong_AsLong(args[13]), layer_kv_heads = PyLong_AsLong(args[14]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const Tensor *q, *key, *value, *slots, *cu_q, *cu_k, *tables = nullptr;
+  Caches c;
+  const bool paged = args[8] != Py_None;
+  if (!layer_tensors(args, device, &q, &key, &value, &c, &slots) ||
+      !int_tensor(args[6], device, 1, &cu_q) || !int_tensor(args[7], device, 1, &cu_k) ||
+      (paged && !int_tensor(args[8], device, 2, &tables)))
+    Py_RETURN_NONE;
+  const int64_t tokens = q->size(0), heads = q->size(1), batch = cu_q->size(0) - 1;
+  if (heads != layer_heads || c.heads != layer_kv_heads) Py_RETURN_NONE;
+  if (batch < 1 || cu_k->size(0) != batch + 1 || block_size != c.page || tokens == 0 ||
+      (paged && (tables->size(0) != batch || tables->size(1) == 0)))
+    Py_RETURN_NONE;
+  // packed rows in the cache's type: where a float32 source is rounded for the cache
+  // anyway, the store leaves a packed copy
+  Tensor k_rows, v_rows;
+  void *kp = key->data_ptr(), *vp = value->data_ptr(), *k_copy = nullptr, *v_copy = nullptr;
+  if (!paged && key->scalar_type() == at::kFloat) {
+    k_rows = at::empty(key->sizes(), q->options());
+    kp = k_copy = k_rows.data_ptr();
+  }
+  if (!paged && value->scalar_type() == at::kFloat) {
+    v_rows = at::empty(value->sizes(), q->options());
+    vp = v_copy = v_rows.data_ptr();
+  }
+  Tensor out = at::empty_like(*q);
+  const int32_t* cq = static_cast<const int32_t*>(cu_q->data_ptr());
+  const int32_t* ck = static_cast<const int32_t*>(cu_k->data_ptr());
+  int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
+  if (code == NVJ_OK)
+    code = paged ? nvj_paged_prefill_attention_launch(
+                       stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
+                       static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(),
+                       tokens, batch, heads, c.heads, c.dim, c.page, tables->size(1), c.num_blocks,
+                       (float)scale, c.dtype)
+                 : nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck,
+                                                out.data_ptr(), tokens, batch, heads, c.heads,
+                                                c.dim, (float)scale, c.dtype);
+  return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+}
+
+// A C++ exception (out of memory in an allocation) becomes a Python one.
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  return F(self, args, nargs);
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"decode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<decode>)),
+     METH_FASTCALL, "store + paged decode attention of one layer"},
+    {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<prefill>)),
+     METH_FASTCALL, "store + prefill attention of one layer"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "nvj_host", nullptr, -1, methods,
+                      nullptr,               nullptr,    nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_nvj_host(void) { return PyModule_Create(&module); }

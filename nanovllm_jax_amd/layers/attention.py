@@ -18,7 +18,7 @@ import torch
 
 from .. import _lib
 from ..utils.context import AttentionContext
-from .paged_attention import paged_attention
+from .paged_attention import DecodeWorkspace, paged_attention
 from .prefill_attention import paged_prefill_attention, variable_length_attention_prefill
 
 __all__ = ["store_kv_to_cache", "Attention"]
@@ -43,6 +43,7 @@ def _raw_stream(device_index: int) -> int:
 
 # the current device without the bookkeeping of torch.cuda.current_device()
 _current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_host_decode = _host_prefill = None     # the native host side, looked up at the first call
 _store_launch = None    # the library's entry point, looked up at the first call
 
 
@@ -181,9 +182,41 @@ class Attention:
                                context.context_lens, self.scale, self.block_size,
                                chunk=context.decode_split, workspace=self.workspace)
 
+    def _native_call(self, q, k, v, context: AttentionContext):
+        """The ordinary call in native code; None when it is not one (see
+        csrc/host/nvj_host.cpp) and has to be looked at piece by piece."""
+        global _host_decode, _host_prefill
+        if _host_decode is None:
+            if not torch.cuda.is_available():
+                return None
+            host = _lib.load_host()
+            _host_prefill, _host_decode = host.prefill, host.decode
+        dev = _current_device()
+        if context.is_prefill:
+            out = _host_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping,
+                                context.cu_seqlens_q, context.cu_seqlens_k, context.block_tables,
+                                self.scale, self.block_size, dev, _raw_stream(dev), self.num_heads,
+                                self.num_kv_heads)
+        else:
+            ws, partials, counters = self.workspace, None, None
+            if ws is not None:
+                if type(ws) is not DecodeWorkspace or ws._clear_next:
+                    return None
+                partials, counters = ws.buffer, ws.counters
+            out = _host_decode(q, k, v, self.k_cache, self.v_cache, context.slot_mapping,
+                               context.block_tables, context.context_lens, self.scale,
+                               self.block_size, context.decode_split, partials, counters, dev,
+                               _raw_stream(dev))
+        if type(out) is int:
+            _lib.check(out, "attention call")
+        return out
+
     def __call__(self, q, k, v, context: AttentionContext):
         if self.k_cache is None or self.v_cache is None:
             raise RuntimeError("set_kv_cache() must be called before the first decode step")
+        out = self._native_call(q, k, v, context)
+        if out is not None:
+            return out
         store_kv_to_cache(k, v, self.k_cache, self.v_cache, context.slot_mapping)
         if context.is_prefill:
             return self._prefill_attention(q, k, v, context)

@@ -97,3 +97,29 @@ def test_qk_rows_in_place_and_unaligned(offset, pad):
         if 0 <= s < 16:
             assert np.array_equal(torch_to_bits(kc)[s], want_k[i])
             assert np.array_equal(torch_to_bits(vc)[s], want_v[i])
+
+
+@pytest.mark.parametrize("tokens,heads,clear", [(1, 1, 1), (3, 2, 257), (40, 8, 576)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_store_with_packed_copies_and_cleared_words(tokens, heads, clear, dtype):
+    print(f"case store rows tokens={tokens} clear={clear} {dtype}", flush=True)
+    from nanovllm_jax_amd import _lib, store_kv_to_cache
+    dev, dt = "cuda:0", torch.bfloat16 if dtype == "bf16" else torch.float16
+    code = _lib.NVJ_DTYPE_BF16 if dtype == "bf16" else _lib.NVJ_DTYPE_F16
+    k = torch.randn(tokens, heads, 128, device=dev)
+    v = torch.randn(tokens, heads, 128, device=dev).to(dt)
+    slots = torch.randperm(64)[:tokens].to(torch.int32)
+    slots[0] = -1
+    slots = slots.to(dev)
+    kc, vc, want_k, want_v = (torch.zeros(64, heads, 128, dtype=dt, device=dev) for _ in range(4))
+    k_rows, v_rows = torch.zeros_like(v), torch.zeros_like(v)
+    words = torch.full((clear + 1,), 7, dtype=torch.int32, device=dev)
+    _lib.check(_lib.load().nvj_store_kvcache_rows_launch(
+        torch.cuda.current_stream().cuda_stream, k.data_ptr(), v.data_ptr(), kc.data_ptr(),
+        vc.data_ptr(), slots.data_ptr(), tokens, heads, 128, 64, _lib.NVJ_DTYPE_F32, code, code,
+        k_rows.data_ptr(), v_rows.data_ptr(), words.data_ptr(), 4 * clear), "rows")
+    store_kv_to_cache(k, v, want_k, want_v, slots)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, want_k) and torch.equal(vc, want_v)
+    assert torch.equal(k_rows, k.to(dt)) and torch.equal(v_rows, v)
+    assert words.tolist() == [0] * clear + [7]
