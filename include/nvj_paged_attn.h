@@ -544,18 +544,16 @@ NVJ_API int nvj_silu_and_mul_launch(void* stream, const void* x, int64_t x_row_s
                             void* y, int32_t num_tokens, int32_t intermediate);
 
 /*
- * One step of the whole decoder stack for up to 16 token rows: a decode batch or a
- * short prefill, up to the logits.  Covers the model of
- * models/qwen3.py:130-172, 285-318, 366-393 and 472-491 (embedding; per layer
- * RMSNorm, fused QKV, QK-RMSNorm, RoPE, KV store, attention, output projection,
- * RMSNorm, SiLU MLP; final norm and tied LM head) as six launches per layer.
+ * One step of the whole decoder stack, a decode batch or the prefill of new prompts,
+ * up to the logits.  Covers the model of models/qwen3.py:130-172, 285-318, 366-393 and
+ * 472-491 (embedding; per layer RMSNorm, fused QKV, QK-RMSNorm, RoPE, KV store,
+ * attention, output projection, RMSNorm, SiLU MLP; final norm and tied LM head).
  *
  * Weights are bf16 [outputs, inputs] row-major, norm weights float32.  Projections
  * and the residual stream are rounded to bf16 where a separate launch would have
- * stored them.  head_dim must be 128, hidden 256, 512, 1024 or 2048,
- * num_heads * head_dim and intermediate multiples of 256 and at most 3072; every
- * pointer 16-byte aligned.
- * Enqueue-only; nothing is allocated.
+ * stored them.  head_dim must be 128; hidden, num_heads * head_dim and intermediate
+ * multiples of 64, hidden at most 8192, vocab a multiple of 8; every operand below
+ * 4 GiB; every pointer 16-byte aligned.  Enqueue-only; nothing is allocated.
  */
 typedef struct nvj_decoder_model {
   const void* embed;          /* [vocab, hidden] bf16, also the LM head */
@@ -597,7 +595,7 @@ typedef struct nvj_decoder_batch {
 } nvj_decoder_batch;
 
 NVJ_API size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
-                            int32_t num_tokens);
+                            int32_t num_tokens, int32_t num_sequences);
 NVJ_API int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* model,
                             const nvj_decoder_layer* layers, const nvj_decoder_batch* batch,
                             void* workspace, size_t workspace_bytes);

@@ -111,7 +111,8 @@ SYMBOLS = {
         _c.c_int32, _c.c_int32]),
     "nvj_silu_and_mul_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int32, _c.c_int32]),
-    "nvj_decoder_step_workspace_bytes": (_c.c_size_t, [_c.POINTER(DecoderModel), _c.c_int32]),
+    "nvj_decoder_step_workspace_bytes": (_c.c_size_t, [
+        _c.POINTER(DecoderModel), _c.c_int32, _c.c_int32]),
     "nvj_decoder_step_launch": (_c.c_int, [
         _c.c_void_p, _c.POINTER(DecoderModel), _c.POINTER(DecoderLayer), _c.POINTER(DecoderBatch),
         _c.c_void_p, _c.c_size_t]),

@@ -1,21 +1,25 @@
-// One step of the whole decoder stack for a small number of token rows (a decode
-// batch, or a short prefill) as a chain of six launches per layer for gfx950.
+// One step of the whole decoder stack (a decode batch, or the prefill of new prompts)
+// as a chain of launches enqueued in one call for gfx950.
 //
 // Covers the layer body of models/qwen3.py:130-172 and :285-318 of the reference
 // (fused QKV, per-head QK-RMSNorm, RoPE, store, attention, output projection,
 // pre-norm with fused residual, SiLU MLP), the embedding and the tied LM head
 // (:366-393, :472-491):
+// With up to 16 token rows, six launches per layer:
 //   1. norm_gemm QKV       RMSNorm in the prologue
 //   2. qk_norm_rope_store
 //   3. attention           the paged decode or the prefill kernel
 //   4. residual_gemm O     adds into the residual stream
 //   5. norm_gemm GATE_UP   RMSNorm in the prologue, SiLU(gate) * up in the epilogue
 //   6. residual_gemm DOWN
+// With more, the products of linear.hip between the norms of layer_glue.hip: QKV with
+// norm, RoPE and store in its epilogue, attention, O, add + norm, GATE_UP with SiLU * up
+// in its epilogue, DOWN, add + norm.
 // The residual stream h holds the unrounded fp32 sums that the next norm is taken
 // over; the sum that follows adds to their bf16 rounding, so every value is
 // rounded where the separate kernels (layer_glue.hip) round it.
 //
-// What bounds it: with few rows every product streams its weights once and the rest
+// What bounds the first form: with few rows every product streams its weights once and the rest
 // is latency, so a launch is worth its fixed 2-3 us only if the weights it
 // needs are all requested before anything else is waited for, by all CUs (one CU
 // alone draws some 50 GB/s).  Each wave therefore issues the loads of its whole
@@ -35,6 +39,7 @@
 #include <stdint.h>
 
 #include "launch.h"
+#include "linear.h"
 #include "nvj_paged_attn.h"
 
 namespace {
@@ -200,8 +205,9 @@ __global__ __launch_bounds__(256) void norm_gemm_kernel(NormGemmArgs a) {
 }
 
 // The same with one chain, for many outputs (the LM head): every wave owns a whole
-// 16-output tile, its weights in flight together.
-template <int RV, int ROWS>
+// 16-output tile, its weights in flight together.  NORM: the rows are normalised here;
+// otherwise a.h holds bf16 rows that have been.
+template <int RV, int ROWS, bool NORM>
 __global__ __launch_bounds__(256) void norm_gemm_wide_kernel(NormGemmArgs a) {
   constexpr int kWaves = 4;
   constexpr int kPieces = 32 * RV;
@@ -215,12 +221,22 @@ __global__ __launch_bounds__(256) void norm_gemm_wide_kernel(NormGemmArgs a) {
   const char* wrow =
       a.weight + (int64_t)min(n0 + r, a.outputs - 1) * (kPieces * 16) + 16 * kg;
   NormPrologue<RV, ROWS> norm;
-  norm.load(a, wave, kWaves, lane);
+  if constexpr (NORM) {
+    norm.load(a, wave, kWaves, lane);
+  } else {
+    const uint4* x = reinterpret_cast<const uint4*>(a.h);
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+      const int m = wave + kWaves * j;
+      for (int p = lane; p < kPieces; p += 64)
+        rows[m * kPieces + (p ^ m)] = x[(int64_t)min(m, a.num_tokens - 1) * kPieces + p];
+    }
+  }
   uint4 w[kDepth];
 #pragma unroll
   for (int i = 0; i < kDepth; ++i) w[i] = *reinterpret_cast<const uint4*>(wrow + 64 * i);
   __builtin_amdgcn_sched_barrier(0);
-  norm.store(rows, a.eps, wave, kWaves, lane);
+  if constexpr (NORM) norm.store(rows, a.eps, wave, kWaves, lane);
   __syncthreads();
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const int m = ROWS * kWaves >= 16 ? r : r % (ROWS * kWaves);
@@ -328,6 +344,18 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict
   }
 }
 
+// dst[m] = src[index[m]], rows of `pieces` 16-byte pieces, one wave per row.
+__global__ __launch_bounds__(256) void copy_rows_kernel(const uint4* __restrict__ src,
+                                                        const int32_t* __restrict__ index,
+                                                        uint4* __restrict__ dst, int num_rows,
+                                                        int pieces, int src_rows) {
+  const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= num_rows) return;
+  const int64_t row = min(max(index[m], 0), src_rows - 1);
+  for (int p = threadIdx.x & 63; p < pieces; p += 64)
+    dst[(int64_t)m * pieces + p] = src[row * pieces + p];
+}
+
 // hidden 256, 512, 1024 or 2048; one row per wave for up to 4 rows, else four
 #define NVJ_BY_ROW(LAUNCH)                                     \
   switch (hidden) {                                            \
@@ -344,10 +372,11 @@ hipError_t launch_norm_gemm(hipStream_t s, const NormGemmArgs& a, int hidden) {
   NVJ_BY_ROW(NVJ_LAUNCH)
 #undef NVJ_LAUNCH
 }
+template <bool NORM>
 hipError_t launch_norm_gemm_wide(hipStream_t s, const NormGemmArgs& a, int hidden) {
   const bool few = a.num_tokens <= 4;
   const dim3 grid((unsigned)((a.outputs + 63) / 64)), block(256);
-#define NVJ_LAUNCH(RV, ROWS) nvj::launch(norm_gemm_wide_kernel<RV, ROWS>, grid, block, s, a)
+#define NVJ_LAUNCH(RV, ROWS) nvj::launch(norm_gemm_wide_kernel<RV, ROWS, NORM>, grid, block, s, a)
   NVJ_BY_ROW(NVJ_LAUNCH)
 #undef NVJ_LAUNCH
 }
@@ -355,10 +384,18 @@ hipError_t launch_norm_gemm_wide(hipStream_t s, const NormGemmArgs& a, int hidde
 
 constexpr size_t round256(size_t n) { return (n + 255) / 256 * 256; }
 
+// Up to kMaxRows rows go through the first form where it is built for the sizes.
+bool few_rows_takes(const nvj_decoder_model& m, int64_t tokens, int64_t sequences) {
+  return tokens <= kMaxRows && sequences <= kMaxRows &&
+         (m.hidden == 256 || m.hidden == 512 || m.hidden == 1024 || m.hidden == 2048) &&
+         residual_gemm_takes((int64_t)m.num_heads * m.head_dim) &&
+         residual_gemm_takes(m.intermediate);
+}
+
 struct StepBuffers {
-  size_t h, qkv, q, o, k_rows, act, bytes;
+  size_t h, y, t, qkv, q, o, k_rows, act, last, bytes;
 };
-StepBuffers step_buffers(const nvj_decoder_model& m, int64_t tokens) {
+StepBuffers step_buffers(const nvj_decoder_model& m, int64_t tokens, int64_t sequences) {
   StepBuffers b;
   size_t at = 0;
   auto take = [&](size_t bytes_per_token) {
@@ -366,15 +403,20 @@ StepBuffers step_buffers(const nvj_decoder_model& m, int64_t tokens) {
     at += round256((size_t)tokens * bytes_per_token);
     return here;
   };
-  b.h = take((size_t)m.hidden * 4);
+  const size_t row = (size_t)m.hidden * 2;
   const size_t q_row = (size_t)m.num_heads * m.head_dim * 2;
   const size_t kv_row = (size_t)m.num_kv_heads * m.head_dim * 2;
+  b.h = take(2 * row);           // few rows: float32; else the bf16 residual
+  b.y = take(row);               // normalised rows
+  b.t = take(row);               // output of a projection
   b.qkv = take(q_row + 2 * kv_row);
   b.q = take(q_row);
   b.o = take(q_row);
-  b.k_rows = take(kv_row);   // packed K
-  take(kv_row);              // and V
+  b.k_rows = take(kv_row);       // packed K (few rows)
+  take(kv_row);                  // and V
   b.act = take((size_t)m.intermediate * 2);
+  b.last = at;                   // the rows that get logits, when not all do
+  at += round256((size_t)sequences * row);
   b.bytes = at;
   return b;
 }
@@ -385,21 +427,197 @@ int check_model(const nvj_decoder_model* m) {
       m->intermediate <= 0 || m->vocab <= 0 || m->max_position <= 0 || m->block_size <= 0 ||
       m->num_blocks <= 0 || m->num_heads % m->num_kv_heads != 0)
     return NVJ_ERR_BAD_SHAPE;
-  // hidden: the row lengths the norm prologue is built for
-  if (m->head_dim != 128 ||
-      (m->hidden != 256 && m->hidden != 512 && m->hidden != 1024 && m->hidden != 2048) ||
-      !residual_gemm_takes((int64_t)m->num_heads * m->head_dim) ||
-      !residual_gemm_takes(m->intermediate))
+  const int64_t q_width = (int64_t)m->num_heads * m->head_dim;
+  const int64_t qkv = q_width + 2 * (int64_t)m->num_kv_heads * m->head_dim;
+  if (m->head_dim != 128 || m->hidden > 8192 || m->intermediate % 16 != 0 ||
+      !nvj::linear_takes(1, qkv, m->hidden) || !nvj::linear_takes(1, m->hidden, q_width) ||
+      !nvj::linear_takes(1, 2 * (int64_t)m->intermediate, m->hidden) ||
+      !nvj::linear_takes(1, m->hidden, m->intermediate) ||
+      !nvj::linear_takes(1, m->vocab, m->hidden))
     return NVJ_ERR_UNSUPPORTED;
   return NVJ_OK;
+}
+
+int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer& l,
+              const nvj_decoder_batch& b, bool first_layer, const void* q,
+              const void* k, const void* v, int64_t kv_stride, void* out) {
+  if (b.is_prefill && !b.block_tables)
+    return nvj_prefill_attention_rows_launch(stream, q, (int64_t)m.num_heads * m.head_dim, k, v, kv_stride, b.cu_seqlens_q,
+                                             b.cu_seqlens_k, out, b.num_tokens, b.num_sequences,
+                                             m.num_heads, m.num_kv_heads, m.head_dim, m.scale,
+                                             NVJ_DTYPE_BF16);
+  if (b.is_prefill)
+    return nvj_paged_prefill_attention_launch(
+        stream, q, l.k_cache, l.v_cache, b.block_tables, b.cu_seqlens_q, b.cu_seqlens_k,
+        out, b.num_tokens, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim, m.block_size,
+        b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16);
+  const uint32_t phases = NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE;
+  if (b.chunk == 0)
+    return nvj_paged_decode_launch_counters(
+        stream, q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, out, b.partials,
+        b.partial_bytes, b.counters, b.counter_bytes, b.num_sequences, m.num_heads, m.num_kv_heads,
+        m.head_dim, m.block_size, b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16,
+        phases | (b.clear_counters && first_layer ? NVJ_PHASE_CLEAR_COUNTERS : 0));
+  return nvj_paged_decode_launch_phases(
+      stream, q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, out, b.partials,
+      b.partial_bytes, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim, m.block_size,
+      b.max_blocks, m.num_blocks, m.scale, b.chunk, NVJ_DTYPE_BF16, phases);
+}
+
+int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
+                     const nvj_decoder_batch& b, char* ws, const StepBuffers& at) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* h = reinterpret_cast<float*>(ws + at.h);
+  const int tokens = b.num_tokens;
+  const int q_width = m.num_heads * m.head_dim, kv_width = m.num_kv_heads * m.head_dim;
+  if (nvj::launch(embed_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
+                  static_cast<const uint4*>(m.embed), b.input_ids, reinterpret_cast<float4*>(h),
+                  tokens, m.hidden / 8, m.vocab) != hipSuccess)
+    return NVJ_ERR_LAUNCH;
+  NormGemmArgs a = {};
+  a.h = reinterpret_cast<const float4*>(h);
+  a.eps = m.eps;
+  a.num_tokens = tokens;
+  const bool packed = b.is_prefill && !b.block_tables;
+  char* k_rows = packed ? ws + at.k_rows : nullptr;
+  char* v_rows = packed ? k_rows + round256((size_t)tokens * kv_width * 2) : nullptr;
+  for (int i = 0; i < m.num_layers; ++i) {
+    const nvj_decoder_layer& l = layers[i];
+    a.weight = static_cast<const char*>(l.qkv);
+    a.norm_weight = l.ln1;
+    a.outputs = q_width + 2 * kv_width;
+    a.out = reinterpret_cast<uint16_t*>(ws + at.qkv);
+    if (launch_norm_gemm<kPlain>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
+    int code = nvj_qk_norm_rope_rows_launch(
+        stream, ws + at.qkv, a.outputs, b.positions, m.cos_sin, m.max_position, l.q_norm, l.k_norm,
+        m.eps, b.slot_mapping, l.k_cache, l.v_cache, ws + at.q, q_width, k_rows, v_rows, kv_width,
+        tokens, m.num_heads, m.num_kv_heads, m.head_dim, (int64_t)m.num_blocks * m.block_size);
+    if (code != NVJ_OK) return code;
+    code = attention(stream, m, l, b, i == 0, ws + at.q, k_rows, v_rows, kv_width,
+                     ws + at.o);
+    if (code != NVJ_OK) return code;
+    if (launch_residual_gemm<4, 1, 2>(s, ws + at.o, l.o, h, tokens, m.hidden, q_width) !=
+        hipSuccess)
+      return NVJ_ERR_LAUNCH;
+    a.weight = static_cast<const char*>(l.gate_up);
+    a.norm_weight = l.ln2;
+    a.outputs = 2 * m.intermediate;
+    a.out = reinterpret_cast<uint16_t*>(ws + at.act);
+    if (launch_norm_gemm<kSiluMul>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
+    if (launch_residual_gemm<2, 4, 4>(s, ws + at.act, l.down, h, tokens, m.hidden,
+                                      m.intermediate) != hipSuccess)
+      return NVJ_ERR_LAUNCH;
+  }
+  if (!b.logits || b.num_sequences == 0) return NVJ_OK;
+  a.weight = static_cast<const char*>(m.embed);
+  a.norm_weight = m.final_norm;
+  a.outputs = m.vocab;
+  a.out = static_cast<uint16_t*>(b.logits);
+  a.row_index = b.is_prefill ? b.last_token_indices : nullptr;
+  a.num_tokens = b.num_sequences;
+  return launch_norm_gemm_wide<true>(s, a, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+}
+
+// The order the library GEMMs sum the output and down projections in (see the top).
+hipError_t output_projection(hipStream_t s, const nvj::LinearArgs& a) {
+  if (a.M <= 128 && a.K % 128 == 0) return nvj::linear_chained(s, a, 4, 1);
+  return nvj::linear(s, a);
+}
+hipError_t down_projection(hipStream_t s, const nvj::LinearArgs& a) {
+  if (a.M <= 128 && a.K % 256 == 0)
+    return a.M > 64 || a.M == 32 ? nvj::linear_chained(s, a, 4, 2) : nvj::linear_chained(s, a, 2, 4);
+  return nvj::linear(s, a);
+}
+
+int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
+                      const nvj_decoder_batch& b, char* ws, const StepBuffers& at) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int tokens = b.num_tokens, pieces = m.hidden / 8;
+  const int q_width = m.num_heads * m.head_dim, kv_width = m.num_kv_heads * m.head_dim;
+  const int qkv_width = q_width + 2 * kv_width;
+  char *h = ws + at.h, *y = ws + at.y, *t = ws + at.t, *qkv = ws + at.qkv, *o = ws + at.o;
+  char* act = ws + at.act;
+  // the embedding rows are the residual
+  if (nvj::launch(copy_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
+                  static_cast<const uint4*>(m.embed), b.input_ids, reinterpret_cast<uint4*>(h),
+                  tokens, pieces, m.vocab) != hipSuccess)
+    return NVJ_ERR_LAUNCH;
+  int code = nvj_add_rms_norm_launch(stream, h, nullptr, layers[0].ln1, m.eps, y, nullptr, tokens,
+                                     m.hidden);
+  if (code != NVJ_OK) return code;
+  nvj::LinearArgs a = {};
+  a.M = tokens;
+  a.positions = b.positions;
+  a.cos_sin = m.cos_sin;
+  a.slot_mapping = b.slot_mapping;
+  a.eps = m.eps;
+  a.max_position = m.max_position;
+  a.num_heads = m.num_heads;
+  a.num_kv_heads = m.num_kv_heads;
+  a.num_slots = (int64_t)m.num_blocks * m.block_size;
+  a.q_out = reinterpret_cast<uint16_t*>(ws + at.q);
+  a.keep_kv = b.is_prefill && !b.block_tables;   // packed prefill reads K and V from the projection
+  auto product = [&](const void* x, const void* w, void* out, int n, int k) {
+    a.x = static_cast<const char*>(x);
+    a.w = static_cast<const char*>(w);
+    a.out = static_cast<uint16_t*>(out);
+    a.N = n;
+    a.K = k;
+  };
+  for (int i = 0; i < m.num_layers; ++i) {
+    const nvj_decoder_layer& l = layers[i];
+    product(y, l.qkv, qkv, qkv_width, m.hidden);
+    a.q_norm = l.q_norm;
+    a.k_norm = l.k_norm;
+    a.k_cache = static_cast<uint16_t*>(l.k_cache);
+    a.v_cache = static_cast<uint16_t*>(l.v_cache);
+    if (nvj::linear_qk_rope(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    code = attention(stream, m, l, b, i == 0, ws + at.q, qkv + 2 * (int64_t)q_width,
+                     qkv + 2 * (int64_t)(q_width + kv_width), qkv_width, o);
+    if (code != NVJ_OK) return code;
+    product(o, l.o, t, m.hidden, q_width);
+    if (output_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    code = nvj_add_rms_norm_launch(stream, t, h, l.ln2, m.eps, y, h, tokens, m.hidden);
+    if (code != NVJ_OK) return code;
+    product(y, l.gate_up, act, 2 * m.intermediate, m.hidden);
+    if (nvj::linear_silu_mul(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    product(act, l.down, t, m.hidden, m.intermediate);
+    if (down_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    const float* next = i + 1 < m.num_layers ? layers[i + 1].ln1 : m.final_norm;
+    code = nvj_add_rms_norm_launch(stream, t, h, next, m.eps, y, h, tokens, m.hidden);
+    if (code != NVJ_OK) return code;
+  }
+  if (!b.logits || b.num_sequences == 0) return NVJ_OK;
+  const char* rows = y;
+  if (b.is_prefill) {
+    if (nvj::launch(copy_rows_kernel, dim3((unsigned)((b.num_sequences + 3) / 4)), dim3(256), s,
+                    reinterpret_cast<const uint4*>(y), b.last_token_indices,
+                    reinterpret_cast<uint4*>(ws + at.last), b.num_sequences, pieces,
+                    tokens) != hipSuccess)
+      return NVJ_ERR_LAUNCH;
+    rows = ws + at.last;
+  }
+  if (few_rows_takes(m, 1, b.num_sequences)) {
+    NormGemmArgs n = {};
+    n.h = reinterpret_cast<const float4*>(rows);
+    n.weight = static_cast<const char*>(m.embed);
+    n.out = static_cast<uint16_t*>(b.logits);
+    n.num_tokens = b.num_sequences;
+    n.outputs = m.vocab;
+    return launch_norm_gemm_wide<false>(s, n, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+  }
+  a.M = b.num_sequences;
+  product(rows, m.embed, b.logits, m.vocab, m.hidden);
+  return nvj::linear(s, a) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }
 
 }  // namespace
 
 extern "C" size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
-                                                   int32_t num_tokens) {
-  if (check_model(model) != NVJ_OK || num_tokens <= 0) return 0;
-  return step_buffers(*model, num_tokens).bytes;
+                                                   int32_t num_tokens,
+                                                   int32_t num_sequences) {
+  if (check_model(model) != NVJ_OK || num_tokens <= 0 || num_sequences < 0) return 0;
+  return step_buffers(*model, num_tokens, num_sequences).bytes;
 }
 
 extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* model,
@@ -413,7 +631,11 @@ extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* mo
   const nvj_decoder_batch& b = *batch;
   if (b.num_tokens < 0 || b.num_sequences < 0 || (!b.is_prefill && b.num_tokens != b.num_sequences))
     return NVJ_ERR_BAD_SHAPE;
-  if (b.num_tokens > kMaxRows || b.num_sequences > kMaxRows) return NVJ_ERR_UNSUPPORTED;
+  if (!nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden, m.intermediate) ||
+      !nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden,
+                         (int64_t)m.num_heads * m.head_dim) ||
+      !nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden, m.hidden))
+    return NVJ_ERR_UNSUPPORTED;
   if (b.num_tokens == 0) return NVJ_OK;
   if (!layers || !m.embed || !m.final_norm || !m.cos_sin || !b.input_ids || !b.positions ||
       !b.slot_mapping || !workspace)
@@ -421,7 +643,7 @@ extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* mo
   if (b.is_prefill ? (!b.cu_seqlens_q || !b.cu_seqlens_k || (b.logits && !b.last_token_indices))
                    : !b.context_lens)
     return NVJ_ERR_NULL_POINTER;
-  const StepBuffers at = step_buffers(m, b.num_tokens);
+  const StepBuffers at = step_buffers(m, b.num_tokens, b.num_sequences);
   if (workspace_bytes < at.bytes) return NVJ_ERR_WORKSPACE;
   uintptr_t bits = reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(m.embed) |
                    reinterpret_cast<uintptr_t>(m.final_norm);
@@ -436,83 +658,8 @@ extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* mo
   }
   if (bits & 15u) return NVJ_ERR_ALIGNMENT;
 
-  hipStream_t s = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
-  float* h = reinterpret_cast<float*>(ws + at.h);
-  const int tokens = b.num_tokens;
-  const int q_width = m.num_heads * m.head_dim;
-
-  hipError_t rc = nvj::launch(embed_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
-                              static_cast<const uint4*>(m.embed), b.input_ids,
-                              reinterpret_cast<float4*>(h), tokens, m.hidden / 8, m.vocab);
-  if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
-
-  NormGemmArgs a = {};
-  a.h = reinterpret_cast<const float4*>(h);
-  a.eps = m.eps;
-  a.num_tokens = tokens;
-  const bool packed = b.is_prefill && !b.block_tables;
-  char* k_rows = packed ? ws + at.k_rows : nullptr;
-  char* v_rows =
-      packed ? k_rows + round256((size_t)tokens * m.num_kv_heads * m.head_dim * 2) : nullptr;
-
-  for (int i = 0; i < m.num_layers; ++i) {
-    const nvj_decoder_layer& l = layers[i];
-    a.weight = static_cast<const char*>(l.qkv);
-    a.norm_weight = l.ln1;
-    a.outputs = q_width + 2 * m.num_kv_heads * m.head_dim;
-    a.out = reinterpret_cast<uint16_t*>(ws + at.qkv);
-    if (launch_norm_gemm<kPlain>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
-
-    int code = nvj_qk_norm_rope_rows_launch(
-        stream, ws + at.qkv, a.outputs, b.positions, m.cos_sin, m.max_position, l.q_norm, l.k_norm,
-        m.eps, b.slot_mapping, l.k_cache, l.v_cache, ws + at.q, q_width, k_rows, v_rows,
-        m.num_kv_heads * m.head_dim, tokens, m.num_heads, m.num_kv_heads, m.head_dim,
-        (int64_t)m.num_blocks * m.block_size);
-    if (code != NVJ_OK) return code;
-    if (packed)
-      code = nvj_prefill_attention_launch(stream, ws + at.q, k_rows, v_rows,
-                                          b.cu_seqlens_q, b.cu_seqlens_k, ws + at.o, tokens,
-                                          b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
-                                          m.scale, NVJ_DTYPE_BF16);
-    else if (b.is_prefill)
-      code = nvj_paged_prefill_attention_launch(
-          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.cu_seqlens_q, b.cu_seqlens_k,
-          ws + at.o, tokens, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
-          m.block_size, b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16);
-    else if (b.chunk == 0)
-      code = nvj_paged_decode_launch_counters(
-          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, ws + at.o,
-          b.partials, b.partial_bytes, b.counters, b.counter_bytes, b.num_sequences, m.num_heads,
-          m.num_kv_heads, m.head_dim, m.block_size, b.max_blocks, m.num_blocks, m.scale,
-          NVJ_DTYPE_BF16,
-          NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE |
-              (b.clear_counters && i == 0 ? NVJ_PHASE_CLEAR_COUNTERS : 0));
-    else
-      code = nvj_paged_decode_launch_phases(
-          stream, ws + at.q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, ws + at.o,
-          b.partials, b.partial_bytes, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim,
-          m.block_size, b.max_blocks, m.num_blocks, m.scale, b.chunk, NVJ_DTYPE_BF16,
-          NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE);
-    if (code != NVJ_OK) return code;
-
-    rc = launch_residual_gemm<4, 1, 2>(s, ws + at.o, l.o, h, tokens, m.hidden, q_width);
-    if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
-    a.weight = static_cast<const char*>(l.gate_up);
-    a.norm_weight = l.ln2;
-    a.outputs = 2 * m.intermediate;
-    a.out = reinterpret_cast<uint16_t*>(ws + at.act);
-    if (launch_norm_gemm<kSiluMul>(s, a, m.hidden) != hipSuccess) return NVJ_ERR_LAUNCH;
-    rc = launch_residual_gemm<2, 4, 4>(s, ws + at.act, l.down, h, tokens, m.hidden, m.intermediate);
-    if (rc != hipSuccess) return NVJ_ERR_LAUNCH;
-  }
-  if (!b.logits) return NVJ_OK;
-  a.weight = static_cast<const char*>(m.embed);
-  a.norm_weight = m.final_norm;
-  a.outputs = m.vocab;
-  a.out = static_cast<uint16_t*>(b.logits);
-  a.row_index = b.is_prefill ? b.last_token_indices : nullptr;
-  a.num_tokens = b.num_sequences;
-  if (a.num_tokens == 0) return NVJ_OK;
-  return launch_norm_gemm_wide(s, a, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+  return few_rows_takes(m, b.num_tokens, b.num_sequences)
+             ? step_of_few_rows(stream, m, layers, b, ws, at)
+             : step_of_many_rows(stream, m, layers, b, ws, at);
 }

@@ -1,0 +1,488 @@
+// Products of activation rows with bf16 weights, C[m][n] = x[m][:] . w[n][:], for
+// prompts (hundreds to thousands of rows) on gfx950, with the element-wise stage that
+// follows a projection of the decoder layer in the epilogue:
+//   kPlain    bf16 rows
+//   kSiluMul  SiLU(gate) * up of the fused gate/up projection (layers/activation.py:22-33
+//             of the reference), half the columns
+//   kQkRope   QK-RMSNorm, RoPE and KV-cache store of the fused QKV projection
+//             (models/qwen3.py:147-166)
+//
+// MFMA-bound, if the operands arrive: a workgroup of 4 waves (2 x 2) computes BM x BN
+// outputs, K in steps of 64.  Rows go global -> LDS directly (16 bytes per lane, whole
+// 128-byte rows, pieces XOR-permuted by the row: no bank conflicts on the operand reads),
+// in a ring of two to four stages, one barrier per step, which stands in the middle of it
+// so that operand reads, copies and matrix instructions run under each other throughout.
+// Measured, 4400 rows: QKV (4096 x 1024) 40.9 us, O (1024 x 2048) 21.9, gate/up (6144 x
+// 1024) with SiLU * up 62.2, down (1024 x 3072) 29.8; library 46.4, 27.6, 56.4 + 16.7,
+// 35.2.  LDS is the next limit: operand reads and arriving copies take 75 % (256 x 256)
+// to 150 % (128 x 128) of the matrix cycles.  Weights straight into registers instead
+// (as in decoder_step.hip) were no way out: 64-byte pieces of 16 rows per load made it
+// 1 us per step whatever the tile.
+//
+// Every output is one chain of v_mfma_f32_16x16x32_bf16 over K in order, which is the
+// order of the library GEMMs at more than 128 rows: the same bits (decoder_step.hip says
+// why that matters).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "launch.h"
+#include "linear.h"
+#include "nvj_paged_attn.h"
+#include "qk_norm_rope.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) char* lds_ptr;
+
+constexpr int kBK = 64;        // reduction per step: rows of 128 bytes, 8 pieces
+
+using nvj::bf16_to_f32;
+using nvj::f32_to_bf16_rne;
+using nvj::LinearArgs;
+enum Epilogue { kPlain, kSiluMul, kQkRope };
+
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const bf16x2 p = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, p);
+}
+
+// One 16-byte global -> LDS copy per lane: lane l's piece lands at lds_base + 16 * l.
+// Counts in vmcnt; the compiler does not see it as a load, so the waits are by hand.
+__device__ __forceinline__ void copy16_to_lds(const char* base, uint32_t offset,
+                                              uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds_base), "v"(offset), "s"(base));
+}
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int BM, int BN, int kStages, Epilogue EPI>
+__global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
+  constexpr int WM = BM / 2, WN = BN / 2;          // per wave
+  constexpr int TM = WM / 16, TN = WN / 16;
+  constexpr int kRows = BM + BN;                   // rows of one stage: x, then w
+  constexpr int kStageBytes = kRows * 128;
+  constexpr int kCopies = kRows / 8 / 4;           // per wave and stage, 8 rows each
+  static_assert(kRows % 32 == 0, "copies are dealt to four waves");
+  constexpr int kOut = EPI == kSiluMul ? BN / 2 : BN;   // columns of the output tile
+  constexpr int kOutStride = kOut * 2 + 16;             // bytes per row of the tile in LDS
+  constexpr int kLds = kStages * kStageBytes > BM * kOutStride ? kStages * kStageBytes
+                                                               : BM * kOutStride;
+  __shared__ __align__(128) char lds[kLds];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // tiles of one weight column block are neighbours, and each XCD (workgroup id % 8)
+  // walks a contiguous part of the list, so a weight tile is fetched by one L2
+  const int total = a.m_tiles * a.n_tiles;
+  const int part = (total + 7) / 8;
+  const int tile = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
+  if (tile >= total) return;
+  const int per_group = a.group_m * a.n_tiles;
+  const int grp = tile / per_group, in_group = tile - grp * per_group;
+  const int gm = min(a.group_m, a.m_tiles - grp * a.group_m);
+  const int n_tile = in_group / gm, m_tile = grp * a.group_m + (in_group - n_tile * gm);
+  const int m0 = m_tile * BM;
+  const int row_bytes = a.K * 2;
+
+  // what this wave copies: instruction j moves LDS rows 8 * (4 * j + wave) .. + 7; lane
+  // l fetches the piece that belongs at position l % 8 of row l / 8
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
+  const char* base[kCopies];
+  uint32_t offset[kCopies];
+  {
+    const int row = lane >> 3, piece = (lane & 7) ^ row;
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) {
+      const int first = 8 * (4 * j + wave);   // a multiple of 8: a block of x or of w rows
+      if (first < BM) {
+        base[j] = a.x;
+        offset[j] = (uint32_t)min(m0 + first + row, a.M - 1) * (uint32_t)row_bytes + 16 * piece;
+      } else {
+        const int c = first - BM + row;       // column of the tile
+        int n;
+        if (EPI == kSiluMul)   // blocks of 16 columns: gate, then the same of up, in turn
+          n = min(n_tile * (BN / 2) + (c >> 5) * 16 + (c & 15), a.N / 2 - 1) +
+              ((c >> 4) & 1 ? a.N / 2 : 0);
+        else
+          n = min(n_tile * BN + c, a.N - 1);
+        base[j] = a.w;
+        offset[j] = (uint32_t)n * (uint32_t)row_bytes + 16 * piece;
+      }
+    }
+  }
+  const int steps = a.K / kBK;
+  auto issue = [&](int step, int stage) {
+    // past the end: the last step again, so that the count of copies in flight holds
+    const uint32_t k = (uint32_t)min(step, steps - 1) * (kBK * 2);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j)
+      copy16_to_lds(base[j], offset[j] + k,
+                    lds0 + (uint32_t)stage * kStageBytes + (uint32_t)(4 * j + wave) * 1024u);
+  };
+
+  f32x4 acc[TM][TN];   // D[n][m]: lane holds n = 4 * kg + e of column m = r
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // Software pipeline over halves of a step (32 of the reduction): while the matrix core
+  // works on the operands of one half, those of the next are read from LDS, and
+  // behind the barrier in the middle of a step the copies of a later one are issued,
+  // one every few matrix instructions.
+  const int x_row = wm * WM + r, w_row = BM + wn * WN + r;
+  bf16x8 xf[2][TM], wf[2][TN];
+  auto read = [&](int stage, int s, int i) {   // operand i of half s of a stage
+    const char* at = lds + stage * kStageBytes + 16 * ((4 * s + kg) ^ (r & 7));
+    if (i < TN) wf[s][i] = *reinterpret_cast<const bf16x8*>(at + (w_row + 16 * i) * 128);
+    else xf[s][i - TN] = *reinterpret_cast<const bf16x8*>(at + (x_row + 16 * (i - TN)) * 128);
+  };
+  auto multiply = [&](int s, int i) {          // matrix instruction i of half s
+    const int mi = i / TN, j = i % TN;
+    acc[mi][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][j], xf[s][mi], acc[mi][j], 0, 0, 0);
+  };
+  constexpr int kMul = TM * TN, kRead = TM + TN;
+#pragma unroll
+  for (int t = 0; t < kStages; ++t) issue(t, t);
+  wait_copies<(kStages - 1) * kCopies>();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kRead; ++i) read(0, 0, i);
+  int stage = 0;
+  for (int step = 0; step < steps; ++step) {
+    int done = 0;
+#pragma unroll
+    for (int i = 0; i < kRead; ++i) {
+      read(stage, 1, i);
+#pragma unroll
+      for (; done < (i + 1) * kMul / kRead; ++done) multiply(0, done);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int next = stage + 1 == kStages ? 0 : stage + 1;
+    wait_copies<(kStages - 2) * kCopies>();   // the next step's rows of this wave are there
+    __syncthreads();   // and everybody's; nobody reads this step's stage any more
+    const uint32_t k = (uint32_t)min(step + kStages, steps - 1) * (kBK * 2);
+    constexpr int kSlots = kRead > kCopies ? kRead : kCopies;
+    done = 0;
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      if (i < kRead) read(next, 0, i);
+      if (i < kCopies)
+        copy16_to_lds(base[i], offset[i] + k,
+                      lds0 + (uint32_t)stage * kStageBytes + (uint32_t)(4 * i + wave) * 1024u);
+#pragma unroll
+      for (; done < (i + 1) * kMul / kSlots; ++done) multiply(1, done);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    stage = next;
+  }
+  wait_copies<0>();   // copies past the last step are still landing
+  __syncthreads();
+
+  // ---- the tile as bf16 rows in LDS, then out in whole pieces ----
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    char* row = lds + (wm * WM + 16 * i + r) * kOutStride;
+    if constexpr (EPI == kSiluMul) {
+#pragma unroll
+      for (int j = 0; j < TN; j += 2) {
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = bf16_to_f32(f32_to_bf16_rne(acc[i][j][e]));
+          const float u = bf16_to_f32(f32_to_bf16_rne(acc[i][j + 1][e]));
+          o[e] = g / (1.0f + expf(-g)) * u;
+        }
+        *reinterpret_cast<uint2*>(row + (wn * (WN / 2) + 8 * j + 4 * kg) * 2) =
+            make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        *reinterpret_cast<uint2*>(row + (wn * WN + 16 * j + 4 * kg) * 2) =
+            make_uint2(pack2(acc[i][j][0], acc[i][j][1]), pack2(acc[i][j][2], acc[i][j][3]));
+    }
+  }
+  __syncthreads();
+  if constexpr (EPI == kQkRope) {
+    // 16 lanes per (row, head), a tile holds whole heads; the positions and slots of a
+    // batch of rows are fetched together, then their table rows: two round trips per
+    // batch instead of two per row
+    constexpr int kHeads = BN / 128, kUnits = BM * kHeads / 16;
+    constexpr int kBatch = kUnits % 5 == 0 ? 5 : kUnits % 4 == 0 ? 4 : 2;
+    static_assert(kUnits % kBatch == 0, "whole batches");
+    const int i = threadIdx.x & 15;
+    for (int u0 = 0; u0 < kUnits; u0 += kBatch) {
+      int pos[kBatch], slot[kBatch];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const int m = ((u0 + b) * 16 + (int)(threadIdx.x >> 4)) / kHeads;
+        const int token = min(m0 + m, a.M - 1);
+        pos[b] = a.positions[token];
+        slot[b] = a.slot_mapping[token];
+      }
+      float4 c4[kBatch], s4[kBatch];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const float* cs = a.cos_sin + (int64_t)min(max(pos[b], 0), a.max_position - 1) * 128 + 4 * i;
+        c4[b] = nvj::load4<true>(cs);
+        s4[b] = nvj::load4<true>(cs + 64);
+      }
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const int unit = (u0 + b) * 16 + (int)(threadIdx.x >> 4);
+        const int m = unit / kHeads, h = unit % kHeads;
+        const int token = m0 + m, head = n_tile * kHeads + h;
+        if (token >= a.M) continue;
+        const uint2* src = reinterpret_cast<const uint2*>(lds + m * kOutStride + 256 * h);
+        uint2 lo = src[i], hi = src[16 + i];
+        const bool is_q = head < a.num_heads;
+        const bool is_k = !is_q && head < a.num_heads + a.num_kv_heads;
+        if (is_q || is_k)
+          nvj::qk_norm_rope<true>(lo, hi, is_q ? a.q_norm : a.k_norm, a.eps, c4[b], s4[b], i);
+        if (is_q || a.keep_kv) {
+          uint2* dst = reinterpret_cast<uint2*>(
+              is_q ? a.q_out + ((int64_t)token * a.num_heads + head) * 128
+                   : a.out + (int64_t)token * a.N + head * 128);
+          dst[i] = lo;
+          dst[16 + i] = hi;
+        }
+        if (!is_q && slot[b] >= 0 && slot[b] < a.num_slots) {
+          const int kvh = head - a.num_heads - (is_k ? 0 : a.num_kv_heads);
+          uint2* row = reinterpret_cast<uint2*>((is_k ? a.k_cache : a.v_cache) +
+                                                ((int64_t)slot[b] * a.num_kv_heads + kvh) * 128);
+          row[i] = lo;
+          row[16 + i] = hi;
+        }
+      }
+    }
+  } else {
+    constexpr int kPieces = kOut / 8;
+    const int n_out = EPI == kSiluMul ? a.N / 2 : a.N;
+    for (int p = threadIdx.x; p < BM * kPieces; p += 256) {
+      const int m = p / kPieces, piece = p % kPieces, n = n_tile * kOut + 8 * piece;
+      if (m0 + m < a.M && n < n_out)
+        *reinterpret_cast<uint4*>(a.out + (int64_t)(m0 + m) * n_out + n) =
+            *reinterpret_cast<const uint4*>(lds + m * kOutStride + 16 * piece);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same for up to 128 rows where the reduction is cut into chains (the order of
+// the library GEMMs for the output and down projections at these sizes): 4 waves =
+// CHAINS chains x 4 / CHAINS row halves of a BM x BN tile; chain c takes every
+// CHAINS-th run of RUN steps of 32.  Each operand of a stage is read by one wave, so a
+// stage is a whole round of the chains (32 * CHAINS * RUN of the reduction) and the
+// waves meet once per round.  Latency-bound: the ring is as deep as LDS allows.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int CHAINS, int RUN, int kStages>
+__global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
+  constexpr int kSubs = CHAINS * RUN / 2;          // 64-wide blocks of a round
+  constexpr int kRows = BM + BN;
+  constexpr int kSubBytes = kRows * 128, kStageBytes = kSubs * kSubBytes;
+  constexpr int kCopies = kSubs * kRows / 8 / 4;   // per wave and stage, 8 rows each
+  static_assert(kSubs * kRows % 32 == 0 && CHAINS * RUN % 2 == 0, "whole blocks, dealt to four waves");
+  constexpr int kSplit = 4 / CHAINS;
+  constexpr int WM = BM / kSplit, TM = WM / 16, TN = BN / 16;
+  constexpr int kRedStride = BN + 4;
+  constexpr int kRed = CHAINS * BM * kRedStride * 4;
+  __shared__ __align__(128) char
+      lds[kStages * kStageBytes > kRed ? kStages * kStageBytes : kRed];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int chain = wave % CHAINS, half = wave / CHAINS;
+  const int n_tile = blockIdx.x, m0 = blockIdx.y * BM;
+  const int row_bytes = a.K * 2;
+  const int rounds = a.K / (32 * CHAINS * RUN);
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
+  const char* base[kCopies];
+  uint32_t offset[kCopies];
+#pragma unroll
+  for (int j = 0; j < kCopies; ++j) {
+    const int group = 4 * j + wave, sub = group / (kRows / 8), first = 8 * (group % (kRows / 8));
+    const int row = lane >> 3, piece = (lane & 7) ^ row;
+    base[j] = first < BM ? a.x : a.w;
+    const int at = first < BM ? min(m0 + first + row, a.M - 1)
+                              : min(n_tile * BN + first - BM + row, a.N - 1);
+    offset[j] = (uint32_t)at * (uint32_t)row_bytes + 128 * sub + 16 * piece;
+  }
+  auto issue = [&](int round, int stage) {
+    const uint32_t k = (uint32_t)min(round, rounds - 1) * (64 * CHAINS * RUN);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j)
+      copy16_to_lds(base[j], offset[j] + k,
+                    lds0 + (uint32_t)stage * kStageBytes + (uint32_t)(4 * j + wave) * 1024u);
+  };
+  f32x4 acc[TM][TN];   // D[n][m]: lane holds n = 4 * kg + e of column m = r
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < kStages - 1; ++t) issue(t, t);
+  int stage = 0;
+  for (int round = 0; round < rounds; ++round) {
+    wait_copies<(kStages - 2) * kCopies>();   // this round's rows of this wave are there
+    __syncthreads();                          // and everybody's; the stage read last is free
+    issue(round + kStages - 1, stage == 0 ? kStages - 1 : stage - 1);
+    const char* at = lds + stage * kStageBytes;
+    stage = stage + 1 == kStages ? 0 : stage + 1;
+#pragma unroll
+    for (int u = 0; u < RUN; ++u) {
+      const int step = chain * RUN + u;   // of the round
+      const char* block = at + (step >> 1) * kSubBytes + 16 * ((4 * (step & 1) + kg) ^ (r & 7));
+      bf16x8 xf[TM], wf[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        wf[j] = *reinterpret_cast<const bf16x8*>(block + (BM + 16 * j + r) * 128);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        xf[i] = *reinterpret_cast<const bf16x8*>(block + (half * WM + 16 * i + r) * 128);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i], acc[i][j], 0, 0, 0);
+    }
+  }
+  wait_copies<0>();
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      *reinterpret_cast<f32x4*>(red + (chain * BM + half * WM + 16 * i + r) * kRedStride + 16 * j +
+                                4 * kg) = acc[i][j];
+  __syncthreads();
+  for (int p = threadIdx.x; p < BM * BN / 4; p += 256) {
+    const int m = p / (BN / 4), n = 4 * (p % (BN / 4));
+    f32x4 v = *reinterpret_cast<const f32x4*>(red + m * kRedStride + n);
+#pragma unroll
+    for (int c = 1; c < CHAINS; ++c)
+      v += *reinterpret_cast<const f32x4*>(red + (c * BM + m) * kRedStride + n);
+    if (m0 + m < a.M && n_tile * BN + n < a.N)
+      *reinterpret_cast<uint2*>(a.out + (int64_t)(m0 + m) * a.N + n_tile * BN + n) =
+          make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+  }
+}
+
+template <int BM, int BN, int CHAINS, int RUN, int ST>
+hipError_t launch_chained(hipStream_t s, const LinearArgs& a) {
+  const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM));
+  return nvj::launch(chained_linear_kernel<BM, BN, CHAINS, RUN, ST>, grid, dim3(256), s, a);
+}
+
+template <int BM, int BN, int ST, Epilogue EPI>
+hipError_t launch_tiles(hipStream_t s, LinearArgs a) {
+  constexpr int kOut = EPI == kSiluMul ? BN / 2 : BN;
+  const int outs = EPI == kSiluMul ? a.N / 2 : a.N;
+  a.m_tiles = (a.M + BM - 1) / BM;
+  a.n_tiles = (outs + kOut - 1) / kOut;
+  const int total = a.m_tiles * a.n_tiles;
+  return nvj::launch(linear_kernel<BM, BN, ST, EPI>, dim3((unsigned)((total + 7) / 8 * 8)),
+                     dim3(256), s, a);
+}
+
+// Tile sizes.  A launch of T tiles takes rounds of 256 (or 512: two workgroups share a
+// CU), each round a fixed 3 us and per step of 64 a time between `low` (few CUs busy)
+// and `full` (all of them: the L2s and the power limit share out).  Measured on an
+// MI355X over 300 .. 4400 rows and the four projections of a 1024-wide layer, us:
+struct TileShape {
+  int bm, bn, per_cu;
+  float low, full;
+};
+constexpr TileShape kShapes[] = {
+    {64, 64, 2, 0.156f, 0.32f},  {32, 128, 2, 0.19f, 0.38f},  {64, 128, 2, 0.24f, 0.50f},
+    {128, 128, 1, 0.356f, 0.46f}, {160, 128, 1, 0.43f, 0.60f}, {160, 128, 2, 0.60f, 1.09f},
+    {192, 128, 1, 0.475f, 0.68f}, {128, 256, 1, 0.62f, 0.90f}, {160, 256, 1, 0.76f, 1.12f},
+    {224, 256, 1, 1.00f, 1.52f}, {256, 256, 1, 1.21f, 1.75f}};
+
+int best_shape(int64_t m, int64_t n, int k, int min_bn) {
+  int best = 0;
+  float best_cost = 0.f;
+  for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+    const TileShape& t = kShapes[i];
+    if (t.bn < min_bn) continue;
+    const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    const int64_t slots = 256 * t.per_cu, whole = tiles / slots, rest = tiles % slots;
+    const float step_full = t.full, per_step = (float)(k / kBK);
+    float cost = (float)whole * (per_step * step_full + 3.f);
+    if (rest > 0)
+      cost += per_step * (t.low + (t.full - t.low) * (float)rest / (float)slots) + 3.f;
+    if (best_cost == 0.f || cost < best_cost) {
+      best_cost = cost;
+      best = i;
+    }
+  }
+  return best;
+}
+
+template <Epilogue EPI>
+hipError_t launch_shape(int shape, hipStream_t s, const LinearArgs& a) {
+  switch (shape) {
+    case 0:
+      if constexpr (EPI != kQkRope) return launch_tiles<64, 64, 4, EPI>(s, a);
+      [[fallthrough]];   // (a tile of whole heads is 128 wide at least)
+    case 1: return launch_tiles<32, 128, 4, EPI>(s, a);
+    case 2: return launch_tiles<64, 128, 3, EPI>(s, a);
+    case 3: return launch_tiles<128, 128, 4, EPI>(s, a);
+    case 4: return launch_tiles<160, 128, 4, EPI>(s, a);
+    case 5: return launch_tiles<160, 128, 2, EPI>(s, a);
+    case 6: return launch_tiles<192, 128, 3, EPI>(s, a);
+    case 7: return launch_tiles<128, 256, 3, EPI>(s, a);
+    case 8: return launch_tiles<160, 256, 3, EPI>(s, a);
+    case 9: return launch_tiles<224, 256, 2, EPI>(s, a);
+    default: return launch_tiles<256, 256, 2, EPI>(s, a);
+  }
+}
+
+}  // namespace
+
+namespace nvj {
+
+bool linear_takes(int64_t m, int64_t n, int64_t k) {
+  // 32-bit lane offsets into both operands; whole steps; 16-byte pieces of output
+  return m >= 1 && n >= 8 && n % 8 == 0 && k >= kBK && k % kBK == 0 && m * k * 2 < (1ll << 32) &&
+         n * k * 2 < (1ll << 32) && m * n < (1ll << 40);
+}
+
+hipError_t linear(hipStream_t s, LinearArgs a) {
+  a.group_m = 8;   // 8 x 4 tiles at a time per XCD: 51 -> 42 us for 160 x 256 tiles at 4400 rows
+  return launch_shape<kPlain>(best_shape(a.M, a.N, a.K, 0), s, a);
+}
+hipError_t linear_silu_mul(hipStream_t s, LinearArgs a) {
+  a.group_m = 8;
+  return launch_shape<kSiluMul>(best_shape(a.M, a.N, a.K, 0), s, a);
+}
+hipError_t linear_qk_rope(hipStream_t s, LinearArgs a) {
+  a.group_m = 8;
+  // columns beyond the last head would be taken for one: 256-wide tiles for an even count only
+  int shape = best_shape(a.M, a.N, a.K, 128);
+  if (a.N % kShapes[shape].bn != 0) shape = 4;
+  return launch_shape<kQkRope>(shape, s, a);
+}
+
+hipError_t linear_chained(hipStream_t s, const LinearArgs& a, int chains, int run) {
+  if (chains == 4 && run == 1) return launch_chained<32, 16, 4, 1, 6>(s, a);
+  if (chains == 4 && run == 2) return launch_chained<32, 16, 4, 2, 4>(s, a);
+  if (chains == 2 && run == 4) return launch_chained<32, 16, 2, 4, 4>(s, a);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace nvj

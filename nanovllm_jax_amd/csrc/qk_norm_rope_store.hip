@@ -29,18 +29,11 @@
 
 #include "launch.h"
 #include "nvj_paged_attn.h"
+#include "qk_norm_rope.h"
 
 namespace {
 
 constexpr int kHeadDim = 128;
-
-__device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-  const uint32_t u = __float_as_uint(f);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((u >> 16) | 0x0040u);
-  return (uint16_t)((u + (((u >> 16) & 1u) + 0x7FFFu)) >> 16);
-}
 
 struct QkArgs {
   const uint16_t* qkv;        // [T, >= (Hq+2Hkv)*128] bf16
@@ -62,37 +55,12 @@ struct QkArgs {
   int64_t num_slots;
 };
 
-// sum of the four elements' squares over the 64 elements of the lower half, in the
-// order of a butterfly over l = 4 * lane + e: masks 32 .. 4 are lanes 8 .. 1 apart,
-// masks 2 and 1 elements of a lane
-__device__ __forceinline__ float butterfly(float (&s)[4]) {
-#pragma unroll
-  for (int m = 8; m >= 1; m >>= 1)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], m, 64);
-  return (s[0] + s[2]) + (s[1] + s[3]);
-}
-
-__device__ __forceinline__ void unpack4(uint2 p, float (&f)[4]) {
-  f[0] = __uint_as_float(p.x << 16); f[1] = __uint_as_float(p.x & 0xFFFF0000u);
-  f[2] = __uint_as_float(p.y << 16); f[3] = __uint_as_float(p.y & 0xFFFF0000u);
-}
-__device__ __forceinline__ uint2 pack4(const float (&f)[4]) {
-  return make_uint2(f32_to_bf16_rne(f[0]) | ((uint32_t)f32_to_bf16_rne(f[1]) << 16),
-                    f32_to_bf16_rne(f[2]) | ((uint32_t)f32_to_bf16_rne(f[3]) << 16));
-}
-
 // WIDE: everything is aligned for 8- and 16-byte accesses; otherwise element by
 // element (rows at odd offsets inside a larger buffer).
 template <bool WIDE>
 __device__ __forceinline__ uint2 load4(const uint16_t* p) {
   if (WIDE) return *reinterpret_cast<const uint2*>(p);
   return make_uint2(p[0] | ((uint32_t)p[1] << 16), p[2] | ((uint32_t)p[3] << 16));
-}
-template <bool WIDE>
-__device__ __forceinline__ float4 load4(const float* p) {
-  if (WIDE) return *reinterpret_cast<const float4*>(p);
-  return make_float4(p[0], p[1], p[2], p[3]);
 }
 template <bool WIDE>
 __device__ __forceinline__ void store4(uint16_t* p, uint2 v) {
@@ -108,7 +76,6 @@ __device__ __forceinline__ void store4(uint16_t* p, uint2 v) {
 // Every load that depends on nothing but the (token, head) is issued together.
 template <bool WIDE>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(QkArgs a) {
-#pragma clang fp contract(off)
   const int heads_total = a.num_heads + 2 * a.num_kv_heads;
   const int64_t unit = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   if (unit >= (int64_t)a.num_tokens * heads_total) return;
@@ -123,33 +90,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(QkArgs a) {
   const bool is_k = !is_q && head < a.num_heads + a.num_kv_heads;
   if (is_q || is_k) {
     const float* cs = a.cos_sin + (int64_t)pos * kHeadDim + 4 * i;
-    const float4 c4 = load4<WIDE>(cs), s4 = load4<WIDE>(cs + 64);
-    const float* w = is_q ? a.q_weight : a.k_weight;
-    float x1[4], x2[4];
-    unpack4(lo, x1);
-    unpack4(hi, x2);
-    if (w != nullptr) {
-      const float4 wl = load4<WIDE>(w + 4 * i), wh = load4<WIDE>(w + 64 + 4 * i);
-      const float w1[4] = {wl.x, wl.y, wl.z, wl.w}, w2[4] = {wh.x, wh.y, wh.z, wh.w};
-      float s[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(x2[e], x2[e], x1[e] * x1[e]);
-      const float r = 1.0f / __builtin_sqrtf(butterfly(s) * (1.0f / kHeadDim) + a.eps);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x1[e] = bf16_to_f32(f32_to_bf16_rne(x1[e] * r * w1[e]));
-        x2[e] = bf16_to_f32(f32_to_bf16_rne(x2[e] * r * w2[e]));
-      }
-    }
-    const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
-    float y1[4], y2[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      y1[e] = x1[e] * c[e] - x2[e] * sn[e];
-      y2[e] = x2[e] * c[e] + x1[e] * sn[e];
-    }
-    lo = pack4(y1);
-    hi = pack4(y2);
+    nvj::qk_norm_rope<WIDE>(lo, hi, is_q ? a.q_weight : a.k_weight, a.eps, nvj::load4<WIDE>(cs),
+                            nvj::load4<WIDE>(cs + 64), i);
   }
   auto put = [&](uint16_t* row) {
     store4<WIDE>(row + 4 * i, lo);

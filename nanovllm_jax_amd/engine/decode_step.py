@@ -37,10 +37,10 @@ from ..layers.prefill_attention import paged_prefill_attention
 from ..layers.qk_rope_store import qk_norm_rope_store
 from ..utils.context import AttentionContext, create_decode_context, create_prefill_context
 
-# Up to this many token rows a step runs as the native chain of fused launches
-# (nvj_decoder_step_launch), beyond it as library GEMMs with the element-wise
+# Up to this many token rows a step is one native call (nvj_decoder_step_launch); beyond
+# it, and for models that call is not built for, it is library GEMMs with the element-wise
 # launches between them.
-_NATIVE_STEP_ROWS = 16
+_NATIVE_STEP_ROWS = 1 << 18
 
 __all__ = ["DecodeModelConfig", "DecodeStepRunner", "prepare_block_tables", "prepare_decode",
            "prepare_prefill", "advance_decode"]
@@ -278,7 +278,7 @@ class DecodeStepRunner:
             layers = (_lib.DecoderLayer * c.num_layers)(
                 *[_lib.DecoderLayer(*key[3 + per * i:3 + per * (i + 1)])
                   for i in range(c.num_layers)])
-            if _lib.load().nvj_decoder_step_workspace_bytes(ctypes.byref(model), 1) > 0:
+            if _lib.load().nvj_decoder_step_workspace_bytes(ctypes.byref(model), 1, 1) > 0:
                 built = (model, layers)
         self._native_model = (key, built)
         return built
@@ -309,7 +309,7 @@ class DecodeStepRunner:
             return None
         if prefill:
             if context.cu_seqlens_k.shape[0] != sequences + 1 or \
-                    not 0 < sequences <= _NATIVE_STEP_ROWS:
+                    sequences == 0:
                 return None
         elif context.context_lens.shape != (tokens,):
             return None
@@ -339,7 +339,7 @@ class DecodeStepRunner:
         logits = torch.empty((sequences, model.vocab), dtype=torch.bfloat16, device=dev)
         b.logits = logits.data_ptr()
         lib = _lib.load()
-        need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens)
+        need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens, sequences)
         scratch = torch.empty(need, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
             code = lib.nvj_decoder_step_launch(

@@ -12,19 +12,22 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,hidden,inter,heads", [(1, 256, 256, 2), (4, 512, 768, 4),
                                                      (5, 1024, 3072, 16), (16, 1024, 512, 8),
-                                                     (16, 2048, 2560, 24)])
+                                                     (16, 2048, 2560, 24), (17, 512, 512, 4),
+                                                     (33, 1024, 768, 6), (128, 256, 256, 2),
+                                                     (129, 320, 448, 6), (300, 1024, 3072, 16),
+                                                     (1100, 1024, 512, 8)])
 @pytest.mark.parametrize("kind", ["decode", "packed", "paged"])
 def test_native_step_equals_the_long_way(rows, hidden, inter, heads, kind, monkeypatch):
     print(f"case native step rows={rows} hidden={hidden} {kind}", flush=True)
     from nanovllm_jax_amd.engine import decode_step as ds
     cfg = ds.DecodeModelConfig(num_layers=2, hidden_size=hidden, num_heads=heads, num_kv_heads=2,
                                head_dim=128, intermediate_size=inter, vocab_size=1000,
-                               max_position=1024, block_size=64, num_kvcache_blocks=80)
+                               max_position=2048, block_size=64, num_kvcache_blocks=2 * rows + 60)
     runner = ds.DecodeStepRunner(cfg, "cuda:0", seed=rows)
     rng = np.random.Generator(np.random.PCG64(rows))
     pages = rng.permutation(cfg.num_kvcache_blocks).tolist()
     if kind == "decode":
-        lens = rng.integers(1, 250, rows).tolist()
+        lens = rng.integers(1, 100, rows).tolist()
     else:                                     # new rows: one long prompt and short ones
         lens = [rows] if rows < 5 else [rows - 3, 2, 1]
     cached = [37] * len(lens) if kind == "paged" else [0] * len(lens)
