@@ -292,3 +292,40 @@ def test_attention_layer_prefill_with_cached_prefix():
                 bits_to_torch(v_new[last], dev), dctx)
     torch.cuda.synchronize()
     assert_close_bf16(torch_to_bits(dout), want[last], what="decode == last chunk row")
+
+
+@pytest.mark.parametrize("batch,Hq,Hkv", [(5, 8, 8), (70, 6, 2), (200, 8, 4)])
+def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
+    """Cached prefixes of very different lengths: tiles are handed out by the keys they walk.
+    Sequences without new tokens, without a prefix, and tiles that tie among them."""
+    print(f"case paged prefill longest first batch={batch} Hq={Hq}", flush=True)
+    import torch
+    from nanovllm_jax_amd import paged_prefill_attention
+    rng = np.random.Generator(np.random.PCG64(batch))
+    new = rng.integers(1, 60, batch)
+    cached = rng.integers(0, 300, batch)
+    new[[0, 1, batch // 2]], cached[[0, 1, batch // 2]] = [17, 300, 0], [1500, 0, 900]
+    total, page = new + cached, 32
+    pages = -(-total // page)
+    ids = rng.permutation(int(pages.sum()))
+    table = np.full((batch, int(pages.max())), -1, np.int32)
+    for i, e in enumerate(np.cumsum(pages)):
+        table[i, :pages[i]] = ids[e - pages[i]:e]
+    dev = "cuda:0"
+    g = torch.Generator(device=dev)
+    g.manual_seed(batch)
+    kc, vc = (torch.randn(int(pages.sum()), page, Hkv, 128, generator=g, device=dev)
+              .to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(int(new.sum()), Hq, 128, generator=g, device=dev).to(torch.bfloat16)
+    cu = lambda n: torch.from_numpy(np.concatenate([[0], np.cumsum(n)]).astype(np.int32)).to(dev)
+    got = paged_prefill_attention(q, kc, vc, torch.from_numpy(table).to(dev), cu(new), cu(total),
+                                  128 ** -0.5)
+    # every sequence on its own: one launch each, where there is nothing to order
+    at = np.concatenate([[0], np.cumsum(new)])
+    for i in range(batch):
+        if new[i] == 0:
+            continue
+        one = paged_prefill_attention(q[at[i]:at[i + 1]].contiguous(), kc, vc,
+                                      torch.from_numpy(table[i:i + 1].copy()).to(dev),
+                                      cu(new[i:i + 1]), cu(total[i:i + 1]), 128 ** -0.5)
+        assert torch.equal(got[at[i]:at[i + 1]], one), f"sequence {i}"
