@@ -244,6 +244,12 @@ NVJ_API int nvj_paged_decode_launch(void* stream,
  * rows (see chunk == 0 above): the equal cut with shared rows is taken whatever
  * the lengths.  Same results to the same tolerance; a measurement and test aid.
  *
+ * NVJ_PHASE_SHORT_ROWS, or-ed in, lets a small launch of the balanced split (no more
+ * (sequence, KV head) rows than compute units) finish each row inside one workgroup
+ * where the lengths say that this is faster than sharing rows.  Same results to the
+ * same tolerance; without it the way rows are cut depends on the lengths alone as
+ * chunk == 0 describes, and with it the last bits.
+ *
  * NVJ_PHASE_VALU_PRODUCTS, or-ed in, runs a measurement variant of the split-K
  * kernel that computes Q.K and P.V with vector-ALU dot products instead of the
  * matrix cores, so that the choice between the two can be timed on any
@@ -264,6 +270,7 @@ NVJ_API int nvj_paged_decode_launch(void* stream,
 #define NVJ_PHASE_CLEAR_COUNTERS 8u
 #define NVJ_PHASE_LOADS_ONLY 16u
 #define NVJ_PHASE_SHARED_ROWS 32u
+#define NVJ_PHASE_SHORT_ROWS 64u
 NVJ_API int nvj_paged_decode_launch_phases(void* stream,
                             const void* q, const void* k_cache, const void* v_cache,
                             const int32_t* block_tables, const int32_t* context_lens,

@@ -127,6 +127,7 @@ NVJ_PHASE_VALU_PRODUCTS = 4
 NVJ_PHASE_CLEAR_COUNTERS = 8
 NVJ_PHASE_LOADS_ONLY = 16
 NVJ_PHASE_SHARED_ROWS = 32
+NVJ_PHASE_SHORT_ROWS = 64
 
 _lock = threading.Lock()
 _lib = None

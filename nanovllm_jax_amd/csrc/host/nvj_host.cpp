@@ -146,7 +146,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                      stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(), table_ptr, lens_ptr,
                      out.data_ptr(), partials, partial_bytes, counters, counter_bytes, batch, heads,
                      c.heads, c.dim, c.page, max_blocks, c.num_blocks, (float)scale, c.dtype,
-                     NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE)
+                     NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE | NVJ_PHASE_SHORT_ROWS)
                : nvj_paged_decode_launch_phases(
                      stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(), table_ptr, lens_ptr,
                      out.data_ptr(), nullptr, 0, batch, heads, c.heads, c.dim, c.page, max_blocks,

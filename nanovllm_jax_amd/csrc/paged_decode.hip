@@ -816,6 +816,49 @@ __device__ __forceinline__ void write_output(const DecodeArgs& a, int b, int kvh
   }
 }
 
+// Result of a row that the 8 waves of a workgroup have walked in 8 parts: every part lies
+// in the K tile of its wave as add_partial_from_lds expects it, and wave w merges and
+// writes its eighth of the head dimensions (4 in every 32), each value by the recurrence
+// of add_partial_from_lds over the parts in order: the same bits as one wave merging all
+// of it, without its 7 x 34 LDS reads in a row (6.7 -> 5.7 us for rows of 256 positions;
+// not in the balanced kernel, whose registers it does not fit).
+template <int D, bool F16, int TILE>
+__device__ __forceinline__ void merge_parts_and_write(const DecodeArgs& a, uint4 (&k_tile)[8][TILE],
+                                                      int b, int kvh, int wave, int lane) {
+  constexpr int STRIDE = D / 32 * 16;
+  const int r = lane & 15, kg = lane >> 4;
+  if (r >= a.group || 32 * kg >= D) return;
+  const int e = wave >> 1, jd = 4 * (wave & 1);
+  float v[8][4], ml[8][2];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    const float* t = reinterpret_cast<const float*>(k_tile[p]) + lane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[p][i] = t[(4 * (jd + i) + e) * STRIDE];
+    ml[p][0] = t[32 * STRIDE];
+    ml[p][1] = t[33 * STRIDE];
+  }
+  float m_run = ml[0][0], l_run = ml[0][1];
+  float acc[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
+#pragma unroll
+  for (int p = 1; p < 8; ++p) {
+    const float m_new = fmaxf(m_run, ml[p][0]);
+    const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+    const float w = __builtin_amdgcn_exp2f((ml[p][0] - m_new) * a.scale_log2e);
+    m_run = m_new;
+    l_run = fmaf(l_run, keep, w * ml[p][1]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = fmaf(acc[i], keep, w * v[p][i]);
+  }
+  const float inv = 1.0f / (l_run + 1e-9f);
+  uint2 o;
+  o.x = Elem<F16>::pack2(acc[0] * inv, acc[1] * inv);
+  o.y = Elem<F16>::pack2(acc[2] * inv, acc[3] * inv);
+  const int head = kvh * a.group + r;
+  reinterpret_cast<uint2*>(a.out + ((int64_t)b * a.num_heads + head) * HeadDim<D>::kPieces)
+      [8 * kg + 2 * e + (wave & 1)] = o;
+}
+
 // Unnormalised partial (D f32 per head) + (max, sum) to the workspace.  A
 // partial record is D + 2 floats of one query head; `rec_base` is the record of
 // the first query head of this wave's KV head.
@@ -909,8 +952,9 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
   if (parts > 1) {
     // value v of lane l at float v * kLanesWithDims + l of the wave's tile
     const bool holds_dims = lane < kLanesWithDims;
+    const bool all_merge = NW == 8 && hpw == 1;
     __syncthreads();   // every wave is done reading its K tile
-    if (part > 0 && holds_dims) {
+    if ((part > 0 || all_merge) && holds_dims) {
       float* mine = reinterpret_cast<float*>(k_tile[wave]) + lane;
 #pragma unroll
       for (int jd = 0; jd < 8; ++jd)
@@ -920,6 +964,12 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
       mine[33 * kLanesWithDims] = l_run;
     }
     __syncthreads();
+    if constexpr (NW == 8) {
+      if (all_merge) {
+        merge_parts_and_write<D, F16>(a, k_tile, b, kvh, wave, lane);
+        return;
+      }
+    }
     if (part > 0) return;
     if (holds_dims) {
       for (int p = 1; p < parts; ++p) {
@@ -1285,6 +1335,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
                                                                     int num_wgs, int min_steps,
                                                                     int hpw, int wr_hpw, int wr_hpw_alt,
                                                                     int wr_tol, int shift,
+                                                                    int short_rows,
                                                                     int32_t* counters) {
   using H = HeadDim<D>;
   constexpr int NW = 8;
@@ -1341,7 +1392,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
       int mine = kept_ctx[0];
 #pragma unroll
       for (int k = 1; k < kKeep; ++k) mine = (b >> 6) == k ? kept_ctx[k] : mine;
-      c = __shfl(mine, b & 63, 64);
+      c = __builtin_amdgcn_readlane(mine, b & 63);
     } else {
       c = min(as_constant(a.context_lens)[b], cap);
     }
@@ -1350,6 +1401,29 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
       for (int i = threadIdx.x; i < a.num_heads * H::kPieces; i += NW * 64)
         orow[i] = make_uint4(0u, 0u, 0u, 0u);
     }
+  }
+
+  // -------------------------------------------------------------------------
+  // Short rows: one KV head of one sequence per workgroup, with no more rows than CUs.
+  // Publishing partials and merging them costs 5-7 us of a small launch, as much as two
+  // rounds of a workgroup's 8 waves over their steps cost it: measured (1 .. 32
+  // sequences of 64 .. 8192 positions, 8 KV heads) rows take 5.7 us + 3.2 per round,
+  // whatever their number (a CU draws 47 GB/s, with any number of loads in flight), the
+  // equal cut 10 us + 2.4 per 1000 wave steps.  4 sequences of 64 / 256 / 512 positions
+  // 10.7 / 11.5 / 11.8 us with the equal cut, 5.3 / 8.4 / 10.0 this way; 32 of 2048
+  // positions 50.1 / 47.  (Tables that hold no more than two rounds go to
+  // paged_decode_whole_kernel at once.)
+  // The row is walked below as a workgroup's run inside one row is: parts meet in LDS.
+  // -------------------------------------------------------------------------
+  bool short_row = false;
+  if (short_rows > 0) {
+    int longest = 0;
+#pragma unroll
+    for (int k = 0; k < kKeep; ++k) longest = max(longest, kept_ctx[k]);
+    const int rounds = (wave_max(longest) + NW * kStep - 1) / (NW * kStep);
+    short_row = rounds <= 2 || (int64_t)rounds * 1333 < 1792 + (int64_t)a.num_kv_heads * total;
+    if (g >= (short_row ? short_rows : num_wgs)) return;
+    if (short_row) hpw = 1;
   }
 
   // -------------------------------------------------------------------------
@@ -1367,7 +1441,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
   // round, by decreasing length, which pairs long rows with short ones.  Every
   // wave of the launch reads the same lengths and takes the same decision.
   // -------------------------------------------------------------------------
-  if (wr_hpw > 0 && total > 0) {
+  if (wr_hpw > 0 && total > 0 && !short_row) {
     // every wave writes all the lengths and step counts itself (the same values
     // from each), so no wave has to wait for another before it reads them back
     int key[kKeep];
@@ -1575,10 +1649,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
   cut.shift = shift;
   cut.units = (cut.axis + (1 << shift) - 1) >> shift;
   cut.nsub = max(1, min(num_wgs * parts, cut.units / min_steps));
-  if (cut.axis == 0 || g * parts >= cut.nsub) return;
-  const int nparts = min(parts, cut.nsub - g * parts);   // parts of this workgroup that have work
-  const int start = cut.start_of(g * parts);
-  const int end = cut.start_of(g * parts + nparts);
+  if (!short_row && (cut.axis == 0 || g * parts >= cut.nsub)) return;
 
   // the sequence whose rows hold axis position x: its index, the steps before
   // it and its length (all wave-uniform)
@@ -1594,8 +1665,8 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
       if (hit != 0ull) {
         const int src = __builtin_ctzll(hit);
         b = k * 64 + src;
-        before = __shfl(kept_excl[k], src, 64);
-        ctx = __shfl(kept_ctx[k], src, 64);
+        before = __builtin_amdgcn_readlane(kept_excl[k], src);
+        ctx = __builtin_amdgcn_readlane(kept_ctx[k], src);
         found = true;
       }
     }
@@ -1610,8 +1681,8 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
         if (hit != 0ull) {
           const int src = __builtin_ctzll(hit);
           b = base + src;
-          before = __shfl(running + incl - n, src, 64);
-          ctx = __shfl(c, src, 64);
+          before = __builtin_amdgcn_readlane(running + incl - n, src);
+          ctx = __builtin_amdgcn_readlane(c, src);
           break;
         }
         running += __builtin_amdgcn_readlane(incl, 63);
@@ -1622,14 +1693,33 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
     ctx = __builtin_amdgcn_readfirstlane(ctx);
   };
 
-  int b0, before0, ctx0;
-  locate(start, b0, before0, ctx0);
-  if (b0 >= batch || ctx0 <= 0) return;   // cannot happen when the prefix sums are right
+  int b0, before0, ctx0, nparts, start, end, hg0, row0, xs, xe;
+  if (short_row) {
+    b0 = g / a.num_kv_heads;
+    hg0 = g - b0 * a.num_kv_heads;
+    int mine = kept_ctx[0];
+#pragma unroll
+    for (int k = 1; k < kKeep; ++k) mine = (b0 >> 6) == k ? kept_ctx[k] : mine;
+    ctx0 = __builtin_amdgcn_readlane(mine, b0 & 63);
+    if (ctx0 <= 0) return;   // (an empty sequence's zeros are written)
+    before0 = start = row0 = 0;
+    end = (ctx0 + kStep - 1) / kStep;
+    nparts = min(NW, end);
+    xs = part < nparts ? part * end / nparts : end;
+    xe = part < nparts ? (part + 1) * end / nparts : end;
+  } else {
+    nparts = min(parts, cut.nsub - g * parts);   // parts of this workgroup that have work
+    start = cut.start_of(g * parts);
+    end = cut.start_of(g * parts + nparts);
+    locate(start, b0, before0, ctx0);
+    if (b0 >= batch || ctx0 <= 0) return;   // cannot happen when the prefix sums are right
+    const int nb = (ctx0 + kStep - 1) / kStep;
+    hg0 = (start - rows_per_seq * before0) / nb;
+    row0 = rows_per_seq * before0 + hg0 * nb;   // axis position of the row's step 0
+    xs = part < nparts ? cut.start_of(g * parts + part) : end;
+    xe = part < nparts ? cut.start_of(g * parts + part + 1) : end;
+  }
   const int nb0 = (ctx0 + kStep - 1) / kStep;
-  const int hg0 = (start - rows_per_seq * before0) / nb0;
-  const int row0 = rows_per_seq * before0 + hg0 * nb0;   // axis position of the row's step 0
-  const int xs = part < nparts ? cut.start_of(g * parts + part) : end;
-  const int xe = part < nparts ? cut.start_of(g * parts + part + 1) : end;
   const int64_t subrun = (int64_t)g * parts + part;
   // Does the whole run of the workgroup lie inside one row?  Then every wave has
   // at most one segment, and the parts of a head meet in LDS before anything is
@@ -2069,10 +2159,23 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
   a.num_blocks = num_blocks;
   a.scale_log2e = scale * kLog2e;
 
-  if (whole && max_blocks > 0) {
-    if ((int64_t)batch * num_kv_heads > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
+  // Short rows: a workgroup per (sequence, KV head), if the CUs and the lengths a wave
+  // keeps allow it.  Where the table itself rules longer rows out, no length needs to be
+  // looked at and the kernel without a split does it (64 / 256 / 512 positions 5.2 / 5.8
+  // / 7.5 us against 5.3 / 8.4 / 10.0 by way of the balanced kernel); otherwise that one
+  // decides on the device.
+  const int64_t all_rows = (int64_t)batch * num_kv_heads;
+  const int short_rows = chunk == 0 && (phases & NVJ_PHASE_SHORT_ROWS) &&
+                                 !(phases & NVJ_PHASE_SHARED_ROWS) && batch <= kKeptSequences &&
+                                 all_rows <= compute_units()
+                             ? (int)all_rows
+                             : 0;
+  const bool all_short = short_rows > 0 && (int64_t)max_blocks * block_size <= 2 * 8 * kStep &&
+                         !(phases & NVJ_PHASE_CLEAR_COUNTERS);
+  if ((whole || all_short) && max_blocks > 0) {
+    if (all_rows > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
     if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;   // there is no second pass
-    const int hpw = heads_per_workgroup(batch, num_kv_heads);
+    const int hpw = all_short ? 1 : heads_per_workgroup(batch, num_kv_heads);
     const dim3 grid((unsigned)(batch * (num_kv_heads / hpw))), block(512);
     hipError_t rc;
     if (loads_only) rc = nvj::launch(paged_decode_whole_kernel<8, 128, false, -1>, grid, block, s, a, hpw);
@@ -2106,13 +2209,13 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
           return NVJ_ERR_LAUNCH;
       }
       if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;
-      const dim3 grid((unsigned)plan.num_wgs);
+      const dim3 grid((unsigned)(short_rows > plan.num_wgs ? short_rows : plan.num_wgs));
       hipError_t rc;
 #define NVJ_LAUNCH_BALANCED(DV, F16V, VGV)                                                     \
   rc = nvj::launch(paged_decode_balanced_kernel<DV, F16V, VGV>, grid, dim3(512), s, a, batch, \
                    plan.num_wgs, kMinBalancedSteps, plan.hpw,                      \
                    (phases & NVJ_PHASE_SHARED_ROWS) ? 0 : plan.wr_hpw, plan.wr_hpw_alt,       \
-                   kWholeRowTolerance, plan.shift, counters)
+                   kWholeRowTolerance, plan.shift, short_rows, counters)
       if (loads_only) NVJ_LAUNCH_BALANCED(128, false, -1);
       else if (valu && group == 4) NVJ_LAUNCH_BALANCED(128, false, 4);
       else if (valu) NVJ_LAUNCH_BALANCED(128, false, 8);

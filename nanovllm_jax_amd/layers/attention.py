@@ -180,7 +180,9 @@ class Attention:
         q = q.to(self.k_cache.dtype)      # layers/attention.py:386-387
         return paged_attention(q, self.k_cache, self.v_cache, context.block_tables,
                                context.context_lens, self.scale, self.block_size,
-                               chunk=context.decode_split, workspace=self.workspace)
+                               chunk=context.decode_split, workspace=self.workspace,
+                               phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+                               | _lib.NVJ_PHASE_SHORT_ROWS)
 
     def _native_call(self, q, k, v, context: AttentionContext):
         """The ordinary call in native code; None when it is not one (see

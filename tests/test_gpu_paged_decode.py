@@ -989,3 +989,26 @@ def test_balanced_split_with_a_very_wide_block_table(B, Hq, Hkv, bs, MB):
     torch.cuda.synchronize()
     assert_close_bf16(torch_to_bits(out), oracle(q, kc, vc, bt, ctx, 0.088, bs),
                       what=f"wide table B={B}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(16, 8, 128), (4, 1, 64), (32, 32, 128)])
+@pytest.mark.parametrize("lens", [[0, 1, 255, 256, 257, 512], [513, 5, 3], [700], [40] * 8,
+                                  [1500, 1480, 1490, 1501, 3, 1499, 1460, 1500]])
+def test_short_rows(lens, Hq, Hkv, D):
+    """Rows finished inside one workgroup (NVJ_PHASE_SHORT_ROWS) around the lengths where
+    the choice flips, with empty sequences, and against the equal cut on the same data."""
+    print(f"case short rows lens={lens} Hq={Hq} Hkv={Hkv} D={D}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    bs = 64
+    NB = sum(-(-n // bs) for n in lens) + 3
+    q, kc, vc, bt, ctx = make_problem(31 + len(lens), len(lens), Hq, Hkv, D, bs, NB, lens)
+    scale = 1.0 / np.sqrt(D)
+    want = oracle(q, kc, vc, bt, ctx, scale, bs)
+    dev = "cuda:0"
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)] + [torch.from_numpy(x).to(dev) for x in (bt, ctx)]
+    both = _lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+    for extra in (_lib.NVJ_PHASE_SHORT_ROWS, 0, _lib.NVJ_PHASE_SHORT_ROWS | _lib.NVJ_PHASE_SHARED_ROWS):
+        got = paged_attention(*t, scale, bs, phases=both | extra)
+        torch.cuda.synchronize()
+        assert_close_bf16(torch_to_bits(got), want, what=f"lens={lens} phases={extra}")
