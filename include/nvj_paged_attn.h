@@ -364,6 +364,29 @@ NVJ_API int nvj_paged_decode_static_launch(void* stream,
                             int32_t num_blocks, float scale, int32_t dtype);
 
 /*
+ * nvj_store_kvcache_launch of the batch's new rows (key, value [batch, num_kv_heads,
+ * head_dim], slot_mapping [batch]) and the decode attention behind it, in one launch with
+ * the same results: attention sees every new row wherever its slot lies.  For chunk 0
+ * (counters and partials as nvj_paged_decode_launch_counters; counters NULL on the null
+ * stream: words of the library's that only such calls use) and NVJ_CHUNK_WHOLE_SEQUENCE.
+ * nvj_paged_decode_store_takes says whether the sizes allow it: 0 no (more than 64 rows or
+ * more than one KV head of a row per compute unit, head_dim other than 128, a fixed chunk:
+ * NVJ_ERR_UNSUPPORTED), 1 yes, and counters and partials are not used, 2 yes.
+ */
+NVJ_API int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads,
+                            int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                            int32_t max_blocks, int32_t num_blocks, int32_t chunk);
+NVJ_API int nvj_paged_decode_store_launch(void* stream, const void* q, const void* key,
+                            const void* value, const int32_t* slot_mapping, void* k_cache,
+                            void* v_cache, const int32_t* block_tables,
+                            const int32_t* context_lens, void* out, void* partials,
+                            size_t partial_bytes, void* counters, size_t counter_bytes,
+                            int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                            int32_t head_dim, int32_t block_size, int32_t max_blocks,
+                            int32_t num_blocks, float scale, int32_t chunk, int32_t dtype,
+                            int32_t k_dtype, int32_t v_dtype);
+
+/*
  * Fused per-head QK-RMSNorm + rotary embedding + KV-cache store: everything the
  * reference runs between the QKV projection and the attention call, in one
  * launch.  Replaces q_norm / k_norm (models/qwen3.py:157-160,

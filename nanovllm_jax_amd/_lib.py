@@ -77,6 +77,10 @@ SYMBOLS = {
         _c.c_void_p, _c.c_void_p, _c.c_size_t, _c.c_void_p, _c.c_size_t,
         _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int32, _c.c_int32,
         _c.c_int32, _c.c_float, _c.c_int32, _c.c_uint32]),
+    "nvj_paged_decode_store_takes": (_c.c_int32, [_c.c_int32] * 8),
+    "nvj_paged_decode_store_launch": (_c.c_int, [_c.c_void_p] * 11 + [
+        _c.c_size_t, _c.c_void_p, _c.c_size_t] + [_c.c_int32] * 7 + [_c.c_float] +
+        [_c.c_int32] * 4),
     "nvj_paged_decode_counters_reset": (_c.c_int, [_c.c_void_p, _c.c_void_p, _c.c_size_t]),
     "nvj_paged_decode_library_counters": (_c.c_int, [_c.POINTER(_c.c_void_p),
                                                      _c.POINTER(_c.c_size_t)]),

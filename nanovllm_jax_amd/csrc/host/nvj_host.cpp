@@ -111,18 +111,26 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   size_t partial_bytes = 0, counter_bytes = 0, clear_bytes = 0;
   Tensor own;
   const Tensor *given, *given_counters;
-  if (chunk == 0) {
+  // store and attention in one launch: 0 not for these sizes, 1 without counters, 2 with
+  int together = nvj_paged_decode_store_takes(batch, heads, c.heads, c.dim, c.page, max_blocks,
+                                              c.num_blocks, chunk);
+  if (chunk == 0 && together != 1) {
     const size_t need = nvj_paged_decode_workspace_bytes(batch, heads, c.dim, max_blocks, c.page,
                                                          c.heads, 0);
     const size_t head = nvj_paged_decode_counter_bytes(batch, heads, c.heads);
     if (need == 0) Py_RETURN_NONE;
     if (args[11] == Py_None) {
-      // a workspace for this call alone: the store clears its counters on the way
+      // a workspace for this call alone; its counters are cleared by the store, unless the
+      // library has some for this stream
       own = at::empty({(int64_t)need}, q->options().dtype(at::kByte));
-      counters = own.data_ptr();
-      counter_bytes = clear_bytes = head;
-      partials = static_cast<char*>(counters) + head;
+      char* base = static_cast<char*>(own.data_ptr());
+      partials = base + head;
       partial_bytes = need - head;
+      if (stream != nullptr) together = 0;
+      if (together == 0) {
+        counters = base;
+        counter_bytes = clear_bytes = head;
+      }
     } else {
       if (!get(args[11], &given) || !get(args[12], &given_counters) ||
           given->device() != q->device() || given_counters->device() != q->device() ||
@@ -136,11 +144,21 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
   }
   Tensor out = at::empty_like(*q);
-  int code = store(stream, *key, *value, c, *slots, nullptr, nullptr, clear_bytes ? counters : nullptr,
+  const int32_t* table_ptr = static_cast<const int32_t*>(tables->data_ptr());
+  const int32_t* lens_ptr = static_cast<const int32_t*>(lens->data_ptr());
+  int code;
+  if (together != 0) {
+    code = nvj_paged_decode_store_launch(
+        stream, q->data_ptr(), key->data_ptr(), value->data_ptr(),
+        static_cast<const int32_t*>(slots->data_ptr()), c.k->data_ptr(), c.v->data_ptr(), table_ptr,
+        lens_ptr, out.data_ptr(), partials, partial_bytes, counters, counter_bytes, batch, heads,
+        c.heads, c.dim, c.page, max_blocks, c.num_blocks, (float)scale, chunk, c.dtype,
+        type_code(key->scalar_type()), type_code(value->scalar_type()));
+    return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+  }
+  code = store(stream, *key, *value, c, *slots, nullptr, nullptr, clear_bytes ? counters : nullptr,
                    clear_bytes);
   if (code == NVJ_OK) {
-    const int32_t* table_ptr = static_cast<const int32_t*>(tables->data_ptr());
-    const int32_t* lens_ptr = static_cast<const int32_t*>(lens->data_ptr());
     code = chunk == 0
                ? nvj_paged_decode_launch_counters(
                      stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(), table_ptr, lens_ptr,

@@ -38,6 +38,7 @@
 
 #include <atomic>
 
+#include "cache_rows.h"
 #include "launch.h"
 #include "nvj_paged_attn.h"
 
@@ -209,16 +210,65 @@ struct DecodeArgs {
   float scale_log2e;
 };
 
+// The new K/V rows of the step, stored by the same launch (NEW kernels: head_dim 128, up to
+// 64 rows).  A store kernel in front of the attention is 2.8 us that a small call waits
+// for.  Here nobody waits for the rows to arrive in the cache: a wave that walks 32 slots
+// of the cache with a new row among them takes that row from `key` and `value` instead
+// (compute_segment).  One compare per step against the slots of all the rows, one per lane,
+// finds it, so that any slot mapping means what it means with the store in front, rows of
+// one sequence in several batch entries included.
+struct NewRows {
+  const void* key;       // [B, Hkv, 128], the cache's type or float32
+  const void* value;
+  const int32_t* slots;  // [B]; < 0 or >= num_slots: not stored
+  int num_slots;
+  bool key_f32, value_f32;
+  int main_wgs;          // workgroups behind these store a row each; 0: workgroup b stores row b
+};
+constexpr int kMaxNewRows = 64;
+
+template <bool F16>
+__device__ __forceinline__ uint4 new_piece(const void* rows, bool f32, int64_t piece) {
+  return f32 ? nvj::load_piece_as_cache_type<true, F16>(rows, piece)
+             : nvj::load_piece_as_cache_type<false, F16>(rows, piece);
+}
+
+// This lane's new slot (of row `lane`), -1 where there is none.
+__device__ __forceinline__ int new_slot_of_lane(const NewRows& n, int batch, int lane) {
+  const int slot = lane < batch ? n.slots[lane] : -1;
+  return slot < n.num_slots ? max(slot, -1) : -1;
+}
+
+// Row `row` into the cache, by one workgroup of `threads` threads.
+template <bool F16>
+__device__ __forceinline__ void store_new_row(const DecodeArgs& a, const NewRows& n, int row,
+                                              int threads) {
+  const int64_t slot = n.slots[row];
+  if (slot < 0 || slot >= n.num_slots) return;
+  const int pieces = a.cache_kv_heads * (kMaxHeadDim / 8);
+  for (int p = threadIdx.x; p < 2 * pieces; p += threads) {
+    const bool is_k = p < pieces;
+    const int at = is_k ? p : p - pieces;
+    char* cache = const_cast<char*>(is_k ? a.k_cache : a.v_cache);
+    reinterpret_cast<uint4*>(cache)[slot * pieces + at] =
+        is_k ? new_piece<F16>(n.key, n.key_f32, (int64_t)row * pieces + at)
+             : new_piece<F16>(n.value, n.value_f32, (int64_t)row * pieces + at);
+  }
+}
+
 // One wave's share of one segment: positions [t0, t1) of sequence b for KV head
 // kvh; t0 is a multiple of 32, t0 < t1.  Leaves the unnormalised result in
 // registers: acc[jd][e] is O[head kvh*group + r][dim 32*kg + 8*e + jd] for the
 // lane (r = lane & 15, kg = lane >> 4), m_run the maximum raw score and l_run
 // the sum of exp((score - m_run) * scale) of that head (the same in the four
 // lanes that share r).  Lanes with r >= group hold padding.
-template <int D, bool F16>
+// NEW: `new_slot` is new_slot_of_lane.
+template <int D, bool F16, bool NEW = false>
 __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds, int b, int kvh,
                                                 int t0, int t1, int lane, f32x4 (&acc)[8],
-                                                float& m_run, float& l_run) {
+                                                float& m_run, float& l_run,
+                                                const NewRows* fresh = nullptr,
+                                                int new_slot = -1) {
   using H = HeadDim<D>;
   const int r = lane & 15;   // MFMA row/column index inside a 16-wide tile
   const int kg = lane >> 4;  // MFMA k-group (which 8 of the 32 reduction slots)
@@ -251,17 +301,26 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
   const int64_t head_bytes = (int64_t)(kvh / a.kv_rep) * (D * 2);
   const const_i32_ptr table = as_constant(a.block_tables + (int64_t)b * a.max_blocks);
 
-  // wave-uniform byte offset of the first position of a step inside the cache
-  auto step_base = [&](int step) -> int64_t {
+  // wave-uniform place of the first position of a step in the cache: its slot if NEW, else
+  // its byte offset at once
+  auto step_place = [&](int step) -> int64_t {
     const int ts = t0 + step * kStep;
     const int page = ts / block_size;
     const int phys = min(max(table[page], 0), num_blocks - 1);
-    return ((int64_t)phys * block_size + (ts - page * block_size)) * row_bytes + head_bytes;
+    const int64_t slot = (int64_t)phys * block_size + (ts - page * block_size);
+    return NEW ? slot : slot * row_bytes + head_bytes;
+  };
+  auto offset_of = [&](int64_t place) { return NEW ? place * row_bytes + head_bytes : place; };
+  // NEW: this KV head's piece of a new row
+  auto fresh_piece = [&](int row, int piece) {
+    return ((int64_t)row * a.cache_kv_heads + kvh / a.kv_rep) * H::kPieces + piece;
   };
 
   uint4 kreg[H::kKLoads], vreg[8];
+  int64_t place;   // of the step at hand
   {
-    const int64_t off = step_base(0);
+    place = step_place(0);
+    const int64_t off = offset_of(place);
     const int last = min(kStep, t1 - t0) - 1;
     issue_k_loads<true, D>(kreg, k_cache + off, lane, last, row_bytes);
     issue_v_loads<true, D>(vreg, v_cache + off, kg, r, last, row_bytes);
@@ -274,20 +333,42 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
 
   // the page lookup of a step is started two steps ahead, so that its latency
   // is not in front of the loads that need the address
-  int64_t off_ahead = nsteps > 1 ? step_base(1) : 0;
+  int64_t place_ahead = nsteps > 1 ? step_place(1) : 0;
   for (int step = 0; step < nsteps; ++step) {
     const int nvalid = min(kStep, t1 - (t0 + step * kStep));
     const bool more = step + 1 < nsteps;
-    const int64_t next_off = off_ahead;
+    const int64_t next_place = place_ahead, next_off = offset_of(next_place);
     int next_last = kStep - 1;
     if (more) next_last = min(kStep, t1 - (t0 + (step + 1) * kStep)) - 1;
-    if (step + 2 < nsteps) off_ahead = step_base(step + 2);
+    if (step + 2 < nsteps) place_ahead = step_place(step + 2);
+
+    // the new rows among this step's positions; the pieces of the first are asked for here
+    // already, while the step's own loads are still on their way
+    unsigned long long hits = 0;
+    uint4 fresh_k, fresh_v;
+    if constexpr (NEW) {
+      hits = __ballot((uint32_t)(new_slot - (int)place) < (uint32_t)nvalid);
+      if (hits != 0) {
+        const int64_t piece = fresh_piece(__builtin_ctzll(hits), r);
+        fresh_k = new_piece<F16>(fresh->key, fresh->key_f32, piece);
+        fresh_v = new_piece<F16>(fresh->value, fresh->value_f32, piece);
+      }
+    }
 
     // ---- K: registers -> LDS (row = position, padded), then next K loads ----
 #pragma unroll
     for (int i = 0; i < H::kKLoads; ++i)
       lds[(H::kPosPerLoad * i + lane / H::kPieces) * H::kLdsRowPieces + lane % H::kPieces] =
           kreg[i];
+    if constexpr (NEW) {
+      for (unsigned long long h = hits; h != 0; h &= h - 1) {
+        const int row = __builtin_ctzll(h);
+        const int pos = __builtin_amdgcn_readlane(new_slot, row) - (int)place;
+        const uint4 piece = h == hits ? fresh_k : new_piece<F16>(fresh->key, fresh->key_f32,
+                                                                 fresh_piece(row, r));
+        if (kg == 0) lds[pos * H::kLdsRowPieces + r] = piece;
+      }
+    }
     // Other lanes read these rows below.  The wave's own LDS accesses complete
     // in order; the fences keep the compiler from moving the reads ahead of the
     // writes (and, at the end of the step, the next writes ahead of the reads).
@@ -357,6 +438,21 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
     pack2_with_rest<F16>(p1[0], p1[1], pbits.z, prest.z);
     pack2_with_rest<F16>(p1[2], p1[3], pbits.w, prest.w);
 
+    if constexpr (NEW) {
+      // Load slot j of k-group kg is position 4 * kg + (j & 3) + 16 * (j >> 2).  Positions
+      // behind the last hold copies of the last: they weigh 0, but what the cache held
+      // there before the step need not be finite.
+      for (unsigned long long h = hits; h != 0; h &= h - 1) {
+        const int row = __builtin_ctzll(h);
+        const int pos = __builtin_amdgcn_readlane(new_slot, row) - (int)place;
+        const uint4 piece = h == hits ? fresh_v : new_piece<F16>(fresh->value, fresh->value_f32,
+                                                                 fresh_piece(row, r));
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (min(4 * kg + (j & 3) + 16 * (j >> 2), nvalid - 1) == pos) vreg[j] = piece;
+      }
+    }
+
     // ---- V: in-lane 8x8 transpose (positions x dims), then next V loads ----
     uint4 vt[8];
 #pragma unroll
@@ -391,6 +487,7 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    place = next_place;
   }
 
   // total of the running sum over the 4 k-groups that share column r
@@ -914,13 +1011,24 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_splitk_kernel(DecodeArgs
 // VG < 0 selects the loads-only measurement variant; VG > 0 selects the
 // vector-ALU measurement variant for exactly VG query heads
 // per KV head (head_dim 128, bf16 only).
-template <int NW, int D, bool F16, int VG = 0>
-__global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs a, int hpw) {
+template <int NW, int D, bool F16, int VG = 0, bool NEW = false>
+__global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs a, int hpw,
+                                                                     NewRows fresh, int batch) {
   using H = HeadDim<D>;
   __shared__ uint4 k_tile[NW][kStep * H::kLdsRowPieces];
   constexpr int kLanesWithDims = D / 32 * 16;   // lanes whose k-group holds real dims
   static_assert(sizeof(uint4) * kStep * H::kLdsRowPieces >= 34 * kLanesWithDims * sizeof(float),
                 "a wave's K tile must hold its partial");
+  int new_slot = -1;
+  if constexpr (NEW) {
+    if (fresh.main_wgs > 0 && (int)blockIdx.x >= fresh.main_wgs) {
+      store_new_row<F16>(a, fresh, blockIdx.x - fresh.main_wgs, NW * 64);
+      return;
+    }
+    if (fresh.main_wgs == 0 && (int)blockIdx.x < batch)
+      store_new_row<F16>(a, fresh, blockIdx.x, NW * 64);
+    new_slot = new_slot_of_lane(fresh, batch, threadIdx.x & 63);
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int parts = NW / hpw;
@@ -946,8 +1054,8 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
       compute_segment_loads_only(a, b, kvh, s0 * kStep, min(ctx, s1 * kStep), lane, acc, m_run,
                                  l_run);
     else
-      compute_segment<D, F16>(a, k_tile[wave], b, kvh, s0 * kStep, min(ctx, s1 * kStep), lane,
-                              acc, m_run, l_run);
+      compute_segment<D, F16, NEW>(a, k_tile[wave], b, kvh, s0 * kStep, min(ctx, s1 * kStep),
+                                   lane, acc, m_run, l_run, &fresh, new_slot);
   }
   if (parts > 1) {
     // value v of lane l at float v * kLanesWithDims + l of the wave's tile
@@ -1330,15 +1438,30 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& a, uint4* lds, int b
 
 // grid.x = num_wgs, block = 512.  `min_steps`: fewest steps a sub-run may have
 // (in units of 1 << shift steps); `shift`: see Cut.
-template <int D, bool F16, int VG = 0>
+template <int D, bool F16, int VG = 0, bool NEW = false>
 __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a, int batch,
                                                                     int num_wgs, int min_steps,
                                                                     int hpw, int wr_hpw, int wr_hpw_alt,
                                                                     int wr_tol, int shift,
                                                                     int short_rows,
-                                                                    int32_t* counters) {
+                                                                    int32_t* counters,
+                                                                    NewRows fresh) {
   using H = HeadDim<D>;
   constexpr int NW = 8;
+  int new_slot = -1;
+  int main_wgs = gridDim.x;
+  if constexpr (NEW) {
+    if (fresh.main_wgs > 0) {
+      main_wgs = fresh.main_wgs;
+      if ((int)blockIdx.x >= main_wgs) {
+        store_new_row<F16>(a, fresh, blockIdx.x - main_wgs, NW * 64);
+        return;
+      }
+    } else if ((int)blockIdx.x < batch) {
+      store_new_row<F16>(a, fresh, blockIdx.x, NW * 64);
+    }
+    new_slot = new_slot_of_lane(fresh, batch, threadIdx.x & 63);
+  }
   __shared__ uint4 k_tile[NW][kStep * H::kLdsRowPieces];
   constexpr int kLanesWithDims = D / 32 * 16;   // lanes whose k-group holds real dims
   static_assert(sizeof(uint4) * kStep * H::kLdsRowPieces >= 34 * kLanesWithDims * sizeof(float),
@@ -1386,7 +1509,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
   // No step belongs to an empty sequence: its output row (zeros, 0 / (0 + 1e-9))
   // is written here, sequence b by workgroup b modulo the grid.  The lengths of
   // the first kKeep * 64 sequences are in registers already.
-  for (int b = g; b < batch; b += gridDim.x) {
+  for (int b = g; b < batch; b += main_wgs) {
     int c;
     if (b < kKeep * 64) {
       int mine = kept_ctx[0];
@@ -1602,7 +1725,8 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
           else if constexpr (VG < 0)
             compute_segment_loads_only(a, seq, kvh, t0, t1, lane, acc, m_run, l_run);
           else
-            compute_segment<D, F16>(a, k_tile[wave], seq, kvh, t0, t1, lane, acc, m_run, l_run);
+            compute_segment<D, F16, NEW>(a, k_tile[wave], seq, kvh, t0, t1, lane, acc, m_run, l_run,
+                                         &fresh, new_slot);
           if (st > 0) {
             // the row started in an earlier part: park the piece for it
             if (holds_dims) {
@@ -1773,7 +1897,8 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
       else if constexpr (VG < 0)
         compute_segment_loads_only(a, sb, kvh, t0, t1, lane, acc, m_run, l_run);
       else
-        compute_segment<D, F16>(a, k_tile[wave], sb, kvh, t0, t1, lane, acc, m_run, l_run);
+        compute_segment<D, F16, NEW>(a, k_tile[wave], sb, kvh, t0, t1, lane, acc, m_run, l_run,
+                                     &fresh, new_slot);
       x += en - st;
     }
 
@@ -1971,6 +2096,15 @@ constexpr int kMinBalancedSteps = 1;
 // positions): 9 % 153 against 165, 15 % 146 against 154, 25 % 137 against 142.
 constexpr int kWholeRowTolerance = 64;
 
+// Whether the table rules out rows (of at most one per CU) that are not short: two rounds
+// of the 8 waves of a workgroup, which take 2.8 us each, what one CU draws.  A third is
+// still less than the balanced split's two passes for one sequence, and where its
+// workgroups have more than a row each to share: 768 positions of 8 KV heads with 1 / 4 /
+// 16 sequences 10.1 / 14.1 / 14.6 us against 11.7 / 12.6 / 16.5.
+bool table_of_short_rows(int64_t rows, int64_t positions) {
+  return positions <= (rows <= 8 || rows >= 128 ? 3 : 2) * 8 * kStep;
+}
+
 // Waves per workgroup of the fixed split = KV heads a workgroup covers: the
 // largest of 8, 4, 2, 1 that divides the number of KV heads.
 int waves_per_workgroup(int num_kv_heads) {
@@ -2097,6 +2231,15 @@ extern "C" size_t nvj_paged_decode_workspace_bytes(int32_t batch, int32_t num_he
 }
 
 namespace {
+// What a kernel gets to know of the new rows, and its grid: a workgroup of its own stores a
+// row if that leaves one workgroup per CU, else one of the `wgs` that attend does.
+NewRows rows_behind(const NewRows* rows, int wgs, int batch, dim3* grid) {
+  NewRows n = rows ? *rows : NewRows{};
+  n.main_wgs = rows && wgs + batch <= compute_units() ? wgs : 0;
+  *grid = dim3((unsigned)(n.main_wgs > 0 ? wgs + batch : rows && batch > wgs ? batch : wgs));
+  return n;
+}
+
 // The launch behind every decode entry point.  `ext_counters` != NULL: the
 // counters of the balanced split live there and `workspace` holds the partials
 // only (no counter header in front of them).
@@ -2105,7 +2248,7 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
                   void* workspace, size_t workspace_bytes, int32_t* ext_counters, int32_t batch,
                   int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
                   int32_t max_blocks, int32_t num_blocks, float scale, int32_t chunk,
-                  int32_t dtype, uint32_t phases) {
+                  int32_t dtype, uint32_t phases, const NewRows* new_rows = nullptr) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   const bool f16 = dtype == NVJ_DTYPE_F16;
   const bool whole = chunk == NVJ_CHUNK_WHOLE_SEQUENCE;
@@ -2170,21 +2313,28 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
                                  all_rows <= compute_units()
                              ? (int)all_rows
                              : 0;
-  const bool all_short = short_rows > 0 && (int64_t)max_blocks * block_size <= 2 * 8 * kStep &&
+  const bool all_short = short_rows > 0 && table_of_short_rows(all_rows, (int64_t)max_blocks * block_size) &&
                          !(phases & NVJ_PHASE_CLEAR_COUNTERS);
   if ((whole || all_short) && max_blocks > 0) {
     if (all_rows > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
     if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;   // there is no second pass
     const int hpw = all_short ? 1 : heads_per_workgroup(batch, num_kv_heads);
-    const dim3 grid((unsigned)(batch * (num_kv_heads / hpw))), block(512);
+    dim3 grid;
+    const dim3 block(512);
+    const NewRows fresh = rows_behind(new_rows, batch * (num_kv_heads / hpw), batch, &grid);
     hipError_t rc;
-    if (loads_only) rc = nvj::launch(paged_decode_whole_kernel<8, 128, false, -1>, grid, block, s, a, hpw);
-    else if (valu && group == 4) rc = nvj::launch(paged_decode_whole_kernel<8, 128, false, 4>, grid, block, s, a, hpw);
-    else if (valu) rc = nvj::launch(paged_decode_whole_kernel<8, 128, false, 8>, grid, block, s, a, hpw);
-    else if (head_dim == 128 && !f16) rc = nvj::launch(paged_decode_whole_kernel<8, 128, false>, grid, block, s, a, hpw);
-    else if (head_dim == 128) rc = nvj::launch(paged_decode_whole_kernel<8, 128, true>, grid, block, s, a, hpw);
-    else if (!f16) rc = nvj::launch(paged_decode_whole_kernel<8, 64, false>, grid, block, s, a, hpw);
-    else rc = nvj::launch(paged_decode_whole_kernel<8, 64, true>, grid, block, s, a, hpw);
+#define NVJ_LAUNCH_WHOLE(...) \
+  rc = nvj::launch(paged_decode_whole_kernel<8, __VA_ARGS__>, grid, block, s, a, hpw, fresh, batch)
+    if (new_rows && f16) NVJ_LAUNCH_WHOLE(128, true, 0, true);
+    else if (new_rows) NVJ_LAUNCH_WHOLE(128, false, 0, true);
+    else if (loads_only) NVJ_LAUNCH_WHOLE(128, false, -1);
+    else if (valu && group == 4) NVJ_LAUNCH_WHOLE(128, false, 4);
+    else if (valu) NVJ_LAUNCH_WHOLE(128, false, 8);
+    else if (head_dim == 128 && !f16) NVJ_LAUNCH_WHOLE(128, false);
+    else if (head_dim == 128) NVJ_LAUNCH_WHOLE(128, true);
+    else if (!f16) NVJ_LAUNCH_WHOLE(64, false);
+    else NVJ_LAUNCH_WHOLE(64, true);
+#undef NVJ_LAUNCH_WHOLE
     return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
   }
 
@@ -2209,14 +2359,18 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
           return NVJ_ERR_LAUNCH;
       }
       if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;
-      const dim3 grid((unsigned)(short_rows > plan.num_wgs ? short_rows : plan.num_wgs));
+      dim3 grid;
+      const NewRows fresh =
+          rows_behind(new_rows, short_rows > plan.num_wgs ? short_rows : plan.num_wgs, batch, &grid);
       hipError_t rc;
-#define NVJ_LAUNCH_BALANCED(DV, F16V, VGV)                                                     \
-  rc = nvj::launch(paged_decode_balanced_kernel<DV, F16V, VGV>, grid, dim3(512), s, a, batch, \
+#define NVJ_LAUNCH_BALANCED(...)                                                               \
+  rc = nvj::launch(paged_decode_balanced_kernel<__VA_ARGS__>, grid, dim3(512), s, a, batch,   \
                    plan.num_wgs, kMinBalancedSteps, plan.hpw,                      \
                    (phases & NVJ_PHASE_SHARED_ROWS) ? 0 : plan.wr_hpw, plan.wr_hpw_alt,       \
-                   kWholeRowTolerance, plan.shift, short_rows, counters)
-      if (loads_only) NVJ_LAUNCH_BALANCED(128, false, -1);
+                   kWholeRowTolerance, plan.shift, short_rows, counters, fresh)
+      if (new_rows && f16) NVJ_LAUNCH_BALANCED(128, true, 0, true);
+      else if (new_rows) NVJ_LAUNCH_BALANCED(128, false, 0, true);
+      else if (loads_only) NVJ_LAUNCH_BALANCED(128, false, -1);
       else if (valu && group == 4) NVJ_LAUNCH_BALANCED(128, false, 4);
       else if (valu) NVJ_LAUNCH_BALANCED(128, false, 8);
       else if (head_dim == 128 && !f16) NVJ_LAUNCH_BALANCED(128, false, 0);
@@ -2357,6 +2511,26 @@ extern "C" int nvj_paged_decode_counters_reset(void* stream, void* counters,
              : NVJ_ERR_LAUNCH;
 }
 
+// Counters of the calls that bring none, on the null stream only: its launches follow each
+// other, and it is never recorded into a graph that another stream replays.
+static __device__ __align__(256) int32_t null_stream_counters[16384];
+
+namespace {
+int null_stream_counters_of_current_device(void** out) {
+  static std::atomic<void*> address[kMaxDevices];
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return NVJ_ERR_LAUNCH;
+  void* p = address[dev].load(std::memory_order_acquire);
+  if (p == nullptr) {
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(null_stream_counters)) != hipSuccess || p == nullptr)
+      return NVJ_ERR_LAUNCH;
+    address[dev].store(p, std::memory_order_release);
+  }
+  *out = p;
+  return NVJ_OK;
+}
+}  // namespace
+
 extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, const void* k_cache,
                                                 const void* v_cache, const int32_t* block_tables,
                                                 const int32_t* context_lens, void* out,
@@ -2385,6 +2559,67 @@ extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, con
                        partial_bytes, static_cast<int32_t*>(counters), batch, num_heads,
                        num_kv_heads, head_dim, block_size, max_blocks, num_blocks, scale, 0, dtype,
                        phases);
+}
+
+// Up to one (sequence, KV head) per CU.  With more, the comparison in every step costs the
+// stream as much as the store kernel in front of it: 1 / 8 / 16 sequences of 8 KV heads
+// (700, 128 .. 2048, 32768 positions) take 12.3 / 16.1 / 319.1 us instead of 13.6 / 17.2 /
+// 321.6, 64 of 4096 159.8 instead of 158.6.
+extern "C" int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads,
+                                                int32_t num_kv_heads, int32_t head_dim,
+                                                int32_t block_size, int32_t max_blocks,
+                                                int32_t num_blocks, int32_t chunk) {
+  if (batch <= 0 || batch > kMaxNewRows || head_dim != 128 || max_blocks <= 0 || block_size <= 0 ||
+      num_blocks <= 0 || num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      (int64_t)num_blocks * block_size > INT32_MAX)
+    return 0;
+  const int64_t rows =
+      (int64_t)batch * num_kv_heads * virtual_heads_per_cache_head(num_heads / num_kv_heads);
+  if (rows > compute_units()) return 0;
+  if (chunk == NVJ_CHUNK_WHOLE_SEQUENCE) return 1;
+  if (chunk != 0 || nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads) >
+                        sizeof(null_stream_counters))
+    return 0;
+  return table_of_short_rows(rows, (int64_t)max_blocks * block_size) ? 1 : 2;
+}
+
+extern "C" int nvj_paged_decode_store_launch(
+    void* stream, const void* q, const void* key, const void* value, const int32_t* slot_mapping,
+    void* k_cache, void* v_cache, const int32_t* block_tables, const int32_t* context_lens,
+    void* out, void* partials, size_t partial_bytes, void* counters, size_t counter_bytes,
+    int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+    int32_t max_blocks, int32_t num_blocks, float scale, int32_t chunk, int32_t dtype,
+    int32_t k_dtype, int32_t v_dtype) {
+  const int takes = nvj_paged_decode_store_takes(batch, num_heads, num_kv_heads, head_dim,
+                                                 block_size, max_blocks, num_blocks, chunk);
+  if (takes == 0) return NVJ_ERR_UNSUPPORTED;
+  if ((k_dtype != dtype && k_dtype != NVJ_DTYPE_F32) || (v_dtype != dtype && v_dtype != NVJ_DTYPE_F32))
+    return NVJ_ERR_BAD_DTYPE;
+  if (!key || !value || !slot_mapping) return NVJ_ERR_NULL_POINTER;
+  if ((reinterpret_cast<uintptr_t>(key) | reinterpret_cast<uintptr_t>(value)) & 15u)
+    return NVJ_ERR_ALIGNMENT;
+  if (takes == 2) {
+    if (!counters && stream) return NVJ_ERR_NULL_POINTER;
+    if (!counters) {
+      const int rc = null_stream_counters_of_current_device(&counters);
+      if (rc != NVJ_OK) return rc;
+    } else {
+      if (reinterpret_cast<uintptr_t>(counters) & 3u) return NVJ_ERR_ALIGNMENT;
+      if (counter_bytes < nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads))
+        return NVJ_ERR_WORKSPACE;
+    }
+  }
+  NewRows n = {};
+  n.key = key;
+  n.value = value;
+  n.slots = slot_mapping;
+  n.num_slots = num_blocks * block_size;
+  n.key_f32 = k_dtype == NVJ_DTYPE_F32;
+  n.value_f32 = v_dtype == NVJ_DTYPE_F32;
+  return launch_decode(stream, q, k_cache, v_cache, block_tables, context_lens, out, partials,
+                       partial_bytes, static_cast<int32_t*>(counters), batch, num_heads,
+                       num_kv_heads, head_dim, block_size, max_blocks, num_blocks, scale, chunk,
+                       dtype, NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE | NVJ_PHASE_SHORT_ROWS, &n);
 }
 
 extern "C" int nvj_paged_decode_static_launch(void* stream, const void* q, const void* k_cache,

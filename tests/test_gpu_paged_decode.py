@@ -1012,3 +1012,71 @@ def test_short_rows(lens, Hq, Hkv, D):
         got = paged_attention(*t, scale, bs, phases=both | extra)
         torch.cuda.synchronize()
         assert_close_bf16(torch_to_bits(got), want, what=f"lens={lens} phases={extra}")
+
+
+@pytest.mark.parametrize("own_workspace", [False, True])
+@pytest.mark.parametrize("dtype,k_f32", [("bf16", True), ("f16", False)])
+@pytest.mark.parametrize("lens,split", [([1], 0), ([700], 0), ([33, 512, 65, 32, 0, 64], 0),
+                                        ([513, 40, 1300, 33, 900], -1), ([100, 3000] * 16, 0),
+                                        ([2, 65] * 32, 0)])
+def test_store_in_the_same_launch(lens, split, dtype, k_f32, own_workspace):
+    """New rows stored by the attention launch itself against the two launches: rows
+    in the middle of a step and at its ends, a row that another entry of the batch also
+    attends to, slots that are not stored, and a cache that holds NaN wherever no position is
+    live before the step."""
+    print(f"case store and attend lens={lens} split={split} {dtype} own={own_workspace}", flush=True)
+    import torch
+    from nanovllm_jax_amd import (Attention, create_decode_context,
+                                  paged_attention, store_kv_to_cache)
+    from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
+    B, D, bs, dev = len(lens), 128, 64, "cuda:0"
+    Hq, Hkv = (16, 8) if B <= 32 else (8, 4)      # 256 KV heads of rows at most
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    pages = [max(1, -(-n // bs)) for n in lens]
+    g = torch.Generator(device=dev).manual_seed(5 + B)
+    order = np.random.default_rng(B).permutation(sum(pages) + 2)
+    table = np.zeros((B, max(pages)), np.int32)
+    at = 0
+    for b, n in enumerate(pages):
+        table[b, :n] = order[at:at + n]
+        at += n
+    if B > 4:                      # two entries of one sequence: each sees the other's new row
+        table[3], lens = table[2], list(lens)
+        lens[3] = max(lens[2] - 1, 1)
+    slots = np.array([table[b, (n - 1) // bs] * bs + (n - 1) % bs if n else -1
+                      for b, n in enumerate(lens)], np.int32)
+    if B > 6:
+        slots[5], slots[6] = -1, (sum(pages) + 2) * bs
+    caches = []
+    for _ in range(2):
+        c = torch.full((sum(pages) + 2, bs, Hkv, D), float("nan"), dtype=dt, device=dev)
+        flat = c.view(-1, Hkv, D)
+        for b, n in enumerate(lens):
+            for p in range(-(-n // bs)):
+                live = min(bs, n - p * bs)
+                first = int(table[b, p]) * bs
+                flat[first:first + live] = torch.randn(live, Hkv, D, generator=g, device=dev).to(dt)
+        flat[slots[(slots >= 0) & (slots < len(flat))]] = float("nan")
+        caches.append(c)
+    q = torch.randn(B, Hq, D, generator=g, device=dev).to(dt)
+    k = torch.randn(B, Hkv, D, generator=g, device=dev).to(torch.float32 if k_f32 else dt)
+    v = torch.randn(B, Hkv, D, generator=g, device=dev).to(dt)
+    t_slots, t_table = torch.from_numpy(slots).to(dev), torch.from_numpy(table).to(dev)
+    t_lens = torch.from_numpy(np.array(lens, np.int32)).to(dev)
+    want_caches = [c.clone() for c in caches]
+    store_kv_to_cache(k, v, *want_caches, t_slots)
+    want = paged_attention(q, *want_caches, t_table, t_lens, D ** -0.5, bs, chunk=split)
+    attn = Attention(Hq, D, D ** -0.5, Hkv, bs)
+    attn.set_kv_cache(*caches)
+    if own_workspace:
+        attn.workspace = DecodeWorkspace.for_shape(B, Hq, D, table.shape[1], bs, Hkv, dev)
+    before = [c.clone() for c in caches]
+    for _ in range(3):             # counters are left ready for the next call
+        for c, old in zip(caches, before):
+            c.copy_(old)
+        got = attn(q, k, v, create_decode_context(t_lens, t_slots, t_table, split))
+        torch.cuda.synchronize()
+        assert not torch.isnan(got).any()
+        torch.testing.assert_close(got.float(), want.float(), rtol=1e-2, atol=2e-3)
+        for c, w in zip(caches, want_caches):
+            assert torch.equal(c.view(torch.int16), w.view(torch.int16))
