@@ -615,7 +615,8 @@ typedef struct nvj_decoder_batch {
   const int32_t* block_tables;   /* [num_sequences, max_blocks]; prefill: NULL = packed rows */
   const int32_t* cu_seqlens_q;   /* prefill: [num_sequences + 1] */
   const int32_t* cu_seqlens_k;
-  const int32_t* last_token_indices;  /* prefill: [num_sequences], the rows that get logits */
+  const int32_t* last_token_indices;  /* prefill: [num_sequences], the rows that get logits;
+                                       * negative counts from the end, NaN where none is named */
   void* partials;                /* decode: as nvj_paged_decode_launch_counters (chunk 0) or */
   size_t partial_bytes;          /*   the workspace of nvj_paged_decode_launch_phases */
   void* counters;

@@ -69,13 +69,28 @@ enum Epilogue { kPlain, kSiluMul };
 
 struct NormGemmArgs {
   const float4* h;            // [rows, hidden] residual stream
-  const int32_t* row_index;   // rows to take from h, or null: row m is row m
+  const int32_t* row_index;   // rows to take from h (row_of_index), or null: row m is row m
   const float* norm_weight;   // [hidden]
   const char* weight;         // [outputs, hidden] bf16
   uint16_t* out;              // kPlain [rows, outputs], kSiluMul [rows, outputs / 2]
   float eps;
   int num_tokens, outputs;
+  int num_rows;               // of h, with row_index
 };
+
+// The row of `rows` that an index names: a negative one counts from the end, as tensor
+// indexing on the host does (a sequence without new tokens in front of all others has
+// index -1).  One that names no row gives `real` = false and row 0, which is in range:
+// its output is NaN.
+struct IndexedRow {
+  int row;
+  bool real;
+};
+__device__ __forceinline__ IndexedRow row_of_index(int index, int rows) {
+  if (index < 0) index += rows;
+  const bool real = (uint32_t)index < (uint32_t)rows;
+  return {real ? index : 0, real};
+}
 
 // RMSNorm of up to 16 rows of h into LDS as bf16, `WAVES` waves, a row each at a time;
 // the arithmetic and its order are those of add_rms_norm_kernel (layer_glue.hip).
@@ -93,14 +108,16 @@ struct NormPrologue {
 #pragma unroll
     for (int j = 0; j < ROWS; ++j) {
       const int token = min(wave + waves * j, a.num_tokens - 1);
-      const int row = a.row_index ? a.row_index[token] : token;
+      IndexedRow at = {token, true};
+      if (a.row_index) at = row_of_index(a.row_index[token], a.num_rows);
 #pragma unroll
       for (int i = 0; i < kPerLane; ++i) {
         const int p = min(lane + 64 * i, kPieces - 1);
-        const float4* src = a.h + (int64_t)row * (kHidden / 4) + 2 * p;
+        const float4* src = a.h + (int64_t)at.row * (kHidden / 4) + 2 * p;
         x[j][i][0] = src[0];
         x[j][i][1] = src[1];
       }
+      if (!at.real) x[j][0][0].x = __builtin_nanf("");   // reaches the whole row by its norm
     }
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
@@ -344,16 +361,22 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict
   }
 }
 
-// dst[m] = src[index[m]], rows of `pieces` 16-byte pieces, one wave per row.
+// dst[m] = src[index[m]], bf16 rows of `pieces` 16-byte pieces, one wave per row.  ROWS: the
+// index is one of row_of_index; otherwise a token id, clamped into the table.
+template <bool ROWS>
 __global__ __launch_bounds__(256) void copy_rows_kernel(const uint4* __restrict__ src,
                                                         const int32_t* __restrict__ index,
                                                         uint4* __restrict__ dst, int num_rows,
                                                         int pieces, int src_rows) {
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= num_rows) return;
-  const int64_t row = min(max(index[m], 0), src_rows - 1);
-  for (int p = threadIdx.x & 63; p < pieces; p += 64)
-    dst[(int64_t)m * pieces + p] = src[row * pieces + p];
+  IndexedRow at = {min(max(index[m], 0), src_rows - 1), true};
+  if (ROWS) at = row_of_index(index[m], src_rows);
+  const uint4 nan = make_uint4(0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u);
+  for (int p = threadIdx.x & 63; p < pieces; p += 64) {
+    const uint4 v = src[(int64_t)at.row * pieces + p];
+    dst[(int64_t)m * pieces + p] = at.real ? v : nan;
+  }
 }
 
 // hidden 256, 512, 1024 or 2048; one row per wave for up to 4 rows, else four
@@ -514,6 +537,7 @@ int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder
   a.outputs = m.vocab;
   a.out = static_cast<uint16_t*>(b.logits);
   a.row_index = b.is_prefill ? b.last_token_indices : nullptr;
+  a.num_rows = tokens;
   a.num_tokens = b.num_sequences;
   return launch_norm_gemm_wide<true>(s, a, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }
@@ -538,7 +562,7 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
   char *h = ws + at.h, *y = ws + at.y, *t = ws + at.t, *qkv = ws + at.qkv, *o = ws + at.o;
   char* act = ws + at.act;
   // the embedding rows are the residual
-  if (nvj::launch(copy_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
+  if (nvj::launch(copy_rows_kernel<false>, dim3((unsigned)((tokens + 3) / 4)), dim3(256), s,
                   static_cast<const uint4*>(m.embed), b.input_ids, reinterpret_cast<uint4*>(h),
                   tokens, pieces, m.vocab) != hipSuccess)
     return NVJ_ERR_LAUNCH;
@@ -590,7 +614,7 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
   if (!b.logits || b.num_sequences == 0) return NVJ_OK;
   const char* rows = y;
   if (b.is_prefill) {
-    if (nvj::launch(copy_rows_kernel, dim3((unsigned)((b.num_sequences + 3) / 4)), dim3(256), s,
+    if (nvj::launch(copy_rows_kernel<true>, dim3((unsigned)((b.num_sequences + 3) / 4)), dim3(256), s,
                     reinterpret_cast<const uint4*>(y), b.last_token_indices,
                     reinterpret_cast<uint4*>(ws + at.last), b.num_sequences, pieces,
                     tokens) != hipSuccess)

@@ -126,3 +126,44 @@ def test_store_with_packed_copies_and_cleared_words(tokens, heads, clear, dtype)
     assert torch.equal(kc, want_k) and torch.equal(vc, want_v)
     assert torch.equal(k_rows, k.to(dt)) and torch.equal(v_rows, v)
     assert words.tolist() == [0] * clear + [7]
+
+
+def _small_runner(seed=0, hidden=512, inter=768, heads=4, vocab=1000, layers=2, blocks=60, **kw):
+    from nanovllm_jax_amd.engine import decode_step as ds
+    cfg = ds.DecodeModelConfig(num_layers=layers, hidden_size=hidden, num_heads=heads,
+                               num_kv_heads=2, head_dim=128, intermediate_size=inter,
+                               vocab_size=vocab, max_position=512, block_size=64,
+                               num_kvcache_blocks=blocks, **kw)
+    return ds, ds.DecodeStepRunner(cfg, "cuda:0", seed=seed)
+
+
+def _close(got, want):
+    """Two orders of bf16 roundings of the same step (as in the comparison above)."""
+    return (got - want).abs().max().item() <= 0.02 * want.abs().max().item() + 0.02
+
+
+# rows of the few-row form, of the many-row form with few and with many sequences
+@pytest.mark.parametrize("lens", [[0, 5, 9], [0, 30, 4], [0] + [2] * 20])
+def test_native_step_first_sequence_without_new_tokens(lens, monkeypatch):
+    print(f"case no new tokens {lens[:3]} of {len(lens)}", flush=True)
+    ds, runner = _small_runner()
+    cached = [40] + [0] * (len(lens) - 1)
+    rng = np.random.Generator(np.random.PCG64(len(lens)))
+    toks = [rng.integers(0, 1000, n + c).tolist() for n, c in zip(lens, cached)]
+    ids, pos, ctx = runner.make_prefill_inputs(toks, [[i] for i in range(len(lens))], cached)
+    assert ctx.last_token_indices[0].item() == -1
+    before = runner.kv_cache.clone()
+    got = runner._native_forward(ids, pos, ctx).float()
+    runner.kv_cache.copy_(before)
+    with monkeypatch.context() as m:
+        m.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+        want = runner.forward(ids, pos, ctx).float()
+    # index -1 is the last row, whatever sequence it belongs to, as host indexing has it
+    assert torch.equal(got[0], got[-1]) and _close(got, want)
+    # one that names no row shows, and harms no other
+    bad = ctx.last_token_indices.clone()
+    bad[0], bad[1] = int(ids.shape[0]), -int(ids.shape[0]) - 1
+    ctx.last_token_indices = bad
+    runner.kv_cache.copy_(before)
+    out = runner._native_forward(ids, pos, ctx).float()
+    assert out[:2].isnan().all() and torch.equal(out[2:], got[2:])
