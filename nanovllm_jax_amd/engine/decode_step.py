@@ -302,14 +302,18 @@ class DecodeStepRunner:
             if t is None or t.dtype != torch.int32 or not t.is_cuda or not t.is_contiguous() \
                     or t.device != self.embed.device:
                 return None
-        sequences = context.cu_seqlens_q.shape[0] - 1 if prefill else tokens
+        sequences = context.cu_seqlens_q.numel() - 1 if prefill else tokens
         if positions.shape != (tokens,) or sl.shape != (tokens,) or input_ids.dim() != 1 or \
                 (bt is not None and (bt.dim() != 2 or bt.shape[0] != sequences
                                      or bt.shape[1] == 0)):
             return None
         if prefill:
-            if context.cu_seqlens_k.shape[0] != sequences + 1 or \
-                    sequences == 0:
+            # any other count of rows, or indices from the host, as tensor indexing takes them
+            last = context.last_token_indices
+            if context.cu_seqlens_k.shape != (sequences + 1,) or sequences == 0 or \
+                    not isinstance(last, torch.Tensor) or last.shape != (sequences,) or \
+                    last.dtype not in (torch.int32, torch.int64) or \
+                    last.device != self.embed.device:
                 return None
         elif context.context_lens.shape != (tokens,):
             return None
@@ -325,7 +329,9 @@ class DecodeStepRunner:
         if prefill:
             b.cu_seqlens_q, b.cu_seqlens_k = (context.cu_seqlens_q.data_ptr(),
                                               context.cu_seqlens_k.data_ptr())
-            last = context.last_token_indices.to(torch.int32).contiguous()
+            if last.dtype == torch.int64:
+                last = last.clamp(-(1 << 31), (1 << 31) - 1).to(torch.int32)
+            last = last.contiguous()
             b.last_token_indices = last.data_ptr()
         else:
             ws = ws0 or self._eager_workspace(context)

@@ -167,3 +167,32 @@ def test_native_step_first_sequence_without_new_tokens(lens, monkeypatch):
     runner.kv_cache.copy_(before)
     out = runner._native_forward(ids, pos, ctx).float()
     assert out[:2].isnan().all() and torch.equal(out[2:], got[2:])
+
+
+@pytest.mark.parametrize("what", ["host", "longer", "shorter", "int64", "strided", "2d"])
+def test_native_step_takes_any_last_token_indices(what):
+    """Logits of exactly the rows asked for, by any tensor that indexes rows."""
+    print(f"case last token indices {what}", flush=True)
+    ds, runner = _small_runner()
+    ids, pos, ctx = runner.make_prefill_inputs([[1, 2, 3], [4, 5], [6, 7, 8, 9]], [[0], [1], [2]])
+    want = runner.forward(ids, pos, ctx).float()
+    last, rows = ctx.last_token_indices, [0, 1, 2]
+    if what == "host":
+        last = last.cpu()
+    elif what == "longer":
+        last, rows = torch.cat([last, last[:1]]), [0, 1, 2, 0]
+    elif what == "shorter":
+        last, rows = last[1:2], [1]
+    elif what == "int64":
+        last = last.long()
+    elif what == "strided":
+        last = last.repeat_interleave(2)[::2]
+    else:
+        last = last[None, :].expand(2, 3)
+    ctx.last_token_indices = last
+    got = runner.forward(ids, pos, ctx).float()
+    assert (runner._native_forward(ids, pos, ctx) is not None) == (what in ("int64", "strided"))
+    if what == "2d":
+        assert got.shape == (2, 3, want.shape[1]) and torch.equal(got[0], got[1])
+        got = got[0]
+    assert got.shape == (len(rows), want.shape[1]) and _close(got, want[rows])
