@@ -1,8 +1,9 @@
-// The host side of one attention call as native code: takes the torch tensors of
-// Attention.__call__ as they are, checks them, allocates the output and enqueues the
-// store and the attention launches (layers/attention.py:436-480 of the reference).
+// The host side of a call as native code.  decode and prefill, one attention call: take the
+// torch tensors of Attention.__call__ as they are, check them, allocate the output and enqueue
+// the store and the attention launches (layers/attention.py:436-480 of the reference).
+// decoder_layers: the weights of a model for the native step.
 //
-// A small call is bound by the host: validation, allocation and two foreign calls of
+// A small attention call is bound by the host: validation, allocation and two foreign calls of
 // 13 and 20 arguments cost 19 us in Python for 14 us of GPU work (one sequence of 700
 // positions).  Here they cost about 5.
 //
@@ -14,6 +15,8 @@
 
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
+
+#include <vector>
 
 #include "nvj_paged_attn.h"
 
@@ -228,6 +231,92 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
 }
 
+// decoder_layers(tensors, num_heads, num_kv_heads, head_dim, device): the weights of a
+// model as nvj_decoder_step_launch wants them, or None when they are not what it takes.
+// tensors: embed, final_norm, cos_sin, then per layer qkv, o, gate_up, down, ln1, ln2, q_norm,
+// k_norm (both may be None), k_cache, v_cache.  Returns (nvj_decoder_layer[] as bytes, hidden,
+// intermediate, vocab, max_position, num_blocks, page).
+//
+// Looked at in full on every step, so that a weight that was replaced, resized or retyped
+// since the last one is seen whatever its address.
+PyObject* decoder_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  constexpr Py_ssize_t kModel = 3, kLayer = 10;
+  if (nargs != 5 || !PyList_Check(args[0])) Py_RETURN_NONE;
+  PyObject* list = args[0];
+  const Py_ssize_t n = PyList_GET_SIZE(list);
+  const int64_t heads = PyLong_AsLong(args[1]), kv_heads = PyLong_AsLong(args[2]),
+                dim = PyLong_AsLong(args[3]), device = PyLong_AsLong(args[4]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (n < kModel + kLayer || (n - kModel) % kLayer != 0 || heads <= 0 || kv_heads <= 0 ||
+      dim <= 0 || heads > INT32_MAX || kv_heads > INT32_MAX || dim > INT32_MAX)
+    Py_RETURN_NONE;
+  auto tensor = [&](Py_ssize_t at, at::ScalarType type) -> const Tensor* {
+    const Tensor* t;
+    if (!get(PyList_GET_ITEM(list, at), &t) || t->layout() != at::kStrided || !t->is_cuda() ||
+        t->device().index() != device || t->scalar_type() != type || !t->is_contiguous() ||
+        t->numel() == 0 || (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15u))
+      return nullptr;
+    return t;
+  };
+  auto matrix = [&](Py_ssize_t at, at::ScalarType type, int64_t rows, int64_t columns) -> void* {
+    const Tensor* t = tensor(at, type);
+    return t && t->dim() == 2 && (rows < 0 || t->size(0) == rows) && t->size(1) == columns
+               ? t->data_ptr()
+               : nullptr;
+  };
+  auto vector = [&](Py_ssize_t at, int64_t size) -> const float* {
+    const Tensor* t = tensor(at, at::kFloat);
+    return t && t->dim() == 1 && t->size(0) == size ? static_cast<const float*>(t->data_ptr())
+                                                    : nullptr;
+  };
+  // sizes come from the first of their kind; everything else has to agree with them
+  const Tensor* embed = tensor(0, at::kBFloat16);
+  const Tensor* gate_up = tensor(kModel + 2, at::kBFloat16);
+  const Tensor* cache = tensor(kModel + 8, at::kBFloat16);
+  if (!embed || embed->dim() != 2 || !gate_up || gate_up->dim() != 2 || gate_up->size(0) % 2 != 0 ||
+      !cache || cache->dim() != 4 || cache->size(2) != kv_heads || cache->size(3) != dim)
+    Py_RETURN_NONE;
+  const int64_t hidden = embed->size(1), intermediate = gate_up->size(0) / 2;
+  const int64_t q_width = heads * dim, kv_width = kv_heads * dim;
+  if (!vector(1, hidden) || !matrix(2, at::kFloat, -1, dim)) Py_RETURN_NONE;
+  const Tensor* cos_sin = tensor(2, at::kFloat);
+  for (int64_t size : {embed->size(0), hidden, gate_up->size(0), cos_sin->size(0), cache->size(0),
+                       cache->size(1)})
+    if (size > INT32_MAX) Py_RETURN_NONE;
+  std::vector<nvj_decoder_layer> layers((n - kModel) / kLayer);
+  Py_ssize_t at = kModel;
+  for (nvj_decoder_layer& l : layers) {
+    l.qkv = matrix(at, at::kBFloat16, q_width + 2 * kv_width, hidden);
+    l.o = matrix(at + 1, at::kBFloat16, hidden, q_width);
+    l.gate_up = matrix(at + 2, at::kBFloat16, 2 * intermediate, hidden);
+    l.down = matrix(at + 3, at::kBFloat16, hidden, intermediate);
+    l.ln1 = vector(at + 4, hidden);
+    l.ln2 = vector(at + 5, hidden);
+    const bool norms = PyList_GET_ITEM(list, at + 6) != Py_None ||
+                       PyList_GET_ITEM(list, at + 7) != Py_None;
+    l.q_norm = norms ? vector(at + 6, dim) : nullptr;
+    l.k_norm = norms ? vector(at + 7, dim) : nullptr;
+    const Tensor* k = tensor(at + 8, at::kBFloat16);
+    const Tensor* v = tensor(at + 9, at::kBFloat16);
+    if (!l.qkv || !l.o || !l.gate_up || !l.down || !l.ln1 || !l.ln2 ||
+        (norms && (!l.q_norm || !l.k_norm)) || !k || !v || k->sizes() != cache->sizes() ||
+        v->sizes() != cache->sizes())
+      Py_RETURN_NONE;
+    l.k_cache = k->data_ptr();
+    l.v_cache = v->data_ptr();
+    at += kLayer;
+  }
+  PyObject* bytes = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(layers.data()),
+                                              layers.size() * sizeof(nvj_decoder_layer));
+  if (!bytes) return nullptr;
+  return Py_BuildValue("(NLLLLLL)", bytes, (long long)hidden, (long long)intermediate,
+                       (long long)embed->size(0), (long long)cos_sin->size(0),
+                       (long long)cache->size(0), (long long)cache->size(1));
+}
+
 // A C++ exception (out of memory in an allocation) becomes a Python one.
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyObject* guarded(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
@@ -241,6 +330,9 @@ PyMethodDef methods[] = {
      METH_FASTCALL, "store + paged decode attention of one layer"},
     {"prefill", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<prefill>)),
      METH_FASTCALL, "store + prefill attention of one layer"},
+    {"decoder_layers",
+     reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<decoder_layers>)),
+     METH_FASTCALL, "the weights of a model, checked, for the native step"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "nvj_host", nullptr, -1, methods,

@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
+from operator import itemgetter
 
 import numpy as np
 import torch
@@ -41,6 +42,7 @@ from ..utils.context import AttentionContext, create_decode_context, create_pref
 # it, and for models that call is not built for, it is library GEMMs with the element-wise
 # launches between them.
 _NATIVE_STEP_ROWS = 1 << 18
+_LAYER_WEIGHTS = itemgetter("qkv", "o", "gate_up", "down", "ln1", "ln2", "q_norm", "k_norm")
 
 __all__ = ["DecodeModelConfig", "DecodeStepRunner", "prepare_block_tables", "prepare_decode",
            "prepare_prefill", "advance_decode"]
@@ -213,7 +215,6 @@ class DecodeStepRunner:
             a.set_kv_cache(self.kv_cache[0, layer], self.kv_cache[1, layer])
             self.attn.append(a)
         self._graph = None
-        self._native_model = None       # (pointers it was built from, model, layers)
         self._eager_ws = None
         self._eager_ws_shapes = set()
 
@@ -244,44 +245,31 @@ class DecodeStepRunner:
         x1, x2 = x.chunk(2, dim=-1)
         return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], dim=-1)
 
-    _LAYER_WEIGHTS = ("qkv", "o", "gate_up", "down", "ln1", "ln2", "q_norm", "k_norm")
-
     def _native(self):
-        """The model as the native step wants it: ``(model, layers)``, or None when it
-        is not one that step is built for.  Rebuilt when a weight or cache tensor has
-        been replaced; the look at the addresses is all an unchanged model costs."""
+        """The model as the native step wants it: ``(model, layers, the memory of
+        layers)``, or None when it is not one that step is built for.  Everything the
+        long way reads on a step is read here on every step too, shapes and types
+        included."""
+        c, n = self.cfg, min(len(self.layers), len(self.attn))
+        if n == 0:
+            return None
+        scale, page = self.attn[0].scale, self.attn[0].block_size
         tensors = [self.embed, self.final_norm, self.cos_sin]
         for lw, a in zip(self.layers, self.attn):
-            tensors += [lw[n] for n in self._LAYER_WEIGHTS]
-            tensors += [a.k_cache, a.v_cache]
-        key = [t.data_ptr() for t in tensors]
-        key.append(self.attn[0].scale)
-        if self._native_model is not None and self._native_model[0] == key:
-            return self._native_model[1]
-        c, a0 = self.cfg, self.attn[0]
-        f32 = {id(t) for lw in self.layers for t in (lw["ln1"], lw["ln2"], lw["q_norm"],
-                                                     lw["k_norm"])}
-        f32 |= {id(self.final_norm), id(self.cos_sin)}
-        ok = all(t.is_cuda and t.is_contiguous() and
-                 t.dtype == (torch.float32 if id(t) in f32 else torch.bfloat16) for t in tensors)
-        ok = ok and all(a.scale == a0.scale and a.block_size == c.block_size and
-                        a.k_cache.shape == a0.k_cache.shape == a.v_cache.shape and
-                        a.k_cache.dim() == 4 for a in self.attn)
-        built = None
-        if ok:
-            model = _lib.DecoderModel(
-                self.embed.data_ptr(), self.final_norm.data_ptr(), self.cos_sin.data_ptr(),
-                c.num_layers, c.hidden_size, c.num_heads, c.num_kv_heads, c.head_dim,
-                c.intermediate_size, self.embed.shape[0], self.cos_sin.shape[0], c.block_size,
-                a0.k_cache.shape[0], c.rms_norm_eps, a0.scale)
-            per = len(self._LAYER_WEIGHTS) + 2
-            layers = (_lib.DecoderLayer * c.num_layers)(
-                *[_lib.DecoderLayer(*key[3 + per * i:3 + per * (i + 1)])
-                  for i in range(c.num_layers)])
-            if _lib.load().nvj_decoder_step_workspace_bytes(ctypes.byref(model), 1, 1) > 0:
-                built = (model, layers)
-        self._native_model = (key, built)
-        return built
+            if a.scale != scale or a.block_size != page:
+                return None
+            tensors += _LAYER_WEIGHTS(lw)
+            tensors += (a.k_cache, a.v_cache)
+        found = _lib.load_host().decoder_layers(tensors, c.num_heads, c.num_kv_heads, c.head_dim,
+                                                self.embed.device.index)
+        if found is None or found[6] != page:
+            return None
+        layers, hidden, intermediate, vocab, max_position, num_blocks, _ = found
+        model = _lib.DecoderModel(
+            self.embed.data_ptr(), self.final_norm.data_ptr(), self.cos_sin.data_ptr(), n, hidden,
+            c.num_heads, c.num_kv_heads, c.head_dim, intermediate, vocab, max_position, page,
+            num_blocks, c.rms_norm_eps, scale)
+        return model, ctypes.cast(layers, ctypes.POINTER(_lib.DecoderLayer)), layers
 
     def _native_forward(self, input_ids, positions, context: AttentionContext):
         """The whole step as one native call, or None when it has to go the long way."""
@@ -320,7 +308,11 @@ class DecodeStepRunner:
         built = self._native()
         if built is None:
             return None
-        model, layers = built
+        model, layers, _memory = built
+        lib, dev = _lib.load(), self.embed.device
+        need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens, sequences)
+        if need == 0:
+            return None
         b = _lib.DecoderBatch(num_tokens=tokens, num_sequences=sequences, is_prefill=int(prefill))
         b.input_ids, b.positions, b.slot_mapping = (input_ids.data_ptr(), positions.data_ptr(),
                                                     sl.data_ptr())
@@ -341,11 +333,8 @@ class DecodeStepRunner:
                 counters = ws._counters_for(4 * (1 + sequences * self.cfg.num_heads))
                 b.counters, b.counter_bytes = counters.data_ptr(), counters.numel() * 4
                 b.clear_counters, ws._clear_next = int(ws._clear_next), False
-        dev = input_ids.device
         logits = torch.empty((sequences, model.vocab), dtype=torch.bfloat16, device=dev)
         b.logits = logits.data_ptr()
-        lib = _lib.load()
-        need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens, sequences)
         scratch = torch.empty(need, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
             code = lib.nvj_decoder_step_launch(

@@ -196,3 +196,88 @@ def test_native_step_takes_any_last_token_indices(what):
         assert got.shape == (2, 3, want.shape[1]) and torch.equal(got[0], got[1])
         got = got[0]
     assert got.shape == (len(rows), want.shape[1]) and _close(got, want[rows])
+
+
+def _decode_inputs(runner, rows):
+    return runner.make_inputs(list(range(rows)), [20 + i for i in range(rows)],
+                              [[i] for i in range(rows)])
+
+
+@pytest.mark.parametrize("rows", [3, 20])
+def test_native_step_reads_the_model_on_every_step(rows, monkeypatch):
+    """What changes between two steps changes the second: a layer's scale, the norms' eps,
+    weights in place, and weights replaced by others."""
+    print(f"case model read on every step rows={rows}", flush=True)
+    ds, runner = _small_runner()
+    inputs = _decode_inputs(runner, rows)
+    first = runner.forward(*inputs).float()
+
+    def both():
+        got = runner.forward(*inputs).float()
+        with monkeypatch.context() as m:
+            m.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+            want = runner.forward(*inputs).float()
+        assert _close(got, want)
+        return got
+
+    attn, lw = runner.attn, runner.layers
+    attn[1].scale = 1.0             # one layer's alone: not a model for the native step
+    assert runner._native_forward(*inputs) is None
+    last = both()
+    assert not torch.equal(last, first)
+    for a in attn:
+        a.scale = 1.0
+    assert runner._native_forward(*inputs) is not None
+    assert not torch.equal(both(), last)
+    for a in attn:
+        a.scale = 128 ** -0.5
+    assert torch.equal(runner.forward(*inputs).float(), first)
+    runner.cfg.rms_norm_eps = 100.0
+    assert not torch.equal(both(), first)
+    runner.cfg.rms_norm_eps = 1e-6
+    kept = lw[1]["down"]
+    lw[1]["down"] = torch.zeros_like(kept)
+    assert not torch.equal(both(), first)
+    lw[1]["down"] = kept
+    for w in lw:                    # no norm of q and k
+        w["q_norm"] = w["k_norm"] = None
+    assert runner._native_forward(*inputs) is not None
+    assert not torch.equal(both(), first)
+
+
+@pytest.mark.parametrize("name,shape", [("qkv", (256, 512)), ("o", (512, 256)),
+                                        ("gate_up", (512, 512)), ("down", (256, 768)),
+                                        ("ln1", (256,)), ("ln2", (256,)), ("q_norm", (64,)),
+                                        ("k_norm", (64,)), ("cos_sin", (512, 64)),
+                                        ("final_norm", (256,))])
+def test_native_step_refuses_weights_of_another_shape(name, shape):
+    """A weight that was replaced by a smaller one is never read past its end: the native
+    step declines, and the long way names the mistake."""
+    print(f"case weight {name} {shape}", flush=True)
+    _, runner = _small_runner()
+    inputs = _decode_inputs(runner, 3)
+    assert runner._native_forward(*inputs) is not None
+    at = runner.layers[1] if name in runner.layers[1] else runner.__dict__
+    at[name] = torch.ones(shape, dtype=at[name].dtype, device="cuda:0")
+    assert runner._native_forward(*inputs) is None
+    with pytest.raises((RuntimeError, ValueError)):
+        runner.forward(*inputs)
+
+
+def test_native_step_declines_what_it_is_not_built_for():
+    print("case weights of another type, layout or alignment", flush=True)
+    _, runner = _small_runner()
+    inputs = _decode_inputs(runner, 3)
+    want = runner.forward(*inputs).float()
+    for name, other in (("qkv", lambda t: t.t().contiguous().t()),                # strided
+                        ("down", lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:]
+                         .view(t.shape))):                                        # 2 bytes off
+        kept = runner.layers[0][name]
+        runner.layers[0][name] = other(kept)
+        assert runner._native_forward(*inputs) is None
+        assert _close(runner.forward(*inputs).float(), want)
+        runner.layers[0][name] = kept
+    runner.attn[0].block_size = 32
+    assert runner._native_forward(*inputs) is None
+    with pytest.raises(ValueError):
+        runner.forward(*inputs)
