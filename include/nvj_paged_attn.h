@@ -608,7 +608,7 @@ typedef struct nvj_decoder_layer {
 } nvj_decoder_layer;
 
 typedef struct nvj_decoder_batch {
-  const int32_t* input_ids;      /* [num_tokens]; out of range is clamped */
+  const int32_t* input_ids;      /* [num_tokens]; outside the vocabulary: a row of NaN */
   const int32_t* positions;      /* [num_tokens] */
   const int32_t* slot_mapping;   /* [num_tokens] */
   const int32_t* context_lens;   /* decode: [num_sequences] */

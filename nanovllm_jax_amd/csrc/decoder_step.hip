@@ -342,7 +342,10 @@ bool residual_gemm_takes(int64_t reduction) {
   return reduction % 256 == 0 && reduction <= 12 * 256;   // both of the forms below: 8 waves
 }
 
-// h[m] = float(embed[ids[m]]), one wave per row.
+__device__ constexpr uint4 kNanPiece = {0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u};
+
+// h[m] = float(embed[ids[m]]), one wave per row; NaN for an id outside the table, which then
+// shows in the logits of its sequence and in no other.
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict__ embed,
                                                          const int32_t* __restrict__ ids,
                                                          float4* __restrict__ h, int num_tokens,
@@ -350,9 +353,10 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= num_tokens) return;
   const int lane = threadIdx.x & 63;
-  const int64_t id = min(max(ids[m], 0), vocab - 1);
+  const int id = ids[m];
+  const bool real = (uint32_t)id < (uint32_t)vocab;
   for (int p = lane; p < pieces; p += 64) {
-    const uint4 v = embed[id * pieces + p];
+    const uint4 v = real ? embed[(int64_t)id * pieces + p] : kNanPiece;
     float4* dst = h + ((int64_t)m * pieces + p) * 2;
     dst[0] = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u),
                          __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u));
@@ -361,22 +365,19 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint4* __restrict
   }
 }
 
-// dst[m] = src[index[m]], bf16 rows of `pieces` 16-byte pieces, one wave per row.  ROWS: the
-// index is one of row_of_index; otherwise a token id, clamped into the table.
-template <bool ROWS>
+// dst[m] = src[index[m]], bf16 rows of `pieces` 16-byte pieces, one wave per row; NaN where
+// the index names none.  FROM_END: a negative one counts from the end (row_of_index).
+template <bool FROM_END>
 __global__ __launch_bounds__(256) void copy_rows_kernel(const uint4* __restrict__ src,
                                                         const int32_t* __restrict__ index,
                                                         uint4* __restrict__ dst, int num_rows,
                                                         int pieces, int src_rows) {
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (m >= num_rows) return;
-  IndexedRow at = {min(max(index[m], 0), src_rows - 1), true};
-  if (ROWS) at = row_of_index(index[m], src_rows);
-  const uint4 nan = make_uint4(0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u);
-  for (int p = threadIdx.x & 63; p < pieces; p += 64) {
-    const uint4 v = src[(int64_t)at.row * pieces + p];
-    dst[(int64_t)m * pieces + p] = at.real ? v : nan;
-  }
+  const int i = index[m];
+  const IndexedRow at = row_of_index(!FROM_END && i < 0 ? src_rows : i, src_rows);
+  for (int p = threadIdx.x & 63; p < pieces; p += 64)
+    dst[(int64_t)m * pieces + p] = at.real ? src[(int64_t)at.row * pieces + p] : kNanPiece;
 }
 
 // hidden 256, 512, 1024 or 2048; one row per wave for up to 4 rows, else four

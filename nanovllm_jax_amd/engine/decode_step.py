@@ -437,10 +437,17 @@ class DecodeStepRunner:
     def make_inputs(self, last_tokens, seq_lens, block_tables):
         ids, pos, ctx, slots, bt = prepare_decode(last_tokens, seq_lens, block_tables,
                                                   self.cfg.block_size)
+        self._check_ids(ids)
         # the lengths are host integers here, as in the reference's filler: pick the split
         split = choose_split(ctx, self.cfg.num_kv_heads, self.cfg.num_heads)
         d_ids, d_pos, d_ctx, d_slots, d_bt = self._upload(ids, pos, ctx, slots, bt)
         return d_ids, d_pos, create_decode_context(d_ctx, d_slots, d_bt, split)
+
+    def _check_ids(self, ids):
+        """Host ids outside the vocabulary are an error here; ids that a caller writes
+        into device tensors give rows of NaN."""
+        if ids.size and int(ids.view(np.uint32).max()) >= self.embed.shape[0]:
+            raise ValueError(f"token ids must be in [0, {self.embed.shape[0]})")
 
     def _upload(self, *arrays):
         """int32 host arrays as device tensors, in one copy that nobody waits for: they
@@ -467,6 +474,7 @@ class DecodeStepRunner:
         from the paged cache."""
         ids, pos, cu_q, cu_k, slots, max_q, max_k = prepare_prefill(
             token_lists, block_tables, self.cfg.block_size, num_cached_tokens)
+        self._check_ids(ids)
         tables = ([prepare_block_tables(block_tables)] if num_cached_tokens is not None else [])
         d_ids, d_pos, d_cu_q, d_cu_k, d_slots, *bt = self._upload(ids, pos, cu_q, cu_k, slots,
                                                                   *tables)

@@ -281,3 +281,24 @@ def test_native_step_declines_what_it_is_not_built_for():
     assert runner._native_forward(*inputs) is None
     with pytest.raises(ValueError):
         runner.forward(*inputs)
+
+
+@pytest.mark.parametrize("rows", [4, 20])
+def test_token_ids_outside_the_vocabulary(rows):
+    """Refused where the ids come from the host; on the device the sequence concerned, and
+    no other, gets NaN logits."""
+    print(f"case ids outside the vocabulary rows={rows}", flush=True)
+    _, runner = _small_runner()
+    lens, tables = [20 + i for i in range(rows)], [[i] for i in range(rows)]
+    for bad in (1000, -1):
+        with pytest.raises(ValueError):
+            runner.make_inputs([0] * (rows - 1) + [bad], lens, tables)
+        with pytest.raises(ValueError):
+            runner.make_prefill_inputs([[1, bad]], [[0]])
+    ids, pos, ctx = runner.make_inputs([999] * rows, lens, tables)
+    want = runner.forward(ids, pos, ctx).float()
+    assert not want.isnan().any()
+    ids[1], ids[2] = 1000, -1
+    got = runner._native_forward(ids, pos, ctx).float()
+    keep = [i for i in range(rows) if i not in (1, 2)]
+    assert got[1:3].isnan().all() and torch.equal(got[keep], want[keep])
