@@ -625,6 +625,7 @@ typedef struct nvj_decoder_batch {
   int32_t num_tokens, num_sequences, max_blocks, chunk, is_prefill, clear_counters;
 } nvj_decoder_batch;
 
+/* Bytes of workspace of one step; 0 for a model or a number of rows it cannot be given. */
 NVJ_API size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
                             int32_t num_tokens, int32_t num_sequences);
 NVJ_API int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* model,

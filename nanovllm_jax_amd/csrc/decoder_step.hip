@@ -462,6 +462,15 @@ int check_model(const nvj_decoder_model* m) {
   return NVJ_OK;
 }
 
+// Whether the products can be given that many rows (32-bit offsets into the operands).
+bool takes_rows(const nvj_decoder_model& m, int64_t tokens, int64_t sequences) {
+  const int64_t q_width = (int64_t)m.num_heads * m.head_dim;
+  return nvj::linear_takes(tokens, m.hidden, m.hidden) &&
+         nvj::linear_takes(tokens, m.hidden, q_width) &&
+         nvj::linear_takes(tokens, m.hidden, m.intermediate) &&
+         nvj::linear_takes(sequences, m.vocab, m.hidden);
+}
+
 int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer& l,
               const nvj_decoder_batch& b, bool first_layer, const void* q,
               const void* k, const void* v, int64_t kv_stride, void* out) {
@@ -641,7 +650,9 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
 extern "C" size_t nvj_decoder_step_workspace_bytes(const nvj_decoder_model* model,
                                                    int32_t num_tokens,
                                                    int32_t num_sequences) {
-  if (check_model(model) != NVJ_OK || num_tokens <= 0 || num_sequences < 0) return 0;
+  if (check_model(model) != NVJ_OK || num_tokens <= 0 || num_sequences < 0 ||
+      !takes_rows(*model, num_tokens, num_sequences > 0 ? num_sequences : 1))
+    return 0;
   return step_buffers(*model, num_tokens, num_sequences).bytes;
 }
 
@@ -656,10 +667,7 @@ extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* mo
   const nvj_decoder_batch& b = *batch;
   if (b.num_tokens < 0 || b.num_sequences < 0 || (!b.is_prefill && b.num_tokens != b.num_sequences))
     return NVJ_ERR_BAD_SHAPE;
-  if (!nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden, m.intermediate) ||
-      !nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden,
-                         (int64_t)m.num_heads * m.head_dim) ||
-      !nvj::linear_takes(b.num_tokens > 0 ? b.num_tokens : 1, m.hidden, m.hidden))
+  if (!takes_rows(m, b.num_tokens > 0 ? b.num_tokens : 1, b.num_sequences > 0 ? b.num_sequences : 1))
     return NVJ_ERR_UNSUPPORTED;
   if (b.num_tokens == 0) return NVJ_OK;
   if (!layers || !m.embed || !m.final_norm || !m.cos_sin || !b.input_ids || !b.positions ||
@@ -671,14 +679,16 @@ extern "C" int nvj_decoder_step_launch(void* stream, const nvj_decoder_model* mo
   const StepBuffers at = step_buffers(m, b.num_tokens, b.num_sequences);
   if (workspace_bytes < at.bytes) return NVJ_ERR_WORKSPACE;
   uintptr_t bits = reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(m.embed) |
-                   reinterpret_cast<uintptr_t>(m.final_norm);
+                   reinterpret_cast<uintptr_t>(m.final_norm) |
+                   reinterpret_cast<uintptr_t>(m.cos_sin) | reinterpret_cast<uintptr_t>(b.logits);
   for (int i = 0; i < m.num_layers; ++i) {
     const nvj_decoder_layer& l = layers[i];
     if (!l.qkv || !l.o || !l.gate_up || !l.down || !l.ln1 || !l.ln2 || !l.k_cache || !l.v_cache)
       return NVJ_ERR_NULL_POINTER;
     if ((l.q_norm == nullptr) != (l.k_norm == nullptr)) return NVJ_ERR_NULL_POINTER;
     for (const void* p : {l.qkv, l.o, l.gate_up, l.down, (const void*)l.ln1, (const void*)l.ln2,
-                          (const void*)l.k_cache, (const void*)l.v_cache})
+                          (const void*)l.q_norm, (const void*)l.k_norm, (const void*)l.k_cache,
+                          (const void*)l.v_cache})
       bits |= reinterpret_cast<uintptr_t>(p);
   }
   if (bits & 15u) return NVJ_ERR_ALIGNMENT;

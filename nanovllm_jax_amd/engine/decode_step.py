@@ -313,6 +313,9 @@ class DecodeStepRunner:
         need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens, sequences)
         if need == 0:
             return None
+        ws = None if prefill else ws0 or self._eager_workspace(context)
+        if ws is not None and not ws.buffer.device == ws.counters.device == dev:
+            return None
         b = _lib.DecoderBatch(num_tokens=tokens, num_sequences=sequences, is_prefill=int(prefill))
         b.input_ids, b.positions, b.slot_mapping = (input_ids.data_ptr(), positions.data_ptr(),
                                                     sl.data_ptr())
@@ -326,13 +329,12 @@ class DecodeStepRunner:
             last = last.contiguous()
             b.last_token_indices = last.data_ptr()
         else:
-            ws = ws0 or self._eager_workspace(context)
             b.context_lens, b.chunk = context.context_lens.data_ptr(), int(context.decode_split)
             b.partials, b.partial_bytes = ws.buffer.data_ptr(), ws.buffer.numel()
             if b.chunk == 0:
                 counters = ws._counters_for(4 * (1 + sequences * self.cfg.num_heads))
                 b.counters, b.counter_bytes = counters.data_ptr(), counters.numel() * 4
-                b.clear_counters, ws._clear_next = int(ws._clear_next), False
+                b.clear_counters = int(ws._clear_next)
         logits = torch.empty((sequences, model.vocab), dtype=torch.bfloat16, device=dev)
         b.logits = logits.data_ptr()
         scratch = torch.empty(need, dtype=torch.uint8, device=dev)
@@ -341,6 +343,8 @@ class DecodeStepRunner:
                 torch.cuda.current_stream(dev).cuda_stream, ctypes.byref(model), layers,
                 ctypes.byref(b), scratch.data_ptr(), need)
         _lib.check(code, "nvj_decoder_step_launch")
+        if b.clear_counters:
+            ws._clear_next = False
         return logits
 
     def forward(self, input_ids, positions, context: AttentionContext):

@@ -128,6 +128,47 @@ def test_workspace_and_chunk_queries():
     assert paged_decode_workspace_bytes(1, 8, 128, 32, 256, 8, 0) == 256 + (256 * 8 + 8) * 130 * 4
 
 
+def test_decoder_step_argument_validation():
+    """The step says beforehand which sizes it cannot be given, and refuses bad pointers."""
+    from nanovllm_jax_amd import _lib
+    lib = _lib.load()
+    p = 0x1000
+    fields = dict(embed=p, final_norm=p, cos_sin=p, num_layers=1, hidden=1024, num_heads=16,
+                  num_kv_heads=8, head_dim=128, intermediate=3072, vocab=1000, max_position=64,
+                  block_size=64, num_blocks=4, eps=1e-6, scale=0.1)
+
+    def need(tokens, sequences, **kw):
+        return lib.nvj_decoder_step_workspace_bytes(
+            ctypes.byref(_lib.DecoderModel(**{**fields, **kw})), tokens, sequences)
+
+    def launch(model=None, layer=None, **batch):
+        m = _lib.DecoderModel(**{**fields, **(model or {})})
+        one = {n: p for n, _ in _lib.DecoderLayer._fields_}
+        layers = (_lib.DecoderLayer * 1)(_lib.DecoderLayer(**{**one, **(layer or {})}))
+        b = _lib.DecoderBatch(**{**dict(input_ids=p, positions=p, slot_mapping=p, context_lens=p,
+                                        block_tables=p, logits=p, num_tokens=1, num_sequences=1,
+                                        max_blocks=1), **batch})
+        return lib.nvj_decoder_step_launch(None, ctypes.byref(m), layers, ctypes.byref(b), p,
+                                           1 << 40)
+
+    assert need(1, 1) > 0 and need(1 << 19, 1) > 0
+    # rows whose products pass the 4 GiB of an operand: said here, refused there
+    limit = (1 << 32) // (2 * 3072)
+    for tokens in (limit + 1, 1 << 20):
+        assert need(tokens, 1) == 0
+        assert launch(num_tokens=tokens, num_sequences=tokens) == -3
+    assert need(1 << 18, 1, hidden=8192, intermediate=29568) == 0
+    assert need(1, 1, hidden=1000) == need(1, 1, head_dim=64) == need(1, 1, vocab=1001) == 0
+    for field in ("embed", "final_norm", "cos_sin"):
+        assert launch(model={field: 0}) == -1 and launch(model={field: p + 4}) == -8
+    for field in ("qkv", "o", "gate_up", "down", "ln1", "ln2", "k_cache", "v_cache"):
+        assert launch(layer={field: 0}) == -1 and launch(layer={field: p + 4}) == -8
+    for field in ("q_norm", "k_norm"):
+        assert launch(layer={field: 0}) == -1 and launch(layer={field: p + 4}) == -8
+    assert launch(logits=p + 8) == -8
+    assert launch(is_prefill=1, cu_seqlens_q=p, cu_seqlens_k=p) == -1     # no last_token_indices
+
+
 def test_host_mirror_refuses_cpu_tensors():
     """No CPU fallback: host tensors are an error, not a slow path."""
     from nanovllm_jax_amd import Attention, create_decode_context, paged_attention, store_kv_to_cache

@@ -302,3 +302,16 @@ def test_token_ids_outside_the_vocabulary(rows):
     got = runner._native_forward(ids, pos, ctx).float()
     keep = [i for i in range(rows) if i not in (1, 2)]
     assert got[1:3].isnan().all() and torch.equal(got[keep], want[keep])
+
+
+def test_native_step_declines_a_workspace_of_another_device():
+    print("case workspace on the host", flush=True)
+    from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
+    _, runner = _small_runner()
+    inputs = _decode_inputs(runner, 3)
+    ws = DecodeWorkspace(1 << 20, "cpu")
+    for a in runner.attn:
+        a.workspace = ws
+    assert runner._native_forward(*inputs) is None
+    with pytest.raises(ValueError):
+        runner.forward(*inputs)
