@@ -38,9 +38,9 @@ from ..layers.prefill_attention import paged_prefill_attention
 from ..layers.qk_rope_store import qk_norm_rope_store
 from ..utils.context import AttentionContext, create_decode_context, create_prefill_context
 
-# Up to this many token rows a step is one native call (nvj_decoder_step_launch); beyond
-# it, and for models that call is not built for, it is library GEMMs with the element-wise
-# launches between them.
+# A step is one native call (nvj_decoder_step_launch) up to this many token rows and where
+# that is the faster way; otherwise, and for models the call is not built for, it is library
+# GEMMs with the element-wise launches between them.
 _NATIVE_STEP_ROWS = 1 << 18
 _LAYER_WEIGHTS = itemgetter("qkv", "o", "gate_up", "down", "ln1", "ln2", "q_norm", "k_norm")
 
@@ -63,6 +63,37 @@ class DecodeModelConfig:
     max_position: int = 4096
     block_size: int = 256
     num_kvcache_blocks: int = 512
+
+
+def _native_step_pays(tokens: int, hidden: int, q_width: int, kv_width: int,
+                      intermediate: int) -> bool:
+    """Whether the native step is at least as fast as library GEMMs for these sizes.
+
+    It saves launches, the passes of the element-wise stages and host work per launch;
+    the library's products are the faster ones where they are large.  Measured per layer,
+    native against library (decode replayed from a graph, prefill eager), us:
+
+    ========================  =====================================================
+    hidden (intermediate)     rows: native / library
+    ========================  =====================================================
+    1024 (3072)               4: 37 / 59, 128: 46 / 64, 800: 72 / 161, 4400: 216 / 240,
+                              8000: 348 / 339, 16000: 643 / 589
+    2048 (6144)               4: 76 / 90, 64: 78 / 94, 200: 102 / 163, 600: 151 / 165,
+                              1200: 203 / 199, 8000: 762 / 672
+    2048 (11008)              48: 98 / 114, 96: 124 / 118, 200: 134 / 162, 600: 212 / 197
+    2560 (9728)               4: 104 / 135, 64: 128 / 125, 96: 144 / 137, 200: 166 / 163,
+                              1200: 368 / 344
+    4096 (12288)              4: 143 / 149, 32: 146 / 144, 64: 174 / 162, 400: 304 / 261
+    5120 (25600)              4: 286 / 326, 32: 316 / 341, 128: 497 / 439
+    8192 (29568)              4: 455 / 423, 64: 499 / 484, 1200: 2042 / 1613
+    ========================  =====================================================
+    """
+    products = tokens * (hidden * (2 * q_width + 2 * kv_width) + 3 * hidden * intermediate)
+    if hidden <= 1024:
+        return products <= 100e9
+    if hidden <= 2560:
+        return tokens <= 64 or (tokens > 128 and products <= 40e9)
+    return hidden <= 5120 and tokens <= 32
 
 
 def prepare_block_tables(block_tables: list[list[int]]) -> np.ndarray:
@@ -309,6 +340,9 @@ class DecodeStepRunner:
         if built is None:
             return None
         model, layers, _memory = built
+        if not _native_step_pays(tokens, model.hidden, model.num_heads * model.head_dim,
+                                 model.num_kv_heads * model.head_dim, model.intermediate):
+            return None
         lib, dev = _lib.load(), self.embed.device
         need = lib.nvj_decoder_step_workspace_bytes(ctypes.byref(model), tokens, sequences)
         if need == 0:

@@ -169,6 +169,20 @@ def test_decoder_step_argument_validation():
     assert launch(is_prefill=1, cu_seqlens_q=p, cu_seqlens_k=p) == -1     # no last_token_indices
 
 
+def test_native_step_is_taken_where_it_was_measured_faster():
+    from nanovllm_jax_amd.engine.decode_step import _native_step_pays as pays
+    for sizes, rows_native, rows_library in (
+            ((1024, 2048, 1024, 3072), (1, 16, 17, 128, 4400), (8000, 16000)),
+            ((2048, 2048, 1024, 6144), (1, 64, 200, 600), (1200, 8000)),
+            ((2048, 2048, 256, 11008), (1, 64, 200), (96, 128, 600, 800)),
+            ((2560, 4096, 1024, 9728), (1, 64), (96, 600, 1200)),
+            ((4096, 4096, 1024, 12288), (1, 32), (48, 64, 400, 1200)),
+            ((5120, 8192, 1024, 25600), (1, 32), (128, 8000)),
+            ((8192, 8192, 1024, 29568), (), (1, 64, 1200))):
+        assert all(pays(rows, *sizes) for rows in rows_native), sizes
+        assert not any(pays(rows, *sizes) for rows in rows_library), sizes
+
+
 def test_host_mirror_refuses_cpu_tensors():
     """No CPU fallback: host tensors are an error, not a slow path."""
     from nanovllm_jax_amd import Attention, create_decode_context, paged_attention, store_kv_to_cache

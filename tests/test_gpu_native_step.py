@@ -315,3 +315,12 @@ def test_native_step_declines_a_workspace_of_another_device():
     assert runner._native_forward(*inputs) is None
     with pytest.raises(ValueError):
         runner.forward(*inputs)
+
+
+def test_wide_models_take_the_library_products():
+    print("case wide model", flush=True)
+    _, runner = _small_runner(hidden=4096, inter=512, heads=2, layers=1)
+    for rows, native in ((32, True), (33, False)):
+        inputs = _decode_inputs(runner, rows)
+        assert (runner._native_forward(*inputs) is not None) == native
+        assert not runner.forward(*inputs).isnan().any()
