@@ -368,7 +368,8 @@ NVJ_API int nvj_paged_decode_static_launch(void* stream,
  * head_dim], slot_mapping [batch]) and the decode attention behind it, in one launch with
  * the same results: attention sees every new row wherever its slot lies.  For chunk 0
  * (counters and partials as nvj_paged_decode_launch_counters; counters NULL on the null
- * stream: words of the library's that only such calls use) and NVJ_CHUNK_WHOLE_SEQUENCE.
+ * stream: two regions of the library's that only such calls use, in turn, each cleared by
+ * the call in front) and NVJ_CHUNK_WHOLE_SEQUENCE.
  * nvj_paged_decode_store_takes says whether the sizes allow it: 0 no (more than 64 rows or
  * more than one KV head of a row per compute unit, head_dim other than 128, a fixed chunk:
  * NVJ_ERR_UNSUPPORTED), 1 yes, and counters and partials are not used, 2 yes.
@@ -385,6 +386,10 @@ NVJ_API int nvj_paged_decode_store_launch(void* stream, const void* q, const voi
                             int32_t head_dim, int32_t block_size, int32_t max_blocks,
                             int32_t num_blocks, float scale, int32_t chunk, int32_t dtype,
                             int32_t k_dtype, int32_t v_dtype);
+
+/* The region the current device's last such call with counters NULL used; word 0 is its
+ * stale flag. */
+NVJ_API int nvj_paged_decode_null_stream_counters(void** counters, size_t* bytes);
 
 /*
  * Fused per-head QK-RMSNorm + rotary embedding + KV-cache store: everything the

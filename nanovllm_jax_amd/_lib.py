@@ -84,6 +84,8 @@ SYMBOLS = {
     "nvj_paged_decode_counters_reset": (_c.c_int, [_c.c_void_p, _c.c_void_p, _c.c_size_t]),
     "nvj_paged_decode_library_counters": (_c.c_int, [_c.POINTER(_c.c_void_p),
                                                      _c.POINTER(_c.c_size_t)]),
+    "nvj_paged_decode_null_stream_counters": (_c.c_int, [_c.POINTER(_c.c_void_p),
+                                                         _c.POINTER(_c.c_size_t)]),
     "nvj_paged_decode_static_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p,
         _c.c_void_p,

@@ -37,6 +37,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 
 #include "cache_rows.h"
 #include "launch.h"
@@ -224,8 +225,10 @@ struct NewRows {
   int num_slots;
   bool key_f32, value_f32;
   int main_wgs;          // workgroups behind these store a row each; 0: workgroup b stores row b
+  int32_t* clear;        // balanced kernel: kNullStreamWords words for workgroup 0 to zero, or null
 };
 constexpr int kMaxNewRows = 64;
+constexpr int kNullStreamWords = 512;   // see null_stream_counters: one per thread of a workgroup
 
 template <bool F16>
 __device__ __forceinline__ uint4 new_piece(const void* rows, bool f32, int64_t piece) {
@@ -1506,6 +1509,10 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
     const int n = steps_of(base + lane);
     total += __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
   }
+  if constexpr (NEW) {
+    static_assert(NW * 64 == kNullStreamWords, "a word per thread");
+    if (g == 0 && fresh.clear != nullptr) fresh.clear[threadIdx.x] = 0;
+  }
   // No step belongs to an empty sequence: its output row (zeros, 0 / (0 + 1e-9))
   // is written here, sequence b by workgroup b modulo the grid.  The lengths of
   // the first kKeep * 64 sequences are in registers already.
@@ -2511,25 +2518,47 @@ extern "C" int nvj_paged_decode_counters_reset(void* stream, void* counters,
              : NVJ_ERR_LAUNCH;
 }
 
-// Counters of the calls that bring none, on the null stream only: its launches follow each
-// other, and it is never recorded into a graph that another stream replays.
-static __device__ __align__(256) int32_t null_stream_counters[16384];
+// Counters of the store-and-attend calls that bring none, on the null stream only: its
+// launches follow each other, and it is never recorded into a graph that another stream
+// replays.  Two regions that such calls use in turn: each launch also zeroes the region of
+// the next one, so that a call begins on cleared counters without a clearing launch in front
+// of it, and a count left wrong by one launch (lengths rewritten under it, say) ends with it.
+static __device__ __align__(256) int32_t null_stream_counters[2][kNullStreamWords];
 
 namespace {
-int null_stream_counters_of_current_device(void** out) {
-  static std::atomic<void*> address[kMaxDevices];
+struct NullStreamCounters {
+  std::mutex lock;   // held over a launch: the order of the launches is the order of the turns
+  int32_t* base = nullptr;
+  int next = 0;      // the region of the next launch
+};
+// Of the current device; null if there is none.
+NullStreamCounters* null_stream_counters_of_current_device() {
+  static NullStreamCounters of_device[kMaxDevices];
   int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return NVJ_ERR_LAUNCH;
-  void* p = address[dev].load(std::memory_order_acquire);
-  if (p == nullptr) {
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(null_stream_counters)) != hipSuccess || p == nullptr)
-      return NVJ_ERR_LAUNCH;
-    address[dev].store(p, std::memory_order_release);
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  return &of_device[dev];
+}
+// With the lock held.
+bool find_base(NullStreamCounters* c) {
+  void* p = nullptr;
+  if (c->base == nullptr) {
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(null_stream_counters)) != hipSuccess) return false;
+    c->base = static_cast<int32_t*>(p);
   }
-  *out = p;
-  return NVJ_OK;
+  return c->base != nullptr;
 }
 }  // namespace
+
+extern "C" int nvj_paged_decode_null_stream_counters(void** counters, size_t* bytes) {
+  if (!counters) return NVJ_ERR_NULL_POINTER;
+  if (bytes) *bytes = kNullStreamWords * sizeof(int32_t);
+  NullStreamCounters* c = null_stream_counters_of_current_device();
+  if (!c) return NVJ_ERR_LAUNCH;
+  std::lock_guard<std::mutex> hold(c->lock);
+  if (!find_base(c)) return NVJ_ERR_LAUNCH;
+  *counters = c->base + (1 - c->next) * kNullStreamWords;
+  return NVJ_OK;
+}
 
 extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, const void* k_cache,
                                                 const void* v_cache, const int32_t* block_tables,
@@ -2578,7 +2607,7 @@ extern "C" int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads
   if (rows > compute_units()) return 0;
   if (chunk == NVJ_CHUNK_WHOLE_SEQUENCE) return 1;
   if (chunk != 0 || nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads) >
-                        sizeof(null_stream_counters))
+                        kNullStreamWords * sizeof(int32_t))
     return 0;
   return table_of_short_rows(rows, (int64_t)max_blocks * block_size) ? 1 : 2;
 }
@@ -2598,28 +2627,37 @@ extern "C" int nvj_paged_decode_store_launch(
   if (!key || !value || !slot_mapping) return NVJ_ERR_NULL_POINTER;
   if ((reinterpret_cast<uintptr_t>(key) | reinterpret_cast<uintptr_t>(value)) & 15u)
     return NVJ_ERR_ALIGNMENT;
+  NewRows n = {};
+  NullStreamCounters* own = nullptr;
+  std::unique_lock<std::mutex> turn;
   if (takes == 2) {
     if (!counters && stream) return NVJ_ERR_NULL_POINTER;
     if (!counters) {
-      const int rc = null_stream_counters_of_current_device(&counters);
-      if (rc != NVJ_OK) return rc;
+      own = null_stream_counters_of_current_device();
+      if (!own) return NVJ_ERR_LAUNCH;
+      turn = std::unique_lock<std::mutex>(own->lock);
+      if (!find_base(own)) return NVJ_ERR_LAUNCH;
+      counters = own->base + own->next * kNullStreamWords;
+      n.clear = own->base + (1 - own->next) * kNullStreamWords;
     } else {
       if (reinterpret_cast<uintptr_t>(counters) & 3u) return NVJ_ERR_ALIGNMENT;
       if (counter_bytes < nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads))
         return NVJ_ERR_WORKSPACE;
     }
   }
-  NewRows n = {};
   n.key = key;
   n.value = value;
   n.slots = slot_mapping;
   n.num_slots = num_blocks * block_size;
   n.key_f32 = k_dtype == NVJ_DTYPE_F32;
   n.value_f32 = v_dtype == NVJ_DTYPE_F32;
-  return launch_decode(stream, q, k_cache, v_cache, block_tables, context_lens, out, partials,
-                       partial_bytes, static_cast<int32_t*>(counters), batch, num_heads,
-                       num_kv_heads, head_dim, block_size, max_blocks, num_blocks, scale, chunk,
-                       dtype, NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE | NVJ_PHASE_SHORT_ROWS, &n);
+  const int rc = launch_decode(
+      stream, q, k_cache, v_cache, block_tables, context_lens, out, partials, partial_bytes,
+      static_cast<int32_t*>(counters), batch, num_heads, num_kv_heads, head_dim, block_size,
+      max_blocks, num_blocks, scale, chunk, dtype,
+      NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE | NVJ_PHASE_SHORT_ROWS, &n);
+  if (own && rc == NVJ_OK) own->next = 1 - own->next;   // (an error has launched nothing)
+  return rc;
 }
 
 extern "C" int nvj_paged_decode_static_launch(void* stream, const void* q, const void* k_cache,

@@ -1080,3 +1080,47 @@ def test_store_in_the_same_launch(lens, split, dtype, k_f32, own_workspace):
         torch.testing.assert_close(got.float(), want.float(), rtol=1e-2, atol=2e-3)
         for c, w in zip(caches, want_caches):
             assert torch.equal(c.view(torch.int16), w.view(torch.int16))
+
+
+def test_counts_left_wrong_by_one_call_end_with_it():
+    """Without a workspace on the null stream the store-and-attend launch uses two counter
+    regions in turn and clears the next one: whatever a launch leaves in its own is gone
+    before that region's next turn."""
+    print("case counters of the null stream", flush=True)
+    import ctypes
+    import torch
+    from nanovllm_jax_amd import Attention, _lib, create_decode_context
+    lib, hip, dev = _lib.load(), _hip_runtime(), "cuda:0"
+    assert torch.cuda.current_stream().cuda_stream == 0
+    Hq, Hkv, D, bs, ctx = 16, 8, 128, 64, [3000, 2500, 2800]
+    q, kc, vc, bt, ctx = make_problem(41, 3, Hq, Hkv, D, bs, sum(-(-c // bs) for c in ctx) + 1, ctx)
+    assert lib.nvj_paged_decode_store_takes(3, Hq, Hkv, D, bs, bt.shape[1], len(kc), 0) == 2
+    attn = Attention(Hq, D, 0.088, Hkv, bs)
+    attn.set_kv_cache(bits_to_torch(kc, dev), bits_to_torch(vc, dev))
+    context = create_decode_context(
+        torch.from_numpy(ctx).to(dev), torch.full((3,), -1, dtype=torch.int32, device=dev),
+        torch.from_numpy(bt).to(dev))
+    tq = bits_to_torch(q, dev)
+    new = torch.zeros(3, Hkv, D, dtype=torch.bfloat16, device=dev)
+    want = oracle(q, kc, vc, bt, ctx, 0.088, bs)
+
+    def region():
+        at, size = ctypes.c_void_p(), ctypes.c_size_t()
+        assert lib.nvj_paged_decode_null_stream_counters(ctypes.byref(at), ctypes.byref(size)) == 0
+        torch.cuda.synchronize()
+        words = (ctypes.c_int32 * (size.value // 4))()
+        assert hip.hipMemcpy(words, at, size.value, 2) == 0          # device to host
+        return at, size.value, words
+
+    first = torch_to_bits(attn(tq, new, new, context))
+    assert_close_bf16(first, want, what="clean")
+    seen = set()
+    for _ in range(4):
+        at, nbytes, words = region()
+        seen.add(at.value)
+        assert not any(words)                        # counters and flag left at zero
+        words[:] = [1] * len(words)                  # as if this launch had been cut short
+        assert hip.hipMemcpy(at, words, nbytes, 1) == 0
+        for _ in range(3):
+            assert np.array_equal(torch_to_bits(attn(tq, new, new, context)), first)
+    assert len(seen) == 2
