@@ -89,6 +89,23 @@ int store(void* stream, const Tensor& key, const Tensor& value, const Caches& c,
       type_code(value.scalar_type()), c.dtype, k_rows, v_rows, clear, clear_bytes);
 }
 
+// The interpreter is free for other threads while a call allocates and enqueues: either can
+// wait, for memory to come back or for room in the queue.  (The caller holds references to
+// every tensor of the call.)
+struct OtherThreadsRun {
+  PyThreadState* state = PyEval_SaveThread();
+  ~OtherThreadsRun() { end(); }
+  void end() {
+    if (state) PyEval_RestoreThread(state);
+    state = nullptr;
+  }
+};
+
+PyObject* result(OtherThreadsRun* released, Tensor* out, int code) {
+  released->end();
+  return code == NVJ_OK ? THPVariable_Wrap(std::move(*out)) : PyLong_FromLong(code);
+}
+
 // decode(q, k, v, k_cache, v_cache, slot_mapping, block_tables, context_lens, scale,
 //        block_size, chunk, partials | None, counters | None, device, stream)
 PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -112,8 +129,8 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   void *partials = nullptr, *counters = nullptr;
   size_t partial_bytes = 0, counter_bytes = 0, clear_bytes = 0;
-  Tensor own;
   const Tensor *given, *given_counters;
+  size_t own_bytes = 0;
   // store and attention in one launch: 0 not for these sizes, 1 without counters, 2 with
   int together = nvj_paged_decode_store_takes(batch, heads, c.heads, c.dim, c.page, max_blocks,
                                               c.num_blocks, chunk);
@@ -125,15 +142,10 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (args[11] == Py_None) {
       // a workspace for this call alone; its counters are cleared by the store, unless the
       // library has some for this stream
-      own = at::empty({(int64_t)need}, q->options().dtype(at::kByte));
-      char* base = static_cast<char*>(own.data_ptr());
-      partials = base + head;
+      own_bytes = need;
       partial_bytes = need - head;
       if (stream != nullptr) together = 0;
-      if (together == 0) {
-        counters = base;
-        counter_bytes = clear_bytes = head;
-      }
+      if (together == 0) counter_bytes = clear_bytes = head;
     } else {
       if (!get(args[11], &given) || !get(args[12], &given_counters) ||
           given->device() != q->device() || given_counters->device() != q->device() ||
@@ -146,10 +158,18 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       if (partial_bytes + head < need || counter_bytes < head) Py_RETURN_NONE;
     }
   }
-  Tensor out = at::empty_like(*q);
   const int32_t* table_ptr = static_cast<const int32_t*>(tables->data_ptr());
   const int32_t* lens_ptr = static_cast<const int32_t*>(lens->data_ptr());
+  Tensor own, out;
   int code;
+  OtherThreadsRun released;
+  if (own_bytes > 0) {
+    own = at::empty({(int64_t)own_bytes}, q->options().dtype(at::kByte));
+    char* base = static_cast<char*>(own.data_ptr());
+    partials = base + (own_bytes - partial_bytes);
+    if (together == 0) counters = base;
+  }
+  out = at::empty_like(*q);
   if (together != 0) {
     code = nvj_paged_decode_store_launch(
         stream, q->data_ptr(), key->data_ptr(), value->data_ptr(),
@@ -157,10 +177,10 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         lens_ptr, out.data_ptr(), partials, partial_bytes, counters, counter_bytes, batch, heads,
         c.heads, c.dim, c.page, max_blocks, c.num_blocks, (float)scale, chunk, c.dtype,
         type_code(key->scalar_type()), type_code(value->scalar_type()));
-    return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+    return result(&released, &out, code);
   }
   code = store(stream, *key, *value, c, *slots, nullptr, nullptr, clear_bytes ? counters : nullptr,
-                   clear_bytes);
+               clear_bytes);
   if (code == NVJ_OK) {
     code = chunk == 0
                ? nvj_paged_decode_launch_counters(
@@ -174,7 +194,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                      c.num_blocks, (float)scale, chunk, c.dtype,
                      NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE);
   }
-  return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+  return result(&released, &out, code);
 }
 
 // prefill(q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k,
@@ -205,7 +225,8 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   // packed rows in the cache's type: where a float32 source is rounded for the cache
   // anyway, the store leaves a packed copy
-  Tensor k_rows, v_rows;
+  Tensor k_rows, v_rows, out;
+  OtherThreadsRun released;
   void *kp = key->data_ptr(), *vp = value->data_ptr(), *k_copy = nullptr, *v_copy = nullptr;
   if (!paged && key->scalar_type() == at::kFloat) {
     k_rows = at::empty(key->sizes(), q->options());
@@ -215,7 +236,7 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     v_rows = at::empty(value->sizes(), q->options());
     vp = v_copy = v_rows.data_ptr();
   }
-  Tensor out = at::empty_like(*q);
+  out = at::empty_like(*q);
   const int32_t* cq = static_cast<const int32_t*>(cu_q->data_ptr());
   const int32_t* ck = static_cast<const int32_t*>(cu_k->data_ptr());
   int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
@@ -228,7 +249,7 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                  : nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck,
                                                 out.data_ptr(), tokens, batch, heads, c.heads,
                                                 c.dim, (float)scale, c.dtype);
-  return code == NVJ_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(code);
+  return result(&released, &out, code);
 }
 
 // decoder_layers(tensors, num_heads, num_kv_heads, head_dim, device): the weights of a
