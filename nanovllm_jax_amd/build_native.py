@@ -1,4 +1,5 @@
-"""Compile the HIP kernels and their C ABI into one shared library for gfx950.
+"""Compile the HIP kernels and their C ABI into one shared library for gfx950, and the
+native host side that is linked to it.
 
 ``hipcc`` cross-compiles without a GPU.  The library is built in-tree
 (``nanovllm_jax_amd/_native/libnvj_paged_attn.so``) so that it travels with the
@@ -133,5 +134,11 @@ def build_c_caller(verbose: bool = True) -> str:
     return out
 
 
+def main(argv: list[str]) -> None:
+    """What the package loads at run time: the library and the host side linked to it."""
+    print(build(extra_flags=tuple(argv)))
+    print(build_host())
+
+
 if __name__ == "__main__":
-    print(build(extra_flags=tuple(sys.argv[1:])))
+    main(sys.argv[1:])

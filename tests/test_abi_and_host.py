@@ -205,6 +205,16 @@ def test_host_mirror_refuses_cpu_tensors():
         attn(q, q[:, :8].contiguous(), q[:, :8].contiguous(), c)
 
 
+def test_build_command_makes_everything_the_package_loads(monkeypatch):
+    from nanovllm_jax_amd import build_native
+    made = []
+    monkeypatch.setattr(build_native, "build",
+                        lambda extra_flags=(): made.append(("library", extra_flags)))
+    monkeypatch.setattr(build_native, "build_host", lambda: made.append(("host", ())))
+    build_native.main(["-g"])
+    assert made == [("library", ("-g",)), ("host", ())]
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     from nanovllm_jax_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)
