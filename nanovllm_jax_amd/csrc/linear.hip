@@ -26,6 +26,7 @@
 #include <stdint.h>
 
 #include "launch.h"
+#include "lds_copy.h"
 #include "linear.h"
 #include "nvj_paged_attn.h"
 #include "qk_norm_rope.h"
@@ -39,6 +40,7 @@ typedef __attribute__((address_space(3))) char* lds_ptr;
 constexpr int kBK = 64;        // reduction per step: rows of 128 bytes, 8 pieces
 
 using nvj::bf16_to_f32;
+using nvj::copy16_to_lds;
 using nvj::f32_to_bf16_rne;
 using nvj::LinearArgs;
 enum Epilogue { kPlain, kSiluMul, kQkRope };
@@ -49,17 +51,6 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, p);
 }
 
-// One 16-byte global -> LDS copy per lane: lane l's piece lands at lds_base + 16 * l.
-// Counts in vmcnt; the compiler does not see it as a load, so the waits are by hand.
-__device__ __forceinline__ void copy16_to_lds(const char* base, uint32_t offset,
-                                              uint32_t lds_base) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2"
-      :
-      : "s"(lds_base), "v"(offset), "s"(base));
-}
 template <int N>
 __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

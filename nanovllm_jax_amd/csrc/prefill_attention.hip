@@ -37,6 +37,7 @@
 #include <stdint.h>
 
 #include "launch.h"
+#include "lds_copy.h"
 #include "nvj_paged_attn.h"
 
 namespace {
@@ -115,20 +116,7 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 __device__ __forceinline__ int k_position(int row, int piece) { return piece ^ (row & 15); }
 __device__ __forceinline__ int v_position(int row, int piece) { return piece ^ (2 * (row & 7)); }
 
-// One 16-byte global -> LDS copy per lane: lane l's piece lands at
-// lds_base + 16 * l (lds_base wave-uniform), fetched from base + offset.
-// Counts in vmcnt like any load; the compiler does not see it as one, so the
-// waits are written out by hand (wait_tiles_in_flight).
-__device__ __forceinline__ void copy16_to_lds(const char* base, uint32_t offset,
-                                              uint32_t lds_base) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2"
-      :
-      : "s"(lds_base), "v"(offset), "s"(base)
-      : "memory");
-}
+using nvj::copy16_to_lds;   // waits: wait_tiles_in_flight
 
 // Cooperative tile copies of a workgroup.  A tile is 512 pieces of K and 512 of
 // V; each wave copies its share of the rows of both (8 rows with 4 waves), 4
