@@ -38,33 +38,25 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bf16.h"
 #include "launch.h"
 #include "linear.h"
 #include "nvj_paged_attn.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
+using nvj::bf16_to_f32;
+using nvj::bf16x8;
+using nvj::f32_to_bf16_rne;
+using nvj::f32x4;
+using nvj::pack2_bf16;
 
 constexpr int kMaxRows = 16;   // token rows of one step: one column tile
 
-__device__ __forceinline__ float bf16_to_f32(uint16_t b) {
-  return __uint_as_float((uint32_t)b << 16);
-}
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-  return __builtin_bit_cast(uint16_t, (__bf16)f);
-}
 __device__ __forceinline__ f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  const bf16x2 p = {(__bf16)lo, (__bf16)hi};
-  return __builtin_bit_cast(uint32_t, p);
-}
-
 enum Epilogue { kPlain, kSiluMul };
 
 struct NormGemmArgs {
@@ -155,10 +147,10 @@ struct NormPrologue {
         const float4 u = x[j][i][0], v = x[j][i][1], gu = g[i][0], gv = g[i][1];
         if (kPieces % 64 == 0 || p < kPieces)
           lds[m * kPieces + (p ^ m)] =
-              make_uint4(pack2(u.x * rs * gu.x, u.y * rs * gu.y),
-                         pack2(u.z * rs * gu.z, u.w * rs * gu.w),
-                         pack2(v.x * rs * gv.x, v.y * rs * gv.y),
-                         pack2(v.z * rs * gv.z, v.w * rs * gv.w));
+              make_uint4(pack2_bf16(u.x * rs * gu.x, u.y * rs * gu.y),
+                         pack2_bf16(u.z * rs * gu.z, u.w * rs * gu.w),
+                         pack2_bf16(v.x * rs * gv.x, v.y * rs * gv.y),
+                         pack2_bf16(v.z * rs * gv.z, v.w * rs * gv.w));
       }
     }
   }

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bf16.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "linear.h"
@@ -33,23 +34,18 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((address_space(3))) char* lds_ptr;
 
 constexpr int kBK = 64;        // reduction per step: rows of 128 bytes, 8 pieces
 
 using nvj::bf16_to_f32;
+using nvj::bf16x8;
 using nvj::copy16_to_lds;
+using nvj::f32x4;
 using nvj::f32_to_bf16_rne;
 using nvj::LinearArgs;
+using nvj::pack2_bf16;
 enum Epilogue { kPlain, kSiluMul, kQkRope };
-
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  const bf16x2 p = {(__bf16)lo, (__bf16)hi};
-  return __builtin_bit_cast(uint32_t, p);
-}
 
 template <int N>
 __device__ __forceinline__ void wait_copies() {
@@ -197,13 +193,14 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
           o[e] = g / (1.0f + expf(-g)) * u;
         }
         *reinterpret_cast<uint2*>(row + (wn * (WN / 2) + 8 * j + 4 * kg) * 2) =
-            make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+            make_uint2(pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3]));
       }
     } else {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
         *reinterpret_cast<uint2*>(row + (wn * WN + 16 * j + 4 * kg) * 2) =
-            make_uint2(pack2(acc[i][j][0], acc[i][j][1]), pack2(acc[i][j][2], acc[i][j][3]));
+            make_uint2(pack2_bf16(acc[i][j][0], acc[i][j][1]),
+                       pack2_bf16(acc[i][j][2], acc[i][j][3]));
     }
   }
   __syncthreads();
@@ -369,7 +366,7 @@ __global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
       v += *reinterpret_cast<const f32x4*>(red + (c * BM + m) * kRedStride + n);
     if (m0 + m < a.M && n_tile * BN + n < a.N)
       *reinterpret_cast<uint2*>(a.out + (int64_t)(m0 + m) * a.N + n_tile * BN + n) =
-          make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+          make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
   }
 }
 

@@ -39,14 +39,19 @@
 #include <atomic>
 #include <mutex>
 
+#include "bf16.h"
 #include "cache_rows.h"
 #include "launch.h"
 #include "nvj_paged_attn.h"
+#include "wave_ops.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
+using nvj::bf16x8;
+using nvj::f16x8;
+using nvj::f32x4;
+using nvj::wave_inclusive_scan;
+using nvj::wave_max;
 
 constexpr int kMaxHeadDim = 128;     // head_dim is a template parameter: 128 or 64
 constexpr int kStep = 32;            // positions per inner step
@@ -64,8 +69,6 @@ template <int D> struct HeadDim {
 constexpr float kNegBig = -1.0e30f;  // stands for -inf without inf-inf hazards
 constexpr float kLog2e = 1.4426950408889634f;
 
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-
 // The cache element type: bf16 (F16 = false) or IEEE half (F16 = true).  The
 // kernels move 16-bit patterns; only the matrix instruction, the rounding of
 // the probabilities and of the output depend on the type.
@@ -76,9 +79,7 @@ template <> struct Elem<false> {
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-    bf16x2 p = {(__bf16)lo, (__bf16)hi};
-    return __builtin_bit_cast(uint32_t, p);
+    return nvj::pack2_bf16(lo, hi);
   }
   // the two values a packed pair stands for
   static __device__ __forceinline__ float low_of(uint32_t pair) {
@@ -94,9 +95,7 @@ template <> struct Elem<true> {
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-    f16x2 p = {(_Float16)lo, (_Float16)hi};   // round to nearest even
-    return __builtin_bit_cast(uint32_t, p);
+    return nvj::pack2_f16(lo, hi);
   }
   static __device__ __forceinline__ float low_of(uint32_t pair) {
     typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
@@ -1091,32 +1090,6 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
     }
   }
   write_output<D, F16>(a, b, kvh, lane, acc, l_run);
-}
-
-// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: a
-// Hillis-Steele scan inside each row of 16 lanes (a lane without a source in
-// its row adds 0), then the last lane of row 0 / row 2 is added to rows 1 / 3
-// (row_bcast:15) and the last lane of row 1 to rows 2 and 3 (row_bcast:31).
-__device__ __forceinline__ int wave_inclusive_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 -> rows 1, 3
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 -> rows 2, 3
-  return x;
-}
-
-// Maximum over the 64 lanes of a wave, wave-uniform, with the same DPP moves (a
-// lane without a source keeps its own value).
-__device__ __forceinline__ int wave_max(int x) {
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));
-  return __builtin_amdgcn_readlane(x, 63);
 }
 
 // ---------------------------------------------------------------------------

@@ -36,14 +36,19 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bf16.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "nvj_paged_attn.h"
+#include "wave_ops.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
+using nvj::bf16x8;
+using nvj::f16x8;
+using nvj::f32x4;
+using nvj::wave_inclusive_scan;   // (with shuffles the sequence lookup took 5 us of a short prompt)
+using nvj::wave_max;
 
 constexpr int kD = 128;
 constexpr int kPieces = 16;          // 16-byte pieces per (position, head) row
@@ -71,7 +76,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast
 // kernel moves 16-bit patterns (held as bf16x8 whatever they mean); only the
 // matrix instruction, the rounding of probabilities and output and the
 // constant 1 depend on the type.
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 template <bool F16> struct Elem;
 template <> struct Elem<false> {
   static constexpr uint32_t kOnes = 0x3F803F80u;   // two bf16 ones
@@ -79,9 +83,7 @@ template <> struct Elem<false> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-    bf16x2 p = {(__bf16)lo, (__bf16)hi};
-    return __builtin_bit_cast(uint32_t, p);
+    return nvj::pack2_bf16(lo, hi);
   }
 };
 template <> struct Elem<true> {
@@ -91,9 +93,7 @@ template <> struct Elem<true> {
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-    f16x2 p = {(_Float16)lo, (_Float16)hi};   // round to nearest even
-    return __builtin_bit_cast(uint32_t, p);
+    return nvj::pack2_f16(lo, hi);
   }
 };
 
@@ -382,30 +382,6 @@ struct PrefillArgs {
   const int32_t* block_tables;   // [B, max_blocks]
   int block_size, max_blocks, num_blocks;
 };
-
-// Inclusive prefix sum over the 64 lanes of a wave with DPP moves.  (With shuffles
-// through LDS the lookup below took 5 us of a short prompt's workgroup.)
-__device__ __forceinline__ int wave_inclusive_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 -> rows 1, 3
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 -> rows 2, 3
-  return x;
-}
-
-// Maximum over the 64 lanes, wave-uniform, with the same DPP moves (a lane without a
-// source keeps its own value).
-__device__ __forceinline__ int wave_max(int x) {
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));
-  return __builtin_amdgcn_readlane(x, 63);
-}
 
 // grid.x = 8 * ceil(tile bound * Hkv / 8) workgroups (see the work-item mapping below).
 // PAGED: keys and values come from the block-paged cache through block_tables,

@@ -8,16 +8,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bf16.h"
+
 namespace nvj {
-
-__device__ __forceinline__ float bf16_to_f32(uint16_t b) {
-  return __uint_as_float((uint32_t)b << 16);
-}
-
-// round to nearest even, NaN kept quiet (the hardware conversion)
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-  return __builtin_bit_cast(uint16_t, (__bf16)f);
-}
 
 __device__ __forceinline__ void unpack4(uint2 p, float (&f)[4]) {
   f[0] = __uint_as_float(p.x << 16); f[1] = __uint_as_float(p.x & 0xFFFF0000u);
