@@ -26,6 +26,7 @@
 #include <stdint.h>
 
 #include "bf16.h"
+#include "device.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "linear.h"
@@ -387,8 +388,8 @@ hipError_t launch_tiles(hipStream_t s, LinearArgs a) {
                      dim3(256), s, a);
 }
 
-// Tile sizes.  A launch of T tiles takes rounds of 256 (or 512: two workgroups share a
-// CU), each round a fixed 3 us and per step of 64 a time between `low` (few CUs busy)
+// Tile sizes.  A launch of T tiles takes rounds of one workgroup per CU (or two, where they
+// share one), each round a fixed 3 us and per step of 64 a time between `low` (few CUs busy)
 // and `full` (all of them: the L2s and the power limit share out).  Measured on an
 // MI355X over 300 .. 4400 rows and the four projections of a 1024-wide layer, us:
 struct TileShape {
@@ -404,11 +405,12 @@ constexpr TileShape kShapes[] = {
 int best_shape(int64_t m, int64_t n, int k, int min_bn) {
   int best = 0;
   float best_cost = 0.f;
+  const int64_t cus = nvj::compute_units();
   for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
     const TileShape& t = kShapes[i];
     if (t.bn < min_bn) continue;
     const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-    const int64_t slots = 256 * t.per_cu, whole = tiles / slots, rest = tiles % slots;
+    const int64_t slots = cus * t.per_cu, whole = tiles / slots, rest = tiles % slots;
     const float step_full = t.full, per_step = (float)(k / kBK);
     float cost = (float)whole * (per_step * step_full + 3.f);
     if (rest > 0)

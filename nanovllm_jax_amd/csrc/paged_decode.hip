@@ -41,6 +41,7 @@
 
 #include "bf16.h"
 #include "cache_rows.h"
+#include "device.h"
 #include "launch.h"
 #include "nvj_paged_attn.h"
 #include "wave_ops.h"
@@ -48,6 +49,7 @@
 namespace {
 
 using nvj::bf16x8;
+using nvj::compute_units;
 using nvj::f16x8;
 using nvj::f32x4;
 using nvj::wave_inclusive_scan;
@@ -2007,27 +2009,6 @@ int virtual_heads_per_cache_head(int group) {
   int rep = 1;
   while (group % rep != 0 || group / rep > 16) ++rep;
   return rep;
-}
-
-// Compute units of the current device (256 on an MI355X), looked up once per
-// device; 256 when no device can be asked (argument checks without a GPU).
-int compute_units() {
-  constexpr int kMaxDevicesSeen = 64;
-  static std::atomic<int> cached[kMaxDevicesSeen];
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesSeen) {
-    (void)hipGetLastError();   // not an error of any launch
-    return 256;
-  }
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (n > 0) return n;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      n <= 0) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  cached[dev].store(n, std::memory_order_relaxed);
-  return n;
 }
 
 // KV heads per 8-wave workgroup of the whole-sequence mode: as many as still

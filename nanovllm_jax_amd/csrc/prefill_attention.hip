@@ -37,6 +37,7 @@
 #include <stdint.h>
 
 #include "bf16.h"
+#include "device.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "nvj_paged_attn.h"
@@ -737,11 +738,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
     }
 }
 
-// Below this many workgroups of two column groups per wave, workgroups of one: one prompt
-// of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1.
-constexpr int64_t kSmallLaunch = 256;
-// Longest tiles first: behind cached prefixes, up to 8 rounds of 512 workgroups.
-constexpr int64_t kLongestFirst = 4096;
+// Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.
+constexpr int64_t kLongestFirstPerCu = 16;
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype) {
@@ -751,15 +749,18 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
   auto tiles_of = [&](int column_groups) {
     return (blocks * a.group + (column_groups - 1) * (int64_t)a.batch) / column_groups;
   };
-  // one column group per wave while the larger workgroups would not fill the 256 CUs
-  const bool small = tiles_of(2 * kWaves) * a.num_kv_heads <= kSmallLaunch;
+  // one column group per wave while the larger workgroups would not fill the CUs: one prompt
+  // of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1
+  const int64_t cus = nvj::compute_units();
+  const bool small = tiles_of(2 * kWaves) * a.num_kv_heads <= cus;
   const int64_t tiles = tiles_of((small ? 1 : 2) * kWaves);
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
   const int64_t items = tiles * a.num_kv_heads;
   if (items > INT32_MAX - 8) return NVJ_ERR_BAD_SHAPE;
   const dim3 grid((unsigned)((items + 7) / 8 * 8)), block(kWaves * 64);
   const int nt = (int)tiles;
-  const bool may_sort = paged && a.batch > 1 && a.batch <= 256 && items <= kLongestFirst &&
+  const bool may_sort = paged && a.batch > 1 && a.batch <= 256 &&
+                        items <= kLongestFirstPerCu * cus &&
                         (int64_t)a.max_blocks * a.block_size >= 1024;
   const bool f16 = dtype == NVJ_DTYPE_F16;
   hipError_t rc;
