@@ -427,8 +427,8 @@ template <Epilogue EPI>
 hipError_t launch_shape(int shape, hipStream_t s, const LinearArgs& a) {
   switch (shape) {
     case 0:
-      if constexpr (EPI != kQkRope) return launch_tiles<64, 64, 4, EPI>(s, a);
-      [[fallthrough]];   // (a tile of whole heads is 128 wide at least)
+      if constexpr (EPI == kQkRope) return hipErrorInvalidValue;   // tiles hold whole heads
+      else return launch_tiles<64, 64, 4, EPI>(s, a);
     case 1: return launch_tiles<32, 128, 4, EPI>(s, a);
     case 2: return launch_tiles<64, 128, 3, EPI>(s, a);
     case 3: return launch_tiles<128, 128, 4, EPI>(s, a);
