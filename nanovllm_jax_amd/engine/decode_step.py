@@ -34,7 +34,7 @@ from ..layers.attention import Attention
 from ..layers.layernorm import rms_norm
 from ..layers.paged_attention import (DecodeWorkspace, choose_split, paged_attention,
                                       paged_decode_workspace_bytes)
-from ..layers.prefill_attention import paged_prefill_attention
+from ..layers.prefill_attention import packed_qkv_attention, paged_prefill_attention
 from ..layers.qk_rope_store import qk_norm_rope_store
 from ..utils.context import AttentionContext, create_decode_context, create_prefill_context
 
@@ -329,7 +329,8 @@ class DecodeStepRunner:
         if prefill:
             # any other count of rows, or indices from the host, as tensor indexing takes them
             last = context.last_token_indices
-            if context.cu_seqlens_k.shape != (sequences + 1,) or sequences == 0 or \
+            offsets = (context.cu_seqlens_q.shape, context.cu_seqlens_k.shape)
+            if offsets != ((sequences + 1,),) * 2 or sequences <= 0 or \
                     not isinstance(last, torch.Tensor) or last.shape != (sequences,) or \
                     last.dtype not in (torch.int32, torch.int64) or \
                     last.device != self.embed.device:
@@ -398,25 +399,26 @@ class DecodeStepRunner:
                 h, residual = self._rms(h, lw["ln1"], residual)
             qkv = F.linear(h, lw["qkv"])
             if self.fused_qk_rope_store:
-                if context.is_prefill and context.block_tables is None:
-                    o = self._rotate_store_prefill(qkv, positions, lw, attn, context)
+                packed = context.is_prefill and context.block_tables is None
+                q = qk_norm_rope_store(qkv, positions, self.cos_sin, lw["q_norm"], lw["k_norm"],
+                                       c.rms_norm_eps, attn.k_cache, attn.v_cache,
+                                       context.slot_mapping, c.num_heads, c.num_kv_heads,
+                                       c.head_dim, in_place=packed)
+                if packed:
+                    o = packed_qkv_attention(q, context.cu_seqlens_q, context.cu_seqlens_k,
+                                             c.num_heads, c.num_kv_heads, c.head_dim, attn.scale)
+                elif context.is_prefill:
+                    # prompt rows behind a cached prefix: keys and values, the rows the
+                    # fused launch just stored included, come from the paged cache
+                    o = paged_prefill_attention(q, attn.k_cache, attn.v_cache,
+                                                context.block_tables, context.cu_seqlens_q,
+                                                context.cu_seqlens_k, attn.scale)
                 else:
-                    q = qk_norm_rope_store(qkv, positions, self.cos_sin, lw["q_norm"],
-                                           lw["k_norm"], c.rms_norm_eps, attn.k_cache,
-                                           attn.v_cache, context.slot_mapping, c.num_heads,
-                                           c.num_kv_heads, c.head_dim)
-                    if context.is_prefill:
-                        # prompt rows behind a cached prefix: keys and values, the rows the
-                        # fused launch just stored included, come from the paged cache
-                        o = paged_prefill_attention(q, attn.k_cache, attn.v_cache,
-                                                    context.block_tables, context.cu_seqlens_q,
-                                                    context.cu_seqlens_k, attn.scale)
-                    else:
-                        o = paged_attention(q, attn.k_cache, attn.v_cache, context.block_tables,
-                                            context.context_lens, attn.scale, attn.block_size,
-                                            chunk=context.decode_split,
-                                            workspace=attn.workspace or
-                                            self._eager_workspace(context))
+                    o = paged_attention(q, attn.k_cache, attn.v_cache, context.block_tables,
+                                        context.context_lens, attn.scale, attn.block_size,
+                                        chunk=context.decode_split,
+                                        workspace=attn.workspace or
+                                        self._eager_workspace(context))
                 h = F.linear(o.reshape(-1, qs), lw["o"])
                 h, residual = self._rms(h, lw["ln2"], residual)
                 h = F.linear(self._silu_mul(F.linear(h, lw["gate_up"])), lw["down"])
@@ -437,39 +439,6 @@ class DecodeStepRunner:
         if context.is_prefill:                           # only the last token of each prompt
             h = h[context.last_token_indices.long()]     # (models/qwen3.py:472-491)
         return F.linear(h, self.embed)                   # logits [T or batch, vocab]
-
-    def _rotate_store_prefill(self, qkv, positions, lw, attn, context):
-        """QK-norm, RoPE and cache store of packed prompt rows in place in the projection
-        buffer, then attention over its q, k and v parts where they are."""
-        c, lib = self.cfg, _lib.load()
-        tokens, width = qkv.shape
-        if not (qkv.is_contiguous() and positions.is_contiguous()
-                and context.slot_mapping.is_contiguous() and positions.dtype == torch.int32
-                and context.slot_mapping.dtype == torch.int32
-                and positions.shape == context.slot_mapping.shape == (tokens,)
-                and attn.k_cache.is_contiguous() and attn.v_cache.is_contiguous()
-                and all(t.dtype == torch.int32 and t.is_contiguous()
-                        for t in (context.cu_seqlens_q, context.cu_seqlens_k))):
-            raise ValueError("prefill metadata must be contiguous int32, one entry per token")
-        q = qkv.data_ptr()
-        k = q + 2 * c.num_heads * c.head_dim
-        v = k + 2 * c.num_kv_heads * c.head_dim
-        out = torch.empty((tokens, c.num_heads, c.head_dim), dtype=qkv.dtype, device=qkv.device)
-        with torch.cuda.device(qkv.device):
-            stream = torch.cuda.current_stream(qkv.device).cuda_stream
-            _lib.check(lib.nvj_qk_norm_rope_rows_launch(
-                stream, q, width, positions.data_ptr(), self.cos_sin.data_ptr(),
-                self.cos_sin.shape[0], lw["q_norm"].data_ptr(), lw["k_norm"].data_ptr(),
-                c.rms_norm_eps, context.slot_mapping.data_ptr(), attn.k_cache.data_ptr(),
-                attn.v_cache.data_ptr(), q, width, k, None, width, tokens, c.num_heads,
-                c.num_kv_heads, c.head_dim, attn.k_cache.numel() // (c.num_kv_heads * c.head_dim)),
-                "nvj_qk_norm_rope_rows_launch")
-            _lib.check(lib.nvj_prefill_attention_rows_launch(
-                stream, q, width, k, v, width, context.cu_seqlens_q.data_ptr(),
-                context.cu_seqlens_k.data_ptr(), out.data_ptr(), tokens,
-                context.cu_seqlens_q.shape[0] - 1, c.num_heads, c.num_kv_heads, c.head_dim,
-                attn.scale, _lib.NVJ_DTYPE_BF16), "nvj_prefill_attention_rows_launch")
-        return out
 
     # -- one decode step ------------------------------------------------------
     def make_inputs(self, last_tokens, seq_lens, block_tables):

@@ -12,7 +12,8 @@ import torch
 
 from .. import _lib
 
-__all__ = ["variable_length_attention_prefill", "paged_prefill_attention"]
+__all__ = ["variable_length_attention_prefill", "packed_qkv_attention",
+           "paged_prefill_attention"]
 
 _DTYPE_CODE = {torch.bfloat16: _lib.NVJ_DTYPE_BF16, torch.float16: _lib.NVJ_DTYPE_F16}
 
@@ -64,6 +65,34 @@ def variable_length_attention_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_s
             cu_seqlens_k.data_ptr(), out.data_ptr(), total, batch, hq, hkv, d, float(scale),
             _DTYPE_CODE[q.dtype])
     _lib.check(code, "nvj_prefill_attention_launch")
+    return out
+
+
+def packed_qkv_attention(qkv, cu_seqlens_q, cu_seqlens_k, num_heads, num_kv_heads, head_dim,
+                         scale):
+    """``variable_length_attention_prefill`` over the q, k and v parts of projection
+    rows ``[total_tokens, (num_heads + 2 * num_kv_heads) * head_dim]`` where they are."""
+    lib = _lib.load()
+    width = (num_heads + 2 * num_kv_heads) * head_dim
+    _require(isinstance(qkv, torch.Tensor) and qkv.is_cuda and qkv.dtype in _DTYPE_CODE
+             and qkv.dim() == 2 and qkv.shape[1] == width and qkv.is_contiguous(),
+             f"qkv must be contiguous bf16 or float16 [total_tokens, {width}] on the GPU")
+    for name, t in (("cu_seqlens_q", cu_seqlens_q), ("cu_seqlens_k", cu_seqlens_k)):
+        _require(isinstance(t, torch.Tensor) and t.dtype == torch.int32 and t.dim() == 1
+                 and t.is_contiguous() and t.device == qkv.device,
+                 f"{name} must be contiguous int32 with one dim on qkv's device")
+    batch = cu_seqlens_q.shape[0] - 1
+    _require(batch >= 0 and cu_seqlens_k.shape[0] == batch + 1, "cu_seqlens shapes disagree")
+    total, q = qkv.shape[0], qkv.data_ptr()
+    k = q + 2 * num_heads * head_dim
+    out = torch.empty((total, num_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
+    with torch.cuda.device(qkv.device):
+        code = lib.nvj_prefill_attention_rows_launch(
+            torch.cuda.current_stream(qkv.device).cuda_stream, q, width, k,
+            k + 2 * num_kv_heads * head_dim, width, cu_seqlens_q.data_ptr(),
+            cu_seqlens_k.data_ptr(), out.data_ptr(), total, batch, num_heads, num_kv_heads,
+            head_dim, float(scale), _DTYPE_CODE[qkv.dtype])
+    _lib.check(code, "nvj_prefill_attention_rows_launch")
     return out
 
 

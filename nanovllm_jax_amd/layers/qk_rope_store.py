@@ -31,7 +31,7 @@ def build_cos_sin_cache(head_dim: int, max_position: int, base: float, device) -
 
 def qk_norm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weight, eps,
                        k_cache, v_cache, slot_mapping, num_heads, num_kv_heads, head_dim,
-                       q_out=None):
+                       q_out=None, in_place=False):
     """Normalise and rotate q and k, write q out and K/V into the paged cache.
 
     qkv            [num_tokens, (num_heads + 2 * num_kv_heads) * head_dim] bf16
@@ -43,7 +43,8 @@ def qk_norm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weig
     slot_mapping   [num_tokens] int32 (``< 0`` skips, ``>= num_slots`` drops)
 
     Returns q ``[num_tokens, num_heads, head_dim]`` bf16, ready for
-    ``paged_attention``.
+    ``paged_attention``.  ``in_place``: q and k are normalised and rotated where they
+    are in ``qkv`` (contiguous), which is returned, ready for ``packed_qkv_attention``.
     """
     lib = _lib.load()
     tensors = [("qkv", qkv), ("positions", positions), ("cos_sin_cache", cos_sin_cache),
@@ -79,6 +80,20 @@ def qk_norm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weig
              and v_cache.is_contiguous(), "caches must be contiguous bf16 of equal shape")
     _require(tuple(k_cache.shape[-2:]) == (num_kv_heads, head_dim), "cache row shape mismatch")
     num_slots = k_cache.numel() // (num_kv_heads * head_dim)
+    q_ptr = q_norm_weight.data_ptr() if q_norm_weight is not None else None
+    k_ptr = k_norm_weight.data_ptr() if k_norm_weight is not None else None
+    if in_place:
+        _require(q_out is None and qkv.is_contiguous(), "in place: a contiguous qkv and no q_out")
+        width, q = qkv.shape[1], qkv.data_ptr()
+        with torch.cuda.device(qkv.device):
+            code = lib.nvj_qk_norm_rope_rows_launch(
+                torch.cuda.current_stream(qkv.device).cuda_stream, q, width, positions.data_ptr(),
+                cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], q_ptr, k_ptr, float(eps),
+                slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), q, width,
+                q + 2 * num_heads * head_dim, None, width, num_tokens, num_heads, num_kv_heads,
+                head_dim, num_slots)
+        _lib.check(code, "nvj_qk_norm_rope_rows_launch")
+        return qkv
     if q_out is None:
         q_out = torch.empty((num_tokens, num_heads, head_dim), dtype=torch.bfloat16,
                             device=qkv.device)
@@ -89,9 +104,7 @@ def qk_norm_rope_store(qkv, positions, cos_sin_cache, q_norm_weight, k_norm_weig
         stream = torch.cuda.current_stream(qkv.device).cuda_stream
         code = lib.nvj_qk_norm_rope_store_launch(
             stream, qkv.data_ptr(), row_stride, positions.data_ptr(), cos_sin_cache.data_ptr(),
-            cos_sin_cache.shape[0],
-            q_norm_weight.data_ptr() if q_norm_weight is not None else None,
-            k_norm_weight.data_ptr() if k_norm_weight is not None else None, float(eps),
+            cos_sin_cache.shape[0], q_ptr, k_ptr, float(eps),
             slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), q_out.data_ptr(),
             num_tokens, num_heads, num_kv_heads, head_dim, num_slots)
     _lib.check(code, "nvj_qk_norm_rope_store_launch")

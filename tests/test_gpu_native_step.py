@@ -203,13 +203,14 @@ def _decode_inputs(runner, rows):
                               [[i] for i in range(rows)])
 
 
-@pytest.mark.parametrize("rows", [3, 20])
+@pytest.mark.parametrize("rows", [3, 20, -3, -20])      # decode; new tokens of a packed prompt
 def test_native_step_reads_the_model_on_every_step(rows, monkeypatch):
     """What changes between two steps changes the second: a layer's scale, the norms' eps,
     weights in place, and weights replaced by others."""
     print(f"case model read on every step rows={rows}", flush=True)
     ds, runner = _small_runner()
-    inputs = _decode_inputs(runner, rows)
+    inputs = _decode_inputs(runner, rows) if rows > 0 else \
+        runner.make_prefill_inputs([list(range(-rows))], [[0]])
     first = runner.forward(*inputs).float()
 
     def both():
@@ -250,12 +251,14 @@ def test_native_step_reads_the_model_on_every_step(rows, monkeypatch):
                                         ("ln1", (256,)), ("ln2", (256,)), ("q_norm", (64,)),
                                         ("k_norm", (64,)), ("cos_sin", (512, 64)),
                                         ("final_norm", (256,))])
-def test_native_step_refuses_weights_of_another_shape(name, shape):
+@pytest.mark.parametrize("kind", ["decode", "packed"])
+def test_native_step_refuses_weights_of_another_shape(name, shape, kind):
     """A weight that was replaced by a smaller one is never read past its end: the native
     step declines, and the long way names the mistake."""
-    print(f"case weight {name} {shape}", flush=True)
+    print(f"case weight {name} {shape} {kind}", flush=True)
     _, runner = _small_runner()
-    inputs = _decode_inputs(runner, 3)
+    inputs = _decode_inputs(runner, 3) if kind == "decode" else \
+        runner.make_prefill_inputs([[1, 2, 3], [4, 5]], [[0], [1]])
     assert runner._native_forward(*inputs) is not None
     at = runner.layers[1] if name in runner.layers[1] else runner.__dict__
     at[name] = torch.ones(shape, dtype=at[name].dtype, device="cuda:0")
@@ -324,3 +327,15 @@ def test_wide_models_take_the_library_products():
         inputs = _decode_inputs(runner, rows)
         assert (runner._native_forward(*inputs) is not None) == native
         assert not runner.forward(*inputs).isnan().any()
+
+
+def test_packed_prefill_refuses_offsets_of_another_length(monkeypatch):
+    print("case cu_seqlens of another length", flush=True)
+    ds, runner = _small_runner()
+    for patch in (False, True):
+        if patch:
+            monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+        ids, pos, ctx = runner.make_prefill_inputs([[1, 2, 3], [4, 5]], [[0], [1]])
+        ctx.cu_seqlens_k = ctx.cu_seqlens_k[:2]
+        with pytest.raises(ValueError):
+            runner.forward(ids, pos, ctx)
