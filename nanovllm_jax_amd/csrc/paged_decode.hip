@@ -2059,11 +2059,18 @@ constexpr int kWholeRowTolerance = 64;
 
 // Whether the table rules out rows (of at most one per CU) that are not short: two rounds
 // of the 8 waves of a workgroup, which take 2.8 us each, what one CU draws.  A third is
-// still less than the balanced split's two passes for one sequence, and where its
-// workgroups have more than a row each to share: 768 positions of 8 KV heads with 1 / 4 /
-// 16 sequences 10.1 / 14.1 / 14.6 us against 11.7 / 12.6 / 16.5.
+// still less than the balanced split's two passes where rows are few, and where its
+// workgroups have a row or more each to share.  Measured with 520 .. 1024 positions and 1 ..
+// 32 KV heads, all rows alike or ragged, the kernel without a split against the balanced one,
+// us at 768 positions: 1 .. 16 rows 9.2 .. 10.9 / 11.8 .. 12.8, 32 rows 12.6 .. 14.2 /
+// 12.6 .. 14.0, 64 rows 13.6 .. 14.7 / 13.7 .. 15.6, 128 rows 15.6 / 17.5, 256 rows 19.4 /
+// 21.3; at 1024 (four rounds) 1 .. 8 rows 10.7 .. 11.8 / 11.8 .. 12.6, 16 rows 12.5 .. 14.6 /
+// 12.7 .. 13.4, 32 rows 17 / 13.3.
+// The balanced kernel does not take a third round for few rows when it finds short lengths
+// in a wider table: its start and its LDS merge make such a row 2.0 .. 2.6 us slower there,
+// and the equal cut as fast (8 rows of 768 positions 12.5 / 12.2).
 bool table_of_short_rows(int64_t rows, int64_t positions) {
-  return positions <= (rows <= 8 || rows >= 128 ? 3 : 2) * 8 * kStep;
+  return positions <= (rows <= 16 || rows >= 128 ? 3 : 2) * 8 * kStep;
 }
 
 // Waves per workgroup of the fixed split = KV heads a workgroup covers: the

@@ -9,7 +9,11 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = {"one": ([700], 16, 8), "few": ([128, 2000, 900, 1, 513], 16, 8),
-          "many rows": ([300 + 7 * i for i in range(40)], 16, 8)}
+          "many rows": ([300 + 7 * i for i in range(40)], 16, 8),
+          # 16 rows and 24, 128 and 120 of a table of three rounds: both sides of its rule
+          "two": ([700, 768], 16, 8), "three": ([700, 768, 513], 16, 8),
+          "sixteen": ([768 - 40 * i for i in range(16)], 16, 8),
+          "fifteen": ([768 - 40 * i for i in range(15)], 16, 8)}
 
 
 def _layer(name, seed, dtype=torch.bfloat16):
@@ -74,7 +78,7 @@ def test_call_on_a_side_stream_and_in_a_graph_without_a_workspace(name):
 
 @pytest.mark.parametrize("streams", ["null", "own"])
 def test_calls_of_several_threads(streams):
-    """Three threads, each a layer of its own: on the null stream, whose counters they share
+    """Several threads, each a layer of its own: on the null stream, whose counters they share
     in turn, or each on a stream of its own."""
     print(f"case threads on {streams} stream", flush=True)
     from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
