@@ -579,6 +579,39 @@ NVJ_API int nvj_silu_and_mul_launch(void* stream, const void* x, int64_t x_row_s
                             void* y, int32_t num_tokens, int32_t intermediate);
 
 /*
+ * The products of the decoder step below for prompts and batches, on their own:
+ *   out[m][n] = x[m][:] . w[n][:], x [rows, reduction], w [outputs, reduction] bf16, fp32 sums
+ *   NVJ_LINEAR_ROWS        out [rows, outputs] bf16, each sum one chain over the reduction
+ *   NVJ_LINEAR_SILU_MUL    out [rows, outputs / 2]: SiLU of the first half of the sums, rounded to
+ *                          bf16, times the second half, rounded likewise; outputs a multiple of 32
+ *   NVJ_LINEAR_CHAINS_c_r  as ROWS, the reduction in c interleaved chains of runs of 32 * r, added
+ *                          in order; reduction a multiple of 32 * c * r
+ * outputs a multiple of 8, reduction of 64; operands below 4 GiB; pointers 16-byte aligned.
+ * `tile`: the tile shape (0 .. 10; not with chains), or -1: by the sizes.
+ */
+#define NVJ_LINEAR_ROWS 0
+#define NVJ_LINEAR_SILU_MUL 1
+#define NVJ_LINEAR_CHAINS_4_1 2
+#define NVJ_LINEAR_CHAINS_4_2 3
+#define NVJ_LINEAR_CHAINS_2_4 4
+NVJ_API int nvj_linear_launch(void* stream, const void* x, const void* w, void* out, int32_t rows,
+                            int32_t outputs, int32_t reduction, int32_t form, int32_t tile);
+
+/*
+ * The fused QKV projection with what follows it: nvj_qk_norm_rope_rows_launch on the rows of
+ * x . w^T, head_dim 128, without the projection going through memory.  qkv_out NULL, or
+ * [rows, (num_heads + 2 * num_kv_heads) * 128]: the new K and V rows also to their columns of
+ * it (q only to q_out).  tile: 1 .. 10 whose width divides the columns, or -1.
+ */
+NVJ_API int nvj_qkv_linear_launch(void* stream, const void* x, const void* w, int32_t rows,
+                            int32_t reduction, const int32_t* positions,
+                            const float* cos_sin_cache, int32_t max_position,
+                            const float* q_norm_weight, const float* k_norm_weight, float eps,
+                            const int32_t* slot_mapping, void* k_cache, void* v_cache, void* q_out,
+                            void* qkv_out, int32_t num_heads, int32_t num_kv_heads,
+                            int64_t num_slots, int32_t tile);
+
+/*
  * One step of the whole decoder stack, a decode batch or the prefill of new prompts,
  * up to the logits.  Covers the model of models/qwen3.py:130-172, 285-318, 366-393 and
  * 472-491 (embedding; per layer RMSNorm, fused QKV, QK-RMSNorm, RoPE, KV store,

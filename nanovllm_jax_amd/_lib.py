@@ -117,12 +117,22 @@ SYMBOLS = {
         _c.c_int32, _c.c_int32]),
     "nvj_silu_and_mul_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int32, _c.c_int32]),
+    "nvj_linear_launch": (_c.c_int, [_c.c_void_p] * 4 + [_c.c_int32] * 5),
+    "nvj_qkv_linear_launch": (_c.c_int, [
+        _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int32, _c.c_void_p, _c.c_void_p,
+        _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_float, _c.c_void_p, _c.c_void_p, _c.c_void_p,
+        _c.c_void_p, _c.c_void_p, _c.c_int32, _c.c_int32, _c.c_int64, _c.c_int32]),
     "nvj_decoder_step_workspace_bytes": (_c.c_size_t, [
         _c.POINTER(DecoderModel), _c.c_int32, _c.c_int32]),
     "nvj_decoder_step_launch": (_c.c_int, [
         _c.c_void_p, _c.POINTER(DecoderModel), _c.POINTER(DecoderLayer), _c.POINTER(DecoderBatch),
         _c.c_void_p, _c.c_size_t]),
 }
+NVJ_LINEAR_ROWS = 0
+NVJ_LINEAR_SILU_MUL = 1
+NVJ_LINEAR_CHAINS_4_1 = 2
+NVJ_LINEAR_CHAINS_4_2 = 3
+NVJ_LINEAR_CHAINS_2_4 = 4
 NVJ_CHUNK_WHOLE_SEQUENCE = -1
 NVJ_STATIC_SCRATCH_BYTES = 16 << 20
 NVJ_ERR_SCRATCH_LIMIT = -7

@@ -30,11 +30,18 @@
 //
 // Order of the sums.  A network of random bf16 weights doubles any difference of one
 // ulp from stage to stage until all roundings differ (two GEMM kernels that sum in
-// different orders end 2-3 % apart in the logits after 28 layers), so these
-// products sum in the order of the GEMMs a step of more rows runs through, and give
-// the same bits: the reduction is cut into `chains` interleaved runs of `run`
-// steps of 32, each chain is accumulated in order and the chains are added in
-// order (struct Chains).
+// different orders end 2-3 % apart in the logits after 28 layers).  The reduction of these
+// products is therefore cut into `chains` interleaved runs of `run` steps of 32, each chain
+// accumulated in order and the chains added in order, as the library GEMMs that the step ran
+// through before did at hidden 1024 / intermediate 3072 (found by comparing the bits of each
+// form with theirs over 1 .. 4400 rows):
+//   rows          QKV, gate/up   O       down
+//   1 .. 16       4 x 1          4 x 1   2 x 4
+//   17 .. 128     one chain      4 x 1   2 x 4 up to 64 but 32, else 4 x 2
+//   more          one chain      one chain
+// That keeps a program's logits where they were at that width, and is all it does: at other
+// widths the library sums in other orders, any of these is as exact (fp32 sums), and a
+// library of another version may differ everywhere.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -544,7 +551,7 @@ int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder
   return launch_norm_gemm_wide<true>(s, a, m.hidden) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }
 
-// The order the library GEMMs sum the output and down projections in (see the top).
+// The orders of the sums of the output and down projections (see the top).
 hipError_t output_projection(hipStream_t s, const nvj::LinearArgs& a) {
   if (a.M <= 128 && a.K % 128 == 0) return nvj::linear_chained(s, a, 4, 1);
   return nvj::linear(s, a);

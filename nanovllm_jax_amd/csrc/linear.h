@@ -26,6 +26,7 @@ struct LinearArgs {
   int max_position, num_heads, num_kv_heads;
   int64_t num_slots;
   int m_tiles, n_tiles, group_m;   // filled in by the launch
+  int tile;                        // 1 + index of the tile shape, 0: by the sizes
 };
 
 // Whether the kernels can be given these sizes at all.

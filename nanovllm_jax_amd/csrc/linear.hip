@@ -19,9 +19,8 @@
 // (as in decoder_step.hip) were no way out: 64-byte pieces of 16 rows per load made it
 // 1 us per step whatever the tile.
 //
-// Every output is one chain of v_mfma_f32_16x16x32_bf16 over K in order, which is the
-// order of the library GEMMs at more than 128 rows: the same bits (decoder_step.hip says
-// why that matters).
+// Every output is one chain of v_mfma_f32_16x16x32_bf16 over K in order, whatever the tile
+// and the rows beside it (decoder_step.hip says where the library GEMMs sum likewise).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -270,8 +269,8 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// The same for up to 128 rows where the reduction is cut into chains (the order of
-// the library GEMMs for the output and down projections at these sizes): 4 waves =
+// The same for up to 128 rows where the reduction is cut into chains (the output and
+// down projections: few outputs, long reductions; decoder_step.hip on the orders): 4 waves =
 // CHAINS chains x 4 / CHAINS row halves of a BM x BN tile; chain c takes every
 // CHAINS-th run of RUN steps of 32.  Each operand of a stage is read by one wave, so a
 // stage is a whole round of the chains (32 * CHAINS * RUN of the reduction) and the
@@ -391,7 +390,8 @@ hipError_t launch_tiles(hipStream_t s, LinearArgs a) {
 // Tile sizes.  A launch of T tiles takes rounds of one workgroup per CU (or two, where they
 // share one), each round a fixed 3 us and per step of 64 a time between `low` (few CUs busy)
 // and `full` (all of them: the L2s and the power limit share out).  Measured on an
-// MI355X over 300 .. 4400 rows and the four projections of a 1024-wide layer, us:
+// MI355X over 300 .. 4400 rows and the four projections of a 1024-wide layer, us
+// (other widths: _native_step_pays in engine/decode_step.py has them against the library's):
 struct TileShape {
   int bm, bn, per_cu;
   float low, full;
@@ -402,11 +402,13 @@ constexpr TileShape kShapes[] = {
     {192, 128, 1, 0.475f, 0.68f}, {128, 256, 1, 0.62f, 0.90f}, {160, 256, 1, 0.76f, 1.12f},
     {224, 256, 1, 1.00f, 1.52f}, {256, 256, 1, 1.21f, 1.75f}};
 
+constexpr int kNumShapes = (int)(sizeof(kShapes) / sizeof(kShapes[0]));
+
 int best_shape(int64_t m, int64_t n, int k, int min_bn) {
   int best = 0;
   float best_cost = 0.f;
   const int64_t cus = nvj::compute_units();
-  for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+  for (int i = 0; i < kNumShapes; ++i) {
     const TileShape& t = kShapes[i];
     if (t.bn < min_bn) continue;
     const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
@@ -454,16 +456,16 @@ bool linear_takes(int64_t m, int64_t n, int64_t k) {
 
 hipError_t linear(hipStream_t s, LinearArgs a) {
   a.group_m = 8;   // 8 x 4 tiles at a time per XCD: 51 -> 42 us for 160 x 256 tiles at 4400 rows
-  return launch_shape<kPlain>(best_shape(a.M, a.N, a.K, 0), s, a);
+  return launch_shape<kPlain>(a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0), s, a);
 }
 hipError_t linear_silu_mul(hipStream_t s, LinearArgs a) {
   a.group_m = 8;
-  return launch_shape<kSiluMul>(best_shape(a.M, a.N, a.K, 0), s, a);
+  return launch_shape<kSiluMul>(a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0), s, a);
 }
 hipError_t linear_qk_rope(hipStream_t s, LinearArgs a) {
   a.group_m = 8;
+  int shape = a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 128);
   // columns beyond the last head would be taken for one: 256-wide tiles for an even count only
-  int shape = best_shape(a.M, a.N, a.K, 128);
   if (a.N % kShapes[shape].bn != 0) shape = 4;
   return launch_shape<kQkRope>(shape, s, a);
 }
@@ -476,3 +478,103 @@ hipError_t linear_chained(hipStream_t s, const LinearArgs& a, int chains, int ru
 }
 
 }  // namespace nvj
+
+namespace {
+// What every product asks of its operands.
+int check_product(const void* x, const void* w, const void* out, int64_t rows, int64_t outputs,
+                  int64_t reduction, int32_t tile) {
+  if (rows < 0 || outputs <= 0 || reduction <= 0 || tile < -1 || tile >= kNumShapes)
+    return NVJ_ERR_BAD_SHAPE;
+  if (!nvj::linear_takes(rows > 0 ? rows : 1, outputs, reduction)) return NVJ_ERR_UNSUPPORTED;
+  if (rows == 0) return NVJ_OK;
+  if (!x || !w || !out) return NVJ_ERR_NULL_POINTER;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+       reinterpret_cast<uintptr_t>(out)) & 15u)
+    return NVJ_ERR_ALIGNMENT;
+  return NVJ_OK;
+}
+}  // namespace
+
+extern "C" int nvj_linear_launch(void* stream, const void* x, const void* w, void* out,
+                                 int32_t rows, int32_t outputs, int32_t reduction, int32_t form,
+                                 int32_t tile) {
+  const int bad = check_product(x, w, out, rows, outputs, reduction, tile);
+  if (bad != NVJ_OK) return bad;
+  const int chains = form == NVJ_LINEAR_CHAINS_2_4 ? 2 : 4;
+  const int run = form == NVJ_LINEAR_CHAINS_4_1 ? 1 : form == NVJ_LINEAR_CHAINS_4_2 ? 2 : 4;
+  switch (form) {
+    case NVJ_LINEAR_ROWS: break;
+    case NVJ_LINEAR_SILU_MUL:
+      if (outputs % 32 != 0) return NVJ_ERR_UNSUPPORTED;
+      break;
+    case NVJ_LINEAR_CHAINS_4_1:
+    case NVJ_LINEAR_CHAINS_4_2:
+    case NVJ_LINEAR_CHAINS_2_4:
+      if (tile >= 0 || reduction % (32 * chains * run) != 0) return NVJ_ERR_UNSUPPORTED;
+      break;
+    default: return NVJ_ERR_BAD_SHAPE;
+  }
+  if (rows == 0) return NVJ_OK;
+  LinearArgs a = {};
+  a.x = static_cast<const char*>(x);
+  a.w = static_cast<const char*>(w);
+  a.out = static_cast<uint16_t*>(out);
+  a.M = rows;
+  a.N = outputs;
+  a.K = reduction;
+  a.tile = tile + 1;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const hipError_t rc = form == NVJ_LINEAR_ROWS       ? nvj::linear(s, a)
+                        : form == NVJ_LINEAR_SILU_MUL ? nvj::linear_silu_mul(s, a)
+                                                      : nvj::linear_chained(s, a, chains, run);
+  return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+}
+
+extern "C" int nvj_qkv_linear_launch(void* stream, const void* x, const void* w, int32_t rows,
+                                     int32_t reduction, const int32_t* positions,
+                                     const float* cos_sin_cache, int32_t max_position,
+                                     const float* q_norm_weight, const float* k_norm_weight,
+                                     float eps, const int32_t* slot_mapping, void* k_cache,
+                                     void* v_cache, void* q_out, void* qkv_out, int32_t num_heads,
+                                     int32_t num_kv_heads, int64_t num_slots, int32_t tile) {
+  if (num_heads <= 0 || num_kv_heads <= 0 || max_position <= 0 || num_slots < 0)
+    return NVJ_ERR_BAD_SHAPE;
+  const int64_t outputs = ((int64_t)num_heads + 2 * (int64_t)num_kv_heads) * 128;
+  if (outputs > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
+  const int bad = check_product(x, w, q_out, rows, outputs, reduction, tile);
+  if (bad != NVJ_OK) return bad;
+  if (tile >= 0 && (kShapes[tile].bn < 128 || outputs % kShapes[tile].bn != 0))
+    return NVJ_ERR_UNSUPPORTED;   // tiles hold whole heads
+  if (rows == 0) return NVJ_OK;
+  if (!positions || !cos_sin_cache || !slot_mapping || !k_cache || !v_cache ||
+      (q_norm_weight == nullptr) != (k_norm_weight == nullptr))
+    return NVJ_ERR_NULL_POINTER;
+  if ((reinterpret_cast<uintptr_t>(cos_sin_cache) | reinterpret_cast<uintptr_t>(q_norm_weight) |
+       reinterpret_cast<uintptr_t>(k_norm_weight) | reinterpret_cast<uintptr_t>(k_cache) |
+       reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(qkv_out)) & 15u)
+    return NVJ_ERR_ALIGNMENT;
+  LinearArgs a = {};
+  a.x = static_cast<const char*>(x);
+  a.w = static_cast<const char*>(w);
+  a.out = static_cast<uint16_t*>(qkv_out);
+  a.M = rows;
+  a.N = (int)outputs;
+  a.K = reduction;
+  a.q_out = static_cast<uint16_t*>(q_out);
+  a.keep_kv = qkv_out != nullptr;
+  a.positions = positions;
+  a.cos_sin = cos_sin_cache;
+  a.q_norm = q_norm_weight;
+  a.k_norm = k_norm_weight;
+  a.slot_mapping = slot_mapping;
+  a.k_cache = static_cast<uint16_t*>(k_cache);
+  a.v_cache = static_cast<uint16_t*>(v_cache);
+  a.eps = eps;
+  a.max_position = max_position;
+  a.num_heads = num_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.num_slots = num_slots;
+  a.tile = tile + 1;
+  return nvj::linear_qk_rope(static_cast<hipStream_t>(stream), a) == hipSuccess ? NVJ_OK
+                                                                                 : NVJ_ERR_LAUNCH;
+}

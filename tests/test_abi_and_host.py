@@ -169,6 +169,27 @@ def test_decoder_step_argument_validation():
     assert launch(is_prefill=1, cu_seqlens_q=p, cu_seqlens_k=p) == -1     # no last_token_indices
 
 
+def test_linear_argument_validation():
+    from nanovllm_jax_amd import _lib
+    lib = _lib.load()
+    p = 0x1000
+
+    def rows(x=p, w=p, out=p, m=4, n=64, k=128, form=0, tile=-1):
+        return lib.nvj_linear_launch(None, x, w, out, m, n, k, form, tile)
+
+    def qkv(x=p, m=4, k=128, cos_sin=p, qn=p, kn=p, tile=-1, hq=2, hkv=1, qkv_out=p):
+        return lib.nvj_qkv_linear_launch(None, x, p, m, k, p, cos_sin, 8, qn, kn, 1e-6, p, p, p, p,
+                                         qkv_out, hq, hkv, 8, tile)
+
+    assert rows(m=0) == qkv(m=0) == 0
+    assert rows(x=0) == rows(out=0) == qkv(x=0) == qkv(cos_sin=0) == qkv(qn=0) == -1
+    assert rows(m=-1) == rows(tile=11) == rows(tile=-2) == rows(form=5) == qkv(hq=0) == -2
+    assert rows(n=12) == rows(k=96) == rows(m=1 << 30) == qkv(k=96) == -3
+    assert rows(form=1, n=40) == rows(form=3, k=128) == rows(form=2, tile=0) == -3
+    assert qkv(tile=0) == qkv(tile=10, hq=1) == -3          # tiles of whole heads
+    assert rows(w=p + 8) == qkv(kn=p + 4) == qkv(qkv_out=p + 2) == -8
+
+
 def test_native_step_is_taken_where_it_was_measured_faster():
     from nanovllm_jax_amd.engine.decode_step import _native_step_pays as pays
     for sizes, rows_native, rows_library in (
