@@ -1,6 +1,8 @@
-"""The native step (six fused launches per layer) against the same step through library
-GEMMs and separate launches, at the edges of its row counts and row lengths; and the QK
-norm / RoPE launch with rows in place, strided and at odd offsets."""
+"""The native step, in both its forms (up to 16 rows, and more), against the same step
+through library GEMMs and separate launches, at the edges of its row counts and row lengths,
+within what two orders of bf16 roundings give (the products have tests of their own against
+float64, test_gpu_linear.py); what it declines or refuses; and the QK norm / RoPE launch with
+rows in place, strided and at odd offsets."""
 import numpy as np
 import pytest
 import torch
@@ -339,3 +341,37 @@ def test_packed_prefill_refuses_offsets_of_another_length(monkeypatch):
         ctx.cu_seqlens_k = ctx.cu_seqlens_k[:2]
         with pytest.raises(ValueError):
             runner.forward(ids, pos, ctx)
+
+
+@pytest.mark.parametrize("rows", [4, 24])
+@pytest.mark.parametrize("kind", ["decode", "packed", "paged"])
+def test_native_step_with_slots_that_are_not_stored(rows, kind, monkeypatch):
+    print(f"case skipped slots rows={rows} {kind}", flush=True)
+    ds, runner = _small_runner()
+    if kind == "decode":
+        ids, pos, ctx = _decode_inputs(runner, rows)
+    else:
+        toks = [list(range(rows - 2)), [5, 6]]
+        cached = [9, 0] if kind == "paged" else None
+        if cached:
+            toks[0] = [1] * 9 + toks[0]
+        ids, pos, ctx = runner.make_prefill_inputs(toks, [[0], [1]], cached)
+    slots = ctx.slot_mapping.clone()
+    slots[1], slots[-1] = -1, 60 * 64                       # skipped, and out of the cache
+    ctx.slot_mapping = slots
+    before = runner.kv_cache.clone()
+    got = runner._native_forward(ids, pos, ctx).float()
+    kv = runner.kv_cache.clone()
+    runner.kv_cache.copy_(before)
+    monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+    want = runner.forward(ids, pos, ctx).float()
+    assert _close(got, want)
+    # rows written by both, and by neither
+    flat = lambda t: t.view(2, 2, -1, 2, 128)
+    written = torch.zeros(60 * 64, dtype=torch.bool, device="cuda:0")
+    written[slots[(slots >= 0) & (slots < 60 * 64)].long()] = True
+    for cache in (kv, runner.kv_cache):
+        same = (flat(cache) == flat(before)).all(-1).all(-1)
+        assert same[:, :, ~written].all() and not same[:, :, written].any()
+    assert ((kv.float() - runner.kv_cache.float()).abs()
+            <= 0.03 + 0.03 * runner.kv_cache.float().abs()).all()
