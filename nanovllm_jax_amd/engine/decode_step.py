@@ -382,7 +382,17 @@ class DecodeStepRunner:
             ws._clear_next = False
         return logits
 
+    def _wait_for_inputs(self, context: AttentionContext):
+        """Inputs are uploaded without a wait, on the stream that was current then; another
+        stream has to wait for them.  (A capture begins behind a device synchronisation.)"""
+        stream, event = context.uploaded
+        here = torch.cuda.current_stream(self.device)
+        if here != stream and not torch.cuda.is_current_stream_capturing():
+            here.wait_event(event)
+
     def forward(self, input_ids, positions, context: AttentionContext):
+        if context.uploaded is not None:
+            self._wait_for_inputs(context)
         logits = self._native_forward(input_ids, positions, context)
         if logits is not None:
             return logits
@@ -448,7 +458,9 @@ class DecodeStepRunner:
         # the lengths are host integers here, as in the reference's filler: pick the split
         split = choose_split(ctx, self.cfg.num_kv_heads, self.cfg.num_heads)
         d_ids, d_pos, d_ctx, d_slots, d_bt = self._upload(ids, pos, ctx, slots, bt)
-        return d_ids, d_pos, create_decode_context(d_ctx, d_slots, d_bt, split)
+        context = create_decode_context(d_ctx, d_slots, d_bt, split)
+        context.uploaded = self._upload_mark()
+        return d_ids, d_pos, context
 
     def _check_ids(self, ids):
         """Host ids outside the vocabulary are an error here; ids that a caller writes
@@ -474,6 +486,11 @@ class DecodeStepRunner:
         block.copy_(host, non_blocking=True)
         return [block[o:o + a.size].view(a.shape) for a, o in zip(arrays, at)]
 
+    def _upload_mark(self):
+        """The current stream and an event behind what it has been given so far."""
+        stream = torch.cuda.current_stream(self.device)
+        return stream, stream.record_event()
+
     def make_prefill_inputs(self, token_lists, block_tables, num_cached_tokens=None):
         """Prefill inputs; with ``num_cached_tokens`` the context carries the block
         tables (as the reference's does when a prefix is cached,
@@ -485,8 +502,10 @@ class DecodeStepRunner:
         tables = ([prepare_block_tables(block_tables)] if num_cached_tokens is not None else [])
         d_ids, d_pos, d_cu_q, d_cu_k, d_slots, *bt = self._upload(ids, pos, cu_q, cu_k, slots,
                                                                   *tables)
-        return d_ids, d_pos, create_prefill_context(d_cu_q, d_cu_k, max_q, max_k, d_slots,
-                                                    block_tables=bt[0] if bt else None)
+        context = create_prefill_context(d_cu_q, d_cu_k, max_q, max_k, d_slots,
+                                         block_tables=bt[0] if bt else None)
+        context.uploaded = self._upload_mark()     # (behind last_token_indices too)
+        return d_ids, d_pos, context
 
     def step(self, input_ids, positions, context):
         """Eager decode step: logits -> greedy token ids [batch] int64."""

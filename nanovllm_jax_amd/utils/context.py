@@ -39,6 +39,10 @@ class AttentionContext:
                         the lengths on the host, may ask for the whole-sequence
                         mode instead (``layers.paged_attention.choose_split``).
                         Not a field of the reference's dataclass.
+    uploaded            (stream, event) when the tensors are still being copied to the
+                        device: they hold their values on that stream, and on others
+                        behind the event (which ``DecodeStepRunner.forward`` waits for).
+                        None: they hold them.  Not a field of the reference's either.
     """
     is_prefill: bool = False
     cu_seqlens_q: Any = None
@@ -50,6 +54,7 @@ class AttentionContext:
     block_tables: Any = None
     last_token_indices: Any = None
     decode_split: int = 0
+    uploaded: Any = None
 
 
 def create_decode_context(context_lens, slot_mapping, block_tables,

@@ -375,3 +375,34 @@ def test_native_step_with_slots_that_are_not_stored(rows, kind, monkeypatch):
         assert same[:, :, ~written].all() and not same[:, :, written].any()
     assert ((kv.float() - runner.kv_cache.float()).abs()
             <= 0.03 + 0.03 * runner.kv_cache.float().abs()).all()
+
+
+@pytest.mark.parametrize("kind", ["decode", "packed"])
+@pytest.mark.parametrize("native", [True, False])
+def test_inputs_reach_a_step_on_another_stream(kind, native, monkeypatch):
+    """Inputs made behind long work on one stream, and a step on another stream at once."""
+    print(f"case inputs of another stream {kind} native={native}", flush=True)
+    ds, runner = _small_runner()
+    if not native:
+        monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+    def make(first):
+        if kind == "decode":
+            return runner.make_inputs([first + i for i in range(20)], [20 + i for i in range(20)],
+                                      [[i] for i in range(20)])
+        return runner.make_prefill_inputs([[first + i for i in range(9)], [first, 8]], [[0], [1]])
+
+    wants = [runner.forward(*make(first)) for first in (0, 500)]
+    assert not torch.equal(*wants)
+    side = torch.cuda.Stream()
+    a = torch.randn(8192, 8192, device="cuda:0")
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    for turn in range(6):     # in turn: memory that is used again holds the other inputs
+        for _ in range(4):
+            torch.mm(a, a)
+        inputs = make(500 * (turn % 2))
+        with torch.cuda.stream(side):
+            got = runner.forward(*inputs)
+        side.synchronize()
+        assert torch.equal(got, wants[turn % 2])
+        torch.cuda.synchronize()
