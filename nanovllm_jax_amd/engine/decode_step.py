@@ -81,19 +81,19 @@ def _native_step_pays(tokens: int, hidden: int, q_width: int, kv_width: int,
     2048 (6144)               4: 76 / 90, 64: 78 / 94, 200: 102 / 163, 600: 151 / 165,
                               1200: 203 / 199, 8000: 762 / 672
     2048 (11008)              48: 98 / 114, 96: 124 / 118, 200: 134 / 162, 600: 212 / 197
-    2560 (9728)               4: 104 / 135, 64: 128 / 125, 96: 144 / 137, 200: 166 / 163,
+    2560 (9728)               4: 104 / 135, 24: 113 / 114, 64: 128 / 125, 96: 144 / 137,
                               1200: 368 / 344
-    4096 (12288)              4: 143 / 149, 32: 146 / 144, 64: 174 / 162, 400: 304 / 261
-    5120 (25600)              4: 286 / 326, 32: 316 / 341, 128: 497 / 439
+    4096 (12288)              4: 143 / 149, 24: 156 / 158, 64: 174 / 162, 400: 304 / 261
+    5120 (25600)              4: 286 / 326, 24: 317 / 356, 128: 497 / 439
     8192 (29568)              4: 455 / 423, 64: 499 / 484, 1200: 2042 / 1613
     ========================  =====================================================
     """
     products = tokens * (hidden * (2 * q_width + 2 * kv_width) + 3 * hidden * intermediate)
     if hidden <= 1024:
         return products <= 100e9
-    if hidden <= 2560:
+    if hidden <= 2048:
         return tokens <= 64 or (tokens > 128 and products <= 40e9)
-    return hidden <= 5120 and tokens <= 32
+    return hidden <= 5120 and tokens <= 24
 
 
 def prepare_block_tables(block_tables: list[list[int]]) -> np.ndarray:

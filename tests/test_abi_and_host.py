@@ -196,9 +196,9 @@ def test_native_step_is_taken_where_it_was_measured_faster():
             ((1024, 2048, 1024, 3072), (1, 16, 17, 128, 4400), (8000, 16000)),
             ((2048, 2048, 1024, 6144), (1, 64, 200, 600), (1200, 8000)),
             ((2048, 2048, 256, 11008), (1, 64, 200), (96, 128, 600, 800)),
-            ((2560, 4096, 1024, 9728), (1, 64), (96, 600, 1200)),
-            ((4096, 4096, 1024, 12288), (1, 32), (48, 64, 400, 1200)),
-            ((5120, 8192, 1024, 25600), (1, 32), (128, 8000)),
+            ((2560, 4096, 1024, 9728), (1, 24), (32, 64, 96, 600, 1200)),
+            ((4096, 4096, 1024, 12288), (1, 24), (32, 48, 64, 400, 1200)),
+            ((5120, 8192, 1024, 25600), (1, 24), (128, 8000)),
             ((8192, 8192, 1024, 29568), (), (1, 64, 1200))):
         assert all(pays(rows, *sizes) for rows in rows_native), sizes
         assert not any(pays(rows, *sizes) for rows in rows_library), sizes
