@@ -12,12 +12,13 @@
 // 128-byte rows, pieces XOR-permuted by the row: no bank conflicts on the operand reads),
 // in a ring of two to four stages, one barrier per step, which stands in the middle of it
 // so that operand reads, copies and matrix instructions run under each other throughout.
-// Measured, 4400 rows: QKV (4096 x 1024) 40.9 us, O (1024 x 2048) 21.9, gate/up (6144 x
-// 1024) with SiLU * up 62.2, down (1024 x 3072) 29.8; library 46.4, 27.6, 56.4 + 16.7,
-// 35.2.  LDS is the next limit: operand reads and arriving copies take 75 % (256 x 256)
-// to 150 % (128 x 128) of the matrix cycles.  Weights straight into registers instead
-// (as in decoder_step.hip) were no way out: 64-byte pieces of 16 rows per load made it
-// 1 us per step whatever the tile.
+// Measured, 4400 rows, alone: QKV (4096 x 1024) without its epilogue 40.9 us, O (1024 x 2048)
+// 21.9, gate/up (6144 x 1024) with SiLU * up 62.2, down (1024 x 3072) 29.8; library 46.4, 27.6,
+// 56.4 + 16.7, 35.2.  In a step: QKV with norm, RoPE and store 51.1, O 22.9, gate/up 62.7,
+// down 33.6, the matrix pipe 36 % (QKV) to 44 % busy.  LDS is the next limit: operand reads
+// and arriving copies take 75 % (256 x 256) to 150 % (128 x 128) of the matrix cycles.
+// Weights straight into registers instead (as in decoder_step.hip) were no way out: 64-byte
+// pieces of 16 rows per load made it 1 us per step whatever the tile.
 //
 // Every output is one chain of v_mfma_f32_16x16x32_bf16 over K in order, whatever the tile
 // and the rows beside it (decoder_step.hip says where the library GEMMs sum likewise).

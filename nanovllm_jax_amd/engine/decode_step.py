@@ -1,13 +1,12 @@
-"""Whole-model decode step harness around the HIP attention path.
+"""Whole-model decode and prefill steps around the HIP attention path.
 
-The measured path of this package is the KV-cache store and the paged decode
-attention, with the element-wise stages next to it (QK-RMSNorm + RoPE + store,
-RMSNorm + residual, SiLU-and-multiply) as single HIP launches; the rest of a
-decode step (embedding, the QKV / output / MLP projections, the LM head,
-greedy pick) is plain ``torch`` here (hipBLASLt GEMMs), written from the
-architecture the reference
-describes: ``models/qwen3.py:130-172`` (attention block: fused QKV, per-head
-QK-RMSNorm when there is no QKV bias, RoPE, attention, output projection),
+A step (embedding, per layer the projections, norms, RoPE, KV store and attention, the tied
+LM head) is one native call where that is the faster way and the model is one it is built
+for: ``nvj_decoder_step_launch``, all of it in kernels of this package.  Otherwise it goes
+the long way: the same attention and element-wise launches with ``torch`` products
+(hipBLASLt GEMMs) between them.  Greedy pick is ``torch`` in both.  Written from the
+architecture the reference describes: ``models/qwen3.py:130-172`` (attention block: fused
+QKV, per-head QK-RMSNorm when there is no QKV bias, RoPE, attention, output projection),
 ``:285-318`` (pre-norm decoder layer with fused residual), ``:366-393`` (stack
 + final norm), ``:472-491`` (tied LM head), ``layers/layernorm.py:31-79``,
 ``layers/rotary_embedding.py:13-37,50-106``, ``layers/activation.py:22-33``.
