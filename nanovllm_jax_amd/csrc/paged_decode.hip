@@ -2554,7 +2554,9 @@ extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, con
 // Up to one (sequence, KV head) per CU.  With more, the comparison in every step costs the
 // stream as much as the store kernel in front of it: 1 / 8 / 16 sequences of 8 KV heads
 // (700, 128 .. 2048, 32768 positions) take 12.3 / 16.1 / 319.1 us instead of 13.6 / 17.2 /
-// 321.6, 64 of 4096 159.8 instead of 158.6.
+// 321.6, 64 of 4096 159.8 instead of 158.6.  The length sets no line: over 1 .. 64 sequences
+// of 1024 .. 32768 positions, 2 / 8 / 32 KV heads, up to one row per CU, one launch is 0.5 ..
+// 2.0 us less than two, at the longest even (32 of 16384 321.9 / 321.7).
 extern "C" int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads,
                                                 int32_t num_kv_heads, int32_t head_dim,
                                                 int32_t block_size, int32_t max_blocks,
