@@ -193,8 +193,12 @@ def load_host():
     """The native host side (``csrc/host/nvj_host.cpp``), loaded once; missing is an
     error, as for the library itself."""
     global _host
-    if _host is None:
-        load()
+    if _host is not None:
+        return _host
+    load()
+    with _lock:
+        if _host is not None:
+            return _host
         path = os.path.join(os.path.dirname(_LIB_PATH), "nvj_host.so")
         if not os.path.exists(path):
             raise NativeLibraryError(

@@ -95,6 +95,23 @@ def _native_step_pays(tokens: int, hidden: int, q_width: int, kv_width: int,
     return hidden <= 5120 and tokens <= 24
 
 
+class _Upload:
+    """The stream the tensors of a context are being uploaded on, and an event behind them.
+    Copies of the context share it; a pickled one is read back with its values in place."""
+    __slots__ = ("stream", "event")
+
+    def __init__(self, device):
+        self.stream = torch.cuda.current_stream(device)
+        self.event = self.stream.record_event()
+
+    def __deepcopy__(self, memo):
+        return self
+
+    def __reduce__(self):
+        self.event.synchronize()
+        return type(None), ()
+
+
 def prepare_block_tables(block_tables: list[list[int]]) -> np.ndarray:
     """Rows padded with -1 to the longest table (``engine/model_runner.py:225-246``)."""
     width = max(len(t) for t in block_tables)
@@ -384,10 +401,9 @@ class DecodeStepRunner:
     def _wait_for_inputs(self, context: AttentionContext):
         """Inputs are uploaded without a wait, on the stream that was current then; another
         stream has to wait for them.  (A capture begins behind a device synchronisation.)"""
-        stream, event = context.uploaded
         here = torch.cuda.current_stream(self.device)
-        if here != stream and not torch.cuda.is_current_stream_capturing():
-            here.wait_event(event)
+        if here != context.uploaded.stream and not torch.cuda.is_current_stream_capturing():
+            here.wait_event(context.uploaded.event)
 
     def forward(self, input_ids, positions, context: AttentionContext):
         if context.uploaded is not None:
@@ -458,7 +474,7 @@ class DecodeStepRunner:
         split = choose_split(ctx, self.cfg.num_kv_heads, self.cfg.num_heads)
         d_ids, d_pos, d_ctx, d_slots, d_bt = self._upload(ids, pos, ctx, slots, bt)
         context = create_decode_context(d_ctx, d_slots, d_bt, split)
-        context.uploaded = self._upload_mark()
+        context.uploaded = _Upload(self.device)
         return d_ids, d_pos, context
 
     def _check_ids(self, ids):
@@ -485,11 +501,6 @@ class DecodeStepRunner:
         block.copy_(host, non_blocking=True)
         return [block[o:o + a.size].view(a.shape) for a, o in zip(arrays, at)]
 
-    def _upload_mark(self):
-        """The current stream and an event behind what it has been given so far."""
-        stream = torch.cuda.current_stream(self.device)
-        return stream, stream.record_event()
-
     def make_prefill_inputs(self, token_lists, block_tables, num_cached_tokens=None):
         """Prefill inputs; with ``num_cached_tokens`` the context carries the block
         tables (as the reference's does when a prefix is cached,
@@ -503,7 +514,7 @@ class DecodeStepRunner:
                                                                   *tables)
         context = create_prefill_context(d_cu_q, d_cu_k, max_q, max_k, d_slots,
                                          block_tables=bt[0] if bt else None)
-        context.uploaded = self._upload_mark()     # (behind last_token_indices too)
+        context.uploaded = _Upload(self.device)     # (behind last_token_indices too)
         return d_ids, d_pos, context
 
     def step(self, input_ids, positions, context):

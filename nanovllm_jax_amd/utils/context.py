@@ -39,10 +39,11 @@ class AttentionContext:
                         the lengths on the host, may ask for the whole-sequence
                         mode instead (``layers.paged_attention.choose_split``).
                         Not a field of the reference's dataclass.
-    uploaded            (stream, event) when the tensors are still being copied to the
-                        device: they hold their values on that stream, and on others
-                        behind the event (which ``DecodeStepRunner.forward`` waits for).
-                        None: they hold them.  Not a field of the reference's either.
+    uploaded            an object with ``stream`` and ``event`` while the tensors may still
+                        be on their way to the device: they hold their values on that
+                        stream, and on others behind the event (which
+                        ``DecodeStepRunner.forward`` waits for).  None: they hold them.
+                        Not a field of the reference's either.
     """
     is_prefill: bool = False
     cu_seqlens_q: Any = None

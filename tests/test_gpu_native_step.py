@@ -406,3 +406,16 @@ def test_inputs_reach_a_step_on_another_stream(kind, native, monkeypatch):
         side.synchronize()
         assert torch.equal(got, wants[turn % 2])
         torch.cuda.synchronize()
+
+
+def test_contexts_can_be_copied_and_pickled():
+    print("case copies of a context", flush=True)
+    import copy
+    import dataclasses
+    import pickle
+    _, runner = _small_runner()
+    ids, pos, ctx = _decode_inputs(runner, 3)
+    want = runner.forward(ids, pos, ctx)
+    for other in (copy.copy(ctx), copy.deepcopy(ctx), dataclasses.replace(ctx),
+                  type(ctx)(**dataclasses.asdict(ctx)), pickle.loads(pickle.dumps(ctx))):
+        assert torch.equal(runner.forward(ids, pos, other), want)
