@@ -131,8 +131,8 @@ def test_other_threads_run_while_a_call_enqueues():
 
     thread = threading.Thread(target=count)
     try:
+        sys.setswitchinterval(100.0)     # (in front of the first wait of the other thread)
         thread.start()
-        sys.setswitchinterval(100.0)
         before = ticks[0]
         for _ in range(5000):       # the other thread may need some calls to wake up in one
             attn(*args)
