@@ -134,13 +134,12 @@ def test_other_threads_run_while_a_call_enqueues():
         sys.setswitchinterval(100.0)     # (in front of the first wait of the other thread)
         thread.start()
         before = ticks[0]
-        for _ in range(5000):       # the other thread may need some calls to wake up in one
+        for _ in range(400):
             attn(*args)
-            if ticks[0] != before:
-                break
         seen = ticks[0] - before
     finally:
         sys.setswitchinterval(interval)
         stop[0] = True
     thread.join()
-    assert seen > 0
+    print("ran", seen, "times in 400 calls", flush=True)
+    assert seen > 10      # (once or twice: something else gave it up)
