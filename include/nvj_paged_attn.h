@@ -512,6 +512,21 @@ NVJ_API int nvj_prefill_attention_rows_launch(void* stream, const void* q, int64
                             int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype);
 
 /*
+ * nvj_prefill_attention_launch and the KV store of its rows in one launch: row t of k and v,
+ * t < num_rows, also goes to slot slot_mapping[t] of the caches [num_slots, num_kv_heads,
+ * head_dim] (`dtype`, as k and v have it; slots < 0 or >= num_slots are not stored), as
+ * nvj_store_kvcache_launch would have done in front.  The attention reads k and v, never the
+ * caches.  Rows beyond what 32 bits count in 16-byte pieces take two launches.
+ */
+NVJ_API int nvj_prefill_attention_store_launch(void* stream, const void* q, const void* k,
+                            const void* v, const int32_t* cu_seqlens_q,
+                            const int32_t* cu_seqlens_k, void* out, const int32_t* slot_mapping,
+                            void* k_cache, void* v_cache, int64_t num_slots,
+                            int32_t total_q_tokens, int32_t num_rows, int32_t batch,
+                            int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float scale,
+                            int32_t dtype);
+
+/*
  * The same attention with keys and values read from the block-paged cache:
  * prompt rows behind a cached prefix (prefix caching, chunked prefill).  The
  * reference prepares exactly this call - cu_seqlens_k > cu_seqlens_q and

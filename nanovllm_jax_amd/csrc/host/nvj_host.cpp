@@ -239,6 +239,13 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   out = at::empty_like(*q);
   const int32_t* cq = static_cast<const int32_t*>(cu_q->data_ptr());
   const int32_t* ck = static_cast<const int32_t*>(cu_k->data_ptr());
+  if (!paged && !k_copy && !v_copy) {   // rows the attention can read as they are
+    const int code = nvj_prefill_attention_store_launch(
+        stream, q->data_ptr(), kp, vp, cq, ck, out.data_ptr(),
+        static_cast<const int32_t*>(slots->data_ptr()), c.k->data_ptr(), c.v->data_ptr(),
+        c.num_blocks * c.page, tokens, tokens, batch, heads, c.heads, c.dim, (float)scale, c.dtype);
+    return result(&released, &out, code);
+  }
   int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
   if (code == NVJ_OK)
     code = paged ? nvj_paged_prefill_attention_launch(

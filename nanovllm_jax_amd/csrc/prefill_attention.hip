@@ -36,6 +36,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "bf16.h"
 #include "device.h"
 #include "launch.h"
@@ -382,6 +384,79 @@ struct PrefillArgs {
   // paged only: k and v are the caches [num_blocks, block_size, Hkv, 16] pieces
   const int32_t* block_tables;   // [B, max_blocks]
   int block_size, max_blocks, num_blocks;
+  // STORE: row t of k and v also goes to slot slots[t] of the caches
+  const int32_t* slots;          // < 0 or >= num_slots: not stored
+  uint4* k_cache;
+  uint4* v_cache;
+  int64_t num_slots;
+  uint32_t row_pieces, new_pieces;   // of a row, of all rows
+};
+
+__device__ __forceinline__ void store_past_l2(uint4* to, const uint4& v) {
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+  const u32x4 t = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(to));
+}
+
+// A workgroup's share of the new rows on their way into the caches.  The attention reads the
+// packed rows and never the caches, so the store needs no place in front of it: a workgroup
+// fetches two pieces of K and V per thread before its tiles and writes them behind, then what
+// is left of its share.  The store's own launch takes 25 us for 156 MB; in here it hides under
+// the tiles' round trips: 128 prompts of 16..300 tokens (32 / 8 heads) 143 -> 130 us, and 117
+// with rows stored past the L2s (inputs of the call before; 140 -> 124 with fresh ones).
+struct StoreShare {
+  static constexpr uint32_t kBatch = 2 * kWaves * 64;
+  uint32_t at, end;
+  uint4 k0, k1, v0, v1;
+  int slot0, slot1;
+
+  // The share is counted from the end, as the tiles are walked: its rows are those that the
+  // tiles of the same time read, and come out of a cache.
+  __device__ __forceinline__ StoreShare(const PrefillArgs& a) {
+    at = (uint32_t)((uint64_t)a.new_pieces * (gridDim.x - 1 - blockIdx.x) / gridDim.x);
+    end = (uint32_t)((uint64_t)a.new_pieces * (gridDim.x - blockIdx.x) / gridDim.x);
+    k0 = k1 = v0 = v1 = make_uint4(0u, 0u, 0u, 0u);
+    slot0 = slot1 = -1;
+  }
+  __device__ __forceinline__ void fetch(const PrefillArgs& a) {
+    if (at >= end) return;
+    const uint32_t p0 = min(at + threadIdx.x, end - 1);   // (past the end: the last one again)
+    const uint32_t p1 = min(at + threadIdx.x + kBatch / 2, end - 1);
+    slot0 = a.slots[p0 / a.row_pieces];
+    slot1 = a.slots[p1 / a.row_pieces];
+    k0 = a.k[p0];
+    v0 = a.v[p0];
+    k1 = a.k[p1];
+    v1 = a.v[p1];
+  }
+  __device__ __forceinline__ void put(const PrefillArgs& a) {
+    if (at >= end) return;
+    const uint32_t p0 = min(at + threadIdx.x, end - 1);
+    const uint32_t p1 = min(at + threadIdx.x + kBatch / 2, end - 1);
+    if (slot0 >= 0 && slot0 < a.num_slots) {
+      const int64_t dst = (int64_t)slot0 * a.row_pieces + p0 % a.row_pieces;
+      store_past_l2(a.k_cache + dst, k0);
+      store_past_l2(a.v_cache + dst, v0);
+    }
+    if (slot1 >= 0 && slot1 < a.num_slots) {
+      const int64_t dst = (int64_t)slot1 * a.row_pieces + p1 % a.row_pieces;
+      store_past_l2(a.k_cache + dst, k1);
+      store_past_l2(a.v_cache + dst, v1);
+    }
+    at = at + min(kBatch, end - at);
+  }
+  __device__ __forceinline__ void finish(const PrefillArgs& a) {
+    while (at < end) {
+      fetch(a);
+      put(a);
+    }
+  }
+};
+struct NoShare {
+  __device__ __forceinline__ NoShare(const PrefillArgs&) {}
+  __device__ __forceinline__ void fetch(const PrefillArgs&) const {}
+  __device__ __forceinline__ void put(const PrefillArgs&) const {}
+  __device__ __forceinline__ void finish(const PrefillArgs&) const {}
 };
 
 // grid.x = 8 * ceil(tile bound * Hkv / 8) workgroups (see the work-item mapping below).
@@ -390,7 +465,9 @@ struct PrefillArgs {
 // LAST len_q positions of the sequence (row j sees keys <= len_k - len_q + j):
 // prompt rows behind a cached prefix.  Otherwise: packed rows, both counted
 // from the start of the sequence as the reference's mask does.
-template <bool F16, bool PAGED, int NG>
+// STORE (packed only): the rows of k and v also go into the caches (StoreShare).
+// STREAM: the output goes past the L2s.
+template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM>
 __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(PrefillArgs a,
                                                                            int num_tiles_bound,
                                                                            bool may_sort) {
@@ -412,10 +489,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   // tile): neighbours share the K/V rows of one (sequence, kv head), which stay
   // in that XCD's L2 instead of being fetched by all eight.  Later tiles of a
   // sequence have more keys to walk and come first.
+  std::conditional_t<STORE, StoreShare, NoShare> share(a);
   const int total_items = num_tiles_bound * a.num_kv_heads;
   const int part = (total_items + 7) / 8;
   const int item = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
-  if (item >= total_items) return;
+  if (item >= total_items) {
+    share.finish(a);
+    return;
+  }
   const int kvh = item / num_tiles_bound;
   const int in_kv = item - kvh * num_tiles_bound;
   // Query tiles are numbered sequence by sequence.  A wave looks at 64 sequences
@@ -454,7 +535,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
 #pragma unroll
     for (int k = 0; k < 4; ++k) real_tiles += __builtin_amdgcn_readlane(incl4[k], 63);
   }
-  if (in_kv >= real_tiles) return;   // beyond the real number of tiles
+  if (in_kv >= real_tiles) {   // beyond the real number of tiles
+    share.finish(a);
+    return;
+  }
   int seq = -1, c0 = 0;   // the sequence, its first column group of this tile
   int q_base = 0, len_q = 0, k_first = 0, k_count = 0;   // of that sequence, from the same loads
   auto take = [&](int base, int k, int src, int tile_of_seq) {
@@ -551,6 +635,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
     }
   }
   if (seq < 0) return;   // (cannot happen: the item is a real tile)
+  share.fetch(a);
   const int k_base = PAGED ? 0 : k_first;
   const int len_k = PAGED ? min(max(k_count, 0), a.max_blocks * a.block_size) : max(k_count, 0);
   // key position of the first token: the new tokens are the tail of the sequence when paged
@@ -733,10 +818,22 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
       const int row = 4 * i + kg, t = block0[g] + row;
       const uint4 o = *reinterpret_cast<const uint4*>(stage + (16 * g + row) * 256 +
                                                       16 * k_position(row, r));
-      if (t < len_q)
-        a.out[((int64_t)(q_base + t) * a.num_heads + head[g]) * kPieces + r] = o;
+      uint4* to = a.out + ((int64_t)(q_base + t) * a.num_heads + head[g]) * kPieces + r;
+      if (t < len_q) {
+        if constexpr (STREAM) store_past_l2(to, o);
+        else *to = o;
+      }
     }
+  share.put(a);
+  share.finish(a);
 }
+
+// Output rows that the L2s (32 MiB together) would not keep anyway are stored past them; left in
+// the L2s they displace the K and V rows that other workgroups are about to read (128 prompts
+// of 16..300 tokens, 166 MB of rows: 130 -> 117 us).  Smaller ones stay where the next launch
+// can find them: an output projection behind 17 MB of rows takes 2.3 us longer than the
+// attention saves (0.4).
+constexpr int64_t kStreamOutBytes = 32 << 20;
 
 // Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.
 constexpr int64_t kLongestFirstPerCu = 16;
@@ -763,25 +860,45 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
                         items <= kLongestFirstPerCu * cus &&
                         (int64_t)a.max_blocks * a.block_size >= 1024;
   const bool f16 = dtype == NVJ_DTYPE_F16;
+  const bool past_l2 = (int64_t)total_q_tokens * a.num_heads * (kD * 2) > kStreamOutBytes;
   hipError_t rc;
-#define NVJ_LAUNCH(F, P)                                                                        \
-  rc = small ? nvj::launch(prefill_attention_kernel<F, P, 1>, grid, block, stream, a, nt, may_sort) \
-             : nvj::launch(prefill_attention_kernel<F, P, 2>, grid, block, stream, a, nt, may_sort)
-  if (paged && f16) NVJ_LAUNCH(true, true);
-  else if (paged) NVJ_LAUNCH(false, true);
-  else if (f16) NVJ_LAUNCH(true, false);
-  else NVJ_LAUNCH(false, false);
+#define NVJ_LAUNCH(F, P, N, S, T) \
+  rc = nvj::launch(prefill_attention_kernel<F, P, N, S, T>, grid, block, stream, a, nt, may_sort)
+#define NVJ_LAUNCH_TYPE(F)                                        \
+  if (paged && small) NVJ_LAUNCH(F, true, 1, false, false);       \
+  else if (paged && past_l2) NVJ_LAUNCH(F, true, 2, false, true); \
+  else if (paged) NVJ_LAUNCH(F, true, 2, false, false);           \
+  else if (small && a.slots) NVJ_LAUNCH(F, false, 1, true, false); \
+  else if (small) NVJ_LAUNCH(F, false, 1, false, false);          \
+  else if (a.slots && past_l2) NVJ_LAUNCH(F, false, 2, true, true); \
+  else if (a.slots) NVJ_LAUNCH(F, false, 2, true, false);         \
+  else if (past_l2) NVJ_LAUNCH(F, false, 2, false, true);         \
+  else NVJ_LAUNCH(F, false, 2, false, false)
+  if (f16) {
+    NVJ_LAUNCH_TYPE(true);
+  } else {
+    NVJ_LAUNCH_TYPE(false);
+  }
+#undef NVJ_LAUNCH_TYPE
 #undef NVJ_LAUNCH
   return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }
 
 }  // namespace
 
-extern "C" int nvj_prefill_attention_rows_launch(
-    void* stream, const void* q, int64_t q_row_stride, const void* k, const void* v,
-    int64_t kv_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, void* out,
-    int32_t total_q_tokens, int32_t batch, int32_t num_heads, int32_t num_kv_heads,
-    int32_t head_dim, float scale, int32_t dtype) {
+namespace {
+struct CacheRows {   // where new rows go: see PrefillArgs
+  const int32_t* slots;
+  void *k_cache, *v_cache;
+  int64_t num_slots;
+  int32_t rows;
+};
+
+int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void* k, const void* v,
+                  int64_t kv_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                  void* out, int32_t total_q_tokens, int32_t batch, int32_t num_heads,
+                  int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype,
+                  const CacheRows* store) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   if (total_q_tokens < 0 || batch < 0 || num_heads <= 0 || num_kv_heads <= 0)
     return NVJ_ERR_BAD_SHAPE;
@@ -812,7 +929,55 @@ extern "C" int nvj_prefill_attention_rows_launch(
   a.num_kv_heads = num_kv_heads;
   a.group = num_heads / num_kv_heads;
   a.scale_log2e = scale * kLog2e;
+  if (store) {
+    a.slots = store->slots;
+    a.k_cache = static_cast<uint4*>(store->k_cache);
+    a.v_cache = static_cast<uint4*>(store->v_cache);
+    a.num_slots = store->num_slots;
+    a.row_pieces = (uint32_t)num_kv_heads * kPieces;
+    a.new_pieces = (uint32_t)store->rows * a.row_pieces;
+  }
   return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype);
+}
+}  // namespace
+
+extern "C" int nvj_prefill_attention_rows_launch(
+    void* stream, const void* q, int64_t q_row_stride, const void* k, const void* v,
+    int64_t kv_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, void* out,
+    int32_t total_q_tokens, int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_dim, float scale, int32_t dtype) {
+  return launch_packed(stream, q, q_row_stride, k, v, kv_row_stride, cu_seqlens_q, cu_seqlens_k,
+                       out, total_q_tokens, batch, num_heads, num_kv_heads, head_dim, scale, dtype,
+                       nullptr);
+}
+
+extern "C" int nvj_prefill_attention_store_launch(
+    void* stream, const void* q, const void* k, const void* v, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, void* out, const int32_t* slot_mapping, void* k_cache,
+    void* v_cache, int64_t num_slots, int32_t total_q_tokens, int32_t num_rows, int32_t batch,
+    int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype) {
+  if (num_rows < 0 || num_slots < 0 || num_kv_heads <= 0 || head_dim <= 0)
+    return NVJ_ERR_BAD_SHAPE;
+  const auto store_alone = [&] {
+    return nvj_store_kvcache_launch(stream, k, v, k_cache, v_cache, slot_mapping, num_rows,
+                                    num_kv_heads, head_dim, num_slots, dtype, dtype, dtype);
+  };
+  if (num_rows > 0) {
+    if (!slot_mapping || !k_cache || !v_cache) return NVJ_ERR_NULL_POINTER;
+    if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15u)
+      return NVJ_ERR_ALIGNMENT;
+  }
+  const CacheRows rows = {slot_mapping, k_cache, v_cache, num_slots, num_rows};
+  // the kernel counts the pieces of all rows in 32 bits
+  const bool together = num_rows > 0 && total_q_tokens > 0 && batch > 0 &&
+                        (int64_t)num_rows * num_kv_heads * kPieces <= UINT32_MAX - 4096;
+  if (!together && num_rows > 0) {
+    const int code = store_alone();
+    if (code != NVJ_OK) return code;
+  }
+  return launch_packed(stream, q, (int64_t)num_heads * kD, k, v, (int64_t)num_kv_heads * kD,
+                       cu_seqlens_q, cu_seqlens_k, out, total_q_tokens, batch, num_heads,
+                       num_kv_heads, head_dim, scale, dtype, together ? &rows : nullptr);
 }
 
 extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const void* k,

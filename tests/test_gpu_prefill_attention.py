@@ -329,3 +329,53 @@ def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
                                       torch.from_numpy(table[i:i + 1].copy()).to(dev),
                                       cu(new[i:i + 1]), cu(total[i:i + 1]), 128 ** -0.5)
         assert torch.equal(got[at[i]:at[i + 1]], one), f"sequence {i}"
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,dtype,padding", [
+    ([1], 8, 8, "bf16", 0),                       # one row: fewer pieces than threads
+    ([0, 0, 0], 4, 2, "f16", 5),                  # rows that belong to no sequence only
+    ([700], 16, 8, "bf16", 0),                    # the small workgroups
+    ([3, 0, 130, 64, 17], 6, 2, "bf16", 9),       # rows behind the last offset are stored too
+    ([250, 31, 0, 300] * 12, 32, 8, "f16", 0),    # shares of more than one batch
+    ([90] * 60, 32, 8, "bf16", 1),                # 44 MB of output: past the L2s
+    ([2100, 1], 8, 1, "bf16", 0),
+])
+def test_prefill_with_the_store_in_the_launch(lens, Hq, Hkv, dtype, padding):
+    """Caches and output bit for bit as the store's own launch and the attention's leave
+    them, slots that are skipped or outside the caches among the rows."""
+    print(f"case prefill with store Hq={Hq} Hkv={Hkv} {dtype} {len(lens)} prompts", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib
+    lib, dev = _lib.load(), "cuda:0"
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    code = {"bf16": _lib.NVJ_DTYPE_BF16, "f16": _lib.NVJ_DTYPE_F16}[dtype]
+    g = torch.Generator(device=dev)
+    g.manual_seed(len(lens) + Hq)
+    rows, T = sum(lens), sum(lens) + padding
+    q, k, v = (torch.randn(T, h, 128, generator=g, device=dev, dtype=dt) for h in (Hq, Hkv, Hkv))
+    cu = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).to(dev)
+    num_slots = T + 7
+    slots = torch.randperm(num_slots, generator=g, device=dev)[:T].to(torch.int32)
+    if T > 4:
+        slots[T // 2], slots[T // 3], slots[1] = -1, num_slots, num_slots + 100
+    caches = [torch.zeros(num_slots, Hkv, 128, dtype=dt, device=dev) for _ in range(4)]
+    outs = [torch.zeros_like(q) for _ in range(2)]
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.nvj_store_kvcache_launch(
+        stream, k.data_ptr(), v.data_ptr(), caches[0].data_ptr(), caches[1].data_ptr(),
+        slots.data_ptr(), T, Hkv, 128, num_slots, code, code, code), "store")
+    _lib.check(lib.nvj_prefill_attention_launch(
+        stream, q.data_ptr(), k.data_ptr(), v.data_ptr(), cu.data_ptr(), cu.data_ptr(),
+        outs[0].data_ptr(), T, len(lens), Hq, Hkv, 128, 128 ** -0.5, code), "attention")
+    _lib.check(lib.nvj_prefill_attention_store_launch(
+        stream, q.data_ptr(), k.data_ptr(), v.data_ptr(), cu.data_ptr(), cu.data_ptr(),
+        outs[1].data_ptr(), slots.data_ptr(), caches[2].data_ptr(), caches[3].data_ptr(),
+        num_slots, T, T, len(lens), Hq, Hkv, 128, 128 ** -0.5, code), "together")
+    torch.cuda.synchronize()
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+    assert torch.equal(outs[0][:rows], outs[1][:rows])
+    assert not outs[1][rows:].any()               # rows of no sequence are left alone
+    if rows > 0 and T > 4:
+        want = k.double().cpu()
+        live = (slots >= 0) & (slots < num_slots)
+        assert torch.equal(caches[2][slots[live].long()].double().cpu(), want[live.cpu()])
