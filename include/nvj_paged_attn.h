@@ -245,8 +245,9 @@ NVJ_API int nvj_paged_decode_launch(void* stream,
  * the lengths.  Same results to the same tolerance; a measurement and test aid.
  *
  * NVJ_PHASE_SHORT_ROWS, or-ed in, lets a small launch of the balanced split (no more
- * (sequence, KV head) rows than compute units) finish each row inside one workgroup
- * where the lengths say that this is faster than sharing rows.  Same results to the
+ * (sequence, KV head) rows than compute units) finish each row inside one workgroup, or
+ * cut rows into pieces of a workgroup each, where the table's size or the lengths say that
+ * this is faster than the equal cut.  Same results to the
  * same tolerance; without it the way rows are cut depends on the lengths alone as
  * chunk == 0 describes, and with it the last bits.
  *

@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -917,18 +918,30 @@ __device__ __forceinline__ void write_output(const DecodeArgs& a, int b, int kvh
   }
 }
 
-// Result of a row that the 8 waves of a workgroup have walked in 8 parts: every part lies
-// in the K tile of its wave as add_partial_from_lds expects it, and wave w merges and
-// writes its eighth of the head dimensions (4 in every 32), each value by the recurrence
-// of add_partial_from_lds over the parts in order: the same bits as one wave merging all
-// of it, without its 7 x 34 LDS reads in a row (6.7 -> 5.7 us for rows of 256 positions;
-// not in the balanced kernel, whose registers it does not fit).
-template <int D, bool F16, int TILE>
-__device__ __forceinline__ void merge_parts_and_write(const DecodeArgs& a, uint4 (&k_tile)[8][TILE],
-                                                      int b, int kvh, int wave, int lane) {
+// A row (or a piece of one) that the 8 waves of a workgroup have walked in 8 parts: every part
+// lies in the K tile of its wave as add_partial_from_lds expects it (park_part), and wave w
+// merges its eighth of the head dimensions (4 in every 32: dims 32 * kg + 8 * e + jd .. + 3 of
+// query head r in lane (r, kg), e = w / 2, jd = 4 * (w % 2)), each value by the recurrence of
+// add_partial_from_lds over the parts in order: the same bits as one wave merging all of
+// it, without its 7 x 34 LDS reads in a row (6.7 -> 5.7 us for rows of 256 positions).
+template <int D>
+__device__ __forceinline__ void park_part(uint4* tile, int lane, const f32x4 (&acc)[8], float m_run,
+                                          float l_run) {
   constexpr int STRIDE = D / 32 * 16;
-  const int r = lane & 15, kg = lane >> 4;
-  if (r >= a.group || 32 * kg >= D) return;
+  if (lane >= STRIDE) return;   // (lanes whose k-group holds no dims)
+  float* mine = reinterpret_cast<float*>(tile) + lane;
+#pragma unroll
+  for (int jd = 0; jd < 8; ++jd)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine[(4 * jd + e) * STRIDE] = acc[jd][e];
+  mine[32 * STRIDE] = m_run;
+  mine[33 * STRIDE] = l_run;
+}
+template <int D, int TILE>
+__device__ __forceinline__ void merge_parts(const DecodeArgs& a, const uint4 (&k_tile)[8][TILE],
+                                            int wave, int lane, float (&acc)[4], float& m_run,
+                                            float& l_run) {
+  constexpr int STRIDE = D / 32 * 16;
   const int e = wave >> 1, jd = 4 * (wave & 1);
   float v[8][4], ml[8][2];
 #pragma unroll
@@ -939,8 +952,10 @@ __device__ __forceinline__ void merge_parts_and_write(const DecodeArgs& a, uint4
     ml[p][0] = t[32 * STRIDE];
     ml[p][1] = t[33 * STRIDE];
   }
-  float m_run = ml[0][0], l_run = ml[0][1];
-  float acc[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
+  m_run = ml[0][0];
+  l_run = ml[0][1];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = v[0][i];
 #pragma unroll
   for (int p = 1; p < 8; ++p) {
     const float m_new = fmaxf(m_run, ml[p][0]);
@@ -951,13 +966,18 @@ __device__ __forceinline__ void merge_parts_and_write(const DecodeArgs& a, uint4
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = fmaf(acc[i], keep, w * v[p][i]);
   }
+}
+// The wave's eighth of a finished row, by lanes with r < group and real dims.
+template <int D, bool F16>
+__device__ __forceinline__ void write_eighth(const DecodeArgs& a, int b, int kvh, int wave, int r,
+                                             int kg, const float (&acc)[4], float l_run) {
   const float inv = 1.0f / (l_run + 1e-9f);
   uint2 o;
   o.x = Elem<F16>::pack2(acc[0] * inv, acc[1] * inv);
   o.y = Elem<F16>::pack2(acc[2] * inv, acc[3] * inv);
   const int head = kvh * a.group + r;
   reinterpret_cast<uint2*>(a.out + ((int64_t)b * a.num_heads + head) * HeadDim<D>::kPieces)
-      [8 * kg + 2 * e + (wave & 1)] = o;
+      [8 * kg + wave] = o;   // piece 4 * kg + e, half wave % 2
 }
 
 // Unnormalised partial (D f32 per head) + (max, sum) to the workspace.  A
@@ -1063,27 +1083,21 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
   }
   if (parts > 1) {
     // value v of lane l at float v * kLanesWithDims + l of the wave's tile
-    const bool holds_dims = lane < kLanesWithDims;
     const bool all_merge = NW == 8 && hpw == 1;
-    __syncthreads();   // every wave is done reading its K tile
-    if ((part > 0 || all_merge) && holds_dims) {
-      float* mine = reinterpret_cast<float*>(k_tile[wave]) + lane;
-#pragma unroll
-      for (int jd = 0; jd < 8; ++jd)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) mine[(4 * jd + e) * kLanesWithDims] = acc[jd][e];
-      mine[32 * kLanesWithDims] = m_run;
-      mine[33 * kLanesWithDims] = l_run;
-    }
+    if (part > 0 || all_merge) park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
     __syncthreads();
     if constexpr (NW == 8) {
       if (all_merge) {
-        merge_parts_and_write<D, F16>(a, k_tile, b, kvh, wave, lane);
+        const int r = lane & 15, kg = lane >> 4;
+        if (r >= a.group || 32 * kg >= D) return;
+        float mine[4];
+        merge_parts<D>(a, k_tile, wave, lane, mine, m_run, l_run);
+        write_eighth<D, F16>(a, b, kvh, wave, r, kg, mine, l_run);
         return;
       }
     }
     if (part > 0) return;
-    if (holds_dims) {
+    if (lane < kLanesWithDims) {
       for (int p = 1; p < parts; ++p) {
         add_partial_from_lds<kLanesWithDims>(
             reinterpret_cast<const float*>(k_tile[wave + p * hpw]) + lane, a.scale_log2e, acc, m_run,
@@ -1414,6 +1428,212 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& a, uint4* lds, int b
   write_output<D, F16>(a, b, kvh, lane, acc, l_run);
 }
 
+// One piece of a row: its 8 waves have left their parts in the K tiles (park_part).  A row of
+// one piece is written at once; else the workgroup publishes the merged piece in slot `slot`
+// and the one that comes last, of `pieces` whose slots lie `stride` apart from `slot0`,
+// merges them and writes the row.  All 8 waves do both, each for its eighth of the dims, and
+// every load of the merge is in flight at once up to 4 pieces per lane group, so that a
+// shared row costs one acknowledged store, one count and one round trip.
+// counter: of the row (see arrive).  stale: the flag in front of all counters.
+template <int D, bool F16, int TILE>
+__device__ __forceinline__ void finish_piece(const DecodeArgs& a, const uint4 (&k_tile)[8][TILE],
+                                             int* lds_flag, int32_t* stale, int32_t* counter, int b,
+                                             int kvh, int slot, int slot0, int stride, int pieces,
+                                             int wave, int lane) {
+  static_assert(D == 128, "four k-groups");
+  float acc[4], m_run, l_run;
+  merge_parts<D>(a, k_tile, wave, lane, acc, m_run, l_run);
+  const int group = a.group;
+  const int dims = 32 * (lane >> 4) + 4 * wave;   // first of the lane's four
+  if (pieces == 1) {
+    if ((lane & 15) < group)
+      write_eighth<D, F16>(a, b, kvh, wave, lane & 15, lane >> 4, acc, l_run);
+    return;
+  }
+  if ((lane & 15) < group) {
+    const int64_t rec = (int64_t)slot * group;
+    const __amdgpu_buffer_rsrc_t wo =
+        device_window(a.part_o + rec * D, (int64_t)group * D * sizeof(float));
+    const vfloat4 mine = {acc[0], acc[1], acc[2], acc[3]};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(vuint4, mine), wo,
+                                           ((lane & 15) * D + dims) * 4, 0, kDeviceScope);
+    if (wave == 0 && lane < 16) {
+      const __amdgpu_buffer_rsrc_t wm =
+          device_window(a.part_ml + rec * 2, (int64_t)group * 2 * sizeof(float));
+      const vfloat2 ml = {m_run, l_run};
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(vuint2, ml), wm, lane * 8, 0,
+                                            kDeviceScope);
+    }
+  }
+  wait_for_stores();
+  __syncthreads();   // the whole piece has reached the device before it is counted
+  if (threadIdx.x == 0) {
+    const int old = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool wrong = old < 0 || old >= pieces;   // see arrive
+    if (wrong) __hip_atomic_store(stale, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (wrong || old + 1 == pieces)
+      __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *lds_flag = !wrong && old + 1 == pieces;
+  }
+  __syncthreads();
+  if (*lds_flag == 0) return;
+  // A row of 16 lanes holds 16 / gp lane groups of gp >= group lanes; lane group lg merges pieces
+  // lg, lg + 16 / gp, ..., then the lane groups are merged.  Lanes of padding heads read a
+  // real record and are dropped.
+  const int gp = group > 8 ? 16 : group > 4 ? 8 : group > 2 ? 4 : group > 1 ? 2 : 1;
+  const int lane_groups = 16 / gp;
+  const int lg = (lane & 15) / gp;
+  const int r = min((lane & 15) - lg * gp, group - 1);
+  const int64_t rec0 = (int64_t)slot0 * group;
+  const int64_t span = (int64_t)(pieces - 1) * stride * group + group;   // records
+  const __amdgpu_buffer_rsrc_t wo = device_window(a.part_o + rec0 * D, span * D * sizeof(float));
+  const __amdgpu_buffer_rsrc_t wm = device_window(a.part_ml + rec0 * 2, span * 2 * sizeof(float));
+  m_run = kNegBig;
+  l_run = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = 0.f;
+  for (int p0 = lg; __any(p0 < pieces); p0 += 4 * lane_groups) {
+    vfloat4 v[4];
+    vfloat2 ml[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      // (absent ones repeat the last with weight 0; a batch of four none of whose k-th exists
+      // in any lane group is not fetched)
+      const int p = p0 + k * lane_groups;
+      if (__any(p < pieces)) {
+        const int rec = min(p, pieces - 1) * stride * group + r;
+        v[k] = __builtin_bit_cast(vfloat4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               wo, (rec * D + dims) * 4, 0, kDeviceScope));
+        ml[k] = __builtin_bit_cast(
+            vfloat2, __builtin_amdgcn_raw_buffer_load_b64(wm, rec * 8, 0, kDeviceScope));
+        if (p >= pieces) ml[k] = vfloat2{kNegBig, 0.f};
+      } else {
+        v[k] = vfloat4{0.f, 0.f, 0.f, 0.f};
+        ml[k] = vfloat2{kNegBig, 0.f};
+      }
+    }
+    const float m_new =
+        fmaxf(m_run, fmaxf(fmaxf(ml[0].x, ml[1].x), fmaxf(ml[2].x, ml[3].x)));
+    const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+    l_run *= keep;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] *= keep;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float w = p0 + k * lane_groups < pieces
+                          ? __builtin_amdgcn_exp2f((ml[k].x - m_new) * a.scale_log2e)
+                          : 0.f;
+      l_run = fmaf(w, ml[k].y, l_run);
+      acc[0] = fmaf(w, v[k].x, acc[0]);
+      acc[1] = fmaf(w, v[k].y, acc[1]);
+      acc[2] = fmaf(w, v[k].z, acc[2]);
+      acc[3] = fmaf(w, v[k].w, acc[3]);
+    }
+    m_run = m_new;
+  }
+#define NVJ_MERGE_LANE_GROUPS(N)                                               \
+  if (gp <= N) {                                                               \
+    const float m_there = row_rotate<N>(m_run), m_new = fmaxf(m_run, m_there); \
+    const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e); \
+    const float w = __builtin_amdgcn_exp2f((m_there - m_new) * a.scale_log2e); \
+    m_run = m_new;                                                             \
+    l_run = l_run * keep + w * row_rotate<N>(l_run);                           \
+    _Pragma("unroll") for (int i = 0; i < 4; ++i)                              \
+      acc[i] = acc[i] * keep + w * row_rotate<N>(acc[i]);                      \
+  }
+  NVJ_MERGE_LANE_GROUPS(8)
+  NVJ_MERGE_LANE_GROUPS(4)
+  NVJ_MERGE_LANE_GROUPS(2)
+  NVJ_MERGE_LANE_GROUPS(1)
+#undef NVJ_MERGE_LANE_GROUPS
+  if ((lane & 15) < group) write_eighth<D, F16>(a, b, kvh, wave, r, lane >> 4, acc, l_run);
+}
+
+// Pieces: every row (sequence, KV head) on workgroups of its own, as many as there are, for
+// launches of few and short rows, where what counts is the chain of round trips.  A row is
+// cut into pieces of equal length, in multiples of one 32-position step for each of the 8
+// waves, the shortest that leave no more pieces than workgroups; the waves of a
+// workgroup walk a piece in equal shares and put it together in LDS.
+// grid.x = max_pieces workgroups (and those that store new rows), block = 512.
+template <bool F16, bool NEW>
+__global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, int batch,
+                                                                  int max_pieces,
+                                                                  int32_t* counters,
+                                                                  NewRows fresh) {
+  constexpr int D = 128, NW = 8;
+  using H = HeadDim<D>;
+  __shared__ uint4 k_tile[NW][kStep * H::kLdsRowPieces];
+  __shared__ int last;
+  const int g = blockIdx.x;
+  int new_slot = -1;
+  if constexpr (NEW) {
+    if (fresh.main_wgs > 0 && g >= fresh.main_wgs) {
+      store_new_row<F16>(a, fresh, g - fresh.main_wgs, NW * 64);
+      return;
+    }
+    if (fresh.main_wgs == 0 && g < batch) store_new_row<F16>(a, fresh, g, NW * 64);
+    new_slot = new_slot_of_lane(fresh, batch, threadIdx.x & 63);
+    static_assert(NW * 64 == kNullStreamWords, "a word per thread");
+    if (g == 0 && fresh.clear != nullptr) fresh.clear[threadIdx.x] = 0;
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int cap = a.max_blocks * a.block_size;
+  // the lengths, one sequence per lane (the host sees to it that there are no more)
+  const int ctx_here = lane < batch ? min(max(a.context_lens[lane], 0), cap) : 0;
+  const int steps_here = (ctx_here + kStep - 1) / kStep;
+  const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(steps_here), 63);
+  if (g < batch && __builtin_amdgcn_readlane(ctx_here, g & 63) <= 0) {
+    // an empty sequence has no piece: its zeros (0 / (0 + 1e-9)) are written here
+    uint4* orow = a.out + (int64_t)g * a.num_heads * H::kPieces;
+    for (int i = threadIdx.x; i < a.num_heads * H::kPieces; i += NW * 64)
+      orow[i] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  // `rounds` of NW steps per piece: the smallest number that fits, between the mean and the
+  // longest row (one piece a row, which fits: the host sees to it).
+  const int most = max_pieces / a.num_kv_heads;   // pieces of all sequences, per KV head
+  int incl = 0, number = 0;
+  auto fits = [&](int rounds) __attribute__((always_inline)) {
+    number = (int)((uint32_t)(steps_here + NW * rounds - 1) / (uint32_t)(NW * rounds));
+    incl = wave_inclusive_scan(number);
+    return __builtin_amdgcn_readlane(incl, 63) <= most;
+  };
+  int lo = max(1, (total + NW * most - 1) / (NW * most));
+  if (!fits(lo)) {
+    int hi = (wave_max(steps_here) + NW - 1) / NW;
+    ++lo;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (fits(mid)) hi = mid;
+      else lo = mid + 1;
+    }
+    (void)fits(lo);
+  }
+  // workgroup g: KV head g % heads of piece g / heads of them all
+  const int at = g / a.num_kv_heads, kvh = g - at * a.num_kv_heads;
+  const unsigned long long hit = __ballot(at < incl);
+  if (hit == 0ull) return;
+  const int b = __builtin_ctzll(hit);
+  const int pieces = __builtin_amdgcn_readlane(number, b);
+  const int first = __builtin_amdgcn_readlane(incl, b) - pieces;
+  const int ctx = __builtin_amdgcn_readlane(ctx_here, b);
+  const int nb = __builtin_amdgcn_readlane(steps_here, b);
+  const int piece = at - first;
+  const int s0 = piece * nb / pieces, s1 = (piece + 1) * nb / pieces;
+  const int w0 = s0 + wave * (s1 - s0) / NW, w1 = s0 + (wave + 1) * (s1 - s0) / NW;
+  f32x4 acc[8];
+#pragma unroll
+  for (int jd = 0; jd < 8; ++jd) acc[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = kNegBig, l_run = 0.f;
+  if (w1 > w0)
+    compute_segment<D, F16, NEW>(a, k_tile[wave], b, kvh, w0 * kStep, min(ctx, w1 * kStep), lane,
+                                 acc, m_run, l_run, &fresh, new_slot);
+  park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
+  __syncthreads();
+  finish_piece<D, F16>(a, k_tile, &last, counters, counters + 1 + b * a.num_kv_heads + kvh, b, kvh,
+                       g, first * a.num_kv_heads + kvh, a.num_kv_heads, pieces, wave, lane);
+}
+
 // grid.x = num_wgs, block = 512.  `min_steps`: fewest steps a sub-run may have
 // (in units of 1 << shift steps); `shift`: see Cut.
 template <int D, bool F16, int VG = 0, bool NEW = false>
@@ -1516,8 +1736,8 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
   // whatever their number (a CU draws 47 GB/s, with any number of loads in flight), the
   // equal cut 10 us + 2.4 per 1000 wave steps.  4 sequences of 64 / 256 / 512 positions
   // 10.7 / 11.5 / 11.8 us with the equal cut, 5.3 / 8.4 / 10.0 this way; 32 of 2048
-  // positions 50.1 / 47.  (Tables that hold no more than two rounds go to
-  // paged_decode_whole_kernel at once.)
+  // positions 50.1 / 47.  (Small tables go to paged_decode_whole_kernel or
+  // paged_decode_pieces_kernel at once; this is for wide ones with short rows in them.)
   // The row is walked below as a workgroup's run inside one row is: parts meet in LDS.
   // -------------------------------------------------------------------------
   bool short_row = false;
@@ -2058,19 +2278,29 @@ constexpr int kMinBalancedSteps = 1;
 constexpr int kWholeRowTolerance = 64;
 
 // Whether the table rules out rows (of at most one per CU) that are not short: two rounds
-// of the 8 waves of a workgroup, which take 2.8 us each, what one CU draws.  A third is
-// still less than the balanced split's two passes where rows are few, and where its
-// workgroups have a row or more each to share.  Measured with 520 .. 1024 positions and 1 ..
-// 32 KV heads, all rows alike or ragged, the kernel without a split against the balanced one,
-// us at 768 positions: 1 .. 16 rows 9.2 .. 10.9 / 11.8 .. 12.8, 32 rows 12.6 .. 14.2 /
-// 12.6 .. 14.0, 64 rows 13.6 .. 14.7 / 13.7 .. 15.6, 128 rows 15.6 / 17.5, 256 rows 19.4 /
-// 21.3; at 1024 (four rounds) 1 .. 8 rows 10.7 .. 11.8 / 11.8 .. 12.6, 16 rows 12.5 .. 14.6 /
-// 12.7 .. 13.4, 32 rows 17 / 13.3.
-// The balanced kernel does not take a third round for few rows when it finds short lengths
-// in a wider table: its start and its LDS merge make such a row 2.0 .. 2.6 us slower there,
-// and the equal cut as fast (8 rows of 768 positions 12.5 / 12.2).
+// of the 8 waves of a workgroup, which take 2.8 us each, what one CU draws; such rows are
+// finished inside one workgroup by the kernel without a split.  With more than half as many
+// rows as CUs a third round is still no worse than what else there is: us, without a split /
+// by pieces, at 512 positions 1 .. 64 rows 8.2 .. 9.8 / 9.0 .. 10.0, 128 rows 10.6 / 10.4, 256
+// rows 13.2 / 13.9; at 768 1 .. 16 rows 9.7 .. 9.9 / 9.0 .. 9.1, 64 rows 13.6 / 10.5, 128 rows
+// 13.7 / 13.2, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
 bool table_of_short_rows(int64_t rows, int64_t positions) {
-  return positions <= (rows <= 16 || rows >= 128 ? 3 : 2) * 8 * kStep;
+  return positions <= (rows > 128 ? 3 : 2) * 8 * kStep;
+}
+
+// Whether a launch of at most one row per CU goes by pieces (paged_decode_pieces_kernel), from
+// what the table can hold; else the balanced kernel looks at the lengths.  Pieces save what
+// the balanced kernel's larger head and its merges by single waves cost a small launch, 3 us:
+// by pieces / balanced, 1 .. 4 sequences of 1000 positions and 8 KV heads 8.9 .. 10.2 / 12.2 ..
+// 13.3 us, 8 of 100 .. 900 9.9 / 12.9, 8 of 128 .. 2048 13.8 / 14.7, 4 of 4096 17.0 / 20.2.
+// Against that a row is cut into whole pieces of one length for all rows, which leaves
+// workgroups idle when lengths differ and rows are many, and one KV head per workgroup
+// streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.7 / 73.4, 64 rows of
+// 1000 .. 16000 53.5 / 55.8 and of 16000 .. 32768 145 / 138, 128 rows of 300 .. 4096 28.9 /
+// 30.2 and of 500 .. 8000 47.3 / 46.0, 256 rows of 100 .. 1500 24.6 / 26.6 and of 128 .. 2048
+// 32.2 / 30.0.
+bool pieces_pay(int64_t rows, int64_t positions) {
+  return rows * positions <= (rows <= 64 ? 1 << 20 : rows <= 128 ? 1 << 19 : 3 << 17);
 }
 
 // Waves per workgroup of the fixed split = KV heads a workgroup covers: the
@@ -2270,10 +2500,10 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
   a.num_blocks = num_blocks;
   a.scale_log2e = scale * kLog2e;
 
-  // Short rows: a workgroup per (sequence, KV head), if the CUs and the lengths a wave
-  // keeps allow it.  Where the table itself rules longer rows out, no length needs to be
-  // looked at and the kernel without a split does it (64 / 256 / 512 positions 5.2 / 5.8
-  // / 7.5 us against 5.3 / 8.4 / 10.0 by way of the balanced kernel); otherwise that one
+  // Short rows: a workgroup per (sequence, KV head) or several, if the CUs and the lengths
+  // a wave keeps allow it.  Where the table itself rules longer rows out, no length needs to
+  // be looked at and the kernel without a split does it (64 / 256 / 512 positions 5.2 / 5.8
+  // / 7.5 us); else small launches go by pieces, and in others the balanced kernel
   // decides on the device.
   const int64_t all_rows = (int64_t)batch * num_kv_heads;
   const int short_rows = chunk == 0 && (phases & NVJ_PHASE_SHORT_ROWS) &&
@@ -2328,6 +2558,23 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
       }
       if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;
       dim3 grid;
+      const int64_t positions = (int64_t)max_blocks * block_size;
+      if (short_rows > 0 && head_dim == 128 && !valu && !loads_only && batch <= 64 &&
+          pieces_pay(all_rows, positions)) {
+        const int64_t rounds = (positions + 8 * kStep - 1) / (8 * kStep);
+        const int max_pieces = (int)std::min<int64_t>(all_rows * rounds, compute_units());
+        const NewRows fresh = rows_behind(new_rows, max_pieces, batch, &grid);
+        hipError_t rc;
+#define NVJ_LAUNCH_PIECES(...)                                                                \
+  rc = nvj::launch(paged_decode_pieces_kernel<__VA_ARGS__>, grid, dim3(512), s, a, batch,     \
+                   max_pieces, counters, fresh)
+        if (new_rows && f16) NVJ_LAUNCH_PIECES(true, true);
+        else if (new_rows) NVJ_LAUNCH_PIECES(false, true);
+        else if (f16) NVJ_LAUNCH_PIECES(true, false);
+        else NVJ_LAUNCH_PIECES(false, false);
+#undef NVJ_LAUNCH_PIECES
+        return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+      }
       const NewRows fresh =
           rows_behind(new_rows, short_rows > plan.num_wgs ? short_rows : plan.num_wgs, batch, &grid);
       hipError_t rc;

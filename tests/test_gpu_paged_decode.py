@@ -1014,6 +1014,65 @@ def test_short_rows(lens, Hq, Hkv, D):
         assert_close_bf16(torch_to_bits(got), want, what=f"lens={lens} phases={extra}")
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv", [
+    ([1000], 16, 8),                              # four pieces a row
+    ([4100], 2, 2),                               # 17, one of them short of a step
+    ([6000, 0, 1, 33], 6, 2),                     # a group of 3, an empty row, one lone row
+    ([300, 2048, 900, 257, 0, 1024, 700, 5], 32, 8),
+    ([3900, 40, 300], 16, 1),                     # a group of 16: one lane group
+    ([5000] + [20] * 63, 4, 4),                   # as many rows as CUs: a piece is the longest row
+    ([1100] * 20, 8, 4),
+])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_rows_in_pieces(lens, Hq, Hkv, dtype):
+    """Rows cut into pieces of a workgroup each, against the oracle; the counters are left
+    at zero, a launch on a counter that is not is flagged and the next is right again, and
+    replays of a graph follow lengths that change."""
+    print(f"case pieces lens={lens[:8]} Hq={Hq} Hkv={Hkv} {dtype}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
+    bs, B, dev = 64, len(lens), "cuda:0"
+    NB = sum(-(-n // bs) for n in lens) + 3
+    q, kc, vc, bt, ctx = make_problem(77 + B + Hq, B, Hq, Hkv, 128, bs, NB, lens)
+    assert bt.shape[1] * bs > 768                 # (smaller tables take no split)
+    scale = 128 ** -0.5
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)]
+    if dtype == "f16":
+        t = [x.half() for x in t]
+    t += [torch.from_numpy(x).to(dev) for x in (bt, ctx)]
+    phases = _lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE | _lib.NVJ_PHASE_SHORT_ROWS
+    ws = DecodeWorkspace.for_shape(B, Hq, 128, bt.shape[1], bs, Hkv, dev)
+    run = lambda: paged_attention(*t, scale, bs, phases=phases, workspace=ws)
+    assert not ws.counters.any()
+    got = run()
+    assert not ws.counters.any()
+    if dtype == "bf16":
+        assert_close_bf16(torch_to_bits(got), oracle(q, kc, vc, bt, ctx, scale, bs), what="pieces")
+    exact = lambda: paged_attention(*t, scale, bs, chunk=_lib.NVJ_CHUNK_WHOLE_SEQUENCE)
+    # two roundings of the same sums to the output's type
+    tol = 2.0 ** -7 if dtype == "bf16" else 2.0 ** -10
+    close = lambda x, y: (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
+    assert close(got, exact())
+    assert torch.equal(run(), got)                # no order of arrival in the result
+    ws.counters[1:1 + B * Hkv] = 1000             # every row: written wrong or not at all, flagged
+    run()
+    torch.cuda.synchronize()
+    if max(lens) > 2048:
+        assert ws.counters[0].item() == 1
+    ws.counters.zero_()
+    assert torch.equal(run(), got)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for _ in range(3):
+        graph.replay()
+        assert close(out, exact())
+        assert not ws.counters.any()
+        t[4].copy_((t[4] * 2 + 1) // 3)
+        torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("own_workspace", [False, True])
 @pytest.mark.parametrize("dtype,k_f32", [("bf16", True), ("f16", False)])
 @pytest.mark.parametrize("lens,split", [([1], 0), ([700], 0), ([33, 512, 65, 32, 0, 64], 0),
