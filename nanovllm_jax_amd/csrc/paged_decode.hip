@@ -1497,20 +1497,13 @@ __device__ __forceinline__ void finish_piece(const DecodeArgs& a, const uint4 (&
     vfloat2 ml[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      // (absent ones repeat the last with weight 0; a batch of four none of whose k-th exists
-      // in any lane group is not fetched)
-      const int p = p0 + k * lane_groups;
-      if (__any(p < pieces)) {
-        const int rec = min(p, pieces - 1) * stride * group + r;
-        v[k] = __builtin_bit_cast(vfloat4, __builtin_amdgcn_raw_buffer_load_b128(
-                                               wo, (rec * D + dims) * 4, 0, kDeviceScope));
-        ml[k] = __builtin_bit_cast(
-            vfloat2, __builtin_amdgcn_raw_buffer_load_b64(wm, rec * 8, 0, kDeviceScope));
-        if (p >= pieces) ml[k] = vfloat2{kNegBig, 0.f};
-      } else {
-        v[k] = vfloat4{0.f, 0.f, 0.f, 0.f};
-        ml[k] = vfloat2{kNegBig, 0.f};
-      }
+      // (absent ones repeat the last with weight 0: a branch around a load costs more than
+      // the load)
+      const int rec = min(p0 + k * lane_groups, pieces - 1) * stride * group + r;
+      v[k] = __builtin_bit_cast(vfloat4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             wo, (rec * D + dims) * 4, 0, kDeviceScope));
+      ml[k] = __builtin_bit_cast(
+          vfloat2, __builtin_amdgcn_raw_buffer_load_b64(wm, rec * 8, 0, kDeviceScope));
     }
     const float m_new =
         fmaxf(m_run, fmaxf(fmaxf(ml[0].x, ml[1].x), fmaxf(ml[2].x, ml[3].x)));
@@ -1547,6 +1540,348 @@ __device__ __forceinline__ void finish_piece(const DecodeArgs& a, const uint4 (&
   NVJ_MERGE_LANE_GROUPS(1)
 #undef NVJ_MERGE_LANE_GROUPS
   if ((lane & 15) < group) write_eighth<D, F16>(a, b, kvh, wave, r, lane >> 4, acc, l_run);
+}
+
+// The balanced split by the equal cut alone, for launches of up to 64 sequences that are offered
+// no other layout: the same cut, the same segments and the same order of every sum as
+// paged_decode_balanced_kernel, so the same bits, with less in front of the first load and less
+// behind the last.  Where a workgroup's run lies inside one row, the waves of a head
+// put its parts together, publish the partial and merge the row between them, each for its
+// share of the dims; one wave alone took 3.2 us for the parts of a workgroup and 4.5 us for
+// a row's partials.  16 / 8 heads, without a store: 1 sequence of 1000 positions 11.7 -> 9.9
+// us, 4 of 100 .. 900 12.0 -> 10.2, 8 of 500 .. 8000 21.0 -> 19.1; a stream of K and V hardly
+// notices (16 x 32768, 64 / 8 heads 319.4 -> 317.1).
+template <bool F16, int HPW>
+struct SharedRows {
+  static constexpr int D = 128, NW = 8;
+  static constexpr int kParts = NW / HPW;
+  static constexpr int kPieces = 8 / kParts;   // 16-byte pieces of a lane's 8 that a wave owns
+  static constexpr int kTile = kStep * HeadDim<D>::kLdsRowPieces;
+
+  // The parked parts 0 .. nparts - 1 of head `h`, this wave's pieces: piece u of the lane is
+  // acc[4 * (i & 1) ..][i >> 1] with i = kPieces * part + u (see add_partial_from_lds).
+  static __device__ __forceinline__ void merge_parts_of_head(const DecodeArgs& a,
+                                                             const uint4 (&k_tile)[NW][kTile],
+                                                             int h, int part, int nparts, int lane,
+                                                             f32x4 (&acc)[kPieces], float& m_run,
+                                                             float& l_run) {
+    constexpr int STRIDE = D / 32 * 16;
+    auto tile = [&](int p) {
+      return reinterpret_cast<const float*>(k_tile[p * HPW + h]) + lane;
+    };
+    auto fetch = [&](int p, float (&t)[4 * kPieces + 2]) {
+      const float* at = tile(p);
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) {
+        const int i = kPieces * part + u, jd = 4 * (i & 1), e = i >> 1;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) t[4 * u + v] = at[(4 * (jd + v) + e) * STRIDE];
+      }
+      t[4 * kPieces] = at[32 * STRIDE];
+      t[4 * kPieces + 1] = at[33 * STRIDE];
+    };
+    float t[kParts][4 * kPieces + 2];
+#pragma unroll
+    for (int p = 0; p < kParts; ++p) fetch(min(p, nparts - 1), t[p]);
+    m_run = t[0][4 * kPieces];
+    l_run = t[0][4 * kPieces + 1];
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u)
+      acc[u] = f32x4{t[0][4 * u], t[0][4 * u + 1], t[0][4 * u + 2], t[0][4 * u + 3]};
+#pragma unroll
+    for (int p = 1; p < kParts; ++p) {
+      if (p < nparts) {
+        const float m_new = fmaxf(m_run, t[p][4 * kPieces]);
+        const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+        const float w = __builtin_amdgcn_exp2f((t[p][4 * kPieces] - m_new) * a.scale_log2e);
+        m_run = m_new;
+        l_run = fmaf(l_run, keep, w * t[p][4 * kPieces + 1]);
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[u][v] = fmaf(acc[u][v], keep, w * t[p][4 * u + v]);
+      }
+    }
+  }
+  static __device__ __forceinline__ void write_pieces(const DecodeArgs& a, int b, int kvh, int part,
+                                                      int lane, const f32x4 (&acc)[kPieces],
+                                                      float l_run) {
+    if ((lane & 15) >= a.group) return;
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+      const float mine[4] = {acc[u][0], acc[u][1], acc[u][2], acc[u][3]};
+      write_eighth<D, F16>(a, b, kvh, kPieces * part + u, lane & 15, lane >> 4, mine, l_run);
+    }
+  }
+  // merge_row for this wave's pieces.
+  static __device__ __forceinline__ void merge_pieces(const DecodeArgs& a, uint4* lds, int b,
+                                                      int kvh, int part, int r0, int r1,
+                                                      const Cut& cut, int lane) {
+    constexpr int kSlots = 64, KG = D / 32;
+    const int first = cut.subrun_of(r0);
+    const int expected = cut.subrun_of(r1 - 1) - first + 1;
+    const int hg = kvh / HPW;
+    const int64_t slot0 = (int64_t)first + (int64_t)b * (a.num_kv_heads / HPW) + hg;
+    const int gp = a.group > 8 ? 16 : a.group > 4 ? 8 : a.group > 2 ? 4 : a.group > 1 ? 2 : 1;
+    const int lane_groups = 16 / gp;
+    const int lg = (lane & 15) / gp;
+    const int r = min((lane & 15) - lg * gp, a.group - 1);
+    const int kg = lane >> 4;
+    const int64_t rec0 = balanced_record(a, slot0, HPW, kvh - hg * HPW);
+    const int rec_stride = HPW * a.group;
+    const int64_t span = (int64_t)(expected - 1) * rec_stride + a.group;
+    const __amdgpu_buffer_rsrc_t wm = device_window(a.part_ml + rec0 * 2, span * 2 * sizeof(float));
+    const __amdgpu_buffer_rsrc_t wo = device_window(a.part_o + rec0 * D, span * D * sizeof(float));
+    const int slot_bytes = rec_stride * D * (int)sizeof(float);
+    const int piece_stride = KG * a.group * 16;
+    const int lane_off = (kg * a.group + r) * 16 + kPieces * part * piece_stride;
+    vfloat2* lds_ml = reinterpret_cast<vfloat2*>(lds);
+    uint8_t* lds_list = reinterpret_cast<uint8_t*>(lds_ml + kSlots * 16);
+    f32x4 acc[kPieces];
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = kNegBig, l_run = 0.f;
+    for (int base = 0; base < expected; base += kSlots) {
+      const int count = min(kSlots, expected - base);
+      const int c = min(lane & 15, a.group - 1);
+      vfloat2 got[kSlots / 4];
+#pragma unroll
+      for (int i = 0; i < kSlots / 4; ++i) {
+        const int s = min(base + 4 * i + kg, expected - 1);
+        got[i] = __builtin_bit_cast(vfloat2, __builtin_amdgcn_raw_buffer_load_b64(
+                                                 wm, (s * rec_stride + c) * 8, 0, kDeviceScope));
+      }
+      // which slots hold a partial, while these are on their way (see merge_row)
+      const int j = first + base + lane;
+      const int g = j / kParts;
+      const bool inside = cut.start_of(g * kParts) >= r0 &&
+                          cut.start_of(min(cut.nsub, g * kParts + kParts)) <= r1;
+      const bool mine_real = lane < count && (!inside || j == g * kParts);
+      const unsigned long long real = __ballot(mine_real);
+      const int nreal = __popcll(real);
+      if (mine_real) lds_list[__popcll(real & ((1ull << lane) - 1ull))] = (uint8_t)lane;
+      float m_chunk = kNegBig;
+#pragma unroll
+      for (int i = 0; i < kSlots / 4; ++i) {
+        lds_ml[(4 * i + kg) * 16 + (lane & 15)] = got[i];
+        const int sl = min(4 * i + kg, count - 1);
+        if ((real >> sl) & 1ull) m_chunk = fmaxf(m_chunk, got[i].x);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (nreal > 0) {
+        m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 16, 64));
+        m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 32, 64));
+        m_chunk = __shfl(m_chunk, (lane & 48) | r, 64);
+        const float m_new = fmaxf(m_run, m_chunk);
+        const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+        m_run = m_new;
+        l_run *= keep;
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u) acc[u] *= keep;
+        for (int done = 0; done < nreal; done += 4 * lane_groups) {
+          float w[4];
+          vfloat4 v[4][kPieces];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int n = done + k * lane_groups + lg;
+            const bool have = n < nreal;
+            const int idx = lds_list[have ? n : 0];
+            const int off = (base + idx) * slot_bytes + lane_off;
+#pragma unroll
+            for (int u = 0; u < kPieces; ++u)
+              v[k][u] = __builtin_bit_cast(
+                  vfloat4, __builtin_amdgcn_raw_buffer_load_b128(wo, off + u * piece_stride, 0,
+                                                                 kDeviceScope));
+            const vfloat2 ml = lds_ml[idx * 16 + r];
+            w[k] = have ? __builtin_amdgcn_exp2f((ml.x - m_new) * a.scale_log2e) : 0.f;
+            l_run = fmaf(w[k], ml.y, l_run);
+          }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+#pragma unroll
+            for (int u = 0; u < kPieces; ++u) {
+              acc[u][0] = fmaf(w[k], v[k][u].x, acc[u][0]);
+              acc[u][1] = fmaf(w[k], v[k][u].y, acc[u][1]);
+              acc[u][2] = fmaf(w[k], v[k][u].z, acc[u][2]);
+              acc[u][3] = fmaf(w[k], v[k][u].w, acc[u][3]);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+#define NVJ_ADD_LANE_GROUPS(N)                                         \
+  if (gp <= N) {                                                       \
+    l_run += row_rotate<N>(l_run);                                     \
+    _Pragma("unroll") for (int u = 0; u < kPieces; ++u)                \
+      _Pragma("unroll") for (int v = 0; v < 4; ++v)                    \
+        acc[u][v] += row_rotate<N>(acc[u][v]);                         \
+  }
+    NVJ_ADD_LANE_GROUPS(8)
+    NVJ_ADD_LANE_GROUPS(4)
+    NVJ_ADD_LANE_GROUPS(2)
+    NVJ_ADD_LANE_GROUPS(1)
+#undef NVJ_ADD_LANE_GROUPS
+    write_pieces(a, b, kvh, part, lane, acc, l_run);
+  }
+};
+
+template <bool F16, int HPW>
+__global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, int batch,
+                                                                  int num_wgs, int min_steps,
+                                                                  int shift, int32_t* counters) {
+  using R = SharedRows<F16, HPW>;
+  constexpr int D = R::D, NW = R::NW, kParts = R::kParts;
+  using H = HeadDim<D>;
+  __shared__ uint4 k_tile[NW][R::kTile];
+  __shared__ int last[HPW];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = blockIdx.x;
+  const int cap = a.max_blocks * a.block_size;
+  const int rows_per_seq = a.num_kv_heads / HPW;
+  const int part = wave / HPW, h_in_row = wave % HPW;
+
+  // the lengths, one sequence per lane (the host sees to it that there are no more)
+  const int kept_ctx = lane < batch ? min(max(a.context_lens[lane], 0), cap) : 0;
+  const int kept_steps = (kept_ctx + kStep - 1) / kStep;
+  const int incl = wave_inclusive_scan(kept_steps);
+  const int kept_before = incl - kept_steps;
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  for (int b = g; b < batch; b += num_wgs) {   // zeros of empty sequences
+    if (__builtin_amdgcn_readlane(kept_ctx, b) > 0) continue;
+    uint4* orow = a.out + (int64_t)b * a.num_heads * H::kPieces;
+    for (int i = threadIdx.x; i < a.num_heads * H::kPieces; i += NW * 64)
+      orow[i] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  Cut cut;
+  cut.axis = rows_per_seq * total;
+  cut.shift = shift;
+  cut.units = (cut.axis + (1 << shift) - 1) >> shift;
+  cut.nsub = max(1, min(num_wgs * kParts, cut.units / min_steps));
+  if (cut.axis == 0 || g * kParts >= cut.nsub) return;
+
+  // the sequence whose rows hold axis position x
+  auto locate = [&](int x, int& b, int& before, int& ctx) __attribute__((always_inline)) {
+    const int lo = rows_per_seq * kept_before;
+    const unsigned long long hit = __ballot(lo <= x && x < lo + rows_per_seq * kept_steps);
+    b = hit != 0ull ? __builtin_ctzll(hit) : batch;
+    before = __builtin_amdgcn_readlane(kept_before, b & 63);
+    ctx = hit != 0ull ? __builtin_amdgcn_readlane(kept_ctx, b & 63) : 0;
+  };
+  const int nparts = min(kParts, cut.nsub - g * kParts);   // parts that have work
+  const int start = cut.start_of(g * kParts), end = cut.start_of(g * kParts + nparts);
+  int b, before, ctx;
+  locate(start, b, before, ctx);
+  if (b >= batch || ctx <= 0) return;   // cannot happen when the prefix sums are right
+  const int nb0 = (ctx + kStep - 1) / kStep;
+  const int hg0 = (start - rows_per_seq * before) / nb0;
+  const int row0 = rows_per_seq * before + hg0 * nb0;
+  const int xs = part < nparts ? cut.start_of(g * kParts + part) : end;
+  const int xe = part < nparts ? cut.start_of(g * kParts + part + 1) : end;
+  if (end <= row0 + nb0) {
+    // The whole run of the workgroup lies inside one row.
+    const int kvh = hg0 * HPW + h_in_row;
+    float m_run = kNegBig, l_run = 0.f;
+    f32x4 mine[R::kPieces];
+    {
+      f32x4 acc[8];
+#pragma unroll
+      for (int jd = 0; jd < 8; ++jd) acc[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (xs < xe)
+        compute_segment<D, F16>(a, k_tile[wave], b, kvh, (xs - row0) * kStep,
+                                min(ctx, (xe - row0) * kStep), lane, acc, m_run, l_run);
+      park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
+    }
+    __syncthreads();
+    R::merge_parts_of_head(a, k_tile, h_in_row, part, nparts, lane, mine, m_run, l_run);
+    if (start == row0 && end == row0 + nb0) {
+      R::write_pieces(a, b, kvh, part, lane, mine, l_run);
+      return;
+    }
+    // the partial, in the slot of part 0 (write_partial_coherent)
+    const int64_t slot = (int64_t)g * kParts + (int64_t)b * rows_per_seq + hg0;
+    const int64_t rec = balanced_record(a, slot, HPW, h_in_row);
+    const int r = lane & 15, kg = lane >> 4;
+    if (r < a.group) {
+      const __amdgpu_buffer_rsrc_t wo =
+          device_window(a.part_o + rec * D, (int64_t)a.group * D * sizeof(float));
+      const int piece_stride = D / 32 * a.group * 16;
+#pragma unroll
+      for (int u = 0; u < R::kPieces; ++u) {
+        const vfloat4 v = {mine[u][0], mine[u][1], mine[u][2], mine[u][3]};
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(vuint4, v), wo,
+            (kg * a.group + r) * 16 + (R::kPieces * part + u) * piece_stride, 0, kDeviceScope);
+      }
+      if (part == 0 && kg == 0) {
+        const __amdgpu_buffer_rsrc_t wm =
+            device_window(a.part_ml + rec * 2, (int64_t)a.group * 2 * sizeof(float));
+        const vfloat2 ml = {m_run, l_run};
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(vuint2, ml), wm, r * 8, 0,
+                                              kDeviceScope);
+      }
+    }
+    wait_for_stores();
+    __syncthreads();   // the whole partial has reached the device before it is counted
+    if (part == 0) {
+      const bool to_merge = arrive(a, counters, b, kvh, row0, row0 + nb0, cut, nparts, lane);
+      if (lane == 0) last[h_in_row] = to_merge;
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(last[h_in_row]))
+      R::merge_pieces(a, k_tile[wave], b, kvh, part, row0, row0 + nb0, cut, lane);
+    return;
+  }
+
+  // Every wave walks its own sub-run across the rows.
+  if (xs >= xe) return;
+  int x = xs;
+  if (part > 0) locate(xs, b, before, ctx);
+  int owed = 0, owed_b[2] = {0, 0}, owed_kvh[2] = {0, 0}, owed_row[2] = {0, 0}, owed_nb[2] = {1, 1};
+  while (x < xe && b < batch) {
+    // ---- the next segment: row (sb, hg), steps [st, en) ----
+    const int sb = b, nb = (ctx + kStep - 1) / kStep, seq0 = rows_per_seq * before;
+    if (x < seq0) break;
+    if (nb == 0 || x >= seq0 + rows_per_seq * nb) {   // empty, or this sequence is finished
+      before += nb;
+      ++b;
+      ctx = b < batch ? __builtin_amdgcn_readlane(kept_ctx, b & 63) : 0;
+      continue;
+    }
+    const int hg = (x - seq0) / nb, row = seq0 + hg * nb;
+    const int st = x - row, en = min(nb, st + (xe - x));
+    const int kvh = hg * HPW + h_in_row;
+    f32x4 acc[8];
+#pragma unroll
+    for (int jd = 0; jd < 8; ++jd) acc[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = kNegBig, l_run = 0.f;
+    compute_segment<D, F16>(a, k_tile[wave], sb, kvh, st * kStep, min(ctx, en * kStep), lane, acc,
+                            m_run, l_run);
+    x += en - st;
+    if (st == 0 && en == nb) {
+      write_output<D, F16>(a, sb, kvh, lane, acc, l_run);
+    } else {
+      const int64_t slot = (int64_t)g * kParts + part + (int64_t)sb * rows_per_seq + hg;
+      write_partial_coherent<D>(a, balanced_record(a, slot, HPW, h_in_row), lane, acc, m_run, l_run);
+      if (arrive(a, counters, sb, kvh, row, row + nb, cut, 1, lane)) {
+        // at most the first and the last segment of a sub-run are not whole rows
+        if (owed == 0) { owed_b[0] = sb; owed_kvh[0] = kvh; owed_row[0] = row; owed_nb[0] = nb; }
+        else { owed_b[1] = sb; owed_kvh[1] = kvh; owed_row[1] = row; owed_nb[1] = nb; }
+        ++owed;
+      }
+    }
+  }
+  for (int i = 0; i < owed; ++i) {
+    const int ob = __builtin_amdgcn_readfirstlane(i == 0 ? owed_b[0] : owed_b[1]);
+    const int okvh = __builtin_amdgcn_readfirstlane(i == 0 ? owed_kvh[0] : owed_kvh[1]);
+    const int orow = __builtin_amdgcn_readfirstlane(i == 0 ? owed_row[0] : owed_row[1]);
+    const int onb = __builtin_amdgcn_readfirstlane(i == 0 ? owed_nb[0] : owed_nb[1]);
+    merge_row<D, F16>(a, k_tile[wave], ob, okvh, HPW, orow, orow + onb, cut, lane);
+  }
 }
 
 // Pieces: every row (sequence, KV head) on workgroups of its own, as many as there are, for
@@ -2573,6 +2908,23 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
         else if (f16) NVJ_LAUNCH_PIECES(true, false);
         else NVJ_LAUNCH_PIECES(false, false);
 #undef NVJ_LAUNCH_PIECES
+        return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+      }
+      if (!new_rows && short_rows == 0 && head_dim == 128 && !valu && !loads_only && batch <= 64 &&
+          (plan.wr_hpw == 0 || (phases & NVJ_PHASE_SHARED_ROWS))) {
+        // nothing but the equal cut on offer
+        hipError_t rc;
+#define NVJ_LAUNCH_SHARED(N)                                                                   \
+  rc = f16 ? nvj::launch(paged_decode_shared_kernel<true, N>, dim3((unsigned)plan.num_wgs),    \
+                         dim3(512), s, a, batch, plan.num_wgs, kMinBalancedSteps, plan.shift,  \
+                         counters)                                                             \
+           : nvj::launch(paged_decode_shared_kernel<false, N>, dim3((unsigned)plan.num_wgs),   \
+                         dim3(512), s, a, batch, plan.num_wgs, kMinBalancedSteps, plan.shift,  \
+                         counters)
+        if (plan.hpw == 1) NVJ_LAUNCH_SHARED(1);
+        else if (plan.hpw == 2) NVJ_LAUNCH_SHARED(2);
+        else NVJ_LAUNCH_SHARED(4);
+#undef NVJ_LAUNCH_SHARED
         return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
       }
       const NewRows fresh =

@@ -1073,6 +1073,40 @@ def test_rows_in_pieces(lens, Hq, Hkv, dtype):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(8, 4), (64, 8), (6, 2), (16, 1)])   # 4, 4, 2, 1 heads side by side
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("hi", [200, 4000])              # sub-runs of one step, and of many
+def test_equal_cut_of_few_and_of_many_sequences(Hq, Hkv, dtype, hi):
+    """Up to 64 sequences have a kernel of their own for the equal cut; with empty sequences
+    behind them the same rows go through the kernel for any number: the same bits."""
+    print(f"case equal cut Hq={Hq} Hkv={Hkv} {dtype} up to {hi}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    rng = np.random.default_rng(Hq + hi)
+    lens = rng.integers(0, hi, 36)
+    lens[[0, 5, 35]] = 0, 1, hi
+    bs = 64
+    NB = int((-(-lens // bs)).sum()) + 2
+    q, kc, vc, bt, ctx = make_problem(Hq + Hkv + hi, 36, Hq, Hkv, 128, bs, NB, lens)
+    wide = np.full((36, 256 * 32 // bs), -1, np.int32)   # a workgroup for every CU either way
+    wide[:, :bt.shape[1]] = bt
+    dev, outs = "cuda:0", []
+    for batch in (36, 70):
+        pad = lambda x: np.concatenate([x, np.zeros((batch - 36, *x.shape[1:]), x.dtype)])
+        t = [bits_to_torch(x, dev) for x in (pad(q), kc, vc)]
+        if dtype == "f16":
+            t = [x.half() for x in t]
+        outs.append(paged_attention(
+            *t, torch.from_numpy(pad(wide)).to(dev), torch.from_numpy(pad(ctx)).to(dev), 128 ** -0.5,
+            bs, chunk=0, phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+            | _lib.NVJ_PHASE_SHARED_ROWS)[:36])
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    if dtype == "bf16":
+        assert_close_bf16(torch_to_bits(outs[0]), oracle(q, kc, vc, bt, ctx, 128 ** -0.5, bs),
+                          what="equal cut")
+
+
 @pytest.mark.parametrize("own_workspace", [False, True])
 @pytest.mark.parametrize("dtype,k_f32", [("bf16", True), ("f16", False)])
 @pytest.mark.parametrize("lens,split", [([1], 0), ([700], 0), ([33, 512, 65, 32, 0, 64], 0),
