@@ -26,6 +26,17 @@ __device__ __forceinline__ void copy16_to_lds(const char* base, uint32_t offset,
       : "s"(lds_base), "v"(offset), "s"(base)
       : "memory", "m0");
 }
+// The same with 4 bytes per lane: lane l's lands at lds_base + 4 * l.
+__device__ __forceinline__ void copy4_to_lds(const void* base, uint32_t offset,
+                                             uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %1, %2"
+      :
+      : "s"(lds_base), "v"(offset), "s"(base)
+      : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 }  // namespace nvj

@@ -53,6 +53,83 @@ __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// QK-RMSNorm, RoPE and KV store of a tile of kHeads heads, in LDS as bf16 rows of `stride`
+// bytes.  16 lanes per (row, head): unit u of a workgroup is row (16 * u + its group of 16
+// lanes) / kHeads; N units at a time.  Bound by round trips where a workgroup is alone on its
+// CU: positions and slots come with the first copies into LDS, table rows a batch ahead (4300
+// rows of 4096 x 1024, us: 256 x 256 tiles 89.7 -> 79.1, 160 x 256 61.1 -> 56.3; 160 x 128, two
+// to a CU, which cover for each other, 50.3 -> 49.5, where 39 are the product's; 128 rows
+// 7.7 -> 7.4 of 5.5).
+//
+// A group of lanes works on the same head in every unit, so the norm's weights are fetched
+// once: behind a store of the unit before they would be fetched again, a round trip a unit.
+template <int kHeads>
+struct RopeHead {
+  int h, head;                 // of the tile, of all
+  bool is_q, is_k, norm;
+  float4 wl, wh;
+  __device__ __forceinline__ RopeHead(const LinearArgs& a, int n_tile) {
+    static_assert(16 % kHeads == 0, "one head per group of lanes");
+    h = (int)(threadIdx.x >> 4) % kHeads;
+    head = n_tile * kHeads + h;
+    is_q = head < a.num_heads;
+    is_k = !is_q && head < a.num_heads + a.num_kv_heads;
+    norm = a.q_norm != nullptr;
+    wl = wh = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (norm && (is_q || is_k)) {
+      const float* w = (is_q ? a.q_norm : a.k_norm) + 4 * (threadIdx.x & 15);
+      wl = nvj::load4<true>(w);
+      wh = nvj::load4<true>(w + 64);
+    }
+  }
+};
+template <int N, int kHeads>
+struct RopeUnits {
+  int slot[N];
+  float4 c4[N], s4[N];
+
+  // places: positions of the tile's rows, then (from place `slots`) their slots, in LDS
+  __device__ __forceinline__ void fetch(const LinearArgs& a, const int* places, int slots, int u0) {
+    const int i = threadIdx.x & 15;
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      const int m = ((u0 + b) * 16 + (int)(threadIdx.x >> 4)) / kHeads;
+      slot[b] = places[slots + m];
+      const float* cs =
+          a.cos_sin + (int64_t)min(max(places[m], 0), a.max_position - 1) * 128 + 4 * i;
+      c4[b] = nvj::load4<true>(cs);
+      s4[b] = nvj::load4<true>(cs + 64);
+    }
+  }
+  __device__ __forceinline__ void rows(const LinearArgs& a, const RopeHead<kHeads>& t,
+                                       const char* lds, int stride, int m0, int u0) const {
+    const int i = threadIdx.x & 15;
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      const int m = ((u0 + b) * 16 + (int)(threadIdx.x >> 4)) / kHeads, token = m0 + m;
+      if (token >= a.M) continue;
+      const uint2* src = reinterpret_cast<const uint2*>(lds + m * stride + 256 * t.h);
+      uint2 lo = src[i], hi = src[16 + i];
+      if (t.is_q || t.is_k)
+        nvj::qk_norm_rope(lo, hi, t.norm, t.wl, t.wh, a.eps, c4[b], s4[b]);
+      if (t.is_q || a.keep_kv) {
+        uint2* dst = reinterpret_cast<uint2*>(
+            t.is_q ? a.q_out + ((int64_t)token * a.num_heads + t.head) * 128
+                   : a.out + (int64_t)token * a.N + t.head * 128);
+        dst[i] = lo;
+        dst[16 + i] = hi;
+      }
+      if (!t.is_q && slot[b] >= 0 && slot[b] < a.num_slots) {
+        const int kvh = t.head - a.num_heads - (t.is_k ? 0 : a.num_kv_heads);
+        uint2* row = reinterpret_cast<uint2*>((t.is_k ? a.k_cache : a.v_cache) +
+                                              ((int64_t)slot[b] * a.num_kv_heads + kvh) * 128);
+        row[i] = lo;
+        row[16 + i] = hi;
+      }
+    }
+  }
+};
+
 template <int BM, int BN, int kStages, Epilogue EPI>
 __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   constexpr int WM = BM / 2, WN = BN / 2;          // per wave
@@ -83,6 +160,22 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   const int n_tile = in_group / gm, m_tile = grp * a.group_m + (in_group - n_tile * gm);
   const int m0 = m_tile * BM;
   const int row_bytes = a.K * 2;
+
+  // kQkRope: positions and slots of the rows first of all, so that nothing waits for them
+  constexpr int kHeads = BN >= 128 ? BN / 128 : 1, kUnits = BM * kHeads / 16;
+  constexpr int kBatch = kUnits % 5 == 0 ? 5 : kUnits % 4 == 0 ? 4 : 2;
+  static_assert(EPI != kQkRope || kUnits % kBatch == 0, "whole batches");
+  constexpr int kPlaces = (BM + 63) / 64 * 64;
+  __shared__ int places[EPI == kQkRope ? 2 * kPlaces : 1];
+  RopeUnits<kBatch, kHeads> units;
+  if constexpr (EPI == kQkRope) {
+    if (64 * wave < kPlaces) {
+      const uint32_t at = (uint32_t)(uintptr_t)(lds_ptr)places + 256u * wave;
+      const uint32_t from = 4u * (uint32_t)min(m0 + 64 * wave + lane, a.M - 1);
+      nvj::copy4_to_lds(a.positions, from, at);
+      nvj::copy4_to_lds(a.slot_mapping, from, at + 4u * kPlaces);
+    }
+  }
 
   // what this wave copies: instruction j moves LDS rows 8 * (4 * j + wave) .. + 7; lane
   // l fetches the piece that belongs at position l % 8 of row l / 8
@@ -146,6 +239,8 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   for (int t = 0; t < kStages; ++t) issue(t, t);
   wait_copies<(kStages - 1) * kCopies>();
   __syncthreads();
+  // few units: the table rows too, under the whole reduction
+  if constexpr (EPI == kQkRope && kUnits == kBatch) units.fetch(a, places, kPlaces, 0);
 #pragma unroll
   for (int i = 0; i < kRead; ++i) read(0, 0, i);
   int stage = 0;
@@ -177,6 +272,7 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
     stage = next;
   }
   wait_copies<0>();   // copies past the last step are still landing
+  if constexpr (EPI == kQkRope && kUnits > kBatch) units.fetch(a, places, kPlaces, 0);
   __syncthreads();
 
   // ---- the tile as bf16 rows in LDS, then out in whole pieces ----
@@ -206,56 +302,13 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   }
   __syncthreads();
   if constexpr (EPI == kQkRope) {
-    // 16 lanes per (row, head), a tile holds whole heads; the positions and slots of a
-    // batch of rows are fetched together, then their table rows: two round trips per
-    // batch instead of two per row
-    constexpr int kHeads = BN / 128, kUnits = BM * kHeads / 16;
-    constexpr int kBatch = kUnits % 5 == 0 ? 5 : kUnits % 4 == 0 ? 4 : 2;
-    static_assert(kUnits % kBatch == 0, "whole batches");
-    const int i = threadIdx.x & 15;
+    // the table rows of a batch of units are on their way while the one before is worked on
+    const RopeHead<kHeads> head(a, n_tile);
     for (int u0 = 0; u0 < kUnits; u0 += kBatch) {
-      int pos[kBatch], slot[kBatch];
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int m = ((u0 + b) * 16 + (int)(threadIdx.x >> 4)) / kHeads;
-        const int token = min(m0 + m, a.M - 1);
-        pos[b] = a.positions[token];
-        slot[b] = a.slot_mapping[token];
-      }
-      float4 c4[kBatch], s4[kBatch];
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const float* cs = a.cos_sin + (int64_t)min(max(pos[b], 0), a.max_position - 1) * 128 + 4 * i;
-        c4[b] = nvj::load4<true>(cs);
-        s4[b] = nvj::load4<true>(cs + 64);
-      }
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int unit = (u0 + b) * 16 + (int)(threadIdx.x >> 4);
-        const int m = unit / kHeads, h = unit % kHeads;
-        const int token = m0 + m, head = n_tile * kHeads + h;
-        if (token >= a.M) continue;
-        const uint2* src = reinterpret_cast<const uint2*>(lds + m * kOutStride + 256 * h);
-        uint2 lo = src[i], hi = src[16 + i];
-        const bool is_q = head < a.num_heads;
-        const bool is_k = !is_q && head < a.num_heads + a.num_kv_heads;
-        if (is_q || is_k)
-          nvj::qk_norm_rope<true>(lo, hi, is_q ? a.q_norm : a.k_norm, a.eps, c4[b], s4[b], i);
-        if (is_q || a.keep_kv) {
-          uint2* dst = reinterpret_cast<uint2*>(
-              is_q ? a.q_out + ((int64_t)token * a.num_heads + head) * 128
-                   : a.out + (int64_t)token * a.N + head * 128);
-          dst[i] = lo;
-          dst[16 + i] = hi;
-        }
-        if (!is_q && slot[b] >= 0 && slot[b] < a.num_slots) {
-          const int kvh = head - a.num_heads - (is_k ? 0 : a.num_kv_heads);
-          uint2* row = reinterpret_cast<uint2*>((is_k ? a.k_cache : a.v_cache) +
-                                                ((int64_t)slot[b] * a.num_kv_heads + kvh) * 128);
-          row[i] = lo;
-          row[16 + i] = hi;
-        }
-      }
+      RopeUnits<kBatch, kHeads> next;
+      if (u0 + kBatch < kUnits) next.fetch(a, places, kPlaces, u0 + kBatch);
+      units.rows(a, head, lds, kOutStride, m0, u0);
+      units = next;
     }
   } else {
     constexpr int kPieces = kOut / 8;

@@ -35,17 +35,16 @@ __device__ __forceinline__ float4 load4(const float* p) {
   return make_float4(p[0], p[1], p[2], p[3]);
 }
 
-// `weight`: [128] or null (no norm); c4, s4: the lane's four cosines and sines of this
-// position; i: the lane in its group of 16 (all 16 are active).
-template <bool WIDE>
-__device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, const float* weight, float eps,
-                                             const float4& c4, const float4& s4, int i) {
+// `norm`: with the RMSNorm, of weights wl and wh (the lane's elements 4i .. and 64 + 4i ..);
+// c4, s4: the lane's four cosines and sines of this position (all 16 lanes are active).
+__device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, bool norm, const float4& wl,
+                                             const float4& wh, float eps, const float4& c4,
+                                             const float4& s4) {
 #pragma clang fp contract(off)
   float x1[4], x2[4];
   unpack4(lo, x1);
   unpack4(hi, x2);
-  if (weight != nullptr) {
-    const float4 wl = load4<WIDE>(weight + 4 * i), wh = load4<WIDE>(weight + 64 + 4 * i);
+  if (norm) {
     const float w1[4] = {wl.x, wl.y, wl.z, wl.w}, w2[4] = {wh.x, wh.y, wh.z, wh.w};
     float s[4];
 #pragma unroll
@@ -77,6 +76,17 @@ __device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, const float* 
   }
   lo = pack4(y1);
   hi = pack4(y2);
+}
+// `weight`: [128] or null (no norm); i: the lane in its group of 16.
+template <bool WIDE>
+__device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, const float* weight, float eps,
+                                             const float4& c4, const float4& s4, int i) {
+  float4 wl = {}, wh = {};
+  if (weight != nullptr) {
+    wl = load4<WIDE>(weight + 4 * i);
+    wh = load4<WIDE>(weight + 64 + 4 * i);
+  }
+  qk_norm_rope(lo, hi, weight != nullptr, wl, wh, eps, c4, s4);
 }
 
 }  // namespace nvj
