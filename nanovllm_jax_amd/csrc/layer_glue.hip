@@ -22,6 +22,7 @@
 
 #include "launch.h"
 #include "nvj_paged_attn.h"
+#include "past_l2.h"
 
 namespace {
 
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(
         o.y = pack2(s[j][2], s[j][3]);
         o.z = pack2(s[j][4], s[j][5]);
         o.w = pack2(s[j][6], s[j][7]);
-        residual_out[row + p] = o;
+        nvj::store_past_l2(residual_out + row + p, o);   // (read again two products later)
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) a = a + s[j][e] * s[j][e];

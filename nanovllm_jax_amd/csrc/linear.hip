@@ -20,6 +20,11 @@
 // Weights straight into registers instead (as in decoder_step.hip) were no way out: 64-byte
 // pieces of 16 rows per load made it 1 us per step whatever the tile.
 //
+// Rows go past the writing XCD's L2 where that was measured to help the step: the plain rows
+// (a norm on all XCDs reads them once), q and the cache rows: 4268 rows in 8 prompts 6310 ->
+// 6184 us with the norm's residual (layer_glue.hip), 128 rows of decode 3517 -> 3492; not SiLU *
+// up and the packed K and V, which the next launch reads several times.
+//
 // Every output is one chain of v_mfma_f32_16x16x32_bf16 over K in order, whatever the tile
 // and the rows beside it (decoder_step.hip says where the library GEMMs sum likewise).
 #include <hip/hip_runtime.h>
@@ -31,6 +36,7 @@
 #include "lds_copy.h"
 #include "linear.h"
 #include "nvj_paged_attn.h"
+#include "past_l2.h"
 #include "qk_norm_rope.h"
 
 namespace {
@@ -46,6 +52,7 @@ using nvj::f32x4;
 using nvj::f32_to_bf16_rne;
 using nvj::LinearArgs;
 using nvj::pack2_bf16;
+using nvj::store_past_l2;
 enum Epilogue { kPlain, kSiluMul, kQkRope };
 
 template <int N>
@@ -116,15 +123,20 @@ struct RopeUnits {
         uint2* dst = reinterpret_cast<uint2*>(
             t.is_q ? a.q_out + ((int64_t)token * a.num_heads + t.head) * 128
                    : a.out + (int64_t)token * a.N + t.head * 128);
-        dst[i] = lo;
-        dst[16 + i] = hi;
+        if (t.is_q) {
+          store_past_l2(dst + i, lo);
+          store_past_l2(dst + 16 + i, hi);
+        } else {
+          dst[i] = lo;
+          dst[16 + i] = hi;
+        }
       }
       if (!t.is_q && slot[b] >= 0 && slot[b] < a.num_slots) {
         const int kvh = t.head - a.num_heads - (t.is_k ? 0 : a.num_kv_heads);
         uint2* row = reinterpret_cast<uint2*>((t.is_k ? a.k_cache : a.v_cache) +
                                               ((int64_t)slot[b] * a.num_kv_heads + kvh) * 128);
-        row[i] = lo;
-        row[16 + i] = hi;
+        store_past_l2(row + i, lo);
+        store_past_l2(row + 16 + i, hi);
       }
     }
   }
@@ -315,9 +327,12 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
     const int n_out = EPI == kSiluMul ? a.N / 2 : a.N;
     for (int p = threadIdx.x; p < BM * kPieces; p += 256) {
       const int m = p / kPieces, piece = p % kPieces, n = n_tile * kOut + 8 * piece;
-      if (m0 + m < a.M && n < n_out)
-        *reinterpret_cast<uint4*>(a.out + (int64_t)(m0 + m) * n_out + n) =
-            *reinterpret_cast<const uint4*>(lds + m * kOutStride + 16 * piece);
+      if (m0 + m < a.M && n < n_out) {
+        uint4* to = reinterpret_cast<uint4*>(a.out + (int64_t)(m0 + m) * n_out + n);
+        const uint4 v = *reinterpret_cast<const uint4*>(lds + m * kOutStride + 16 * piece);
+        if constexpr (EPI == kPlain) store_past_l2(to, v);
+        else *to = v;
+      }
     }
   }
 }

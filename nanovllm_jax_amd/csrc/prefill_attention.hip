@@ -43,6 +43,7 @@
 #include "launch.h"
 #include "lds_copy.h"
 #include "nvj_paged_attn.h"
+#include "past_l2.h"
 #include "wave_ops.h"
 
 namespace {
@@ -50,6 +51,7 @@ namespace {
 using nvj::bf16x8;
 using nvj::f16x8;
 using nvj::f32x4;
+using nvj::store_past_l2;
 using nvj::wave_inclusive_scan;   // (with shuffles the sequence lookup took 5 us of a short prompt)
 using nvj::wave_max;
 
@@ -391,12 +393,6 @@ struct PrefillArgs {
   int64_t num_slots;
   uint32_t row_pieces, new_pieces;   // of a row, of all rows
 };
-
-__device__ __forceinline__ void store_past_l2(uint4* to, const uint4& v) {
-  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-  const u32x4 t = {v.x, v.y, v.z, v.w};
-  __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(to));
-}
 
 // A workgroup's share of the new rows on their way into the caches.  The attention reads the
 // packed rows and never the caches, so the store needs no place in front of it: a workgroup
