@@ -49,6 +49,7 @@
 #include "launch.h"
 #include "linear.h"
 #include "nvj_paged_attn.h"
+#include "read_ahead.h"
 
 namespace {
 
@@ -472,7 +473,8 @@ bool takes_rows(const nvj_decoder_model& m, int64_t tokens, int64_t sequences) {
 
 int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer& l,
               const nvj_decoder_batch& b, bool first_layer, const void* q,
-              const void* k, const void* v, int64_t kv_stride, void* out) {
+              const void* k, const void* v, int64_t kv_stride, void* out,
+              const nvj::ReadAhead* ahead = nullptr) {
   if (b.is_prefill && !b.block_tables)
     return nvj_prefill_attention_rows_launch(stream, q, (int64_t)m.num_heads * m.head_dim, k, v, kv_stride, b.cu_seqlens_q,
                                              b.cu_seqlens_k, out, b.num_tokens, b.num_sequences,
@@ -485,11 +487,11 @@ int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer&
         b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16);
   const uint32_t phases = NVJ_PHASE_SPLITK | NVJ_PHASE_COMBINE;
   if (b.chunk == 0)
-    return nvj_paged_decode_launch_counters(
+    return nvj::paged_decode_launch_ahead(
         stream, q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, out, b.partials,
         b.partial_bytes, b.counters, b.counter_bytes, b.num_sequences, m.num_heads, m.num_kv_heads,
         m.head_dim, m.block_size, b.max_blocks, m.num_blocks, m.scale, NVJ_DTYPE_BF16,
-        phases | (b.clear_counters && first_layer ? NVJ_PHASE_CLEAR_COUNTERS : 0));
+        phases | (b.clear_counters && first_layer ? NVJ_PHASE_CLEAR_COUNTERS : 0), ahead);
   return nvj_paged_decode_launch_phases(
       stream, q, l.k_cache, l.v_cache, b.block_tables, b.context_lens, out, b.partials,
       b.partial_bytes, b.num_sequences, m.num_heads, m.num_kv_heads, m.head_dim, m.block_size,
@@ -513,6 +515,16 @@ int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder
   const bool packed = b.is_prefill && !b.block_tables;
   char* k_rows = packed ? ws + at.k_rows : nullptr;
   char* v_rows = packed ? k_rows + round256((size_t)tokens * kv_width * 2) : nullptr;
+  // The attention reads weights ahead (read_ahead.h), in the order in which they are needed, as
+  // many as HBM moves beside the K and V that the table holds in the 10 us that the launch
+  // takes of its own.  A chunk is what one workgroup of the product takes, so that it goes to
+  // the L2 of the XCD that asks for it (16 rows of the gate/up matrix instead of 8 and 8: 1058
+  // us instead of 1036).  us a step without / with: 4 rows of 100 .. 900 positions 1080 / 1036,
+  // 1 of 500 1023 / 982, 16 of 100 .. 400 (output and gate/up) 1250 / 1221; with all four
+  // behind 8 rows of 1000 .. 2500 it would be 1349 / 1440.
+  const int64_t ahead_bytes =
+      b.is_prefill ? 0
+                   : (50 << 20) - (int64_t)tokens * b.max_blocks * m.block_size * kv_width * 4;
   for (int i = 0; i < m.num_layers; ++i) {
     const nvj_decoder_layer& l = layers[i];
     a.weight = static_cast<const char*>(l.qkv);
@@ -525,8 +537,23 @@ int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder
         m.eps, b.slot_mapping, l.k_cache, l.v_cache, ws + at.q, q_width, k_rows, v_rows, kv_width,
         tokens, m.num_heads, m.num_kv_heads, m.head_dim, (int64_t)m.num_blocks * m.block_size);
     if (code != NVJ_OK) return code;
+    nvj::ReadAhead ahead = {};
+    int64_t left = ahead_bytes;
+    const auto fits = [&](int64_t rows, int64_t columns) {
+      return (left -= rows * columns * 2) >= 0;
+    };
+    const char* gate_up = static_cast<const char*>(l.gate_up);
+    if (fits(m.hidden, q_width)) ahead.add_matrix(l.o, m.hidden, q_width, 8);
+    if (fits(2 * (int64_t)m.intermediate, m.hidden)) {
+      ahead.add_matrix(gate_up, m.intermediate, m.hidden, 8);
+      ahead.add_matrix(gate_up + (int64_t)m.intermediate * m.hidden * 2, m.intermediate, m.hidden,
+                       8);
+    }
+    if (fits(m.hidden, m.intermediate)) ahead.add_matrix(l.down, m.hidden, m.intermediate, 8);
+    if (i + 1 < m.num_layers && fits(q_width + 2 * kv_width, m.hidden))
+      ahead.add_matrix(layers[i + 1].qkv, q_width + 2 * kv_width, m.hidden, 16);
     code = attention(stream, m, l, b, i == 0, ws + at.q, k_rows, v_rows, kv_width,
-                     ws + at.o);
+                     ws + at.o, &ahead);
     if (code != NVJ_OK) return code;
     if (launch_residual_gemm<4, 1, 2>(s, ws + at.o, l.o, h, tokens, m.hidden, q_width) !=
         hipSuccess)
@@ -560,6 +587,23 @@ hipError_t down_projection(hipStream_t s, const nvj::LinearArgs& a) {
   if (a.M <= 128 && a.K % 256 == 0)
     return a.M > 64 || a.M == 32 ? nvj::linear_chained(s, a, 4, 2) : nvj::linear_chained(s, a, 2, 4);
   return nvj::linear(s, a);
+}
+
+// Up to this many rows every product is one round of small workgroups.
+constexpr int kStepRowsOfOneRound = 128;
+
+// Weights are read ahead (read_ahead.h) by the gate/up product, which is long and is where the
+// next layer's first products follow, and with more rows by the output projection too, whose
+// workgroups leave CUs free; with few rows it is over before they arrive.  us a step without /
+// with: decode of 128 x 1024 positions 3475 / 3380, 64 x 500 1880 / 1770, 24 x 100 .. 1000
+// 1678 / 1570; prefill of 200 tokens 1828 / 1645, 4268 6110 / 5800.  A launch is given what
+// makes up 128 MB with its own weights.  Beyond that it waits for HBM itself, whatever the order
+// of the reads, without / with, 6 layers: 2048 (6144) with 50 + 50 MB, 64 rows 542 / 520; 2560
+// (9728), 4 rows, with 100 + 31 MB 581 / 566 and with 100 + 81 581 / 618; 4096 (12288), 4 rows,
+// with 201 + 50 MB 823 / 855.
+void read_ahead(nvj::LinearArgs& a, const void* w, int64_t rows, int64_t columns, int chunk) {
+  if ((int64_t)a.N * a.K * 2 + a.ahead.total() + rows * columns * 2 <= (128 << 20))
+    a.ahead.add_matrix(w, rows, columns, chunk);
 }
 
 int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
@@ -609,11 +653,22 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
                      qkv + 2 * (int64_t)(q_width + kv_width), qkv_width, o);
     if (code != NVJ_OK) return code;
     product(o, l.o, t, m.hidden, q_width);
+    if (tokens > kStepRowsOfOneRound) {
+      read_ahead(a, l.gate_up, 2 * (int64_t)m.intermediate, m.hidden, 16);
+      read_ahead(a, l.down, m.hidden, m.intermediate, 8);
+    }
     if (output_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    a.ahead = {};
     code = nvj_add_rms_norm_launch(stream, t, h, l.ln2, m.eps, y, h, tokens, m.hidden);
     if (code != NVJ_OK) return code;
     product(y, l.gate_up, act, 2 * m.intermediate, m.hidden);
+    if (i + 1 < m.num_layers) {
+      read_ahead(a, layers[i + 1].qkv, qkv_width, m.hidden, 8);
+      read_ahead(a, layers[i + 1].o, m.hidden, q_width, 8);
+    }
+    if (tokens <= kStepRowsOfOneRound) read_ahead(a, l.down, m.hidden, m.intermediate, 8);
     if (nvj::linear_silu_mul(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
+    a.ahead = {};
     product(act, l.down, t, m.hidden, m.intermediate);
     if (down_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
     const float* next = i + 1 < m.num_layers ? layers[i + 1].ln1 : m.final_norm;

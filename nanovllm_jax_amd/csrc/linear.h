@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "read_ahead.h"
+
 namespace nvj {
 
 struct LinearArgs {
@@ -25,6 +27,7 @@ struct LinearArgs {
   float eps;
   int max_position, num_heads, num_kv_heads;
   int64_t num_slots;
+  ReadAhead ahead;                 // by workgroups of its own behind the product's
   int m_tiles, n_tiles, group_m;   // filled in by the launch
   int tile;                        // 1 + index of the tile shape, 0: by the sizes
 };

@@ -164,6 +164,10 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   // walks a contiguous part of the list, so a weight tile is fetched by one L2
   const int total = a.m_tiles * a.n_tiles;
   const int part = (total + 7) / 8;
+  if ((int)blockIdx.x >= 8 * part) {
+    nvj::read_chunk<256>(a.ahead, (int)blockIdx.x - 8 * part);
+    return;
+  }
   const int tile = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
   if (tile >= total) return;
   const int per_group = a.group_m * a.n_tiles;
@@ -362,6 +366,11 @@ __global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
   const int chain = wave % CHAINS, half = wave / CHAINS;
+  if ((int)blockIdx.y * BM >= a.M) {
+    const int row = (int)blockIdx.y - (a.M + BM - 1) / BM;
+    nvj::read_chunk<256>(a.ahead, row * (int)gridDim.x + (int)blockIdx.x);
+    return;
+  }
   const int n_tile = blockIdx.x, m0 = blockIdx.y * BM;
   const int row_bytes = a.K * 2;
   const int rounds = a.K / (32 * CHAINS * RUN);
@@ -441,7 +450,9 @@ __global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
 
 template <int BM, int BN, int CHAINS, int RUN, int ST>
 hipError_t launch_chained(hipStream_t s, const LinearArgs& a) {
-  const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM));
+  const unsigned columns = (unsigned)((a.N + BN - 1) / BN);
+  const dim3 grid(columns, (unsigned)((a.M + BM - 1) / BM) +
+                               (a.ahead.chunks() + columns - 1) / columns);
   return nvj::launch(chained_linear_kernel<BM, BN, CHAINS, RUN, ST>, grid, dim3(256), s, a);
 }
 
@@ -452,8 +463,8 @@ hipError_t launch_tiles(hipStream_t s, LinearArgs a) {
   a.m_tiles = (a.M + BM - 1) / BM;
   a.n_tiles = (outs + kOut - 1) / kOut;
   const int total = a.m_tiles * a.n_tiles;
-  return nvj::launch(linear_kernel<BM, BN, ST, EPI>, dim3((unsigned)((total + 7) / 8 * 8)),
-                     dim3(256), s, a);
+  const dim3 grid((unsigned)((total + 7) / 8 * 8) + a.ahead.chunks());
+  return nvj::launch(linear_kernel<BM, BN, ST, EPI>, grid, dim3(256), s, a);
 }
 
 // Tile sizes.  A launch of T tiles takes rounds of one workgroup per CU (or two, where they

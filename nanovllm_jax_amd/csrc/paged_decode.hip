@@ -45,6 +45,7 @@
 #include "device.h"
 #include "launch.h"
 #include "nvj_paged_attn.h"
+#include "read_ahead.h"
 #include "wave_ops.h"
 
 namespace {
@@ -1732,10 +1733,15 @@ struct SharedRows {
 template <bool F16, int HPW>
 __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, int batch,
                                                                   int num_wgs, int min_steps,
-                                                                  int shift, int32_t* counters) {
+                                                                  int shift, int32_t* counters,
+                                                                  nvj::ReadAhead ahead) {
   using R = SharedRows<F16, HPW>;
   constexpr int D = R::D, NW = R::NW, kParts = R::kParts;
   using H = HeadDim<D>;
+  if ((int)blockIdx.x >= num_wgs) {
+    nvj::read_chunk<512>(ahead, (int)blockIdx.x - num_wgs);
+    return;
+  }
   __shared__ uint4 k_tile[NW][R::kTile];
   __shared__ int last[HPW];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2781,7 +2787,8 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
                   void* workspace, size_t workspace_bytes, int32_t* ext_counters, int32_t batch,
                   int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
                   int32_t max_blocks, int32_t num_blocks, float scale, int32_t chunk,
-                  int32_t dtype, uint32_t phases, const NewRows* new_rows = nullptr) {
+                  int32_t dtype, uint32_t phases, const NewRows* new_rows = nullptr,
+                  const nvj::ReadAhead* ahead = nullptr) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   const bool f16 = dtype == NVJ_DTYPE_F16;
   const bool whole = chunk == NVJ_CHUNK_WHOLE_SEQUENCE;
@@ -2913,14 +2920,14 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
       if (!new_rows && short_rows == 0 && head_dim == 128 && !valu && !loads_only && batch <= 64 &&
           (plan.wr_hpw == 0 || (phases & NVJ_PHASE_SHARED_ROWS))) {
         // nothing but the equal cut on offer
+        const nvj::ReadAhead more = ahead ? *ahead : nvj::ReadAhead{};
+        const dim3 shared_grid((unsigned)plan.num_wgs + more.chunks());
         hipError_t rc;
 #define NVJ_LAUNCH_SHARED(N)                                                                   \
-  rc = f16 ? nvj::launch(paged_decode_shared_kernel<true, N>, dim3((unsigned)plan.num_wgs),    \
-                         dim3(512), s, a, batch, plan.num_wgs, kMinBalancedSteps, plan.shift,  \
-                         counters)                                                             \
-           : nvj::launch(paged_decode_shared_kernel<false, N>, dim3((unsigned)plan.num_wgs),   \
-                         dim3(512), s, a, batch, plan.num_wgs, kMinBalancedSteps, plan.shift,  \
-                         counters)
+  rc = f16 ? nvj::launch(paged_decode_shared_kernel<true, N>, shared_grid, dim3(512), s, a,     \
+                         batch, plan.num_wgs, kMinBalancedSteps, plan.shift, counters, more)   \
+           : nvj::launch(paged_decode_shared_kernel<false, N>, shared_grid, dim3(512), s, a,    \
+                         batch, plan.num_wgs, kMinBalancedSteps, plan.shift, counters, more)
         if (plan.hpw == 1) NVJ_LAUNCH_SHARED(1);
         else if (plan.hpw == 2) NVJ_LAUNCH_SHARED(2);
         else NVJ_LAUNCH_SHARED(4);
@@ -3120,7 +3127,7 @@ extern "C" int nvj_paged_decode_null_stream_counters(void** counters, size_t* by
   return NVJ_OK;
 }
 
-extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, const void* k_cache,
+int nvj::paged_decode_launch_ahead(void* stream, const void* q, const void* k_cache,
                                                 const void* v_cache, const int32_t* block_tables,
                                                 const int32_t* context_lens, void* out,
                                                 void* partials, size_t partial_bytes,
@@ -3129,7 +3136,7 @@ extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, con
                                                 int32_t num_kv_heads, int32_t head_dim,
                                                 int32_t block_size, int32_t max_blocks,
                                                 int32_t num_blocks, float scale, int32_t dtype,
-                                                uint32_t phases) {
+                                                uint32_t phases, const ReadAhead* ahead) {
   if (batch > 0 && max_blocks > 0) {
     const size_t need = nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads);
     if (!counters) {
@@ -3147,7 +3154,23 @@ extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, con
   return launch_decode(stream, q, k_cache, v_cache, block_tables, context_lens, out, partials,
                        partial_bytes, static_cast<int32_t*>(counters), batch, num_heads,
                        num_kv_heads, head_dim, block_size, max_blocks, num_blocks, scale, 0, dtype,
-                       phases);
+                       phases, nullptr, ahead);
+}
+
+extern "C" int nvj_paged_decode_launch_counters(void* stream, const void* q, const void* k_cache,
+                                                const void* v_cache, const int32_t* block_tables,
+                                                const int32_t* context_lens, void* out,
+                                                void* partials, size_t partial_bytes,
+                                                void* counters, size_t counter_bytes,
+                                                int32_t batch, int32_t num_heads,
+                                                int32_t num_kv_heads, int32_t head_dim,
+                                                int32_t block_size, int32_t max_blocks,
+                                                int32_t num_blocks, float scale, int32_t dtype,
+                                                uint32_t phases) {
+  return nvj::paged_decode_launch_ahead(stream, q, k_cache, v_cache, block_tables, context_lens,
+                                        out, partials, partial_bytes, counters, counter_bytes,
+                                        batch, num_heads, num_kv_heads, head_dim, block_size,
+                                        max_blocks, num_blocks, scale, dtype, phases, nullptr);
 }
 
 // Up to one (sequence, KV head) per CU.  With more, the comparison in every step costs the

@@ -1,0 +1,79 @@
+// Memory that a launch reads on behalf of the launches behind it.
+//
+// The products of a decoder layer wait for their weights: a layer's 31 MB (hidden 1024) come
+// from HBM on every step, and a launch asks for them only when it starts.  Workgroups
+// behind a launch's own read the weights of the next products meanwhile, into the Infinity
+// Cache and the L2s, while HBM has nothing else to do.  Nothing depends on it: what has not
+// arrived, or has been displaced, is fetched as before.
+#ifndef NVJ_READ_AHEAD_H_
+#define NVJ_READ_AHEAD_H_
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+namespace nvj {
+
+// Up to kRegions regions of count[i] chunks of bytes[i] bytes each (a multiple of 16), a
+// workgroup per chunk.
+struct ReadAhead {
+  static constexpr int kRegions = 5;
+  const char* base[kRegions];
+  int bytes[kRegions], count[kRegions];
+  int used;
+
+  int64_t total() const {
+    int64_t n = 0;
+    for (int i = 0; i < used; ++i) n += (int64_t)bytes[i] * count[i];
+    return n;
+  }
+  unsigned chunks() const {
+    unsigned n = 0;
+    for (int i = 0; i < used; ++i) n += (unsigned)count[i];
+    return n;
+  }
+  // The rows of a bf16 matrix, `rows_per_chunk` to a chunk; nothing where they do not divide.
+  void add_matrix(const void* w, int64_t rows, int64_t columns, int rows_per_chunk) {
+    if (used == kRegions || rows % rows_per_chunk != 0 || columns % 8 != 0) return;
+    base[used] = static_cast<const char*>(w);
+    bytes[used] = (int)(columns * 2 * rows_per_chunk);
+    count[used++] = (int)(rows / rows_per_chunk);
+  }
+};
+
+// One chunk, by a workgroup of THREADS; `chunk` counts through the regions.
+template <int THREADS>
+__device__ __forceinline__ void read_chunk(const ReadAhead& ahead, int chunk) {
+#pragma unroll
+  for (int i = 0; i < ReadAhead::kRegions; ++i) {
+    if (chunk >= 0 && chunk < ahead.count[i]) {
+      const char* from = ahead.base[i] + (int64_t)chunk * ahead.bytes[i];
+      for (int at = 16 * threadIdx.x; at < ahead.bytes[i]; at += 4 * 16 * THREADS) {
+        uint4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[u] = *reinterpret_cast<const uint4*>(from +
+                                                 min(at + u * 16 * THREADS, ahead.bytes[i] - 16));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)   // (the values are needed by nobody, the reads are)
+          asm volatile("" ::"v"(v[u].x), "v"(v[u].y), "v"(v[u].z), "v"(v[u].w));
+      }
+    }
+    chunk -= ahead.count[i];
+  }
+}
+
+// nvj_paged_decode_launch_counters; where the launch takes the kernel for few sequences, with
+// memory to read by workgroups behind its own.
+int paged_decode_launch_ahead(void* stream, const void* q, const void* k_cache,
+                              const void* v_cache, const int32_t* block_tables,
+                              const int32_t* context_lens, void* out, void* partials,
+                              size_t partial_bytes, void* counters, size_t counter_bytes,
+                              int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+                              int32_t head_dim, int32_t block_size, int32_t max_blocks,
+                              int32_t num_blocks, float scale, int32_t dtype, uint32_t phases,
+                              const ReadAhead* ahead);
+
+}  // namespace nvj
+
+#endif  // NVJ_READ_AHEAD_H_

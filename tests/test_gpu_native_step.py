@@ -419,3 +419,35 @@ def test_contexts_can_be_copied_and_pickled():
     for other in (copy.copy(ctx), copy.deepcopy(ctx), dataclasses.replace(ctx),
                   type(ctx)(**dataclasses.asdict(ctx)), pickle.loads(pickle.dumps(ctx))):
         assert torch.equal(runner.forward(ids, pos, other), want)
+
+
+@pytest.mark.parametrize("rows,hidden,inter,heads,wide_mb", [
+    (1, 256, 256, 2, 0), (3, 1024, 3072, 16, 0), (3, 1024, 3072, 16, 25), (16, 1024, 3072, 16, 40),
+    (16, 2048, 6144, 16, 0), (16, 2048, 6144, 16, 51), (17, 320, 448, 6, 0),
+    (40, 2048, 2560, 24, 0), (20, 2560, 9728, 16, 0), (129, 320, 448, 6, 0),
+    (200, 1024, 3072, 16, 0)])
+@pytest.mark.parametrize("layers", [1, 3])
+def test_weights_read_ahead(rows, hidden, inter, heads, wide_mb, layers, monkeypatch):
+    """Which weights a launch reads ahead depends on the layer, the row count, the widths and,
+    up to 16 rows, on the K and V that the block table holds: every set of them against the
+    library's products, to what two orders of bf16 roundings give (as above)."""
+    print(f"case read ahead rows={rows} hidden={hidden} layers={layers} {wide_mb}", flush=True)
+    from nanovllm_jax_amd.engine import decode_step as ds
+    cfg = ds.DecodeModelConfig(num_layers=layers, hidden_size=hidden, num_heads=heads,
+                               num_kv_heads=2, head_dim=128, intermediate_size=inter,
+                               vocab_size=1000, max_position=64, block_size=64,
+                               num_kvcache_blocks=rows)
+    runner = ds.DecodeStepRunner(cfg, "cuda:0", seed=rows)
+    inputs = runner.make_inputs([7 * i % 1000 for i in range(rows)],
+                                [1 + 5 * i % 64 for i in range(rows)], [[i] for i in range(rows)])
+    # 1 KB of K and V a position
+    inputs[2].block_tables = torch.nn.functional.pad(
+        inputs[2].block_tables, (0, (wide_mb << 20) // (rows * 64 * 1024)), value=-1).contiguous()
+    runner.kv_cache.normal_()
+    before = runner.kv_cache.clone()
+    got = runner._native_forward(*inputs).float()
+    runner.kv_cache.copy_(before)
+    monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
+    want = runner.forward(*inputs).float()
+    torch.cuda.synchronize()
+    assert (got - want).abs().max().item() <= 0.02 * want.abs().max().item() + 0.02
