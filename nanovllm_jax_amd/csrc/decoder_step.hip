@@ -589,21 +589,32 @@ hipError_t down_projection(hipStream_t s, const nvj::LinearArgs& a) {
   return nvj::linear(s, a);
 }
 
-// Up to this many rows every product is one round of small workgroups.
-constexpr int kStepRowsOfOneRound = 128;
+// Weights are read ahead (read_ahead.h) by the norms, whose few workgroups leave HBM idle, and by
+// the gate/up product, which is long and has the next layer's first products behind it.  The
+// norm in front of the MLP takes the down projection, so that the gate/up product carries less;
+// up to kReadRows rows it takes the gate/up matrix instead, which that product is still waiting
+// for then, and the norm behind the MLP the next layer's first two.  us a step without / by the
+// gate/up product alone / like this, up to kReadRows first: 17 rows of 50 .. 200 positions 1433 /
+// 1354 / 1335, 24 of 100 .. 1000 1680 / 1570 / 1552, 64 of 500 1880 / 1774 / 1739; like this,
+// and as with fewer rows: 80 of 200 .. 400 1893 / 1850 / 1830, 1847, 100 of 200 .. 400 1911 / 1895 /
+// 1880, 1890, 128 of 1024 3475 / 3400 / 3378, 3375; a prompt of 200 tokens 1830 / 1648 / 1636, 1666
+// (the middle one with the output projection's help), of 4268 6110 / 5837 / 5815, 5865.
+constexpr int kReadRows = 64;
 
-// Weights are read ahead (read_ahead.h) by the gate/up product, which is long and is where the
-// next layer's first products follow, and with more rows by the output projection too, whose
-// workgroups leave CUs free; with few rows it is over before they arrive.  us a step without /
-// with: decode of 128 x 1024 positions 3475 / 3380, 64 x 500 1880 / 1770, 24 x 100 .. 1000
-// 1678 / 1570; prefill of 200 tokens 1828 / 1645, 4268 6110 / 5800.  A launch is given what
-// makes up 128 MB with its own weights.  Beyond that it waits for HBM itself, whatever the order
-// of the reads, without / with, 6 layers: 2048 (6144) with 50 + 50 MB, 64 rows 542 / 520; 2560
-// (9728), 4 rows, with 100 + 31 MB 581 / 566 and with 100 + 81 581 / 618; 4096 (12288), 4 rows,
-// with 201 + 50 MB 823 / 855.
-void read_ahead(nvj::LinearArgs& a, const void* w, int64_t rows, int64_t columns, int chunk) {
-  if ((int64_t)a.N * a.K * 2 + a.ahead.total() + rows * columns * 2 <= (128 << 20))
-    a.ahead.add_matrix(w, rows, columns, chunk);
+// A norm is over in 5 us, and waits for what it reads ahead.
+constexpr int64_t kNormReads = 20 << 20;
+
+// A gate/up product is given what makes up 128 MB with its own weights.  Beyond that it waits
+// for HBM itself, whatever the order of the reads; us of 6 layers without / with: 2048 (6144)
+// with 50 + 50 MB, 64 rows 542 / 520; 2560 (9728), 4 rows, with 100 + 31 MB 581 / 566 and with
+// 100 + 81 581 / 618; 4096 (12288), 4 rows, with 201 + 50 MB 823 / 855.
+constexpr int64_t kProductReads = 128 << 20;
+
+bool read_ahead(nvj::ReadAhead& ahead, int64_t limit, const void* w, int64_t rows, int64_t columns,
+                int chunk = 8) {
+  if (ahead.total() + rows * columns * 2 > limit) return false;
+  ahead.add_matrix(w, rows, columns, chunk);
+  return true;
 }
 
 int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
@@ -653,26 +664,31 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
                      qkv + 2 * (int64_t)(q_width + kv_width), qkv_width, o);
     if (code != NVJ_OK) return code;
     product(o, l.o, t, m.hidden, q_width);
-    if (tokens > kStepRowsOfOneRound) {
-      read_ahead(a, l.gate_up, 2 * (int64_t)m.intermediate, m.hidden, 16);
-      read_ahead(a, l.down, m.hidden, m.intermediate, 8);
-    }
     if (output_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
-    a.ahead = {};
-    code = nvj_add_rms_norm_launch(stream, t, h, l.ln2, m.eps, y, h, tokens, m.hidden);
+    const int64_t gate_up = 2 * (int64_t)m.intermediate;
+    const int64_t left = kProductReads - gate_up * m.hidden * 2;
+    const bool few = tokens <= kReadRows;
+    nvj::ReadAhead by_norm2 = {}, by_norm1 = {}, by_product = {};
+    if (few) read_ahead(by_norm2, kNormReads, l.gate_up, gate_up, m.hidden, 16);
+    if (i + 1 < m.num_layers) {
+      const nvj_decoder_layer& next = layers[i + 1];
+      if (!few || !read_ahead(by_norm1, kNormReads, next.qkv, qkv_width, m.hidden))
+        read_ahead(by_product, left, next.qkv, qkv_width, m.hidden);
+      if (!few || !read_ahead(by_norm1, kNormReads, next.o, m.hidden, q_width))
+        read_ahead(by_product, left, next.o, m.hidden, q_width);
+    }
+    if (few || !read_ahead(by_norm2, kNormReads, l.down, m.hidden, m.intermediate))
+      read_ahead(by_product, left, l.down, m.hidden, m.intermediate);
+    code = nvj::add_rms_norm(stream, t, h, l.ln2, m.eps, y, h, tokens, m.hidden, by_norm2);
     if (code != NVJ_OK) return code;
     product(y, l.gate_up, act, 2 * m.intermediate, m.hidden);
-    if (i + 1 < m.num_layers) {
-      read_ahead(a, layers[i + 1].qkv, qkv_width, m.hidden, 8);
-      read_ahead(a, layers[i + 1].o, m.hidden, q_width, 8);
-    }
-    if (tokens <= kStepRowsOfOneRound) read_ahead(a, l.down, m.hidden, m.intermediate, 8);
+    a.ahead = by_product;
     if (nvj::linear_silu_mul(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
     a.ahead = {};
     product(act, l.down, t, m.hidden, m.intermediate);
     if (down_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
     const float* next = i + 1 < m.num_layers ? layers[i + 1].ln1 : m.final_norm;
-    code = nvj_add_rms_norm_launch(stream, t, h, next, m.eps, y, h, tokens, m.hidden);
+    code = nvj::add_rms_norm(stream, t, h, next, m.eps, y, h, tokens, m.hidden, by_norm1);
     if (code != NVJ_OK) return code;
   }
   if (!b.logits || b.num_sequences == 0) return NVJ_OK;

@@ -23,6 +23,7 @@
 #include "launch.h"
 #include "nvj_paged_attn.h"
 #include "past_l2.h"
+#include "read_ahead.h"
 
 namespace {
 
@@ -47,14 +48,20 @@ __device__ __forceinline__ void unpack8(const uint4& p, float (&f)[8]) {
   f[6] = bf16_lo(p.w); f[7] = bf16_hi(p.w);
 }
 
-// grid.x = ceil(num_tokens / 4), block = 256 (4 waves, one token row each).
+// grid.x = ceil(num_tokens / 4) and the workgroups that read ahead, block = 256 (4 waves, one
+// token row each).
 // PIECES = 16-byte pieces per lane, a compile-time bound so the row stays in
 // registers between the two passes.
 template <int PIECES, bool RESIDUAL>
 __global__ __launch_bounds__(256) void add_rms_norm_kernel(
     const uint4* __restrict__ x, const uint4* residual, const float* __restrict__ weight,
-    float eps, uint4* __restrict__ y, uint4* residual_out, int num_tokens, int row_pieces) {
+    float eps, uint4* __restrict__ y, uint4* residual_out, int num_tokens, int row_pieces,
+    nvj::ReadAhead ahead) {
 #pragma clang fp contract(off)
+  if ((int)blockIdx.x * 4 >= num_tokens) {
+    nvj::read_chunk<256>(ahead, (int)blockIdx.x - (num_tokens + 3) / 4);
+    return;
+  }
   const int token = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (token >= num_tokens) return;
   const int lane = threadIdx.x & 63;
@@ -157,20 +164,20 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(const uint4* __restri
 template <int PIECES>
 hipError_t launch_add_rms_norm(hipStream_t stream, const uint4* x, const uint4* residual,
                          const float* weight, float eps, uint4* y, uint4* residual_out,
-                         int num_tokens, int row_pieces) {
-  const dim3 grid((unsigned)((num_tokens + 3) / 4)), block(256);
+                         int num_tokens, int row_pieces, const nvj::ReadAhead& ahead) {
+  const dim3 grid((unsigned)((num_tokens + 3) / 4) + ahead.chunks()), block(256);
   if (residual != nullptr)
     return nvj::launch(add_rms_norm_kernel<PIECES, true>, grid, block, stream, x, residual, weight,
-                       eps, y, residual_out, num_tokens, row_pieces);
+                       eps, y, residual_out, num_tokens, row_pieces, ahead);
   return nvj::launch(add_rms_norm_kernel<PIECES, false>, grid, block, stream, x, nullptr, weight,
-                     eps, y, nullptr, num_tokens, row_pieces);
+                     eps, y, nullptr, num_tokens, row_pieces, ahead);
 }
 
 }  // namespace
 
-extern "C" int nvj_add_rms_norm_launch(void* stream, const void* x, const void* residual,
-                                       const float* weight, float eps, void* y,
-                                       void* residual_out, int32_t num_tokens, int32_t hidden) {
+int nvj::add_rms_norm(void* stream, const void* x, const void* residual, const float* weight,
+                      float eps, void* y, void* residual_out, int32_t num_tokens, int32_t hidden,
+                      const ReadAhead& ahead) {
   if (num_tokens < 0 || hidden <= 0) return NVJ_ERR_BAD_SHAPE;
   if (hidden % 8 != 0 || hidden > 64 * 8 * kMaxPiecesPerLane) return NVJ_ERR_UNSUPPORTED;
   if (num_tokens == 0) return NVJ_OK;
@@ -188,12 +195,22 @@ extern "C" int nvj_add_rms_norm_launch(void* stream, const void* x, const void* 
   const auto yp = static_cast<uint4*>(y);
   const auto op = static_cast<uint4*>(residual_out);
   hipError_t rc;
-  if (per_lane <= 1) rc = launch_add_rms_norm<1>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces);
-  else if (per_lane <= 2) rc = launch_add_rms_norm<2>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces);
-  else if (per_lane <= 4) rc = launch_add_rms_norm<4>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces);
-  else if (per_lane <= 8) rc = launch_add_rms_norm<8>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces);
-  else rc = launch_add_rms_norm<16>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces);
+#define NVJ_LAUNCH(N) \
+  launch_add_rms_norm<N>(s, xp, rp, weight, eps, yp, op, num_tokens, row_pieces, ahead)
+  if (per_lane <= 1) rc = NVJ_LAUNCH(1);
+  else if (per_lane <= 2) rc = NVJ_LAUNCH(2);
+  else if (per_lane <= 4) rc = NVJ_LAUNCH(4);
+  else if (per_lane <= 8) rc = NVJ_LAUNCH(8);
+  else rc = NVJ_LAUNCH(16);
+#undef NVJ_LAUNCH
   return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+}
+
+extern "C" int nvj_add_rms_norm_launch(void* stream, const void* x, const void* residual,
+                                       const float* weight, float eps, void* y,
+                                       void* residual_out, int32_t num_tokens, int32_t hidden) {
+  return nvj::add_rms_norm(stream, x, residual, weight, eps, y, residual_out, num_tokens, hidden,
+                           nvj::ReadAhead{});
 }
 
 extern "C" int nvj_silu_and_mul_launch(void* stream, const void* x, int64_t x_row_stride, void* y,

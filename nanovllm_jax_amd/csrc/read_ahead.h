@@ -74,6 +74,11 @@ int paged_decode_launch_ahead(void* stream, const void* q, const void* k_cache,
                               int32_t num_blocks, float scale, int32_t dtype, uint32_t phases,
                               const ReadAhead* ahead);
 
+// nvj_add_rms_norm_launch, with memory to read by workgroups behind its own.
+int add_rms_norm(void* stream, const void* x, const void* residual, const float* weight, float eps,
+                 void* y, void* residual_out, int32_t num_tokens, int32_t hidden,
+                 const ReadAhead& ahead);
+
 }  // namespace nvj
 
 #endif  // NVJ_READ_AHEAD_H_
