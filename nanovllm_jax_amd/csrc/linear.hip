@@ -108,6 +108,41 @@ struct RopeUnits {
       s4[b] = nvj::load4<true>(cs + 64);
     }
   }
+  // The tile of 32 x 128: positions and slots through scalar loads of the four rows that a wave
+  // has in each unit.  In LDS, where the others have them, their 512 bytes beside its ring would
+  // leave one workgroup to a CU: a prompt of 400 tokens 1898 us instead of 1827.  (The tile of
+  // 64 x 128 has the room: 200 and 700 tokens 1535 and 2094 us, like this 1548 and 2115.)
+  struct Places {
+    int position[N], slot[N];
+    __device__ __forceinline__ Places(const LinearArgs& a, int m0, int wave) {
+      typedef const __attribute__((address_space(4))) int* const_int_ptr;
+      const const_int_ptr positions = (const_int_ptr)(uintptr_t)a.positions;
+      const const_int_ptr slots = (const_int_ptr)(uintptr_t)a.slot_mapping;
+      const int group = (threadIdx.x >> 4) & 3;
+#pragma unroll
+      for (int b = 0; b < N; ++b) {
+        position[b] = slot[b] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int token = min(m0 + 16 * b + 4 * wave + j, a.M - 1);
+          const int p = positions[token], s = slots[token];
+          position[b] = group == j ? p : position[b];
+          slot[b] = group == j ? s : slot[b];
+        }
+      }
+    }
+  };
+  __device__ __forceinline__ void fetch(const LinearArgs& a, const Places& places) {
+    const int i = threadIdx.x & 15;
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      slot[b] = places.slot[b];
+      const float* cs =
+          a.cos_sin + (int64_t)min(max(places.position[b], 0), a.max_position - 1) * 128 + 4 * i;
+      c4[b] = nvj::load4<true>(cs);
+      s4[b] = nvj::load4<true>(cs + 64);
+    }
+  }
   __device__ __forceinline__ void rows(const LinearArgs& a, const RopeHead<kHeads>& t,
                                        const char* lds, int stride, int m0, int u0) const {
     const int i = threadIdx.x & 15;
@@ -182,9 +217,10 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   constexpr int kBatch = kUnits % 5 == 0 ? 5 : kUnits % 4 == 0 ? 4 : 2;
   static_assert(EPI != kQkRope || kUnits % kBatch == 0, "whole batches");
   constexpr int kPlaces = (BM + 63) / 64 * 64;
-  __shared__ int places[EPI == kQkRope ? 2 * kPlaces : 1];
+  constexpr bool kFewUnits = EPI == kQkRope && kUnits == 2 && kHeads == 1;
+  __shared__ int places[EPI == kQkRope && !kFewUnits ? 2 * kPlaces : 1];
   RopeUnits<kBatch, kHeads> units;
-  if constexpr (EPI == kQkRope) {
+  if constexpr (EPI == kQkRope && !kFewUnits) {
     if (64 * wave < kPlaces) {
       const uint32_t at = (uint32_t)(uintptr_t)(lds_ptr)places + 256u * wave;
       const uint32_t from = 4u * (uint32_t)min(m0 + 64 * wave + lane, a.M - 1);
@@ -256,7 +292,10 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   wait_copies<(kStages - 1) * kCopies>();
   __syncthreads();
   // few units: the table rows too, under the whole reduction
-  if constexpr (EPI == kQkRope && kUnits == kBatch) units.fetch(a, places, kPlaces, 0);
+  if constexpr (kFewUnits)
+    units.fetch(a, typename RopeUnits<kBatch, kHeads>::Places(a, m0, wave));
+  else if constexpr (EPI == kQkRope && kUnits == kBatch)
+    units.fetch(a, places, kPlaces, 0);
 #pragma unroll
   for (int i = 0; i < kRead; ++i) read(0, 0, i);
   int stage = 0;
@@ -322,7 +361,8 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
     const RopeHead<kHeads> head(a, n_tile);
     for (int u0 = 0; u0 < kUnits; u0 += kBatch) {
       RopeUnits<kBatch, kHeads> next;
-      if (u0 + kBatch < kUnits) next.fetch(a, places, kPlaces, u0 + kBatch);
+      if constexpr (!kFewUnits)
+        if (u0 + kBatch < kUnits) next.fetch(a, places, kPlaces, u0 + kBatch);
       units.rows(a, head, lds, kOutStride, m0, u0);
       units = next;
     }
