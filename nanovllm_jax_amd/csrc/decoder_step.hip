@@ -498,6 +498,16 @@ int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer&
       b.max_blocks, m.num_blocks, m.scale, b.chunk, NVJ_DTYPE_BF16, phases);
 }
 
+// Whether the weights of a layer have left the Infinity Cache (256 MB) by the time the next step
+// comes to it; else there is nothing to read ahead.  us without / with: 12 layers of 1024 (3072),
+// 378 MB, 64 rows 763 / 698, a prompt of 400 tokens 887 / 827; 28 of 512 (1536), 245 MB, 1319 /
+// 1289; 6 of 1024, 189 MB, 337 / 342 and 392 / 392; 3 of 1024 178 / 182.
+bool weights_leave_the_cache(const nvj_decoder_model& m) {
+  const int64_t q = (int64_t)m.num_heads * m.head_dim, kv = (int64_t)m.num_kv_heads * m.head_dim;
+  const int64_t rows = 2 * (q + kv) + 3 * (int64_t)m.intermediate;   // of `hidden` elements
+  return rows * m.hidden * 2 * m.num_layers > (200 << 20);
+}
+
 int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
                      const nvj_decoder_batch& b, char* ws, const StepBuffers& at) {
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -523,7 +533,7 @@ int step_of_few_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder
   // 1 of 500 1023 / 982, 16 of 100 .. 400 (output and gate/up) 1250 / 1221; with all four
   // behind 8 rows of 1000 .. 2500 it would be 1349 / 1440.
   const int64_t ahead_bytes =
-      b.is_prefill ? 0
+      b.is_prefill || !weights_leave_the_cache(m) ? 0
                    : (50 << 20) - (int64_t)tokens * b.max_blocks * m.block_size * kv_width * 4;
   for (int i = 0; i < m.num_layers; ++i) {
     const nvj_decoder_layer& l = layers[i];
@@ -619,6 +629,7 @@ bool read_ahead(nvj::ReadAhead& ahead, int64_t limit, const void* w, int64_t row
 
 int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer* layers,
                       const nvj_decoder_batch& b, char* ws, const StepBuffers& at) {
+  const bool ahead = weights_leave_the_cache(m);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int tokens = b.num_tokens, pieces = m.hidden / 8;
   const int q_width = m.num_heads * m.head_dim, kv_width = m.num_kv_heads * m.head_dim;
@@ -666,18 +677,19 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
     product(o, l.o, t, m.hidden, q_width);
     if (output_projection(s, a) != hipSuccess) return NVJ_ERR_LAUNCH;
     const int64_t gate_up = 2 * (int64_t)m.intermediate;
-    const int64_t left = kProductReads - gate_up * m.hidden * 2;
+    const int64_t norm_reads = ahead ? kNormReads : 0;
+    const int64_t left = ahead ? kProductReads - gate_up * m.hidden * 2 : 0;
     const bool few = tokens <= kReadRows;
     nvj::ReadAhead by_norm2 = {}, by_norm1 = {}, by_product = {};
-    if (few) read_ahead(by_norm2, kNormReads, l.gate_up, gate_up, m.hidden, 16);
+    if (few) read_ahead(by_norm2, norm_reads, l.gate_up, gate_up, m.hidden, 16);
     if (i + 1 < m.num_layers) {
       const nvj_decoder_layer& next = layers[i + 1];
-      if (!few || !read_ahead(by_norm1, kNormReads, next.qkv, qkv_width, m.hidden))
+      if (!few || !read_ahead(by_norm1, norm_reads, next.qkv, qkv_width, m.hidden))
         read_ahead(by_product, left, next.qkv, qkv_width, m.hidden);
-      if (!few || !read_ahead(by_norm1, kNormReads, next.o, m.hidden, q_width))
+      if (!few || !read_ahead(by_norm1, norm_reads, next.o, m.hidden, q_width))
         read_ahead(by_product, left, next.o, m.hidden, q_width);
     }
-    if (few || !read_ahead(by_norm2, kNormReads, l.down, m.hidden, m.intermediate))
+    if (few || !read_ahead(by_norm2, norm_reads, l.down, m.hidden, m.intermediate))
       read_ahead(by_product, left, l.down, m.hidden, m.intermediate);
     code = nvj::add_rms_norm(stream, t, h, l.ln2, m.eps, y, h, tokens, m.hidden, by_norm2);
     if (code != NVJ_OK) return code;

@@ -421,16 +421,16 @@ def test_contexts_can_be_copied_and_pickled():
         assert torch.equal(runner.forward(ids, pos, other), want)
 
 
-@pytest.mark.parametrize("rows,hidden,inter,heads,wide_mb", [
-    (1, 256, 256, 2, 0), (3, 1024, 3072, 16, 0), (3, 1024, 3072, 16, 25), (16, 1024, 3072, 16, 40),
-    (16, 2048, 6144, 16, 0), (16, 2048, 6144, 16, 51), (17, 320, 448, 6, 0),
-    (40, 2048, 2560, 24, 0), (20, 2560, 9728, 16, 0), (129, 320, 448, 6, 0),
-    (200, 1024, 3072, 16, 0)])
-@pytest.mark.parametrize("layers", [1, 3])
-def test_weights_read_ahead(rows, hidden, inter, heads, wide_mb, layers, monkeypatch):
-    """Which weights a launch reads ahead depends on the layer, the row count, the widths and,
-    up to 16 rows, on the K and V that the block table holds: every set of them against the
-    library's products, to what two orders of bf16 roundings give (as above)."""
+@pytest.mark.parametrize("rows,hidden,inter,heads,layers,wide_mb", [
+    (3, 1024, 3072, 16, 8, 0), (3, 1024, 3072, 16, 8, 25), (16, 1024, 3072, 16, 8, 40),
+    (4, 2048, 3072, 16, 4, 0), (16, 2048, 3072, 16, 4, 51), (5, 1024, 3072, 16, 1, 0),
+    (17, 320, 34816, 6, 4, 0), (40, 2048, 4096, 24, 3, 0), (20, 2560, 9728, 16, 2, 0),
+    (64, 1024, 3072, 16, 8, 0), (129, 320, 34816, 6, 4, 0), (200, 1024, 3072, 16, 8, 0)])
+def test_weights_read_ahead(rows, hidden, inter, heads, layers, wide_mb, monkeypatch):
+    """Which weights a launch reads ahead depends on the size of the model (200 MB of layers, all
+    but one case here), the row count, the widths and, up to 16 rows, on the K and V that the
+    block table holds: every set of them against the library's products.  Two orders of bf16
+    roundings leave the logits of 28 layers of random weights 2-3 % apart."""
     print(f"case read ahead rows={rows} hidden={hidden} layers={layers} {wide_mb}", flush=True)
     from nanovllm_jax_amd.engine import decode_step as ds
     cfg = ds.DecodeModelConfig(num_layers=layers, hidden_size=hidden, num_heads=heads,
@@ -450,4 +450,4 @@ def test_weights_read_ahead(rows, hidden, inter, heads, wide_mb, layers, monkeyp
     monkeypatch.setattr(ds, "_NATIVE_STEP_ROWS", 0)
     want = runner.forward(*inputs).float()
     torch.cuda.synchronize()
-    assert (got - want).abs().max().item() <= 0.02 * want.abs().max().item() + 0.02
+    assert (got - want).norm().item() <= 0.03 * want.norm().item()
