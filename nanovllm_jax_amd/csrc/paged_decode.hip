@@ -2618,17 +2618,6 @@ constexpr int kMinBalancedSteps = 1;
 // positions): 9 % 153 against 165, 15 % 146 against 154, 25 % 137 against 142.
 constexpr int kWholeRowTolerance = 64;
 
-// Whether the table rules out rows (of at most one per CU) that are not short: two rounds
-// of the 8 waves of a workgroup, which take 2.8 us each, what one CU draws; such rows are
-// finished inside one workgroup by the kernel without a split.  With more than half as many
-// rows as CUs a third round is still no worse than what else there is: us, without a split /
-// by pieces, at 512 positions 1 .. 64 rows 8.2 .. 9.8 / 9.0 .. 10.0, 128 rows 10.6 / 10.4, 256
-// rows 13.2 / 13.9; at 768 1 .. 16 rows 9.7 .. 9.9 / 9.0 .. 9.1, 64 rows 13.6 / 10.5, 128 rows
-// 13.7 / 13.2, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
-bool table_of_short_rows(int64_t rows, int64_t positions) {
-  return positions <= (rows > 128 ? 3 : 2) * 8 * kStep;
-}
-
 // Whether a launch of at most one row per CU goes by pieces (paged_decode_pieces_kernel), from
 // what the table can hold; else the balanced kernel looks at the lengths.  Pieces save what
 // the balanced kernel's larger head and its merges by single waves cost a small launch, 3 us:
@@ -2642,6 +2631,27 @@ bool table_of_short_rows(int64_t rows, int64_t positions) {
 // 32.2 / 30.0.
 bool pieces_pay(int64_t rows, int64_t positions) {
   return rows * positions <= (rows <= 64 ? 1 << 20 : rows <= 128 ? 1 << 19 : 3 << 17);
+}
+
+// Whether pieces are what a launch of that many rows takes if its table is not one of short rows.
+bool pieces_take(int64_t batch, int head_dim, int64_t rows, int64_t positions) {
+  return head_dim == 128 && batch <= 64 && pieces_pay(rows, positions);
+}
+
+// Whether the table rules out rows (of at most one per CU) that are not short: up to three
+// rounds of the 8 waves of a workgroup, which take 1.2 (head_dim 64) to 2.8 us each, what one
+// CU draws; such rows are finished inside one workgroup by the kernel without a split.  us,
+// without a split / by the balanced kernel, at 768 positions, equal or ragged: head_dim 64, 1 ..
+// 16 rows 7.6 .. 8.7 / 12.1 .. 13.2, 24 .. 64 rows 7.7 .. 9.3 / 12.1 .. 13.5, 65 .. 128 rows 8.3 ..
+// 9.9 / 12.4 .. 13.9; head_dim 128, 65 .. 128 sequences of one row 10.4 .. 11.6 / 13.2 .. 14.6.
+// (At 1024 equal lengths the balanced kernel is still 2 .. 5 us behind; lengths that differ
+// have not been measured there.)
+// Where pieces are the other choice, up to 128 rows, the third round is theirs: without a
+// split / by pieces, at 512 positions 1 .. 64 rows 8.2 .. 9.8 / 9.0 .. 10.0, 128 rows 10.6 / 10.4,
+// 256 rows 13.2 / 13.9; at 768 1 .. 16 rows 9.7 .. 9.9 / 9.0 .. 9.1, 64 rows 13.6 / 10.5, 128 rows
+// 13.7 / 13.2, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
+bool table_of_short_rows(int64_t rows, int64_t positions, bool pieces) {
+  return positions <= (pieces && rows <= 128 ? 2 : 3) * 8 * kStep;
 }
 
 // Waves per workgroup of the fixed split = KV heads a workgroup covers: the
@@ -2853,7 +2863,10 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
                                  all_rows <= compute_units()
                              ? (int)all_rows
                              : 0;
-  const bool all_short = short_rows > 0 && table_of_short_rows(all_rows, (int64_t)max_blocks * block_size) &&
+  const int64_t positions = (int64_t)max_blocks * block_size;
+  const bool by_pieces = short_rows > 0 && !valu && !loads_only &&
+                         pieces_take(batch, head_dim, all_rows, positions);
+  const bool all_short = short_rows > 0 && table_of_short_rows(all_rows, positions, by_pieces) &&
                          !(phases & NVJ_PHASE_CLEAR_COUNTERS);
   if ((whole || all_short) && max_blocks > 0) {
     if (all_rows > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
@@ -2900,9 +2913,7 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
       }
       if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;
       dim3 grid;
-      const int64_t positions = (int64_t)max_blocks * block_size;
-      if (short_rows > 0 && head_dim == 128 && !valu && !loads_only && batch <= 64 &&
-          pieces_pay(all_rows, positions)) {
+      if (by_pieces) {
         const int64_t rounds = (positions + 8 * kStep - 1) / (8 * kStep);
         const int max_pieces = (int)std::min<int64_t>(all_rows * rounds, compute_units());
         const NewRows fresh = rows_behind(new_rows, max_pieces, batch, &grid);
@@ -3194,7 +3205,8 @@ extern "C" int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads
   if (chunk != 0 || nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads) >
                         kNullStreamWords * sizeof(int32_t))
     return 0;
-  return table_of_short_rows(rows, (int64_t)max_blocks * block_size) ? 1 : 2;
+  const int64_t positions = (int64_t)max_blocks * block_size;
+  return table_of_short_rows(rows, positions, pieces_take(batch, head_dim, rows, positions)) ? 1 : 2;
 }
 
 extern "C" int nvj_paged_decode_store_launch(

@@ -1014,6 +1014,36 @@ def test_short_rows(lens, Hq, Hkv, D):
         assert_close_bf16(torch_to_bits(got), want, what=f"lens={lens} phases={extra}")
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D", [(1, 2, 1, 64), (2, 16, 8, 64), (5, 32, 8, 64), (64, 4, 2, 64),
+                                        (65, 8, 1, 128), (128, 8, 1, 128)])
+@pytest.mark.parametrize("positions", [513, 768, 769])
+def test_short_rows_that_do_not_go_by_pieces(B, Hq, Hkv, D, positions):
+    """Three rounds of a workgroup are short rows wherever pieces are not the other choice
+    (head_dim 64, more than 64 sequences): the launch takes no workspace, and says so by
+    running without one; a table beyond them is refused without one."""
+    print(f"case short rows, no pieces B={B} Hkv={Hkv} D={D} {positions}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib
+    bs, dev, lib = 32, "cuda:0", _lib.load()
+    lens = np.random.default_rng(B + positions).integers(0, positions + 1, B)
+    lens[-1] = positions
+    NB = int((-(-lens // bs)).sum())
+    q, kc, vc, bt, ctx = make_problem(B + positions, B, Hq, Hkv, D, bs, NB, lens)
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)] + [torch.from_numpy(x).to(dev) for x in (bt, ctx)]
+    out = torch.empty_like(t[0])
+    counters = torch.zeros(1 << 14, dtype=torch.int32, device=dev)
+    code = lib.nvj_paged_decode_launch_counters(
+        torch.cuda.current_stream().cuda_stream, *(x.data_ptr() for x in t), out.data_ptr(), None, 0,
+        counters.data_ptr(), counters.numel() * 4, B, Hq, Hkv, D, bs, bt.shape[1], NB, D ** -0.5,
+        _lib.NVJ_DTYPE_BF16,
+        _lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE | _lib.NVJ_PHASE_SHORT_ROWS)
+    torch.cuda.synchronize()
+    assert code == (0 if positions <= 768 else -4)       # NVJ_ERR_WORKSPACE: nothing was launched
+    if code == 0:
+        assert_close_bf16(torch_to_bits(out), oracle(q, kc, vc, bt, ctx, D ** -0.5, bs),
+                          what=f"B={B} D={D} positions={positions}")
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv", [
     ([1000], 16, 8),                              # four pieces a row
     ([4100], 2, 2),                               # 17, one of them short of a step
