@@ -406,11 +406,6 @@ __global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
   const int chain = wave % CHAINS, half = wave / CHAINS;
-  if ((int)blockIdx.y * BM >= a.M) {
-    const int row = (int)blockIdx.y - (a.M + BM - 1) / BM;
-    nvj::read_chunk<256>(a.ahead, row * (int)gridDim.x + (int)blockIdx.x);
-    return;
-  }
   const int n_tile = blockIdx.x, m0 = blockIdx.y * BM;
   const int row_bytes = a.K * 2;
   const int rounds = a.K / (32 * CHAINS * RUN);
@@ -490,9 +485,7 @@ __global__ __launch_bounds__(256) void chained_linear_kernel(LinearArgs a) {
 
 template <int BM, int BN, int CHAINS, int RUN, int ST>
 hipError_t launch_chained(hipStream_t s, const LinearArgs& a) {
-  const unsigned columns = (unsigned)((a.N + BN - 1) / BN);
-  const dim3 grid(columns, (unsigned)((a.M + BM - 1) / BM) +
-                               (a.ahead.chunks() + columns - 1) / columns);
+  const dim3 grid((unsigned)((a.N + BN - 1) / BN), (unsigned)((a.M + BM - 1) / BM));
   return nvj::launch(chained_linear_kernel<BM, BN, CHAINS, RUN, ST>, grid, dim3(256), s, a);
 }
 
