@@ -451,3 +451,47 @@ def test_weights_read_ahead(rows, hidden, inter, heads, layers, wide_mb, monkeyp
     want = runner.forward(*inputs).float()
     torch.cuda.synchronize()
     assert (got - want).norm().item() <= 0.03 * want.norm().item()
+
+
+@pytest.mark.parametrize("rows,hidden,inter,heads,layers,wide_mb", [
+    (3, 1024, 3072, 16, 8, 0), (3, 1024, 3072, 16, 8, 25), (16, 1024, 3072, 16, 8, 40),
+    (4, 2048, 3072, 16, 4, 0), (16, 2048, 3072, 16, 4, 51), (17, 320, 34816, 6, 4, 0),
+    (40, 2048, 4096, 24, 3, 0), (20, 2560, 9728, 16, 2, 0), (64, 1024, 3072, 16, 8, 0),
+    (129, 320, 34816, 6, 4, 0), (200, 1024, 3072, 16, 8, 0)])
+@pytest.mark.parametrize("kind", ["decode", "packed"])
+def test_reading_ahead_changes_no_bit(rows, hidden, inter, heads, layers, wide_mb, kind):
+    """Layers of up to 200 MB are not read ahead, larger models are.  A layer in front whose
+    output and down projections are zero adds nothing to the (bf16) embedding rows, so the same
+    layers are run with it, beyond the line, and without it, below: the same logits and the
+    same cache rows, bit for bit."""
+    print(f"case no bit rows={rows} hidden={hidden} layers={layers} {wide_mb} {kind}", flush=True)
+    from nanovllm_jax_amd.engine import decode_step as ds
+    cfg = ds.DecodeModelConfig(num_layers=layers, hidden_size=hidden, num_heads=heads,
+                               num_kv_heads=2, head_dim=128, intermediate_size=inter,
+                               vocab_size=1000, max_position=256, block_size=64,
+                               num_kvcache_blocks=rows + 4)
+    runner = ds.DecodeStepRunner(cfg, "cuda:0", seed=rows + layers)
+    weights = sum(runner.layers[0][n].nbytes for n in ("qkv", "o", "gate_up", "down"))
+    assert (layers - 1) * weights <= 200 << 20 < layers * weights
+    for name in ("o", "down"):
+        runner.layers[0][name].zero_()
+    ids = [7 * i % 1000 for i in range(rows)]
+    if kind == "decode":
+        inputs = runner.make_inputs(ids, [1 + 5 * i % 64 for i in range(rows)],
+                                    [[i] for i in range(rows)])
+        # 1 KB of K and V a position
+        inputs[2].block_tables = torch.nn.functional.pad(
+            inputs[2].block_tables, (0, (wide_mb << 20) // (rows * 64 * 1024)),
+            value=-1).contiguous()
+    else:
+        inputs = runner.make_prefill_inputs([ids], [list(range(-(-rows // 64)))])
+    before = runner.kv_cache.clone()
+    with_it = runner._native_forward(*inputs)
+    kv = runner.kv_cache.clone()
+    runner.kv_cache.copy_(before)
+    del runner.layers[0], runner.attn[0]
+    for _ in range(2):            # (the second with whatever the caches hold by then)
+        without = runner._native_forward(*inputs)
+        torch.cuda.synchronize()
+        assert not without.isnan().any() and torch.equal(with_it, without)
+        assert torch.equal(kv[:, 1:].view(torch.int16), runner.kv_cache[:, 1:].view(torch.int16))
