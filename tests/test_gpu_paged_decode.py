@@ -1137,6 +1137,41 @@ def test_equal_cut_of_few_and_of_many_sequences(Hq, Hkv, dtype, hi):
                           what="equal cut")
 
 
+@pytest.mark.parametrize("Hq,Hkv,parts", [(8, 4, 2), (64, 8, 2), (6, 2, 4), (16, 1, 8)])
+def test_equal_cut_of_wide_tables_and_long_rows(Hq, Hkv, parts):
+    """The same two kernels where the table is so wide that the cut goes by units of two steps
+    or more ((units + 2) * sub-runs has to fit 31 bits), with rows that several hundred
+    sub-runs share, whose partials are merged in several passes."""
+    print(f"case equal cut, wide table Hq={Hq} Hkv={Hkv}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    lens = np.random.default_rng(Hkv).integers(0, 300, 36)
+    lens[[3, 17, 35]] = 0, 9000, 20000
+    bs, dev, outs = 64, "cuda:0", []
+    NB = int((-(-lens // bs)).sum()) + 2
+    q, kc, vc, bt, ctx = make_problem(Hq + Hkv, 36, Hq, Hkv, 128, bs, NB, lens)
+    side_by_side = 8 // parts                        # KV heads of a workgroup, from batch 32 up
+    rows = Hkv // side_by_side
+    subruns = torch.cuda.get_device_properties(0).multi_processor_count * parts
+    steps = (1 << 31) // subruns // (36 * rows) + 2  # of the table: one step more than fits
+    shift = lambda batch: next(s for s in range(9)
+                               if ((batch * rows * steps >> s) + 2) * subruns < 1 << 31)
+    assert shift(36) == shift(70) == 1
+    wide = torch.full((70, -(-steps * 32 // bs)), -1, dtype=torch.int32, device=dev)
+    wide[:36, :bt.shape[1]] = torch.from_numpy(bt).to(dev)
+    for batch in (36, 70):
+        pad = lambda x: np.concatenate([x, np.zeros((batch - 36, *x.shape[1:]), x.dtype)])
+        t = [bits_to_torch(x, dev) for x in (pad(q), kc, vc)]
+        outs.append(paged_attention(
+            *t, wide[:batch].contiguous(), torch.from_numpy(pad(ctx)).to(dev), 128 ** -0.5,
+            bs, chunk=0, phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+            | _lib.NVJ_PHASE_SHARED_ROWS)[:36])
+        torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert_close_bf16(torch_to_bits(outs[0]), oracle(q, kc, vc, bt, ctx, 128 ** -0.5, bs),
+                      what="equal cut, wide table")
+
+
 @pytest.mark.parametrize("own_workspace", [False, True])
 @pytest.mark.parametrize("dtype,k_f32", [("bf16", True), ("f16", False)])
 @pytest.mark.parametrize("lens,split", [([1], 0), ([700], 0), ([33, 512, 65, 32, 0, 64], 0),
