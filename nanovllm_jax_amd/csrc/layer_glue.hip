@@ -52,7 +52,9 @@ __device__ __forceinline__ void unpack8(const uint4& p, float (&f)[8]) {
 // token row each).
 // PIECES = 16-byte pieces per lane, a compile-time bound so the row stays in
 // registers between the two passes.
-template <int PIECES, bool RESIDUAL>
+// PAST_L2: see kResidualPastL2Bytes (with a flag at run time the compiler makes one ordinary store
+// of the two).
+template <int PIECES, bool RESIDUAL, bool PAST_L2>
 __global__ __launch_bounds__(256) void add_rms_norm_kernel(
     const uint4* __restrict__ x, const uint4* residual, const float* __restrict__ weight,
     float eps, uint4* __restrict__ y, uint4* residual_out, int num_tokens, int row_pieces,
@@ -110,7 +112,8 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(
         o.y = pack2(s[j][2], s[j][3]);
         o.z = pack2(s[j][4], s[j][5]);
         o.w = pack2(s[j][6], s[j][7]);
-        nvj::store_past_l2(residual_out + row + p, o);   // (read again two products later)
+        if constexpr (PAST_L2) nvj::store_past_l2(residual_out + row + p, o);
+        else residual_out[row + p] = o;
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) a = a + s[j][e] * s[j][e];
@@ -161,16 +164,29 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(const uint4* __restri
   y[i] = out;
 }
 
+// The residual is read again two products later.  Up to 10 MB of it goes past the L2s, which then
+// keep what those products read: a step of 12 layers of 1024 (3072) 1530 -> 1524 us with 4 MB,
+// 2455 -> 2448 with 8.7, 3319 either way with 12; the norm alone 7.3 -> 6.8 with 8 (4096 rows of
+// 1024), 9.2 -> 8.9 with 12, where 1 MB copied in between makes it 19.0 -> 19.9.  More of it is
+// stored like any other row: past the L2s a norm of 16 MB (8192 rows of 1024) took 11.2 .. 11.6
+// us instead of 10.9, of 40 MB (5000 of 4096) 32.1 instead of 27.2, of 64 MB 46.9 instead of 43.4;
+// steps of 16 .. 64 MB were as fast either way.
+constexpr int64_t kResidualPastL2Bytes = 10 << 20;
+
 template <int PIECES>
 hipError_t launch_add_rms_norm(hipStream_t stream, const uint4* x, const uint4* residual,
                          const float* weight, float eps, uint4* y, uint4* residual_out,
                          int num_tokens, int row_pieces, const nvj::ReadAhead& ahead) {
   const dim3 grid((unsigned)((num_tokens + 3) / 4) + ahead.chunks()), block(256);
+  const bool past_l2 = (int64_t)num_tokens * row_pieces * 16 <= kResidualPastL2Bytes;
+  if (residual != nullptr && past_l2)
+    return nvj::launch(add_rms_norm_kernel<PIECES, true, true>, grid, block, stream, x, residual,
+                       weight, eps, y, residual_out, num_tokens, row_pieces, ahead);
   if (residual != nullptr)
-    return nvj::launch(add_rms_norm_kernel<PIECES, true>, grid, block, stream, x, residual, weight,
-                       eps, y, residual_out, num_tokens, row_pieces, ahead);
-  return nvj::launch(add_rms_norm_kernel<PIECES, false>, grid, block, stream, x, nullptr, weight,
-                     eps, y, nullptr, num_tokens, row_pieces, ahead);
+    return nvj::launch(add_rms_norm_kernel<PIECES, true, false>, grid, block, stream, x, residual,
+                       weight, eps, y, residual_out, num_tokens, row_pieces, ahead);
+  return nvj::launch(add_rms_norm_kernel<PIECES, false, false>, grid, block, stream, x, nullptr,
+                     weight, eps, y, nullptr, num_tokens, row_pieces, ahead);
 }
 
 }  // namespace

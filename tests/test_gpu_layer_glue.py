@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,hidden", [(128, 1024), (1, 8), (7, 520), (33, 4096), (5, 8192),
-                                      (0, 1024)])
+                                      (0, 1024),
+                                      (5120, 1024), (5121, 1024)])   # residuals of 10 MB, and more
 @pytest.mark.parametrize("with_residual", [False, True])
 def test_add_rms_norm_bit_exact(T, hidden, with_residual):
     import torch
