@@ -2627,10 +2627,22 @@ constexpr int kWholeRowTolerance = 64;
 // workgroups idle when lengths differ and rows are many, and one KV head per workgroup
 // streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.7 / 73.4, 64 rows of
 // 1000 .. 16000 53.5 / 55.8 and of 16000 .. 32768 145 / 138, 128 rows of 300 .. 4096 28.9 /
-// 30.2 and of 500 .. 8000 47.3 / 46.0, 256 rows of 100 .. 1500 24.6 / 26.6 and of 128 .. 2048
-// 32.2 / 30.0.
+// 30.2 and of 500 .. 8000 47.3 / 46.0.
+// Equal rows that leave a quarter of the workgroups idle (86 .. 96 rows) end earlier: 88 rows of
+// 3000 29.0 / 30.2, 96 of 3000 31.2 / 32.0 and of 4096 41.3 / 39.2, 88 of 5952 52.6 / 49.6.
+// Beyond 128 rows the mean row has less than two pieces, and where long rows find none to spare
+// one workgroup walks all of a row: 144 rows of 1024 or 20 positions, a third of them long, 14.5 /
+// 14.1, 192 of 1024 equal 21.3 / 23.6; but a fifth of 144 short and the others 2048 long 31.9 /
+// 30.0, 136 of 2880 46.2 / 40.2, 224 of 832 or 20 15.1 / 14.0 and of 1536 or 20 24.1 / 18.8, 8 of
+// 256 of 1536 and the others of 20 20.5 / 14.6.
+// Within the line single steps of the search remain, at worst 16 sequences, one of 1536 and the
+// others of 307, 14.9 / 13.5; of 1386 mixes of lengths 13 were more than 2.5 % behind.
 bool pieces_pay(int64_t rows, int64_t positions) {
-  return rows * positions <= (rows <= 64 ? 1 << 20 : rows <= 128 ? 1 << 19 : 3 << 17);
+  const int64_t cus = compute_units();
+  if (rows > cus - cus / 4) return false;
+  const bool idle = cus / rows * rows <= cus - cus / 4;   // with equal rows
+  return rows * positions <=
+         (rows <= 64 ? 1 << 20 : rows > 128 ? 3 << 16 : idle ? 5 << 16 : 1 << 19);
 }
 
 // Whether pieces are what a launch of that many rows takes if its table is not one of short rows.

@@ -1044,17 +1044,46 @@ def test_short_rows_that_do_not_go_by_pieces(B, Hq, Hkv, D, positions):
                           what=f"B={B} D={D} positions={positions}")
 
 
-@pytest.mark.parametrize("lens,Hq,Hkv", [
-    ([1000], 16, 8),                              # four pieces a row
-    ([4100], 2, 2),                               # 17, one of them short of a step
-    ([6000, 0, 1, 33], 6, 2),                     # a group of 3, an empty row, one lone row
-    ([300, 2048, 900, 257, 0, 1024, 700, 5], 32, 8),
-    ([3900, 40, 300], 16, 1),                     # a group of 16: one lane group
-    ([5000] + [20] * 63, 4, 4),                   # as many rows as CUs: a piece is the longest row
-    ([1100] * 20, 8, 4),
+def route_of_pieces(batch, kv_heads, max_blocks, bs, lens=None):
+    """Where a launch of short rows goes (head_dim 128, groups of 16 at most), as the host
+    decides it: "table", every row inside one workgroup, "pieces", or "balanced".  With lengths,
+    pieces by way of the kernel's own choice as well: "pieces" when the mean length per workgroup
+    is one that fits, "search" when a longer one has to be looked for."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rows, positions = batch * kv_heads, max_blocks * bs
+    most_idle = cus - cus // 4
+    pays = (1 << 20 if rows <= 64 else 0 if rows > most_idle else 3 << 16 if rows > 128 else
+            5 << 16 if cus // rows * rows <= most_idle else 1 << 19)
+    takes = batch <= 64 and rows * positions <= pays
+    if rows > cus or batch > 256:
+        return "balanced"
+    if positions <= (512 if takes and rows <= 128 else 768):
+        return "table"
+    if not takes or lens is None:
+        return "pieces" if takes else "balanced"
+    most = min(rows * -(-positions // 256), cus) // kv_heads
+    steps = [-(-n // 32) for n in lens]
+    mean = max(1, -(-sum(steps) // (8 * most)))
+    return "pieces" if sum(-(-n // (8 * mean)) for n in steps) <= most else "search"
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,route", [
+    ([1000], 16, 8, "pieces"),                    # four pieces a row
+    ([4100], 2, 2, "pieces"),                     # 17, one of them short of a step
+    ([6000, 0, 1, 33], 6, 2, "pieces"),           # a group of 3, an empty row, one lone row
+    ([300, 2048, 900, 257, 0, 1024, 700, 5], 32, 8, "pieces"),
+    ([3900, 40, 300], 16, 1, "pieces"),           # a group of 16: one lane group
+    ([5000] + [20] * 63, 4, 4, "balanced"),       # as many rows as CUs
+    ([1100] * 20, 8, 4, "pieces"),
+    ([1000] * 17 + [20] * 31, 4, 4, "search"),    # one row too many for two pieces each: the longest
+    ([1000] * 9 + [20] * 15, 16, 8, "search"),    # the same with more heads
+    ([1024, 1000, 800] + [20 * i for i in range(21)], 16, 8, "search"),
+    ([7878] * 7, 32, 8, "search"),                # one longer than the mean fits: four pieces a row
+    ([4096] * 12, 16, 8, "balanced"),             # 96 equal rows would leave a quarter of the CUs idle
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-def test_rows_in_pieces(lens, Hq, Hkv, dtype):
+def test_rows_in_pieces(lens, Hq, Hkv, route, dtype):
     """Rows cut into pieces of a workgroup each, against the oracle; the counters are left
     at zero, a launch on a counter that is not is flagged and the next is right again, and
     replays of a graph follow lengths that change."""
@@ -1065,7 +1094,7 @@ def test_rows_in_pieces(lens, Hq, Hkv, dtype):
     bs, B, dev = 64, len(lens), "cuda:0"
     NB = sum(-(-n // bs) for n in lens) + 3
     q, kc, vc, bt, ctx = make_problem(77 + B + Hq, B, Hq, Hkv, 128, bs, NB, lens)
-    assert bt.shape[1] * bs > 768                 # (smaller tables take no split)
+    assert route_of_pieces(B, Hkv, bt.shape[1], bs, lens) == route
     scale = 128 ** -0.5
     t = [bits_to_torch(x, dev) for x in (q, kc, vc)]
     if dtype == "f16":
