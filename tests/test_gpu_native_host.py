@@ -10,10 +10,12 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = {"one": ([700], 16, 8), "few": ([128, 2000, 900, 1, 513], 16, 8),
           "many rows": ([300 + 7 * i for i in range(40)], 16, 8),
-          # 16 rows and 24, 128 and 120 of a table of three rounds: both sides of its rule
+          # a table of three rounds: 16 rows and 24, both sides of the rule for a side stream;
+          # 128, 120 and 136, both sides of the rule for counters at hand
           "two": ([700, 768], 16, 8), "three": ([700, 768, 513], 16, 8),
           "sixteen": ([768 - 40 * i for i in range(16)], 16, 8),
-          "fifteen": ([768 - 40 * i for i in range(15)], 16, 8)}
+          "fifteen": ([768 - 40 * i for i in range(15)], 16, 8),
+          "seventeen": ([768 - 40 * i for i in range(17)], 16, 8)}
 
 
 def _layer(name, seed, dtype=torch.bfloat16):

@@ -1203,10 +1203,16 @@ def test_equal_cut_of_wide_tables_and_long_rows(Hq, Hkv, parts):
 
 @pytest.mark.parametrize("own_workspace", [False, True])
 @pytest.mark.parametrize("dtype,k_f32", [("bf16", True), ("f16", False)])
-@pytest.mark.parametrize("lens,split", [([1], 0), ([700], 0), ([33, 512, 65, 32, 0, 64], 0),
-                                        ([513, 40, 1300, 33, 900], -1), ([100, 3000] * 16, 0),
-                                        ([2, 65] * 32, 0)])
-def test_store_in_the_same_launch(lens, split, dtype, k_f32, own_workspace):
+@pytest.mark.parametrize("lens,split,route", [
+    ([1], 0, "table"), ([700], 0, "pieces"), ([33, 512, 65, 32, 0, 64], 0, "table"),
+    ([513, 40, 1300, 33, 900], -1, "table"), ([100, 3000] * 16, 0, "balanced"),
+    ([2, 65] * 32, 0, "table"),
+    ([768 - 37 * i for i in range(17)], 0, "table"),   # three rounds, more than 128 rows
+    ([100, 1000, 700, 300, 900, 64, 513], 0, "pieces"),   # new rows by workgroups to spare,
+    ([100, 2000, 1025, 300, 1500, 64, 513, 1999], 0, "pieces"),   # and by those of the pieces,
+    ([1000, 33] + [64, 1, 65, 900, 257, 513] * 3, 0, "pieces"),   # with one piece a row for most
+])
+def test_store_in_the_same_launch(lens, split, route, dtype, k_f32, own_workspace):
     """New rows stored by the attention launch itself against the two launches: rows
     in the middle of a step and at its ends, a row that another entry of the batch also
     attends to, slots that are not stored, and a cache that holds NaN wherever no position is
@@ -1250,6 +1256,7 @@ def test_store_in_the_same_launch(lens, split, dtype, k_f32, own_workspace):
     v = torch.randn(B, Hkv, D, generator=g, device=dev).to(dt)
     t_slots, t_table = torch.from_numpy(slots).to(dev), torch.from_numpy(table).to(dev)
     t_lens = torch.from_numpy(np.array(lens, np.int32)).to(dev)
+    assert split or route_of_pieces(B, Hkv, table.shape[1], bs) == route
     want_caches = [c.clone() for c in caches]
     store_kv_to_cache(k, v, *want_caches, t_slots)
     want = paged_attention(q, *want_caches, t_table, t_lens, D ** -0.5, bs, chunk=split)
