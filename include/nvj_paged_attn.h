@@ -517,7 +517,8 @@ NVJ_API int nvj_prefill_attention_rows_launch(void* stream, const void* q, int64
  * t < num_rows, also goes to slot slot_mapping[t] of the caches [num_slots, num_kv_heads,
  * head_dim] (`dtype`, as k and v have it; slots < 0 or >= num_slots are not stored), as
  * nvj_store_kvcache_launch would have done in front.  The attention reads k and v, never the
- * caches.  Rows beyond what 32 bits count in 16-byte pieces take two launches.
+ * caches.  Rows beyond what 32 bits count in 16-byte pieces take two launches, and so do
+ * hundreds of prompts of a few tokens, where that is faster.
  */
 NVJ_API int nvj_prefill_attention_store_launch(void* stream, const void* q, const void* k,
                             const void* v, const int32_t* cu_seqlens_q,

@@ -407,10 +407,12 @@ struct StoreShare {
   int slot0, slot1;
 
   // The share is counted from the end, as the tiles are walked: its rows are those that the
-  // tiles of the same time read, and come out of a cache.
+  // tiles of the same time read, and come out of a cache.  Whole heads, so that no two
+  // workgroups write to one cache line (shares of 16 .. 64 pieces: 2 % of the launch).
   __device__ __forceinline__ StoreShare(const PrefillArgs& a) {
-    at = (uint32_t)((uint64_t)a.new_pieces * (gridDim.x - 1 - blockIdx.x) / gridDim.x);
-    end = (uint32_t)((uint64_t)a.new_pieces * (gridDim.x - blockIdx.x) / gridDim.x);
+    const uint64_t heads = a.new_pieces / kPieces;
+    at = kPieces * (uint32_t)(heads * (gridDim.x - 1 - blockIdx.x) / gridDim.x);
+    end = kPieces * (uint32_t)(heads * (gridDim.x - blockIdx.x) / gridDim.x);
     k0 = k1 = v0 = v1 = make_uint4(0u, 0u, 0u, 0u);
     slot0 = slot1 = -1;
   }
@@ -425,16 +427,17 @@ struct StoreShare {
     k1 = a.k[p1];
     v1 = a.v[p1];
   }
+  // (Nothing is stored past the end: hundreds of stores of one piece cost a workgroup with few
+  // pieces 1 .. 2 us.)
   __device__ __forceinline__ void put(const PrefillArgs& a) {
     if (at >= end) return;
-    const uint32_t p0 = min(at + threadIdx.x, end - 1);
-    const uint32_t p1 = min(at + threadIdx.x + kBatch / 2, end - 1);
-    if (slot0 >= 0 && slot0 < a.num_slots) {
+    const uint32_t p0 = at + threadIdx.x, p1 = p0 + kBatch / 2;
+    if (p0 < end && slot0 >= 0 && slot0 < a.num_slots) {
       const int64_t dst = (int64_t)slot0 * a.row_pieces + p0 % a.row_pieces;
       store_past_l2(a.k_cache + dst, k0);
       store_past_l2(a.v_cache + dst, v0);
     }
-    if (slot1 >= 0 && slot1 < a.num_slots) {
+    if (p1 < end && slot1 >= 0 && slot1 < a.num_slots) {
       const int64_t dst = (int64_t)slot1 * a.row_pieces + p1 % a.row_pieces;
       store_past_l2(a.k_cache + dst, k1);
       store_past_l2(a.v_cache + dst, v1);
@@ -831,22 +834,46 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
 // attention saves (0.4).
 constexpr int64_t kStreamOutBytes = 32 << 20;
 
+// The most query tiles that a launch can have, per KV head, and whether they are of one column
+// group per wave instead of two.
+struct TileBound {
+  bool small;
+  int64_t tiles;
+};
+TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads) {
+  // every sequence adds at most one partly filled token block and one partly filled tile
+  const int64_t blocks = (tokens + 15 * batch) / 16;
+  auto tiles_of = [&](int column_groups) {
+    return (blocks * group + (column_groups - 1) * batch) / column_groups;
+  };
+  // one column group per wave while the larger workgroups would not fill the CUs: one prompt
+  // of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1
+  const bool small = tiles_of(2 * kWaves) * num_kv_heads <= nvj::compute_units();
+  return {small, tiles_of((small ? 1 : 2) * kWaves)};
+}
+
+// Whether the store of new rows rides in the attention launch.  A share costs its workgroup about
+// 1 us: over more than three rounds of two workgroups per CU that is more than a launch of the
+// store's own, unless the shares are large.  us in one launch / in two, 64 / 8 heads: 300
+// prompts of 4 tokens 48.6 / 44.1, 200 of up to 17 34.8 / 32.4, 500 of 9 104.9 / 98.5 (31, 59 and 61
+// pieces a share); from 80 pieces on -19 .. +2 %, with fewer rounds -22 .. -1 %.
+bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
+                 int64_t num_kv_heads) {
+  const int64_t tiles =
+      tile_bound(tokens, batch, num_heads / num_kv_heads, num_kv_heads).tiles * num_kv_heads;
+  return tiles <= 6 * nvj::compute_units() || rows * num_kv_heads * kPieces >= 80 * tiles;
+}
+
 // Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.
 constexpr int64_t kLongestFirstPerCu = 16;
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype) {
-  // every sequence adds at most one partly filled token block and one partly filled tile
   if (((int64_t)total_q_tokens + 15) * a.group > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const int64_t blocks = ((int64_t)total_q_tokens + 15 * (int64_t)a.batch) / 16;
-  auto tiles_of = [&](int column_groups) {
-    return (blocks * a.group + (column_groups - 1) * (int64_t)a.batch) / column_groups;
-  };
-  // one column group per wave while the larger workgroups would not fill the CUs: one prompt
-  // of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1
   const int64_t cus = nvj::compute_units();
-  const bool small = tiles_of(2 * kWaves) * a.num_kv_heads <= cus;
-  const int64_t tiles = tiles_of((small ? 1 : 2) * kWaves);
+  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group, a.num_kv_heads);
+  const bool small = bound.small;
+  const int64_t tiles = bound.tiles;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
   const int64_t items = tiles * a.num_kv_heads;
   if (items > INT32_MAX - 8) return NVJ_ERR_BAD_SHAPE;
@@ -966,7 +993,8 @@ extern "C" int nvj_prefill_attention_store_launch(
   const CacheRows rows = {slot_mapping, k_cache, v_cache, num_slots, num_rows};
   // the kernel counts the pieces of all rows in 32 bits
   const bool together = num_rows > 0 && total_q_tokens > 0 && batch > 0 &&
-                        (int64_t)num_rows * num_kv_heads * kPieces <= UINT32_MAX - 4096;
+                        (int64_t)num_rows * num_kv_heads * kPieces <= UINT32_MAX - 4096 &&
+                        store_rides(total_q_tokens, num_rows, batch, num_heads, num_kv_heads);
   if (!together && num_rows > 0) {
     const int code = store_alone();
     if (code != NVJ_OK) return code;

@@ -339,6 +339,9 @@ def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
     ([250, 31, 0, 300] * 12, 32, 8, "f16", 0),    # shares of more than one batch
     ([90] * 60, 32, 8, "bf16", 1),                # 44 MB of output: past the L2s
     ([2100, 1], 8, 1, "bf16", 0),
+    ([5, 9, 1] * 30, 32, 8, "f16", 3),            # shares of three or four rows of a head
+    ([12, 0, 20] * 100, 32, 8, "bf16", 0),        # ... of six, over many rounds
+    ([4, 1, 6] * 100, 64, 8, "bf16", 2),          # few tokens, many rounds: two launches
 ])
 def test_prefill_with_the_store_in_the_launch(lens, Hq, Hkv, dtype, padding):
     """Caches and output bit for bit as the store's own launch and the attention's leave
