@@ -501,7 +501,9 @@ int attention(void* stream, const nvj_decoder_model& m, const nvj_decoder_layer&
 // Whether the weights of a layer have left the Infinity Cache (256 MB) by the time the next step
 // comes to it; else there is nothing to read ahead.  us without / with: 12 layers of 1024 (3072),
 // 378 MB, 64 rows 763 / 698, a prompt of 400 tokens 887 / 827; 28 of 512 (1536), 245 MB, 1319 /
-// 1289; 6 of 1024, 189 MB, 337 / 342 and 392 / 392; 3 of 1024 178 / 182.
+// 1289; 6 of 1024, 189 MB, 337 / 342 and 392 / 392; 3 of 1024 178 / 182.  Close to the line the LM
+// head decides what stays: 7 of 1024, 220 MB, 20 rows 413 / 386 with a head of 311 MB, 303 / 313 with
+// one of 16.
 bool weights_leave_the_cache(const nvj_decoder_model& m) {
   const int64_t q = (int64_t)m.num_heads * m.head_dim, kv = (int64_t)m.num_kv_heads * m.head_dim;
   const int64_t rows = 2 * (q + kv) + 3 * (int64_t)m.intermediate;   // of `hidden` elements

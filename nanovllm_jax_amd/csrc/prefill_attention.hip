@@ -399,7 +399,7 @@ struct PrefillArgs {
 // fetches two pieces of K and V per thread before its tiles and writes them behind, then what
 // is left of its share.  The store's own launch takes 25 us for 156 MB; in here it hides under
 // the tiles' round trips: 128 prompts of 16..300 tokens (32 / 8 heads) 143 -> 130 us, and 117
-// with rows stored past the L2s (inputs of the call before; 140 -> 124 with fresh ones).
+// with rows stored past the L2s (inputs of the call before; 140 -> 123 with fresh ones).
 struct StoreShare {
   static constexpr uint32_t kBatch = 2 * kWaves * 64;
   uint32_t at, end;
