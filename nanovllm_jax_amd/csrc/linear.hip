@@ -1,7 +1,7 @@
 // Products of activation rows with bf16 weights, C[m][n] = x[m][:] . w[n][:], for
 // prompts (hundreds to thousands of rows) on gfx950, with the element-wise stage that
 // follows a projection of the decoder layer in the epilogue:
-//   kPlain    bf16 rows
+//   kPlain    bf16 rows (kRowsPastL2: the same, stored past the L2)
 //   kSiluMul  SiLU(gate) * up of the fused gate/up projection (layers/activation.py:22-33
 //             of the reference), half the columns
 //   kQkRope   QK-RMSNorm, RoPE and KV-cache store of the fused QKV projection
@@ -14,14 +14,15 @@
 // so that operand reads, copies and matrix instructions run under each other throughout.
 // Measured, 4400 rows, alone: QKV (4096 x 1024) without its epilogue 40.9 us, O (1024 x 2048)
 // 21.9, gate/up (6144 x 1024) with SiLU * up 62.2, down (1024 x 3072) 29.8; library 46.4, 27.6,
-// 56.4 + 16.7, 35.2.  In a step: QKV with norm, RoPE and store 51.1, O 22.9, gate/up 62.7,
-// down 33.6, the matrix pipe 36 % (QKV) to 44 % busy.  LDS is the next limit: operand reads
+// 56.4 + 16.7, 35.2.  In a step of 4268: QKV with norm, RoPE and store 50.6, O 19.8, gate/up
+// 64.0 (beside the workgroups that read ahead), down 27.2, the matrix pipe 38 % (QKV) to 52 %
+// (O, down) busy.  LDS is the next limit: operand reads
 // and arriving copies take 75 % (256 x 256) to 150 % (128 x 128) of the matrix cycles.
 // Weights straight into registers instead (as in decoder_step.hip) were no way out: 64-byte
 // pieces of 16 rows per load made it 1 us per step whatever the tile.
 //
-// Rows go past the writing XCD's L2 where that was measured to help the step: the plain rows
-// (a norm on all XCDs reads them once), q and the cache rows: 4268 rows in 8 prompts 6310 ->
+// Rows go past the writing XCD's L2 where that was measured to help the step: 4 .. 24 MB of plain
+// rows (a norm on all XCDs reads them once), q and the cache rows: 4268 rows in 8 prompts 6310 ->
 // 6184 us with the norm's residual (layer_glue.hip), 128 rows of decode 3517 -> 3492; not SiLU *
 // up and the packed K and V, which the next launch reads several times.
 //
@@ -53,7 +54,7 @@ using nvj::f32_to_bf16_rne;
 using nvj::LinearArgs;
 using nvj::pack2_bf16;
 using nvj::store_past_l2;
-enum Epilogue { kPlain, kSiluMul, kQkRope };
+enum Epilogue { kPlain, kRowsPastL2, kSiluMul, kQkRope };
 
 template <int N>
 __device__ __forceinline__ void wait_copies() {
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
       if (m0 + m < a.M && n < n_out) {
         uint4* to = reinterpret_cast<uint4*>(a.out + (int64_t)(m0 + m) * n_out + n);
         const uint4 v = *reinterpret_cast<const uint4*>(lds + m * kOutStride + 16 * piece);
-        if constexpr (EPI == kPlain) store_past_l2(to, v);
+        if constexpr (EPI == kRowsPastL2) store_past_l2(to, v);
         else *to = v;
       }
     }
@@ -538,6 +539,14 @@ int best_shape(int64_t m, int64_t n, int k, int min_bn) {
   return best;
 }
 
+// Plain rows that go past the L2s.  Smaller outputs stay where a norm behind them finds them, larger
+// ones are written more slowly that way.  us with the norm behind, past the L2s / not: 1000 rows of
+// 1024 (2 MB) 13.0 / 12.7, 200 of 4096 16.2 / 15.6, 2048 of 1024 20.2 / 20.3, 2048 of 4096 34.9 /
+// 35.9, 3000 of 4096 44.7 / 45.3, 4268 of 4096 (35 MB) 65.1 / 61.7, 8192 of 4096 114 / 102.
+// (A flag of the kernel instead of a kernel of its own costs registers, and 1 .. 3 % of a large
+// product.)
+constexpr int64_t kPastL2From = 4 << 20, kPastL2To = 24 << 20;
+
 template <Epilogue EPI>
 hipError_t launch_shape(int shape, hipStream_t s, const LinearArgs& a) {
   switch (shape) {
@@ -569,7 +578,10 @@ bool linear_takes(int64_t m, int64_t n, int64_t k) {
 
 hipError_t linear(hipStream_t s, LinearArgs a) {
   a.group_m = 8;   // 8 x 4 tiles at a time per XCD: 51 -> 42 us for 160 x 256 tiles at 4400 rows
-  return launch_shape<kPlain>(a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0), s, a);
+  const int shape = a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0);
+  const int64_t bytes = (int64_t)a.M * a.N * 2;
+  return bytes >= kPastL2From && bytes <= kPastL2To ? launch_shape<kRowsPastL2>(shape, s, a)
+                                                    : launch_shape<kPlain>(shape, s, a);
 }
 hipError_t linear_silu_mul(hipStream_t s, LinearArgs a) {
   a.group_m = 8;

@@ -60,6 +60,20 @@ def test_rows_of_every_tile(tile, reduction):
 
 
 @pytest.mark.parametrize("tile", [-1] + list(range(len(TILES))))
+@pytest.mark.parametrize("rows,outputs", [(2048, 1024), (513, 4104), (1543, 8152), (1545, 8152)])
+def test_rows_past_the_l2_of_every_tile(tile, rows, outputs):
+    """4 to 24 MB of rows are stored by kernels of their own: both ends, and beyond."""
+    print(f"case linear past L2 tile={tile} {rows} x {outputs}", flush=True)
+    x, w = _operands(500 + tile + rows, rows, outputs, 128)
+    want, bound = _exact(x, w)
+    whole, out = _guarded(rows, outputs)
+    _linear(x, w, out, 0, tile)
+    err = (out.double() - want).abs()
+    assert (err <= HALF_ULP * want.abs() + 1.01 * bound).all()
+    assert (whole[0] == 1).all() and (whole[-1] == 1).all()
+
+
+@pytest.mark.parametrize("tile", [-1] + list(range(len(TILES))))
 def test_silu_mul_of_every_tile(tile):
     print(f"case linear silu tile={tile}", flush=True)
     bm, bn = TILES[tile] if tile >= 0 else (128, 128)
