@@ -2637,8 +2637,7 @@ constexpr int kWholeRowTolerance = 64;
 // 256 of 1536 and the others of 20 20.5 / 14.6.
 // Within the line single steps of the search remain, at worst 16 sequences, one of 1536 and the
 // others of 307, 14.9 / 13.5; of 1386 mixes of lengths 13 were more than 2.5 % behind.
-bool pieces_pay(int64_t rows, int64_t positions) {
-  const int64_t cus = compute_units();
+bool pieces_pay(int64_t rows, int64_t positions, int64_t cus) {
   if (rows > cus - cus / 4) return false;
   const bool idle = cus / rows * rows <= cus - cus / 4;   // with equal rows
   return rows * positions <=
@@ -2646,8 +2645,8 @@ bool pieces_pay(int64_t rows, int64_t positions) {
 }
 
 // Whether pieces are what a launch of that many rows takes if its table is not one of short rows.
-bool pieces_take(int64_t batch, int head_dim, int64_t rows, int64_t positions) {
-  return head_dim == 128 && batch <= 64 && pieces_pay(rows, positions);
+bool pieces_take(int64_t batch, int head_dim, int64_t rows, int64_t positions, int64_t cus) {
+  return head_dim == 128 && batch <= 64 && pieces_pay(rows, positions, cus);
 }
 
 // Whether the table rules out rows (of at most one per CU) that are not short: up to three
@@ -2870,14 +2869,14 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
   // / 7.5 us); else small launches go by pieces, and in others the balanced kernel
   // decides on the device.
   const int64_t all_rows = (int64_t)batch * num_kv_heads;
-  const int short_rows = chunk == 0 && (phases & NVJ_PHASE_SHORT_ROWS) &&
-                                 !(phases & NVJ_PHASE_SHARED_ROWS) && batch <= kKeptSequences &&
-                                 all_rows <= compute_units()
-                             ? (int)all_rows
-                             : 0;
+  const int64_t cus = chunk == 0 && (phases & NVJ_PHASE_SHORT_ROWS) &&
+                              !(phases & NVJ_PHASE_SHARED_ROWS) && batch <= kKeptSequences
+                          ? compute_units()
+                          : 0;
+  const int short_rows = all_rows <= cus ? (int)all_rows : 0;
   const int64_t positions = (int64_t)max_blocks * block_size;
   const bool by_pieces = short_rows > 0 && !valu && !loads_only &&
-                         pieces_take(batch, head_dim, all_rows, positions);
+                         pieces_take(batch, head_dim, all_rows, positions, cus);
   const bool all_short = short_rows > 0 && table_of_short_rows(all_rows, positions, by_pieces) &&
                          !(phases & NVJ_PHASE_CLEAR_COUNTERS);
   if ((whole || all_short) && max_blocks > 0) {
@@ -3212,13 +3211,15 @@ extern "C" int32_t nvj_paged_decode_store_takes(int32_t batch, int32_t num_heads
     return 0;
   const int64_t rows =
       (int64_t)batch * num_kv_heads * virtual_heads_per_cache_head(num_heads / num_kv_heads);
-  if (rows > compute_units()) return 0;
+  const int64_t cus = compute_units();
+  if (rows > cus) return 0;
   if (chunk == NVJ_CHUNK_WHOLE_SEQUENCE) return 1;
   if (chunk != 0 || nvj_paged_decode_counter_bytes(batch, num_heads, num_kv_heads) >
                         kNullStreamWords * sizeof(int32_t))
     return 0;
   const int64_t positions = (int64_t)max_blocks * block_size;
-  return table_of_short_rows(rows, positions, pieces_take(batch, head_dim, rows, positions)) ? 1 : 2;
+  return table_of_short_rows(rows, positions, pieces_take(batch, head_dim, rows, positions, cus)) ? 1
+                                                                                                  : 2;
 }
 
 extern "C" int nvj_paged_decode_store_launch(

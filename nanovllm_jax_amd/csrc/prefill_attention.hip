@@ -840,7 +840,8 @@ struct TileBound {
   bool small;
   int64_t tiles;
 };
-TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads) {
+TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads,
+                     int64_t cus) {
   // every sequence adds at most one partly filled token block and one partly filled tile
   const int64_t blocks = (tokens + 15 * batch) / 16;
   auto tiles_of = [&](int column_groups) {
@@ -848,7 +849,7 @@ TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
   };
   // one column group per wave while the larger workgroups would not fill the CUs: one prompt
   // of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1
-  const bool small = tiles_of(2 * kWaves) * num_kv_heads <= nvj::compute_units();
+  const bool small = tiles_of(2 * kWaves) * num_kv_heads <= cus;
   return {small, tiles_of((small ? 1 : 2) * kWaves)};
 }
 
@@ -858,20 +859,19 @@ TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
 // prompts of 4 tokens 48.6 / 44.1, 200 of up to 17 34.8 / 32.4, 500 of 9 104.9 / 98.5 (31, 59 and 61
 // pieces a share); from 80 pieces on -19 .. +2 %, with fewer rounds -22 .. -1 %.
 bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
-                 int64_t num_kv_heads) {
+                 int64_t num_kv_heads, int64_t cus) {
   const int64_t tiles =
-      tile_bound(tokens, batch, num_heads / num_kv_heads, num_kv_heads).tiles * num_kv_heads;
-  return tiles <= 6 * nvj::compute_units() || rows * num_kv_heads * kPieces >= 80 * tiles;
+      tile_bound(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus).tiles * num_kv_heads;
+  return tiles <= 6 * cus || rows * num_kv_heads * kPieces >= 80 * tiles;
 }
 
 // Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.
 constexpr int64_t kLongestFirstPerCu = 16;
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
-                   int32_t dtype) {
+                   int32_t dtype, int64_t cus) {
   if (((int64_t)total_q_tokens + 15) * a.group > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const int64_t cus = nvj::compute_units();
-  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group, a.num_kv_heads);
+  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group, a.num_kv_heads, cus);
   const bool small = bound.small;
   const int64_t tiles = bound.tiles;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
@@ -921,7 +921,7 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
                   int64_t kv_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                   void* out, int32_t total_q_tokens, int32_t batch, int32_t num_heads,
                   int32_t num_kv_heads, int32_t head_dim, float scale, int32_t dtype,
-                  const CacheRows* store) {
+                  const CacheRows* store, int64_t cus) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   if (total_q_tokens < 0 || batch < 0 || num_heads <= 0 || num_kv_heads <= 0)
     return NVJ_ERR_BAD_SHAPE;
@@ -960,7 +960,8 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
     a.row_pieces = (uint32_t)num_kv_heads * kPieces;
     a.new_pieces = (uint32_t)store->rows * a.row_pieces;
   }
-  return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype);
+  return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype,
+                        cus);
 }
 }  // namespace
 
@@ -971,7 +972,7 @@ extern "C" int nvj_prefill_attention_rows_launch(
     int32_t head_dim, float scale, int32_t dtype) {
   return launch_packed(stream, q, q_row_stride, k, v, kv_row_stride, cu_seqlens_q, cu_seqlens_k,
                        out, total_q_tokens, batch, num_heads, num_kv_heads, head_dim, scale, dtype,
-                       nullptr);
+                       nullptr, nvj::compute_units());
 }
 
 extern "C" int nvj_prefill_attention_store_launch(
@@ -991,17 +992,18 @@ extern "C" int nvj_prefill_attention_store_launch(
       return NVJ_ERR_ALIGNMENT;
   }
   const CacheRows rows = {slot_mapping, k_cache, v_cache, num_slots, num_rows};
+  const int64_t cus = nvj::compute_units();   // (asked for once: 70 ns of a call of 5 us)
   // the kernel counts the pieces of all rows in 32 bits
   const bool together = num_rows > 0 && total_q_tokens > 0 && batch > 0 &&
                         (int64_t)num_rows * num_kv_heads * kPieces <= UINT32_MAX - 4096 &&
-                        store_rides(total_q_tokens, num_rows, batch, num_heads, num_kv_heads);
+                        store_rides(total_q_tokens, num_rows, batch, num_heads, num_kv_heads, cus);
   if (!together && num_rows > 0) {
     const int code = store_alone();
     if (code != NVJ_OK) return code;
   }
   return launch_packed(stream, q, (int64_t)num_heads * kD, k, v, (int64_t)num_kv_heads * kD,
                        cu_seqlens_q, cu_seqlens_k, out, total_q_tokens, batch, num_heads,
-                       num_kv_heads, head_dim, scale, dtype, together ? &rows : nullptr);
+                       num_kv_heads, head_dim, scale, dtype, together ? &rows : nullptr, cus);
 }
 
 extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const void* k,
@@ -1056,5 +1058,6 @@ extern "C" int nvj_paged_prefill_attention_launch(
   a.block_size = block_size;
   a.max_blocks = max_blocks;
   a.num_blocks = num_blocks;
-  return launch_prefill(static_cast<hipStream_t>(stream), a, true, total_q_tokens, dtype);
+  return launch_prefill(static_cast<hipStream_t>(stream), a, true, total_q_tokens, dtype,
+                        nvj::compute_units());
 }
