@@ -2628,20 +2628,19 @@ constexpr int kWholeRowTolerance = 64;
 // streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.7 / 73.4, 64 rows of
 // 1000 .. 16000 53.5 / 55.8 and of 16000 .. 32768 145 / 138, 128 rows of 300 .. 4096 28.9 /
 // 30.2 and of 500 .. 8000 47.3 / 46.0.
-// Equal rows that leave a quarter of the workgroups idle (86 .. 96 rows) end earlier: 88 rows of
-// 3000 29.0 / 30.2, 96 of 3000 31.2 / 32.0 and of 4096 41.3 / 39.2, 88 of 5952 52.6 / 49.6.
+// Equal rows that leave a quarter of the workgroups idle are the worst within the line there: 96
+// of 4096 41.3 / 39.2, 88 of 5952 52.6 / 49.6; other lengths in the same tables are 9 .. 36 % less.
 // Beyond 128 rows the mean row has less than two pieces, and where long rows find none to spare
-// one workgroup walks all of a row: 144 rows of 1024 or 20 positions, a third of them long, 14.5 /
-// 14.1, 192 of 1024 equal 21.3 / 23.6; but a fifth of 144 short and the others 2048 long 31.9 /
-// 30.0, 136 of 2880 46.2 / 40.2, 224 of 832 or 20 15.1 / 14.0 and of 1536 or 20 24.1 / 18.8, 8 of
-// 256 of 1536 and the others of 20 20.5 / 14.6.
-// Within the line single steps of the search remain, at worst 16 sequences, one of 1536 and the
-// others of 307, 14.9 / 13.5; of 1386 mixes of lengths 13 were more than 2.5 % behind.
+// one workgroup walks all of a row.  1309 mixes of 130 .. 256 rows and 832 .. 1927 positions
+// (equal, evenly spread, one, a third, half or most of them long), by pieces / balanced: up to 192
+// rows 0.80 .. 0.91 in the mean and up to 1.11, to 224 rows 0.87 .. 0.91 and 1.25, to 256 rows
+// 0.95 .. 0.98 and 1.26.  168 rows of 1131 equal 22.8 / 25.2, 136 of 1927 or 20, a few long, 9.2 /
+// 13.2, 144 of 1536 or 20, most long, 25.6 / 23.4, 224 of 832 or 20, a third long, 15.1 / 14.0; but
+// 136 of 2880 equal 46.2 / 40.2, 224 of 1536 or 20, a third long, 24.1 / 18.8, 8 of 256 of 1536 and
+// the others of 20 20.5 / 14.6.
 bool pieces_pay(int64_t rows, int64_t positions, int64_t cus) {
-  if (rows > cus - cus / 4) return false;
-  const bool idle = cus / rows * rows <= cus - cus / 4;   // with equal rows
-  return rows * positions <=
-         (rows <= 64 ? 1 << 20 : rows > 128 ? 3 << 16 : idle ? 5 << 16 : 1 << 19);
+  if (rows > cus - cus / 8) return false;
+  return rows * positions <= (rows <= 64 ? 1 << 20 : rows <= 128 ? 1 << 19 : 1 << 18);
 }
 
 // Whether pieces are what a launch of that many rows takes if its table is not one of short rows.

@@ -1052,9 +1052,8 @@ def route_of_pieces(batch, kv_heads, max_blocks, bs, lens=None):
     import torch
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     rows, positions = batch * kv_heads, max_blocks * bs
-    most_idle = cus - cus // 4
-    pays = (1 << 20 if rows <= 64 else 0 if rows > most_idle else 3 << 16 if rows > 128 else
-            5 << 16 if cus // rows * rows <= most_idle else 1 << 19)
+    pays = (1 << 20 if rows <= 64 else 1 << 19 if rows <= 128 else
+            1 << 18 if rows <= cus - cus // 8 else 0)
     takes = batch <= 64 and rows * positions <= pays
     if rows > cus or batch > 256:
         return "balanced"
@@ -1080,7 +1079,8 @@ def route_of_pieces(batch, kv_heads, max_blocks, bs, lens=None):
     ([1000] * 9 + [20] * 15, 16, 8, "search"),    # the same with more heads
     ([1024, 1000, 800] + [20 * i for i in range(21)], 16, 8, "search"),
     ([7878] * 7, 32, 8, "search"),                # one longer than the mean fits: four pieces a row
-    ([4096] * 12, 16, 8, "balanced"),             # 96 equal rows would leave a quarter of the CUs idle
+    ([1500] + [20] * 31, 16, 8, "balanced"),      # no pieces to spare for a long row
+    ([1000, 900] + [70] * 26, 16, 8, "search"),   # the most rows that go by pieces
 ])
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 def test_rows_in_pieces(lens, Hq, Hkv, route, dtype):
