@@ -726,7 +726,7 @@ int step_of_many_rows(void* stream, const nvj_decoder_model& m, const nvj_decode
   }
   a.M = b.num_sequences;
   product(rows, m.embed, b.logits, m.vocab, m.hidden);
-  return nvj::linear(s, a) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
+  return nvj::linear(s, a, true) == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }
 
 }  // namespace

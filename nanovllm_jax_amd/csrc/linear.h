@@ -35,7 +35,9 @@ struct LinearArgs {
 // Whether the kernels can be given these sizes at all.
 bool linear_takes(int64_t m, int64_t n, int64_t k);
 
-hipError_t linear(hipStream_t s, LinearArgs a);            // bf16 rows
+// bf16 rows; `for_later`: no launch of this step reads them.  (An argument of the host alone: one
+// more field in LinearArgs and the QKV kernel loads its arguments in four pieces, 7.6 -> 8.3 us.)
+hipError_t linear(hipStream_t s, LinearArgs a, bool for_later = false);
 hipError_t linear_silu_mul(hipStream_t s, LinearArgs a);   // SiLU(gate) * up; N / 2 a multiple of 16
 hipError_t linear_qk_rope(hipStream_t s, LinearArgs a);    // QK-norm, RoPE, KV store
 // The reduction cut into `chains` interleaved runs of `run` steps of 32, summed in order:

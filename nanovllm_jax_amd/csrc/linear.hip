@@ -542,7 +542,9 @@ int best_shape(int64_t m, int64_t n, int k, int min_bn) {
 // Plain rows that go past the L2s.  Smaller outputs stay where a norm behind them finds them, larger
 // ones are written more slowly that way.  us with the norm behind, past the L2s / not: 1000 rows of
 // 1024 (2 MB) 13.0 / 12.7, 200 of 4096 16.2 / 15.6, 2048 of 1024 20.2 / 20.3, 2048 of 4096 34.9 /
-// 35.9, 3000 of 4096 44.7 / 45.3, 4268 of 4096 (35 MB) 65.1 / 61.7, 8192 of 4096 114 / 102.
+// 35.9, 3000 of 4096 44.7 / 45.3, 4268 of 4096 (35 MB) 65.1 / 61.7, 8192 of 4096 114 / 102.  Logits
+// always do, and the next step's weights stay where they are instead: a graph of 106 rows (32 MB
+// of them) 1849 / 1853, of 128 3389 / 3393.
 // (A flag of the kernel instead of a kernel of its own costs registers, and 1 .. 3 % of a large
 // product.)
 constexpr int64_t kPastL2From = 4 << 20, kPastL2To = 24 << 20;
@@ -576,12 +578,12 @@ bool linear_takes(int64_t m, int64_t n, int64_t k) {
          n * k * 2 < (1ll << 32) && m * n < (1ll << 40);
 }
 
-hipError_t linear(hipStream_t s, LinearArgs a) {
+hipError_t linear(hipStream_t s, LinearArgs a, bool for_later) {
   a.group_m = 8;   // 8 x 4 tiles at a time per XCD: 51 -> 42 us for 160 x 256 tiles at 4400 rows
   const int shape = a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0);
   const int64_t bytes = (int64_t)a.M * a.N * 2;
-  return bytes >= kPastL2From && bytes <= kPastL2To ? launch_shape<kRowsPastL2>(shape, s, a)
-                                                    : launch_shape<kPlain>(shape, s, a);
+  const bool past_l2 = for_later || (bytes >= kPastL2From && bytes <= kPastL2To);
+  return past_l2 ? launch_shape<kRowsPastL2>(shape, s, a) : launch_shape<kPlain>(shape, s, a);
 }
 hipError_t linear_silu_mul(hipStream_t s, LinearArgs a) {
   a.group_m = 8;
