@@ -372,6 +372,23 @@ __device__ __forceinline__ void probabilities_of_tile(f32x4 (&sc)[NG][2], bf16x8
   }
 }
 
+// x / d for 0 <= x < 2^31 as a multiplication (a division by a number only known at run time is 20
+// instructions and more, and a workgroup had eight of them in front of its first tile).  With
+// bits = ceil(log2 d) the multiplier m = ceil(2^(31 + bits) / d) has 32 bits, and x * m / 2^(31 +
+// bits) exceeds x / d by less than x / 2^31 / d: the whole part is the same.
+struct Divisor {
+  uint32_t multiplier, bits;
+  int32_t d;
+  Divisor() = default;
+  explicit Divisor(int64_t divisor) : bits(0), d((int32_t)divisor) {
+    while (((int64_t)1 << bits) < divisor) ++bits;
+    multiplier = (uint32_t)((((uint64_t)1 << (31 + bits)) + divisor - 1) / divisor);
+  }
+  __device__ __forceinline__ int divide(int x) const {
+    return (int)(__umulhi(2u * (uint32_t)x, multiplier) >> bits);
+  }
+};
+
 struct PrefillArgs {
   const uint4* q;       // Tq rows of Hq * 16 pieces, q_stride pieces apart
   const uint4* k;       // Tk rows of Hkv * 16 pieces, kv_row_bytes apart
@@ -381,7 +398,9 @@ struct PrefillArgs {
   const int32_t* cu_k;  // [B + 1]; paged: the keys of a sequence, cached and new together
   int64_t q_stride;
   uint32_t kv_row_bytes;   // < 2^24 (checked by the host)
-  int batch, num_heads, num_kv_heads, group;
+  int batch, num_heads, num_kv_heads;
+  Divisor group;        // num_heads / num_kv_heads
+  Divisor tiles;        // query tiles per KV head, at most
   float scale_log2e;
   // paged only: k and v are the caches [num_blocks, block_size, Hkv, 16] pieces
   const int32_t* block_tables;   // [B, max_blocks]
@@ -391,7 +410,8 @@ struct PrefillArgs {
   uint4* k_cache;
   uint4* v_cache;
   int64_t num_slots;
-  uint32_t row_pieces, new_pieces;   // of a row, of all rows
+  Divisor row_pieces;                // of a row
+  uint32_t new_pieces, share_pieces; // of all rows, of a workgroup
 };
 
 // A workgroup's share of the new rows on their way into the caches.  The attention reads the
@@ -410,9 +430,9 @@ struct StoreShare {
   // tiles of the same time read, and come out of a cache.  Whole heads, so that no two
   // workgroups write to one cache line (shares of 16 .. 64 pieces: 2 % of the launch).
   __device__ __forceinline__ StoreShare(const PrefillArgs& a) {
-    const uint64_t heads = a.new_pieces / kPieces;
-    at = kPieces * (uint32_t)(heads * (gridDim.x - 1 - blockIdx.x) / gridDim.x);
-    end = kPieces * (uint32_t)(heads * (gridDim.x - blockIdx.x) / gridDim.x);
+    const uint64_t from = (uint64_t)a.share_pieces * (gridDim.x - 1 - blockIdx.x);
+    at = (uint32_t)min(from, (uint64_t)a.new_pieces);
+    end = (uint32_t)min(from + a.share_pieces, (uint64_t)a.new_pieces);
     k0 = k1 = v0 = v1 = make_uint4(0u, 0u, 0u, 0u);
     slot0 = slot1 = -1;
   }
@@ -420,12 +440,15 @@ struct StoreShare {
     if (at >= end) return;
     const uint32_t p0 = min(at + threadIdx.x, end - 1);   // (past the end: the last one again)
     const uint32_t p1 = min(at + threadIdx.x + kBatch / 2, end - 1);
-    slot0 = a.slots[p0 / a.row_pieces];
-    slot1 = a.slots[p1 / a.row_pieces];
+    slot0 = a.slots[a.row_pieces.divide(p0)];
+    slot1 = a.slots[a.row_pieces.divide(p1)];
     k0 = a.k[p0];
     v0 = a.v[p0];
     k1 = a.k[p1];
     v1 = a.v[p1];
+  }
+  static __device__ __forceinline__ int64_t place(const PrefillArgs& a, int slot, uint32_t p) {
+    return (int64_t)slot * a.row_pieces.d + (p - a.row_pieces.divide(p) * a.row_pieces.d);
   }
   // (Nothing is stored past the end: hundreds of stores of one piece cost a workgroup with few
   // pieces 1 .. 2 us.)
@@ -433,12 +456,12 @@ struct StoreShare {
     if (at >= end) return;
     const uint32_t p0 = at + threadIdx.x, p1 = p0 + kBatch / 2;
     if (p0 < end && slot0 >= 0 && slot0 < a.num_slots) {
-      const int64_t dst = (int64_t)slot0 * a.row_pieces + p0 % a.row_pieces;
+      const int64_t dst = place(a, slot0, p0);
       store_past_l2(a.k_cache + dst, k0);
       store_past_l2(a.v_cache + dst, v0);
     }
     if (p1 < end && slot1 >= 0 && slot1 < a.num_slots) {
-      const int64_t dst = (int64_t)slot1 * a.row_pieces + p1 % a.row_pieces;
+      const int64_t dst = place(a, slot1, p1);
       store_past_l2(a.k_cache + dst, k1);
       store_past_l2(a.v_cache + dst, v1);
     }
@@ -458,6 +481,199 @@ struct NoShare {
   __device__ __forceinline__ void finish(const PrefillArgs&) const {}
 };
 
+// The query tile of a workgroup and its sequence.
+struct QueryTile {
+  int seq, kvh;
+  int c0;                                // its first column group of the sequence's
+  int q_base, len_q, k_first, k_count;   // of that sequence, from the loads of the search
+};
+
+// Query tiles are numbered sequence by sequence.  A wave looks at 64 * K sequences at a time, a
+// lane for each K neighbours, their offsets fetched in one round trip (a loop over the sequences
+// one by one cost a batch of 128 short prompts more than its tiles).  What a workgroup does in
+// front of its first tile is a chain of dependent instructions that nothing covers.  With a lane
+// for every fourth group of 64 instead, fetched and scanned group by group, and divisions as
+// divisions: 128 prompts of 16..300 tokens 122.9 us, now 115.2, 128 of 128 (32 / 8 heads) 87.1 / 79.2,
+// 300 of 4 (64 / 8) 44.9 / 38.3, one of 200 7.6 / 7.1, 8 of 4096 971 / 946.
+template <bool PAGED, int kColumnGroups, int K>
+struct SequenceTiles {
+  const PrefillArgs& a;
+  int first;            // sequence of this lane
+  int cq[K + 1], ck[K + 1];
+  int nt[K], mine;      // tiles of each, of all
+  int upto, total;      // tiles up to and including this lane's, of all lanes
+
+  __device__ __forceinline__ SequenceTiles(const PrefillArgs& args, int base, int lane)
+      : a(args), first(base + K * lane) {
+#pragma unroll
+    for (int j = 0; j <= K; ++j) {   // (behind the last sequence: empty ones)
+      const int s = min(first + j, a.batch);
+      cq[j] = a.cu_q[s];
+      ck[j] = a.cu_k[s];
+    }
+    mine = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      const uint32_t blocks = (uint32_t)(max(cq[j + 1] - cq[j], 0) + 15) / 16;
+      nt[j] = (int)((blocks * a.group.d + kColumnGroups - 1) / kColumnGroups);
+      mine += nt[j];
+    }
+    upto = wave_inclusive_scan(mine);
+    total = __builtin_amdgcn_readlane(upto, 63);
+  }
+  // Tile `tile` of sequence j of lane `src`.
+  __device__ __forceinline__ void take(int src, int j, int tile, QueryTile* t) const {
+    int q0 = cq[0], q1 = cq[1], k0 = ck[0], k1 = ck[1];
+#pragma unroll
+    for (int i = 1; i < K; ++i) {
+      if (j == i) {
+        q0 = cq[i];
+        q1 = cq[i + 1];
+        k0 = ck[i];
+        k1 = ck[i + 1];
+      }
+    }
+    t->seq = __builtin_amdgcn_readlane(first, src) + j;
+    t->c0 = tile * kColumnGroups;
+    t->q_base = __builtin_amdgcn_readlane(q0, src);
+    t->len_q = __builtin_amdgcn_readlane(q1, src) - t->q_base;
+    t->k_first = __builtin_amdgcn_readlane(k0, src);
+    t->k_count = __builtin_amdgcn_readlane(k1, src) - t->k_first;
+  }
+  // tile `id`, counted from `base` on; 0 <= id < total
+  __device__ __forceinline__ void by_sequence(int id, QueryTile* t) const {
+    const int src = __popcll(__ballot(upto <= id));   // lanes whose sequences end in front of it
+    int tile = id - __builtin_amdgcn_readlane(upto - mine, src), j = 0;
+#pragma unroll
+    for (int i = 0; i < K - 1; ++i) {
+      const int n = __builtin_amdgcn_readlane(nt[i], src);
+      if (j == i && tile >= n) {
+        tile -= n;
+        ++j;
+      }
+    }
+    take(src, j, tile, t);
+  }
+  // Behind cached prefixes of very different lengths the tiles are walked by the keys they
+  // have, most first: with few rounds of workgroups a long tile that starts late is what
+  // the launch waits for (16 sequences of 130..5600 keys 239 -> 222 us).  Where lengths
+  // are alike the order by sequence is the better one (the search costs 0.5 us per
+  // workgroup and neighbours no longer share their keys in L2: 12 prompts of 853..1475
+  // tokens 170 -> 177 us).
+  __device__ __forceinline__ int keys_of(int j) const {
+    return min(max(ck[j + 1] - ck[j], 0), a.max_blocks * a.block_size);
+  }
+  __device__ __forceinline__ bool uneven(int* longest) const {
+    int keys = 0, most = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (nt[j] > 0) {
+        const int n = keys_of(j);
+        most = max(most, max(n, cq[j + 1] - cq[j]));
+        keys += n >> 5;
+      }
+    keys = __builtin_amdgcn_readlane(wave_inclusive_scan(keys), 63);
+    *longest = wave_max(most);
+    return *longest >= 1024 && (int64_t)*longest * a.batch * 3 > (int64_t)keys * 128;
+  }
+  // No sort: the number of tiles that walk more than T keys is a sum over the sequences
+  // of a closed form, so item i is found by bisection of T.
+  __device__ __forceinline__ int beyond(int j, int T) const {   // tiles that walk more, of sequence j
+    const int len_q = cq[j + 1] - cq[j];
+    const int x = T - max(keys_of(j) - len_q, 0);   // the first tile past token x - 1 of the sequence
+    const int past = x < 0 ? 0 : x >= len_q ? nt[j] : (x >> 4) * a.group.d / kColumnGroups;
+    return max(nt[j] - past, 0);
+  }
+  __device__ __forceinline__ int count_beyond(int T) const {
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) n += beyond(j, T);
+    return __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
+  }
+  __device__ __forceinline__ void longest_first(int item, int longest, QueryTile* t) const {
+    constexpr int kLevel = 128;   // keys: tiles this close in length count as equal
+    // smallest level L with at most `item` tiles beyond (L + 1) * kLevel keys
+    int lo = 0, hi = longest / kLevel;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (count_beyond((mid + 1) * kLevel) <= item) hi = mid;
+      else lo = mid + 1;
+    }
+    const int before = count_beyond((lo + 1) * kLevel);
+    int above[K], level[K], sum = 0;   // tiles beyond the level and in it
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      above[j] = beyond(j, (lo + 1) * kLevel);
+      // level 0 takes everything that is left, tiles without any key included
+      level[j] = (lo == 0 ? nt[j] : beyond(j, lo * kLevel)) - above[j];
+      sum += level[j];
+    }
+    const int end = before + wave_inclusive_scan(sum);
+    const int src = __popcll(__ballot(end <= item));
+    int at = item - __builtin_amdgcn_readlane(end - sum, src), j = 0;
+    int last = __builtin_amdgcn_readlane(nt[0] - above[0], src) - 1;
+#pragma unroll
+    for (int i = 0; i < K - 1; ++i) {
+      const int n = __builtin_amdgcn_readlane(level[i], src);
+      if (j == i && at >= n) {
+        at -= n;
+        ++j;
+        last = __builtin_amdgcn_readlane(nt[i + 1] - above[i + 1], src) - 1;
+      }
+    }
+    take(src, j, last - at, t);   // the later tiles of a sequence walk more keys
+  }
+  // Item `item` of a KV head's list, all sequences being here; false beyond the real tiles.
+  __device__ __forceinline__ bool find(int item, bool may_sort, QueryTile* t) const {
+    if (item >= total) return false;
+    int longest;
+    if (PAGED && may_sort && uneven(&longest)) longest_first(item, longest, t);
+    else by_sequence(total - 1 - item, t);
+    return true;
+  }
+};
+
+// False when the workgroup has no tile.
+template <bool PAGED, int kColumnGroups>
+__device__ __forceinline__ bool find_query_tile(const PrefillArgs& a, bool may_sort, int lane,
+                                                QueryTile* t) {
+  // Work item -> workgroup, XCD-aware.  Consecutive workgroup ids land on
+  // different XCDs (8 of them, each with its own L2), so the work list is cut
+  // into 8 contiguous parts and workgroup id L takes item (L % 8) * part + L / 8:
+  // one XCD then walks neighbouring items.  Items are ordered (kv head, query
+  // tile): neighbours share the K/V rows of one (sequence, kv head), which stay
+  // in that XCD's L2 instead of being fetched by all eight.  Later tiles of a
+  // sequence have more keys to walk and come first.
+  // The work list is sized for a bound on the tiles, and the items beyond the real ones sit at its
+  // end, where they delay nothing.  The real tiles are walked from the last one down.
+  const int total_items = a.tiles.d * a.num_kv_heads;
+  const int part = (total_items + 7) / 8;
+  const int place = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
+  if (place >= total_items) return false;
+  t->kvh = a.tiles.divide(place);
+  const int item = place - t->kvh * a.tiles.d;
+  if (a.batch <= 64)
+    return SequenceTiles<PAGED, kColumnGroups, 1>(a, 0, lane).find(item, may_sort, t);
+  if (a.batch <= 128)
+    return SequenceTiles<PAGED, kColumnGroups, 2>(a, 0, lane).find(item, may_sort, t);
+  if (a.batch <= 256)
+    return SequenceTiles<PAGED, kColumnGroups, 4>(a, 0, lane).find(item, may_sort, t);
+  int real_tiles = 0;
+  for (int base = 0; base < a.batch; base += 256)
+    real_tiles += SequenceTiles<PAGED, kColumnGroups, 4>(a, base, lane).total;
+  if (item >= real_tiles) return false;
+  int id = real_tiles - 1 - item;
+  for (int base = 0; base < a.batch; base += 256) {
+    const SequenceTiles<PAGED, kColumnGroups, 4> tiles(a, base, lane);
+    if (id < tiles.total) {
+      tiles.by_sequence(id, t);
+      return true;
+    }
+    id -= tiles.total;
+  }
+  return false;   // (cannot happen: the item is a real tile)
+}
+
 // grid.x = 8 * ceil(tile bound * Hkv / 8) workgroups (see the work-item mapping below).
 // PAGED: keys and values come from the block-paged cache through block_tables,
 // sequence i has len_k = cu_k[i+1] - cu_k[i] keys, and its len_q query rows are the
@@ -468,7 +684,6 @@ struct NoShare {
 // STREAM: the output goes past the L2s.
 template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM>
 __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(PrefillArgs a,
-                                                                           int num_tiles_bound,
                                                                            bool may_sort) {
   constexpr int kColumnGroups = NG * kWaves;   // per workgroup
   __shared__ uint4 k_ring[kKStages * kTileBytes / 16];
@@ -479,167 +694,21 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   const int lane = tid & 63;
   const int r = lane & 15;
   const int kg = lane >> 4;
-  const const_i32_ptr cu_q = (const_i32_ptr)(uintptr_t)a.cu_q;
 
-  // Work item -> workgroup, XCD-aware.  Consecutive workgroup ids land on
-  // different XCDs (8 of them, each with its own L2), so the work list is cut
-  // into 8 contiguous parts and workgroup id L takes item (L % 8) * part + L / 8:
-  // one XCD then walks neighbouring items.  Items are ordered (kv head, query
-  // tile): neighbours share the K/V rows of one (sequence, kv head), which stay
-  // in that XCD's L2 instead of being fetched by all eight.  Later tiles of a
-  // sequence have more keys to walk and come first.
   std::conditional_t<STORE, StoreShare, NoShare> share(a);
-  const int total_items = num_tiles_bound * a.num_kv_heads;
-  const int part = (total_items + 7) / 8;
-  const int item = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
-  if (item >= total_items) {
+  QueryTile tile;
+  if (!find_query_tile<PAGED, kColumnGroups>(a, may_sort, lane, &tile)) {
     share.finish(a);
     return;
   }
-  const int kvh = item / num_tiles_bound;
-  const int in_kv = item - kvh * num_tiles_bound;
-  // Query tiles are numbered sequence by sequence.  A wave looks at 64 sequences
-  // at a time, one per lane, with the offsets of 256 sequences fetched together
-  // (one round trip per 256 sequences; a loop over the sequences one by one cost
-  // a batch of 128 short prompts more than its tiles).  First the real number of
-  // tiles: the work list was sized for a bound, and the items beyond the real
-  // tiles sit at its end, where they delay nothing.  The real tiles are walked
-  // from the last one down (the later tiles of a sequence have more keys).
-  const int group = a.group;
-  int nt4[4], incl4[4], qb4[4], ql4[4], kb4[4], kl4[4];
-  auto load_offsets = [&](int base) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      nt4[k] = incl4[k] = 0;
-      if (base + 64 * k < a.batch) {
-        const int s = min(base + 64 * k + lane, a.batch - 1);
-        qb4[k] = a.cu_q[s];
-        ql4[k] = a.cu_q[s + 1] - qb4[k];
-        kb4[k] = a.cu_k[s];
-        kl4[k] = a.cu_k[s + 1] - kb4[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (base + 64 * k < a.batch) {
-        nt4[k] = base + 64 * k + lane < a.batch
-                     ? ((max(ql4[k], 0) + 15) / 16 * group + kColumnGroups - 1) / kColumnGroups
-                     : 0;
-        incl4[k] = wave_inclusive_scan(nt4[k]);   // tiles up to and including this lane's sequence
-      }
-  };
-  int real_tiles = 0;
-  for (int base = 0; base < a.batch; base += 256) {
-    load_offsets(base);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) real_tiles += __builtin_amdgcn_readlane(incl4[k], 63);
-  }
-  if (in_kv >= real_tiles) {   // beyond the real number of tiles
-    share.finish(a);
-    return;
-  }
-  int seq = -1, c0 = 0;   // the sequence, its first column group of this tile
-  int q_base = 0, len_q = 0, k_first = 0, k_count = 0;   // of that sequence, from the same loads
-  auto take = [&](int base, int k, int src, int tile_of_seq) {
-    seq = base + 64 * k + src;
-    c0 = tile_of_seq * kColumnGroups;
-    q_base = __builtin_amdgcn_readlane(qb4[k], src);
-    len_q = __builtin_amdgcn_readlane(ql4[k], src);
-    k_first = __builtin_amdgcn_readlane(kb4[k], src);
-    k_count = __builtin_amdgcn_readlane(kl4[k], src);
-  };
-  // Behind cached prefixes of very different lengths the tiles are walked by the keys they
-  // have, most first: with few rounds of workgroups a long tile that starts late is what
-  // the launch waits for (16 sequences of 130..5600 keys 239 -> 222 us).  Where lengths
-  // are alike the order by sequence is the better one (the search costs 0.5 us per
-  // workgroup and neighbours no longer share their keys in L2: 12 prompts of 853..1475
-  // tokens 170 -> 177 us).
-  bool longest_first = false;
-  int longest = 0;
-  const int cap = PAGED ? a.max_blocks * a.block_size : 0;
-  if (PAGED && may_sort) {
-    int keys = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (64 * k < a.batch && nt4[k] > 0) {
-        const int n = min(max(kl4[k], 0), cap);
-        longest = max(longest, max(n, ql4[k]));
-        keys += n >> 5;
-      }
-    keys = __builtin_amdgcn_readlane(wave_inclusive_scan(keys), 63);
-    longest = wave_max(longest);
-    longest_first = longest >= 1024 && (int64_t)longest * a.batch * 3 > (int64_t)keys * 128;
-  }
-  if (PAGED && longest_first) {
-    // No sort: the number of tiles that walk more than T keys is a sum over the sequences
-    // of a closed form, so item i is found by bisection of T.
-    auto beyond = [&](int k, int T) {   // tiles of this lane's sequence in group k that walk more
-      const int off = max(min(max(kl4[k], 0), cap) - ql4[k], 0);
-      const int x = T - off;            // the first tile past token x - 1 of the sequence
-      const int first = x < 0 ? 0 : x >= ql4[k] ? nt4[k] : (x >> 4) * group / kColumnGroups;
-      return max(nt4[k] - first, 0);
-    };
-    auto count_beyond = [&](int T) {
-      int n = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (64 * k < a.batch) n += beyond(k, T);
-      return __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
-    };
-    constexpr int kLevel = 128;   // keys: tiles this close in length count as equal
-    // smallest level L with at most in_kv tiles beyond (L + 1) * kLevel keys
-    int lo = 0, hi = longest / kLevel;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (count_beyond((mid + 1) * kLevel) <= in_kv) hi = mid;
-      else lo = mid + 1;
-    }
-    int before = count_beyond((lo + 1) * kLevel);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (64 * k < a.batch && seq < 0) {
-        const int above = beyond(k, (lo + 1) * kLevel);
-        // level 0 takes everything that is left, tiles without any key included
-        const int mine = (lo == 0 ? nt4[k] : beyond(k, lo * kLevel)) - above;
-        const int incl = wave_inclusive_scan(mine);
-        const int at = before + incl - mine;
-        const unsigned long long hit = __ballot(mine > 0 && in_kv >= at && in_kv < at + mine);
-        if (hit != 0ull) {
-          const int src = __builtin_ctzll(hit);
-          // the later tiles of a sequence walk more keys
-          const int last = __builtin_amdgcn_readlane(nt4[k] - above, src) - 1;
-          take(0, k, src, last - (in_kv - __builtin_amdgcn_readlane(at, src)));
-        }
-        before += __builtin_amdgcn_readlane(incl, 63);
-      }
-    }
-  } else {
-    const int tile_id = real_tiles - 1 - in_kv;
-    int before = 0;   // tiles of the sequences in front of this group of 64
-    for (int base = 0; base < a.batch && seq < 0; base += 256) {
-      if (a.batch > 256) load_offsets(base);   // (a smaller batch is still in registers)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (base + 64 * k < a.batch && seq < 0) {
-          const int first = before + incl4[k] - nt4[k];
-          const unsigned long long hit =
-              __ballot(nt4[k] > 0 && tile_id >= first && tile_id < first + nt4[k]);
-          if (hit != 0ull) {
-            const int src = __builtin_ctzll(hit);
-            take(base, k, src, tile_id - __builtin_amdgcn_readlane(first, src));
-          }
-          before += __builtin_amdgcn_readlane(incl4[k], 63);
-        }
-      }
-    }
-  }
-  if (seq < 0) return;   // (cannot happen: the item is a real tile)
+  const int seq = tile.seq, kvh = tile.kvh, c0 = tile.c0, q_base = tile.q_base, len_q = tile.len_q;
+  const int k_first = tile.k_first, k_count = tile.k_count;
   share.fetch(a);
   const int k_base = PAGED ? 0 : k_first;
   const int len_k = PAGED ? min(max(k_count, 0), a.max_blocks * a.block_size) : max(k_count, 0);
   // key position of the first token: the new tokens are the tail of the sequence when paged
   const int off = PAGED ? max(len_k - len_q, 0) : 0;
-  const int token_end = min((c0 + kColumnGroups - 1) / group * 16 + 16, len_q);   // of the tile
+  const int token_end = min(a.group.divide(c0 + kColumnGroups - 1) * 16 + 16, len_q);   // of the tile
   const int k_end = min(len_k, off + token_end);   // keys [0, k_end) are visible to some row
   const int nsteps = (k_end + kKeys - 1) / kKeys;
 
@@ -650,8 +719,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const int c = c0 + NG * wave + g;
-    block0[g] = c / group * 16;
-    head[g] = kvh * group + c % group;
+    const int block = a.group.divide(c);
+    block0[g] = block * 16;
+    head[g] = kvh * a.group.d + (c - block * a.group.d);
     token[g] = block0[g] + r;
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
     const uint4* qrow = a.q + (int64_t)(q_base + min(token[g], len_q - 1)) * a.q_stride +
@@ -669,7 +739,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   const char* v_head =
       reinterpret_cast<const char*>(a.v + kvh * kPieces) + (int64_t)k_base * row_bytes;
   const const_i32_ptr table =
-      PAGED ? (const_i32_ptr)(uintptr_t)(a.block_tables + (int64_t)seq * a.max_blocks) : cu_q;
+      (const_i32_ptr)(uintptr_t)(PAGED ? a.block_tables + (int64_t)seq * a.max_blocks : a.cu_q);
 
   const lds_ptr k_lds = (lds_ptr)k_ring;
   const lds_ptr v_lds = (lds_ptr)v_ring;
@@ -870,15 +940,19 @@ constexpr int64_t kLongestFirstPerCu = 16;
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype, int64_t cus) {
-  if (((int64_t)total_q_tokens + 15) * a.group > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group, a.num_kv_heads, cus);
+  if (((int64_t)total_q_tokens + 15) * a.group.d > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
+  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group.d, a.num_kv_heads, cus);
   const bool small = bound.small;
   const int64_t tiles = bound.tiles;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
   const int64_t items = tiles * a.num_kv_heads;
   if (items > INT32_MAX - 8) return NVJ_ERR_BAD_SHAPE;
   const dim3 grid((unsigned)((items + 7) / 8 * 8)), block(kWaves * 64);
-  const int nt = (int)tiles;
+  a.tiles = Divisor(tiles);
+  if (a.slots) {   // whole heads, as many for each workgroup
+    const int64_t heads = a.new_pieces / kPieces;
+    a.share_pieces = (uint32_t)((heads + grid.x - 1) / grid.x * kPieces);
+  }
   const bool may_sort = paged && a.batch > 1 && a.batch <= 256 &&
                         items <= kLongestFirstPerCu * cus &&
                         (int64_t)a.max_blocks * a.block_size >= 1024;
@@ -886,7 +960,7 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
   const bool past_l2 = (int64_t)total_q_tokens * a.num_heads * (kD * 2) > kStreamOutBytes;
   hipError_t rc;
 #define NVJ_LAUNCH(F, P, N, S, T) \
-  rc = nvj::launch(prefill_attention_kernel<F, P, N, S, T>, grid, block, stream, a, nt, may_sort)
+  rc = nvj::launch(prefill_attention_kernel<F, P, N, S, T>, grid, block, stream, a, may_sort)
 #define NVJ_LAUNCH_TYPE(F)                                        \
   if (paged && small) NVJ_LAUNCH(F, true, 1, false, false);       \
   else if (paged && past_l2) NVJ_LAUNCH(F, true, 2, false, true); \
@@ -950,15 +1024,15 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
   a.batch = batch;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;
-  a.group = num_heads / num_kv_heads;
+  a.group = Divisor(num_heads / num_kv_heads);
   a.scale_log2e = scale * kLog2e;
   if (store) {
     a.slots = store->slots;
     a.k_cache = static_cast<uint4*>(store->k_cache);
     a.v_cache = static_cast<uint4*>(store->v_cache);
     a.num_slots = store->num_slots;
-    a.row_pieces = (uint32_t)num_kv_heads * kPieces;
-    a.new_pieces = (uint32_t)store->rows * a.row_pieces;
+    a.row_pieces = Divisor((int64_t)num_kv_heads * kPieces);
+    a.new_pieces = (uint32_t)store->rows * (uint32_t)a.row_pieces.d;
   }
   return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype,
                         cus);
@@ -993,9 +1067,9 @@ extern "C" int nvj_prefill_attention_store_launch(
   }
   const CacheRows rows = {slot_mapping, k_cache, v_cache, num_slots, num_rows};
   const int64_t cus = nvj::compute_units();   // (asked for once: 70 ns of a call of 5 us)
-  // the kernel counts the pieces of all rows in 32 bits
+  // the kernel counts the pieces of all rows in 31 bits
   const bool together = num_rows > 0 && total_q_tokens > 0 && batch > 0 &&
-                        (int64_t)num_rows * num_kv_heads * kPieces <= UINT32_MAX - 4096 &&
+                        (int64_t)num_rows * num_kv_heads * kPieces <= INT32_MAX - 4096 &&
                         store_rides(total_q_tokens, num_rows, batch, num_heads, num_kv_heads, cus);
   if (!together && num_rows > 0) {
     const int code = store_alone();
@@ -1052,7 +1126,7 @@ extern "C" int nvj_paged_prefill_attention_launch(
   a.batch = batch;
   a.num_heads = num_heads;
   a.num_kv_heads = num_kv_heads;
-  a.group = num_heads / num_kv_heads;
+  a.group = Divisor(num_heads / num_kv_heads);
   a.scale_log2e = scale * kLog2e;
   a.block_tables = block_tables;
   a.block_size = block_size;

@@ -45,6 +45,26 @@ def test_prefill_ragged_batch(Hq, Hkv):
         assert np.array_equal(got[cu_q[i]], np.repeat(v[cu_k[i]], G, axis=0))
 
 
+@pytest.mark.parametrize("batch,Hq,Hkv", [(1, 7, 7), (63, 6, 2), (64, 10, 2), (127, 3, 3),
+                                           (128, 12, 2), (129, 6, 2), (255, 5, 1), (256, 14, 2),
+                                           (257, 6, 2), (512, 3, 1), (513, 6, 2)])
+def test_prefill_finds_the_tiles_of_every_sequence(batch, Hq, Hkv):
+    """Batches at the edges of what the lanes of a wave hold (one, two or four sequences each, then
+    256 at a time), groups that are no power of two, empty sequences at both ends and beside each
+    other."""
+    print(f"case prefill lookup batch={batch} Hq={Hq} Hkv={Hkv}", flush=True)
+    from oracle.paged_attention_oracle import variable_length_attention_prefill_ref
+    rng = np.random.Generator(np.random.PCG64(900 + batch))
+    lens = rng.integers(0, 20, size=batch)
+    lens[rng.integers(0, batch, size=2)] = [140, 75]
+    if batch > 1:
+        lens[[0, 1, batch // 2, batch - 1]] = 0
+    lens = [int(x) for x in lens]
+    q, k, v, cu_q, cu_k = _problem(910 + batch, lens, lens, Hq, Hkv)
+    want = variable_length_attention_prefill_ref(q, k, v, cu_q, cu_k, 128 ** -0.5)
+    assert_close_bf16(run_hip(q, k, v, cu_q, cu_k, 128 ** -0.5), want, what=f"batch {batch}")
+
+
 @pytest.mark.parametrize("batch", [65, 130, 300, 600])
 def test_prefill_batches_of_many_short_prompts(batch):
     """More sequences than the 64 a wave looks at together, and than the 256 whose
