@@ -64,13 +64,13 @@ constexpr int kPieces = 16;          // 16-byte pieces per (position, head) row
 constexpr int kWaves = 4;
 constexpr int kKeys = 32;            // keys per step
 constexpr int kTileBytes = kKeys * kD * 2;   // one K or V tile in LDS: 32 rows of 256 bytes
-// Both rings hold 4 tiles, tile t in slot t % 4: iteration i reads K of tile i and
+// RING: tiles of K and of V in LDS.  4, tile t in slot t % 4: iteration i reads K of tile i and
 // V of tile i-1 while tiles i+1 (landing) and i+2 (just issued) are on their way.
 // A ring of 3 would do for K; 4 makes the slot of every tile of an iteration a
 // function of i % 4, so that a loop unrolled 4 times has every LDS offset as an
 // instruction immediate.
-constexpr int kKStages = 4;
-constexpr int kVStages = 4;
+// 3, fetched one tile ahead, with one column group per wave: three workgroups to a CU, for prompts
+// whose workgroups have little but their head and tail (tile_form).
 constexpr float kNegBig = -1.0e30f;
 constexpr float kLazyLog2 = 8.0f;    // running max moves only for gains above 2^8
 constexpr float kLog2e = 1.4426950408889634f;
@@ -554,16 +554,18 @@ struct SequenceTiles {
     }
     take(src, j, tile, t);
   }
-  // Behind cached prefixes of very different lengths the tiles are walked by the keys they
-  // have, most first: with few rounds of workgroups a long tile that starts late is what
-  // the launch waits for (16 sequences of 130..5600 keys 239 -> 222 us).  Where lengths
-  // are alike the order by sequence is the better one (the search costs 0.5 us per
-  // workgroup and neighbours no longer share their keys in L2: 12 prompts of 853..1475
-  // tokens 170 -> 177 us).
+  // With few rounds of workgroups a long tile that starts late is what the launch waits for: tiles
+  // are then walked by the keys they have, most first.  Behind cached prefixes where those are of
+  // very different lengths (16 sequences of 130..5600 keys 239 -> 222 us; where they are alike
+  // the order by sequence is the better one, as the search costs 0.5 us per workgroup and
+  // neighbours no longer share their keys in L2: 12 prompts of 853..1475 tokens 170 -> 177 us),
+  // packed prompts always (few tiles: launch_prefill).
   __device__ __forceinline__ int keys_of(int j) const {
-    return min(max(ck[j + 1] - ck[j], 0), a.max_blocks * a.block_size);
+    const int keys = max(ck[j + 1] - ck[j], 0);
+    return PAGED ? min(keys, a.max_blocks * a.block_size) : keys;
   }
-  __device__ __forceinline__ bool uneven(int* longest) const {
+  static constexpr int kLevel = 128;   // keys: tiles this close in length count as equal
+  __device__ __forceinline__ bool by_length(int* longest) const {
     int keys = 0, most = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j)
@@ -572,15 +574,17 @@ struct SequenceTiles {
         most = max(most, max(n, cq[j + 1] - cq[j]));
         keys += n >> 5;
       }
-    keys = __builtin_amdgcn_readlane(wave_inclusive_scan(keys), 63);
     *longest = wave_max(most);
+    if (!PAGED) return *longest > kLevel;
+    keys = __builtin_amdgcn_readlane(wave_inclusive_scan(keys), 63);
     return *longest >= 1024 && (int64_t)*longest * a.batch * 3 > (int64_t)keys * 128;
   }
   // No sort: the number of tiles that walk more than T keys is a sum over the sequences
   // of a closed form, so item i is found by bisection of T.
   __device__ __forceinline__ int beyond(int j, int T) const {   // tiles that walk more, of sequence j
     const int len_q = cq[j + 1] - cq[j];
-    const int x = T - max(keys_of(j) - len_q, 0);   // the first tile past token x - 1 of the sequence
+    // the first tile past token x - 1 of the sequence
+    const int x = T - (PAGED ? max(keys_of(j) - len_q, 0) : 0);
     const int past = x < 0 ? 0 : x >= len_q ? nt[j] : (x >> 4) * a.group.d / kColumnGroups;
     return max(nt[j] - past, 0);
   }
@@ -591,7 +595,6 @@ struct SequenceTiles {
     return __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
   }
   __device__ __forceinline__ void longest_first(int item, int longest, QueryTile* t) const {
-    constexpr int kLevel = 128;   // keys: tiles this close in length count as equal
     // smallest level L with at most `item` tiles beyond (L + 1) * kLevel keys
     int lo = 0, hi = longest / kLevel;
     while (lo < hi) {
@@ -627,8 +630,11 @@ struct SequenceTiles {
   __device__ __forceinline__ bool find(int item, bool may_sort, QueryTile* t) const {
     if (item >= total) return false;
     int longest;
-    if (PAGED && may_sort && uneven(&longest)) longest_first(item, longest, t);
-    else by_sequence(total - 1 - item, t);
+    // (packed prompts only with the larger workgroups, launch_prefill: the rest is shorter without)
+    if ((PAGED || kColumnGroups == 2 * kWaves) && may_sort && by_length(&longest))
+      longest_first(item, longest, t);
+    else
+      by_sequence(total - 1 - item, t);
     return true;
   }
 };
@@ -682,12 +688,14 @@ __device__ __forceinline__ bool find_query_tile(const PrefillArgs& a, bool may_s
 // from the start of the sequence as the reference's mask does.
 // STORE (packed only): the rows of k and v also go into the caches (StoreShare).
 // STREAM: the output goes past the L2s.
-template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM>
-__global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(PrefillArgs a,
-                                                                           bool may_sort) {
+template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM, int RING>
+__global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attention_kernel(
+    PrefillArgs a, bool may_sort) {
+  static_assert(RING == 4 || (RING == 3 && NG == 1), "tiles in LDS");
+  constexpr int kAhead = RING - 2;             // tiles fetched ahead
   constexpr int kColumnGroups = NG * kWaves;   // per workgroup
-  __shared__ uint4 k_ring[kKStages * kTileBytes / 16];
-  __shared__ uint4 v_ring[kVStages * kTileBytes / 16];
+  __shared__ uint4 k_ring[RING * kTileBytes / 16];
+  __shared__ uint4 v_ring[RING * kTileBytes / 16];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -769,11 +777,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   if (nsteps > 0) {
     // V "of tile -1" (probabilities are zero there, but 0 * NaN is not 0)
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-    uint4* v_before = v_ring + (kVStages - 1) * (kTileBytes / 16);
+    uint4* v_before = v_ring + (RING - 1) * (kTileBytes / 16);
     for (int p = tid; p < kTileBytes / 16; p += kWaves * 64) v_before[p] = zero;
     copier.issue(0, 0, 0);
-    copier.issue(1, 1, 1);
-    wait_tiles_in_flight<1>();
+    if (kAhead > 1) copier.issue(1, 1, 1);
+    wait_tiles_in_flight<kAhead - 1>();
   }
   __syncthreads();
 
@@ -804,10 +812,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   // only while it turns scores into probabilities (vector ALU work that the
   // other wave of the SIMD can overlap with its own matrix instructions).
   __builtin_amdgcn_s_setprio(1);
-#define NVJ_END_OF_TILE()       \
-  do {                          \
-    wait_tiles_in_flight<1>();  \
-    __syncthreads();            \
+#define NVJ_END_OF_TILE()               \
+  do {                                  \
+    wait_tiles_in_flight<kAhead - 1>(); \
+    __syncthreads();                    \
   } while (0)
   // a plain tile whose ring slots are known when the code is written: every LDS
   // offset is an immediate, the copies use the lanes' precomputed offsets
@@ -824,19 +832,26 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   // any tile, ring slots computed at run time
 #define NVJ_TILE(MASKED, i, row_limit, key_limit)                                            \
   do {                                                                                       \
-    scores_of_tile<F16, NG>(kaddr, ((i) & 3) * kTileBytes, qreg, sc);                            \
-    accumulate_tile<F16, NG>(vaddr, (((i) + 3) & 3) * kTileBytes, pb, acc, lacc);                \
+    if (RING == 3) copier.issue((i) + 1, slot(i, 1), slot(i, 1));                            \
+    scores_of_tile<F16, NG>(kaddr, slot(i, 0) * kTileBytes, qreg, sc);                       \
+    accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);          \
     __builtin_amdgcn_s_setprio(0);                                                           \
-    probabilities_of_tile<MASKED, F16, NG>(sc, pb, acc, lacc, m_run, mneg, sl2, kg, token,        \
-                                       row_limit, key_limit);                                \
+    probabilities_of_tile<MASKED, F16, NG>(sc, pb, acc, lacc, m_run, mneg, sl2, kg, token,   \
+                                           row_limit, key_limit);                            \
     __builtin_amdgcn_s_setprio(1);                                                           \
-    copier.issue((i) + 2, ((i) + 2) & 3, ((i) + 2) & 3);                                     \
+    if (RING == 4) copier.issue((i) + 2, slot(i, 2), slot(i, 2));                            \
+    third = slot(i, 1);                                                                      \
     NVJ_END_OF_TILE();                                                                       \
   } while (0)
 
+  int third = 0;   // a ring of 3: the slot of tile i
+  const auto slot = [&](int i, int ahead) {   // of tile i + ahead (of tile i - 1: ahead = RING - 1)
+    if (RING == 4) return (i + ahead) & 3;
+    return third + ahead < 3 ? third + ahead : third + ahead - 3;
+  };
   int i = 0;
   // four plain tiles at a time while the tiles they fetch (up to i + 5) are full ones
-  for (; i + 4 <= n_plain && i + 5 < nsteps - 1; i += 4) {
+  for (; RING == 4 && i + 4 <= n_plain && i + 5 < nsteps - 1; i += 4) {
     NVJ_PLAIN_TILE_AT(0, i);
     NVJ_PLAIN_TILE_AT(1, i + 1);
     NVJ_PLAIN_TILE_AT(2, i + 2);
@@ -849,9 +864,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   }
   // the last tile of the wave is still to be accumulated; its V stays in place
   // until the copies of two iterations from now
-  if (n_active > 0) accumulate_tile<F16, NG>(vaddr, ((i + 3) & 3) * kTileBytes, pb, acc, lacc);
+  if (n_active > 0) accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);
   for (; i < nsteps; ++i) {
-    copier.issue(i + 2, (i + 2) & 3, (i + 2) & 3);
+    copier.issue(i + kAhead, slot(i, kAhead), slot(i, kAhead));
+    third = slot(i, 1);
     NVJ_END_OF_TILE();
   }
   wait_tiles_in_flight<0>();   // copies past the last tile are still landing in LDS
@@ -904,23 +920,37 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
 // attention saves (0.4).
 constexpr int64_t kStreamOutBytes = 32 << 20;
 
-// The most query tiles that a launch can have, per KV head, and whether they are of one column
-// group per wave instead of two.
-struct TileBound {
-  bool small;
+// How a launch is cut: column groups per wave, tiles of K and V in LDS, and the most query tiles that
+// it can have, per KV head.
+struct TileForm {
+  int groups, ring;
   int64_t tiles;
 };
-TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads,
-                     int64_t cus) {
+TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
+                   bool paged) {
   // every sequence adds at most one partly filled token block and one partly filled tile
   const int64_t blocks = (tokens + 15 * batch) / 16;
   auto tiles_of = [&](int column_groups) {
     return (blocks * group + (column_groups - 1) * batch) / column_groups;
   };
-  // one column group per wave while the larger workgroups would not fill the CUs: one prompt
-  // of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of 70..90 tokens, 32 heads, 10.8 -> 9.1
-  const bool small = tiles_of(2 * kWaves) * num_kv_heads <= cus;
-  return {small, tiles_of((small ? 1 : 2) * kWaves)};
+  const int64_t wide = tiles_of(2 * kWaves), narrow = tiles_of(kWaves);
+  // One column group per wave while the larger workgroups would leave CUs idle or start a second
+  // round with little to do: one prompt of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of
+  // 70..90, 32 heads, 10.8 -> 9.1; up to 1.5 of them a CU, one prompt of 3000, 16 heads, 62 -> 50,
+  // of 1500, 32 heads, 35 -> 29, 8 of 30..200 behind 500..4000 82 -> 66 (two a CU: 79 .. 111 %).
+  if (wide * num_kv_heads * 2 <= cus * 3) return {1, 4, narrow};
+  // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
+  // Three small ones to a CU instead, us: 100 prompts of 4 tokens, 16 / 8 heads (2 groups) 11.1 ->
+  // 8.1, 200 of 16, 32 / 8 (4) 26.0 -> 22.3, 100 of 60, 32 / 32 (4) 67.4 -> 55.4, 60 of 20..60, 32 / 8
+  // (12) 17.1 -> 14.8, 40 of 100, 16 / 8 (14) 19.8 -> 17.6; 60 of 20..60, 16 / 8 (6) 10.7 -> 11.2, the
+  // only one slower.  Beyond that -13 .. +13 %, with 8 heads to a KV head (8 groups and more) -3 ..
+  // +18 %.  Behind cached prefixes, which they would fetch for fewer rows, three of them are
+  // no better than two (-1 .. +10 % against the larger ones), and two are up to 4 groups
+  // (100 prompts of 16 behind 200..800, 32 / 8, 48.4 -> 45.1; 32 / 32 188 -> 185).
+  const int64_t groups = (tokens + 16 * batch - 1) / (16 * batch) * group;   // of a mean prompt
+  if (groups <= 4) return {1, paged ? 4 : 3, narrow};
+  if (groups <= 14 && group <= 4 && !paged) return {1, 3, narrow};
+  return {2, 4, wide};
 }
 
 // Whether the store of new rows rides in the attention launch.  A share costs its workgroup about
@@ -931,19 +961,23 @@ TileBound tile_bound(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
 bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
                  int64_t num_kv_heads, int64_t cus) {
   const int64_t tiles =
-      tile_bound(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus).tiles * num_kv_heads;
+      tile_form(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus, false).tiles *
+      num_kv_heads;
   return tiles <= 6 * cus || rows * num_kv_heads * kPieces >= 80 * tiles;
 }
 
-// Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.
+// Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.  Packed
+// prompts of more than a round and at most 5 / 4: 8 of 500 tokens, 16 / 8 heads, 21.7 -> 19.7 us, 4
+// of 1000 31.0 -> 28.4, 2 of 1000, 32 / 8, 30.0 -> 27.1, 8 of 165..945 27.1 -> 27.0; with 4 a CU and
+// more -5 .. +12 %.
 constexpr int64_t kLongestFirstPerCu = 16;
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype, int64_t cus) {
   if (((int64_t)total_q_tokens + 15) * a.group.d > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const TileBound bound = tile_bound(total_q_tokens, a.batch, a.group.d, a.num_kv_heads, cus);
-  const bool small = bound.small;
-  const int64_t tiles = bound.tiles;
+  const TileForm form =
+      tile_form(total_q_tokens, a.batch, a.group.d, a.num_kv_heads, cus, paged);
+  const int64_t tiles = form.tiles;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
   const int64_t items = tiles * a.num_kv_heads;
   if (items > INT32_MAX - 8) return NVJ_ERR_BAD_SHAPE;
@@ -953,30 +987,44 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
     const int64_t heads = a.new_pieces / kPieces;
     a.share_pieces = (uint32_t)((heads + grid.x - 1) / grid.x * kPieces);
   }
-  const bool may_sort = paged && a.batch > 1 && a.batch <= 256 &&
-                        items <= kLongestFirstPerCu * cus &&
-                        (int64_t)a.max_blocks * a.block_size >= 1024;
+  const bool may_sort =
+      a.batch > 1 && a.batch <= 256 &&
+      (paged ? items <= kLongestFirstPerCu * cus && (int64_t)a.max_blocks * a.block_size >= 1024
+             : form.groups == 2 && items * 2 <= cus * 5);
   const bool f16 = dtype == NVJ_DTYPE_F16;
   const bool past_l2 = (int64_t)total_q_tokens * a.num_heads * (kD * 2) > kStreamOutBytes;
   hipError_t rc;
-#define NVJ_LAUNCH(F, P, N, S, T) \
-  rc = nvj::launch(prefill_attention_kernel<F, P, N, S, T>, grid, block, stream, a, may_sort)
-#define NVJ_LAUNCH_TYPE(F)                                        \
-  if (paged && small) NVJ_LAUNCH(F, true, 1, false, false);       \
-  else if (paged && past_l2) NVJ_LAUNCH(F, true, 2, false, true); \
-  else if (paged) NVJ_LAUNCH(F, true, 2, false, false);           \
-  else if (small && a.slots) NVJ_LAUNCH(F, false, 1, true, false); \
-  else if (small) NVJ_LAUNCH(F, false, 1, false, false);          \
-  else if (a.slots && past_l2) NVJ_LAUNCH(F, false, 2, true, true); \
-  else if (a.slots) NVJ_LAUNCH(F, false, 2, true, false);         \
-  else if (past_l2) NVJ_LAUNCH(F, false, 2, false, true);         \
-  else NVJ_LAUNCH(F, false, 2, false, false)
+#define NVJ_LAUNCH(F, P, N, S, T, R)                                                              \
+  rc = nvj::launch(prefill_attention_kernel<F, P, N, S, T, R>, grid, block, stream, a, may_sort)
+#define NVJ_LAUNCH_STREAM(F, P, N, S, R)           \
+  if (past_l2) NVJ_LAUNCH(F, P, N, S, true, R);    \
+  else NVJ_LAUNCH(F, P, N, S, false, R)
+#define NVJ_LAUNCH_PACKED(F, S)                       \
+  if (form.groups == 2) {                             \
+    NVJ_LAUNCH_STREAM(F, false, 2, S, 4);             \
+  } else if (form.ring == 3) {                        \
+    NVJ_LAUNCH_STREAM(F, false, 1, S, 3);             \
+  } else {                                            \
+    NVJ_LAUNCH(F, false, 1, S, false, 4);             \
+  }
+#define NVJ_LAUNCH_TYPE(F)                            \
+  if (paged && form.groups == 1) {                    \
+    NVJ_LAUNCH_STREAM(F, true, 1, false, 4);          \
+  } else if (paged) {                                 \
+    NVJ_LAUNCH_STREAM(F, true, 2, false, 4);          \
+  } else if (a.slots) {                               \
+    NVJ_LAUNCH_PACKED(F, true)                        \
+  } else {                                            \
+    NVJ_LAUNCH_PACKED(F, false)                       \
+  }
   if (f16) {
     NVJ_LAUNCH_TYPE(true);
   } else {
     NVJ_LAUNCH_TYPE(false);
   }
 #undef NVJ_LAUNCH_TYPE
+#undef NVJ_LAUNCH_PACKED
+#undef NVJ_LAUNCH_STREAM
 #undef NVJ_LAUNCH
   return rc == hipSuccess ? NVJ_OK : NVJ_ERR_LAUNCH;
 }

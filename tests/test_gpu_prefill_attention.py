@@ -65,6 +65,33 @@ def test_prefill_finds_the_tiles_of_every_sequence(batch, Hq, Hkv):
     assert_close_bf16(run_hip(q, k, v, cu_q, cu_k, 128 ** -0.5), want, what=f"batch {batch}")
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,dtype", [
+    ([33, 1, 0, 64, 20, 5, 32, 17, 31, 15] * 15 + [129, 300, 65], 32, 8, "bf16"),  # three workgroups
+    ([60, 16, 97, 1, 250] * 8, 32, 32, "f16"),                                     # to a CU
+    ([3] * 150 + [160, 0], 16, 8, "bf16"),
+    ([500, 433, 512, 0, 640, 1, 500, 700, 505], 16, 8, "bf16"),    # longest tiles first
+    ([1000, 999, 97], 32, 8, "f16"),
+])
+def test_prefill_is_the_same_however_a_launch_is_cut(lens, Hq, Hkv, dtype):
+    """Launches of many or uneven prompts have workgroups, rings and orders of their own; a row's
+    sums are in the same order in all of them: bit for bit as every prompt by itself."""
+    print(f"case prefill forms {len(lens)} prompts Hq={Hq} Hkv={Hkv} {dtype}", flush=True)
+    import torch
+    from nanovllm_jax_amd import variable_length_attention_prefill
+    dev, dt = "cuda:0", {"bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    g = torch.Generator(device=dev)
+    g.manual_seed(len(lens))
+    T = sum(lens)
+    q, k, v = (torch.randn(T, h, 128, generator=g, device=dev).to(dt) for h in (Hq, Hkv, Hkv))
+    cu = lambda n: torch.from_numpy(np.concatenate([[0], np.cumsum(n)]).astype(np.int32)).to(dev)
+    got = variable_length_attention_prefill(q, k, v, cu(lens), cu(lens))
+    at = np.concatenate([[0], np.cumsum(lens)])
+    for i, n in enumerate(lens):
+        part = slice(int(at[i]), int(at[i + 1]))
+        one = variable_length_attention_prefill(q[part], k[part], v[part], cu([n]), cu([n]))
+        assert torch.equal(got[part], one), f"prompt {i} of {n} tokens"
+
+
 @pytest.mark.parametrize("batch", [65, 130, 300, 600])
 def test_prefill_batches_of_many_short_prompts(batch):
     """More sequences than the 64 a wave looks at together, and than the 256 whose
