@@ -134,7 +134,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   size_t own_bytes = 0;
   // Without counters at hand (no workspace, another stream than the null stream) the split
   // takes a launch more; up to three rounds of a workgroup are shorter than that (1 or 2
-  // sequences of 768 positions 9.8 us without a split, 9.1 + 2.8 with it).
+  // sequences of 768 positions 9.4 us without a split, 7.7 .. 9.0 + 2.8 with it).
   if (chunk == 0 && args[11] == Py_None && stream != nullptr && batch * c.heads <= 16 &&
       max_blocks * c.page <= 768)
     chunk = NVJ_CHUNK_WHOLE_SEQUENCE;

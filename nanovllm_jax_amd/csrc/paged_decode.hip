@@ -43,6 +43,7 @@
 #include "bf16.h"
 #include "cache_rows.h"
 #include "device.h"
+#include "divisor.h"
 #include "launch.h"
 #include "nvj_paged_attn.h"
 #include "read_ahead.h"
@@ -211,7 +212,11 @@ struct DecodeArgs {
   // "virtual" KV heads of group = G / kv_rep query heads each (kv_rep = 1
   // otherwise); cache_kv_heads is the number of heads a cache row really holds.
   int num_heads, num_kv_heads, group, kv_rep, cache_kv_heads, block_size, max_blocks, num_blocks;
+  nvj::Divisor page;   // block_size
   float scale_log2e;
+  __device__ __forceinline__ int cache_head(int kvh) const {
+    return kv_rep == 1 ? kvh : kvh / kv_rep;
+  }
 };
 
 // The new K/V rows of the step, stored by the same launch (NEW kernels: head_dim 128, up to
@@ -268,13 +273,14 @@ __device__ __forceinline__ void store_new_row(const DecodeArgs& a, const NewRows
 // lane (r = lane & 15, kg = lane >> 4), m_run the maximum raw score and l_run
 // the sum of exp((score - m_run) * scale) of that head (the same in the four
 // lanes that share r).  Lanes with r >= group hold padding.
-// NEW: `new_slot` is new_slot_of_lane.
+// NEW: `new_slot` is new_slot_of_lane.  first_block: the first step's entry of the block table, if
+// the caller has it (>= 0).
 template <int D, bool F16, bool NEW = false>
 __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds, int b, int kvh,
                                                 int t0, int t1, int lane, f32x4 (&acc)[8],
                                                 float& m_run, float& l_run,
                                                 const NewRows* fresh = nullptr,
-                                                int new_slot = -1) {
+                                                int new_slot = -1, int first_block = -1) {
   using H = HeadDim<D>;
   const int r = lane & 15;   // MFMA row/column index inside a 16-wide tile
   const int kg = lane >> 4;  // MFMA k-group (which 8 of the 32 reduction slots)
@@ -304,28 +310,28 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
   }
 
   const uint32_t row_bytes = (uint32_t)a.cache_kv_heads * (D * 2);  // one position, all heads
-  const int64_t head_bytes = (int64_t)(kvh / a.kv_rep) * (D * 2);
+  const int64_t head_bytes = (int64_t)a.cache_head(kvh) * (D * 2);
   const const_i32_ptr table = as_constant(a.block_tables + (int64_t)b * a.max_blocks);
 
   // wave-uniform place of the first position of a step in the cache: its slot if NEW, else
   // its byte offset at once
-  auto step_place = [&](int step) -> int64_t {
+  auto step_place = [&](int step, int known) -> int64_t {
     const int ts = t0 + step * kStep;
-    const int page = ts / block_size;
-    const int phys = min(max(table[page], 0), num_blocks - 1);
+    const int page = a.page.divide(ts);
+    const int phys = min(max(known >= 0 ? known : table[page], 0), num_blocks - 1);
     const int64_t slot = (int64_t)phys * block_size + (ts - page * block_size);
     return NEW ? slot : slot * row_bytes + head_bytes;
   };
   auto offset_of = [&](int64_t place) { return NEW ? place * row_bytes + head_bytes : place; };
   // NEW: this KV head's piece of a new row
   auto fresh_piece = [&](int row, int piece) {
-    return ((int64_t)row * a.cache_kv_heads + kvh / a.kv_rep) * H::kPieces + piece;
+    return ((int64_t)row * a.cache_kv_heads + a.cache_head(kvh)) * H::kPieces + piece;
   };
 
   uint4 kreg[H::kKLoads], vreg[8];
   int64_t place;   // of the step at hand
   {
-    place = step_place(0);
+    place = step_place(0, first_block);
     const int64_t off = offset_of(place);
     const int last = min(kStep, t1 - t0) - 1;
     issue_k_loads<true, D>(kreg, k_cache + off, lane, last, row_bytes);
@@ -339,14 +345,14 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
 
   // the page lookup of a step is started two steps ahead, so that its latency
   // is not in front of the loads that need the address
-  int64_t place_ahead = nsteps > 1 ? step_place(1) : 0;
+  int64_t place_ahead = nsteps > 1 ? step_place(1, -1) : 0;
   for (int step = 0; step < nsteps; ++step) {
     const int nvalid = min(kStep, t1 - (t0 + step * kStep));
     const bool more = step + 1 < nsteps;
     const int64_t next_place = place_ahead, next_off = offset_of(next_place);
     int next_last = kStep - 1;
     if (more) next_last = min(kStep, t1 - (t0 + (step + 1) * kStep)) - 1;
-    if (step + 2 < nsteps) place_ahead = step_place(step + 2);
+    if (step + 2 < nsteps) place_ahead = step_place(step + 2, -1);
 
     // the new rows among this step's positions; the pieces of the first are asked for here
     // already, while the step's own loads are still on their way
@@ -615,11 +621,11 @@ __device__ __forceinline__ void compute_segment_valu(const DecodeArgs& a, uint4*
   const bool publisher = kg == 0 && (r & (16 / G - 1)) == 0;
 
   const uint32_t row_bytes = (uint32_t)a.cache_kv_heads * (D * 2);
-  const int64_t head_bytes = (int64_t)(kvh / a.kv_rep) * (D * 2);
+  const int64_t head_bytes = (int64_t)a.cache_head(kvh) * (D * 2);
   const const_i32_ptr table = as_constant(a.block_tables + (int64_t)b * a.max_blocks);
   auto step_base = [&](int step) -> int64_t {
     const int ts = t0 + step * kStep;
-    const int page = ts / block_size;
+    const int page = a.page.divide(ts);
     const int phys = min(max(table[page], 0), num_blocks - 1);
     return ((int64_t)phys * block_size + (ts - page * block_size)) * row_bytes + head_bytes;
   };
@@ -828,11 +834,11 @@ __device__ __forceinline__ void compute_segment_loads_only(const DecodeArgs& a, 
   const int block_size = a.block_size, num_blocks = a.num_blocks;
   const int nsteps = (t1 - t0 + kStep - 1) / kStep;
   const uint32_t row_bytes = (uint32_t)a.cache_kv_heads * (D * 2);
-  const int64_t head_bytes = (int64_t)(kvh / a.kv_rep) * (D * 2);
+  const int64_t head_bytes = (int64_t)a.cache_head(kvh) * (D * 2);
   const const_i32_ptr table = as_constant(a.block_tables + (int64_t)b * a.max_blocks);
   auto step_base = [&](int step) -> int64_t {
     const int ts = t0 + step * kStep;
-    const int page = ts / block_size;
+    const int page = a.page.divide(ts);
     const int phys = min(max(table[page], 0), num_blocks - 1);
     return ((int64_t)phys * block_size + (ts - page * block_size)) * row_bytes + head_bytes;
   };
@@ -919,7 +925,7 @@ __device__ __forceinline__ void write_output(const DecodeArgs& a, int b, int kvh
   }
 }
 
-// A row (or a piece of one) that the 8 waves of a workgroup have walked in 8 parts: every part
+// A row (or a piece of one) that the 8 waves of a workgroup have walked in up to 8 parts: every part
 // lies in the K tile of its wave as add_partial_from_lds expects it (park_part), and wave w
 // merges its eighth of the head dimensions (4 in every 32: dims 32 * kg + 8 * e + jd .. + 3 of
 // query head r in lane (r, kg), e = w / 2, jd = 4 * (w % 2)), each value by the recurrence of
@@ -941,7 +947,7 @@ __device__ __forceinline__ void park_part(uint4* tile, int lane, const f32x4 (&a
 template <int D, int TILE>
 __device__ __forceinline__ void merge_parts(const DecodeArgs& a, const uint4 (&k_tile)[8][TILE],
                                             int wave, int lane, float (&acc)[4], float& m_run,
-                                            float& l_run) {
+                                            float& l_run, int parts) {
   constexpr int STRIDE = D / 32 * 16;
   const int e = wave >> 1, jd = 4 * (wave & 1);
   float v[8][4], ml[8][2];
@@ -959,6 +965,7 @@ __device__ __forceinline__ void merge_parts(const DecodeArgs& a, const uint4 (&k
   for (int i = 0; i < 4; ++i) acc[i] = v[0][i];
 #pragma unroll
   for (int p = 1; p < 8; ++p) {
+    if (p >= parts) break;
     const float m_new = fmaxf(m_run, ml[p][0]);
     const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
     const float w = __builtin_amdgcn_exp2f((ml[p][0] - m_new) * a.scale_log2e);
@@ -1024,6 +1031,17 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_splitk_kernel(DecodeArgs
                         m_run, l_run);
 }
 
+// The steps [first, end) of part `part` of NPARTS: one each while there are no more steps than
+// parts (the first parts have one then, which leaves fewer to merge), else equal shares.
+struct PartOfSteps {
+  int first, end;
+};
+template <int NPARTS>
+__device__ __forceinline__ PartOfSteps part_of_steps(int part, int steps) {
+  if (steps <= NPARTS) return {min(part, steps), min(part + 1, steps)};
+  return {part * steps / NPARTS, (part + 1) * steps / NPARTS};
+}
+
 // Whole-sequence split: every sequence is finished inside one workgroup, so
 // there is no workspace and no second pass.  grid.x = batch * (num_kv_heads /
 // hpw), block = NW * 64.  Workgroup (b, head group hg) owns `hpw` KV heads of
@@ -1033,11 +1051,15 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_splitk_kernel(DecodeArgs
 // wave's K tile is free by then and exactly holds its 34 floats per lane) and
 // the wave of part 0 merges them and writes the output.  Meant for batches of
 // similar lengths: a workgroup's time follows its sequence's length.
+// With a handful of steps the instructions in front of the first load count: divisions by hpw, by
+// its number of parts and by the block size, five in a row, were 0.8 us and more of a launch (one
+// sequence of 100 positions 6.9 -> 5.3 us, of 300 8.7 -> 8.0).
 // VG < 0 selects the loads-only measurement variant; VG > 0 selects the
 // vector-ALU measurement variant for exactly VG query heads
 // per KV head (head_dim 128, bf16 only).
 template <int NW, int D, bool F16, int VG = 0, bool NEW = false>
 __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs a, int hpw,
+                                                                     nvj::Divisor groups,
                                                                      NewRows fresh, int batch) {
   using H = HeadDim<D>;
   __shared__ uint4 k_tile[NW][kStep * H::kLdsRowPieces];
@@ -1056,16 +1078,18 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int parts = NW / hpw;
-  const int groups = a.num_kv_heads / hpw;
-  const int b = blockIdx.x / groups;
-  const int hg = blockIdx.x - b * groups;
-  const int part = wave / hpw;
+  const int log_hpw = __builtin_ctz(hpw), parts = NW >> log_hpw;
+  const int b = groups.divide(blockIdx.x);
+  const int hg = blockIdx.x - b * groups.d;
+  const int part = wave >> log_hpw;
   const int kvh = hg * hpw + (wave - part * hpw);
   const int ctx = min(max(as_constant(a.context_lens)[b], 0), a.max_blocks * a.block_size);
   const int steps = (ctx + kStep - 1) / kStep;
-  const int s0 = (int)((int64_t)part * steps / parts);
-  const int s1 = (int)((int64_t)(part + 1) * steps / parts);
+  const bool all_merge = NW == 8 && hpw == 1;
+  const PartOfSteps mine =
+      all_merge ? part_of_steps<NW>(part, steps)
+                : PartOfSteps{part * steps * hpw / NW, (part + 1) * steps * hpw / NW};
+  const int s0 = mine.first, s1 = mine.end;
 
   f32x4 acc[8];
 #pragma unroll
@@ -1084,16 +1108,16 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_whole_kernel(DecodeArgs 
   }
   if (parts > 1) {
     // value v of lane l at float v * kLanesWithDims + l of the wave's tile
-    const bool all_merge = NW == 8 && hpw == 1;
-    if (part > 0 || all_merge) park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
+    const int parked = all_merge ? max(min(steps, NW), 1) : parts;   // (an empty row: zeros)
+    if ((part > 0 || all_merge) && part < parked) park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
     __syncthreads();
     if constexpr (NW == 8) {
       if (all_merge) {
         const int r = lane & 15, kg = lane >> 4;
         if (r >= a.group || 32 * kg >= D) return;
-        float mine[4];
-        merge_parts<D>(a, k_tile, wave, lane, mine, m_run, l_run);
-        write_eighth<D, F16>(a, b, kvh, wave, r, kg, mine, l_run);
+        float merged[4];
+        merge_parts<D>(a, k_tile, wave, lane, merged, m_run, l_run, parked);
+        write_eighth<D, F16>(a, b, kvh, wave, r, kg, merged, l_run);
         return;
       }
     }
@@ -1429,7 +1453,7 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& a, uint4* lds, int b
   write_output<D, F16>(a, b, kvh, lane, acc, l_run);
 }
 
-// One piece of a row: its 8 waves have left their parts in the K tiles (park_part).  A row of
+// One piece of a row: `parts` of its 8 waves have left a part in the K tiles (park_part).  A row of
 // one piece is written at once; else the workgroup publishes the merged piece in slot `slot`
 // and the one that comes last, of `pieces` whose slots lie `stride` apart from `slot0`,
 // merges them and writes the row.  All 8 waves do both, each for its eighth of the dims, and
@@ -1440,10 +1464,10 @@ template <int D, bool F16, int TILE>
 __device__ __forceinline__ void finish_piece(const DecodeArgs& a, const uint4 (&k_tile)[8][TILE],
                                              int* lds_flag, int32_t* stale, int32_t* counter, int b,
                                              int kvh, int slot, int slot0, int stride, int pieces,
-                                             int wave, int lane) {
+                                             int wave, int lane, int parts) {
   static_assert(D == 128, "four k-groups");
   float acc[4], m_run, l_run;
-  merge_parts<D>(a, k_tile, wave, lane, acc, m_run, l_run);
+  merge_parts<D>(a, k_tile, wave, lane, acc, m_run, l_run, parts);
   const int group = a.group;
   const int dims = 32 * (lane >> 4) + 4 * wave;   // first of the lane's four
   if (pieces == 1) {
@@ -1479,9 +1503,9 @@ __device__ __forceinline__ void finish_piece(const DecodeArgs& a, const uint4 (&
   __syncthreads();
   if (*lds_flag == 0) return;
   // A row of 16 lanes holds 16 / gp lane groups of gp >= group lanes; lane group lg merges pieces
-  // lg, lg + 16 / gp, ..., then the lane groups are merged.  Lanes of padding heads read a
-  // real record and are dropped.
-  const int gp = group > 8 ? 16 : group > 4 ? 8 : group > 2 ? 4 : group > 1 ? 2 : 1;
+  // lg, lg + 16 / gp, ..., then the lane groups are merged; up to four pieces need one group
+  // only, and no merge of groups.  Lanes of padding heads read a real record and are dropped.
+  const int gp = group > 8 || pieces <= 4 ? 16 : group > 4 ? 8 : group > 2 ? 4 : group > 1 ? 2 : 1;
   const int lane_groups = 16 / gp;
   const int lg = (lane & 15) / gp;
   const int r = min((lane & 15) - lg * gp, group - 1);
@@ -1890,16 +1914,40 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
   }
 }
 
+// x / d for 0 <= x, 0 < d, both below 2^20, as a handful of instructions: (x + 0.5) / d is at least
+// 0.5 / d away from a whole number, and its error less than x / d * 2^-21.5.
+__device__ __forceinline__ int divide_small(int x, int d) {
+  return (int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+__device__ __forceinline__ int divide_small_up(int x, int d) { return divide_small(x + d - 1, d); }
+
+// The shortest piece, in steps.  A step less is 0.2 us less of one wave's chain, and pieces of fewer
+// than 8 steps leave waves idle but have fewer parts to put together and let more CUs draw a row;
+// yet each piece is a partial more for the one that merges them.  So a row gets up to `enough` pieces:
+// 12, or what is merged in one round of loads, 8 with more than 4 query heads a KV head and 4 with
+// more than 8; but no piece is longer than 8 steps, one a wave, while there are workgroups.  us,
+// one sequence, 8 KV heads, at most 8 / 12 / 16 / 32 pieces a row: 768 positions 7.82 / 7.72 / 7.73 /
+// 7.70 (in pieces of 8 steps 8.75, of one 8.81), 1500 8.97 / 8.42 / 8.56 / 9.22, 2048 9.14 / 8.89 /
+// 8.91 / 10.21; 64 query heads at most 8 / 12, 1087 positions 8.81 / 9.76, 2 sequences of 1325 9.55 /
+// 10.99.  Where a wave has more than a step, the longest of a workgroup has as many as in a piece
+// of the next multiple of 8: that is taken if it leaves more than enough pieces (11101 positions in
+// 22 of 16 steps 13.55, in 32 of 11 14.03; 3 of 3400, 64 query heads, 7 of 16 14.06, 10 of 11 14.45).
+constexpr int kShortestPiece = 2;
+constexpr int kHeldEntries = 4;   // registers of a wave for the block table
+
 // Pieces: every row (sequence, KV head) on workgroups of its own, as many as there are, for
-// launches of few and short rows, where what counts is the chain of round trips.  A row is
-// cut into pieces of equal length, in multiples of one 32-position step for each of the 8
-// waves, the shortest that leave no more pieces than workgroups; the waves of a
-// workgroup walk a piece in equal shares and put it together in LDS.
-// grid.x = max_pieces workgroups (and those that store new rows), block = 512.
+// launches of few and short rows, where what counts is the chain of round trips and the
+// instructions between them (a wave issues one in 4.5 to 9 cycles here).  A row is cut into
+// pieces of equal length to a step, about the shortest that leave no more pieces than `most`
+// per KV head; the waves of a workgroup walk a piece in equal shares and put it together in LDS.
+// Pieces in multiples of 8 steps, found by bisection, with divisions in front of the first load
+// and the block table behind the lengths were 9.06 us for one sequence of 768 positions and 8 KV
+// heads, 12.3 for 8 of 100 .. 1500, 9.4 for 8 of 100 .. 900 and 21.0 for 16 of 100 .. 2000; now 7.67,
+// 11.0, 8.2 and 19.8.
+// grid.x = main_wgs >= most * KV heads workgroups (and those that store new rows), block = 512.
 template <bool F16, bool NEW>
 __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, int batch,
-                                                                  int max_pieces,
-                                                                  int32_t* counters,
+                                                                  int most, int32_t* counters,
                                                                   NewRows fresh) {
   constexpr int D = 128, NW = 8;
   using H = HeadDim<D>;
@@ -1920,8 +1968,18 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int cap = a.max_blocks * a.block_size;
-  // the lengths, one sequence per lane (the host sees to it that there are no more)
-  const int ctx_here = lane < batch ? min(max(a.context_lens[lane], 0), cap) : 0;
+  // the lengths, one sequence per lane (the host sees to it that there are no more), and with
+  // them a small block table, so that the wave's first load need not wait for another one
+  const int len_here = a.context_lens[min(lane, batch - 1)];
+  const int64_t entries = (int64_t)batch * a.max_blocks;
+  int held[kHeldEntries] = {};
+  if (entries <= 64 * kHeldEntries) {
+#pragma unroll
+    for (int i = 0; i < kHeldEntries; ++i)
+      if (i == 0 || entries > 64 * i)
+        held[i] = a.block_tables[min(64 * i + lane, (int)entries - 1)];
+  }
+  const int ctx_here = lane < batch ? min(max(len_here, 0), cap) : 0;
   const int steps_here = (ctx_here + kStep - 1) / kStep;
   const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(steps_here), 63);
   if (g < batch && __builtin_amdgcn_readlane(ctx_here, g & 63) <= 0) {
@@ -1930,28 +1988,28 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
     for (int i = threadIdx.x; i < a.num_heads * H::kPieces; i += NW * 64)
       orow[i] = make_uint4(0u, 0u, 0u, 0u);
   }
-  // `rounds` of NW steps per piece: the smallest number that fits, between the mean and the
-  // longest row (one piece a row, which fits: the host sees to it).
-  const int most = max_pieces / a.num_kv_heads;   // pieces of all sequences, per KV head
-  int incl = 0, number = 0;
-  auto fits = [&](int rounds) __attribute__((always_inline)) {
-    number = (int)((uint32_t)(steps_here + NW * rounds - 1) / (uint32_t)(NW * rounds));
-    incl = wave_inclusive_scan(number);
-    return __builtin_amdgcn_readlane(incl, 63) <= most;
-  };
-  int lo = max(1, (total + NW * most - 1) / (NW * most));
-  if (!fits(lo)) {
-    int hi = (wave_max(steps_here) + NW - 1) / NW;
-    ++lo;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (fits(mid)) hi = mid;
-      else lo = mid + 1;
-    }
-    (void)fits(lo);
-  }
+  // Steps per piece.  ceil(total / (most - rows)) always fits, as a row has at most one piece
+  // more than its share (with a row for every piece, so does `total`); two shorter lengths are
+  // tried with it, in one scan of three counts of 10 bits (none exceeds most + 64): the least
+  // there can be, and one between.  (A search by bisection found the shortest, at a scan and a
+  // division per try: 1.1 us of 8 ragged sequences' 12.3.)
+  const int rows = __popcll(__ballot(steps_here > 0));
+  const int enough = max(rows, 1) * (a.group > 8 ? 4 : a.group > 4 ? 8 : 12);
+  const int shortest = min(max(divide_small_up(total, enough), kShortestPiece), NW);
+  const int length2 = max(shortest, divide_small_up(total, max(most - rows, 1)));
+  const int length1 = max(shortest, divide_small_up(total, most - rows / 2));
+  int length0 = max(shortest, divide_small_up(total, most));
+  if (length0 > NW && most > enough) length0 = (length0 + NW - 1) / NW * NW;
+  const int n0 = divide_small_up(steps_here, length0), n1 = divide_small_up(steps_here, length1);
+  const int n2 = divide_small_up(steps_here, length2);
+  const int counts = wave_inclusive_scan(n0 | n1 << 10 | n2 << 20);
+  const int all = __builtin_amdgcn_readlane(counts, 63);
+  const int pick = (all & 1023) <= most ? 0 : (all >> 10 & 1023) <= most ? 10 : 20;
+  const int number = pick == 0 ? n0 : pick == 10 ? n1 : n2;
+  const int incl = counts >> pick & 1023;
   // workgroup g: KV head g % heads of piece g / heads of them all
-  const int at = g / a.num_kv_heads, kvh = g - at * a.num_kv_heads;
+  const int at = __builtin_amdgcn_readfirstlane(divide_small(g, a.num_kv_heads));
+  const int kvh = g - at * a.num_kv_heads;
   const unsigned long long hit = __ballot(at < incl);
   if (hit == 0ull) return;
   const int b = __builtin_ctzll(hit);
@@ -1960,19 +2018,32 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
   const int ctx = __builtin_amdgcn_readlane(ctx_here, b);
   const int nb = __builtin_amdgcn_readlane(steps_here, b);
   const int piece = at - first;
-  const int s0 = piece * nb / pieces, s1 = (piece + 1) * nb / pieces;
-  const int w0 = s0 + wave * (s1 - s0) / NW, w1 = s0 + (wave + 1) * (s1 - s0) / NW;
+  const int share = __builtin_amdgcn_readfirstlane(divide_small(nb, pieces));
+  const int more = nb - share * pieces;   // the first pieces take a step more
+  const int s0 = piece * share + min(piece, more), steps = share + (piece < more);
+  const int parts = min(steps, NW);
+  const PartOfSteps mine = part_of_steps<NW>(wave, steps);
+  const int w0 = s0 + mine.first, w1 = s0 + mine.end;
+  int first_block = -1;
+  if (entries <= 64 * kHeldEntries && w1 > w0) {
+    const int at = b * a.max_blocks + a.page.divide(w0 * kStep);
+    int entry = held[0];
+#pragma unroll
+    for (int i = 1; i < kHeldEntries; ++i)
+      if (at >> 6 == i) entry = held[i];
+    first_block = max(__builtin_amdgcn_readlane(entry, at & 63), 0);
+  }
   f32x4 acc[8];
 #pragma unroll
   for (int jd = 0; jd < 8; ++jd) acc[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = kNegBig, l_run = 0.f;
   if (w1 > w0)
     compute_segment<D, F16, NEW>(a, k_tile[wave], b, kvh, w0 * kStep, min(ctx, w1 * kStep), lane,
-                                 acc, m_run, l_run, &fresh, new_slot);
-  park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
+                                 acc, m_run, l_run, &fresh, new_slot, first_block);
+  if (wave < parts) park_part<D>(k_tile[wave], lane, acc, m_run, l_run);
   __syncthreads();
   finish_piece<D, F16>(a, k_tile, &last, counters, counters + 1 + b * a.num_kv_heads + kvh, b, kvh,
-                       g, first * a.num_kv_heads + kvh, a.num_kv_heads, pieces, wave, lane);
+                       g, first * a.num_kv_heads + kvh, a.num_kv_heads, pieces, wave, lane, parts);
 }
 
 // grid.x = num_wgs, block = 512.  `min_steps`: fewest steps a sub-run may have
@@ -2621,20 +2692,20 @@ constexpr int kWholeRowTolerance = 64;
 // Whether a launch of at most one row per CU goes by pieces (paged_decode_pieces_kernel), from
 // what the table can hold; else the balanced kernel looks at the lengths.  Pieces save what
 // the balanced kernel's larger head and its merges by single waves cost a small launch, 3 us:
-// by pieces / balanced, 1 .. 4 sequences of 1000 positions and 8 KV heads 8.9 .. 10.2 / 12.2 ..
-// 13.3 us, 8 of 100 .. 900 9.9 / 12.9, 8 of 128 .. 2048 13.8 / 14.7, 4 of 4096 17.0 / 20.2.
+// by pieces / balanced, 1 .. 4 sequences of 1000 positions and 8 KV heads 8.3 .. 9.2 / 11.9 ..
+// 12.8 us, 8 of 100 .. 900 8.6 / 13.0, 8 of 128 .. 2048 11.1 / 14.4, 4 of 4096 15.4 / 19.6.
 // Against that a row is cut into whole pieces of one length for all rows, which leaves
 // workgroups idle when lengths differ and rows are many, and one KV head per workgroup
-// streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.7 / 73.4, 64 rows of
-// 1000 .. 16000 53.5 / 55.8 and of 16000 .. 32768 145 / 138, 128 rows of 300 .. 4096 28.9 /
-// 30.2 and of 500 .. 8000 47.3 / 46.0.
-// Equal rows that leave a quarter of the workgroups idle are the worst within the line there: 96
-// of 4096 41.3 / 39.2, 88 of 5952 52.6 / 49.6; other lengths in the same tables are 9 .. 36 % less.
+// streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.0 / 72.8, 64 rows of
+// 1000 .. 16000 52.2 / 54.2 and of 16000 .. 32768 137.3 / 137.2, 128 rows of 300 .. 4096 28.7 /
+// 29.9 and of 500 .. 8000 45.4 / 45.5; equal rows that leave a quarter of the workgroups idle are
+// the worst within the line there: 96 of 4096 37.5 / 39.5, 88 of 5952 50.0 / 50.1.
 // Beyond 128 rows the mean row has less than two pieces, and where long rows find none to spare
 // one workgroup walks all of a row.  1309 mixes of 130 .. 256 rows and 832 .. 1927 positions
 // (equal, evenly spread, one, a third, half or most of them long), by pieces / balanced: up to 192
 // rows 0.80 .. 0.91 in the mean and up to 1.11, to 224 rows 0.87 .. 0.91 and 1.25, to 256 rows
-// 0.95 .. 0.98 and 1.26.  168 rows of 1131 equal 22.8 / 25.2, 136 of 1927 or 20, a few long, 9.2 /
+// 0.95 .. 0.98 and 1.26 (with pieces of 8 steps; 168 rows of 1131 equal were 22.8 / 25.2 then and
+// are 21.0 / 23.5, 224 of them 27.0 / 27.0).  136 of 1927 or 20, a few long, 9.2 /
 // 13.2, 144 of 1536 or 20, most long, 25.6 / 23.4, 224 of 832 or 20, a third long, 15.1 / 14.0; but
 // 136 of 2880 equal 46.2 / 40.2, 224 of 1536 or 20, a third long, 24.1 / 18.8, 8 of 256 of 1536 and
 // the others of 20 20.5 / 14.6.
@@ -2657,9 +2728,10 @@ bool pieces_take(int64_t batch, int head_dim, int64_t rows, int64_t positions, i
 // (At 1024 equal lengths the balanced kernel is still 2 .. 5 us behind; lengths that differ
 // have not been measured there.)
 // Where pieces are the other choice, up to 128 rows, the third round is theirs: without a
-// split / by pieces, at 512 positions 1 .. 64 rows 8.2 .. 9.8 / 9.0 .. 10.0, 128 rows 10.6 / 10.4,
-// 256 rows 13.2 / 13.9; at 768 1 .. 16 rows 9.7 .. 9.9 / 9.0 .. 9.1, 64 rows 13.6 / 10.5, 128 rows
-// 13.7 / 13.2, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
+// split / by pieces, at 288 positions 1 .. 64 rows 7.2 .. 8.0 / 7.0 .. 9.9, at 512 1 .. 32 rows 8.0
+// .. 8.7 / 7.2 .. 10.3 (the more, the more query heads share a KV head), 64 rows 8.5 .. 9.7 / 8.1 ..
+// 9.0, 128 rows 9.9 / 10.4; at 768 1 .. 16 rows 9.4 .. 9.9 / 7.7 .. 9.0, 64 rows 11.3 .. 12.1 /
+// 9.1, 128 rows 13.3 / 13.0, and, with pieces of 8 steps, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
 bool table_of_short_rows(int64_t rows, int64_t positions, bool pieces) {
   return positions <= (pieces && rows <= 128 ? 2 : 3) * 8 * kStep;
 }
@@ -2858,6 +2930,7 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
   a.kv_rep = kv_rep;
   a.cache_kv_heads = cache_kv_heads;
   a.block_size = block_size;
+  a.page = nvj::Divisor(block_size);
   a.max_blocks = max_blocks;
   a.num_blocks = num_blocks;
   a.scale_log2e = scale * kLog2e;
@@ -2887,7 +2960,8 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
     const NewRows fresh = rows_behind(new_rows, batch * (num_kv_heads / hpw), batch, &grid);
     hipError_t rc;
 #define NVJ_LAUNCH_WHOLE(...) \
-  rc = nvj::launch(paged_decode_whole_kernel<8, __VA_ARGS__>, grid, block, s, a, hpw, fresh, batch)
+  rc = nvj::launch(paged_decode_whole_kernel<8, __VA_ARGS__>, grid, block, s, a, hpw,     \
+                   nvj::Divisor(num_kv_heads / hpw), fresh, batch)
     if (new_rows && f16) NVJ_LAUNCH_WHOLE(128, true, 0, true);
     else if (new_rows) NVJ_LAUNCH_WHOLE(128, false, 0, true);
     else if (loads_only) NVJ_LAUNCH_WHOLE(128, false, -1);
@@ -2924,13 +2998,14 @@ int launch_decode(void* stream, const void* q, const void* k_cache, const void* 
       if (!(phases & NVJ_PHASE_SPLITK)) return NVJ_OK;
       dim3 grid;
       if (by_pieces) {
-        const int64_t rounds = (positions + 8 * kStep - 1) / (8 * kStep);
-        const int max_pieces = (int)std::min<int64_t>(all_rows * rounds, compute_units());
-        const NewRows fresh = rows_behind(new_rows, max_pieces, batch, &grid);
+        const int64_t per_row =
+            (positions + kShortestPiece * kStep - 1) / (kShortestPiece * kStep);
+        const int most = (int)std::min<int64_t>(batch * per_row, cus / num_kv_heads);
+        const NewRows fresh = rows_behind(new_rows, most * num_kv_heads, batch, &grid);
         hipError_t rc;
 #define NVJ_LAUNCH_PIECES(...)                                                                \
   rc = nvj::launch(paged_decode_pieces_kernel<__VA_ARGS__>, grid, dim3(512), s, a, batch,     \
-                   max_pieces, counters, fresh)
+                   most, counters, fresh)
         if (new_rows && f16) NVJ_LAUNCH_PIECES(true, true);
         else if (new_rows) NVJ_LAUNCH_PIECES(false, true);
         else if (f16) NVJ_LAUNCH_PIECES(true, false);

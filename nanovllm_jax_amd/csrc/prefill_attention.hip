@@ -40,6 +40,7 @@
 
 #include "bf16.h"
 #include "device.h"
+#include "divisor.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "nvj_paged_attn.h"
@@ -49,6 +50,7 @@
 namespace {
 
 using nvj::bf16x8;
+using nvj::Divisor;
 using nvj::f16x8;
 using nvj::f32x4;
 using nvj::store_past_l2;
@@ -371,23 +373,6 @@ __device__ __forceinline__ void probabilities_of_tile(f32x4 (&sc)[NG][2], bf16x8
     pb[g] = as_bf16x8(pbits);
   }
 }
-
-// x / d for 0 <= x < 2^31 as a multiplication (a division by a number only known at run time is 20
-// instructions and more, and a workgroup had eight of them in front of its first tile).  With
-// bits = ceil(log2 d) the multiplier m = ceil(2^(31 + bits) / d) has 32 bits, and x * m / 2^(31 +
-// bits) exceeds x / d by less than x / 2^31 / d: the whole part is the same.
-struct Divisor {
-  uint32_t multiplier, bits;
-  int32_t d;
-  Divisor() = default;
-  explicit Divisor(int64_t divisor) : bits(0), d((int32_t)divisor) {
-    while (((int64_t)1 << bits) < divisor) ++bits;
-    multiplier = (uint32_t)((((uint64_t)1 << (31 + bits)) + divisor - 1) / divisor);
-  }
-  __device__ __forceinline__ int divide(int x) const {
-    return (int)(__umulhi(2u * (uint32_t)x, multiplier) >> bits);
-  }
-};
 
 struct PrefillArgs {
   const uint4* q;       // Tq rows of Hq * 16 pieces, q_stride pieces apart

@@ -1132,6 +1132,42 @@ def test_rows_in_pieces(lens, Hq, Hkv, route, dtype):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,bs,width", [
+    ([32 * i - 5 for i in range(1, 18)], 8, 2, 64, 1152),  # 1 .. 17 steps, with as many waves idle
+    ([1, 0, 31, 32, 33, 64, 65, 2000], 16, 8, 64, 2048),   # lone steps beside a row of many pieces
+    ([704, 736, 768, 800], 6, 2, 32, 832),                 # 22 .. 25 steps: a longer piece from 24 on
+    ([2048, 1, 2047, 100], 16, 8, 32, 2048),               # the most entries of a table that are held
+    ([2080, 1, 2047, 100], 16, 8, 32, 2080),               # and some more
+    ([1000, 95, 97, 3000, 192], 32, 2, 96, 3072),          # pages that are no power of two, a group of 16
+    ([3000], 1, 1, 96, 32 * 32768 // 96 * 96),             # the widest table for one row
+    ([100000, 7], 1, 1, 64, 262144),                       # thousands of steps
+])
+def test_pieces_of_any_number_of_steps(lens, Hq, Hkv, bs, width):
+    """Rows cut at any step, walked by fewer than eight waves or by all of them, against the
+    oracle and, the sums being the same up to their order, closely against whole rows."""
+    print(f"case steps of pieces lens={lens[:8]} Hq={Hq} Hkv={Hkv} {bs} {width}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
+    B, dev = len(lens), "cuda:0"
+    NB = sum(-(-n // bs) for n in lens) + 3
+    q, kc, vc, bt, ctx = make_problem(7 + B + Hq, B, Hq, Hkv, 128, bs, NB, lens)
+    assert route_of_pieces(B, Hkv, width // bs, bs) == "pieces"
+    wide = np.full((B, width // bs), -1, np.int32)
+    wide[:, :bt.shape[1]] = bt
+    scale = 128 ** -0.5
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)] + [torch.from_numpy(x).to(dev)
+                                                        for x in (wide, ctx)]
+    ws = DecodeWorkspace.for_shape(B, Hq, 128, wide.shape[1], bs, Hkv, dev)
+    got = paged_attention(*t, scale, bs, phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+                          | _lib.NVJ_PHASE_SHORT_ROWS, workspace=ws)
+    assert not ws.counters.any()
+    assert_close_bf16(torch_to_bits(got), oracle(q, kc, vc, bt, ctx, scale, bs), what="steps")
+    whole = paged_attention(*t, scale, bs, chunk=_lib.NVJ_CHUNK_WHOLE_SEQUENCE)
+    # two roundings of the same sums to bfloat16
+    assert (got.float() - whole.float()).abs().max() <= 2.0 ** -7 * whole.float().abs().max()
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(8, 4), (64, 8), (6, 2), (16, 1)])   # 4, 4, 2, 1 heads side by side
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("hi", [200, 4000])              # sub-runs of one step, and of many
