@@ -1178,6 +1178,20 @@ constexpr int kWholeRowTightTolerance = 8;
 // (every wave checks the deal of all of them, 64 per pass).
 constexpr int kMaxWholeRowWorkgroups = 256;
 
+// x / d for unsigned x of 32 bits by a reciprocal of d: (x + 0.5) / d is at least 0.5 / d away from a
+// whole number, and the reciprocal, one Newton step behind an estimate of 20 bits and more, is off
+// by less than 2^-39 of itself.  A wave divides by the same two numbers a dozen times in a launch,
+// at some 25 instructions each by way of the compiler and at four here.
+__device__ __forceinline__ double reciprocal(int d) {   // d: wave-uniform
+  const double x = d, r = __builtin_amdgcn_rcp(x);
+  const uint2 bits = __builtin_bit_cast(uint2, __builtin_fma(__builtin_fma(-x, r, 1.0), r, r));
+  return __builtin_bit_cast(double, make_uint2(__builtin_amdgcn_readfirstlane(bits.x),
+                                               __builtin_amdgcn_readfirstlane(bits.y)));
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t x, double per) {
+  return (uint32_t)(((double)x + 0.5) * per);
+}
+
 // The cut of the axis: sub-run j covers the axis positions whose unit
 // (position >> shift) lies in [floor(j * units / nsub), floor((j+1) * units / nsub)).
 // shift is 0 unless the axis is so long that units * nsub would not fit 31 bits
@@ -1188,12 +1202,19 @@ struct Cut {
   int units;   // ceil(axis >> shift)
   int nsub;    // sub-runs in use, 1 <= nsub <= units
   int shift;
+  double per_unit, per_subrun;   // reciprocals of units and nsub
+  __device__ __forceinline__ Cut(int axis, int shift, int most, int min_steps)
+      : axis(axis), units((axis + (1 << shift) - 1) >> shift), shift(shift) {
+    nsub = max(1, min(most, min_steps == 1 ? units : units / min_steps));
+    per_unit = reciprocal(max(units, 1));
+    per_subrun = reciprocal(nsub);
+  }
   __device__ __forceinline__ int start_of(int j) const {
-    const uint32_t u = (uint32_t)j * (uint32_t)units / (uint32_t)nsub;
+    const uint32_t u = quotient((uint32_t)j * (uint32_t)units, per_subrun);
     return min(axis, (int)(u << shift));
   }
   __device__ __forceinline__ int subrun_of(int x) const {
-    return (int)((((uint32_t)(x >> shift) + 1u) * (uint32_t)nsub - 1u) / (uint32_t)units);
+    return (int)quotient(((uint32_t)(x >> shift) + 1u) * (uint32_t)nsub - 1u, per_unit);
   }
 };
 
@@ -1638,7 +1659,12 @@ struct SharedRows {
       write_eighth<D, F16>(a, b, kvh, kPieces * part + u, lane & 15, lane >> 4, mine, l_run);
     }
   }
-  // merge_row for this wave's pieces.
+  // merge_row for this wave's pieces.  The whole of it runs once in a launch, so its instructions
+  // count as they stand, cold in the instruction cache: pairs by slots, as merge_row has them, are
+  // 16 loads, LDS writes and masked maxima whatever the group; by heads they are 4 for up to four.
+  // The one round of loads left in front of it is the partials' own.  With the reciprocals of Cut,
+  // 16 / 8 heads: 4 sequences of 100 .. 900 positions 10.2 -> 9.1 us, 1 of 700 9.7 -> 8.6, of 8000
+  // 17.9 -> 14.3, 4 of 3000 15.0 -> 13.8, 16 of 1000 16.2 -> 15.1; 32 / 8 heads the same.
   static __device__ __forceinline__ void merge_pieces(const DecodeArgs& a, uint4* lds, int b,
                                                       int kvh, int part, int r0, int r1,
                                                       const Cut& cut, int lane) {
@@ -1668,13 +1694,15 @@ struct SharedRows {
     float m_run = kNegBig, l_run = 0.f;
     for (int base = 0; base < expected; base += kSlots) {
       const int count = min(kSlots, expected - base);
-      const int c = min(lane & 15, a.group - 1);
-      vfloat2 got[kSlots / 4];
+      // the (max, sum) pairs of the heads, a slot per lane, the last over again
+      const int slot_at = min(base + lane, expected - 1) * rec_stride * 8;
+      vfloat2 got[16];
 #pragma unroll
-      for (int i = 0; i < kSlots / 4; ++i) {
-        const int s = min(base + 4 * i + kg, expected - 1);
-        got[i] = __builtin_bit_cast(vfloat2, __builtin_amdgcn_raw_buffer_load_b64(
-                                                 wm, (s * rec_stride + c) * 8, 0, kDeviceScope));
+      for (int c = 0; c < 16; ++c) {
+        if (c > 0 && c % 4 == 0 && c >= a.group) break;
+        got[c] = __builtin_bit_cast(
+            vfloat2, __builtin_amdgcn_raw_buffer_load_b64(wm, slot_at, min(c, a.group - 1) * 8,
+                                                          kDeviceScope));
       }
       // which slots hold a partial, while these are on their way (see merge_row)
       const int j = first + base + lane;
@@ -1685,53 +1713,74 @@ struct SharedRows {
       const unsigned long long real = __ballot(mine_real);
       const int nreal = __popcll(real);
       if (mine_real) lds_list[__popcll(real & ((1ull << lane) - 1ull))] = (uint8_t)lane;
-      float m_chunk = kNegBig;
-#pragma unroll
-      for (int i = 0; i < kSlots / 4; ++i) {
-        lds_ml[(4 * i + kg) * 16 + (lane & 15)] = got[i];
-        const int sl = min(4 * i + kg, count - 1);
-        if ((real >> sl) & 1ull) m_chunk = fmaxf(m_chunk, got[i].x);
-      }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (nreal > 0) {
-        m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 16, 64));
-        m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 32, 64));
-        m_chunk = __shfl(m_chunk, (lane & 48) | r, 64);
-        const float m_new = fmaxf(m_run, m_chunk);
-        const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
-        m_run = m_new;
-        l_run *= keep;
+      for (int done = 0; done < nreal; done += 4 * lane_groups) {
+        // the partials; the first are asked for while the pairs are on their way
+        int idx[4];
+        vfloat4 v[4][kPieces];
 #pragma unroll
-        for (int u = 0; u < kPieces; ++u) acc[u] *= keep;
-        for (int done = 0; done < nreal; done += 4 * lane_groups) {
-          float w[4];
-          vfloat4 v[4][kPieces];
+        for (int k = 0; k < 4; ++k) {
+          const int n = done + k * lane_groups + lg;
+          idx[k] = lds_list[n < nreal ? n : 0];
+          const int off = (base + idx[k]) * slot_bytes + lane_off;
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int n = done + k * lane_groups + lg;
-            const bool have = n < nreal;
-            const int idx = lds_list[have ? n : 0];
-            const int off = (base + idx) * slot_bytes + lane_off;
+          for (int u = 0; u < kPieces; ++u)
+            v[k][u] = __builtin_bit_cast(
+                vfloat4, __builtin_amdgcn_raw_buffer_load_b128(wo, off + u * piece_stride, 0,
+                                                               kDeviceScope));
+        }
+        if (done == 0) {
+          // their maxima over the slots, four heads at a time: two halving steps leave lane L
+          // with head L % 4 of the four
+          float m_chunk = kNegBig;
 #pragma unroll
-            for (int u = 0; u < kPieces; ++u)
-              v[k][u] = __builtin_bit_cast(
-                  vfloat4, __builtin_amdgcn_raw_buffer_load_b128(wo, off + u * piece_stride, 0,
-                                                                 kDeviceScope));
-            const vfloat2 ml = lds_ml[idx * 16 + r];
-            w[k] = have ? __builtin_amdgcn_exp2f((ml.x - m_new) * a.scale_log2e) : 0.f;
-            l_run = fmaf(w[k], ml.y, l_run);
-          }
+          for (int c = 0; c < 16; c += 4) {
+            if (c > 0 && c >= a.group) break;
+            float m[4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-#pragma unroll
-            for (int u = 0; u < kPieces; ++u) {
-              acc[u][0] = fmaf(w[k], v[k][u].x, acc[u][0]);
-              acc[u][1] = fmaf(w[k], v[k][u].y, acc[u][1]);
-              acc[u][2] = fmaf(w[k], v[k][u].z, acc[u][2]);
-              acc[u][3] = fmaf(w[k], v[k][u].w, acc[u][3]);
+            for (int i = 0; i < 4; ++i) {
+              lds_ml[(c + i) * kSlots + lane] = got[c + i];
+              m[i] = mine_real ? fmaxf(got[c + i].x, kNegBig) : kNegBig;
             }
+            const bool odd = lane & 1, upper = lane & 2;
+            const float m0 = fmaxf(odd ? m[1] : m[0], dpp_partner<kDppQuadXor1>(odd ? m[0] : m[1]));
+            const float m2 = fmaxf(odd ? m[3] : m[2], dpp_partner<kDppQuadXor1>(odd ? m[2] : m[3]));
+            float most = fmaxf(upper ? m2 : m0, dpp_partner<kDppQuadXor2>(upper ? m0 : m2));
+            most = fmaxf(most, row_rotate<4>(most));
+            most = fmaxf(most, row_rotate<8>(most));
+            most = wave_xor_max(wave_xor_max(most, 16), 32);
+            most = __shfl(most, (lane & 48) | (r & 3), 64);
+            if (r >= c) m_chunk = most;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          const float m_new = fmaxf(m_run, m_chunk);
+          const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+          m_run = m_new;
+          l_run *= keep;
+#pragma unroll
+          for (int u = 0; u < kPieces; ++u) acc[u] *= keep;
+        }
+        float w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const vfloat2 ml = lds_ml[r * kSlots + idx[k]];
+          w[k] = done + k * lane_groups + lg < nreal
+                     ? __builtin_amdgcn_exp2f((ml.x - m_run) * a.scale_log2e)
+                     : 0.f;
+          l_run = fmaf(w[k], ml.y, l_run);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+          for (int u = 0; u < kPieces; ++u) {
+            acc[u][0] = fmaf(w[k], v[k][u].x, acc[u][0]);
+            acc[u][1] = fmaf(w[k], v[k][u].y, acc[u][1]);
+            acc[u][2] = fmaf(w[k], v[k][u].z, acc[u][2]);
+            acc[u][3] = fmaf(w[k], v[k][u].w, acc[u][3]);
           }
         }
       }
@@ -1787,11 +1836,7 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
     for (int i = threadIdx.x; i < a.num_heads * H::kPieces; i += NW * 64)
       orow[i] = make_uint4(0u, 0u, 0u, 0u);
   }
-  Cut cut;
-  cut.axis = rows_per_seq * total;
-  cut.shift = shift;
-  cut.units = (cut.axis + (1 << shift) - 1) >> shift;
-  cut.nsub = max(1, min(num_wgs * kParts, cut.units / min_steps));
+  const Cut cut(rows_per_seq * total, shift, num_wgs * kParts, min_steps);
   if (cut.axis == 0 || g * kParts >= cut.nsub) return;
 
   // the sequence whose rows hold axis position x
@@ -1808,7 +1853,7 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
   locate(start, b, before, ctx);
   if (b >= batch || ctx <= 0) return;   // cannot happen when the prefix sums are right
   const int nb0 = (ctx + kStep - 1) / kStep;
-  const int hg0 = (start - rows_per_seq * before) / nb0;
+  const int hg0 = (int)quotient(start - rows_per_seq * before, reciprocal(nb0));
   const int row0 = rows_per_seq * before + hg0 * nb0;
   const int xs = part < nparts ? cut.start_of(g * kParts + part) : end;
   const int xe = part < nparts ? cut.start_of(g * kParts + part + 1) : end;
@@ -1882,7 +1927,7 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
       ctx = b < batch ? __builtin_amdgcn_readlane(kept_ctx, b & 63) : 0;
       continue;
     }
-    const int hg = (x - seq0) / nb, row = seq0 + hg * nb;
+    const int hg = (int)quotient(x - seq0, reciprocal(nb)), row = seq0 + hg * nb;
     const int st = x - row, en = min(nb, st + (xe - x));
     const int kvh = hg * HPW + h_in_row;
     f32x4 acc[8];
@@ -2382,11 +2427,7 @@ __global__ __launch_bounds__(512) void paged_decode_balanced_kernel(DecodeArgs a
   const int rows_per_seq = a.num_kv_heads / hpw;
   const int part = wave / hpw;
   const int h_in_row = wave - part * hpw;
-  Cut cut;
-  cut.axis = rows_per_seq * total;
-  cut.shift = shift;
-  cut.units = (cut.axis + (1 << shift) - 1) >> shift;
-  cut.nsub = max(1, min(num_wgs * parts, cut.units / min_steps));
+  const Cut cut(rows_per_seq * total, shift, num_wgs * parts, min_steps);
   if (!short_row && (cut.axis == 0 || g * parts >= cut.nsub)) return;
 
   // the sequence whose rows hold axis position x: its index, the steps before
