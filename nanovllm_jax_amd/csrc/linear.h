@@ -28,7 +28,7 @@ struct LinearArgs {
   int max_position, num_heads, num_kv_heads;
   int64_t num_slots;
   ReadAhead ahead;                 // by workgroups behind the product's own (not linear_chained)
-  int m_tiles, n_tiles, group_m;   // filled in by the launch
+  int m_tiles, n_tiles;            // filled in by the launch
   int tile;                        // 1 + index of the tile shape, 0: by the sizes
 };
 

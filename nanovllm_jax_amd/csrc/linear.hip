@@ -33,6 +33,7 @@
 
 #include "bf16.h"
 #include "device.h"
+#include "divisor.h"
 #include "launch.h"
 #include "lds_copy.h"
 #include "linear.h"
@@ -178,6 +179,10 @@ struct RopeUnits {
   }
 };
 
+// Row tiles that are walked side by side: 8 x 4 tiles at a time per XCD (51 -> 42 us for 160 x 256
+// tiles at 4400 rows).
+constexpr int kGroupM = 8;
+
 template <int BM, int BN, int kStages, Epilogue EPI>
 __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   constexpr int WM = BM / 2, WN = BN / 2;          // per wave
@@ -206,10 +211,14 @@ __global__ __launch_bounds__(256) void linear_kernel(LinearArgs a) {
   }
   const int tile = ((int)blockIdx.x % 8) * part + (int)blockIdx.x / 8;
   if (tile >= total) return;
-  const int per_group = a.group_m * a.n_tiles;
-  const int grp = tile / per_group, in_group = tile - grp * per_group;
-  const int gm = min(a.group_m, a.m_tiles - grp * a.group_m);
-  const int n_tile = in_group / gm, m_tile = grp * a.group_m + (in_group - n_tile * gm);
+  const int per_group = kGroupM * a.n_tiles;
+  // (two divisions in front of the first copy: 18.0 -> 17.8 us for gate/up of 1000 rows)
+  const int grp = (int)nvj::quotient(tile, nvj::reciprocal(per_group));
+  const int in_group = tile - grp * per_group;
+  const int gm = min(kGroupM, a.m_tiles - grp * kGroupM);
+  const int n_tile = gm == kGroupM ? in_group / kGroupM
+                                   : (int)nvj::quotient(in_group, nvj::reciprocal(gm));
+  const int m_tile = grp * kGroupM + (in_group - n_tile * gm);
   const int m0 = m_tile * BM;
   const int row_bytes = a.K * 2;
 
@@ -579,18 +588,15 @@ bool linear_takes(int64_t m, int64_t n, int64_t k) {
 }
 
 hipError_t linear(hipStream_t s, LinearArgs a, bool for_later) {
-  a.group_m = 8;   // 8 x 4 tiles at a time per XCD: 51 -> 42 us for 160 x 256 tiles at 4400 rows
   const int shape = a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0);
   const int64_t bytes = (int64_t)a.M * a.N * 2;
   const bool past_l2 = for_later || (bytes >= kPastL2From && bytes <= kPastL2To);
   return past_l2 ? launch_shape<kRowsPastL2>(shape, s, a) : launch_shape<kPlain>(shape, s, a);
 }
 hipError_t linear_silu_mul(hipStream_t s, LinearArgs a) {
-  a.group_m = 8;
   return launch_shape<kSiluMul>(a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 0), s, a);
 }
 hipError_t linear_qk_rope(hipStream_t s, LinearArgs a) {
-  a.group_m = 8;
   int shape = a.tile > 0 ? a.tile - 1 : best_shape(a.M, a.N, a.K, 128);
   // columns beyond the last head would be taken for one: 256-wide tiles for an even count only
   if (a.N % kShapes[shape].bn != 0) shape = 4;

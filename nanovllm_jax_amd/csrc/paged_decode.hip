@@ -51,10 +51,13 @@
 
 namespace {
 
+typedef __attribute__((address_space(3))) char* lds_ptr;
 using nvj::bf16x8;
 using nvj::compute_units;
 using nvj::f16x8;
 using nvj::f32x4;
+using nvj::quotient;
+using nvj::reciprocal;
 using nvj::wave_inclusive_scan;
 using nvj::wave_max;
 
@@ -1178,20 +1181,6 @@ constexpr int kWholeRowTightTolerance = 8;
 // (every wave checks the deal of all of them, 64 per pass).
 constexpr int kMaxWholeRowWorkgroups = 256;
 
-// x / d for unsigned x of 32 bits by a reciprocal of d: (x + 0.5) / d is at least 0.5 / d away from a
-// whole number, and the reciprocal, one Newton step behind an estimate of 20 bits and more, is off
-// by less than 2^-39 of itself.  A wave divides by the same two numbers a dozen times in a launch,
-// at some 25 instructions each by way of the compiler and at four here.
-__device__ __forceinline__ double reciprocal(int d) {   // d: wave-uniform
-  const double x = d, r = __builtin_amdgcn_rcp(x);
-  const uint2 bits = __builtin_bit_cast(uint2, __builtin_fma(__builtin_fma(-x, r, 1.0), r, r));
-  return __builtin_bit_cast(double, make_uint2(__builtin_amdgcn_readfirstlane(bits.x),
-                                               __builtin_amdgcn_readfirstlane(bits.y)));
-}
-__device__ __forceinline__ uint32_t quotient(uint32_t x, double per) {
-  return (uint32_t)(((double)x + 0.5) * per);
-}
-
 // The cut of the axis: sub-run j covers the axis positions whose unit
 // (position >> shift) lies in [floor(j * units / nsub), floor((j+1) * units / nsub)).
 // shift is 0 unless the axis is so long that units * nsub would not fit 31 bits
@@ -1811,11 +1800,12 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
   using R = SharedRows<F16, HPW>;
   constexpr int D = R::D, NW = R::NW, kParts = R::kParts;
   using H = HeadDim<D>;
+  __shared__ uint4 k_tile[NW][R::kTile];
   if ((int)blockIdx.x >= num_wgs) {
-    nvj::read_chunk<512>(ahead, (int)blockIdx.x - num_wgs);
+    nvj::read_chunk_by_lds<NW * 64>(ahead, (int)blockIdx.x - num_wgs,
+                                    (uint32_t)(uintptr_t)(lds_ptr)&k_tile[0][0]);
     return;
   }
-  __shared__ uint4 k_tile[NW][R::kTile];
   __shared__ int last[HPW];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;

@@ -12,6 +12,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "lds_copy.h"
+
 namespace nvj {
 
 // Up to kRegions regions of count[i] chunks of bytes[i] bytes each (a multiple of 16), a
@@ -61,6 +63,27 @@ __device__ __forceinline__ void read_chunk(const ReadAhead& ahead, int chunk) {
     }
     chunk -= ahead.count[i];
   }
+}
+
+// The same by way of LDS (1 KB a wave, from `lds`), for kernels whose registers leave a CU one such
+// workgroup at a time: nothing waits between the reads of a chunk.  us a step with registers / LDS
+// in the attention of a layer of 1024 (3072), a graph: 1 sequence of 100 positions 916 / 882, 4 of
+// 100 .. 900 1009 / 991, 2 of 2000 1057 / 1037, 6 of 900 1194 / 1161, 8 of 1000 1280 / 1258, and 1
+// of 500, 16 of 100 .. 400, 4 of 3000 938 / 940, 1186 / 1182, 1206 / 1212.  (Fewer workgroups with
+// several chunks each: 80 .. 256 of them within 2 % either way.)
+template <int THREADS>
+__device__ __forceinline__ void read_chunk_by_lds(const ReadAhead& ahead, int chunk, uint32_t lds) {
+  lds += (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 1024u;
+#pragma unroll
+  for (int i = 0; i < ReadAhead::kRegions; ++i) {
+    if (chunk >= 0 && chunk < ahead.count[i]) {
+      const char* from = ahead.base[i] + (int64_t)chunk * ahead.bytes[i];
+      for (int at = 16 * threadIdx.x; at < ahead.bytes[i]; at += 16 * THREADS)
+        copy16_to_lds(from, (uint32_t)at, lds);
+    }
+    chunk -= ahead.count[i];
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may land in LDS that is another's
 }
 
 // nvj_paged_decode_launch_counters; where the launch takes the kernel for few sequences, with
