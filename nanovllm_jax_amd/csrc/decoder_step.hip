@@ -50,6 +50,7 @@
 #include "linear.h"
 #include "nvj_paged_attn.h"
 #include "read_ahead.h"
+#include "wave_ops.h"
 
 namespace {
 
@@ -146,8 +147,7 @@ struct NormPrologue {
           }
         }
       }
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+      sum = nvj::wave_sum(sum);
       const float rs = 1.0f / __builtin_sqrtf(sum * (1.0f / (float)kHidden) + eps);
 #pragma unroll
       for (int i = 0; i < kPerLane; ++i) {

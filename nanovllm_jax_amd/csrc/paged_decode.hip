@@ -60,6 +60,8 @@ using nvj::quotient;
 using nvj::reciprocal;
 using nvj::wave_inclusive_scan;
 using nvj::wave_max;
+using nvj::wave_xor_add;
+using nvj::wave_xor_max;
 
 constexpr int kMaxHeadDim = 128;     // head_dim is a template parameter: 128 or 64
 constexpr int kStep = 32;            // positions per inner step
@@ -124,10 +126,6 @@ __device__ __forceinline__ void pack2_with_rest(float a, float b, uint32_t& main
   rest = Elem<F16>::pack2(a - Elem<F16>::low_of(main), b - Elem<F16>::high_of(main));
 }
 
-
-__device__ __forceinline__ float wave_xor_max(float x, int mask) {
-  return fmaxf(x, __shfl_xor(x, mask, 64));
-}
 
 // K/V are read exactly once per call: non-temporal loads stream them past the
 // caches instead of allocating lines that will never be hit again.  `base` is
@@ -417,8 +415,8 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
     }
     float mx = fmaxf(fmaxf(fmaxf(s0[0], s0[1]), fmaxf(s0[2], s0[3])),
                      fmaxf(fmaxf(s1[0], s1[1]), fmaxf(s1[2], s1[3])));
-    mx = wave_xor_max(mx, 16);
-    mx = wave_xor_max(mx, 32);
+    mx = wave_xor_max<16>(mx);
+    mx = wave_xor_max<32>(mx);
     const float m_new = fmaxf(m_run, mx);
     const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
     const float mneg = -m_new * scale_log2e;
@@ -506,8 +504,8 @@ __device__ __forceinline__ void compute_segment(const DecodeArgs& a, uint4* lds,
   }
 
   // total of the running sum over the 4 k-groups that share column r
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = wave_xor_add<16>(l_run);
+  l_run = wave_xor_add<32>(l_run);
 }
 
 // ---------------------------------------------------------------------------
@@ -699,8 +697,8 @@ __device__ __forceinline__ void compute_segment_valu(const DecodeArgs& a, uint4*
     mx = fmaxf(mx, dpp_partner<kDppQuadXor1>(mx));
     if (G <= 4) mx = fmaxf(mx, dpp_partner<kDppQuadXor2>(mx));
     if (G <= 2) mx = fmaxf(mx, dpp_partner<kDppHalfMirror>(mx));
-    mx = wave_xor_max(mx, 16);
-    mx = wave_xor_max(mx, 32);
+    mx = wave_xor_max<16>(mx);
+    mx = wave_xor_max<32>(mx);
     const float m_new = fmaxf(m_run, mx);
     const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
     const float mneg = -m_new * scale_log2e;
@@ -776,15 +774,15 @@ __device__ __forceinline__ void compute_segment_valu(const DecodeArgs& a, uint4*
   l_run += dpp_partner<kDppQuadXor1>(l_run);
   if (G <= 4) l_run += dpp_partner<kDppQuadXor2>(l_run);
   if (G <= 2) l_run += dpp_partner<kDppHalfMirror>(l_run);
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = wave_xor_add<16>(l_run);
+  l_run = wave_xor_add<32>(l_run);
 #pragma unroll
   for (int h = 0; h < G; ++h)
 #pragma unroll
     for (int jd = 0; jd < 8; ++jd) {
       float o = acc[h][jd];
-      o += __shfl_xor(o, 16, 64);
-      o += __shfl_xor(o, 32, 64);
+      o = wave_xor_add<16>(o);
+      o = wave_xor_add<32>(o);
       acc[h][jd] = o;
     }
 
@@ -1400,8 +1398,8 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& a, uint4* lds, int b
         const int sl = min(4 * i + (lane >> 4), count - 1);
         if ((real >> sl) & 1ull) m_chunk = fmaxf(m_chunk, got[i].x);
       }
-      m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 16, 64));
-      m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, 32, 64));
+      m_chunk = wave_xor_max<16>(m_chunk);
+      m_chunk = wave_xor_max<32>(m_chunk);
       m_chunk = __shfl(m_chunk, (lane & 48) | r, 64);
       const float m_new = fmaxf(m_run, m_chunk);
       const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
@@ -1739,7 +1737,7 @@ struct SharedRows {
             float most = fmaxf(upper ? m2 : m0, dpp_partner<kDppQuadXor2>(upper ? m0 : m2));
             most = fmaxf(most, row_rotate<4>(most));
             most = fmaxf(most, row_rotate<8>(most));
-            most = wave_xor_max(wave_xor_max(most, 16), 32);
+            most = wave_xor_max<32>(wave_xor_max<16>(most));
             most = __shfl(most, (lane & 48) | (r & 3), 64);
             if (r >= c) m_chunk = most;
           }

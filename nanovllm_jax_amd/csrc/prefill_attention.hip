@@ -54,6 +54,7 @@ using nvj::Divisor;
 using nvj::f16x8;
 using nvj::f32x4;
 using nvj::store_past_l2;
+using nvj::wave_combine;
 using nvj::wave_inclusive_scan;   // (with shuffles the sequence lookup took 5 us of a short prompt)
 using nvj::wave_max;
 
@@ -340,8 +341,8 @@ __device__ __forceinline__ void probabilities_of_tile(f32x4 (&sc)[NG][2], bf16x8
     // is unchanged because both carry the same reference.
     float mx = max_of8(s0, s1);
     if (__any(fmaf(mx, sl2, mneg[g]) > kLazyLog2)) {
-      mx = max2(mx, __shfl_xor(mx, 16, 64));
-      mx = max2(mx, __shfl_xor(mx, 32, 64));
+      mx = wave_combine<16>(mx, max2);
+      mx = wave_combine<32>(mx, max2);
       const float m_new = max2(m_run[g], mx);
       const float alpha = __builtin_amdgcn_exp2f((m_run[g] - m_new) * sl2);
       m_run[g] = m_new;

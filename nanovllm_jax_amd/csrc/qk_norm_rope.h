@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "bf16.h"
+#include "wave_ops.h"
 
 namespace nvj {
 
@@ -17,15 +18,7 @@ __device__ __forceinline__ void unpack4(uint2 p, float (&f)[4]) {
   f[2] = __uint_as_float(p.y << 16); f[3] = __uint_as_float(p.y & 0xFFFF0000u);
 }
 __device__ __forceinline__ uint2 pack4(const float (&f)[4]) {
-  return make_uint2(f32_to_bf16_rne(f[0]) | ((uint32_t)f32_to_bf16_rne(f[1]) << 16),
-                    f32_to_bf16_rne(f[2]) | ((uint32_t)f32_to_bf16_rne(f[3]) << 16));
-}
-
-// the value of another lane of the row of 16 (a DPP control)
-template <int CTRL>
-__device__ __forceinline__ float row_move(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL,
-                                                               0xF, 0xF, false));
+  return make_uint2(pack2_bf16(f[0], f[1]), pack2_bf16(f[2], f[3]));
 }
 
 // WIDE: the pointers are 16-byte aligned.
@@ -54,7 +47,7 @@ __device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, bool norm, co
 #pragma unroll
     for (int e = 0; e < 4; ++e) s[e] += row_move<0x128>(s[e]);                    // row_ror:8
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] += row_move<0x1B>(row_move<0x141>(s[e]));   // i ^ 7 ^ 3
+    for (int e = 0; e < 4; ++e) s[e] += row_move<0x124>(s[e]);   // row_ror:4, i ^ 4 or i ^ 4 ^ 8
 #pragma unroll
     for (int e = 0; e < 4; ++e) s[e] += row_move<0x4E>(s[e]);                     // i ^ 2
 #pragma unroll
@@ -63,9 +56,11 @@ __device__ __forceinline__ void qk_norm_rope(uint2& lo, uint2& hi, bool norm, co
     const float r = 1.0f / __builtin_sqrtf(sum * (1.0f / 128) + eps);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      x1[e] = bf16_to_f32(f32_to_bf16_rne(x1[e] * r * w1[e]));
-      x2[e] = bf16_to_f32(f32_to_bf16_rne(x2[e] * r * w2[e]));
+      x1[e] = x1[e] * r * w1[e];
+      x2[e] = x2[e] * r * w2[e];
     }
+    unpack4(pack4(x1), x1);
+    unpack4(pack4(x2), x2);
   }
   const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
   float y1[4], y2[4];
