@@ -232,8 +232,12 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   // packed rows in the cache's type: where a float32 source is rounded for the cache
   // anyway, the store leaves a packed copy
-  Tensor k_rows, v_rows, out;
+  Tensor k_rows, v_rows, parts, out;
   OtherThreadsRun released;
+  const size_t part_bytes = paged ? nvj_paged_prefill_split_workspace_bytes(
+                                        tokens, batch, heads, c.heads, c.page, tables->size(1))
+                                  : 0;
+  if (part_bytes) parts = at::empty({(int64_t)part_bytes}, q->options().dtype(at::kByte));
   void *kp = key->data_ptr(), *vp = value->data_ptr(), *k_copy = nullptr, *v_copy = nullptr;
   if (!paged && key->scalar_type() == at::kFloat) {
     k_rows = at::empty(key->sizes(), q->options());
@@ -255,11 +259,11 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
   if (code == NVJ_OK)
-    code = paged ? nvj_paged_prefill_attention_launch(
+    code = paged ? nvj_paged_prefill_split_launch(
                        stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
                        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(),
-                       tokens, batch, heads, c.heads, c.dim, c.page, tables->size(1), c.num_blocks,
-                       (float)scale, c.dtype)
+                       part_bytes ? parts.data_ptr() : nullptr, part_bytes, tokens, batch, heads,
+                       c.heads, c.dim, c.page, tables->size(1), c.num_blocks, (float)scale, c.dtype)
                  : nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck,
                                                 out.data_ptr(), tokens, batch, heads, c.heads,
                                                 c.dim, (float)scale, c.dtype);

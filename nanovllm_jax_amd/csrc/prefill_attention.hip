@@ -75,6 +75,7 @@ constexpr int kTileBytes = kKeys * kD * 2;   // one K or V tile in LDS: 32 rows 
 // 3, fetched one tile ahead, with one column group per wave: three workgroups to a CU, for prompts
 // whose workgroups have little but their head and tail (tile_form).
 constexpr float kNegBig = -1.0e30f;
+constexpr int kShortestPart = 8;     // tiles, a multiple of the ring's 4
 constexpr float kLazyLog2 = 8.0f;    // running max moves only for gains above 2^8
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -403,6 +404,10 @@ struct PrefillArgs {
   int64_t num_slots;
   Divisor row_pieces;                // of a row
   uint32_t new_pieces, share_pieces; // of all rows, of a workgroup
+  // SPLIT: the parts that the keys of a query tile may be cut into, and where those leave theirs
+  Divisor splits;
+  float* part_o;     // [workgroups of a part, splits, wave, 8, 64 lanes, 4]
+  float2* part_ml;   // [workgroups of a part, splits, wave, 16 rows]: reference point, sum
 };
 
 // A workgroup's share of the new rows on their way into the caches.  The attention reads the
@@ -671,6 +676,37 @@ __device__ __forceinline__ bool find_query_tile(const PrefillArgs& a, bool may_s
   return false;   // (cannot happen: the item is a real tile)
 }
 
+// The keys that the rows of a query tile see.
+template <bool PAGED, int kColumnGroups>
+struct VisibleKeys {
+  int off;      // key position of the first token: the new tokens are the tail when paged
+  int k_end;    // keys [0, k_end) are visible to some row
+  int nsteps;   // in tiles
+  __device__ __forceinline__ VisibleKeys(const PrefillArgs& a, const QueryTile& tile) {
+    const int len_k =
+        PAGED ? min(max(tile.k_count, 0), a.max_blocks * a.page.d) : max(tile.k_count, 0);
+    off = PAGED ? max(len_k - tile.len_q, 0) : 0;
+    const int token_end =   // of the tile
+        min(a.group.divide(tile.c0 + kColumnGroups - 1) * 16 + 16, tile.len_q);
+    k_end = min(len_k, off + token_end);
+    nsteps = (k_end + kKeys - 1) / kKeys;
+  }
+};
+
+// The tiles [first, end) of part `part` of a query tile's keys: whole rounds of the ring, and no part
+// so short that its head and tail are most of it.
+struct KeyPart {
+  int first, end, count;   // count: parts that have keys
+  __device__ __forceinline__ KeyPart(const PrefillArgs& a, int nsteps, int part) {
+    const int each = nsteps <= 2 * kShortestPart
+                         ? 2 * kShortestPart
+                         : max((a.splits.divide(nsteps + a.splits.d - 1) + 3) & ~3, kShortestPart);
+    count = (int)nvj::quotient(nsteps + each - 1, nvj::reciprocal(each));
+    first = part * each;
+    end = min(first + each, nsteps);
+  }
+};
+
 // grid.x = 8 * ceil(tile bound * Hkv / 8) workgroups (see the work-item mapping below).
 // PAGED: keys and values come from the block-paged cache through block_tables,
 // sequence i has len_k = cu_k[i+1] - cu_k[i] keys, and its len_q query rows are the
@@ -679,7 +715,9 @@ __device__ __forceinline__ bool find_query_tile(const PrefillArgs& a, bool may_s
 // from the start of the sequence as the reference's mask does.
 // STORE (packed only): the rows of k and v also go into the caches (StoreShare).
 // STREAM: the output goes past the L2s.
-template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM, int RING>
+// SPLIT (paged only): workgroup (x, y) takes part y of the keys and leaves what it has for
+// prefill_merge_kernel, unless the tile has no other part.
+template <bool F16, bool PAGED, int NG, bool STORE, bool STREAM, int RING, bool SPLIT = false>
 __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attention_kernel(
     PrefillArgs a, bool may_sort) {
   static_assert(RING == 4 || (RING == 3 && NG == 1), "tiles in LDS");
@@ -701,15 +739,19 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
     return;
   }
   const int seq = tile.seq, kvh = tile.kvh, c0 = tile.c0, q_base = tile.q_base, len_q = tile.len_q;
-  const int k_first = tile.k_first, k_count = tile.k_count;
   share.fetch(a);
-  const int k_base = PAGED ? 0 : k_first;
-  const int len_k = PAGED ? min(max(k_count, 0), a.max_blocks * a.page.d) : max(k_count, 0);
-  // key position of the first token: the new tokens are the tail of the sequence when paged
-  const int off = PAGED ? max(len_k - len_q, 0) : 0;
-  const int token_end = min(a.group.divide(c0 + kColumnGroups - 1) * 16 + 16, len_q);   // of the tile
-  const int k_end = min(len_k, off + token_end);   // keys [0, k_end) are visible to some row
-  const int nsteps = (k_end + kKeys - 1) / kKeys;
+  const int k_base = PAGED ? 0 : tile.k_first;
+  const VisibleKeys<PAGED, kColumnGroups> keys(a, tile);
+  const int off = keys.off, k_end = keys.k_end;
+  int first_tile = 0, nsteps = keys.nsteps;   // this workgroup's tiles, up to nsteps
+  bool whole = true;
+  if constexpr (SPLIT) {
+    const KeyPart part(a, keys.nsteps, blockIdx.y);
+    if (blockIdx.y > 0 && part.first >= keys.nsteps) return;
+    first_tile = part.first;
+    nsteps = part.end;
+    whole = part.count <= 1;
+  }
 
   // ---- Q^T of both column groups as B operands: column r of group g is token
   // block0[g] + r of head[g]; tokens beyond the sequence are zero ----
@@ -765,14 +807,14 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   // and starts the copies of tile i+2 into the ring slots last read in iteration
   // i-1 (K of tile i-1, V of tile i-2).  Before the barrier that ends it, every
   // lane waits for its copies of tile i+1.
-  if (nsteps > 0) {
+  if (nsteps > first_tile) {
     // V "of tile -1" (probabilities are zero there, but 0 * NaN is not 0)
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
     uint4* v_before = v_ring + (RING - 1) * (kTileBytes / 16);
     for (int p = tid; p < kTileBytes / 16; p += kWaves * 64) v_before[p] = zero;
-    copier.look_up(0);
-    copier.issue(0, 0, 0);
-    if (kAhead > 1) copier.issue(1, 1, 1);
+    copier.look_up(first_tile);
+    copier.issue(first_tile, 0, 0);
+    if (kAhead > 1) copier.issue(first_tile + 1, 1, 1);
     wait_tiles_in_flight<kAhead - 1>();
   }
   __syncthreads();
@@ -841,7 +883,7 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
     if (RING == 4) return (i + ahead) & 3;
     return third + ahead < 3 ? third + ahead : third + ahead - 3;
   };
-  int i = 0;
+  int i = first_tile;
   // four plain tiles at a time while the tiles they fetch (up to i + 5) are full ones
   for (; RING == 4 && i + 4 <= n_plain && i + 5 < nsteps - 1; i += 4) {
     NVJ_PLAIN_TILE_AT(0, i);
@@ -856,7 +898,7 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   }
   // the last tile of the wave is still to be accumulated; its V stays in place
   // until the copies of two iterations from now
-  if (n_active > 0) accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);
+  if (n_active > first_tile) accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);
   for (; i < nsteps; ++i) {
     copier.issue(i + kAhead, slot(i, kAhead), slot(i, kAhead));
     third = slot(i, 1);
@@ -866,6 +908,16 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
 #undef NVJ_TILE
 #undef NVJ_PLAIN_TILE_AT
 #undef NVJ_END_OF_TILE
+
+  if (SPLIT && !whole) {
+    const int64_t rec = ((int64_t)blockIdx.x * a.splits.d + blockIdx.y) * kWaves + wave;
+    float4* o = reinterpret_cast<float4*>(a.part_o) + rec * (8 * 64) + lane;
+#pragma unroll
+    for (int jd = 0; jd < 8; ++jd)
+      o[64 * jd] = make_float4(acc[0][jd][0], acc[0][jd][1], acc[0][jd][2], acc[0][jd][3]);
+    if (kg == 0) a.part_ml[rec * 16 + r] = make_float2(m_run[0], lacc[0][0]);
+    return;
+  }
 
   // ---- epilogue: acc[g][jd][e] is O[token][dim = 16*jd + 4*kg + e].  The rows are
   // turned in LDS (16-byte pieces permuted by the row as for K) so that every
@@ -905,6 +957,59 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   share.finish(a);
 }
 
+// Puts the parts of every query tile together, in their order.  Eight workgroups to a tile, so that
+// all partials of a wave are on their way at once.  grid.x as in the launch of the parts, grid.y = the
+// eighths of the head dimension, block = 4 waves, a column group each.
+template <bool F16>
+__global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs a, bool may_sort) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4, jd = blockIdx.y;
+  QueryTile tile;
+  if (!find_query_tile<true, kWaves>(a, may_sort, lane, &tile)) return;
+  const VisibleKeys<true, kWaves> keys(a, tile);
+  const int count = KeyPart(a, keys.nsteps, 0).count;
+  const int c = tile.c0 + wave, block = a.group.divide(c);
+  if (count <= 1 || block * 16 >= tile.len_q) return;
+  const int64_t rec = (int64_t)blockIdx.x * a.splits.d * kWaves + wave;
+  const f32x4* o = reinterpret_cast<const f32x4*>(a.part_o) + rec * (8 * 64) + 64 * jd + lane;
+  const float2* ml = a.part_ml + rec * 16 + r;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float m_run = kNegBig, l = 0.f;
+  constexpr int kBatch = 8;   // parts on their way together
+  for (int s = 0; s < count; s += kBatch) {
+    f32x4 v[kBatch];
+    float2 p[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int at = min(s + j, count - 1) * kWaves;
+      v[j] = o[(int64_t)at * (8 * 64)];
+      p[j] = ml[at * 16];
+    }
+    float m_new = m_run;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) m_new = max2(m_new, p[j].x);
+    const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+    m_run = m_new;
+    acc *= keep;
+    l *= keep;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (s + j >= count) continue;
+      const float w = __builtin_amdgcn_exp2f((p[j].x - m_new) * a.scale_log2e);
+      l = fmaf(w, p[j].y, l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, v[j][e], acc[e]);
+    }
+  }
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const int t = block * 16 + r, head = tile.kvh * a.group.d + (c - block * a.group.d);
+  if (t >= tile.len_q) return;
+  uint2* to = reinterpret_cast<uint2*>(
+      a.out + ((int64_t)(tile.q_base + t) * a.num_heads + head) * kPieces + 2 * jd) + kg;
+  *to = make_uint2(Elem<F16>::pack2(acc[0] * inv, acc[1] * inv),
+                   Elem<F16>::pack2(acc[2] * inv, acc[3] * inv));
+}
+
 // Output rows that the L2s (32 MiB together) would not keep anyway are stored past them; left in
 // the L2s they displace the K and V rows that other workgroups are about to read (128 prompts
 // of 16..300 tokens, 166 MB of rows: 130 -> 117 us).  Smaller ones stay where the next launch
@@ -918,6 +1023,12 @@ struct TileForm {
   int groups, ring;
   int64_t tiles;
 };
+// Query tiles of one column group per wave, per KV head, if the last block and the last tile of
+// every sequence are half full.
+int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group) {
+  return ((2 * tokens + 15 * batch) * group + 16 * (kWaves - 1) * batch + 16 * kWaves) /
+         (32 * kWaves);
+}
 TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
                    bool paged) {
   // every sequence adds at most one partly filled token block and one partly filled tile
@@ -930,17 +1041,23 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
   // round with little to do: one prompt of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of
   // 70..90, 32 heads, 10.8 -> 9.1; up to 1.5 of them a CU, one prompt of 3000, 16 heads, 62 -> 50,
   // of 1500, 32 heads, 35 -> 29, 8 of 30..200 behind 500..4000 82 -> 66 (two a CU: 79 .. 111 %).
-  if (wide * num_kv_heads * 2 <= cus * 3) return {1, 4, narrow};
+  // Behind cached prefixes, where the tiles of a sequence are equally long, up to one round of the
+  // small ones: 3 of 180 behind 2800, 64 / 8, 75 us in 288 larger ones and 95 in 576.
+  if (paged ? expected_tiles(tokens, batch, group) * num_kv_heads <= 2 * cus
+            : wide * num_kv_heads * 2 <= cus * 3)
+    return {1, 4, narrow};
   // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
   // Three small ones to a CU instead, us: 100 prompts of 4 tokens, 16 / 8 heads (2 groups) 11.1 ->
   // 8.1, 200 of 16, 32 / 8 (4) 26.0 -> 22.3, 100 of 60, 32 / 32 (4) 67.4 -> 55.4, 60 of 20..60, 32 / 8
   // (12) 17.1 -> 14.8, 40 of 100, 16 / 8 (14) 19.8 -> 17.6; 60 of 20..60, 16 / 8 (6) 10.7 -> 11.2, the
   // only one slower.  Beyond that -13 .. +13 %, with 8 heads to a KV head (8 groups and more) -3 ..
   // +18 %.  Behind cached prefixes, which they would fetch for fewer rows, three of them are
-  // no better than two (-1 .. +10 % against the larger ones), and two are up to 4 groups
-  // (100 prompts of 16 behind 200..800, 32 / 8, 48.4 -> 45.1; 32 / 32 188 -> 185).
+  // no better than two (-1 .. +10 % against the larger ones), and two are up to 4 groups and one
+  // block of 16 tokens (100 prompts of 16 behind 200..800, 32 / 8, 48.4 -> 45.1; 32 / 32 188 -> 185;
+  // but 32 of 31..86 behind 1100..1700, 32 / 32, 181 -> 188).
   const int64_t groups = (tokens + 16 * batch - 1) / (16 * batch) * group;   // of a mean prompt
-  if (groups <= 4) return {1, paged ? 4 : 3, narrow};
+  if (groups <= 4 && !paged) return {1, 3, narrow};
+  if (groups <= 4 && tokens <= 16 * batch) return {1, 4, narrow};
   if (groups <= 14 && group <= 4 && !paged) return {1, 3, narrow};
   return {2, 4, wide};
 }
@@ -964,6 +1081,34 @@ bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
 // more -5 .. +12 %.
 constexpr int64_t kLongestFirstPerCu = 16;
 
+constexpr int64_t kMostSplits = 32;
+
+// Parts that a query tile's keys may be cut into; 1: none.  Few rows behind a long prefix are a
+// workgroup or two per KV head, each drawing 50 GB/s, 0.47 us a tile of keys, for thousands of keys,
+// while the other CUs idle; in parts they fill one round of two workgroups a CU.  us, whole / in
+// parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 18, 13 behind 5300, 16 / 8, 79 / 14.5, 270 behind
+// 4200, 32 / 8, 68 / 38.5, 500 behind 5000 81 / 63, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 27, 16
+// of 16..60 behind 64..4000 62 / 47.  Against that the partials and the launch that merges them are
+// 4 us, whatever the lengths turn out to be, which the host does not know: tables of up to 512
+// positions are never cut (9 tokens behind 256, 10.6 / 12.3), those of busier launches from 1024 or
+// 2048 positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
+// where every query head has keys of its own and half the CUs draw, HBM is the bound (6 of 21..39
+// behind 3000, 32 / 32, 64 / 68).  More than a round of them is slower (4 of 100..300 behind 1000..4000,
+// 34.7 / 40.2 at twice the parts), parts of 4 tiles or 12 instead of 8 +3 .. -1 and -0.7 .. +1.4 us.
+int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
+                   int64_t positions) {
+  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
+  if (form.groups != 1 || batch > 256) return 1;
+  const int64_t workgroups =
+      std::max<int64_t>(expected_tiles(tokens, batch, group) * num_kv_heads, 1);
+  if (positions <= 2 * kKeys * kShortestPart || (group == 1 && workgroups * 2 > cus)) return 1;
+  const int64_t shortest =
+      kKeys * kShortestPart * (workgroups * 4 <= cus ? 1 : workgroups * 2 <= cus ? 2 : 4);
+  return std::max<int64_t>(
+      std::min<int64_t>({2 * cus / workgroups, positions / shortest, kMostSplits}), 1);
+}
+constexpr size_t kPartBytes = kWaves * (8 * 64 * sizeof(float4) + 16 * sizeof(float2));
+
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
                    int32_t dtype, int64_t cus) {
   if (((int64_t)total_q_tokens + 15) * a.group.d > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
@@ -984,6 +1129,17 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
       (paged ? items <= kLongestFirstPerCu * cus && (int64_t)a.max_blocks * a.page.d >= 1024
              : form.groups == 2 && items * 2 <= cus * 5);
   const bool f16 = dtype == NVJ_DTYPE_F16;
+  if (a.part_o) {
+    const dim3 parts(grid.x, (unsigned)a.splits.d), eighths(grid.x, 8);
+    a.part_ml = reinterpret_cast<float2*>(a.part_o + (int64_t)grid.x * a.splits.d * kWaves * 8 * 64 * 4);
+    const auto split = f16 ? prefill_attention_kernel<true, true, 1, false, false, 4, true>
+                           : prefill_attention_kernel<false, true, 1, false, false, 4, true>;
+    const auto merge = f16 ? prefill_merge_kernel<true> : prefill_merge_kernel<false>;
+    if (nvj::launch(split, parts, block, stream, a, may_sort) != hipSuccess ||
+        nvj::launch(merge, eighths, block, stream, a, may_sort) != hipSuccess)
+      return NVJ_ERR_LAUNCH;
+    return NVJ_OK;
+  }
   const bool past_l2 = (int64_t)total_q_tokens * a.num_heads * (kD * 2) > kStreamOutBytes;
   hipError_t rc;
 #define NVJ_LAUNCH(F, P, N, S, T, R)                                                              \
@@ -1132,12 +1288,13 @@ extern "C" int nvj_prefill_attention_launch(void* stream, const void* q, const v
                                            head_dim, scale, dtype);
 }
 
-extern "C" int nvj_paged_prefill_attention_launch(
-    void* stream, const void* q, const void* k_cache, const void* v_cache,
-    const int32_t* block_tables, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
-    void* out, int32_t total_q_tokens, int32_t batch, int32_t num_heads, int32_t num_kv_heads,
-    int32_t head_dim, int32_t block_size, int32_t max_blocks, int32_t num_blocks, float scale,
-    int32_t dtype) {
+namespace {
+int launch_paged(void* stream, const void* q, const void* k_cache, const void* v_cache,
+                 const int32_t* block_tables, const int32_t* cu_seqlens_q,
+                 const int32_t* cu_seqlens_k, void* out, int32_t total_q_tokens, int32_t batch,
+                 int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                 int32_t max_blocks, int32_t num_blocks, float scale, int32_t dtype,
+                 bool may_split, void* workspace, size_t workspace_bytes) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   if (total_q_tokens < 0 || batch < 0 || num_heads <= 0 || num_kv_heads <= 0 || block_size <= 0 ||
       max_blocks < 0 || num_blocks <= 0)
@@ -1172,6 +1329,54 @@ extern "C" int nvj_paged_prefill_attention_launch(
   a.page = Divisor(block_size);
   a.max_blocks = max_blocks;
   a.num_blocks = num_blocks;
-  return launch_prefill(static_cast<hipStream_t>(stream), a, true, total_q_tokens, dtype,
-                        nvj::compute_units());
+  const int64_t cus = nvj::compute_units();
+  if (may_split) {
+    const size_t need = nvj_paged_prefill_split_workspace_bytes(
+        total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks);
+    if (need > 0) {
+      if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
+      if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
+      a.splits = Divisor(key_splits(total_q_tokens, batch, a.group.d, num_kv_heads, cus,
+                                    (int64_t)max_blocks * block_size));
+      a.part_o = static_cast<float*>(workspace);
+    }
+  }
+  return launch_prefill(static_cast<hipStream_t>(stream), a, true, total_q_tokens, dtype, cus);
+}
+}  // namespace
+
+extern "C" int nvj_paged_prefill_attention_launch(
+    void* stream, const void* q, const void* k_cache, const void* v_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    void* out, int32_t total_q_tokens, int32_t batch, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_dim, int32_t block_size, int32_t max_blocks, int32_t num_blocks, float scale,
+    int32_t dtype) {
+  return launch_paged(stream, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, out,
+                      total_q_tokens, batch, num_heads, num_kv_heads, head_dim, block_size,
+                      max_blocks, num_blocks, scale, dtype, false, nullptr, 0);
+}
+
+extern "C" size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens, int32_t batch,
+                                                          int32_t num_heads, int32_t num_kv_heads,
+                                                          int32_t block_size, int32_t max_blocks) {
+  if (total_q_tokens <= 0 || batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads != 0 || block_size <= 0 || max_blocks <= 0)
+    return 0;
+  const int64_t cus = nvj::compute_units(), group = num_heads / num_kv_heads;
+  const int64_t splits = key_splits(total_q_tokens, batch, group, num_kv_heads, cus,
+                                    (int64_t)max_blocks * block_size);
+  if (splits <= 1) return 0;
+  const int64_t tiles = tile_form(total_q_tokens, batch, group, num_kv_heads, cus, true).tiles;
+  return (size_t)((tiles * num_kv_heads + 7) / 8 * 8 * splits) * kPartBytes;
+}
+
+extern "C" int nvj_paged_prefill_split_launch(
+    void* stream, const void* q, const void* k_cache, const void* v_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    void* out, void* workspace, size_t workspace_bytes, int32_t total_q_tokens, int32_t batch,
+    int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+    int32_t max_blocks, int32_t num_blocks, float scale, int32_t dtype) {
+  return launch_paged(stream, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, out,
+                      total_q_tokens, batch, num_heads, num_kv_heads, head_dim, block_size,
+                      max_blocks, num_blocks, scale, dtype, true, workspace, workspace_bytes);
 }

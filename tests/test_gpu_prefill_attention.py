@@ -378,6 +378,63 @@ def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
         assert torch.equal(got[at[i]:at[i + 1]], one), f"sequence {i}"
 
 
+@pytest.mark.parametrize("new,cached,Hq,Hkv,bs,splits", [
+    ([1], [2000], 8, 8, 64, True),                    # one row, with parts for every ring of tiles
+    ([30, 0, 17], [1500, 700, 31], 16, 8, 256, True),  # an empty sequence, tiles of one part
+    ([5, 16, 40], [512, 480, 3000], 12, 2, 32, True),  # 16, 17 and 95 tiles, a group of 6
+    ([100], [4097], 32, 2, 96, True),                 # a group of 16, pages that are no power of two
+    ([300], [2000], 8, 4, 64, True),                  # parts that rows in front do not see
+    ([20, 30, 9], [0, 5000, 1111], 4, 1, 64, True),   # no prefix beside a long one
+    ([700], [1200], 64, 8, 64, False),                # enough workgroups without
+    ([9], [256], 8, 2, 64, False),                    # nothing to cut
+])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_paged_prefill_with_the_keys_in_parts(new, cached, Hq, Hkv, bs, splits, dtype):
+    """Few rows behind long prefixes, their keys cut into parts and put together again, against
+    the oracle and against the launch that walks all keys in one workgroup; nothing but live keys
+    is read, and nothing is taken over from the workspace."""
+    print(f"case keys in parts {new} {cached} Hq={Hq} Hkv={Hkv} bs={bs} {dtype}", flush=True)
+    import torch
+    from nanovllm_jax_amd import _lib
+    from oracle.paged_attention_oracle import paged_prefill_attention_ref
+    lens_k = [a + b for a, b in zip(new, cached)]
+    q, kc, vc, bt, cu_q, cu_k = _paged_problem(60 + Hq + bs, lens_k, new, Hq, Hkv, bs)
+    scale, dev, lib = 128 ** -0.5, "cuda:0", _lib.load()
+    live = np.zeros(kc.shape[:2], bool)
+    for i, n in enumerate(lens_k):
+        live[bt[i, np.arange(n) // bs], np.arange(n) % bs] = True
+    want = paged_prefill_attention_ref(q, kc, vc, bt, cu_q, cu_k, scale)
+    kc[~live], vc[~live] = 0x7FC0, 0x7FC0             # NaN
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)]
+    if dtype == "f16":
+        t = [x.half() for x in t]
+    t += [torch.from_numpy(x).to(dev) for x in (bt, cu_q, cu_k)]
+    sizes = (sum(new), len(new), Hq, Hkv)
+    need = lib.nvj_paged_prefill_split_workspace_bytes(*sizes, bs, bt.shape[1])
+    assert (need > 0) == bool(splits)
+    ws = torch.full((max(need, 16),), 0xFF, dtype=torch.uint8, device=dev)       # NaN
+    stream = torch.cuda.current_stream().cuda_stream
+    tail = (*sizes, 128, bs, bt.shape[1], kc.shape[0], scale,
+            _lib.NVJ_DTYPE_BF16 if dtype == "bf16" else _lib.NVJ_DTYPE_F16)
+    out, whole = torch.full_like(t[0], 7.0), torch.empty_like(t[0])
+    ptrs = [x.data_ptr() for x in t]
+    if need:
+        assert lib.nvj_paged_prefill_split_launch(stream, *ptrs, out.data_ptr(), ws.data_ptr(),
+                                                  need - 1, *tail) == -4      # NVJ_ERR_WORKSPACE
+    for _ in range(2):
+        _lib.check(lib.nvj_paged_prefill_split_launch(stream, *ptrs, out.data_ptr(), ws.data_ptr(),
+                                                      need, *tail), "split")
+    _lib.check(lib.nvj_paged_prefill_attention_launch(stream, *ptrs, whole.data_ptr(), *tail), "whole")
+    torch.cuda.synchronize()
+    if dtype == "bf16":
+        assert_close_bf16(torch_to_bits(out), want, what="keys in parts")
+    # each rounds its probabilities and its result to the 16-bit type
+    tol = 2.0 ** -6 if dtype == "bf16" else 2.0 ** -9
+    assert (out.float() - whole.float()).abs().max() <= tol * whole.float().abs().max()
+    if not splits:
+        assert torch.equal(out, whole)
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,dtype,padding", [
     ([1], 8, 8, "bf16", 0),                       # one row: fewer pieces than threads
     ([0, 0, 0], 4, 2, "f16", 5),                  # rows that belong to no sequence only
