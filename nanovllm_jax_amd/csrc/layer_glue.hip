@@ -59,7 +59,10 @@ __global__ __launch_bounds__(256) void add_rms_norm_kernel(
     nvj::ReadAhead ahead) {
 #pragma clang fp contract(off)
   if ((int)blockIdx.x * 4 >= num_tokens) {
-    nvj::read_chunk<256>(ahead, (int)blockIdx.x - (num_tokens + 3) / 4);
+    __shared__ uint4 landing[256];
+    nvj::read_chunk_by_lds<256>(
+        ahead, (int)blockIdx.x - (num_tokens + 3) / 4,
+        (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)landing);
     return;
   }
   const int token = blockIdx.x * 4 + (threadIdx.x >> 6);

@@ -70,7 +70,10 @@ __device__ __forceinline__ void read_chunk(const ReadAhead& ahead, int chunk) {
 // in the attention of a layer of 1024 (3072), a graph: 1 sequence of 100 positions 916 / 882, 4 of
 // 100 .. 900 1009 / 991, 2 of 2000 1057 / 1037, 6 of 900 1194 / 1161, 8 of 1000 1280 / 1258, and 1
 // of 500, 16 of 100 .. 400, 4 of 3000 938 / 940, 1186 / 1182, 1206 / 1212.  (Fewer workgroups with
-// several chunks each: 80 .. 256 of them within 2 % either way.)
+// several chunks each: 80 .. 256 of them within 2 % either way.)  In the norms, whose chunks are
+// two batches of registers: 24 of 100 .. 900 1451 / 1440, 100 of 200 .. 400 1848 / 1828, 128 of 1024
+// 3325 / 3310, a prompt of 200 tokens 1571 / 1550.  (Not in the products: 4268 tokens -0.3 %, 24 rows
+// +1 %.)
 template <int THREADS>
 __device__ __forceinline__ void read_chunk_by_lds(const ReadAhead& ahead, int chunk, uint32_t lds) {
   lds += (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 1024u;
