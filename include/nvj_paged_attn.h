@@ -562,19 +562,21 @@ NVJ_API int nvj_paged_prefill_attention_launch(void* stream, const void* q, cons
  * most of the GPU idle: the keys of a tile are cut into parts, which a second launch puts
  * together, in the order of the keys.  The sums are in another order then than
  * nvj_paged_prefill_attention_launch's, whose results are the same however a batch is put together.
+ * `max_keys`: the most keys that a sequence has, if known, else 0: what the tables hold; nothing but
+ * the number of parts follows from it, and it has to be the same in both calls.
  * `workspace`: nvj_paged_prefill_split_workspace_bytes, 16-byte aligned; where that is 0 this is
  * nvj_paged_prefill_attention_launch.
  */
 NVJ_API size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens, int32_t batch,
                             int32_t num_heads, int32_t num_kv_heads, int32_t block_size,
-                            int32_t max_blocks);
+                            int32_t max_blocks, int32_t max_keys);
 NVJ_API int nvj_paged_prefill_split_launch(void* stream, const void* q, const void* k_cache,
                             const void* v_cache, const int32_t* block_tables,
                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, void* out,
                             void* workspace, size_t workspace_bytes, int32_t total_q_tokens,
                             int32_t batch, int32_t num_heads, int32_t num_kv_heads,
                             int32_t head_dim, int32_t block_size, int32_t max_blocks,
-                            int32_t num_blocks, float scale, int32_t dtype);
+                            int32_t num_blocks, int32_t max_keys, float scale, int32_t dtype);
 
 /*
  * RMSNorm over the last dimension, optionally fused with the residual add.

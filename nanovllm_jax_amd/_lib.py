@@ -114,9 +114,9 @@ SYMBOLS = {
         _c.c_void_p] * 10 + [_c.c_int64] + [_c.c_int32] * 6 + [_c.c_float, _c.c_int32]),
     "nvj_paged_prefill_attention_launch": (_c.c_int, [
         _c.c_void_p] * 8 + [_c.c_int32] * 8 + [_c.c_float, _c.c_int32]),
-    "nvj_paged_prefill_split_workspace_bytes": (_c.c_size_t, [_c.c_int32] * 6),
+    "nvj_paged_prefill_split_workspace_bytes": (_c.c_size_t, [_c.c_int32] * 7),
     "nvj_paged_prefill_split_launch": (_c.c_int, [
-        _c.c_void_p] * 9 + [_c.c_size_t] + [_c.c_int32] * 8 + [_c.c_float, _c.c_int32]),
+        _c.c_void_p] * 9 + [_c.c_size_t] + [_c.c_int32] * 9 + [_c.c_float, _c.c_int32]),
     "nvj_add_rms_norm_launch": (_c.c_int, [
         _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_float, _c.c_void_p, _c.c_void_p,
         _c.c_int32, _c.c_int32]),

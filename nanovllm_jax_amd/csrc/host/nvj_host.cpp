@@ -206,14 +206,16 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 // prefill(q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k,
 //         block_tables | None, scale, block_size, device, stream, num_heads,
-//         num_kv_heads)
+//         num_kv_heads, max_seqlen_k)
 PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  if (nargs != 15) Py_RETURN_NONE;
+  if (nargs != 16) Py_RETURN_NONE;
   const int64_t device = PyLong_AsLong(args[11]);
   void* stream = PyLong_AsVoidPtr(args[12]);
   const double scale = PyFloat_AsDouble(args[9]);
   const long block_size = PyLong_AsLong(args[10]);
   const long layer_heads = PyLong_AsLong(args[13]), layer_kv_heads = PyLong_AsLong(args[14]);
+  const long most = PyLong_AsLong(args[15]);
+  const int32_t max_keys = most > 0 && most <= INT32_MAX ? (int32_t)most : 0;
   if (PyErr_Occurred()) {
     PyErr_Clear();
     Py_RETURN_NONE;
@@ -235,7 +237,8 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor k_rows, v_rows, parts, out;
   OtherThreadsRun released;
   const size_t part_bytes = paged ? nvj_paged_prefill_split_workspace_bytes(
-                                        tokens, batch, heads, c.heads, c.page, tables->size(1))
+                                        tokens, batch, heads, c.heads, c.page, tables->size(1),
+                                        max_keys)
                                   : 0;
   if (part_bytes) parts = at::empty({(int64_t)part_bytes}, q->options().dtype(at::kByte));
   void *kp = key->data_ptr(), *vp = value->data_ptr(), *k_copy = nullptr, *v_copy = nullptr;
@@ -263,7 +266,8 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                        stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
                        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(),
                        part_bytes ? parts.data_ptr() : nullptr, part_bytes, tokens, batch, heads,
-                       c.heads, c.dim, c.page, tables->size(1), c.num_blocks, (float)scale, c.dtype)
+                       c.heads, c.dim, c.page, tables->size(1), c.num_blocks, max_keys,
+                       (float)scale, c.dtype)
                  : nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck,
                                                 out.data_ptr(), tokens, batch, heads, c.heads,
                                                 c.dim, (float)scale, c.dtype);

@@ -1089,8 +1089,8 @@ constexpr int64_t kMostSplits = 32;
 // parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 18, 13 behind 5300, 16 / 8, 79 / 14.5, 270 behind
 // 4200, 32 / 8, 68 / 38.5, 500 behind 5000 81 / 63, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 27, 16
 // of 16..60 behind 64..4000 62 / 47.  Against that the partials and the launch that merges them are
-// 4 us, whatever the lengths turn out to be, which the host does not know: tables of up to 512
-// positions are never cut (9 tokens behind 256, 10.6 / 12.3), those of busier launches from 1024 or
+// 4 us, whatever the lengths turn out to be, of which the host knows an upper bound: up to 512
+// positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), those of busier launches from 1024 or
 // 2048 positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
 // where every query head has keys of its own and half the CUs draw, HBM is the bound (6 of 21..39
 // behind 3000, 32 / 32, 64 / 68).  More than a round of them is slower (4 of 100..300 behind 1000..4000,
@@ -1106,6 +1106,9 @@ int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
       kKeys * kShortestPart * (workgroups * 4 <= cus ? 1 : workgroups * 2 <= cus ? 2 : 4);
   return std::max<int64_t>(
       std::min<int64_t>({2 * cus / workgroups, positions / shortest, kMostSplits}), 1);
+}
+int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
+  return max_keys > 0 ? std::min(max_keys, max_blocks * block_size) : max_blocks * block_size;
 }
 constexpr size_t kPartBytes = kWaves * (8 * 64 * sizeof(float4) + 16 * sizeof(float2));
 
@@ -1294,7 +1297,7 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
                  const int32_t* cu_seqlens_k, void* out, int32_t total_q_tokens, int32_t batch,
                  int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
                  int32_t max_blocks, int32_t num_blocks, float scale, int32_t dtype,
-                 bool may_split, void* workspace, size_t workspace_bytes) {
+                 bool may_split, int32_t max_keys, void* workspace, size_t workspace_bytes) {
   if (dtype != NVJ_DTYPE_BF16 && dtype != NVJ_DTYPE_F16) return NVJ_ERR_BAD_DTYPE;
   if (total_q_tokens < 0 || batch < 0 || num_heads <= 0 || num_kv_heads <= 0 || block_size <= 0 ||
       max_blocks < 0 || num_blocks <= 0)
@@ -1332,12 +1335,12 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
   const int64_t cus = nvj::compute_units();
   if (may_split) {
     const size_t need = nvj_paged_prefill_split_workspace_bytes(
-        total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks);
+        total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks, max_keys);
     if (need > 0) {
       if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
       if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
       a.splits = Divisor(key_splits(total_q_tokens, batch, a.group.d, num_kv_heads, cus,
-                                    (int64_t)max_blocks * block_size));
+                                    most_keys(max_blocks, block_size, max_keys)));
       a.part_o = static_cast<float*>(workspace);
     }
   }
@@ -1353,18 +1356,19 @@ extern "C" int nvj_paged_prefill_attention_launch(
     int32_t dtype) {
   return launch_paged(stream, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, out,
                       total_q_tokens, batch, num_heads, num_kv_heads, head_dim, block_size,
-                      max_blocks, num_blocks, scale, dtype, false, nullptr, 0);
+                      max_blocks, num_blocks, scale, dtype, false, 0, nullptr, 0);
 }
 
 extern "C" size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens, int32_t batch,
                                                           int32_t num_heads, int32_t num_kv_heads,
-                                                          int32_t block_size, int32_t max_blocks) {
+                                                          int32_t block_size, int32_t max_blocks,
+                                                          int32_t max_keys) {
   if (total_q_tokens <= 0 || batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || block_size <= 0 || max_blocks <= 0)
     return 0;
   const int64_t cus = nvj::compute_units(), group = num_heads / num_kv_heads;
   const int64_t splits = key_splits(total_q_tokens, batch, group, num_kv_heads, cus,
-                                    (int64_t)max_blocks * block_size);
+                                    most_keys(max_blocks, block_size, max_keys));
   if (splits <= 1) return 0;
   const int64_t tiles = tile_form(total_q_tokens, batch, group, num_kv_heads, cus, true).tiles;
   return (size_t)((tiles * num_kv_heads + 7) / 8 * 8 * splits) * kPartBytes;
@@ -1375,8 +1379,9 @@ extern "C" int nvj_paged_prefill_split_launch(
     const int32_t* block_tables, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
     void* out, void* workspace, size_t workspace_bytes, int32_t total_q_tokens, int32_t batch,
     int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
-    int32_t max_blocks, int32_t num_blocks, float scale, int32_t dtype) {
+    int32_t max_blocks, int32_t num_blocks, int32_t max_keys, float scale, int32_t dtype) {
   return launch_paged(stream, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, out,
                       total_q_tokens, batch, num_heads, num_kv_heads, head_dim, block_size,
-                      max_blocks, num_blocks, scale, dtype, true, workspace, workspace_bytes);
+                      max_blocks, num_blocks, scale, dtype, true, max_keys, workspace,
+                      workspace_bytes);
 }

@@ -410,21 +410,22 @@ def test_paged_prefill_with_the_keys_in_parts(new, cached, Hq, Hkv, bs, splits, 
         t = [x.half() for x in t]
     t += [torch.from_numpy(x).to(dev) for x in (bt, cu_q, cu_k)]
     sizes = (sum(new), len(new), Hq, Hkv)
-    need = lib.nvj_paged_prefill_split_workspace_bytes(*sizes, bs, bt.shape[1])
-    assert (need > 0) == bool(splits)
+    need = lib.nvj_paged_prefill_split_workspace_bytes(*sizes, bs, bt.shape[1], 0)
+    assert (need > 0) == splits
+    assert lib.nvj_paged_prefill_split_workspace_bytes(*sizes, bs, bt.shape[1], 512) == 0
     ws = torch.full((max(need, 16),), 0xFF, dtype=torch.uint8, device=dev)       # NaN
     stream = torch.cuda.current_stream().cuda_stream
-    tail = (*sizes, 128, bs, bt.shape[1], kc.shape[0], scale,
-            _lib.NVJ_DTYPE_BF16 if dtype == "bf16" else _lib.NVJ_DTYPE_F16)
+    end = (scale, _lib.NVJ_DTYPE_BF16 if dtype == "bf16" else _lib.NVJ_DTYPE_F16)
+    tail = (*sizes, 128, bs, bt.shape[1], kc.shape[0])
     out, whole = torch.full_like(t[0], 7.0), torch.empty_like(t[0])
     ptrs = [x.data_ptr() for x in t]
     if need:
         assert lib.nvj_paged_prefill_split_launch(stream, *ptrs, out.data_ptr(), ws.data_ptr(),
-                                                  need - 1, *tail) == -4      # NVJ_ERR_WORKSPACE
+                                                  need - 1, *tail, 0, *end) == -4      # NVJ_ERR_WORKSPACE
     for _ in range(2):
         _lib.check(lib.nvj_paged_prefill_split_launch(stream, *ptrs, out.data_ptr(), ws.data_ptr(),
-                                                      need, *tail), "split")
-    _lib.check(lib.nvj_paged_prefill_attention_launch(stream, *ptrs, whole.data_ptr(), *tail), "whole")
+                                                      need, *tail, 0, *end), "split")
+    _lib.check(lib.nvj_paged_prefill_attention_launch(stream, *ptrs, whole.data_ptr(), *tail, *end), "whole")
     torch.cuda.synchronize()
     if dtype == "bf16":
         assert_close_bf16(torch_to_bits(out), want, what="keys in parts")
