@@ -1091,7 +1091,7 @@ constexpr int64_t kMostSplits = 32;
 // of 16..60 behind 64..4000 62 / 47.  Against that the partials and the launch that merges them are
 // 4 us, whatever the lengths turn out to be, of which the host knows an upper bound: up to 512
 // positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), those of busier launches from 1024 or
-// 2048 positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
+// 1536 positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
 // where every query head has keys of its own and half the CUs draw, HBM is the bound (6 of 21..39
 // behind 3000, 32 / 32, 64 / 68).  More than a round of them is slower (4 of 100..300 behind 1000..4000,
 // 34.7 / 40.2 at twice the parts), parts of 4 tiles or 12 instead of 8 +3 .. -1 and -0.7 .. +1.4 us.
@@ -1103,7 +1103,7 @@ int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
       std::max<int64_t>(expected_tiles(tokens, batch, group) * num_kv_heads, 1);
   if (positions <= 2 * kKeys * kShortestPart || (group == 1 && workgroups * 2 > cus)) return 1;
   const int64_t shortest =
-      kKeys * kShortestPart * (workgroups * 4 <= cus ? 1 : workgroups * 2 <= cus ? 2 : 4);
+      kKeys * kShortestPart * (workgroups * 4 <= cus ? 1 : workgroups * 2 <= cus ? 2 : 3);
   return std::max<int64_t>(
       std::min<int64_t>({2 * cus / workgroups, positions / shortest, kMostSplits}), 1);
 }
