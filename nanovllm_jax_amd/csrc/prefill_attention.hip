@@ -958,7 +958,7 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
 }
 
 // Puts the parts of every query tile together, in their order.  Eight workgroups to a tile, so that
-// all partials of a wave are on their way at once.  grid.x as in the launch of the parts, grid.y = the
+// all partials of a wave, up to 16, are on their way at once (by eights: +0.2 .. +1 us).  grid.x as in the launch of the parts, grid.y = the
 // eighths of the head dimension, block = 4 waves, a column group each.
 template <bool F16>
 __global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs a, bool may_sort) {
@@ -975,32 +975,38 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs 
   const float2* ml = a.part_ml + rec * 16 + r;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   float m_run = kNegBig, l = 0.f;
-  constexpr int kBatch = 8;   // parts on their way together
-  for (int s = 0; s < count; s += kBatch) {
-    f32x4 v[kBatch];
-    float2 p[kBatch];
+  // `batch` parts on their way together
+  auto take = [&](auto batch) __attribute__((always_inline)) {
+    constexpr int kBatch = decltype(batch)::value;
+    for (int s = 0; s < count; s += kBatch) {
+      f32x4 v[kBatch];
+      float2 p[kBatch];
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int at = min(s + j, count - 1) * kWaves;
-      v[j] = o[(int64_t)at * (8 * 64)];
-      p[j] = ml[at * 16];
+      for (int j = 0; j < kBatch; ++j) {
+        const int at = min(s + j, count - 1) * kWaves;
+        v[j] = o[(int64_t)at * (8 * 64)];
+        p[j] = ml[at * 16];
+      }
+      float m_new = m_run;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) m_new = max2(m_new, p[j].x);
+      const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+      m_run = m_new;
+      acc *= keep;
+      l *= keep;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        if (s + j >= count) continue;
+        const float w = __builtin_amdgcn_exp2f((p[j].x - m_new) * a.scale_log2e);
+        l = fmaf(w, p[j].y, l);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, v[j][e], acc[e]);
+      }
     }
-    float m_new = m_run;
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) m_new = max2(m_new, p[j].x);
-    const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
-    m_run = m_new;
-    acc *= keep;
-    l *= keep;
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      if (s + j >= count) continue;
-      const float w = __builtin_amdgcn_exp2f((p[j].x - m_new) * a.scale_log2e);
-      l = fmaf(w, p[j].y, l);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, v[j][e], acc[e]);
-    }
-  }
+  };
+  if (count <= 4) take(std::integral_constant<int, 4>());
+  else if (count <= 8) take(std::integral_constant<int, 8>());
+  else take(std::integral_constant<int, 16>());
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   const int t = block * 16 + r, head = tile.kvh * a.group.d + (c - block * a.group.d);
   if (t >= tile.len_q) return;
@@ -1086,15 +1092,17 @@ constexpr int64_t kMostSplits = 32;
 // Parts that a query tile's keys may be cut into; 1: none.  Few rows behind a long prefix are a
 // workgroup or two per KV head, each drawing 50 GB/s, 0.47 us a tile of keys, for thousands of keys,
 // while the other CUs idle; in parts they fill one round of two workgroups a CU.  us, whole / in
-// parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 18, 13 behind 5300, 16 / 8, 79 / 14.5, 270 behind
-// 4200, 32 / 8, 68 / 38.5, 500 behind 5000 81 / 63, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 27, 16
-// of 16..60 behind 64..4000 62 / 47.  Against that the partials and the launch that merges them are
+// parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 17, 13 behind 5300, 16 / 8, 79 / 14, 270 behind
+// 4200, 32 / 8, 68 / 38, 500 behind 5000 81 / 62, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 26, 16
+// of 16..60 behind 64..4000 62 / 46.  Against that the partials and the launch that merges them are
 // 4 us, whatever the lengths turn out to be, of which the host knows an upper bound: up to 512
-// positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), those of busier launches from 1024 or
-// 1536 positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
-// where every query head has keys of its own and half the CUs draw, HBM is the bound (6 of 21..39
-// behind 3000, 32 / 32, 64 / 68).  More than a round of them is slower (4 of 100..300 behind 1000..4000,
-// 34.7 / 40.2 at twice the parts), parts of 4 tiles or 12 instead of 8 +3 .. -1 and -0.7 .. +1.4 us.
+// positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), in busier launches from 1024 or 1536
+// positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
+// not where every query head has keys of its own and half the CUs draw: HBM is the bound then (6 of
+// 21..39 behind 3000, 32 / 32, 64 / 68).  More than a round of parts is slower (4 of 100..300 behind
+// 1000..4000, 34.7 / 40.2 at twice as many), three quarters of one better where there are many to put
+// together (30 behind 5000 18.5 / 16.9, 20 behind 4000, 32 / 32, 28 / 22.5).  Parts of 4 tiles or of 12
+// instead of 8: +3 .. -1 and -0.7 .. +1.4 us.
 int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
                    int64_t positions) {
   const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
@@ -1102,10 +1110,11 @@ int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
   const int64_t workgroups =
       std::max<int64_t>(expected_tiles(tokens, batch, group) * num_kv_heads, 1);
   if (positions <= 2 * kKeys * kShortestPart || (group == 1 && workgroups * 2 > cus)) return 1;
-  const int64_t shortest =
-      kKeys * kShortestPart * (workgroups * 4 <= cus ? 1 : workgroups * 2 <= cus ? 2 : 3);
-  return std::max<int64_t>(
-      std::min<int64_t>({2 * cus / workgroups, positions / shortest, kMostSplits}), 1);
+  const bool few = workgroups * 4 <= cus;
+  const int64_t shortest = kKeys * kShortestPart * (few ? 1 : workgroups * 2 <= cus ? 2 : 3);
+  return std::max<int64_t>(std::min<int64_t>({(few ? 3 * cus / 2 : 2 * cus) / workgroups,
+                                              positions / shortest, kMostSplits}),
+                           1);
 }
 int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
   return max_keys > 0 ? std::min(max_keys, max_blocks * block_size) : max_blocks * block_size;
