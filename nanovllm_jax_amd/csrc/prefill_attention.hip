@@ -898,7 +898,8 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   }
   // the last tile of the wave is still to be accumulated; its V stays in place
   // until the copies of two iterations from now
-  if (n_active > first_tile) accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);
+  if (n_active > first_tile)
+    accumulate_tile<F16, NG>(vaddr, slot(i, RING - 1) * kTileBytes, pb, acc, lacc);
   for (; i < nsteps; ++i) {
     copier.issue(i + kAhead, slot(i, kAhead), slot(i, kAhead));
     third = slot(i, 1);
@@ -957,9 +958,10 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   share.finish(a);
 }
 
-// Puts the parts of every query tile together, in their order.  Eight workgroups to a tile, so that
-// all partials of a wave, up to 16, are on their way at once (by eights: +0.2 .. +1 us).  grid.x as in the launch of the parts, grid.y = the
-// eighths of the head dimension, block = 4 waves, a column group each.
+// Puts the parts of every query tile together, in their order.  grid.x as in the launch of the parts,
+// grid.y = the eighths of the head dimension, block = 4 waves, a column group each.  Bound by the
+// launch and its round trips: eight workgroups to a tile, so that all partials of a wave, up to 16,
+// are on their way at once (by eights: +0.2 .. +1 us).
 template <bool F16>
 __global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs a, bool may_sort) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
