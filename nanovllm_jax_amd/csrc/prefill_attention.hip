@@ -406,8 +406,8 @@ struct PrefillArgs {
   uint32_t new_pieces, share_pieces; // of all rows, of a workgroup
   // SPLIT: the parts that the keys of a query tile may be cut into, and where those leave theirs
   Divisor splits;
-  float* part_o;     // [workgroups of a part, splits, wave, 8, 64 lanes, 4]
-  float2* part_ml;   // [workgroups of a part, splits, wave, 16 rows]: reference point, sum
+  float* part_o;     // [workgroups of a part, splits, column group, 8, 64 lanes, 4]
+  float2* part_ml;   // [workgroups of a part, splits, column group, 16 rows]: reference point, sum
 };
 
 // A workgroup's share of the new rows on their way into the caches.  The attention reads the
@@ -911,12 +911,17 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
 #undef NVJ_END_OF_TILE
 
   if (SPLIT && !whole) {
-    const int64_t rec = ((int64_t)blockIdx.x * a.splits.d + blockIdx.y) * kWaves + wave;
+    const int64_t rec =
+        ((int64_t)blockIdx.x * a.splits.d + blockIdx.y) * kColumnGroups + NG * wave;
     float4* o = reinterpret_cast<float4*>(a.part_o) + rec * (8 * 64) + lane;
 #pragma unroll
-    for (int jd = 0; jd < 8; ++jd)
-      o[64 * jd] = make_float4(acc[0][jd][0], acc[0][jd][1], acc[0][jd][2], acc[0][jd][3]);
-    if (kg == 0) a.part_ml[rec * 16 + r] = make_float2(m_run[0], lacc[0][0]);
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int jd = 0; jd < 8; ++jd)
+        o[64 * (8 * g + jd)] =
+            make_float4(acc[g][jd][0], acc[g][jd][1], acc[g][jd][2], acc[g][jd][3]);
+      if (kg == 0) a.part_ml[(rec + g) * 16 + r] = make_float2(m_run[g], lacc[g][0]);
+    }
     return;
   }
 
@@ -959,20 +964,20 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
 }
 
 // Puts the parts of every query tile together, in their order.  grid.x as in the launch of the parts,
-// grid.y = the eighths of the head dimension, block = 4 waves, a column group each.  Bound by the
-// launch and its round trips: eight workgroups to a tile, so that all partials of a wave, up to 16,
-// are on their way at once (by eights: +0.2 .. +1 us).
-template <bool F16>
-__global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs a, bool may_sort) {
+// grid.y = the eighths of the head dimension, block = a wave for each of the GROUPS column groups.
+// Bound by the launch and its round trips: eight workgroups to a tile, so that all partials of a wave,
+// up to 16, are on their way at once (by eights: +0.2 .. +1 us).
+template <bool F16, int GROUPS>
+__global__ __launch_bounds__(GROUPS * 64) void prefill_merge_kernel(PrefillArgs a, bool may_sort) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4, jd = blockIdx.y;
   QueryTile tile;
-  if (!find_query_tile<true, kWaves>(a, may_sort, lane, &tile)) return;
-  const VisibleKeys<true, kWaves> keys(a, tile);
+  if (!find_query_tile<true, GROUPS>(a, may_sort, lane, &tile)) return;
+  const VisibleKeys<true, GROUPS> keys(a, tile);
   const int count = KeyPart(a, keys.nsteps, 0).count;
   const int c = tile.c0 + wave, block = a.group.divide(c);
   if (count <= 1 || block * 16 >= tile.len_q) return;
-  const int64_t rec = (int64_t)blockIdx.x * a.splits.d * kWaves + wave;
+  const int64_t rec = (int64_t)blockIdx.x * a.splits.d * GROUPS + wave;
   const f32x4* o = reinterpret_cast<const f32x4*>(a.part_o) + rec * (8 * 64) + 64 * jd + lane;
   const float2* ml = a.part_ml + rec * 16 + r;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -985,7 +990,7 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_merge_kernel(PrefillArgs 
       float2 p[kBatch];
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) {
-        const int at = min(s + j, count - 1) * kWaves;
+        const int at = min(s + j, count - 1) * GROUPS;
         v[j] = o[(int64_t)at * (8 * 64)];
         p[j] = ml[at * 16];
       }
@@ -1031,27 +1036,29 @@ struct TileForm {
   int groups, ring;
   int64_t tiles;
 };
-// Query tiles of one column group per wave, per KV head, if the last block and the last tile of
-// every sequence are half full.
-int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group) {
-  return ((2 * tokens + 15 * batch) * group + 16 * (kWaves - 1) * batch + 16 * kWaves) /
-         (32 * kWaves);
+// Query tiles per KV head, at most: every sequence adds at most one partly filled token block and one
+// partly filled tile.
+int64_t most_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_groups) {
+  const int64_t blocks = (tokens + 15 * batch) / 16;
+  return (blocks * group + (column_groups - 1) * batch) / column_groups;
+}
+// The same if the last block and the last tile of every sequence are half full.
+int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_groups) {
+  return ((2 * tokens + 15 * batch) * group + 16 * (column_groups - 1) * batch +
+          16 * column_groups) /
+         (32 * column_groups);
 }
 TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
                    bool paged) {
-  // every sequence adds at most one partly filled token block and one partly filled tile
-  const int64_t blocks = (tokens + 15 * batch) / 16;
-  auto tiles_of = [&](int column_groups) {
-    return (blocks * group + (column_groups - 1) * batch) / column_groups;
-  };
-  const int64_t wide = tiles_of(2 * kWaves), narrow = tiles_of(kWaves);
+  const int64_t wide = most_tiles(tokens, batch, group, 2 * kWaves);
+  const int64_t narrow = most_tiles(tokens, batch, group, kWaves);
   // One column group per wave while the larger workgroups would leave CUs idle or start a second
   // round with little to do: one prompt of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of
   // 70..90, 32 heads, 10.8 -> 9.1; up to 1.5 of them a CU, one prompt of 3000, 16 heads, 62 -> 50,
   // of 1500, 32 heads, 35 -> 29, 8 of 30..200 behind 500..4000 82 -> 66 (two a CU: 79 .. 111 %).
   // Behind cached prefixes, where the tiles of a sequence are equally long, up to one round of the
   // small ones: 3 of 180 behind 2800, 64 / 8, 75 us in 288 larger ones and 95 in 576.
-  if (paged ? expected_tiles(tokens, batch, group) * num_kv_heads <= 2 * cus
+  if (paged ? expected_tiles(tokens, batch, group, kWaves) * num_kv_heads <= 2 * cus
             : wide * num_kv_heads * 2 <= cus * 3)
     return {1, 4, narrow};
   // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
@@ -1095,7 +1102,7 @@ constexpr int64_t kMostSplits = 32;
 // workgroup or two per KV head, each drawing 50 GB/s, 0.47 us a tile of keys, for thousands of keys,
 // while the other CUs idle; in parts they fill one round of two workgroups a CU.  us, whole / in
 // parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 17, 13 behind 5300, 16 / 8, 79 / 14, 270 behind
-// 4200, 32 / 8, 68 / 38, 500 behind 5000 81 / 62, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 26, 16
+// 4200, 32 / 8, 68 / 38, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 26, 16
 // of 16..60 behind 64..4000 62 / 46.  Against that the partials and the launch that merges them are
 // 4 us, whatever the lengths turn out to be, of which the host knows an upper bound: up to 512
 // positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), in busier launches from 1024 or 1536
@@ -1105,12 +1112,15 @@ constexpr int64_t kMostSplits = 32;
 // 1000..4000, 34.7 / 40.2 at twice as many), three quarters of one better where there are many to put
 // together (30 behind 5000 18.5 / 16.9, 20 behind 4000, 32 / 32, 28 / 22.5).  Parts of 4 tiles or of 12
 // instead of 8: +3 .. -1 and -0.7 .. +1.4 us.
-int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
-                   int64_t positions) {
-  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
+struct SplitForm {
+  TileForm form;
+  int64_t splits;
+};
+int64_t key_splits(const TileForm& form, int64_t tokens, int64_t batch, int64_t group,
+                   int64_t num_kv_heads, int64_t cus, int64_t positions) {
   if (form.groups != 1 || batch > 256) return 1;
   const int64_t workgroups =
-      std::max<int64_t>(expected_tiles(tokens, batch, group) * num_kv_heads, 1);
+      std::max<int64_t>(expected_tiles(tokens, batch, group, kWaves) * num_kv_heads, 1);
   if (positions <= 2 * kKeys * kShortestPart || (group == 1 && workgroups * 2 > cus)) return 1;
   const bool few = workgroups * 4 <= cus;
   const int64_t shortest = kKeys * kShortestPart * (few ? 1 : workgroups * 2 <= cus ? 2 : 3);
@@ -1118,16 +1128,35 @@ int64_t key_splits(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
                                               positions / shortest, kMostSplits}),
                            1);
 }
+
+// The form of a launch in parts.  In the small workgroups every wave reads a whole tile of keys out of
+// LDS for 16 rows, which is what bounds two of them to a CU (0.69 us a tile; the larger ones 1.2 for
+// twice the rows).  Where the small ones would be cut into two or three parts or none at all the larger
+// ones in parts, up to two a CU, are the shorter way behind more than 4096 positions.  us, before /
+// so: 500 behind 5000, 32 / 8 heads, 69 / 60, 700 behind 5000 90 / 81, 512 behind 8000, 64 / 8, 157 /
+// 133, 400 behind 4000, 32 / 32, 68 / 51, 6 of 23..44 behind 8555..10940, 64 / 8, 148 / 99; 50 launches
+// drawn from 70 .. 400 large workgroups -2 .. +49 %.  Up to 4096 positions the partials cost more
+// (1000 behind 2000 55 / 62), with fewer rows many small parts are as good (270 behind 4200 37.6 / 36.4,
+// 150 behind 4000, 32 / 32, 29 / 33), with more large workgroups than CUs two parts each are not
+// (4 of 244..494 behind 3357..5499, 368 of them, 125 / 151).
+SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads,
+                     int64_t cus, int64_t positions) {
+  const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
+  const int64_t large =
+      std::max<int64_t>(expected_tiles(tokens, batch, group, 2 * kWaves) * num_kv_heads, 1);
+  if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 && large <= cus)
+    return {{2, 4, most_tiles(tokens, batch, group, 2 * kWaves)}, 2 * cus / large};
+  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
+  return {form, key_splits(form, tokens, batch, group, num_kv_heads, cus, positions)};
+}
 int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
   return max_keys > 0 ? std::min(max_keys, max_blocks * block_size) : max_blocks * block_size;
 }
-constexpr size_t kPartBytes = kWaves * (8 * 64 * sizeof(float4) + 16 * sizeof(float2));
+constexpr size_t kGroupBytes = (8 * 64 * sizeof(float4) + 16 * sizeof(float2));
 
-int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_q_tokens,
-                   int32_t dtype, int64_t cus) {
+int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, const TileForm& form,
+                   int32_t total_q_tokens, int32_t dtype, int64_t cus) {
   if (((int64_t)total_q_tokens + 15) * a.group.d > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
-  const TileForm form =
-      tile_form(total_q_tokens, a.batch, a.group.d, a.num_kv_heads, cus, paged);
   const int64_t tiles = form.tiles;
   if (tiles > INT32_MAX) return NVJ_ERR_BAD_SHAPE;
   const int64_t items = tiles * a.num_kv_heads;
@@ -1145,14 +1174,21 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, int32_t total_
   const bool f16 = dtype == NVJ_DTYPE_F16;
   if (a.part_o) {
     const dim3 parts(grid.x, (unsigned)a.splits.d), eighths(grid.x, 8);
-    a.part_ml = reinterpret_cast<float2*>(a.part_o + (int64_t)grid.x * a.splits.d * kWaves * 8 * 64 * 4);
-    const auto split = f16 ? prefill_attention_kernel<true, true, 1, false, false, 4, true>
-                           : prefill_attention_kernel<false, true, 1, false, false, 4, true>;
-    const auto merge = f16 ? prefill_merge_kernel<true> : prefill_merge_kernel<false>;
-    if (nvj::launch(split, parts, block, stream, a, may_sort) != hipSuccess ||
-        nvj::launch(merge, eighths, block, stream, a, may_sort) != hipSuccess)
-      return NVJ_ERR_LAUNCH;
-    return NVJ_OK;
+    a.part_ml = reinterpret_cast<float2*>(a.part_o + (int64_t)grid.x * a.splits.d * form.groups *
+                                                         kWaves * 8 * 64 * 4);
+    const auto go = [&](auto groups) {
+      constexpr int NG = decltype(groups)::value;
+      const auto split = f16 ? prefill_attention_kernel<true, true, NG, false, false, 4, true>
+                             : prefill_attention_kernel<false, true, NG, false, false, 4, true>;
+      const auto merge =
+          f16 ? prefill_merge_kernel<true, NG * kWaves> : prefill_merge_kernel<false, NG * kWaves>;
+      const dim3 waves(NG * kWaves * 64);
+      return nvj::launch(split, parts, block, stream, a, may_sort) == hipSuccess &&
+             nvj::launch(merge, eighths, waves, stream, a, may_sort) == hipSuccess;
+    };
+    const bool ok = form.groups == 2 ? go(std::integral_constant<int, 2>())
+                                     : go(std::integral_constant<int, 1>());
+    return ok ? NVJ_OK : NVJ_ERR_LAUNCH;
   }
   const bool past_l2 = (int64_t)total_q_tokens * a.num_heads * (kD * 2) > kStreamOutBytes;
   hipError_t rc;
@@ -1244,8 +1280,9 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
     a.row_pieces = Divisor((int64_t)num_kv_heads * kPieces);
     a.new_pieces = (uint32_t)store->rows * (uint32_t)a.row_pieces.d;
   }
-  return launch_prefill(static_cast<hipStream_t>(stream), a, false, total_q_tokens, dtype,
-                        cus);
+  return launch_prefill(static_cast<hipStream_t>(stream), a, false,
+                        tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, false),
+                        total_q_tokens, dtype, cus);
 }
 }  // namespace
 
@@ -1344,18 +1381,21 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
   a.max_blocks = max_blocks;
   a.num_blocks = num_blocks;
   const int64_t cus = nvj::compute_units();
+  TileForm form = tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true);
   if (may_split) {
     const size_t need = nvj_paged_prefill_split_workspace_bytes(
         total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks, max_keys);
     if (need > 0) {
       if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
       if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
-      a.splits = Divisor(key_splits(total_q_tokens, batch, a.group.d, num_kv_heads, cus,
-                                    most_keys(max_blocks, block_size, max_keys)));
+      const SplitForm cut = split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus,
+                                       most_keys(max_blocks, block_size, max_keys));
+      form = cut.form;
+      a.splits = Divisor(cut.splits);
       a.part_o = static_cast<float*>(workspace);
     }
   }
-  return launch_prefill(static_cast<hipStream_t>(stream), a, true, total_q_tokens, dtype, cus);
+  return launch_prefill(static_cast<hipStream_t>(stream), a, true, form, total_q_tokens, dtype, cus);
 }
 }  // namespace
 
@@ -1378,11 +1418,11 @@ extern "C" size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens
       num_heads % num_kv_heads != 0 || block_size <= 0 || max_blocks <= 0)
     return 0;
   const int64_t cus = nvj::compute_units(), group = num_heads / num_kv_heads;
-  const int64_t splits = key_splits(total_q_tokens, batch, group, num_kv_heads, cus,
-                                    most_keys(max_blocks, block_size, max_keys));
-  if (splits <= 1) return 0;
-  const int64_t tiles = tile_form(total_q_tokens, batch, group, num_kv_heads, cus, true).tiles;
-  return (size_t)((tiles * num_kv_heads + 7) / 8 * 8 * splits) * kPartBytes;
+  const SplitForm cut = split_form(total_q_tokens, batch, group, num_kv_heads, cus,
+                                   most_keys(max_blocks, block_size, max_keys));
+  if (cut.splits <= 1) return 0;
+  const int64_t workgroups = (cut.form.tiles * num_kv_heads + 7) / 8 * 8;
+  return (size_t)(workgroups * cut.splits * cut.form.groups * kWaves) * kGroupBytes;
 }
 
 extern "C" int nvj_paged_prefill_split_launch(

@@ -385,6 +385,9 @@ def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
     ([100], [4097], 32, 2, 96, True),                 # a group of 16, pages that are no power of two
     ([300], [2000], 8, 4, 64, True),                  # parts that rows in front do not see
     ([20, 30, 9], [0, 5000, 1111], 4, 1, 64, True),   # no prefix beside a long one
+    ([500], [4200], 32, 8, 256, True),                # larger workgroups in parts
+    ([23, 0, 44, 37, 5, 31], [4300, 0, 100, 2000, 64, 4096], 64, 8, 64, True),   # ... tiles of one part
+    ([400], [4100], 32, 32, 64, True),                # ... no group, three column groups in the last
     ([700], [1200], 64, 8, 64, False),                # enough workgroups without
     ([9], [256], 8, 2, 64, False),                    # nothing to cut
 ])
