@@ -198,7 +198,7 @@ class Attention:
             out = _host_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping,
                                 context.cu_seqlens_q, context.cu_seqlens_k, context.block_tables,
                                 self.scale, self.block_size, dev, _raw_stream(dev), self.num_heads,
-                                self.num_kv_heads, context.max_seqlen_k)
+                                self.num_kv_heads, getattr(context, "max_seqlen_k", 0))
         else:
             ws, partials, counters = self.workspace, None, None
             if ws is not None:

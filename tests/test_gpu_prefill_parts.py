@@ -1,0 +1,85 @@
+"""Prefill behind a cached prefix through the layer, where keys are cut into parts: what the
+context says of the longest sequence, memory that is short, other streams, graphs and threads."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from helpers import bits_to_torch, torch_to_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(new, cached, Hq=32, Hkv=8, bs=64, dtype="bf16", width=0, seed=1):
+    """A layer, its q, k and v, the fields of a context, and the result of the oracle."""
+    import torch
+    from nanovllm_jax_amd import Attention
+    from oracle.paged_attention_oracle import paged_prefill_attention_ref, store_kv_to_cache_ref
+    rng = np.random.Generator(np.random.PCG64(seed))
+    dev, total = "cuda:0", [a + b for a, b in zip(new, cached)]
+    pages = [-(-n // bs) for n in total]
+    table = np.full((len(new), max(max(pages), width)), -1, np.int32)
+    ids, at = rng.permutation(sum(pages) + 2), 0
+    for i, n in enumerate(pages):
+        table[i, :n] = ids[at:at + n]
+        at += n
+    slots = [np.zeros(0, np.int32)]
+    for i, (a, b) in enumerate(zip(cached, total)):
+        p = np.arange(a, b)
+        slots.append((table[i, p // bs] * bs + p % bs).astype(np.int32))
+    slots = np.concatenate(slots)
+    cu = lambda n: np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    draw = lambda *shape: torch.from_numpy(rng.standard_normal(shape, np.float32)).to(
+        torch.bfloat16 if dtype == "bf16" else torch.float16)
+    q, k, v = (draw(sum(new), h, 128) for h in (Hq, Hkv, Hkv))
+    kc, vc = (draw(sum(pages) + 2, bs, Hkv, 128) for _ in range(2))
+    flat = (-1, Hkv, 128)
+    bits = [torch_to_bits(x) for x in (k, v, kc, vc)]
+    wk, wv = store_kv_to_cache_ref(bits[0], bits[1], bits[2].reshape(flat), bits[3].reshape(flat),
+                                   slots, negative_slots="skip")
+    want = paged_prefill_attention_ref(torch_to_bits(q), wk.reshape(kc.shape), wv.reshape(vc.shape),
+                                       table, cu(new), cu(total), 128 ** -0.5, return_f32=True,
+                                       dtype=dtype)
+    attn = Attention(Hq, 128, 128 ** -0.5, Hkv, bs)
+    attn.set_kv_cache(kc.to(dev), vc.to(dev))
+    up = lambda a: torch.from_numpy(a).to(dev)
+    fields = dict(is_prefill=True, cu_seqlens_q=up(cu(new)), cu_seqlens_k=up(cu(total)),
+                  slot_mapping=up(slots), block_tables=up(table))
+    return attn, [x.to(dev) for x in (q, k, v)], fields, want
+
+
+def _check(out, want):
+    """Probabilities and results are rounded to the 16-bit type, sums are not: a rounding each,
+    and as much again for the oracle's."""
+    import torch
+    got = out.float().cpu().numpy()
+    tol = 2.0 ** -6 if out.dtype == torch.bfloat16 else 2.0 ** -9
+    assert np.abs(got - want).max() <= tol * np.abs(want).max()
+
+
+def _parts(fields, Hq, Hkv, bs, max_keys):
+    """Bytes of partials, 0 where keys are not cut."""
+    from nanovllm_jax_amd import _lib
+    table, cu = fields["block_tables"], fields["cu_seqlens_q"]
+    return _lib.load().nvj_paged_prefill_split_workspace_bytes(
+        int(cu[-1]), len(cu) - 1, Hq, Hkv, bs, table.shape[1], max_keys)
+
+
+@pytest.fixture
+def native_only(monkeypatch):
+    """The general path is no way out."""
+    from nanovllm_jax_amd.layers import attention
+
+    def refused(*_):
+        raise AssertionError("declined by the native call")
+    monkeypatch.setattr(attention, "store_kv_to_cache", refused)
+
+
+@pytest.mark.parametrize("paged", [True, False])
+def test_context_without_the_longest_length(paged, native_only):
+    """A context object of a caller's own need not have a field that no launch needs."""
+    print(f"case context without max_seqlen_k paged={paged}", flush=True)
+    attn, qkv, fields, want = _call([9, 33], [1500, 0] if paged else [0, 0])
+    if not paged:
+        fields.update(block_tables=None, cu_seqlens_k=fields["cu_seqlens_q"])
+    _check(attn(*qkv, SimpleNamespace(**fields)), want)
