@@ -204,6 +204,15 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return result(&released, &out, code);
 }
 
+// What a context says of the longest sequence, 0 (not known) for anything but a whole number that
+// is at hand: it is a hint, and asking a tensor for it would wait for the GPU.
+int32_t known_keys(PyObject* o) {
+  if (THPVariable_Check(o) || !PyIndex_Check(o)) return 0;
+  const Py_ssize_t n = PyNumber_AsSsize_t(o, nullptr);   // clipped, no error
+  if (n == -1 && PyErr_Occurred()) PyErr_Clear();
+  return n > 0 && n <= INT32_MAX ? (int32_t)n : 0;
+}
+
 // prefill(q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k,
 //         block_tables | None, scale, block_size, device, stream, num_heads,
 //         num_kv_heads, max_seqlen_k)
@@ -214,8 +223,6 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const double scale = PyFloat_AsDouble(args[9]);
   const long block_size = PyLong_AsLong(args[10]);
   const long layer_heads = PyLong_AsLong(args[13]), layer_kv_heads = PyLong_AsLong(args[14]);
-  const long most = PyLong_AsLong(args[15]);
-  const int32_t max_keys = most > 0 && most <= INT32_MAX ? (int32_t)most : 0;
   if (PyErr_Occurred()) {
     PyErr_Clear();
     Py_RETURN_NONE;
@@ -223,6 +230,7 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor *q, *key, *value, *slots, *cu_q, *cu_k, *tables = nullptr;
   Caches c;
   const bool paged = args[8] != Py_None;
+  const int32_t max_keys = paged ? known_keys(args[15]) : 0;
   if (!layer_tensors(args, device, &q, &key, &value, &c, &slots) ||
       !int_tensor(args[6], device, 1, &cu_q) || !int_tensor(args[7], device, 1, &cu_k) ||
       (paged && !int_tensor(args[8], device, 2, &tables)))

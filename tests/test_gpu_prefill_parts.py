@@ -83,3 +83,28 @@ def test_context_without_the_longest_length(paged, native_only):
     if not paged:
         fields.update(block_tables=None, cu_seqlens_k=fields["cu_seqlens_q"])
     _check(attn(*qkv, SimpleNamespace(**fields)), want)
+
+
+@pytest.mark.parametrize("paged", [True, False])
+@pytest.mark.parametrize("longest", [None, 1533.0, "on the host", "on the device", "numpy", -1,
+                                     1 << 40, 1 << 70])
+def test_longest_length_that_is_no_number_at_hand(longest, paged, native_only):
+    """It is a hint: whatever stands there, the call is the ordinary one, and nothing is asked of a
+    tensor, which would wait for the GPU (and cannot be, in a capture)."""
+    print(f"case max_seqlen_k {longest} paged={paged}", flush=True)
+    import torch
+    from nanovllm_jax_amd import AttentionContext
+    attn, qkv, fields, want = _call([9, 33], [1500, 0] if paged else [0, 0])
+    if not paged:
+        fields.update(block_tables=None, cu_seqlens_k=fields["cu_seqlens_q"])
+    longest = {"on the host": torch.tensor(1533), "on the device": torch.tensor(1533).cuda(),
+               "numpy": np.int64(1533)}.get(longest, longest)
+    context = AttentionContext(max_seqlen_k=longest, **fields)
+    attn(*qkv, AttentionContext(**fields))       # code objects are loaded
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        out = attn(*qkv, context)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    _check(out, want)
