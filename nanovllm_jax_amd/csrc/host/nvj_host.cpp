@@ -244,11 +244,6 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // anyway, the store leaves a packed copy
   Tensor k_rows, v_rows, parts, out;
   OtherThreadsRun released;
-  const size_t part_bytes = paged ? nvj_paged_prefill_split_workspace_bytes(
-                                        tokens, batch, heads, c.heads, c.page, tables->size(1),
-                                        max_keys)
-                                  : 0;
-  if (part_bytes) parts = at::empty({(int64_t)part_bytes}, q->options().dtype(at::kByte));
   void *kp = key->data_ptr(), *vp = value->data_ptr(), *k_copy = nullptr, *v_copy = nullptr;
   if (!paged && key->scalar_type() == at::kFloat) {
     k_rows = at::empty(key->sizes(), q->options());
@@ -259,6 +254,16 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     vp = v_copy = v_rows.data_ptr();
   }
   out = at::empty_like(*q);
+  size_t part_bytes = paged ? nvj_paged_prefill_split_workspace_bytes(
+                                  tokens, batch, heads, c.heads, c.page, tables->size(1), max_keys)
+                            : 0;
+  if (part_bytes) {   // (behind everything that a call cannot do without)
+    try {
+      parts = at::empty({(int64_t)part_bytes}, q->options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {
+      part_bytes = 0;   // no memory to spare: the keys stay whole
+    }
+  }
   const int32_t* cq = static_cast<const int32_t*>(cu_q->data_ptr());
   const int32_t* ck = static_cast<const int32_t*>(cu_k->data_ptr());
   if (!paged && !k_copy && !v_copy) {   // rows the attention can read as they are
@@ -269,16 +274,20 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return result(&released, &out, code);
   }
   int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
-  if (code == NVJ_OK)
-    code = paged ? nvj_paged_prefill_split_launch(
-                       stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
-                       static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(),
-                       part_bytes ? parts.data_ptr() : nullptr, part_bytes, tokens, batch, heads,
-                       c.heads, c.dim, c.page, tables->size(1), c.num_blocks, max_keys,
-                       (float)scale, c.dtype)
-                 : nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck,
-                                                out.data_ptr(), tokens, batch, heads, c.heads,
-                                                c.dim, (float)scale, c.dtype);
+  if (code == NVJ_OK && part_bytes)
+    code = nvj_paged_prefill_split_launch(
+        stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
+        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(), parts.data_ptr(),
+        part_bytes, tokens, batch, heads, c.heads, c.dim, c.page, tables->size(1), c.num_blocks,
+        max_keys, (float)scale, c.dtype);
+  else if (code == NVJ_OK && paged)
+    code = nvj_paged_prefill_attention_launch(
+        stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
+        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(), tokens, batch,
+        heads, c.heads, c.dim, c.page, tables->size(1), c.num_blocks, (float)scale, c.dtype);
+  else if (code == NVJ_OK)
+    code = nvj_prefill_attention_launch(stream, q->data_ptr(), kp, vp, cq, ck, out.data_ptr(),
+                                        tokens, batch, heads, c.heads, c.dim, (float)scale, c.dtype);
   return result(&released, &out, code);
 }
 

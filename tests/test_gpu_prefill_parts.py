@@ -108,3 +108,34 @@ def test_longest_length_that_is_no_number_at_hand(longest, paged, native_only):
     finally:
         torch.cuda.set_sync_debug_mode("default")
     _check(out, want)
+
+
+@pytest.mark.parametrize("new,cached,Hq,Hkv", [([30], [5000], 32, 8), ([500], [4200], 32, 8)])
+def test_partials_that_find_no_memory(new, cached, Hq, Hkv):
+    """Without memory for partials a call is what it is where keys are not cut."""
+    print(f"case no memory for partials {new} {cached}", flush=True)
+    import torch
+    from nanovllm_jax_amd import create_prefill_context, paged_prefill_attention
+    attn, qkv, f, want = _call(new, cached, Hq, Hkv)
+    context = create_prefill_context(f["cu_seqlens_q"], f["cu_seqlens_k"], max(new),
+                                     new[0] + cached[0], f["slot_mapping"], f["block_tables"])
+    need = _parts(f, Hq, Hkv, 64, context.max_seqlen_k)
+    assert need > 4 << 20
+    room, held = torch.empty_like(qkv[0]), []    # room for the result, and none for the partials
+    torch.cuda.synchronize()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(need, dtype=torch.uint8, device="cuda:0"))
+        del room
+        out = attn(*qkv, context)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    del held
+    whole = paged_prefill_attention(qkv[0], attn.k_cache, attn.v_cache, f["block_tables"],
+                                    f["cu_seqlens_q"], f["cu_seqlens_k"], attn.scale)
+    assert torch.equal(out, whole)
+    _check(out, want)
+    _check(attn(*qkv, context), want)            # and with memory again
