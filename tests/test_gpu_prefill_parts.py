@@ -139,3 +139,18 @@ def test_partials_that_find_no_memory(new, cached, Hq, Hkv):
     assert torch.equal(out, whole)
     _check(out, want)
     _check(attn(*qkv, context), want)            # and with memory again
+
+
+def test_longest_length_not_known_means_whole():
+    """Without a bound on the lengths keys stay whole, however wide the tables: the bits are those
+    of every other way to this call, alone or in a batch."""
+    print("case unknown longest length", flush=True)
+    import torch
+    from nanovllm_jax_amd import AttentionContext, paged_prefill_attention
+    attn, qkv, fields, want = _call([30, 5], [3000, 100])
+    assert _parts(fields, 32, 8, 64, 0) > 0
+    out = attn(*qkv, AttentionContext(**fields))
+    whole = paged_prefill_attention(qkv[0], attn.k_cache, attn.v_cache, fields["block_tables"],
+                                    fields["cu_seqlens_q"], fields["cu_seqlens_k"], attn.scale)
+    assert torch.equal(out, whole)
+    _check(out, want)
