@@ -2033,8 +2033,13 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
   const int length1 = max(shortest, divide_small_up(total, most - rows / 2));
   int length0 = max(shortest, divide_small_up(total, most));
   if (length0 > NW && most > enough) length0 = (length0 + NW - 1) / NW * NW;
-  const int n0 = divide_small_up(steps_here, length0), n1 = divide_small_up(steps_here, length1);
-  const int n2 = divide_small_up(steps_here, length2);
+  // A row of up to a step a wave is one piece whatever the length, as one step would be: it is no
+  // longer in one workgroup, and there is nothing to put together across workgroups (one sequence of 83
+  // positions, 8 / 1 heads, in tables of 1024, 6.9 us in pieces of 2 steps, 4.9 whole; 44 of 129
+  // 7.9 / 6.1).
+  const int to_cut = steps_here <= NW ? min(steps_here, 1) : steps_here;
+  const int n0 = divide_small_up(to_cut, length0), n1 = divide_small_up(to_cut, length1);
+  const int n2 = divide_small_up(to_cut, length2);
   const int counts = wave_inclusive_scan(n0 | n1 << 10 | n2 << 20);
   const int all = __builtin_amdgcn_readlane(counts, 63);
   const int pick = (all & 1023) <= most ? 0 : (all >> 10 & 1023) <= most ? 10 : 20;

@@ -1168,6 +1168,37 @@ def test_pieces_of_any_number_of_steps(lens, Hq, Hkv, bs, width):
     assert (got.float() - whole.float()).abs().max() <= 2.0 ** -7 * whole.float().abs().max()
 
 
+def _partials_written(lens, Hq, Hkv, bs, width):
+    """Partials (of all heads that share a KV head) that a launch by pieces leaves."""
+    import torch
+    from nanovllm_jax_amd import _lib, paged_attention
+    from nanovllm_jax_amd.layers.paged_attention import DecodeWorkspace
+    B, dev = len(lens), "cuda:0"
+    NB = sum(-(-n // bs) for n in lens) + 3
+    q, kc, vc, bt, ctx = make_problem(5 + B, B, Hq, Hkv, 128, bs, NB, lens)
+    wide = np.full((B, width // bs), -1, np.int32)
+    wide[:, :bt.shape[1]] = bt
+    assert route_of_pieces(B, Hkv, width // bs, bs) == "pieces"
+    t = [bits_to_torch(x, dev) for x in (q, kc, vc)] + [torch.from_numpy(x).to(dev)
+                                                        for x in (wide, ctx)]
+    ws = DecodeWorkspace.for_shape(B, Hq, 128, wide.shape[1], bs, Hkv, dev)
+    ws.buffer.fill_(0xFF)
+    got = paged_attention(*t, 128 ** -0.5, bs, phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
+                          | _lib.NVJ_PHASE_SHORT_ROWS, workspace=ws)
+    assert_close_bf16(torch_to_bits(got), oracle(q, kc, vc, bt, ctx, 128 ** -0.5, bs), what="pieces")
+    records = ws.buffer.numel() // (130 * 4)         # 128 sums, a maximum and their total
+    rows = ws.buffer[:records * 512].view(records, 512)
+    return int((rows != 0xFF).any(1).sum()) // (Hq // Hkv)
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,width", [([83], 8, 1, 1024), ([256, 1, 65, 0], 16, 8, 1024),
+                                               ([129] * 44, 8, 1, 1024), ([82, 26, 200], 64, 8, 1024)])
+def test_rows_of_a_step_a_wave_stay_whole(lens, Hq, Hkv, width):
+    """Up to 8 steps are a step for each wave of one workgroup: nothing to gain from a second one."""
+    print(f"case short rows in one piece {lens[:4]}", flush=True)
+    assert _partials_written(lens, Hq, Hkv, 64, width) == 0
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(8, 4), (64, 8), (6, 2), (16, 1)])   # 4, 4, 2, 1 heads side by side
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("hi", [200, 4000])              # sub-runs of one step, and of many
