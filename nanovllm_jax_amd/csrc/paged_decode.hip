@@ -1956,9 +1956,11 @@ __device__ __forceinline__ int divide_small_up(int x, int d) { return divide_sma
 
 // The shortest piece, in steps.  A step less is 0.2 us less of one wave's chain, and pieces of fewer
 // than 8 steps leave waves idle but have fewer parts to put together and let more CUs draw a row;
-// yet each piece is a partial more for the one that merges them.  So a row gets up to `enough` pieces:
-// 12, or what is merged in one round of loads, 8 with more than 4 query heads a KV head and 4 with
-// more than 8; but no piece is longer than 8 steps, one a wave, while there are workgroups.  us,
+// yet each piece is a partial more for the one that merges them.  So the longest row gets up to
+// `per_row` pieces: 12, or what is merged in one round of loads, 8 with more than 4 query heads a KV
+// head and 4 with more than 8 (the mean row: a row of 4021 positions among 60 of 1 was 63 pieces of 2
+// steps, 18.9 us, in 16 of 8 11.2; one of 1892 among 9 of 20, 64 / 8 heads, 12.3 / 9.7); but no piece
+// is longer than 8 steps, one a wave, while there are workgroups.  us,
 // one sequence, 8 KV heads, at most 8 / 12 / 16 / 32 pieces a row: 768 positions 7.82 / 7.72 / 7.73 /
 // 7.70 (in pieces of 8 steps 8.75, of one 8.81), 1500 8.97 / 8.42 / 8.56 / 9.22, 2048 9.14 / 8.89 /
 // 8.91 / 10.21; 64 query heads at most 8 / 12, 1087 positions 8.81 / 9.76, 2 sequences of 1325 9.55 /
@@ -2027,8 +2029,11 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
   // there can be, and one between.  (A search by bisection found the shortest, at a scan and a
   // division per try: 1.1 us of 8 ragged sequences' 12.3.)
   const int rows = __popcll(__ballot(steps_here > 0));
-  const int enough = max(rows, 1) * (a.group > 8 ? 4 : a.group > 4 ? 8 : 12);
-  const int shortest = min(max(divide_small_up(total, enough), kShortestPiece), NW);
+  const int per_row = a.group > 8 ? 4 : a.group > 4 ? 8 : 12;   // what is put together at once
+  const int enough = max(rows, 1) * per_row;
+  int shortest = min(max(divide_small_up(total, enough), kShortestPiece), NW);
+  if (__any(steps_here > per_row * shortest))   // (equal rows pay no maximum: 0.07 us)
+    shortest = min(divide_small_up(wave_max(steps_here), per_row), NW);
   const int length2 = max(shortest, divide_small_up(total, max(most - rows, 1)));
   const int length1 = max(shortest, divide_small_up(total, most - rows / 2));
   int length0 = max(shortest, divide_small_up(total, most));

@@ -1199,6 +1199,18 @@ def test_rows_of_a_step_a_wave_stay_whole(lens, Hq, Hkv, width):
     assert _partials_written(lens, Hq, Hkv, 64, width) == 0
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,width", [
+    ([4021] + [1] * 60, 8, 1, 4032), ([2616] + [20] * 11, 8, 1, 4096), ([20] * 9 + [1892], 64, 8, 1920),
+    ([1, 5964] + [1] * 5, 28, 4, 24000)])
+def test_a_long_row_among_short_ones_is_cut_by_its_own_length(lens, Hq, Hkv, width):
+    """What one workgroup puts together is bounded by the longest row, not by the mean one: as
+    many partials as fit a round of loads, or pieces of 8 steps."""
+    print(f"case long row among short ones {max(lens)} of {len(lens)}", flush=True)
+    steps = -(-max(lens) // 32)
+    enough = {1: 12, 2: 12, 4: 12, 7: 8, 8: 8}[Hq // Hkv]
+    assert _partials_written(lens, Hq, Hkv, 32, width) <= max(enough, -(-steps // 8)) * Hkv
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(8, 4), (64, 8), (6, 2), (16, 1)])   # 4, 4, 2, 1 heads side by side
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("hi", [200, 4000])              # sub-runs of one step, and of many
