@@ -1186,7 +1186,8 @@ def _partials_written(lens, Hq, Hkv, bs, width):
     got = paged_attention(*t, 128 ** -0.5, bs, phases=_lib.NVJ_PHASE_SPLITK | _lib.NVJ_PHASE_COMBINE
                           | _lib.NVJ_PHASE_SHORT_ROWS, workspace=ws)
     assert_close_bf16(torch_to_bits(got), oracle(q, kc, vc, bt, ctx, 128 ** -0.5, bs), what="pieces")
-    records = ws.buffer.numel() // (130 * 4)         # 128 sums, a maximum and their total
+    head = _lib.load().nvj_paged_decode_counter_bytes(B, Hq, Hkv)    # counted, and not in it
+    records = (ws.buffer.numel() - head) // (130 * 4)    # 128 sums, a maximum and their total
     rows = ws.buffer[:records * 512].view(records, 512)
     return int((rows != 0xFF).any(1).sum()) // (Hq // Hkv)
 
@@ -1209,6 +1210,18 @@ def test_a_long_row_among_short_ones_is_cut_by_its_own_length(lens, Hq, Hkv, wid
     steps = -(-max(lens) // 32)
     enough = {1: 12, 2: 12, 4: 12, 7: 8, 8: 8}[Hq // Hkv]
     assert _partials_written(lens, Hq, Hkv, 32, width) <= max(enough, -(-steps // 8)) * Hkv
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,width,pieces", [
+    ([51 * 32] * 10 + [1] * 21, 4, 4, 1664, 40),     # of 16 steps; 17 always fit
+    ([32 * n for n in (32, 30, 28, 25, 22, 20, 15, 12, 8, 5, 4)], 16, 16, 1024, 8),   # of 24; 41
+    ([35 * 32] * 16 + [32] * 32, 8, 4, 1120, 32),    # of 32, the second of the two; 37
+])
+def test_pieces_of_lengths_that_differ_much(lens, Hq, Hkv, width, pieces):
+    """Where the shorter lengths do not fit, multiples of 8 steps are tried in front of the one that
+    always does.  Pieces of rows that have more than one."""
+    print(f"case lengths that differ much {len(lens)} rows Hq={Hq} Hkv={Hkv}", flush=True)
+    assert _partials_written(lens, Hq, Hkv, 32, width) == pieces * Hkv
 
 
 @pytest.mark.parametrize("Hq,Hkv", [(8, 4), (64, 8), (6, 2), (16, 1)])   # 4, 4, 2, 1 heads side by side
