@@ -1647,11 +1647,16 @@ struct SharedRows {
     }
   }
   // merge_row for this wave's pieces.  The whole of it runs once in a launch, so its instructions
-  // count as they stand, cold in the instruction cache: pairs by slots, as merge_row has them, are
-  // 16 loads, LDS writes and masked maxima whatever the group; by heads they are 4 for up to four.
-  // The one round of loads left in front of it is the partials' own.  With the reciprocals of Cut,
-  // 16 / 8 heads: 4 sequences of 100 .. 900 positions 10.2 -> 9.1 us, 1 of 700 9.7 -> 8.6, of 8000
-  // 17.9 -> 14.3, 4 of 3000 15.0 -> 13.8, 16 of 1000 16.2 -> 15.1; 32 / 8 heads the same.
+  // count as they stand, cold in the instruction cache.  HEADS, up to four query heads a KV head: the
+  // (max, sum) pairs are fetched by heads, a slot per lane, 4 loads, LDS writes and masked maxima
+  // where by slots, as merge_row has them, they are 16; and the one round of loads left in front of it
+  // is the partials' own.  With the reciprocals of Cut, 16 / 8 heads: 4 sequences of 100 .. 900 positions
+  // 10.5 -> 8.9 us, 1 of 700 10.1 -> 8.5, of 8000 18.2 -> 13.6, 4 of 3000 15.4 -> 13.9, 16 of 1000 16.6 ->
+  // 15.2; 32 / 8 heads the same.  By heads every lane's pair lies in a line of its own, so with more of
+  // them it costs more than it saves, us by slots / by heads: 64 / 8 heads, 4 of 3000 15.9 / 17.3, 1 of
+  // 8252 among 32 of 20 40.2 / 47.7; 16 / 1, 1 of 700 9.7 / 11.0, of 8000 16.7 / 30.0; only one short
+  // sequence with 7 or 8 is the other way round (8 / 1, 1 of 700 9.3 / 8.8, 28 / 4 9.5 / 9.1).
+  template <bool HEADS>
   static __device__ __forceinline__ void merge_pieces(const DecodeArgs& a, uint4* lds, int b,
                                                       int kvh, int part, int r0, int r1,
                                                       const Cut& cut, int lane) {
@@ -1673,23 +1678,35 @@ struct SharedRows {
     const int slot_bytes = rec_stride * D * (int)sizeof(float);
     const int piece_stride = KG * a.group * 16;
     const int lane_off = (kg * a.group + r) * 16 + kPieces * part * piece_stride;
-    vfloat2* lds_ml = reinterpret_cast<vfloat2*>(lds);
+    vfloat2* lds_ml = reinterpret_cast<vfloat2*>(lds);   // HEADS: [4][kSlots], else [kSlots][16]
     uint8_t* lds_list = reinterpret_cast<uint8_t*>(lds_ml + kSlots * 16);
     f32x4 acc[kPieces];
 #pragma unroll
     for (int u = 0; u < kPieces; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = kNegBig, l_run = 0.f;
+    const auto fence = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const auto rescale = [&](float m_chunk) __attribute__((always_inline)) {
+      const float m_new = fmaxf(m_run, m_chunk);
+      const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
+      m_run = m_new;
+      l_run *= keep;
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) acc[u] *= keep;
+    };
     for (int base = 0; base < expected; base += kSlots) {
       const int count = min(kSlots, expected - base);
-      // the (max, sum) pairs of the heads, a slot per lane, the last over again
-      const int slot_at = min(base + lane, expected - 1) * rec_stride * 8;
-      vfloat2 got[16];
+      constexpr int kPairs = HEADS ? 4 : kSlots / 4;
+      vfloat2 got[kPairs];   // (past the end the last slot or head over again)
 #pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        if (c > 0 && c % 4 == 0 && c >= a.group) break;
-        got[c] = __builtin_bit_cast(
-            vfloat2, __builtin_amdgcn_raw_buffer_load_b64(wm, slot_at, min(c, a.group - 1) * 8,
-                                                          kDeviceScope));
+      for (int i = 0; i < kPairs; ++i) {
+        const int slot = min(base + (HEADS ? lane : 4 * i + kg), expected - 1);
+        const int head = min(HEADS ? i : lane & 15, a.group - 1);
+        got[i] = __builtin_bit_cast(vfloat2, __builtin_amdgcn_raw_buffer_load_b64(
+                                                 wm, (slot * rec_stride + head) * 8, 0, kDeviceScope));
       }
       // which slots hold a partial, while these are on their way (see merge_row)
       const int j = first + base + lane;
@@ -1700,11 +1717,22 @@ struct SharedRows {
       const unsigned long long real = __ballot(mine_real);
       const int nreal = __popcll(real);
       if (mine_real) lds_list[__popcll(real & ((1ull << lane) - 1ull))] = (uint8_t)lane;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if constexpr (!HEADS) {
+        float m_chunk = kNegBig;
+#pragma unroll
+        for (int i = 0; i < kPairs; ++i) {
+          lds_ml[(4 * i + kg) * 16 + (lane & 15)] = got[i];
+          const int sl = min(4 * i + kg, count - 1);
+          if ((real >> sl) & 1ull) m_chunk = fmaxf(m_chunk, got[i].x);
+        }
+        fence();
+        if (nreal > 0)
+          rescale(__shfl(wave_xor_max<32>(wave_xor_max<16>(m_chunk)), (lane & 48) | r, 64));
+      } else {
+        fence();
+      }
       for (int done = 0; done < nreal; done += 4 * lane_groups) {
-        // the partials; the first are asked for while the pairs are on their way
+        // the partials; by heads the first are asked for while the pairs are on their way
         int idx[4];
         vfloat4 v[4][kPieces];
 #pragma unroll
@@ -1718,18 +1746,14 @@ struct SharedRows {
                 vfloat4, __builtin_amdgcn_raw_buffer_load_b128(wo, off + u * piece_stride, 0,
                                                                kDeviceScope));
         }
-        if (done == 0) {
-          // their maxima over the slots, four heads at a time: two halving steps leave lane L
-          // with head L % 4 of the four
-          float m_chunk = kNegBig;
-#pragma unroll
-          for (int c = 0; c < 16; c += 4) {
-            if (c > 0 && c >= a.group) break;
+        if constexpr (HEADS) {
+          if (done == 0) {
+            // their maxima over the slots: two halving steps leave lane L with head L % 4
             float m[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              lds_ml[(c + i) * kSlots + lane] = got[c + i];
-              m[i] = mine_real ? fmaxf(got[c + i].x, kNegBig) : kNegBig;
+              lds_ml[i * kSlots + lane] = got[i];
+              m[i] = mine_real ? fmaxf(got[i].x, kNegBig) : kNegBig;
             }
             const bool odd = lane & 1, upper = lane & 2;
             const float m0 = fmaxf(odd ? m[1] : m[0], dpp_partner<kDppQuadXor1>(odd ? m[0] : m[1]));
@@ -1738,23 +1762,15 @@ struct SharedRows {
             most = fmaxf(most, row_rotate<4>(most));
             most = fmaxf(most, row_rotate<8>(most));
             most = wave_xor_max<32>(wave_xor_max<16>(most));
-            most = __shfl(most, (lane & 48) | (r & 3), 64);
-            if (r >= c) m_chunk = most;
+            most = __shfl(most, (lane & 48) | r, 64);
+            fence();
+            rescale(most);
           }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          const float m_new = fmaxf(m_run, m_chunk);
-          const float keep = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2e);
-          m_run = m_new;
-          l_run *= keep;
-#pragma unroll
-          for (int u = 0; u < kPieces; ++u) acc[u] *= keep;
         }
         float w[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const vfloat2 ml = lds_ml[r * kSlots + idx[k]];
+          const vfloat2 ml = lds_ml[HEADS ? r * kSlots + idx[k] : idx[k] * 16 + r];
           w[k] = done + k * lane_groups + lg < nreal
                      ? __builtin_amdgcn_exp2f((ml.x - m_run) * a.scale_log2e)
                      : 0.f;
@@ -1895,8 +1911,12 @@ __global__ __launch_bounds__(512) void paged_decode_shared_kernel(DecodeArgs a, 
       if (lane == 0) last[h_in_row] = to_merge;
     }
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(last[h_in_row]))
-      R::merge_pieces(a, k_tile[wave], b, kvh, part, row0, row0 + nb0, cut, lane);
+    if (__builtin_amdgcn_readfirstlane(last[h_in_row])) {
+      if (a.group > 4)
+        R::template merge_pieces<false>(a, k_tile[wave], b, kvh, part, row0, row0 + nb0, cut, lane);
+      else
+        R::template merge_pieces<true>(a, k_tile[wave], b, kvh, part, row0, row0 + nb0, cut, lane);
+    }
     return;
   }
 
