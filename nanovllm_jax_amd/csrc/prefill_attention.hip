@@ -1093,7 +1093,9 @@ bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
 // Longest tiles first: behind cached prefixes, up to 8 rounds of two workgroups per CU.  Packed
 // prompts of more than a round and at most 5 / 4: 8 of 500 tokens, 16 / 8 heads, 21.7 -> 19.7 us, 4
 // of 1000 31.0 -> 28.4, 2 of 1000, 32 / 8, 30.0 -> 27.1, 8 of 165..945 27.1 -> 27.0; with 4 a CU and
-// more -5 .. +12 %.
+// more -5 .. +12 %.  Each XCD takes an eighth of the list: unless that is whole KV heads, one gets
+// the long tiles and another the short ones (8 / 1 heads, 11 of 624..775 30.8 -> 40.7, 28 / 4, 3 of
+// 823..968 31.0 -> 39.4).
 constexpr int64_t kLongestFirstPerCu = 16;
 
 constexpr int64_t kMostSplits = 32;
@@ -1170,7 +1172,7 @@ int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, const TileForm
   const bool may_sort =
       a.batch > 1 && a.batch <= 256 &&
       (paged ? items <= kLongestFirstPerCu * cus && (int64_t)a.max_blocks * a.page.d >= 1024
-             : form.groups == 2 && items * 2 <= cus * 5);
+             : form.groups == 2 && items * 2 <= cus * 5 && a.num_kv_heads % 8 == 0);
   const bool f16 = dtype == NVJ_DTYPE_F16;
   if (a.part_o) {
     const dim3 parts(grid.x, (unsigned)a.splits.d), eighths(grid.x, 8);
