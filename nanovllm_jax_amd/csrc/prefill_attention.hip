@@ -1058,8 +1058,12 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
   // of 1500, 32 heads, 35 -> 29, 8 of 30..200 behind 500..4000 82 -> 66 (two a CU: 79 .. 111 %).
   // Behind cached prefixes, where the tiles of a sequence are equally long, up to one round of the
   // small ones: 3 of 180 behind 2800, 64 / 8, 75 us in 288 larger ones and 95 in 576.
+  // Packed prompts of more than a round that are longer than a block and whose KV heads do not fill
+  // the XCDs evenly keep the larger ones, all of which run at once (8 / 1 heads, 6 of 186..1642 39 us,
+  // in small ones 45, 28 / 4, one of 1731 42 / 47).
+  const bool even = num_kv_heads % 8 == 0 || tokens <= 16 * batch;
   if (paged ? expected_tiles(tokens, batch, group, kWaves) * num_kv_heads <= 2 * cus
-            : wide * num_kv_heads * 2 <= cus * 3)
+            : wide * num_kv_heads * 2 <= cus * (even ? 3 : 2))
     return {1, 4, narrow};
   // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
   // Three small ones to a CU instead, us: 100 prompts of 4 tokens, 16 / 8 heads (2 groups) 11.1 ->
