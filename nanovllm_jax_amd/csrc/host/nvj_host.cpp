@@ -257,15 +257,16 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   // Without a length known to the host the keys stay whole: tables are often wider than what is
   // in them, where parts only cost their second launch (2 of 1 token behind 2 in tables of 1280
   // positions, 32 / 8 heads, 5.1 us whole, 7.0 in parts).
-  size_t part_bytes =
-      max_keys > 0 ? nvj_paged_prefill_split_workspace_bytes(tokens, batch, heads, c.heads, c.page,
-                                                             tables->size(1), max_keys)
-                   : 0;
+  bool may_cut = max_keys > 0;
+  const size_t part_bytes =
+      may_cut ? nvj_paged_prefill_split_workspace_bytes(tokens, batch, heads, c.heads, c.page,
+                                                        tables->size(1), max_keys)
+              : 0;
   if (part_bytes) {   // (behind everything that a call cannot do without)
     try {
       parts = at::empty({(int64_t)part_bytes}, q->options().dtype(at::kByte));
     } catch (const c10::OutOfMemoryError&) {
-      part_bytes = 0;   // no memory to spare: the keys stay whole
+      may_cut = false;   // no memory to spare: the keys stay whole
     }
   }
   const int32_t* cq = static_cast<const int32_t*>(cu_q->data_ptr());
@@ -278,12 +279,12 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return result(&released, &out, code);
   }
   int code = store(stream, *key, *value, c, *slots, k_copy, v_copy, nullptr, 0);
-  if (code == NVJ_OK && part_bytes)
+  if (code == NVJ_OK && may_cut)
     code = nvj_paged_prefill_split_launch(
         stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),
-        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(), parts.data_ptr(),
-        part_bytes, tokens, batch, heads, c.heads, c.dim, c.page, tables->size(1), c.num_blocks,
-        max_keys, (float)scale, c.dtype);
+        static_cast<const int32_t*>(tables->data_ptr()), cq, ck, out.data_ptr(),
+        part_bytes ? parts.data_ptr() : nullptr, part_bytes, tokens, batch, heads, c.heads, c.dim,
+        c.page, tables->size(1), c.num_blocks, max_keys, (float)scale, c.dtype);
   else if (code == NVJ_OK && paged)
     code = nvj_paged_prefill_attention_launch(
         stream, q->data_ptr(), c.k->data_ptr(), c.v->data_ptr(),

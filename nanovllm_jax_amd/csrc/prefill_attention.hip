@@ -1042,42 +1042,55 @@ int64_t most_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_
   const int64_t blocks = (tokens + 15 * batch) / 16;
   return (blocks * group + (column_groups - 1) * batch) / column_groups;
 }
-// The same if the last block and the last tile of every sequence are half full.
+// The same if the last block and the last tile of every sequence are half full, but no less than
+// sequences of a token or a few have.
 int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_groups) {
-  return ((2 * tokens + 15 * batch) * group + 16 * (column_groups - 1) * batch +
-          16 * column_groups) /
-         (32 * column_groups);
+  const int64_t half_full = ((2 * tokens + 15 * batch) * group + 16 * (column_groups - 1) * batch +
+                             16 * column_groups) /
+                            (32 * column_groups);
+  return std::max(half_full,
+                  std::min(tokens, batch) * ((group + column_groups - 1) / column_groups));
 }
+// positions (paged): the most that a sequence has.
 TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
-                   bool paged) {
+                   bool paged, int64_t positions) {
   const int64_t wide = most_tiles(tokens, batch, group, 2 * kWaves);
   const int64_t narrow = most_tiles(tokens, batch, group, kWaves);
+  const int64_t groups = (tokens + 16 * batch - 1) / (16 * batch) * group;   // of a mean prompt
+  const bool xcds_even = num_kv_heads % 8 == 0;   // each takes whole KV heads
   // One column group per wave while the larger workgroups would leave CUs idle or start a second
   // round with little to do: one prompt of 700 tokens, 16 / 8 heads, 21.0 -> 16.2 us; 4 of
   // 70..90, 32 heads, 10.8 -> 9.1; up to 1.5 of them a CU, one prompt of 3000, 16 heads, 62 -> 50,
-  // of 1500, 32 heads, 35 -> 29, 8 of 30..200 behind 500..4000 82 -> 66 (two a CU: 79 .. 111 %).
-  // Behind cached prefixes, where the tiles of a sequence are equally long, up to one round of the
-  // small ones: 3 of 180 behind 2800, 64 / 8, 75 us in 288 larger ones and 95 in 576.
-  // Packed prompts of more than a round that are longer than a block and whose KV heads do not fill
-  // the XCDs evenly keep the larger ones, all of which run at once (8 / 1 heads, 6 of 186..1642 39 us,
-  // in small ones 45, 28 / 4, one of 1731 42 / 47).
-  const bool even = num_kv_heads % 8 == 0 || tokens <= 16 * batch;
-  if (paged ? expected_tiles(tokens, batch, group, kWaves) * num_kv_heads <= 2 * cus
-            : wide * num_kv_heads * 2 <= cus * (even ? 3 : 2))
+  // of 1500, 32 heads, 35 -> 29 (two a CU: 79 .. 111 %).
+  if (wide * num_kv_heads <= cus) return {1, 4, narrow};
+  if (paged) {
+    // Behind cached prefixes, where the tiles of a sequence are equally long, up to 1.5 of the small
+    // ones a CU, and up to two where the keys are few: every small one fetches all of them for half the
+    // rows; 1.25 where the XCDs are not filled evenly.  us, larger / small: 4 of 55..268, at most 277
+    // keys, 32 / 8 heads, 12.0 / 10.3, 2 of 167..263, 557 keys, 64 / 8, 17.7 / 15.4; beyond the line 14
+    // of 3..243, up to 4424 keys, 28 / 4, 94 / 118, 170 of 1..30, 866 keys, 8 / 1, 28.7 / 36.2 (and
+    // within it 32 of 6..40, 3765 keys, 16 / 8, 84 / 102).
+    const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
+    if (!xcds_even) return {small * 4 <= cus * 5 ? 1 : 2, 4, small * 4 <= cus * 5 ? narrow : wide};
+    if (small * 2 <= cus * 3 || (small <= 2 * cus && positions <= 2048)) return {1, 4, narrow};
+    // Prompts of up to 4 groups and 8 tokens, few of which have a second block: the larger
+    // workgroups are mostly empty (with more tokens 155 of 1..63, 16 in the mean, at most 1722 keys, 32
+    // / 8 heads, 140 us in larger ones, 149 in small ones).
+    if (groups <= 4 && tokens <= 8 * batch) return {1, 4, narrow};
+    return {2, 4, wide};
+  }
+  // Prompts that are longer than a block and whose KV heads do not fill the XCDs evenly keep the
+  // larger ones, all of which run at once (8 / 1 heads, 6 of 186..1642 39 us, in small ones 45, 28 / 4,
+  // one of 1731 42 / 47).
+  if ((xcds_even || tokens <= 16 * batch) && wide * num_kv_heads * 2 <= cus * 3)
     return {1, 4, narrow};
   // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
   // Three small ones to a CU instead, us: 100 prompts of 4 tokens, 16 / 8 heads (2 groups) 11.1 ->
   // 8.1, 200 of 16, 32 / 8 (4) 26.0 -> 22.3, 100 of 60, 32 / 32 (4) 67.4 -> 55.4, 60 of 20..60, 32 / 8
   // (12) 17.1 -> 14.8, 40 of 100, 16 / 8 (14) 19.8 -> 17.6; 60 of 20..60, 16 / 8 (6) 10.7 -> 11.2, the
   // only one slower.  Beyond that -13 .. +13 %, with 8 heads to a KV head (8 groups and more) -3 ..
-  // +18 %.  Behind cached prefixes, which they would fetch for fewer rows, three of them are
-  // no better than two (-1 .. +10 % against the larger ones), and two are up to 4 groups and one
-  // block of 16 tokens (100 prompts of 16 behind 200..800, 32 / 8, 48.4 -> 45.1; 32 / 32 188 -> 185;
-  // but 32 of 31..86 behind 1100..1700, 32 / 32, 181 -> 188).
-  const int64_t groups = (tokens + 16 * batch - 1) / (16 * batch) * group;   // of a mean prompt
-  if (groups <= 4 && !paged) return {1, 3, narrow};
-  if (groups <= 4 && tokens <= 16 * batch) return {1, 4, narrow};
-  if (groups <= 14 && group <= 4 && !paged) return {1, 3, narrow};
+  // +18 %.
+  if (groups <= 4 || (groups <= 14 && group <= 4)) return {1, 3, narrow};
   return {2, 4, wide};
 }
 
@@ -1089,7 +1102,7 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
 bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
                  int64_t num_kv_heads, int64_t cus) {
   const int64_t tiles =
-      tile_form(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus, false).tiles *
+      tile_form(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus, false, 0).tiles *
       num_kv_heads;
   return tiles <= 6 * cus || rows * num_kv_heads * kPieces >= 80 * tiles;
 }
@@ -1152,7 +1165,7 @@ SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
       std::max<int64_t>(expected_tiles(tokens, batch, group, 2 * kWaves) * num_kv_heads, 1);
   if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 && large <= cus)
     return {{2, 4, most_tiles(tokens, batch, group, 2 * kWaves)}, 2 * cus / large};
-  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
+  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true, positions);
   return {form, key_splits(form, tokens, batch, group, num_kv_heads, cus, positions)};
 }
 int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
@@ -1287,7 +1300,7 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
     a.new_pieces = (uint32_t)store->rows * (uint32_t)a.row_pieces.d;
   }
   return launch_prefill(static_cast<hipStream_t>(stream), a, false,
-                        tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, false),
+                        tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, false, 0),
                         total_q_tokens, dtype, cus);
 }
 }  // namespace
@@ -1387,15 +1400,16 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
   a.max_blocks = max_blocks;
   a.num_blocks = num_blocks;
   const int64_t cus = nvj::compute_units();
-  TileForm form = tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true);
+  const int64_t positions = most_keys(max_blocks, block_size, max_keys);
+  TileForm form = tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true, positions);
   if (may_split) {
     const size_t need = nvj_paged_prefill_split_workspace_bytes(
         total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks, max_keys);
     if (need > 0) {
       if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
       if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
-      const SplitForm cut = split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus,
-                                       most_keys(max_blocks, block_size, max_keys));
+      const SplitForm cut =
+          split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, positions);
       form = cut.form;
       a.splits = Divisor(cut.splits);
       a.part_o = static_cast<float*>(workspace);
