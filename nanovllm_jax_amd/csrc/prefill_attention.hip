@@ -1121,13 +1121,19 @@ constexpr int64_t kMostSplits = 32;
 // workgroup or two per KV head, each drawing 50 GB/s, 0.47 us a tile of keys, for thousands of keys,
 // while the other CUs idle; in parts they fill one round of two workgroups a CU.  us, whole / in
 // parts: 30 tokens behind 5000, 32 / 8 heads, 75 / 17, 13 behind 5300, 16 / 8, 79 / 14, 270 behind
-// 4200, 32 / 8, 68 / 38, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 26, 16
-// of 16..60 behind 64..4000 62 / 46.  Against that the partials and the launch that merges them are
-// 4 us, whatever the lengths turn out to be, of which the host knows an upper bound: up to 512
-// positions nothing is cut (9 tokens behind 256, 10.6 / 12.3), in busier launches from 1024 or 1536
-// positions on (10 of 43..51 behind 162..400, 14 / 18, 9 of 26..49 behind 89..799 19.4 / 20.2), and
-// not where every query head has keys of its own and half the CUs draw: HBM is the bound then (6 of
-// 21..39 behind 3000, 32 / 32, 64 / 68).  More than a round of parts is slower (4 of 100..300 behind
+// 4200, 32 / 8, 68 / 38, 8 of 13..16 behind 800..5000, 16 / 8, 78 / 26.  Against that the partials and
+// the launch that merges them are 2 .. 10 us and more, whatever the lengths turn out to be, of which
+// the host knows a bound: so the more workgroups there are, the longer the keys have to be.  us, whole / in
+// parts, behind up to 512 positions 9 tokens behind 256, 10.6 / 12.3; 768: 21 sequences of 1 or 2 tokens,
+// 8 / 1, 42 workgroups, 12.1 / 13.9; 1024: 49 of 1..6, 4 / 4, 196 of them, 14.4 / 19.7; 2048: 32 of 3 or
+// 4, 28 / 4, 256 of them, 24.2 / 34.8, 90 of 7, 8 / 1, 197 of them, 29.1 / 42.0; beyond 8 of 1..7 behind
+// 4400, 32 / 32, 256 of them, 96.7 / 120, 53 of 1..3 behind 6500, 4 / 4, 212 of them, 124 / 154.  Sequences of
+// more than a block of tokens, whose tiles share their keys, gain up to a round (1 of 213 behind 1900, 64
+// / 8, 224 of them, 33.9 / 31.7, 6 of 27 behind 3050 48 / 41); where every query head has keys of its own
+// HBM is the bound earlier.  6361 launches drawn from 1..260 sequences of 1..700 tokens behind up to
+// 12000 positions, where the bound is known, against a workgroup for every tile: 1.27 times as fast in
+// the mean, 0.4 % of them more than 5 % slower, at worst 0.78.
+// More than a round of parts is slower (4 of 100..300 behind
 // 1000..4000, 34.7 / 40.2 at twice as many), three quarters of one better where there are many to put
 // together (30 behind 5000 18.5 / 16.9, 20 behind 4000, 32 / 32, 28 / 22.5).  Parts of 4 tiles or of 12
 // instead of 8: +3 .. -1 and -0.7 .. +1.4 us.
@@ -1135,12 +1141,27 @@ struct SplitForm {
   TileForm form;
   int64_t splits;
 };
+// The most workgroups whose keys are cut.
+int64_t most_to_cut(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
+                    int64_t positions) {
+  const bool xcds_even = num_kv_heads % 8 == 0;
+  if (positions <= 2 * kKeys * kShortestPart) return 0;
+  if (positions <= 768) return cus / 8;
+  if (positions <= 1024) return cus / 4;
+  if (positions <= 2048) return cus * (xcds_even ? 4 : 3) / 8;
+  const int64_t most = positions <= 4096 ? cus * (xcds_even ? 6 : 5) / 8
+                       : xcds_even       ? cus * 15 / 16
+                                         : cus * 6 / 8;
+  if (group == 1) return std::min(most, cus * 6 / 8);
+  return xcds_even && tokens > 16 * batch ? cus : most;
+}
 int64_t key_splits(const TileForm& form, int64_t tokens, int64_t batch, int64_t group,
                    int64_t num_kv_heads, int64_t cus, int64_t positions) {
-  if (form.groups != 1 || batch > 256) return 1;
   const int64_t workgroups =
       std::max<int64_t>(expected_tiles(tokens, batch, group, kWaves) * num_kv_heads, 1);
-  if (positions <= 2 * kKeys * kShortestPart || (group == 1 && workgroups * 2 > cus)) return 1;
+  if (form.groups != 1 || batch > 256 ||
+      workgroups > most_to_cut(tokens, batch, group, num_kv_heads, cus, positions))
+    return 1;
   const bool few = workgroups * 4 <= cus;
   const int64_t shortest = kKeys * kShortestPart * (few ? 1 : workgroups * 2 <= cus ? 2 : 3);
   return std::max<int64_t>(std::min<int64_t>({(few ? 3 * cus / 2 : 2 * cus) / workgroups,
@@ -1153,17 +1174,20 @@ int64_t key_splits(const TileForm& form, int64_t tokens, int64_t batch, int64_t 
 // twice the rows).  Where the small ones would be cut into two or three parts or none at all the larger
 // ones in parts, up to two a CU, are the shorter way behind more than 4096 positions.  us, before /
 // so: 500 behind 5000, 32 / 8 heads, 69 / 60, 700 behind 5000 90 / 81, 512 behind 8000, 64 / 8, 157 /
-// 133, 400 behind 4000, 32 / 32, 68 / 51, 6 of 23..44 behind 8555..10940, 64 / 8, 148 / 99; 50 launches
-// drawn from 70 .. 400 large workgroups -2 .. +49 %.  Up to 4096 positions the partials cost more
-// (1000 behind 2000 55 / 62), with fewer rows many small parts are as good (270 behind 4200 37.6 / 36.4,
-// 150 behind 4000, 32 / 32, 29 / 33), with more large workgroups than CUs two parts each are not
-// (4 of 244..494 behind 3357..5499, 368 of them, 125 / 151).
+// 133, 400 behind 4000, 32 / 32, 68 / 51, 6 of 23..44 behind 8555..10940, 64 / 8, 148 / 99.  Up to
+// 4096 positions the partials cost more (1000 behind 2000 55 / 62), with fewer rows many small parts
+// are as good (270 behind 4200 37.6 / 36.4, 150 behind 4000, 32 / 32, 29 / 33), with as many large
+// workgroups as CUs two parts each are not (168 of 5..18 behind 3500, 8 / 1, 250 of them, 119 / 160, 4 of
+// 244..494 behind 3357..5499, 368 of them, 125 / 151), and nor are they where they are hardly fewer than
+// the small ones, half empty (55 of 2 behind 2500, 16 / 8, 126 / 153, 7 of 12 behind 7350, 32 / 32, 138 /
+// 174).
 SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads,
                      int64_t cus, int64_t positions) {
   const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
   const int64_t large =
       std::max<int64_t>(expected_tiles(tokens, batch, group, 2 * kWaves) * num_kv_heads, 1);
-  if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 && large <= cus)
+  if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 &&
+      large * 16 <= cus * (num_kv_heads % 8 == 0 ? 15 : 12) && large * 4 <= small * 3)
     return {{2, 4, most_tiles(tokens, batch, group, 2 * kWaves)}, 2 * cus / large};
   const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true, positions);
   return {form, key_splits(form, tokens, batch, group, num_kv_heads, cus, positions)};
