@@ -1116,6 +1116,7 @@ bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
 constexpr int64_t kLongestFirstPerCu = 16;
 
 constexpr int64_t kMostSplits = 32;
+constexpr int64_t kNeverCut = 2 * kKeys * kShortestPart;   // positions
 
 // Parts that a query tile's keys may be cut into; 1: none.  Few rows behind a long prefix are a
 // workgroup or two per KV head, each drawing 50 GB/s, 0.47 us a tile of keys, for thousands of keys,
@@ -1145,7 +1146,7 @@ struct SplitForm {
 int64_t most_to_cut(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
                     int64_t positions) {
   const bool xcds_even = num_kv_heads % 8 == 0;
-  if (positions <= 2 * kKeys * kShortestPart) return 0;
+  if (positions <= kNeverCut) return 0;
   if (positions <= 768) return cus / 8;
   if (positions <= 1024) return cus / 4;
   if (positions <= 2048) return cus * (xcds_even ? 4 : 3) / 8;
@@ -1195,7 +1196,13 @@ SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
 int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
   return max_keys > 0 ? std::min(max_keys, max_blocks * block_size) : max_blocks * block_size;
 }
-constexpr size_t kGroupBytes = (8 * 64 * sizeof(float4) + 16 * sizeof(float2));
+// Bytes of the partials of a launch, 0 where its keys are not cut.
+size_t part_bytes(const SplitForm& cut, int64_t num_kv_heads) {
+  constexpr size_t kGroupBytes = 8 * 64 * sizeof(float4) + 16 * sizeof(float2);
+  if (cut.splits <= 1) return 0;
+  const int64_t workgroups = (cut.form.tiles * num_kv_heads + 7) / 8 * 8;
+  return (size_t)(workgroups * cut.splits * cut.form.groups * kWaves) * kGroupBytes;
+}
 
 int launch_prefill(hipStream_t stream, PrefillArgs a, bool paged, const TileForm& form,
                    int32_t total_q_tokens, int32_t dtype, int64_t cus) {
@@ -1425,21 +1432,19 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
   a.num_blocks = num_blocks;
   const int64_t cus = nvj::compute_units();
   const int64_t positions = most_keys(max_blocks, block_size, max_keys);
-  TileForm form = tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true, positions);
-  if (may_split) {
-    const size_t need = nvj_paged_prefill_split_workspace_bytes(
-        total_q_tokens, batch, num_heads, num_kv_heads, block_size, max_blocks, max_keys);
-    if (need > 0) {
-      if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
-      if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
-      const SplitForm cut =
-          split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, positions);
-      form = cut.form;
-      a.splits = Divisor(cut.splits);
-      a.part_o = static_cast<float*>(workspace);
-    }
+  const SplitForm cut =
+      may_split ? split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, positions)
+                : SplitForm{tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true,
+                                      positions),
+                            1};
+  if (const size_t need = part_bytes(cut, num_kv_heads)) {
+    if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
+    if (reinterpret_cast<uintptr_t>(workspace) & 15u) return NVJ_ERR_ALIGNMENT;
+    a.splits = Divisor(cut.splits);
+    a.part_o = static_cast<float*>(workspace);
   }
-  return launch_prefill(static_cast<hipStream_t>(stream), a, true, form, total_q_tokens, dtype, cus);
+  return launch_prefill(static_cast<hipStream_t>(stream), a, true, cut.form, total_q_tokens, dtype,
+                        cus);
 }
 }  // namespace
 
@@ -1461,12 +1466,11 @@ extern "C" size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens
   if (total_q_tokens <= 0 || batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || block_size <= 0 || max_blocks <= 0)
     return 0;
-  const int64_t cus = nvj::compute_units(), group = num_heads / num_kv_heads;
-  const SplitForm cut = split_form(total_q_tokens, batch, group, num_kv_heads, cus,
-                                   most_keys(max_blocks, block_size, max_keys));
-  if (cut.splits <= 1) return 0;
-  const int64_t workgroups = (cut.form.tiles * num_kv_heads + 7) / 8 * 8;
-  return (size_t)(workgroups * cut.splits * cut.form.groups * kWaves) * kGroupBytes;
+  const int64_t positions = most_keys(max_blocks, block_size, max_keys);
+  if (positions <= kNeverCut) return 0;   // (without asking for the CUs, 70 ns)
+  return part_bytes(split_form(total_q_tokens, batch, num_heads / num_kv_heads, num_kv_heads,
+                               nvj::compute_units(), positions),
+                    num_kv_heads);
 }
 
 extern "C" int nvj_paged_prefill_split_launch(
