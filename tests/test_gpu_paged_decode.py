@@ -1047,8 +1047,8 @@ def test_short_rows_that_do_not_go_by_pieces(B, Hq, Hkv, D, positions):
 def route_of_pieces(batch, kv_heads, max_blocks, bs, lens=None):
     """Where a launch of short rows goes (head_dim 128, groups of 16 at most), as the host
     decides it: "table", every row inside one workgroup, "pieces", or "balanced".  With lengths,
-    pieces by way of the kernel's own choice as well: "pieces" when the mean length per workgroup
-    is one that fits, "search" when a longer one has to be looked for."""
+    which of them leave more pieces of the mean length, in multiples of 8 steps, than there are
+    workgroups: "search", the kernel then takes a longer length than its first."""
     import torch
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     rows, positions = batch * kv_heads, max_blocks * bs
@@ -1068,7 +1068,7 @@ def route_of_pieces(batch, kv_heads, max_blocks, bs, lens=None):
 
 
 @pytest.mark.parametrize("lens,Hq,Hkv,route", [
-    ([1000], 16, 8, "pieces"),                    # four pieces a row
+    ([1000], 16, 8, "pieces"),                    # eleven pieces a row
     ([4100], 2, 2, "pieces"),                     # 17, one of them short of a step
     ([6000, 0, 1, 33], 6, 2, "pieces"),           # a group of 3, an empty row, one lone row
     ([300, 2048, 900, 257, 0, 1024, 700, 5], 32, 8, "pieces"),
