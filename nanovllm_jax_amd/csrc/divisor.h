@@ -8,10 +8,9 @@
 namespace nvj {
 
 // x / d for 0 <= x < 2^31 as a multiplication (a division by a number only known at run time is 20
-// instructions and more, and a
-// launch's workgroups are in front of their first load meanwhile).  With
-// bits = ceil(log2 d) the multiplier m = ceil(2^(31 + bits) / d) has 32 bits, and x * m / 2^(31 +
-// bits) exceeds x / d by less than x / 2^31 / d: the whole part is the same.
+// instructions and more, and a launch's workgroups are in front of their first load meanwhile).  With
+// bits = ceil(log2 d) the multiplier m = ceil(2^(31 + bits) / d) has 32 bits, and x * m / 2^(31 + bits)
+// exceeds x / d by less than x / 2^31 / d: the whole part is the same.
 struct Divisor {
   uint32_t multiplier, bits;
   int32_t d;

@@ -1996,9 +1996,11 @@ constexpr int kHeldEntries = 4;   // registers of a wave for the block table
 // pieces of equal length to a step, about the shortest that leave no more pieces than `most`
 // per KV head; the waves of a workgroup walk a piece in equal shares and put it together in LDS.
 // Pieces in multiples of 8 steps, found by bisection, with divisions in front of the first load
-// and the block table behind the lengths were 9.06 us for one sequence of 768 positions and 8 KV
-// heads, 12.3 for 8 of 100 .. 1500, 9.4 for 8 of 100 .. 900 and 21.0 for 16 of 100 .. 2000; now 7.67,
-// 11.0, 8.2 and 19.8.
+// and the block table behind the lengths were 9.1 us for one sequence of 768 positions and 8 KV
+// heads, 14.3 for 8 of 100 .. 1500, 10.0 for 8 of 100 .. 900 and 22.7 for 16 of 100 .. 2000; now 8.2,
+// 12.9, 8.7 and 21.1.  Of 9000 drawn decode launches (those of the other kernels among them) 0.3 % are
+// more than 3 % slower, 18 in all, the worst 128 / 8 heads, one of 8145 positions beside one of 1, 20.3 ->
+// 24.9.
 // grid.x = main_wgs >= most * KV heads workgroups (and those that store new rows), block = 512.
 template <bool F16, bool NEW>
 __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, int batch,
@@ -2762,23 +2764,20 @@ constexpr int kWholeRowTolerance = 64;
 // Whether a launch of at most one row per CU goes by pieces (paged_decode_pieces_kernel), from
 // what the table can hold; else the balanced kernel looks at the lengths.  Pieces save what
 // the balanced kernel's larger head and its merges by single waves cost a small launch, 3 us:
-// by pieces / balanced, 1 .. 4 sequences of 1000 positions and 8 KV heads 8.3 .. 9.2 / 11.9 ..
-// 12.8 us, 8 of 100 .. 900 8.6 / 13.0, 8 of 128 .. 2048 11.1 / 14.4, 4 of 4096 15.4 / 19.6.
+// by pieces / balanced, 1 .. 4 sequences of 1000 positions and 8 KV heads 8.4 .. 9.2 / 13.0 ..
+// 14.0 us, 8 of 100 .. 900 8.7 / 13.6, 8 of 128 .. 2048 12.9 / 15.5, 4 of 4096 17.1 / 21.0.
 // Against that a row is cut into whole pieces of one length for all rows, which leaves
 // workgroups idle when lengths differ and rows are many, and one KV head per workgroup
-// streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 69.0 / 72.8, 64 rows of
-// 1000 .. 16000 52.2 / 54.2 and of 16000 .. 32768 137.3 / 137.2, 128 rows of 300 .. 4096 28.7 /
-// 29.9 and of 500 .. 8000 45.4 / 45.5; equal rows that leave a quarter of the workgroups idle are
-// the worst within the line there: 96 of 4096 37.5 / 39.5, 88 of 5952 50.0 / 50.1.
+// streams slower.  At the line, us: 32 rows of 500 .. 32000 positions 56.0 / 62.0, 64 rows of
+// 1000 .. 16000 55.6 / 58.9, 128 rows of 300 .. 4096 33.0 / 34.4; equal rows that leave a quarter of the
+// workgroups idle are the worst within it: 96 of 4096 39.4 / 40.6, 88 of 5952 52.0 / 50.7; beyond, 64
+// rows of 16000 .. 32768 137.7 / 134.2, 128 of 500 .. 8000 60.2 / 57.0.
 // Beyond 128 rows the mean row has less than two pieces, and where long rows find none to spare
-// one workgroup walks all of a row.  1309 mixes of 130 .. 256 rows and 832 .. 1927 positions
-// (equal, evenly spread, one, a third, half or most of them long), by pieces / balanced: up to 192
-// rows 0.80 .. 0.91 in the mean and up to 1.11, to 224 rows 0.87 .. 0.91 and 1.25, to 256 rows
-// 0.95 .. 0.98 and 1.26 (with pieces of 8 steps; 168 rows of 1131 equal were 22.8 / 25.2 then and
-// are 21.0 / 23.5, 224 of them 27.0 / 27.0).  136 of 1927 or 20, a few long, 9.2 /
-// 13.2, 144 of 1536 or 20, most long, 25.6 / 23.4, 224 of 832 or 20, a third long, 15.1 / 14.0; but
-// 136 of 2880 equal 46.2 / 40.2, 224 of 1536 or 20, a third long, 24.1 / 18.8, 8 of 256 of 1536 and
-// the others of 20 20.5 / 14.6.
+// one workgroup walks all of a row.  39648 launches drawn from 132 .. 256 rows and 832 .. 1927 positions
+// (equal, evenly spread, one, a third, half or most of them long), by pieces / balanced: within the
+// line up to 192 rows 0.86 in the mean, 7 % of them above 1.03, to 224 rows 0.88 and 16 %, at worst 1.23
+// (176 of 1344 or 20, half of them long, 24.0 / 19.6); beyond it 0.95 .. 0.97, 28 %, and 1.84 (8 of 248
+// rows of 1920 and the others of 1, 26.7 / 14.5).
 bool pieces_pay(int64_t rows, int64_t positions, int64_t cus) {
   if (rows > cus - cus / 8) return false;
   return rows * positions <= (rows <= 64 ? 1 << 20 : rows <= 128 ? 1 << 19 : 1 << 18);
@@ -2798,10 +2797,11 @@ bool pieces_take(int64_t batch, int head_dim, int64_t rows, int64_t positions, i
 // (At 1024 equal lengths the balanced kernel is still 2 .. 5 us behind; lengths that differ
 // have not been measured there.)
 // Where pieces are the other choice, up to 128 rows, the third round is theirs: without a
-// split / by pieces, at 288 positions 1 .. 64 rows 7.2 .. 8.0 / 7.0 .. 9.9, at 512 1 .. 32 rows 8.0
-// .. 8.7 / 7.2 .. 10.3 (the more, the more query heads share a KV head), 64 rows 8.5 .. 9.7 / 8.1 ..
-// 9.0, 128 rows 9.9 / 10.4; at 768 1 .. 16 rows 9.4 .. 9.9 / 7.7 .. 9.0, 64 rows 11.3 .. 12.1 /
-// 9.1, 128 rows 13.3 / 13.0, and, with pieces of 8 steps, 192 rows 15.4 / 16.2, 256 rows 18.4 / 19.0.
+// split / by pieces, at 288 positions 1 .. 64 rows 7.1 .. 8.3 / 6.8 .. 8.8, at 512 1 .. 32 rows 7.7
+// .. 9.0 / 7.0 .. 9.5 (the more, the more query heads share a KV head), 64 rows 8.3 .. 8.5 / 8.7 ..
+// 9.4, 128 rows 9.4 .. 10.7 / 10.3 .. 11.1; at 768 1 .. 16 rows 9.0 .. 10.1 / 7.1 .. 9.6, 64 rows 9.8 ..
+// 10.5 / 9.2 .. 10.0, 128 rows 13.7 .. 14.0 / 13.3 .. 14.2, 192 rows 15.4 .. 15.7 / 16.0 .. 16.3, 256
+// rows 18.1 .. 18.4 / 18.8 .. 19.3.
 bool table_of_short_rows(int64_t rows, int64_t positions, bool pieces) {
   return positions <= (pieces && rows <= 128 ? 2 : 3) * 8 * kStep;
 }

@@ -75,7 +75,7 @@ constexpr int kTileBytes = kKeys * kD * 2;   // one K or V tile in LDS: 32 rows 
 // 3, fetched one tile ahead, with one column group per wave: three workgroups to a CU, for prompts
 // whose workgroups have little but their head and tail (tile_form).
 constexpr float kNegBig = -1.0e30f;
-constexpr int kShortestPart = 8;     // tiles, a multiple of the ring's 4
+constexpr int kShortestPart = 8;     // tiles, a multiple of the ring's 4 (the last part may be shorter)
 constexpr float kLazyLog2 = 8.0f;    // running max moves only for gains above 2^8
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -693,8 +693,8 @@ struct VisibleKeys {
   }
 };
 
-// The tiles [first, end) of part `part` of a query tile's keys: whole rounds of the ring, and no part
-// so short that its head and tail are most of it.
+// The tiles [first, end) of part `part` of a query tile's keys: whole rounds of the ring, and none so
+// short that its head and tail are most of it but for the last, which takes what is left over.
 struct KeyPart {
   int first, end, count;   // count: parts that have keys
   __device__ __forceinline__ KeyPart(const PrefillArgs& a, int nsteps, int part) {
@@ -804,9 +804,10 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
   // the matrix core, then accumulates tile i-1 (probabilities kept from the
   // previous iteration) while the vector ALU turns the scores of tile i into
   // probabilities.  Iteration i therefore reads K of tile i and V of tile i-1,
-  // and starts the copies of tile i+2 into the ring slots last read in iteration
-  // i-1 (K of tile i-1, V of tile i-2).  Before the barrier that ends it, every
-  // lane waits for its copies of tile i+1.
+  // and starts the copies of a tile to come: with a ring of 4 those of tile i+2 at its end, into
+  // the ring slots last read in iteration i-1 (V of tile i-2); with a ring of 3 those of
+  // tile i+1 at its start, into the slot of tile i-2, which nothing reads any more.  Before the barrier
+  // that ends it, every lane waits for its copies of tile i+1.
   if (nsteps > first_tile) {
     // V "of tile -1" (probabilities are zero there, but 0 * NaN is not 0)
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -828,10 +829,9 @@ __global__ __launch_bounds__(kWaves * 64, RING == 3 ? 3 : 2) void prefill_attent
       block0[0] >= len_q ? 0 : min(nsteps, (off + block0[NG - 1] + 15) / kKeys + 1);
   const int n_plain = min(min(off + block0[0] + 1, k_end) / kKeys, n_active);
 
-  // Tile t lives in ring slot t % 4 (K and V alike).  Iteration i: scores of tile
-  // i, accumulation of tile i-1, probabilities of tile i, copies of tile i+2 into
-  // the slot last read in iteration i-1, wait for this lane's copies of tile i+1,
-  // barrier.
+  // Tile t lives in ring slot t % RING (K and V alike).  Iteration i: (a ring of 3: copies of
+  // tile i+1,) scores of tile i, accumulation of tile i-1, probabilities of tile i, (a ring of 4: copies
+  // of tile i+2,) wait for this lane's copies of tile i+1, barrier.
   lds_ptr kaddr[4], vaddr[8];
   k_read_addresses(k_lds, r, kg, kaddr);
   v_read_addresses(v_lds, r, kg, vaddr);
@@ -1085,11 +1085,12 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
   if ((xcds_even || tokens <= 16 * batch) && wide * num_kv_heads * 2 <= cus * 3)
     return {1, 4, narrow};
   // Prompts of few column groups: the larger workgroups are mostly empty or mostly head and tail.
-  // Three small ones to a CU instead, us: 100 prompts of 4 tokens, 16 / 8 heads (2 groups) 11.1 ->
-  // 8.1, 200 of 16, 32 / 8 (4) 26.0 -> 22.3, 100 of 60, 32 / 32 (4) 67.4 -> 55.4, 60 of 20..60, 32 / 8
-  // (12) 17.1 -> 14.8, 40 of 100, 16 / 8 (14) 19.8 -> 17.6; 60 of 20..60, 16 / 8 (6) 10.7 -> 11.2, the
-  // only one slower.  Beyond that -13 .. +13 %, with 8 heads to a KV head (8 groups and more) -3 ..
-  // +18 %.
+  // Three small ones to a CU instead, us with the store: 100 prompts of 4 tokens, 16 / 8 heads (2 groups)
+  // 12.5 -> 8.2, 200 of 16, 32 / 8 (4) 31.0 -> 23.0, 100 of 60, 32 / 32 (4) 71 -> 57, 60 of 20..60, 32 / 8
+  // (12) 17.9 -> 15.2, 16 / 8 (6) 12.1 -> 9.9, 40 of 100, 16 / 8 (14) 21.4 -> 18.0.  Larger against small
+  // ones over drawn launches: up to 4 groups 1.37 in the mean (421 launches, at worst 0.965), 5 to 14
+  // with up to 4 heads to a KV head 1.09 (200, 0.915, 4 % of them below 0.97); beyond the line, with 7 or 8
+  // heads, 1.05 (150, 27 % of them below 0.97), 15 to 30 groups 1.05 (188, 18 %).
   if (groups <= 4 || (groups <= 14 && group <= 4)) return {1, 3, narrow};
   return {2, 4, wide};
 }
