@@ -562,10 +562,11 @@ NVJ_API int nvj_paged_prefill_attention_launch(void* stream, const void* q, cons
  * most of the GPU idle: the keys of a tile are cut into parts, which a second launch puts
  * together, in the order of the keys.  The sums are in another order then than
  * nvj_paged_prefill_attention_launch's, whose results are the same however a batch is put together.
- * `max_keys`: the most keys that a sequence has, if known, else 0: what the tables hold; nothing but
- * the number of parts follows from it, and it has to be the same in both calls.
- * `workspace`: nvj_paged_prefill_split_workspace_bytes, 16-byte aligned; where that is 0 this is
- * nvj_paged_prefill_attention_launch.
+ * `max_keys`: the most keys that a sequence has, if known, else 0: what the tables hold.  The number of
+ * parts, the form of the workgroups and with them the layout and the size of the workspace follow
+ * from it, so it has to be the same in both calls; a value below the true lengths costs speed only.
+ * `workspace`: nvj_paged_prefill_split_workspace_bytes (at most 65 MiB), 16-byte aligned; where that is 0
+ * this is nvj_paged_prefill_attention_launch.
  */
 NVJ_API size_t nvj_paged_prefill_split_workspace_bytes(int32_t total_q_tokens, int32_t batch,
                             int32_t num_heads, int32_t num_kv_heads, int32_t block_size,

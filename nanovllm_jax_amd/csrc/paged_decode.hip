@@ -1999,8 +1999,8 @@ constexpr int kHeldEntries = 4;   // registers of a wave for the block table
 // and the block table behind the lengths were 9.1 us for one sequence of 768 positions and 8 KV
 // heads, 14.3 for 8 of 100 .. 1500, 10.0 for 8 of 100 .. 900 and 22.7 for 16 of 100 .. 2000; now 8.2,
 // 12.9, 8.7 and 21.1.  Of 9000 drawn decode launches (those of the other kernels among them) 0.3 % are
-// more than 3 % slower, 18 in all, the worst 128 / 8 heads, one of 8145 positions beside one of 1, 20.3 ->
-// 24.9.
+// more than 3 % slower, one of them 18 % (128 / 8 heads, a row of 8145 positions beside one of 1, 20.3 ->
+// 24.9).
 // grid.x = main_wgs >= most * KV heads workgroups (and those that store new rows), block = 512.
 template <bool F16, bool NEW>
 __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, int batch,

@@ -6,11 +6,18 @@ names, argument order and return shapes, for the decode phase and for the
 prefill phase (:331-364).  Everything runs on the HIP library only; there is no
 alternate dispatch.
 
-Differences a caller can observe, both deliberate:
+Differences a caller can observe, all deliberate:
 * the cache is updated in place and the very same tensors are returned (the
   reference returns new arrays that alias the donated inputs);
 * a negative slot stores nothing (the reference's docstring, :57-58; its code
-  writes row 0 instead).
+  writes row 0 instead);
+* a prefill call of few rows behind long cached prefixes cuts the keys into parts
+  (``nvj_paged_prefill_split_launch``), for which it takes up to 65 MiB of torch's
+  memory while it runs, if there are.  The order of the sums, and so the last bits of a
+  row, then depend on the batch that the row is in, on ``context.max_seqlen_k`` and on the
+  width of the tables.  Nothing is cut where ``max_seqlen_k`` is 0 or up to 512, nor on
+  the general path (3-D caches, tensors that have to be converted first).
+  ``store_kv_to_cache`` and ``paged_prefill_attention`` give the same bits in any batch.
 """
 from __future__ import annotations
 

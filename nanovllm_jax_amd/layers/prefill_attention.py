@@ -104,7 +104,8 @@ def paged_prefill_attention(q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_
     query rows of a sequence are its last ``len_q`` positions.  This is the call
     the reference's prefill context describes when ``cu_seqlens_k >
     cu_seqlens_q`` (``engine/model_runner.py:286-312``); run it after the new
-    rows have been stored.
+    rows have been stored.  Every row's keys are walked in one piece: its bits are the
+    same however a batch is put together (``Attention`` may cut long ones into parts).
 
     q [total_tokens, num_heads, head_dim] bf16 or float16; k_cache, v_cache
     [num_blocks, block_size, num_kv_heads, head_dim] of the same dtype;

@@ -17,8 +17,8 @@ def _bucket_to_power_of_2(value: int, min_bucket: int = 16, max_bucket: int = 81
     """``value`` rounded up to a power of two and clamped into [min_bucket,
     max_bucket]: what the reference's helper of this name returns
     (``utils/context.py:18-32``; it buckets the static max lengths to limit
-    recompilation).  The HIP kernels never read these fields; the contexts carry
-    them so that code written against the reference sees the same values."""
+    recompilation).  The contexts carry the same values; ``max_seqlen_k`` is a hint to the
+    layer besides, which need not be exact."""
     return max(min_bucket, min(max_bucket, 1 << max(int(value) - 1, 0).bit_length()))
 
 
@@ -33,6 +33,10 @@ class AttentionContext:
                         -1 means "do not store".
     block_tables        [batch, max_blocks] int32, logical -> physical page,
                         padded with -1.
+    max_seqlen_k        the longest sequence, cached and new tokens together, rounded up: with
+                        ``block_tables`` a hint from which the layer decides whether the keys
+                        are cut into parts.  0 or no whole number: not known, nothing is cut; a
+                        value below the true lengths costs speed only.
     decode_split        how the decode kernel divides the positions of the batch
                         (``chunk`` of ``paged_attention``): 0 = balanced on the
                         device from ``context_lens``; the filler, which knows
