@@ -2036,9 +2036,12 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
       if (i == 0 || entries > 64 * i)
         held[i] = a.block_tables[min(64 * i + lane, (int)entries - 1)];
   }
+  // workgroup g: KV head g % heads of piece g / heads of them all
+  const int at = __builtin_amdgcn_readfirstlane(divide_small(g, a.num_kv_heads));
+  const int kvh = g - at * a.num_kv_heads;
   const int ctx_here = lane < batch ? min(max(len_here, 0), cap) : 0;
   const int steps_here = (ctx_here + kStep - 1) / kStep;
-  const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(steps_here), 63);
+  int total = __builtin_amdgcn_readlane(wave_inclusive_scan(steps_here), 63);
   if (g < batch && __builtin_amdgcn_readlane(ctx_here, g & 63) <= 0) {
     // an empty sequence has no piece: its zeros (0 / (0 + 1e-9)) are written here
     uint4* orow = a.out + (int64_t)g * a.num_heads * H::kPieces;
@@ -2053,39 +2056,40 @@ __global__ __launch_bounds__(512) void paged_decode_pieces_kernel(DecodeArgs a, 
   const int rows = __popcll(__ballot(steps_here > 0));
   const int per_row = a.group > 8 ? 4 : a.group > 4 ? 8 : 12;   // what is put together at once
   const int enough = max(rows, 1) * per_row;
-  int shortest = min(max(divide_small_up(total, enough), kShortestPiece), NW);
-  if (__any(steps_here > per_row * shortest))   // (equal rows pay no maximum: 0.07 us)
-    shortest = min(divide_small_up(wave_max(steps_here), per_row), NW);
-  const int length2 = max(shortest, divide_small_up(total, max(most - rows, 1)));
-  int length1 = max(shortest, divide_small_up(total, most - rows / 2));
-  int length0 = max(shortest, divide_small_up(total, most));
+  // (What follows stays in vector registers: the compiler takes a value that is the same in all lanes
+  // to scalar ones and back, and a launch of 7.59 us was 7.87.)
+  asm("" : "+v"(total));
+  int length0 = max(min(max(divide_small_up(total, enough), kShortestPiece), NW),
+                    divide_small_up(total, most));
+  if (__any(steps_here > (int)__umul24(per_row, length0)))   // (equal rows pay no maximum: 0.07 us)
+    length0 = max(length0, min(divide_small_up(wave_max(steps_here), per_row), NW));
+  int length1 = max(length0, divide_small_up(total, most - rows / 2));
+  const int length2 = max(length0, divide_small_up(total, max(most - rows, 1)));
   if (length0 > NW && most > enough) length0 = (length0 + NW - 1) / NW * NW;
   // A row of up to a step a wave is one piece whatever the length, as one step would be: it is no
   // longer in one workgroup, and there is nothing to put together across workgroups (one sequence of 83
   // positions, 8 / 1 heads, in tables of 1024, 6.9 us in pieces of 2 steps, 4.9 whole; 44 of 129
   // 7.9 / 6.1).
   const int to_cut = steps_here <= NW ? min(steps_here, 1) : steps_here;
+  const uint32_t n2 = divide_small_up(to_cut, length2);
+  uint32_t numbers, counts;   // three of 10 bits each
+  auto shortest_that_fits = [&]() __attribute__((always_inline)) {   // where its number is
+    const uint32_t n0 = divide_small_up(to_cut, length0), n1 = divide_small_up(to_cut, length1);
+    numbers = n0 | n1 << 10 | n2 << 20;
+    counts = wave_inclusive_scan(numbers);
+    const int all = __builtin_amdgcn_readlane(counts, 63);
+    return (all & 1023) <= most ? 0 : (all >> 10 & 1023) <= most ? 10 : 20;
+  };
+  int pick = shortest_that_fits();
   // Lengths that differ much can leave only the one that always fits.  Two multiples of 8 in front of
   // it are tried then: with up to 8 steps more than one of them a wave has one more to walk (10 rows of
-  // 1609 positions and 21 of 1, 4 / 4 heads, in pieces of 17 steps 15.0 us, of 16 12.1; 0.05 us for
-  // launches that have no use for it).
-  const int n2 = divide_small_up(to_cut, length2);
-  int n0, n1, counts, pick;
-  for (bool again = length2 > NW;; again = false) {
-    n0 = divide_small_up(to_cut, length0);
-    n1 = divide_small_up(to_cut, length1);
-    counts = wave_inclusive_scan(n0 | n1 << 10 | n2 << 20);
-    const int all = __builtin_amdgcn_readlane(counts, 63);
-    pick = (all & 1023) <= most ? 0 : (all >> 10 & 1023) <= most ? 10 : 20;
-    if (pick < 20 || !again) break;
+  // 1609 positions and 21 of 1, 4 / 4 heads, in pieces of 17 steps 15.0 us, of 16 12.1).
+  if (pick == 20 && __builtin_amdgcn_readfirstlane(length2) > NW) {
     length0 = (length1 + NW) / NW * NW;
     length1 = ((length0 + length2) / 2 + NW - 1) / NW * NW;
+    pick = shortest_that_fits();
   }
-  const int number = pick == 0 ? n0 : pick == 10 ? n1 : n2;
-  const int incl = counts >> pick & 1023;
-  // workgroup g: KV head g % heads of piece g / heads of them all
-  const int at = __builtin_amdgcn_readfirstlane(divide_small(g, a.num_kv_heads));
-  const int kvh = g - at * a.num_kv_heads;
+  const int number = numbers >> pick & 1023, incl = counts >> pick & 1023;
   const unsigned long long hit = __ballot(at < incl);
   if (hit == 0ull) return;
   const int b = __builtin_ctzll(hit);
