@@ -1143,19 +1143,34 @@ struct SplitForm {
   TileForm form;
   int64_t splits;
 };
-// The most workgroups whose keys are cut.
+// The most workgroups whose keys are cut.  `streams`: sequences times KV heads, the keys that are not
+// shared.  Where most workgroups have keys of their own HBM is the bound earlier than where several walk
+// the same ones, so the lines lie higher for few streams.  In parts / whole, means of 51000 launches drawn
+// from this side of the lines and beyond, by workgroups (and streams): up to 1024 positions 65 .. 72 0.96, 81
+// .. 96 1.00 (0.88 and 0.90 where tables are as long as what is in them, 1.05 and 1.09 where they are
+// longer); 2048, KV heads a multiple of 8, 129 .. 192 (up to 128) 0.94, (more) 1.07, 193 .. 224 (up to
+// 128) 0.98; others 97 .. 128 0.88, 129 .. 160 (up to 32) 0.94, (more) 1.02, 161 .. 192 (up to 32) 0.97;
+// 4096, a multiple of 8, 193 .. 256 (up to 160) 0.86, (more) 1.11; others 161 .. 192 (up to 64) 0.86, (more)
+// 0.97 and now and then far longer (94 of 3..6 behind 2600, 6 / 2, 188 of them, 50.2 us whole, 66.7), 193 ..
+// 224 (up to 32) 0.86, (more) 1.03, 225 .. 256 (up to 32) 0.99.
 int64_t most_to_cut(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
                     int64_t positions) {
   const bool xcds_even = num_kv_heads % 8 == 0;
+  const int64_t streams = batch * num_kv_heads;
   if (positions <= kNeverCut) return 0;
   if (positions <= 768) return cus / 8;
-  if (positions <= 1024) return cus / 4;
-  if (positions <= 2048) return cus * (xcds_even ? 4 : 3) / 8;
-  const int64_t most = positions <= 4096 ? cus * (xcds_even ? 6 : 5) / 8
-                       : xcds_even       ? cus * 15 / 16
-                                         : cus * 6 / 8;
-  if (group == 1) return std::min(most, cus * 6 / 8);
-  return xcds_even && tokens > 16 * batch ? cus : most;
+  if (positions <= 1024) return cus * 9 / 32;
+  if (positions <= 2048) {
+    if (group == 1 || (xcds_even ? streams * 2 : streams * 8) > cus) return cus / 2;
+    return cus * (xcds_even ? 6 : 5) / 8;
+  }
+  if (positions <= 4096) {
+    if (group == 1) return cus * (xcds_even ? 6 : 5) / 8;
+    if (xcds_even) return streams * 8 <= cus * 5 ? cus : cus * 6 / 8;
+    return cus * (streams * 8 <= cus ? 7 : streams * 4 <= cus ? 6 : 5) / 8;
+  }
+  if (group == 1 || !xcds_even) return cus * 6 / 8;
+  return tokens > 16 * batch ? cus : cus * 15 / 16;
 }
 int64_t key_splits(const TileForm& form, int64_t tokens, int64_t batch, int64_t group,
                    int64_t num_kv_heads, int64_t cus, int64_t positions) {
@@ -1178,18 +1193,19 @@ int64_t key_splits(const TileForm& form, int64_t tokens, int64_t batch, int64_t 
 // so: 500 behind 5000, 32 / 8 heads, 69 / 60, 700 behind 5000 90 / 81, 512 behind 8000, 64 / 8, 157 /
 // 133, 400 behind 4000, 32 / 32, 68 / 51, 6 of 23..44 behind 8555..10940, 64 / 8, 148 / 99.  Up to
 // 4096 positions the partials cost more (1000 behind 2000 55 / 62), with fewer rows many small parts
-// are as good (270 behind 4200 37.6 / 36.4, 150 behind 4000, 32 / 32, 29 / 33), with as many large
-// workgroups as CUs two parts each are not (168 of 5..18 behind 3500, 8 / 1, 250 of them, 119 / 160, 4 of
-// 244..494 behind 3357..5499, 368 of them, 125 / 151), and nor are they where they are hardly fewer than
-// the small ones, half empty (55 of 2 behind 2500, 16 / 8, 126 / 153, 7 of 12 behind 7350, 32 / 32, 138 /
-// 174).
+// are as good (270 behind 4200 37.6 / 36.4, 150 behind 4000, 32 / 32, 29 / 33), with more large workgroups
+// than CUs two parts each are not (4 of 244..494 behind 3357..5499, 368 of them, 125 / 151), and where the
+// XCDs are not filled evenly earlier (193 .. 208 of them 0.94, 209 .. 224 0.96, 225 .. 256 1.02, where they are
+// 241 .. 256 0.87; 168 of 5..18 behind 3500, 8 / 1, 250 of them, 119 / 160), and nor are they where they are
+// hardly fewer than the small ones, half empty (55 of 2 behind 2500, 16 / 8, 126 / 153, 7 of 12 behind
+// 7350, 32 / 32, 138 / 174).
 SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads,
                      int64_t cus, int64_t positions) {
   const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
   const int64_t large =
       std::max<int64_t>(expected_tiles(tokens, batch, group, 2 * kWaves) * num_kv_heads, 1);
   if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 &&
-      large * 16 <= cus * (num_kv_heads % 8 == 0 ? 15 : 12) && large * 4 <= small * 3)
+      large * 16 <= cus * (num_kv_heads % 8 == 0 ? 16 : 13) && large * 4 <= small * 3)
     return {{2, 4, most_tiles(tokens, batch, group, 2 * kWaves)}, 2 * cus / large};
   const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true, positions);
   return {form, key_splits(form, tokens, batch, group, num_kv_heads, cus, positions)};

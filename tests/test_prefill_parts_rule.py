@@ -35,6 +35,24 @@ def test_keys_are_cut_where_parts_are_faster(tokens, batch, heads, kv_heads, pos
     assert _bytes(tokens, batch, heads, kv_heads, 4 * positions, 512) == 0
 
 
+@pytest.mark.parametrize("tokens,batch,heads,kv_heads,positions,cut", [
+    # workgroups at and past the line: up to 1024 positions 72
+    (72, 5, 32, 8, 1024, True), (80, 6, 32, 8, 1024, False), (9, 9, 16, 8, 1024, True),
+    # up to 2048 half the CUs (128), more where few sequences and KV heads share them
+    (370, 1, 32, 8, 2048, True), (400, 1, 32, 8, 2048, False), (64, 17, 32, 8, 2048, False),
+    (330, 1, 28, 4, 2048, True), (360, 1, 28, 4, 2048, False), (160, 16, 28, 4, 2048, False),
+    # up to 4096
+    (16, 16, 64, 8, 4096, True), (17, 17, 64, 8, 4096, False), (30, 30, 32, 8, 4096, False),
+    (850, 2, 16, 1, 4096, True), (960, 3, 16, 1, 4096, False), (411, 94, 6, 2, 2688, False),
+    (48, 48, 16, 1, 4096, True), (66, 66, 16, 1, 4096, False), (40, 40, 16, 1, 4096, True),
+    # larger workgroups in parts, up to one a CU, 13 / 16 of that where the XCDs are not filled evenly
+    (990, 1, 32, 8, 8192, True), (1050, 1, 32, 8, 8192, False), (390, 2, 64, 4, 8192, True),
+    (410, 2, 64, 4, 8192, False),
+])
+def test_lines_of_the_cut(tokens, batch, heads, kv_heads, positions, cut):
+    assert (_bytes(tokens, batch, heads, kv_heads, positions) > 0) == cut
+
+
 def test_partials_have_a_bound():
     """No launch asks for more than 65 MiB of partials, half-empty batches included."""
     most = 0
