@@ -1051,9 +1051,8 @@ int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t col
   return std::max(half_full,
                   std::min(tokens, batch) * ((group + column_groups - 1) / column_groups));
 }
-// positions (paged): the most that a sequence has.
 TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
-                   bool paged, int64_t positions) {
+                   bool paged) {
   const int64_t wide = most_tiles(tokens, batch, group, 2 * kWaves);
   const int64_t narrow = most_tiles(tokens, batch, group, kWaves);
   const int64_t groups = (tokens + 16 * batch - 1) / (16 * batch) * group;   // of a mean prompt
@@ -1064,19 +1063,20 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
   // of 1500, 32 heads, 35 -> 29 (two a CU: 79 .. 111 %).
   if (wide * num_kv_heads <= cus) return {1, 4, narrow};
   if (paged) {
-    // Behind cached prefixes, where the tiles of a sequence are equally long, up to 1.5 of the small
-    // ones a CU, and up to two where the keys are few: every small one fetches all of them for half the
-    // rows; 1.25 where the XCDs are not filled evenly.  us, larger / small: 4 of 55..268, at most 277
-    // keys, 32 / 8 heads, 12.0 / 10.3, 2 of 167..263, 557 keys, 64 / 8, 17.7 / 15.4; beyond the line 14
-    // of 3..243, up to 4424 keys, 28 / 4, 94 / 118, 170 of 1..30, 866 keys, 8 / 1, 28.7 / 36.2 (and
-    // within it 32 of 6..40, 3765 keys, 16 / 8, 84 / 102).
+    // Behind cached prefixes, where the tiles of a sequence are equally long, up to two of the small
+    // ones a CU: 4 of 55..268, at most 277 keys, 32 / 8 heads, 10.3 us in small ones, 12.0 in larger, 2
+    // of 167..263, 557 keys, 64 / 8, 15.4 / 17.7; with 385 .. 512 of them behind more than 2048
+    // positions 0.86 times as long in the mean (1100 drawn launches).  Unless the XCDs take whole KV
+    // heads one of them gets nothing but real tiles, so there the bound counts: small ones in the
+    // place of larger, by eighths of the bound, 449 .. 512 0.82 (2050 drawn launches, 1.5 % of them longer),
+    // 513 .. 576 1.14 (14 of 3..243, up to 4424 keys, 28 / 4, 118 us / 94).
     const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
-    if (!xcds_even) return {small * 4 <= cus * 5 ? 1 : 2, 4, small * 4 <= cus * 5 ? narrow : wide};
-    if (small * 2 <= cus * 3 || (small <= 2 * cus && positions <= 2048)) return {1, 4, narrow};
-    // Prompts of up to 4 groups and 8 tokens, few of which have a second block: the larger
-    // workgroups are mostly empty (with more tokens 155 of 1..63, 16 in the mean, at most 1722 keys, 32
-    // / 8 heads, 140 us in larger ones, 149 in small ones).
-    if (groups <= 4 && tokens <= 8 * batch) return {1, 4, narrow};
+    if ((xcds_even ? small : narrow * num_kv_heads) <= 2 * cus) return {1, 4, narrow};
+    // More of them, but of sequences of a column group or two, or of up to 4 groups and 12 tokens, few of
+    // which have a second block: the larger workgroups are mostly empty (1 or 2 query heads a KV head 0.88,
+    // 4 and 6 .. 12 tokens 0.89; 12 .. 16 tokens 0.95 where some have more than 16, at worst 1.28).
+    if (small > 2 * cus && (groups <= 2 || (xcds_even && groups <= 4 && tokens <= 12 * batch)))
+      return {1, 4, narrow};
     return {2, 4, wide};
   }
   // Prompts that are longer than a block and whose KV heads do not fill the XCDs evenly keep the
@@ -1103,7 +1103,7 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
 bool store_rides(int64_t tokens, int64_t rows, int64_t batch, int64_t num_heads,
                  int64_t num_kv_heads, int64_t cus) {
   const int64_t tiles =
-      tile_form(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus, false, 0).tiles *
+      tile_form(tokens, batch, num_heads / num_kv_heads, num_kv_heads, cus, false).tiles *
       num_kv_heads;
   return tiles <= 6 * cus || rows * num_kv_heads * kPieces >= 80 * tiles;
 }
@@ -1207,7 +1207,7 @@ SplitForm split_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_k
   if (batch <= 256 && positions > 4096 && small * 4 > cus * 3 &&
       large * 16 <= cus * (num_kv_heads % 8 == 0 ? 16 : 13) && large * 4 <= small * 3)
     return {{2, 4, most_tiles(tokens, batch, group, 2 * kWaves)}, 2 * cus / large};
-  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true, positions);
+  const TileForm form = tile_form(tokens, batch, group, num_kv_heads, cus, true);
   return {form, key_splits(form, tokens, batch, group, num_kv_heads, cus, positions)};
 }
 int64_t most_keys(int64_t max_blocks, int64_t block_size, int64_t max_keys) {
@@ -1348,7 +1348,7 @@ int launch_packed(void* stream, const void* q, int64_t q_row_stride, const void*
     a.new_pieces = (uint32_t)store->rows * (uint32_t)a.row_pieces.d;
   }
   return launch_prefill(static_cast<hipStream_t>(stream), a, false,
-                        tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, false, 0),
+                        tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, false),
                         total_q_tokens, dtype, cus);
 }
 }  // namespace
@@ -1451,8 +1451,7 @@ int launch_paged(void* stream, const void* q, const void* k_cache, const void* v
   const int64_t positions = most_keys(max_blocks, block_size, max_keys);
   const SplitForm cut =
       may_split ? split_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, positions)
-                : SplitForm{tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true,
-                                      positions),
+                : SplitForm{tile_form(total_q_tokens, batch, a.group.d, num_kv_heads, cus, true),
                             1};
   if (const size_t need = part_bytes(cut, num_kv_heads)) {
     if (!workspace || workspace_bytes < need) return NVJ_ERR_WORKSPACE;
