@@ -1042,13 +1042,15 @@ int64_t most_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_
   const int64_t blocks = (tokens + 15 * batch) / 16;
   return (blocks * group + (column_groups - 1) * batch) / column_groups;
 }
-// The same if the last block and the last tile of every sequence are half full, but no less than
-// sequences of a token or a few have.
+// The same if the last block and the last tile of every sequence are half full.
+int64_t half_full_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_groups) {
+  return ((2 * tokens + 15 * batch) * group + 16 * (column_groups - 1) * batch +
+          16 * column_groups) /
+         (32 * column_groups);
+}
+// And no less than sequences of a token or a few have.
 int64_t expected_tiles(int64_t tokens, int64_t batch, int64_t group, int64_t column_groups) {
-  const int64_t half_full = ((2 * tokens + 15 * batch) * group + 16 * (column_groups - 1) * batch +
-                             16 * column_groups) /
-                            (32 * column_groups);
-  return std::max(half_full,
+  return std::max(half_full_tiles(tokens, batch, group, column_groups),
                   std::min(tokens, batch) * ((group + column_groups - 1) / column_groups));
 }
 TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_heads, int64_t cus,
@@ -1072,10 +1074,19 @@ TileForm tile_form(int64_t tokens, int64_t batch, int64_t group, int64_t num_kv_
     // 513 .. 576 1.14 (14 of 3..243, up to 4424 keys, 28 / 4, 118 us / 94).
     const int64_t small = expected_tiles(tokens, batch, group, kWaves) * num_kv_heads;
     if ((xcds_even ? small : narrow * num_kv_heads) <= 2 * cus) return {1, 4, narrow};
-    // More of them, but of sequences of a column group or two, or of up to 4 groups and 12 tokens, few of
-    // which have a second block: the larger workgroups are mostly empty (1 or 2 query heads a KV head 0.88,
-    // 4 and 6 .. 12 tokens 0.89; 12 .. 16 tokens 0.95 where some have more than 16, at worst 1.28).
-    if (small > 2 * cus && (groups <= 2 || (xcds_even && groups <= 4 && tokens <= 12 * batch)))
+    // Nor do the larger ones fit a round there once their bound is more than two a CU, so half-full
+    // tiles count again: 0.89 (1400 drawn launches; 72 of 1..4 behind 1744, 28 / 4, 60.1 us / 82.0).
+    const bool second_round = wide * num_kv_heads > 2 * cus;
+    if (!xcds_even && second_round &&
+        half_full_tiles(tokens, batch, group, kWaves) * num_kv_heads <= 2 * cus)
+      return {1, 4, narrow};
+    // More of them, but of sequences of a column group or two, or of up to 4 groups and a block of 16
+    // tokens, few of which have a second: the larger workgroups are mostly empty (1 or 2 query heads a
+    // KV head 0.88, 4 and 6 .. 12 tokens 0.89, 12 .. 16 tokens up to 8 a CU 0.92, one in seven longer
+    // and at worst 1.46, where nearly all keys are long; more than 8 a CU 0.99, 31 % of them longer).
+    if (small > 2 * cus &&
+        (groups <= 2 || ((xcds_even || second_round) && groups <= 4 &&
+                         tokens <= (small <= 8 * cus ? 16 : 12) * batch)))
       return {1, 4, narrow};
     return {2, 4, wide};
   }

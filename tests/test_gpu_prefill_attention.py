@@ -378,6 +378,39 @@ def test_paged_prefill_longest_tiles_first(batch, Hq, Hkv):
         assert torch.equal(got[at[i]:at[i + 1]], one), f"sequence {i}"
 
 
+@pytest.mark.parametrize("batch,most,Hq,Hkv", [
+    (72, 4, 28, 4), (70, 4, 28, 4),     # KV heads that do not fill the XCDs, around two rounds
+    (169, 7, 6, 2), (61, 25, 32, 8),    # up to a block of tokens in the mean, some with two
+    (140, 27, 32, 8), (165, 27, 32, 8), # the same at eight workgroups a CU and beyond
+])
+def test_paged_prefill_of_many_short_sequences(batch, most, Hq, Hkv):
+    """Small or large workgroups: a sequence's bits are those it has alone."""
+    print(f"case paged prefill, many short batch={batch} Hq={Hq}", flush=True)
+    import torch
+    from nanovllm_jax_amd import paged_prefill_attention
+    rng = np.random.Generator(np.random.PCG64(batch))
+    new = rng.integers(1, most + 1, batch)
+    total = new + rng.integers(0, 200, batch)
+    pages = -(-total // 32)
+    ends = np.cumsum(pages)
+    table = np.full((batch, int(pages.max())), -1, np.int32)
+    for i, e in enumerate(ends):
+        table[i, :pages[i]] = np.arange(e - pages[i], e)[::-1]
+    dev = "cuda:0"
+    g = torch.Generator(device=dev).manual_seed(batch)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=dev).to(torch.bfloat16)
+    kc, vc = (draw(int(ends[-1]), 32, Hkv, 128) for _ in range(2))
+    q = draw(int(new.sum()), Hq, 128)
+    up = lambda x: torch.from_numpy(np.ascontiguousarray(x, np.int32)).to(dev)
+    cu = lambda n: up(np.concatenate([[0], np.cumsum(n)]))
+    got = paged_prefill_attention(q, kc, vc, up(table), cu(new), cu(total), 128 ** -0.5)
+    at = np.concatenate([[0], np.cumsum(new)])
+    for i in range(batch):
+        one = paged_prefill_attention(q[at[i]:at[i + 1]].contiguous(), kc, vc, up(table[i:i + 1]),
+                                      cu(new[i:i + 1]), cu(total[i:i + 1]), 128 ** -0.5)
+        assert torch.equal(got[at[i]:at[i + 1]], one), f"sequence {i}"
+
+
 @pytest.mark.parametrize("new,cached,Hq,Hkv,bs,splits", [
     ([1], [2000], 8, 8, 64, True),                    # one row, with parts for every ring of tiles
     ([30, 0, 17], [1500, 700, 31], 16, 8, 256, True),  # an empty sequence, tiles of one part
