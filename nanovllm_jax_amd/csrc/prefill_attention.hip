@@ -1143,9 +1143,9 @@ constexpr int64_t kNeverCut = 2 * kKeys * kShortestPart;   // positions
 // 4400, 32 / 32, 256 of them, 96.7 / 120, 53 of 1..3 behind 6500, 4 / 4, 212 of them, 124 / 154.  Sequences of
 // more than a block of tokens, whose tiles share their keys, gain up to a round (1 of 213 behind 1900, 64
 // / 8, 224 of them, 33.9 / 31.7, 6 of 27 behind 3050 48 / 41); where every query head has keys of its own
-// HBM is the bound earlier.  6361 launches drawn from 1..260 sequences of 1..700 tokens behind up to
-// 12000 positions, where the bound is known, against a workgroup for every tile: 1.27 times as fast in
-// the mean, 0.4 % of them more than 5 % slower, at worst 0.78.
+// HBM is the bound earlier.  4206 launches drawn from 1..260 sequences of 1..700 tokens behind up to
+// 12000 positions, where the bound is known, against a workgroup for every tile: 1.21 times as fast in
+// the mean, 0.3 % of them more than 5 % slower, at worst 0.85.
 // More than a round of parts is slower (4 of 100..300 behind
 // 1000..4000, 34.7 / 40.2 at twice as many), three quarters of one better where there are many to put
 // together (30 behind 5000 18.5 / 16.9, 20 behind 4000, 32 / 32, 28 / 22.5).  Parts of 4 tiles or of 12
